@@ -86,6 +86,19 @@ int tfcc_rocm_graph_destroy(void* graph_exec);
 int tfcc_rocm_memcpy_h2d(void* stream, void* dst_device, const void* src_host, size_t bytes);
 int tfcc_rocm_memcpy_d2h(void* stream, void* dst_host, const void* src_device, size_t bytes);
 int tfcc_rocm_memcpy_d2d_async(void* stream, void* dst, const void* src, size_t bytes);
+/* Page-locked host memory and copies between it and the device that are only enqueued on the stream.
+ * copy_to_pinned: all pieces, then *flag_pinned = epoch, raised by the GPU when every byte has arrived, for a host
+ * that polls instead of waiting for the stream.  `arrivals_device`: one zeroed word per stream, left zero. */
+int tfcc_rocm_host_malloc(void** ptr, size_t bytes);
+int tfcc_rocm_host_free(void* ptr);
+int tfcc_rocm_copy_from_pinned(void* stream, void* dst_device, const void* src_pinned, size_t bytes);
+typedef struct tfcc_rocm_copy_piece {
+  const void* src;
+  void* dst;
+  uint64_t bytes;
+} tfcc_rocm_copy_piece;
+int tfcc_rocm_copy_to_pinned(void* stream, const tfcc_rocm_copy_piece* pieces, unsigned count,
+                             unsigned* arrivals_device, unsigned* flag_pinned, unsigned epoch);
 /* fill `count` elements of `elem_size` (1, 2, 4 or 8) bytes with the bit pattern `value` */
 int tfcc_rocm_fill_async(void* stream, void* dst, uint64_t value, int elem_size, size_t count);
 

@@ -40,6 +40,23 @@ int tfcc_rocm_runtime_model_run(void* model, const void* inputs, size_t len, voi
                                 size_t* outputs_len);
 int tfcc_rocm_runtime_buffer_free(void* buffer);
 
+/* Model::run without the messages: the inputs are read where they lie (dtype: DataType of
+ * tfcc_runtime/proto/common.proto:5-20) and the outputs stay in one block of host memory that belongs to
+ * the result, page-locked where the process-wide bound of 256 MB allows.  result_output describes output
+ * `index`: its pointers are valid, and its data may be written, until result_free. */
+typedef struct tfcc_rocm_runtime_array {
+  const char* name;
+  int dtype;
+  const unsigned* shape;
+  size_t rank;
+  void* data;
+  size_t bytes;
+} tfcc_rocm_runtime_array;
+int tfcc_rocm_runtime_model_run_arrays(void* model, const tfcc_rocm_runtime_array* inputs, size_t count,
+                                       void** result, size_t* outputs);
+int tfcc_rocm_runtime_result_output(void* result, size_t index, tfcc_rocm_runtime_array* output);
+int tfcc_rocm_runtime_result_free(void* result);
+
 /* Model::test(npz, stream), model.cpp:185-280: runs the entrance graph on the arrays of an .npz and
  * compares every output found there; *passed = 1 when all are similar.  The summary text comes
  * back in *report (release with tfcc_rocm_runtime_buffer_free). */

@@ -1,0 +1,96 @@
+"""Model.run on numpy arrays: what it takes and returns equals the message form (run_serialized), at the sizes where its
+transfers change course, and its outputs stay valid for as long as they are held."""
+import gc
+import importlib
+
+import numpy as np
+import pytest
+
+NP = [np.float32, np.float64, np.int8, np.uint8, np.int16, np.uint16, np.int32, np.uint32, np.int64, np.uint64]
+
+
+@pytest.fixture(scope="module")
+def mf(pkg):
+    return importlib.import_module("wechat_tfcc_amd.modelfile")
+
+
+@pytest.fixture(scope="module")
+def rt(pkg):
+    return importlib.import_module("wechat_tfcc_amd.runtime_api")
+
+
+def copies(mf, rt, specs, host):
+    """a model that hands its inputs back: specs = [(dtype code, shape)]"""
+    g = mf.GraphBuilder("copies")
+    for i, (dtype, shape) in enumerate(specs):
+        x = g.input("x%d" % i, dtype, list(shape))
+        y = g._symbol("y%d" % i, dtype, mf.VARIABLE, list(shape))
+        g.node("base.Identity", [x], [y])
+        g.output(y)
+    return rt.Model(mf.write_model([g], g.name), host=host)
+
+
+def values(rng, dtype, shape):
+    if np.dtype(dtype).kind == "f":
+        return rng.standard_normal(shape).astype(dtype)
+    info = np.iinfo(dtype)
+    return rng.integers(info.min, info.max, shape, dtype=dtype, endpoint=True)
+
+
+def round_trip(mf, rt, shapes, host):
+    rng = np.random.default_rng(len(shapes))
+    specs = [(mf.DTYPE_OF[np.dtype(NP[i % len(NP)])], s) for i, s in enumerate(shapes)]
+    model = copies(mf, rt, specs, host)
+    inputs = {"x%d" % i: values(rng, NP[i % len(NP)], s) for i, s in enumerate(shapes)}
+    out = model.run(inputs)
+    message = mf.decode_outputs(model.run_serialized(mf.encode_inputs(inputs)))
+    assert list(out) == list(message) == ["y%d" % i for i in range(len(shapes))]
+    for i in range(len(shapes)):
+        got = out["y%d" % i]
+        assert got.dtype == inputs["x%d" % i].dtype and got.flags.writeable and got.flags.c_contiguous
+        assert np.array_equal(got, inputs["x%d" % i]) and np.array_equal(message["y%d" % i], got)
+
+
+def test_every_type_on_the_host_device(mf, rt):
+    round_trip(mf, rt, [(3,), (2, 3), (1,), (5,), (7, 1), (2, 2, 2), (9,), (4,), (3, 3), (2,)], True)
+
+
+def test_what_is_not_an_input_raises(mf, rt):
+    model = copies(mf, rt, [(mf.FLOAT, (2, 2))], True)
+    with pytest.raises(KeyError):
+        model.run({"x0": np.zeros((2, 2), np.float16)})
+    with pytest.raises(KeyError):
+        model.run({"x0": np.zeros((2, 2), ">f4")})
+    with pytest.raises(rt.RuntimeError_):
+        model.run({"nobody": np.zeros((2, 2), np.float32)})
+    with pytest.raises(rt.RuntimeError_, match="type not match"):
+        model.run({"x0": np.zeros((2, 2), np.float64)})
+    view = np.arange(8, dtype=np.float32).reshape(4, 2)[::2]  # not contiguous
+    assert np.array_equal(model.run({"x0": view})["y0"], view)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shapes", [
+    [(1,)], [(3,), (5,), (1,), (4093,)],                     # bytes that are no multiple of 16
+    [(4096,)], [(4097,)],                                    # one workgroup's 16 KB, and one element more
+    [(65536,)], [(65537,)],                                  # the first staged chunk of 256 KB
+    [((8 << 20) // 4 + 77,)], [(1 << 20,), (1 << 19,), (777,)],  # more than the staging block holds
+    [(i + 1,) for i in range(17)],                           # more pieces than one launch takes
+])
+def test_sizes_where_the_transfers_change(mf, rt, dev, shapes):
+    round_trip(mf, rt, shapes, False)
+
+
+@pytest.mark.gpu
+def test_outputs_outlive_the_model_and_later_runs(mf, rt, dev):
+    # 9 MB each: blocks of 16 MB, of which the process-wide bound admits sixteen; the runs beyond it get ordinary memory
+    n = (9 << 20) // 4
+    model = copies(mf, rt, [(mf.FLOAT, (n,))], False)
+    held = []
+    for i in range(20):
+        held.append(model.run({"x0": np.full(n, i, np.float32)})["y0"])
+    model.close()
+    for i, y in enumerate(held):
+        assert (y == i).all()
+    del held
+    gc.collect()

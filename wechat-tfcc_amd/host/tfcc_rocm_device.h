@@ -36,12 +36,71 @@ class ROCMDevice : public Device {
   static unsigned getDeviceCount();
 };
 
+// Page-locked host blocks, shared by all sessions and threads of the process: a block costs the driver hundreds of
+// microseconds to make, so freed ones are kept for the next request of their size class (powers of two).  Blocks in use
+// and kept together never exceed kMaxTotal; trim() gives the kept ones back (every session does that when it ends).
+class PinnedPool {
+  std::mutex _mtx;
+  std::map<void*, size_t> _live;
+  std::multimap<size_t, void*> _kept;
+  size_t _total = 0;
+
+  void trimLocked();
+
+ public:
+  static constexpr size_t kMaxBlock = size_t(64) << 20, kMaxTotal = size_t(256) << 20;
+  static PinnedPool& instance();
+  void* take(size_t bytes);  // nullptr: too large, the bound is reached, or there is no GPU
+  void give(void* block);
+  void trim();
+};
+
+// Host memory of a result: from the pool where that has room, ordinary memory otherwise.
+class HostBlock {
+  void* _data = nullptr;
+  bool _pinned = false;
+
+ public:
+  HostBlock() = default;
+  HostBlock(size_t bytes, bool gpu);  // gpu: ask the pool first
+  HostBlock(HostBlock&& o) noexcept : _data(o._data), _pinned(o._pinned) { o._data = nullptr; }
+  HostBlock& operator=(HostBlock&& o) noexcept {
+    std::swap(_data, o._data);
+    std::swap(_pinned, o._pinned);
+    return *this;
+  }
+  ~HostBlock();
+  char* data() const { return static_cast<char*>(_data); }
+  bool pinned() const { return _pinned; }
+};
+
 class ROCMSession : public Session {
   ROCMDevice& _device;
   void* _stream;  // hipStream_t
   bool _recording = false;  // the stream's launches are being recorded into a graph, not run
+  // host transfers: the block uploads are staged in and how much of it the stream may still read, the word the GPU
+  // raises after a download, the counter it needs for that
+  char* _staging = nullptr;
+  size_t _stagingSize = 0;
+  mutable size_t _stagingUsed = 0;
+  unsigned* _flag = nullptr;
+  unsigned* _arrivals = nullptr;
+  unsigned _epoch = 0;
+
+  bool reserveStaging(size_t bytes);
+  void waitForFlag();
 
  public:
+  struct HostRead {
+    const void* device;
+    void* host;
+    size_t bytes;
+  };
+  // device <- host memory that may be changed as soon as the call returns; the copy itself is ordered on the stream
+  void upload(void* device, const void* host, size_t bytes);
+  // host <- device, complete when the call returns.  pinned: the host addresses lie in blocks of PinnedPool.
+  void download(const std::vector<HostRead>& reads, bool pinned);
+
   explicit ROCMSession(ROCMDevice& device);
   ROCMSession(ROCMDevice& device, std::unique_ptr<Allocator> allocator);
   ~ROCMSession() override;

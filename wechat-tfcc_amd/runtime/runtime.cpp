@@ -165,27 +165,34 @@ std::string Node::debugString() const {
   return ss.str();
 }
 
-static DataItem parse_item(wire::Reader r) {
-  DataItem item;
+static InputView parse_item(wire::Reader r) {
+  InputView item;
   uint32_t f, t;
   while (r.next(f, t)) {
     if (f == 1 && t == 2) item.name = r.bytes();
     else if (f == 2 && t == 0) item.dtype = static_cast<DataType>(r.varint());
     else if (f == 3) r.repeatedVarint(t, item.shape);
-    else if (f == 4 && t == 2) item.data = r.bytes();
+    else if (f == 4 && t == 2) std::tie(item.data, item.bytes) = r.view();
     else r.skip(t);
   }
   return item;
 }
 
-static std::vector<DataItem> parse_items(const std::string& bytes, uint32_t field) {
-  std::vector<DataItem> items;
-  wire::Reader r(bytes);
+static std::vector<InputView> parse_views(const void* bytes, size_t len, uint32_t field) {
+  std::vector<InputView> items;
+  wire::Reader r(bytes, len);
   uint32_t f, t;
   while (r.next(f, t)) {
     if (f == field && t == 2) items.push_back(parse_item(r.sub()));
     else r.skip(t);
   }
+  return items;
+}
+
+static std::vector<DataItem> parse_items(const std::string& bytes, uint32_t field) {
+  std::vector<DataItem> items;
+  for (InputView& v : parse_views(bytes.data(), bytes.size(), field))
+    items.push_back({std::move(v.name), v.dtype, std::move(v.shape), std::string(v.data ? v.data : "", v.bytes)});
   return items;
 }
 
@@ -202,6 +209,7 @@ static std::string serialize_items(const std::vector<DataItem>& items, uint32_t 
   return w.take();
 }
 
+std::vector<InputView> parse_input_views(const void* bytes, size_t len) { return parse_views(bytes, len, 1); }
 std::vector<DataItem> parse_inputs(const std::string& bytes) { return parse_items(bytes, 1); }
 std::string serialize_inputs(const std::vector<DataItem>& items) { return serialize_items(items, 1); }
 std::vector<DataItem> parse_outputs(const std::string& bytes) { return parse_items(bytes, 2); }
@@ -663,75 +671,118 @@ Graph& Model::getGraph(const std::string& name) {
 
 namespace {
 template <class T>
-void add_input(Graph& graph, const proto::DataItem& item) {
+void add_input(Graph& graph, const proto::InputView& item, ROCMSession* rocm) {
   Shape shape(item.shape);
-  if (item.data.size() != static_cast<size_t>(shape.area()) * sizeof(T)) throw RuntimeError("Invalid data size");
+  if (item.bytes != static_cast<size_t>(shape.area()) * sizeof(T)) throw RuntimeError("Invalid data size");
   const SymbolInfo& info = graph.getSymbolManager().getSymbolInfo(item.name);
   if (is_value(info.stype)) {
     T v;
-    if (item.data.size() < sizeof(T)) throw RuntimeError("Invalid data size");
-    std::memcpy(&v, item.data.data(), sizeof(T));
+    if (item.bytes < sizeof(T)) throw RuntimeError("Invalid data size");
+    std::memcpy(&v, item.data, sizeof(T));
     graph.setInput(item.name, v);
     return;
   }
   Variable<T> v(shape);
-  if (v.size() > 0)
-    data::set(v, reinterpret_cast<const T*>(item.data.data()));
+  if (v.size() > 0) {
+    if (rocm) rocm->upload(v.data(), item.data, item.bytes);
+    else data::set(v, reinterpret_cast<const T*>(item.data));
+  }
   graph.setInput(item.name, std::move(v));
 }
 
 template <class T>
-void get_output(Graph& graph, const std::string& name, proto::DataItem& out) {
-  const SymbolInfo& info = graph.getSymbolManager().getSymbolInfo(name);
-  out.name = name;
-  out.dtype = info.dtype;
-  if (is_value(info.stype)) {
-    T v = graph.getValue(name, T());
+void describe_output(Graph& graph, const std::string& name, RunResult::Output& out) {
+  if (is_value(graph.getSymbolManager().getSymbolInfo(name).stype)) {
     out.shape = {1};
-    out.data.assign(reinterpret_cast<const char*>(&v), sizeof(T));
+    out.bytes = sizeof(T);
     return;
   }
   const Tensor<T>& tensor = graph.getTensor(name, T());
   out.shape = tensor.shape().toVector();
-  std::vector<T> v = data::get(tensor);
-  out.data.assign(reinterpret_cast<const char*>(v.data()), v.size() * sizeof(T));
+  out.bytes = static_cast<size_t>(tensor.size()) * sizeof(T);
+}
+
+template <class T>
+void get_output(Graph& graph, const RunResult::Output& out, char* host, bool rocm, std::vector<ROCMSession::HostRead>& reads) {
+  if (out.bytes == 0) return;
+  if (is_value(graph.getSymbolManager().getSymbolInfo(out.name).stype)) {
+    const T v = graph.getValue(out.name, T());
+    std::memcpy(host, &v, sizeof(T));
+    return;
+  }
+  const Tensor<T>& tensor = graph.getTensor(out.name, T());
+  if (rocm) reads.push_back({tensor.data(), host, out.bytes});
+  else ::tfcc::Operation<T>::getCurrentInterface().getDataInterface().get(tensor, reinterpret_cast<T*>(host));
 }
 }  // namespace
 
-void Model::run(const std::vector<proto::DataItem>& inputs, std::vector<proto::DataItem>& outputs) {
+RunResult Model::run(const std::vector<proto::InputView>& inputs) {
   Graph& graph = getEntranceGraph();
-  for (const proto::DataItem& item : inputs) {
+  auto* rocm = dynamic_cast<ROCMSession*>(Session::getThreadDefault());
+  for (const proto::InputView& item : inputs) {
     switch (item.dtype) {
 #define TFCC_RUNTIME_INPUT(T, E) \
-  case E: add_input<T>(graph, item); break;
+  case E: add_input<T>(graph, item, rocm); break;
       TFCC_RUNTIME_FOR_ALL_TYPES(TFCC_RUNTIME_INPUT)
 #undef TFCC_RUNTIME_INPUT
-      case BOOL: add_input<uint8_t>(graph, item); break;
+      case BOOL: add_input<uint8_t>(graph, item, rocm); break;
       default: throw RuntimeError("Invalid input dtype");
     }
   }
   graph.process();
+  RunResult result;
+  size_t total = 0;
   for (const std::string& name : graph.getOutputs()) {
-    outputs.emplace_back();
-    switch (graph.getSymbolManager().getSymbolInfo(name).dtype) {
+    const DataType dtype = graph.getSymbolManager().getSymbolInfo(name).dtype;
+    result.outputs.push_back({name, dtype, {}, total, 0});
+    RunResult::Output& out = result.outputs.back();
+    switch (dtype) {
+#define TFCC_RUNTIME_DESCRIBE(T, E) \
+  case E: describe_output<T>(graph, name, out); break;
+      TFCC_RUNTIME_FOR_ALL_TYPES(TFCC_RUNTIME_DESCRIBE)
+#undef TFCC_RUNTIME_DESCRIBE
+      case BOOL: describe_output<uint8_t>(graph, name, out); break;
+      default: throw RuntimeError("Invalid output type");
+    }
+    total += (out.bytes + 255) / 256 * 256;
+  }
+  result.block = HostBlock(total, rocm != nullptr);
+  std::vector<ROCMSession::HostRead> reads;
+  for (const RunResult::Output& out : result.outputs) {
+    char* host = result.block.data() + out.offset;
+    switch (out.dtype) {
 #define TFCC_RUNTIME_OUTPUT(T, E) \
-  case E: get_output<T>(graph, name, outputs.back()); break;
+  case E: get_output<T>(graph, out, host, rocm != nullptr, reads); break;
       TFCC_RUNTIME_FOR_ALL_TYPES(TFCC_RUNTIME_OUTPUT)
 #undef TFCC_RUNTIME_OUTPUT
-      case BOOL: get_output<uint8_t>(graph, name, outputs.back()); break;
+      case BOOL: get_output<uint8_t>(graph, out, host, rocm != nullptr, reads); break;
       default: throw RuntimeError("Invalid output type");
     }
   }
+  if (rocm) rocm->download(reads, result.block.pinned());
+  return result;
+}
+
+void Model::run(const std::vector<proto::DataItem>& inputs, std::vector<proto::DataItem>& outputs) {
+  std::vector<proto::InputView> views;
+  for (const proto::DataItem& item : inputs)
+    views.push_back({item.name, item.dtype, item.shape, item.data.data(), item.data.size()});
+  const RunResult result = run(views);
+  for (const RunResult::Output& out : result.outputs)
+    outputs.push_back({out.name, out.dtype, out.shape, std::string(result.block.data() + out.offset, out.bytes)});
 }
 
 void Model::run(const std::string& inputs, std::string& outputs) {
-  std::vector<proto::DataItem> in, out;
+  std::vector<proto::InputView> in;
   try {
-    in = proto::parse_inputs(inputs);
+    in = proto::parse_input_views(inputs.data(), inputs.size());
   } catch (wire::ParseError& e) {
     throw RuntimeError(std::string("Invalid inputs: ") + e.what());
   }
-  run(in, out);
+  const RunResult result = run(in);
+  std::vector<proto::DataItem> out;
+  for (const RunResult::Output& o : result.outputs)
+    out.push_back({o.name, o.dtype, o.shape, std::string(result.block.data() + o.offset, o.bytes)});
   outputs = proto::serialize_outputs(out);
 }
 

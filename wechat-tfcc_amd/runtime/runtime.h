@@ -26,6 +26,7 @@
 
 #include "archive.h"
 #include "tfcc_interfaces.h"
+#include "tfcc_rocm_device.h"
 #include "wire.h"
 
 namespace tfcc {
@@ -126,6 +127,15 @@ struct DataItem {  // data.proto:5-10
   std::vector<unsigned> shape;
   std::string data;
 };
+// the same without the copy: `data` points into memory of the caller's (for parse_input_views into `bytes`)
+struct InputView {
+  std::string name;
+  DataType dtype = UNKNOW;
+  std::vector<unsigned> shape;
+  const char* data = nullptr;
+  size_t bytes = 0;
+};
+std::vector<InputView> parse_input_views(const void* bytes, size_t len);
 std::vector<DataItem> parse_inputs(const std::string& bytes);          // Inputs{items = 1}
 std::string serialize_inputs(const std::vector<DataItem>& items);      // for callers and tests
 std::vector<DataItem> parse_outputs(const std::string& bytes);         // Outputs{items = 2}
@@ -370,6 +380,18 @@ class Graph {
   static bool isRecordDetailError() { return _recordDetailError; }
 };
 
+// The graph outputs of one run in one block of host memory.
+struct RunResult {
+  struct Output {
+    std::string name;
+    DataType dtype;
+    std::vector<unsigned> shape;
+    size_t offset, bytes;
+  };
+  HostBlock block;
+  std::vector<Output> outputs;
+};
+
 // ---- model ----------------------------------------------------------------------------------------------
 class Model {
   struct PerSession {
@@ -397,6 +419,7 @@ class Model {
   // copied host -> device, the entrance graph runs, every graph output is copied back
   void run(const std::string& inputs, std::string& outputs);
   void run(const std::vector<proto::DataItem>& inputs, std::vector<proto::DataItem>& outputs);
+  RunResult run(const std::vector<proto::InputView>& inputs);
 
   // runs the entrance graph on the arrays of an .npz and compares each output present there
   // (model.cpp:185-280); prints a summary to `stream`

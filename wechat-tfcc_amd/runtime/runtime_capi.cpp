@@ -81,6 +81,40 @@ int tfcc_rocm_runtime_model_run(void* model, const void* inputs, size_t len, voi
   });
 }
 
+int tfcc_rocm_runtime_model_run_arrays(void* model, const tfcc_rocm_runtime_array* inputs, size_t count, void** result,
+                                       size_t* outputs) {
+  return guarded([&] {
+    if ((inputs == nullptr && count > 0) || result == nullptr || outputs == nullptr)
+      throw tfcc::InvalidArgumentError("null argument");
+    std::vector<tfcc::runtime::proto::InputView> views(count);
+    for (size_t i = 0; i < count; ++i) {
+      tfcc::runtime::proto::InputView& v = views[i];
+      v.name = inputs[i].name;
+      v.dtype = static_cast<tfcc::runtime::DataType>(inputs[i].dtype);
+      v.shape.assign(inputs[i].shape, inputs[i].shape + inputs[i].rank);
+      v.data = static_cast<const char*>(inputs[i].data);
+      v.bytes = inputs[i].bytes;
+    }
+    std::unique_ptr<tfcc::runtime::RunResult> r(new tfcc::runtime::RunResult(as_model(model).run(views)));
+    *outputs = r->outputs.size();
+    *result = r.release();
+  });
+}
+
+int tfcc_rocm_runtime_result_output(void* result, size_t index, tfcc_rocm_runtime_array* output) {
+  return guarded([&] {
+    if (result == nullptr || output == nullptr) throw tfcc::InvalidArgumentError("null argument");
+    auto& r = *static_cast<tfcc::runtime::RunResult*>(result);
+    const tfcc::runtime::RunResult::Output& o = r.outputs.at(index);
+    *output = {o.name.c_str(), static_cast<int>(o.dtype), o.shape.data(), o.shape.size(), r.block.data() + o.offset, o.bytes};
+  });
+}
+
+int tfcc_rocm_runtime_result_free(void* result) {
+  delete static_cast<tfcc::runtime::RunResult*>(result);
+  return 0;
+}
+
 int tfcc_rocm_runtime_buffer_free(void* buffer) {
   std::free(buffer);
   return 0;

@@ -10,6 +10,7 @@
 #include <cstring>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
 
 namespace tfcc {
@@ -66,6 +67,11 @@ class Reader {
   std::string bytes() {
     Reader r = sub();
     return std::string(reinterpret_cast<const char*>(r._p), static_cast<size_t>(r._end - r._p));
+  }
+  // the bytes themselves, where the parent buffer holds them
+  std::pair<const char*, size_t> view() {
+    Reader r = sub();
+    return {reinterpret_cast<const char*>(r._p), static_cast<size_t>(r._end - r._p)};
   }
   // next key; false at the end of the message
   bool next(uint32_t& field, uint32_t& type) {

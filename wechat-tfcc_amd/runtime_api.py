@@ -17,6 +17,9 @@ SYMBOLS = {
     "tfcc_rocm_runtime_model_destroy": (C.c_int, [_VP]),
     "tfcc_rocm_runtime_model_run": (C.c_int, [_VP, _VP, C.c_size_t, C.POINTER(_VP), C.POINTER(C.c_size_t)]),
     "tfcc_rocm_runtime_buffer_free": (C.c_int, [_VP]),
+    "tfcc_rocm_runtime_model_run_arrays": (C.c_int, [_VP, _VP, C.c_size_t, C.POINTER(_VP), C.POINTER(C.c_size_t)]),
+    "tfcc_rocm_runtime_result_output": (C.c_int, [_VP, C.c_size_t, _VP]),
+    "tfcc_rocm_runtime_result_free": (C.c_int, [_VP]),
     "tfcc_rocm_runtime_model_test": (C.c_int, [_VP, _VP, C.c_size_t, C.POINTER(C.c_int), C.POINTER(_VP)]),
     "tfcc_rocm_runtime_set_fusion": (C.c_int, [C.c_int]),
     "tfcc_rocm_runtime_model_step_count": (C.c_int, [_VP, C.POINTER(C.c_size_t)]),
@@ -25,6 +28,19 @@ SYMBOLS = {
 }
 
 _lib = None
+
+
+_model_calls = None
+
+
+def _calls():
+    """the compiled half of Model.run (host/model_calls.cpp)"""
+    global _model_calls
+    if _model_calls is None:
+        lib()
+        from . import _model_calls as module
+        _model_calls = module
+    return _model_calls
 
 
 class RuntimeError_(RuntimeError):
@@ -88,8 +104,8 @@ class Model:
             lib().tfcc_rocm_runtime_buffer_free(out)
 
     def run(self, arrays):
-        """{name: ndarray} -> {name: ndarray}"""
-        return modelfile.decode_outputs(self.run_serialized(modelfile.encode_inputs(arrays)))
+        """{name: ndarray} -> {name: ndarray}: what run_serialized does with the messages of modelfile, without them"""
+        return _calls().run(self._h.value or 0, arrays, RuntimeError_)
 
     def test(self, npz_bytes):
         passed, report = C.c_int(), _VP()
