@@ -170,6 +170,20 @@ def lib():
     return _lib
 
 
+_calls = None
+
+
+def _native():
+    """The compiled form of the operators below on plain operands (host/tensor_calls.cpp).  Each of its functions returns
+    None for what the Python form that follows the call has to see to."""
+    global _calls
+    if _calls is None:
+        lib()
+        from . import _tensor_calls
+        _calls = _tensor_calls
+    return _calls
+
+
 def check(status):
     if status != 0:
         raise TfccRocmError("tfcc_rocm error %d: %s" % (status, lib().tfcc_rocm_last_error_string().decode()))
@@ -252,6 +266,9 @@ def matmul_plan(shape_a, shape_b, shape_bias=None):
 
 def blas_matmul(a, b, bias=None):
     """tfcc::blas::matmul(a, b[, bias]) on fp32 device tensors."""
+    done = _native().blas_matmul(a, b, bias)
+    if done is not None:
+        return done
     import torch
     for t in (a, b) + (() if bias is None else (bias,)):
         if t.dtype != torch.float32:
@@ -330,6 +347,9 @@ def sgemm_grouped(a, bs, biases):
 def reduce_sum(a, row):
     """tfcc::mkl::quantization::reduce_sum: int32 sums over the last (row=True) or the
     second-to-last (row=False) dimension."""
+    done = _native().reduce_sum(a, row)
+    if done is not None:
+        return done
     import torch
     if a.numel() == 0 or a.dim() < 2:
         raise InvalidArgumentError("invalid input tensor a")
@@ -386,6 +406,9 @@ def _check_scalar(t, name):
 
 def quantization_matmul(a, reduce_a, min_a, max_a, b, reduce_b, min_b, max_b):
     """tfcc::mkl::quantization::matmul: returns (int32 C, minC, maxC); ranges are 1-element device tensors."""
+    done = _native().quantization_matmul(a, reduce_a, min_a, max_a, b, reduce_b, min_b, max_b)
+    if done is not None:
+        return done
     import torch
     a, b, reduce_a, reduce_b = a.contiguous(), b.contiguous(), reduce_a.contiguous(), reduce_b.contiguous()
     for t, nm in ((min_a, "minA"), (max_a, "maxA"), (min_b, "minB"), (max_b, "maxB")):
@@ -415,6 +438,10 @@ def quantization_matmul_requantize(a, reduce_a, min_a, max_a, b, reduce_b, min_b
                                    want_acc=False, colsum_exact=False):
     """matmul followed by requantize<uint8_t> in one kernel.  Returns (uint8 Q, int32 C or None, minC, maxC).
     colsum_exact: the caller's promise that reduce_b holds the true column sums of b."""
+    done = _native().quantization_matmul_requantize(a, reduce_a, min_a, max_a, b, reduce_b, min_b, max_b, min_out, max_out, want_acc,
+                                                    colsum_exact)
+    if done is not None:
+        return done
     import torch
     a, b, reduce_a, reduce_b = a.contiguous(), b.contiguous(), reduce_a.contiguous(), reduce_b.contiguous()
     for t, nm in ((min_a, "minA"), (max_a, "maxA"), (min_b, "minB"), (max_b, "maxB"), (min_out, "minOutput"),
@@ -441,6 +468,10 @@ def gemv_dequant(a, b, reduce_a, reduce_b, offset_a, offset_b, scale_a, scale_b,
     """Skinny (M <= 8) product with optional fused per-channel dequantize.  Returns (f32 or None, int32 or None).
     no_alloc: through the entry point that allocates nothing (the caller then passes `out` / `acc` too).
     colsum_exact: the caller vouches that reduce_b holds the true column sums of b."""
+    if out is None and acc is None and not no_alloc:
+        done = _native().gemv_dequant(a, b, reduce_a, reduce_b, offset_a, offset_b, scale_a, scale_b, want_acc, colsum_exact)
+        if done is not None:
+            return done
     import torch
     a, b = a.contiguous(), b.contiguous()
     m, k, n = a.shape[0], a.shape[1], b.shape[1]
@@ -472,6 +503,9 @@ def gemv_pack(b):
 
 def gemv_dequant_packed(a, packed, n, reduce_a, reduce_b, offset_a, offset_b, scale_a, scale_b, want_acc=True):
     """gemv_dequant on weights packed by gemv_pack (n: the column count of the original matrix)."""
+    done = _native().gemv_dequant_packed(a, packed, n, reduce_a, reduce_b, offset_a, offset_b, scale_a, scale_b, want_acc)
+    if done is not None:
+        return done
     import torch
     a = a.contiguous()
     m, k = a.shape
@@ -499,6 +533,9 @@ def requantize(a, min_in, max_in, min_out, max_out, out_dtype):
 
 def dequantize(a, min_v, max_v):
     """tfcc::quantization::dequantize(a, minValue, maxValue)"""
+    done = _native().dequantize(a, min_v, max_v)
+    if done is not None:
+        return done
     import torch
     if a.numel() == 0:
         raise InvalidArgumentError("invalid tensor")
@@ -514,6 +551,10 @@ def dequantize(a, min_v, max_v):
 
 def quantize(a, out_dtype, min_v=None, max_v=None):
     """tfcc::quantization::quantize<T>(a) -> (q, min, max), or quantize<T>(a, min, max) -> q"""
+    if min_v is None and max_v is None:
+        done = _native().quantize(a, out_dtype)
+        if done is not None:
+            return done
     import torch
     if a.numel() == 0:
         raise InvalidArgumentError("invalid tensor")
