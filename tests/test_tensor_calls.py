@@ -45,7 +45,7 @@ def test_same_bits_as_the_python_form(pkg, dev, monkeypatch, m, k, n):
             for exact in (False, True):
                 outs += pkg.quantization_matmul_requantize(a, row, lo, hi, b, col, lo, hi, one(-9e5), one(9e5), want_acc=acc,
                                                            colsum_exact=exact)
-        if m <= 8:
+        if m <= 8 and k % 16 == 0:  # the packed form takes no other k
             scale = torch.rand(n, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
             for acc in (False, True):
                 outs += pkg.gemv_dequant(a, b, row, col, -128, 3, 0.02, scale, want_acc=acc)

@@ -464,108 +464,89 @@ bool takes_128_tiles(unsigned m, unsigned n, unsigned fillBatch) {
 
 int k_groups_of_plain_product(unsigned m, unsigned n, unsigned k, unsigned fillBatch) {
   if (takes_128_tiles(m, n, fillBatch)) return 1;
-  if (k % 32 == 0) {
-    int best, ksplit;
-    unsigned long long tiles;
-    choose_dma_tiles(m, n, k, fillBatch, best, tiles, ksplit);
-    return ksplit;
-  }
-  const unsigned long long small = (unsigned long long)((m + 63) / 64) * ((n + 63) / 64) * fillBatch;
-  const unsigned long long flat = (unsigned long long)((m + 31) / 32) * ((n + 95) / 96) * fillBatch;
-  const bool preferFlat = ((flat + 255) / 256) * (32 * 96) < ((small + 255) / 256) * (64 * 64);
-  if (preferFlat && flat <= 320 && k >= 512) return 4;
-  if (small <= 320 && k >= 512) return 4;
-  if (small <= 640 && k >= 256) return 2;
-  return 1;
+  int best, ksplit;
+  unsigned long long tiles;
+  choose_dma_tiles(m, n, k, fillBatch, best, tiles, ksplit);
+  return ksplit;
 }
 
 // Picks the tile configuration from the shape of one product and the number of batch entries that
 // count towards filling the chip (`fillBatch`), and launches.
-int dispatch(hipStream_t s, const SgemmParams& p, bool vec, bool tb, unsigned fillBatch, unsigned lda, unsigned ldb,
-             unsigned ldc) {
+int dispatch(hipStream_t s, const SgemmParams& p, bool vec, bool small, bool tb, unsigned fillBatch) {
   const unsigned m = p.M, n = p.N, k = p.K;
-  const unsigned long long rowsB = tb ? n : k;
   if (tb) {
+    const int groups = k_groups_of_plain_product(m, n, k, fillBatch);
     if (vec) {
-      const int groups = k_groups_of_plain_product(m, n, k, fillBatch);
       if (groups == 4) return launch<2, 2, 1, 1, true, 4, true>(s, p);
       if (groups == 2) return launch<2, 2, 1, 1, true, 2, true>(s, p);
       return launch<2, 2, 1, 1, true, 1, true>(s, p);
     }
-    TFCC_REQUIRE((unsigned long long)m * ldc < (1ull << 32) && (unsigned long long)m * lda < (1ull << 32) &&
-                 rowsB * ldb < (1ull << 32), "sgemm: operand larger than 2^32 elements");
+    TFCC_REQUIRE((unsigned long long)m * p.ldc < (1ull << 32) && (unsigned long long)m * p.lda < (1ull << 32) &&
+                 (unsigned long long)n * p.ldb < (1ull << 32), "sgemm: operand larger than 2^32 elements");
+    if (groups == 4) return launch<2, 2, 1, 1, false, 4, true>(s, p);
+    if (groups == 2) return launch<2, 2, 1, 1, false, 2, true>(s, p);
     return launch<2, 2, 1, 1, false, 1, true>(s, p);
   }
   // One product (or a few that share A) of at most eight rows: a single pass over B decides the time, and the
   // streaming kernel makes it without tiles.  A true batch keeps the tiled kernels, whose sums the fused attention
   // kernel reproduces bit for bit.
   if (fillBatch == 1 && sgemm_detail::sgemv_supported(p)) return sgemm_detail::sgemv_launch(s, p);
-  // 128x128 tiles once there are enough of them to fill the 256 CUs twice over, else 64x64
-  if (vec) {
-    // (whole slabs of K: four hand-scheduled wavefronts of 32 x 128 on a shared ring, two workgroups per CU -
-    // 4096^3: 150 TFLOP/s against 141 for the same tiles scheduled by the compiler)
-    if (takes_128_tiles(m, n, fillBatch)) return k % 32 == 0 ? sgemm_detail::sgemm_wave96_launch(s, p, 1, 4) : launch<4, 1, 1, 4, true>(s, p);
-    // few 64x64 tiles and a long K: several K groups per workgroup keep the CUs that have a tile busy
-    const unsigned long long small = (unsigned long long)((m + 63) / 64) * ((n + 63) / 64) * fillBatch;
-    // 32x96 tiles when they cover the 256 CUs in fewer tile-area rounds than 64x64 tiles would
-    const unsigned long long flat = (unsigned long long)((m + 31) / 32) * ((n + 95) / 96) * fillBatch;
-    const bool preferFlat = ((flat + 255) / 256) * (32 * 96) < ((small + 255) / 256) * (64 * 64);
-    if (k % 32 == 0) {
-      // whole slabs of K: the kernels that copy the slabs straight into LDS
-      int best, ksplit;
-      unsigned long long bestTiles;
-      choose_dma_tiles(m, n, k, fillBatch, best, bestTiles, ksplit);
-      // The hand-scheduled kernel of sgemm_wave96.hip (one wavefront per SIMD, no vector instruction between its
-      // matrix ops) takes every product with four K groups - the groups as the four wavefronts of a workgroup on
-      // 32 x 96, 32 x 64 and 32 x 32 tiles, four pairs of wavefronts on 64 x 64 tiles (1024 x 768 x 3072: 36.3
-      // against 45.9 us for the kernels of sgemm_dma.hip, 128 x 768 x 3072: 8.6 against 11.4 with the operands in
-      // cache, 960 x 1024 x 2048: 34.4 against 41.9) ...
-      if (ksplit == 4) {
-        // (Tiles of 16 x 96 from 16x16x4 matrix ops - the same bits, 256 tiles instead of 192 for 128 x 768 x 3072 and
-        // a quarter less matrix time - were built and measured: 7.6 against 8.3 us with the operands in cache, 10.1
-        // against 9.8 with them in HBM, where the wait for the first slab and the bytes in flight decide, not the
-        // matrix ops.  The table's tiles keep the product.)
-        const int c = kTiles[best].config;
-        return sgemm_detail::sgemm_wave96_launch(s, p, 4, c == 0 ? 2 : c == 1 ? 3 : c == 2 ? 2 : 1, c == 0 ? 2 : 1);
-      }
-      // ... with two K groups the 64 x 64 tiles (two pairs of wavefronts) and the 32 x 32 tiles (two wavefronts):
-      // 1024^3 20.1 against 24.2 us, 400 x 400 x 256 5.3 against 7.3; on 32 x 96 and 32 x 64 tiles the kernels of
-      // sgemm_dma.hip are as fast or faster and keep the product ...
-      if (ksplit == 2 && kTiles[best].config == 0) return sgemm_detail::sgemm_wave96_launch(s, p, 2, 2, 2);
-      if (ksplit == 2 && kTiles[best].config == 3) return sgemm_detail::sgemm_wave96_launch(s, p, 2, 1, 1);
-      // ... and without K groups the products whose 128 x 96 tiles fill at least 70 % of the CUs in each of their
-      // rounds (or 128 x 128 tiles 85 %), K >= 512: four wavefronts of 32 x 96 (32 x 128) share each copy of B
-      // (1024 x 3072 x 768 with GELU: 39.3 against 42.4 us in 64 x 64 tiles, 1536^3: 69 against 80, 2048^3 in
-      // 128 x 128 tiles: 120 against 136; below those fills, or with a short K, the tiles of the table win).  The
-      // sums are the same in every case: the K groups of the table, ascending k inside a group.
-      if (ksplit == 1 && k >= 512) {
-        const unsigned long long wide = (unsigned long long)((m + 127) / 128) * ((n + 95) / 96) * fillBatch;
-        const unsigned long long wide4 = (unsigned long long)((m + 127) / 128) * ((n + 127) / 128) * fillBatch;
-        const bool ok3 = wide * 100 >= 70 * 256 * ((wide + 255) / 256), ok4 = wide4 * 100 >= 85 * 256 * ((wide4 + 255) / 256);
-        const unsigned long long cost3 = ((wide + 255) / 256) * 96, cost4 = ((wide4 + 255) / 256) * 128;
-        if (ok4 && (!ok3 || cost4 < cost3)) return sgemm_detail::sgemm_wave96_launch(s, p, 1, 4);
-        if (ok3) return sgemm_detail::sgemm_wave96_launch(s, p, 1);
-      }
-      // What is left runs on the kernels of sgemm_dma.hip.  Several products in one launch (p.batch counts them;
-      // fillBatch = 1 chose the configuration of a single one so that each is summed exactly as on its own): when
-      // they fill the chip without the K groups, one group per tile plays all of them; and when 128 x 96 tiles over
-      // all of them still occupy most of the CUs in one round, twelve wavefronts share each copy of B among four
-      // times the rows (the sums are those of the 32 x 96 tiles).
-      const bool serial = ksplit > 1 && bestTiles * (p.batch / fillBatch) * kTiles[best].waves >= 256ull * 8;
-      if (serial && kTiles[best].config == 1) {
-        const unsigned long long wide = (unsigned long long)((m + 127) / 128) * ((n + 95) / 96) * p.batch;
-        if (wide <= 256 && wide >= 160) return sgemm_detail::sgemm_dma_launch(s, p, 5, ksplit, true);
-      }
-      return sgemm_detail::sgemm_dma_launch(s, p, kTiles[best].config, ksplit, serial);
-    }
-    if (preferFlat && flat <= 320 && k >= 512) return launch<1, 3, 1, 1, true, 4>(s, p);
-    if (small <= 320 && k >= 512) return launch<2, 2, 1, 1, true, 4>(s, p);
-    if (small <= 640 && k >= 256) return launch<2, 2, 1, 1, true, 2>(s, p);
-    return launch<2, 2, 1, 1, true>(s, p);
+  if (!small) {  // operands past the reach of a buffer descriptor
+    TFCC_REQUIRE((unsigned long long)m * p.ldc < (1ull << 32) && (unsigned long long)m * p.lda < (1ull << 32) &&
+                 (unsigned long long)k * p.ldb < (1ull << 32), "sgemm: operand larger than 2^32 elements");
+    return launch<2, 2, 1, 1, false>(s, p);
   }
-  TFCC_REQUIRE((unsigned long long)m * ldc < (1ull << 32) && (unsigned long long)m * lda < (1ull << 32) &&
-               rowsB * ldb < (1ull << 32), "sgemm: operand larger than 2^32 elements");
-  return launch<2, 2, 1, 1, false>(s, p);
+  // Everything else runs on the kernels that copy K slabs straight into LDS, whatever its alignment (333 x 1003 x 517:
+  // 8.8 us against 64.7 for register-staged slabs fetched word by word, 2000 x 1501 x 3003: 138 against 350).
+  // 128x128 tiles once there are enough of them to fill the 256 CUs twice over: four hand-scheduled wavefronts of
+  // 32 x 128 on a shared ring, two workgroups per CU - 4096^3: 150 TFLOP/s against 141 for the same tiles scheduled by
+  // the compiler.
+  if (takes_128_tiles(m, n, fillBatch)) return sgemm_detail::sgemm_wave96_launch(s, p, 1, 4);
+  int best, ksplit;
+  unsigned long long bestTiles;
+  choose_dma_tiles(m, n, k, fillBatch, best, bestTiles, ksplit);
+  // The hand-scheduled kernel of sgemm_wave96.hip (one wavefront per SIMD, no vector instruction between its
+  // matrix ops) takes every product with four K groups - the groups as the four wavefronts of a workgroup on
+  // 32 x 96, 32 x 64 and 32 x 32 tiles, four pairs of wavefronts on 64 x 64 tiles (1024 x 768 x 3072: 36.3
+  // against 45.9 us for the kernels of sgemm_dma.hip, 128 x 768 x 3072: 8.6 against 11.4 with the operands in
+  // cache, 960 x 1024 x 2048: 34.4 against 41.9) ...
+  if (ksplit == 4) {
+    // (Tiles of 16 x 96 from 16x16x4 matrix ops - the same bits, 256 tiles instead of 192 for 128 x 768 x 3072 and
+    // a quarter less matrix time - were built and measured: 7.6 against 8.3 us with the operands in cache, 10.1
+    // against 9.8 with them in HBM, where the wait for the first slab and the bytes in flight decide, not the
+    // matrix ops.  The table's tiles keep the product.)
+    const int c = kTiles[best].config;
+    return sgemm_detail::sgemm_wave96_launch(s, p, 4, c == 0 ? 2 : c == 1 ? 3 : c == 2 ? 2 : 1, c == 0 ? 2 : 1);
+  }
+  // ... with two K groups the 64 x 64 tiles (two pairs of wavefronts) and the 32 x 32 tiles (two wavefronts):
+  // 1024^3 20.1 against 24.2 us, 400 x 400 x 256 5.3 against 7.3; on 32 x 96 and 32 x 64 tiles the kernels of
+  // sgemm_dma.hip are as fast or faster and keep the product ...
+  if (ksplit == 2 && kTiles[best].config == 0) return sgemm_detail::sgemm_wave96_launch(s, p, 2, 2, 2);
+  if (ksplit == 2 && kTiles[best].config == 3) return sgemm_detail::sgemm_wave96_launch(s, p, 2, 1, 1);
+  // ... and without K groups the products whose 128 x 96 tiles fill at least 70 % of the CUs in each of their
+  // rounds (or 128 x 128 tiles 85 %), K >= 512: four wavefronts of 32 x 96 (32 x 128) share each copy of B
+  // (1024 x 3072 x 768 with GELU: 39.3 against 42.4 us in 64 x 64 tiles, 1536^3: 69 against 80, 2048^3 in
+  // 128 x 128 tiles: 120 against 136; below those fills, or with a short K, the tiles of the table win).  The
+  // sums are the same in every case: the K groups of the table, ascending k inside a group.
+  if (ksplit == 1 && k >= 512) {
+    const unsigned long long wide = (unsigned long long)((m + 127) / 128) * ((n + 95) / 96) * fillBatch;
+    const unsigned long long wide4 = (unsigned long long)((m + 127) / 128) * ((n + 127) / 128) * fillBatch;
+    const bool ok3 = wide * 100 >= 70 * 256 * ((wide + 255) / 256), ok4 = wide4 * 100 >= 85 * 256 * ((wide4 + 255) / 256);
+    const unsigned long long cost3 = ((wide + 255) / 256) * 96, cost4 = ((wide4 + 255) / 256) * 128;
+    if (ok4 && (!ok3 || cost4 < cost3)) return sgemm_detail::sgemm_wave96_launch(s, p, 1, 4);
+    if (ok3) return sgemm_detail::sgemm_wave96_launch(s, p, 1);
+  }
+  // What is left runs on the kernels of sgemm_dma.hip.  Several products in one launch (p.batch counts them;
+  // fillBatch = 1 chose the configuration of a single one so that each is summed exactly as on its own): when
+  // they fill the chip without the K groups, one group per tile plays all of them; and when 128 x 96 tiles over
+  // all of them still occupy most of the CUs in one round, twelve wavefronts share each copy of B among four
+  // times the rows (the sums are those of the 32 x 96 tiles).
+  const bool serial = ksplit > 1 && bestTiles * (p.batch / fillBatch) * kTiles[best].waves >= 256ull * 8;
+  if (serial && kTiles[best].config == 1) {
+    const unsigned long long wide = (unsigned long long)((m + 127) / 128) * ((n + 95) / 96) * p.batch;
+    if (wide <= 256 && wide >= 160) return sgemm_detail::sgemm_dma_launch(s, p, 5, ksplit, true);
+  }
+  return sgemm_detail::sgemm_dma_launch(s, p, kTiles[best].config, ksplit, serial);
 }
 
 }  // namespace
@@ -617,14 +598,14 @@ extern "C" int tfcc_rocm_sgemm_general(void* stream, const tfcc_rocm_sgemm_desc*
   const unsigned batch = p.batch;
   const bool tb = d->trans_b != 0;
   const unsigned long long rowsB = tb ? n : k, colsB = tb ? k : n;  // B as stored
+  const bool small = (((unsigned long long)m + 256) * d->lda + k + 256 < (1ull << 30)) &&
+                     ((rowsB + 256) * d->ldb + colsB + 1024 < (1ull << 30));
   const bool vec = (k % 4 == 0) && (n % 4 == 0) && ((uintptr_t)d->a % 16 == 0) && ((uintptr_t)d->b % 16 == 0) &&
                    ((uintptr_t)d->c % 16 == 0) && (d->lda % 4 == 0) && (d->ldb % 4 == 0) && (d->ldc % 4 == 0) &&
                    (p.strideA % 4 == 0) && (p.strideB % 4 == 0) && (p.strideC % 4 == 0) && (p.innerA % 4 == 0) &&
-                   (p.innerB % 4 == 0) && (p.innerC % 4 == 0) &&
-                   (((unsigned long long)m + 256) * d->lda + k + 256 < (1ull << 30)) &&
-                   ((rowsB + 256) * d->ldb + colsB + 1024 < (1ull << 30));
+                   (p.innerB % 4 == 0) && (p.innerC % 4 == 0) && small;
   hipStream_t s = as_stream(stream);
-  return dispatch(s, p, vec, tb, batch, d->lda, d->ldb, d->ldc);
+  return dispatch(s, p, vec, small, tb, batch);
 }
 
 extern "C" int tfcc_rocm_sgemm_grouped(void* stream, const float* a, const float* const* b, const float* const* bias,
@@ -636,21 +617,19 @@ extern "C" int tfcc_rocm_sgemm_grouped(void* stream, const float* a, const float
   p.A = a; p.M = m; p.N = n; p.K = k; p.batch = groups; p.batchInner = 1;
   p.lda = k; p.ldb = n; p.ldc = n;
   p.groups = groups;
-  bool aligned = (uintptr_t)a % 16 == 0;
   for (unsigned g = 0; g < 4; ++g) {
     const unsigned src = g < groups ? g : 0;
     TFCC_REQUIRE(b[src] && c[src], "grouped sgemm: null operand");
     p.groupB[g] = b[src];
     p.groupBias[g] = bias ? bias[src] : nullptr;
     p.groupC[g] = c[src];
-    aligned = aligned && (uintptr_t)b[src] % 16 == 0 && (uintptr_t)c[src] % 16 == 0;
   }
   p.B = p.groupB[0];
   p.C = p.groupC[0];
-  const bool vec = aligned && (k % 4 == 0) && (n % 4 == 0) && (((unsigned long long)m + 256) * k + k + 256 < (1ull << 30)) &&
-                   (((unsigned long long)k + 256) * n + n + 1024 < (1ull << 30));
+  const bool small = (((unsigned long long)m + 256) * k + k + 256 < (1ull << 30)) &&
+                     (((unsigned long long)k + 256) * n + n + 1024 < (1ull << 30));
   // the tile configuration is the one a single product of this shape gets, so that every product
   // of the group is summed in exactly the order of a launch of its own
-  return dispatch(as_stream(stream), p, vec, false, 1, k, n, n);
+  return dispatch(as_stream(stream), p, false, small, false, 1);
 }
 

@@ -14,8 +14,9 @@
 // slabs per K group is kept in flight; one barrier per slab, placed before the slab's last step so
 // that the freed stage is refilled while that step's matrix ops run.
 //
-// Taken only for 16-byte aligned operands and strides, K a multiple of 32 (a partial slab of A
-// cannot be zeroed on its way into LDS) and B not transposed.
+// Taken for B not transposed.  Addresses need to be multiples of four bytes only, and the range check of a copy looks
+// at every word.  A partial slab of A cannot be zeroed on its way into LDS: RAGGED (K not a multiple of 32) masks the
+// operands of the slab in which K ends as they are read.
 #include "common.hpp"
 #include "lds_dma.hpp"
 #include "sgemm_params.hpp"
@@ -42,7 +43,7 @@ __device__ __forceinline__ int row_swizzle(int row) { return (row >> 1) & 7; }
 // accumulator per would-be group (slab s goes to accumulator s % VSPLIT) and the same final additions in
 // group order - bit for bit the result of KSPLIT = VSPLIT, for launches that fill the chip without
 // splitting K across wavefronts (several products in one launch).
-template <int WGM, int WGN, int NI, int KSPLIT, int STAGES, int VSPLIT = 1>
+template <int WGM, int WGN, int NI, int KSPLIT, int STAGES, int VSPLIT, bool RAGGED>
 __global__ __launch_bounds__(WGM * WGN * 64 * KSPLIT) void sgemm_dma_kernel(const SgemmParams p) {
   static_assert(VSPLIT == 1 || KSPLIT == 1, "accumulators per would-be group only without real groups");
   static_assert(NI == 1 || NI == 3 || NI == 4, "a lane reads its B operands as one word, three words 32 columns apart or four consecutive words");
@@ -155,9 +156,18 @@ __global__ __launch_bounds__(WGM * WGN * 64 * KSPLIT) void sgemm_dma_kernel(cons
   const int arow = wm * 32 + lrow;
   const int aBase = arow * (BK * 4), aSwz = row_swizzle(arow);
   const int bBase = A_BYTES + (4 * g) * (BN * 4) + (wn * WN + (STRIDED ? lrow : NI * lrow)) * 4;
-  auto readOps = [&](unsigned stage, int kb, v4f& a, BOps& b) {
+  auto readOps = [&](unsigned slab, unsigned stage, int kb, v4f& a, BOps& b) {
     const unsigned char* st = gsm + stage * STAGE_BYTES;
     a = *reinterpret_cast<const v4f*>(st + aBase + (((2 * kb + g) ^ aSwz) << 4));
+    if constexpr (RAGGED) {
+      const unsigned k0 = (slab * KSPLIT + grp) * BK;
+      if (k0 + BK > K) {
+        asm volatile("" ::: "memory");  // a real (wave-uniform) branch, taken by the last slab only
+        const int left = (int)K - (int)(k0 + 8 * kb + 4 * g);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) a[s] = s < left ? a[s] : 0.f;
+      }
+    }
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       if constexpr (NI == 4) {
@@ -220,7 +230,7 @@ __global__ __launch_bounds__(WGM * WGN * 64 * KSPLIT) void sgemm_dma_kernel(cons
   if constexpr (!PRIVATE_RING) __syncthreads();
   v4f fa[2];
   BOps fb[2];
-  readOps(0, 0, fa[0], fb[0]);
+  readOps(0, 0, 0, fa[0], fb[0]);
   for (unsigned ko = 0; ko < (KT + VSPLIT - 1) / VSPLIT; ++ko) {
 #pragma unroll
     for (int v = 0; v < VSPLIT; ++v) {  // a slab past the end of K is all zeros
@@ -228,13 +238,13 @@ __global__ __launch_bounds__(WGM * WGN * 64 * KSPLIT) void sgemm_dma_kernel(cons
       const unsigned cur = kt % STAGES, nxt = (kt + 1) % STAGES;
 #pragma unroll
       for (int kb = 0; kb < KS - 1; ++kb) {
-        readOps(cur, kb + 1, fa[(kb + 1) & 1], fb[(kb + 1) & 1]);
+        readOps(kt, cur, kb + 1, fa[(kb + 1) & 1], fb[(kb + 1) & 1]);
         mma(accs[v], fa[kb & 1], fb[kb & 1]);
       }
       wait_vmcnt<COPIES*(STAGES - 2)>();
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the reads of slab kt have returned
       if constexpr (!PRIVATE_RING) __syncthreads();
-      readOps(nxt, 0, fa[0], fb[0]);
+      readOps(kt + 1, nxt, 0, fa[0], fb[0]);
       issueSlab(kt + STAGES);
       mma(accs[v], fa[(KS - 1) & 1], fb[(KS - 1) & 1]);
     }
@@ -360,15 +370,15 @@ __global__ __launch_bounds__(WGM * WGN * 64 * KSPLIT) void sgemm_dma_kernel(cons
   }
 }
 
-template <int WGM, int WGN, int NI, int KSPLIT, int STAGES, int VSPLIT = 1>
-int launch(hipStream_t stream, SgemmParams p) {
+template <int WGM, int WGN, int NI, int KSPLIT, int STAGES, int VSPLIT, bool RAGGED>
+int launch_form(hipStream_t stream, SgemmParams p) {
   constexpr int GW = WGM * WGN, BM = WGM * 32, BN = WGN * 32 * NI;
   constexpr int STAGE_BYTES = (BM + BN) * BK * 4, UNITS = STAGE_BYTES / 1024;
   constexpr int COPIES = (UNITS + GW - 1) / GW;
   constexpr size_t lds = (size_t)KSPLIT * (STAGES * STAGE_BYTES + (COPIES * GW != UNITS ? 1024 : 0));
   static_assert(lds <= 160 * 1024 && (size_t)(KSPLIT - 1) * BM * BN * sizeof(float) <= lds, "LDS budget");
   if (!sgemm_detail::set_tiles(p, BM, BN)) return set_error(TFCC_ROCM_INVALID_ARGUMENT, "sgemm: too many tiles");
-  auto kern = sgemm_dma_kernel<WGM, WGN, NI, KSPLIT, STAGES, VSPLIT>;
+  auto kern = sgemm_dma_kernel<WGM, WGN, NI, KSPLIT, STAGES, VSPLIT, RAGGED>;
   static bool attrSet[16] = {};  // per device: the attribute belongs to the function on one device
   int dev = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));
@@ -380,6 +390,12 @@ int launch(hipStream_t stream, SgemmParams p) {
   }
   hipLaunchKernelGGL(kern, dim3(p.chunk * 8), dim3(GW * 64 * KSPLIT), lds, stream, p);
   return check_launch("sgemm");
+}
+
+template <int WGM, int WGN, int NI, int KSPLIT, int STAGES, int VSPLIT = 1>
+int launch(hipStream_t stream, const SgemmParams& p) {
+  return p.K % BK != 0 ? launch_form<WGM, WGN, NI, KSPLIT, STAGES, VSPLIT, true>(stream, p)
+                       : launch_form<WGM, WGN, NI, KSPLIT, STAGES, VSPLIT, false>(stream, p);
 }
 
 }  // namespace

@@ -34,7 +34,9 @@
 // The arithmetic is that of sgemm_dma.hip instruction for instruction (k pairs (8kb + s, 8kb + 4 + s) in ascending
 // kb, s; groups added in group order), so a product has the same bits whichever kernel the dispatcher picks for its
 // number of K groups.  Replaces the same oneDNN calls (tfcc/mkl/interfaces/tfcc_mklblasinterface.cpp:41-67, 69-78,
-// 87-118).  Taken for 16-byte aligned operands and strides, K a multiple of 32, B not transposed.
+// 87-118).  Taken for B not transposed.  The copies need addresses that are multiples of four bytes only, and their range
+// check looks at every word, so operands that are not aligned to 16 bytes, rows whose length is no multiple of four and
+// a K that is no multiple of 32 take the RAGGED form of the same loop.
 #include "common.hpp"
 #include "copy_offsets.hpp"
 #include "lds_dma.hpp"
@@ -56,7 +58,7 @@ __device__ __forceinline__ int a_row_swizzle(int row) {
   return BK == 32 ? (row >> 1) & 7 : BK == 16 ? (row >> 2) & 3 : (row >> 2) & 1;
 }
 
-template <int WGM, int KSPLIT, int BK, int STAGES, bool PLAIN, int NI, bool RAMP>
+template <int WGM, int KSPLIT, int BK, int STAGES, bool PLAIN, int NI, bool RAMP, bool RAGGED>
 __global__ __launch_bounds__(64 * WGM * KSPLIT > 256 ? 64 * WGM * KSPLIT : 256) void sgemm_wave96_kernel(
     const float* hotA, const float* hotB, const float* hotB1, const float* hotB2, unsigned hotM, unsigned hotN,
     unsigned hotK, unsigned hotLda, unsigned hotLdb, unsigned hotBatch, const SgemmParams p) {
@@ -153,12 +155,14 @@ __global__ __launch_bounds__(64 * WGM * KSPLIT > 256 ? 64 * WGM * KSPLIT : 256) 
     }
   }
   // ring slab t of this group covers k0(t) .. k0(t) + BK - 1; past the end of K it is all zeros
-  const unsigned slabs32 = K / 32;                                      // the launcher checks K % 32 == 0
+  const unsigned slabs32 = RAGGED ? (K + 31) / 32 : K / 32;             // the launcher checks K % 32 == 0 unless RAGGED
   const unsigned T = ((slabs32 + KSPLIT - 1) / KSPLIT) * SUB;            // ring slabs per group
   auto k0Of = [&](unsigned t) { return ((t / SUB) * KSPLIT + grp) * 32u + (t % SUB) * BK; };
   // Nothing of a copy's set-up runs on the vector unit (a vector instruction between two matrix ops delays the
   // second by some 15 cycles): the lane offsets never change, the slab's k goes into the scalar offset, and a slab
-  // past the end of K is read through a descriptor of size zero, which makes every lane read zeros.
+  // past the end of K is read through a descriptor of size zero, which makes every lane read zeros.  RAGGED: the last
+  // slab of K is a partial one, whose rows of B past K have to fail the range check; so the slab's k goes into the
+  // descriptor (base up, size down: scalar work too), and the lane offset alone is what is checked against what is left.
   auto issueCopy = [&](unsigned t, unsigned stage, int c) {
     const unsigned k0 = k0Of(t);
     const bool live = k0 < K;
@@ -167,8 +171,16 @@ __global__ __launch_bounds__(64 * WGM * KSPLIT > 256 ? 64 * WGM * KSPLIT : 256) 
     const unsigned dst = ldsGroup + stage * STAGE_BYTES + u * 1024;
     const unsigned so = isA ? k0 * 4u : k0 * ldb * 4u;
     w96_v4i rsrc = isA ? rsrcA : rsrcB;
-    rsrc[2] = live ? rsrc[2] : 0;
-    dma16s(rsrc, dst, off[c], live ? so : 0u);
+    if constexpr (RAGGED) {
+      const unsigned long long base = (((unsigned long long)(unsigned)rsrc[1] << 32) | (unsigned)rsrc[0]) + so;
+      rsrc[0] = (int)(unsigned)base;
+      rsrc[1] = (int)(unsigned)(base >> 32);
+      rsrc[2] = live ? rsrc[2] - (int)so : 0;
+      dma16s(rsrc, dst, off[c], 0u);
+    } else {
+      rsrc[2] = live ? rsrc[2] : 0;
+      dma16s(rsrc, dst, off[c], live ? so : 0u);
+    }
   };
 
   // the first slabs are on their way before anything else is set up (RAMP: all but the last stage's, which is asked
@@ -255,8 +267,16 @@ __global__ __launch_bounds__(64 * WGM * KSPLIT > 256 ? 64 * WGM * KSPLIT : 256) 
   // One k step: twelve matrix ops on `cur`; in the issue slots between them the reads of the operands of step
   // (ldStage, ldKb) into `nxt` and, in a slab's last step, the copies of the slab that takes its stage.  fixedStage:
   // ldStage is a constant where the call is written.
-  auto step = [&](const Ops& cur, Ops& nxt, unsigned ldStage, int ldKb, bool fixedStage, bool dma, unsigned dmaSlab,
-                  unsigned dmaStage) __attribute__((always_inline)) {
+  // kEnd: of the four values of A (k ascending) only the first kEnd lie inside K (4 everywhere but at the end of K).
+  auto step = [&](const Ops& full, Ops& nxt, unsigned ldStage, int ldKb, bool fixedStage, bool dma, unsigned dmaSlab,
+                  unsigned dmaStage, bool tail, int kEnd) __attribute__((always_inline)) {
+    Ops cur = full;
+    if (tail) {
+      // past the end of a row of A lies the next one: against the zero rows of B its values would do no harm unless
+      // they are not finite
+#pragma unroll
+      for (int s = 0; s < 4; ++s) cur.a[s] = s < kEnd ? cur.a[s] : 0.f;
+    }
     const unsigned char* st = gsm + ldStage * STAGE_BYTES;
 #pragma unroll
     for (int m = 0; m < 4 * NI; ++m) {
@@ -298,23 +318,28 @@ __global__ __launch_bounds__(64 * WGM * KSPLIT > 256 ? 64 * WGM * KSPLIT : 256) 
     for (int j = 0; j < NI; ++j) ops[0].b[s][j] = *reinterpret_cast<const float*>(gsm + bBase + s * (BN * 4) + j * 128);
   // one ring slab in stage `stage`: KS steps starting on the operands in `first`; the next slab's first operands end
   // up in `first` again when KS is even, in `other` when it is odd (then the loops below alternate the two)
-  auto slab = [&](unsigned t, unsigned stage, bool fixedStage, Ops& first, Ops& other) __attribute__((always_inline)) {
+  auto slab = [&](unsigned t, unsigned stage, bool fixedStage, Ops& first, Ops& other,
+                  bool tail = false) __attribute__((always_inline)) {
     const unsigned next = stage + 1 == STAGES ? 0 : stage + 1;
+    const int left = tail ? (int)K - (int)k0Of(t) - 4 * g : 0;  // values of K from this lane's first one on
 #pragma unroll
     for (int kb = 0; kb < KS - 1; ++kb)
       step(kb & 1 ? other : first, kb & 1 ? first : other, stage, kb + 1, fixedStage, RAMP && kb == 0 && t == 0,
-           (unsigned)(STAGES - 1), (unsigned)(STAGES - 1));
+           (unsigned)(STAGES - 1), (unsigned)(STAGES - 1), tail, left - 8 * kb);
     wait_vmcnt<COPIES*(STAGES - 2)>();
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the reads of slab t have returned
     if constexpr (SHARED) __syncthreads();
-    step((KS - 1) & 1 ? other : first, (KS - 1) & 1 ? first : other, next, 0, fixedStage, true, t + STAGES, stage);
+    step((KS - 1) & 1 ? other : first, (KS - 1) & 1 ? first : other, next, 0, fixedStage, true, t + STAGES, stage,
+         tail, left - 8 * (KS - 1));
   };
   // U slabs per trip with the stages written out (a multiple of the ring depth, even when the operand sets
   // alternate); what is left of T after whole trips runs with the stage counted.  T is a multiple of 32 / BK.
   constexpr int ALT = (KS & 1) ? 2 : 1;
   constexpr int U = STAGES % ALT == 0 ? STAGES : STAGES * ALT;
+  // RAGGED: the last slab of 32 k, in which K may end, runs on its own, with A masked.
+  const unsigned TF = RAGGED ? T - SUB : T;
   unsigned t = 0;
-  for (; t + U <= T; t += U) {
+  for (; t + U <= TF; t += U) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const bool odd = (KS & 1) && (u & 1);
@@ -322,12 +347,23 @@ __global__ __launch_bounds__(64 * WGM * KSPLIT > 256 ? 64 * WGM * KSPLIT : 256) 
     }
   }
   unsigned stage = 0;  // U is a multiple of the ring depth
-  for (; t < T; t += ALT) {
+  for (; t < TF; t += ALT) {
     slab(t, stage, false, ops[0], ops[1]);
     stage = stage + 1 == STAGES ? 0 : stage + 1;
     if constexpr (KS & 1) {
       slab(t + 1, stage, false, ops[1], ops[0]);
       stage = stage + 1 == STAGES ? 0 : stage + 1;
+    }
+  }
+  if constexpr (RAGGED) {
+    static_assert(SUB % ALT == 0, "the operand sets alternate evenly over a slab of 32 k");
+    for (; t < T; t += ALT) {
+      slab(t, stage, false, ops[0], ops[1], true);
+      stage = stage + 1 == STAGES ? 0 : stage + 1;
+      if constexpr (KS & 1) {
+        slab(t + 1, stage, false, ops[1], ops[0], true);
+        stage = stage + 1 == STAGES ? 0 : stage + 1;
+      }
     }
   }
   wait_vmcnt<0>();
@@ -448,16 +484,21 @@ int launch_wave96(hipStream_t stream, SgemmParams p) {
   const bool sameStart = p.batch == 1 || (p.strideA == 0 && p.innerA == 0 && p.strideB == 0 && p.innerB == 0);
   const bool plain = p.groups ? p.groups <= 3 : sameStart;
   TFCC_REQUIRE(p.batch < (1u << 30), "sgemm: batch of %u", p.batch);
-  auto kern = plain ? sgemm_wave96_kernel<WGM, KSPLIT, BK, STAGES, true, NI, RAMP>
-                    : sgemm_wave96_kernel<WGM, KSPLIT, BK, STAGES, false, NI, RAMP>;
-  static bool attrSet[16][2] = {};  // per device: the attribute belongs to the function on one device
+  // a piece of four columns that crosses the end of B's last row passes the range check on the lane offset alone
+  const bool ragged = p.K % 32 != 0 || p.N % 4 != 0;
+  auto kern = plain ? (ragged ? sgemm_wave96_kernel<WGM, KSPLIT, BK, STAGES, true, NI, RAMP, true>
+                              : sgemm_wave96_kernel<WGM, KSPLIT, BK, STAGES, true, NI, RAMP, false>)
+                    : (ragged ? sgemm_wave96_kernel<WGM, KSPLIT, BK, STAGES, false, NI, RAMP, true>
+                              : sgemm_wave96_kernel<WGM, KSPLIT, BK, STAGES, false, NI, RAMP, false>);
+  static bool attrSet[16][4] = {};  // per device: the attribute belongs to the function on one device
   int dev = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));
   TFCC_REQUIRE(dev >= 0 && dev < 16, "device index %d", dev);
-  if (!attrSet[dev][plain]) {
+  const int which = (plain ? 1 : 0) + (ragged ? 2 : 0);
+  if (!attrSet[dev][which]) {
     TFCC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attrSet[dev][plain] = true;
+    attrSet[dev][which] = true;
   }
   const unsigned hotBatch = p.batch | (p.groups ? 1u << 30 : 0u);
   hipLaunchKernelGGL(kern, dim3(p.chunk * 8), dim3(64 * WGM * KSPLIT), lds, stream, p.A, p.groups ? p.groupB[0] : p.B,
