@@ -5,8 +5,8 @@
 // driver), tfcc/mkl/gemm/tfcc_mklsinglethreadgemm.h:93-141 (blocking / packing) and the 24x4x2
 // micro-kernel tfcc/mkl/gemm/tfcc_mklmatmulkernel.h:142-260.
 //
-// Layout.  A is [M,K] uint8 and B is [K,N] int8, both row-major in HBM.  A workgroup of four
-// wavefronts owns a BM x BN tile of C and walks K in slabs of BK bytes:
+// Layout.  A is [M,K] uint8 and B is [K,N] int8, both row-major in HBM, of any size and alignment.  Four wavefronts
+// (or two groups of four, KSPLIT) own a BM x BN tile of C and walk K in slabs of BK bytes:
 //   * A slab: 128-bit global loads (16 consecutive k of one row), xor 0x80 turns the uint8 into
 //     int8 (a' = a - 128), 128-bit LDS stores into As[row][k] with the 16-byte chunks of a row
 //     xor-swizzled by the row index so that both the stores and the matrix-core operand reads are
@@ -31,28 +31,16 @@
 #include "gemv.hpp"
 #include "qgemm_dma.hpp"
 #include "qgemm_params.hpp"
+#include "qgemm_small.hpp"
 
 namespace tfcc_rocm {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
+typedef qgemm_v4i v4i;
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 namespace {
 
 constexpr int kThreads = 256;
-
-// 4x4 byte transpose: in r[q] = bytes (n0..n3) of k-row q; out c[j] = bytes (k0..k3) of column j
-__device__ __forceinline__ void transpose4x4(const unsigned r[4], unsigned c[4]) {
-  // v_perm_b32(hi, lo, sel): selector bytes 0-3 pick from lo, 4-7 from hi
-  unsigned t0 = __builtin_amdgcn_perm(r[1], r[0], 0x05010400u);  // r0.b0 r1.b0 r0.b1 r1.b1
-  unsigned t1 = __builtin_amdgcn_perm(r[1], r[0], 0x07030602u);  // r0.b2 r1.b2 r0.b3 r1.b3
-  unsigned t2 = __builtin_amdgcn_perm(r[3], r[2], 0x05010400u);
-  unsigned t3 = __builtin_amdgcn_perm(r[3], r[2], 0x07030602u);
-  c[0] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);  // t0.lo16 t2.lo16
-  c[1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);  // t0.hi16 t2.hi16
-  c[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
-  c[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
-}
 
 template <int BK>
 __device__ __forceinline__ int swizzled_chunk(int row, int chunk) {
@@ -61,8 +49,10 @@ __device__ __forceinline__ int swizzled_chunk(int row, int chunk) {
   return chunk ^ ((row / RP) & (CH - 1));
 }
 
-template <int BM, int BN, int BK, bool ALIGNED, bool REQUANT>
-__global__ __launch_bounds__(kThreads) void qgemm_kernel(const QGemmParams p) {
+// KSPLIT = 2: two groups of four wavefronts on the same tile, one with the even slabs of K and one with the odd ones,
+// each with LDS buffers of its own; they then exchange halves of their partial sums and finish half the tile each.
+template <int BM, int BN, int BK, int KSPLIT, bool REQUANT>
+__global__ __launch_bounds__(kThreads * KSPLIT) void qgemm_kernel(const QGemmParams p) {
   constexpr int WM = BM / 2, WN = BN / 2;  // wavefront sub-tile
   constexpr int MI = WM / 32, NI = WN / 32;
   constexpr int CH = BK / 16;
@@ -72,10 +62,11 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(const QGemmParams p) {
   static_assert(NI == 4 || NI == 2, "column interleave assumes 2 or 4 blocks per wavefront");
 
   extern __shared__ __align__(16) unsigned char smem[];
-  unsigned char* As = smem;                       // [2][BM][BK]
-  unsigned char* Bs = smem + 2 * BM * BK;         // [2][BN][BK]
+  const int grp = KSPLIT > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads) : 0;
+  unsigned char* As = smem + grp * 2 * (BM + BN) * BK;  // [2][BM][BK]
+  unsigned char* Bs = As + 2 * BM * BK;                 // [2][BN][BK]
 
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x - grp * kThreads;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -111,7 +102,7 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(const QGemmParams p) {
     float mnA = *p.minA, mxA = *p.maxA, mnB = *p.minB, mxB = *p.maxB;
     qmatmul_offsets(mnA, mxA, mnB, mxB, &offA, &offB);
     qmatmul_range(mnA, mxA, mnB, mxB, &minC, &maxC);
-    if (blockIdx.x == 0 && tid == 0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
       if (p.minC) *p.minC = minC;
       if (p.maxC) *p.maxC = maxC;
     }
@@ -125,72 +116,74 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(const QGemmParams p) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
 
-  v4i aReg[A_ITEMS];
-  unsigned bReg[B_ITEMS][16];
+  struct Slab {
+    v4i a[A_ITEMS];
+    unsigned b[B_ITEMS][16];
+  };
+  Slab slab;
   int colsum[4] = {0, 0, 0, 0};  // true column sums of this thread's 4 columns over its k chunks
 
   // ---- global -> registers
-  // In the aligned path every global read is a raw buffer load: an offset past the end of the
-  // operand (rows >= M of A, rows >= K of B) returns zero without a branch.  Bytes of A beyond K
-  // inside a row and columns of B beyond N read neighbouring data; they only ever meet zero
-  // B rows or columns that are never stored.
+  // Every global read is a raw buffer load: an offset past the end of the operand (rows >= M of A, rows >= K of B)
+  // returns zero without a branch.  Bytes of A beyond K inside a row and columns of B beyond N read neighbouring data;
+  // they only ever meet zero B rows or columns that are never stored.  A load may have any byte address; what its range
+  // check cannot do is return the valid bytes of one that crosses the end of the operand.  So every load is moved back
+  // to end inside the operand, and in the slab in which K ends, where that can have changed something, the bytes are
+  // shifted to their places (1344 x 959 x 1948: 20 us against 120 when ragged operands were read byte by byte).
+  const unsigned sizeA = M * K, sizeB = K * N, lastA = sizeA - 16, lastB = sizeB - 4;
   const __amdgpu_buffer_rsrc_t rsrcA =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(A), 0, ALIGNED ? (int)(M * K) : 0, 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(A), 0, (int)sizeA, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrcB =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<signed char*>(B), 0, ALIGNED ? (int)(K * N) : 0, 0x00020000);
-  auto loadA = [&](unsigned k0) {
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<signed char*>(B), 0, (int)sizeB, 0x00020000);
+  auto loadA = [&](unsigned k0, v4i (&aReg)[A_ITEMS]) {
 #pragma unroll
     for (int it = 0; it < A_ITEMS; ++it) {
       const int w = tid + it * kThreads;
       const int row = w / CH, ch = w % CH;
-      const unsigned gr = m0 + row, gk = k0 + ch * 16;
-      v4i v = {0, 0, 0, 0};
-      if constexpr (ALIGNED) {
-        v = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrcA, gr * K + gk, 0, 0));
-      } else {
-        if (gr < M) {
-          unsigned char tmp[16];
+      const unsigned at = (m0 + row) * K + k0 + ch * 16;
+      aReg[it] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrcA, min(at, lastA), 0, 0));
+    }
+    if (k0 + BK >= K) {
+      asm volatile("" ::: "memory");  // a real (wave-uniform) branch: the wait for the loads stays inside
 #pragma unroll
-          for (int q = 0; q < 16; ++q) tmp[q] = (gk + q < K) ? A[(size_t)gr * K + gk + q] : 0;
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            v[q] = (int)(tmp[4 * q] | (tmp[4 * q + 1] << 8) | (tmp[4 * q + 2] << 16) | ((unsigned)tmp[4 * q + 3] << 24));
-        }
+      for (int it = 0; it < A_ITEMS; ++it) {
+        const int w = tid + it * kThreads;
+        const unsigned at = (m0 + w / CH) * K + k0 + (w % CH) * 16;
+        aReg[it] = moved16(aReg[it], max(at, lastA) - lastA);
       }
-      aReg[it] = v;
     }
   };
-  auto loadB = [&](unsigned k0) {
+  auto loadB = [&](unsigned k0, unsigned (&bReg)[B_ITEMS][16]) {
 #pragma unroll
     for (int it = 0; it < B_ITEMS; ++it) {
       const int w = tid + it * kThreads;
       const int nd = w % (BN / 4), ch = w / (BN / 4);
-      const unsigned gn = n0 + nd * 4, gk = k0 + ch * 16;
+      const unsigned at = (k0 + ch * 16) * N + n0 + nd * 4;
 #pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        unsigned v = 0;
-        if constexpr (ALIGNED) {
-          v = __builtin_amdgcn_raw_buffer_load_b32(rsrcB, (gk + q) * N + gn, 0, 0);
-        } else {
-          if (gk + q < K) {
+      for (int q = 0; q < 16; ++q)
+        bReg[it][q] = __builtin_amdgcn_raw_buffer_load_b32(rsrcB, min(at + q * N, lastB), 0, 0);
+    }
+    if (k0 + BK >= K) {
+      asm volatile("" ::: "memory");
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (gn + e < N) v |= (unsigned)(unsigned char)B[(size_t)(gk + q) * N + gn + e] << (8 * e);
-          }
-        }
-        bReg[it][q] = v;
+      for (int it = 0; it < B_ITEMS; ++it) {
+        const int w = tid + it * kThreads;
+        unsigned at = (k0 + w / (BN / 4) * 16) * N + n0 + w % (BN / 4) * 4;
+        asm volatile("" : "+v"(at));  // worked out again, instead of keeping every load's offset in a register
+#pragma unroll
+        for (int q = 0; q < 16; ++q) bReg[it][q] = moved4(bReg[it][q], max(at + q * N, lastB) - lastB);
       }
     }
   };
   // ---- registers -> LDS (A: uint8 -> int8; B: transpose, column interleave, column sums)
-  auto storeTiles = [&](int buf) {
+  auto storeTiles = [&](int buf, const Slab& slab) {
     unsigned char* as = As + buf * BM * BK;
     unsigned char* bs = Bs + buf * BN * BK;
 #pragma unroll
     for (int it = 0; it < A_ITEMS; ++it) {
       const int w = tid + it * kThreads;
       const int row = w / CH, ch = w % CH;
-      v4i v = aReg[it] ^ (int)0x80808080;
+      v4i v = slab.a[it] ^ (int)0x80808080;
       *reinterpret_cast<v4i*>(as + row * BK + swizzled_chunk<BK>(row, ch) * 16) = v;
     }
 #pragma unroll
@@ -201,7 +194,7 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(const QGemmParams p) {
 #pragma unroll
       for (int kq = 0; kq < 4; ++kq) {
         unsigned c4[4];
-        transpose4x4(&bReg[it][4 * kq], c4);
+        transpose4x4(&slab.b[it][4 * kq], c4);
 #pragma unroll
         for (int j = 0; j < 4; ++j) col[j][kq] = c4[j];
       }
@@ -220,19 +213,20 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(const QGemmParams p) {
     }
   };
 
-  const unsigned KT = (K + BK - 1) / BK;
-  loadA(0);
-  loadB(0);
-  storeTiles(0);
+  // every group makes the same number of steps (the barriers are workgroup-wide); a slab past the end of K is zeros
+  const unsigned KT = ((K + BK - 1) / BK + KSPLIT - 1) / KSPLIT;
+  auto load = [&](unsigned kt) __attribute__((always_inline)) {
+    loadA((kt * KSPLIT + grp) * BK, slab.a);
+    loadB((kt * KSPLIT + grp) * BK, slab.b);
+  };
+  load(0);
+  storeTiles(0, slab);
   __syncthreads();
 
   const int lrow = lane & 31, khalf = lane >> 5;
   for (unsigned kt = 0; kt < KT; ++kt) {
     const int buf = kt & 1;
-    if (kt + 1 < KT) {
-      loadA((kt + 1) * BK);
-      loadB((kt + 1) * BK);
-    }
+    if (kt + 1 < KT) load(kt + 1);
     const unsigned char* as = As + buf * BM * BK + (wm * WM) * BK;
     const unsigned char* bs = Bs + buf * BN * BK + (wn * WN) * BK;
 #pragma unroll
@@ -254,15 +248,38 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(const QGemmParams p) {
         for (int j = 0; j < NI; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], acc[i][j], 0, 0, 0);
     }
-    if (kt + 1 < KT) storeTiles(buf ^ 1);
+    if (kt + 1 < KT) storeTiles(buf ^ 1, slab);
     __syncthreads();
   }
 
   // ---- epilogue.  LDS is free now: reuse it for the per-tile row / column terms.
   int* colTerm = reinterpret_cast<int*>(smem);            // [BN]  indexed by tile column
   int* rowTerm = colTerm + BN;                             // [BM]
-  for (int i = tid; i < BN; i += kThreads) colTerm[i] = 0;
-  __syncthreads();
+  for (int i = threadIdx.x; i < BN; i += kThreads * KSPLIT) colTerm[i] = 0;
+  if constexpr (KSPLIT > 1) {
+    // registers 0-7 of every block are finished by group 0, registers 8-15 by group 1
+    int* give = rowTerm + BM + (grp * 4 + wave) * (MI * NI * 8 * 64);
+    const int* take = rowTerm + BM + ((grp ^ 1) * 4 + wave) * (MI * NI * 8 * 64);
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) give[((i * NI + j) * 8 + r) * 64 + lane] = grp == 0 ? acc[i][j][8 + r] : acc[i][j][r];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          const unsigned other = (unsigned)take[((i * NI + j) * 8 + r) * 64 + lane];
+          // the group's eight registers move to the front, whichever they were
+          acc[i][j][r] = (int)((grp == 0 ? (unsigned)acc[i][j][r] : (unsigned)acc[i][j][8 + r]) + other);
+        }
+  } else {
+    __syncthreads();
+  }
   {
     // every thread owned the same 4 columns in every slab: nd = tid % (BN/4) (+ it*256 % (BN/4) = 0)
     const int nd = tid % (BN / 4);
@@ -273,12 +290,12 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(const QGemmParams p) {
   const int* __restrict__ rsA = p.rowsumA + (size_t)bi * p.strideRA;
   const int* __restrict__ csB = p.colsumB + (size_t)bi * p.strideRB;
   const unsigned global = (unsigned)offA * (unsigned)offB * K;
-  for (int i = tid; i < BN; i += kThreads) {
+  for (int i = threadIdx.x; i < BN; i += kThreads * KSPLIT) {
     unsigned gn = n0 + i;
     unsigned cs = gn < N ? (unsigned)csB[gn] : 0u;
     colTerm[i] = (int)(128u * (unsigned)colTerm[i] + cs * (unsigned)offA);
   }
-  for (int i = tid; i < BM; i += kThreads) {
+  for (int i = threadIdx.x; i < BM; i += kThreads * KSPLIT) {
     unsigned gm = m0 + i;
     unsigned rs = gm < M ? (unsigned)rsA[gm] : 0u;
     rowTerm[i] = (int)(global + rs * (unsigned)offB);
@@ -303,7 +320,7 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(const QGemmParams p) {
   int ct[NI];
 #pragma unroll
   for (int j = 0; j < NI; ++j) ct[j] = colTerm[colBase + j];
-  const bool vecOK = ALIGNED && (gcol + NI <= N);     // N % 4 == 0 and base pointers aligned when ALIGNED
+  const bool vecOK = p.vectorStores && gcol + NI <= N;
 
   // FLAVOUR 0: int32 only; 1: requantize, double shortcut; 2: exact int64 path; 3: constant fill; 4: int32 shortcut
   auto storeTile = [&](auto flavour) {
@@ -311,8 +328,8 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(const QGemmParams p) {
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int trow = wm * WM + i * 32 + 8 * (r / 4) + 4 * khalf + (r & 3);
+      for (int r = 0; r < 16 / KSPLIT; ++r) {
+        const int trow = wm * WM + i * 32 + (KSPLIT > 1 ? 16 * grp : 0) + 8 * (r / 4) + 4 * khalf + (r & 3);
         const unsigned grow = m0 + trow;
         if (grow >= M) continue;
         const int rt = rowTerm[trow];
@@ -366,7 +383,7 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(const QGemmParams p) {
   }
 }
 
-template <int BM, int BN, int BK, bool ALIGNED, bool REQUANT>
+template <int BM, int BN, int BK, int KSPLIT, bool REQUANT>
 int launch(hipStream_t stream, QGemmParams p) {
   p.tilesM = (p.M + BM - 1) / BM;
   p.tilesN = (p.N + BN - 1) / BN;
@@ -374,9 +391,11 @@ int launch(hipStream_t stream, QGemmParams p) {
   if (total > 0x7fffffffull) return set_error(TFCC_ROCM_INVALID_ARGUMENT, "quantized matmul: too many tiles");
   p.tilesTotal = (unsigned)total;
   p.chunk = (p.tilesTotal + 7) / 8;
-  constexpr size_t lds = 2 * (size_t)(BM + BN) * BK;
-  static_assert(lds >= (size_t)(BM + BN) * 4, "epilogue terms must fit in the slab buffers");
-  auto kern = qgemm_kernel<BM, BN, BK, ALIGNED, REQUANT>;
+  p.vectorStores = p.N % 4 == 0 && p.strideC % 4 == 0 && (uintptr_t)p.C % 16 == 0 && (uintptr_t)p.Q % 4 == 0;
+  constexpr size_t lds = KSPLIT * 2 * (size_t)(BM + BN) * BK;
+  static_assert(lds <= 160 * 1024 && lds >= (size_t)(BM + BN) * 4 + (KSPLIT > 1 ? (size_t)BM * BN * 4 : 0),
+                "epilogue terms and exchanged sums must fit in the slab buffers");
+  auto kern = qgemm_kernel<BM, BN, BK, KSPLIT, REQUANT>;
   static bool attrSet[16] = {};  // per device: the attribute belongs to the function on one device
   int dev = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));
@@ -386,24 +405,30 @@ int launch(hipStream_t stream, QGemmParams p) {
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attrSet[dev] = true;
   }
-  hipLaunchKernelGGL(kern, dim3(p.chunk * 8), dim3(kThreads), lds, stream, p);
+  hipLaunchKernelGGL(kern, dim3(p.chunk * 8), dim3(kThreads * KSPLIT), lds, stream, p);
   return check_launch("quantized matmul");
 }
 
+// Where the lines lie (us; "slabs" are the kernels of this file, t64 the number of 64 x 128 tiles):
+//   t64 <= 64, or at most 32 rows: the kernel without slabs (gemm_u8s8_small.hip), aligned or not - 256 x 1024 x 1024 6.2
+//     against 8.1 in direct-to-LDS slabs, 64 x 4096 x 4096 15.5 against 23.6, 256 x 1023 x 1025 10.1 against 12.4 in
+//     slabs; past it 512 x 1023 x 1025 17.2 against 12.6, 640 x 1024 x 1024 9.9 against 8.3;
+//   then the direct-to-LDS kernels for what they take (K and N multiples of 16), slabs for the rest:
+//   t64 <= 256: 64 x 128 tiles, two K groups (2048 x 3001 x 1001: 27 against 33 with one);
+//   128 x 128 tiles <= 256: those with two K groups (2000 x 2000 x 2001: 24.8 against 28.2 and 31.0);
+//   above, as many tiles as possible - 64 x 128 (3001 x 2001 x 3001: 61 against 67) - until 128 x 128 tiles fill the CUs
+//     three times over (4000 x 1000 x 4001: 48 against 57).
+//   A K of at most 256, two slabs, is not split (2000 x 64 x 2001: 8.8 against 10.7).
 template <bool REQUANT>
 int dispatch(hipStream_t stream, const QGemmParams& p) {
+  const unsigned long long t64 = (unsigned long long)((p.M + 63) / 64) * ((p.N + 127) / 128) * p.batch;
+  const unsigned long long t128 = (unsigned long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
+  const bool loads = (unsigned long long)p.M * p.K >= 16 && (unsigned long long)p.K * p.N >= 4;  // operands as long as one load
+  if (!loads || ((t64 <= 64 || p.M <= 32) && qgemm_small_supported(p))) return qgemm_small_launch(stream, p, QSmallOutputs{});
   if (qgemm_dma_supported(p, REQUANT)) return qgemm_dma_launch(stream, p, REQUANT);
-  const bool aligned = (p.K % 16 == 0) && (p.N % 4 == 0) && ((uintptr_t)p.A % 16 == 0) &&
-                       ((uintptr_t)p.B % 4 == 0) && (p.strideA % 16 == 0) && (p.strideB % 4 == 0) &&
-                       (p.C == nullptr || ((uintptr_t)p.C % 16 == 0 && p.strideC % 4 == 0)) &&
-                       (!REQUANT || ((uintptr_t)p.Q % 4 == 0 && p.strideC % 4 == 0));
-  // big tiles once they fill the 256 CUs reasonably; otherwise 128x128
-  const unsigned long long big = (unsigned long long)((p.M + 255) / 256) * ((p.N + 255) / 256) * p.batch;
-  if (aligned) {
-    if (big >= 192) return launch<256, 256, 64, true, REQUANT>(stream, p);
-    return launch<128, 128, 128, true, REQUANT>(stream, p);
-  }
-  return launch<128, 128, 128, false, REQUANT>(stream, p);
+  if (p.K > 256 && t64 <= 256) return launch<64, 128, 128, 2, REQUANT>(stream, p);
+  if (p.K > 256 && t128 <= 256) return launch<128, 128, 128, 2, REQUANT>(stream, p);
+  return t128 >= 768 ? launch<128, 128, 128, 1, REQUANT>(stream, p) : launch<64, 128, 128, 1, REQUANT>(stream, p);
 }
 
 int fill_params(const tfcc_rocm_qgemm_desc* d, QGemmParams& p) {

@@ -1,0 +1,295 @@
+// uint8 x int8 -> int32 products that are too small, too short or too ragged for the kernels with a pipeline of slabs:
+// every byte is asked for at once and the wait for memory is paid about once.
+//
+// A product of 77 x 1001 x 1237 is 200 million operations and 1.3 MB: 0.1 us of matrix time and 0.3 us of traffic.  What
+// it costs is latency, and a kernel that walks K slab by slab through LDS pays a trip to memory per slab (84 us in 128 x
+// 128 tiles).  Here a workgroup owns BM x 64 outputs and its wavefronts deal the steps of 64 k among themselves; a
+// wavefront has two steps in flight and nothing goes through LDS on the way in: the operand of A is 16 consecutive k of a
+// row, loaded as it lies, and a lane turns its 16(k) x 4(n) bytes of B into operand order with byte permutes.  The
+// partial tiles are added in LDS (integer adds: any order gives the same sum) and every thread finishes four columns.
+//
+// Any K, N and alignment: buffer loads take any byte address, and those that would cross the end of an operand are moved
+// back to end with it.  Arithmetic and epilogue
+// are those of gemm_u8s8.hip (tfcc/mkl/operations/tfcc_mklquantization.cpp:33-69,176-201).
+#include "common.hpp"
+#include "gemv.hpp"
+#include "qgemm_params.hpp"
+#include "qgemm_small.hpp"
+
+namespace tfcc_rocm {
+
+typedef qgemm_v4i v4i;
+
+namespace {
+
+constexpr int kCols = 64;    // columns of a tile
+constexpr int kPitch = 68;   // words per tile row in LDS: the four row groups of a store fall on different banks
+
+// The requantize scalars of the launch; the values themselves where the ranges lie in device memory.
+__device__ __forceinline__ RequantScalars requant_scalars(const QGemmParams& p, float minC, float maxC) {
+  if (p.minOut) return make_requant_scalars(TFCC_ROCM_S32, TFCC_ROCM_U8, minC, maxC, *p.minOut, *p.maxOut);
+  RequantScalars rq;
+  rq.inScale = p.inScale; rq.inMin = p.inMin; rq.outScale = p.outScale; rq.outOffset = p.outOffset;
+  rq.inLowest = -2147483648LL; rq.outLowest = 0; rq.outHighest = 255; rq.mode = 0; rq.fillValue = 0;
+  finish_requant_scalars(rq, 4294967295.0);
+  return rq;
+}
+__device__ __forceinline__ void offsets_and_range(const QGemmParams& p, bool store, int& oA, int& oB, float& minC, float& maxC) {
+  oA = p.offsetA;
+  oB = p.offsetB;
+  minC = maxC = 0.f;
+  if (!p.minA) return;
+  const float mnA = *p.minA, mxA = *p.maxA, mnB = *p.minB, mxB = *p.maxB;
+  qmatmul_offsets(mnA, mxA, mnB, mxB, &oA, &oB);
+  qmatmul_range(mnA, mxA, mnB, mxB, &minC, &maxC);
+  if (store) {
+    if (p.minC) *p.minC = minC;
+    if (p.maxC) *p.maxC = maxC;
+  }
+}
+__device__ __forceinline__ unsigned requantized(int v, const RequantScalars& rq) {
+  const double off = (double)((unsigned)v ^ 0x80000000u);  // v - INT32_MIN
+  if (rq.mode) return (unsigned)rq.fillValue;
+  if (rq.fast32OK) return (unsigned)requantize_one_fast32(off, rq);
+  if (rq.fastOK) return (unsigned)requantize_one_fast(off, rq);
+  return (unsigned)requantize_one_exact((long long)v, rq);
+}
+
+// Operands shorter than one load (A below 16 bytes or B below 4, so K below 16): a thread per result.
+__global__ __launch_bounds__(256) void qgemm_tiny_kernel(const QGemmParams p, const QSmallOutputs o, unsigned long long total) {
+  const unsigned long long i = (unsigned long long)blockIdx.x * 256 + threadIdx.x;
+  int oA, oB;
+  float minC, maxC;
+  offsets_and_range(p, i == 0, oA, oB, minC, maxC);
+  if (i >= total) return;
+  const unsigned n = (unsigned)(i % p.N), m = (unsigned)(i / p.N % p.M), bi = (unsigned)(i / p.N / p.M);
+  const unsigned char* A = p.A + (size_t)bi * p.strideA + (size_t)m * p.K;
+  const signed char* B = p.B + (size_t)bi * p.strideB + n;
+  unsigned sum = 0;
+  for (unsigned k = 0; k < p.K; ++k) sum += (unsigned)((int)A[k] * (int)B[(size_t)k * p.N]);
+  sum += (unsigned)oA * (unsigned)oB * p.K + (unsigned)p.rowsumA[(size_t)bi * p.strideRA + m] * (unsigned)oB +
+         (unsigned)p.colsumB[(size_t)bi * p.strideRB + n] * (unsigned)oA;
+  const size_t at = (size_t)bi * p.strideC + (size_t)m * p.N + n;
+  if (p.C) p.C[at] = (int)sum;
+  if (o.f32Out) o.f32Out[at] = (float)((double)(int)sum * ((double)o.scaleA * (double)o.scaleB[n]));
+  if (p.Q) p.Q[at] = (unsigned char)requantized((int)sum, requant_scalars(p, minC, maxC));
+}
+
+template <int BM, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmParams p, const QSmallOutputs o) {
+  constexpr int kThreads = WAVES * 64, RB = BM / 16, WORKERS = WAVES - 1;
+  __shared__ int tile[BM * kPitch];
+  __shared__ int sums[kCols];
+  __shared__ struct { RequantScalars rq; int offsetA, offsetB; } shared;
+  const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, kg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  for (int i = tid; i < BM * kPitch; i += kThreads) tile[i] = 0;
+  if (tid < kCols) sums[tid] = 0;
+
+  unsigned tm, tn, bi;
+  {
+    // each XCD a contiguous run of tiles, the tiles of one column block next to each other: B is the larger operand
+    const unsigned xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
+    const unsigned L = xcd * p.chunk + slot;
+    if (slot >= p.chunk || L >= p.tilesTotal) return;
+    bi = udiv_apply(L, p.perBatchMagic, p.perBatchShift);
+    const unsigned t = L - bi * (p.tilesM * p.tilesN);
+    tn = udiv_apply(t, p.bandMagic, p.bandShift);  // here: division by tilesM
+    tm = t - tn * p.tilesM;
+  }
+  const unsigned m0 = tm * BM, n0 = tn * kCols;
+  const unsigned M = p.M, N = p.N, K = p.K;
+  const unsigned sizeA = M * K, sizeB = K * N;
+  const __amdgpu_buffer_rsrc_t rsrcA = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<unsigned char*>(p.A + (size_t)bi * p.strideA), 0, (int)sizeA, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrcB = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<signed char*>(p.B + (size_t)bi * p.strideB), 0, (int)sizeB, 0x00020000);
+  __syncthreads();  // the tile is clear; passed before the loads are asked for, whose return it would wait for
+
+  // What the finish needs besides the sums.  The requantize scalars are a few hundred double operations: the last
+  // wavefront works them out for all while the operands travel, and does nothing else (next to loads in flight they
+  // would cost every wavefront the registers for both).
+  auto prepare = [&]() __attribute__((always_inline)) {
+    int oA, oB;
+    float minC, maxC;
+    offsets_and_range(p, blockIdx.x == 0 && lane == 0, oA, oB, minC, maxC);
+    if (lane == 0) {
+      shared.offsetA = oA;
+      shared.offsetB = oB;
+    }
+    if (p.Q) {
+      const RequantScalars rq = requant_scalars(p, minC, maxC);
+      if (lane == 0) shared.rq = rq;
+    }
+  };
+
+  const unsigned steps = (K + 63) / 64;
+  const unsigned offA = (m0 + j) * K + kg * 16, offB = kg * 16 * N + n0 + j * 4;
+  v4i acc[RB][4];
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[i][e] = v4i{0, 0, 0, 0};
+  int colsum[4] = {0, 0, 0, 0};
+
+  // Every load is moved back far enough to end inside its operand.  That changes the bytes only of what crosses the end
+  // or lies behind it, which happens in the step in which K ends (and in the one behind it that evens out a pair): those
+  // are put right there.  (Rows of A past M and columns of B past N hold whatever they hold: they are not stored.)
+  const unsigned lastA = sizeA - 16, lastB = sizeB - 4;
+  if (wave == WORKERS) prepare();
+  else for (unsigned s = wave; s < steps; s += 2 * WORKERS) {
+    v4i a[2][RB];
+    unsigned b[2][16];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const unsigned ka = offA + (s + u * WORKERS) * 64, kb = offB + (s + u * WORKERS) * 64 * N;
+#pragma unroll
+      for (int q = 0; q < 16; ++q) b[u][q] = __builtin_amdgcn_raw_buffer_load_b32(rsrcB, min(kb + q * N, lastB), 0, 0);
+#pragma unroll
+      for (int i = 0; i < RB; ++i)
+        a[u][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrcA, min(ka + i * 16 * K, lastA), 0, 0));
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const unsigned step = s + u * WORKERS;
+      if (step + 1 >= steps) {
+        unsigned ka = offA + step * 64, kb = offB + step * 64 * N;
+        asm volatile("" : "+v"(ka), "+v"(kb));  // worked out again, instead of keeping every load's offset in a register
+#pragma unroll
+        for (int q = 0; q < 16; ++q) b[u][q] = moved4(b[u][q], max(kb + q * N, lastB) - lastB);
+#pragma unroll
+        for (int i = 0; i < RB; ++i) a[u][i] = moved16(a[u][i], max(ka + i * 16 * K, lastA) - lastA);
+      }
+      unsigned col[4][4];  // [column][k quad]
+#pragma unroll
+      for (int kq = 0; kq < 4; ++kq) {
+        unsigned c4[4];
+        transpose4x4(&b[u][4 * kq], c4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) col[e][kq] = c4[e];
+      }
+#pragma unroll
+      for (int i = 0; i < RB; ++i) a[u][i] = a[u][i] ^ (int)0x80808080;  // a' = a - 128
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const v4i bv = {(int)col[e][0], (int)col[e][1], (int)col[e][2], (int)col[e][3]};
+#pragma unroll
+        for (int i = 0; i < RB; ++i) acc[i][e] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[u][i], bv, acc[i][e], 0, 0, 0);
+        if (!p.colsumExact) {
+#pragma unroll
+          for (int kq = 0; kq < 4; ++kq) colsum[e] = __builtin_amdgcn_sdot4((int)col[e][kq], 0x01010101, colsum[e], false);
+        }
+      }
+    }
+  }
+
+  // lane (j, kg) holds rows 16 i + 4 kg + r of column 4 j + e; column 4 j + e lies at word e * 16 + j of its tile row
+  if (wave < (int)min(steps, (unsigned)WORKERS)) {
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) atomicAdd(&tile[(16 * i + 4 * kg + r) * kPitch + e * 16 + j], acc[i][e][r]);
+    if (!p.colsumExact) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) atomicAdd(&sums[e * 16 + j], colsum[e]);
+    }
+  }
+  __syncthreads();
+
+  const unsigned offsetA = (unsigned)shared.offsetA, offsetB = (unsigned)shared.offsetB, global = offsetA * offsetB * K;
+  const int* __restrict__ rowsumA = p.rowsumA + (size_t)bi * p.strideRA;
+  const int* __restrict__ colsumB = p.colsumB + (size_t)bi * p.strideRB;
+  for (int idx = tid; idx < BM * 16; idx += kThreads) {
+    const int row = idx >> 4, c = idx & 15;
+    const unsigned grow = m0 + row, gcol = n0 + 4 * c;
+    if (grow >= M || gcol >= N) continue;
+    const unsigned rt = global + (unsigned)rowsumA[grow] * offsetB;
+    const size_t at = (size_t)bi * p.strideC + (size_t)grow * N + gcol;
+    const unsigned left = N - gcol;
+    int v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const unsigned cs = e < (int)left ? (unsigned)colsumB[gcol + e] : 0u;
+      const unsigned own = p.colsumExact ? cs : (unsigned)sums[e * 16 + c];
+      v[e] = (int)((unsigned)tile[row * kPitch + e * 16 + c] + 128u * own + cs * offsetA + rt);
+    }
+    const bool four = left >= 4 && p.vectorStores;
+    if (p.C) {
+      if (four) *reinterpret_cast<v4i*>(p.C + at) = v4i{v[0], v[1], v[2], v[3]};
+      else
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (e < (int)left) p.C[at + e] = v[e];
+    }
+    if (o.f32Out) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e < (int)left) o.f32Out[at + e] = (float)((double)v[e] * ((double)o.scaleA * (double)o.scaleB[gcol + e]));
+    }
+    if (p.Q) {
+      const RequantScalars& rq = shared.rq;
+      unsigned q[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) q[e] = requantized(v[e], rq);
+      if (four) *reinterpret_cast<unsigned*>(p.Q + at) = q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24);
+      else
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (e < (int)left) p.Q[at + e] = (unsigned char)q[e];
+    }
+  }
+}
+
+template <int BM, int WAVES>
+int launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o) {
+  p.tilesM = (p.M + BM - 1) / BM;
+  p.tilesN = (p.N + kCols - 1) / kCols;
+  const unsigned long long total = (unsigned long long)p.tilesM * p.tilesN * p.batch;
+  if (total > 0x7fffffffull) return set_error(TFCC_ROCM_INVALID_ARGUMENT, "quantized matmul: too many tiles");
+  p.tilesTotal = (unsigned)total;
+  p.chunk = (p.tilesTotal + 7) / 8;
+  const UDiv perBatch = udiv_prepare(p.tilesM * p.tilesN), rows = udiv_prepare(p.tilesM);
+  p.perBatchMagic = perBatch.magic; p.perBatchShift = perBatch.shift;
+  p.bandMagic = rows.magic; p.bandShift = rows.shift;
+  hipLaunchKernelGGL((qgemm_small_kernel<BM, WAVES>), dim3(p.chunk * 8), dim3(WAVES * 64), 0, stream, p, o);
+  return check_launch("quantized matmul (small)");
+}
+
+}  // namespace
+
+bool qgemm_small_supported(const QGemmParams& p) {
+  return ((unsigned long long)p.M + 64) * p.K + 4096 < (1ull << 31) && ((unsigned long long)p.K + 4160) * p.N + 4096 < (1ull << 31);
+}
+
+// Rows per tile and wavefronts by the amount of work, in steps of 16 rows x 64 columns x 64 k (measured, us):
+//   up to 4096 steps, or at most 16 rows, tiles of 16 rows: there latency is all there is, and the most workgroups share
+//     it (77 x 1001 x 1237: 7.1 in 16 rows, 8.2 in 32, 11.3 in 64);
+//   from there tiles of 32 rows, which load half as much of B per product (128 x 768 x 3072: 6.3 against 6.9);
+//   above 12000 steps tiles of 64 rows while there are 128 of them (700 x 2001 x 803: 18.6 against 21.2 and 22.7; 100 x
+//     4001 x 4003, 126 tiles: 34 against 22 in 32 rows).
+// Wavefronts: 4 for at most six steps of k, or when 8 of each tile would be more than eight per CU (1024 x 768 x 768 in 32
+// rows: 8.1 with 4, 10.8 with 8); 16 on the smallest tiles when they are few and K is long (32 x 3292 x 704: 8.4 against
+// 8.7 and 10.7 with 8 and 4); 8 otherwise.
+int qgemm_small_launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o) {
+  if ((unsigned long long)p.M * p.K < 16 || (unsigned long long)p.K * p.N < 4) {
+    const unsigned long long total = (unsigned long long)p.M * p.N * p.batch;
+    if ((total + 255) / 256 > 0x7fffffffull) return set_error(TFCC_ROCM_INVALID_ARGUMENT, "quantized matmul: too many results");
+    hipLaunchKernelGGL(qgemm_tiny_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, p, o, total);
+    return check_launch("quantized matmul (tiny)");
+  }
+  p.vectorStores = p.N % 4 == 0 && p.strideC % 4 == 0 && (uintptr_t)p.C % 16 == 0 && (uintptr_t)p.Q % 4 == 0;
+  const unsigned steps = (p.K + 63) / 64;
+  const unsigned long long columns = (unsigned long long)((p.N + 63) / 64) * p.batch;
+  const unsigned long long tiles16 = (p.M + 15) / 16 * columns, tiles32 = (p.M + 31) / 32 * columns, tiles64 = (p.M + 63) / 64 * columns;
+  const unsigned long long work = tiles16 * steps;
+  if (work > 12000 && tiles64 >= 128) return steps <= 6 ? launch<64, 4>(stream, p, o) : launch<64, 8>(stream, p, o);
+  if (work > 4096 && p.M > 16)
+    return steps <= 6 || tiles32 * 8 > 2048 ? launch<32, 4>(stream, p, o) : launch<32, 8>(stream, p, o);
+  if (steps <= 6 || tiles16 * 8 > 2048) return launch<16, 4>(stream, p, o);
+  return tiles16 <= 128 && steps >= 30 ? launch<16, 16>(stream, p, o) : launch<16, 8>(stream, p, o);
+}
+
+}  // namespace tfcc_rocm

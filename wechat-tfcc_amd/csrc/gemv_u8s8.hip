@@ -18,10 +18,11 @@
 
 #include "common.hpp"
 #include "gemv.hpp"
+#include "qgemm_small.hpp"
 
 namespace tfcc_rocm {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
+typedef qgemm_v4i v4i;
 
 namespace {
 
@@ -47,17 +48,6 @@ struct GemvParams {
   unsigned M, N, K;
   unsigned colGroups, groupsPerXcd;
 };
-
-__device__ __forceinline__ void transpose4x4(const unsigned r[4], unsigned c[4]) {
-  unsigned t0 = __builtin_amdgcn_perm(r[1], r[0], 0x05010400u);
-  unsigned t1 = __builtin_amdgcn_perm(r[1], r[0], 0x07030602u);
-  unsigned t2 = __builtin_amdgcn_perm(r[3], r[2], 0x05010400u);
-  unsigned t3 = __builtin_amdgcn_perm(r[3], r[2], 0x07030602u);
-  c[0] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
-  c[1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
-  c[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
-  c[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
-}
 
 __global__ __launch_bounds__(kThreads) void gemv_kernel(const GemvParams p) {
   __shared__ int red[kWaves][kPartRows][kCols];
@@ -393,8 +383,17 @@ extern "C" int tfcc_rocm_gemv_u8s8s32_flags(void* stream, const uint8_t* a, cons
   if (gemv_supported(a, b, m, n, k))
     return gemv_launch(s, a, reinterpret_cast<const signed char*>(b), rowsum_a, colsum_b, offset_a,
                        offset_b, nullptr, nullptr, m, n, k, acc_out, scale_a, scale_b, f32_out, colsumExact);
-  // shapes the skinny kernel does not take (m > 8, unaligned): general kernel, then dequantize
-  TFCC_REQUIRE(acc_out != nullptr, "skinny quantized matmul: this shape needs acc_out (m > 8 or unaligned operands)");
+  // ragged shapes and alignments: the kernel for small products of any alignment finishes the floats itself
+  if (m <= (unsigned)kMaxM) {
+    QGemmParams q{};
+    q.A = a; q.B = reinterpret_cast<const signed char*>(b); q.rowsumA = rowsum_a; q.colsumB = colsum_b; q.C = acc_out;
+    q.strideC = (uint64_t)m * n;
+    q.M = m; q.N = n; q.K = k; q.batch = 1;
+    q.offsetA = offset_a; q.offsetB = offset_b; q.colsumExact = colsumExact ? 1 : 0;
+    if (qgemm_small_supported(q)) return qgemm_small_launch(s, q, QSmallOutputs{f32_out, scale_b, scale_a});
+  }
+  // more than eight rows: general kernel, then dequantize
+  TFCC_REQUIRE(acc_out != nullptr, "skinny quantized matmul: this shape needs acc_out (m > 8)");
   tfcc_rocm_qgemm_desc d{};
   d.a = a; d.b = b; d.rowsum_a = rowsum_a; d.colsum_b = colsum_b;
   d.m = m; d.n = n; d.k = k; d.batch = 1; d.stride_c = (uint64_t)m * n;

@@ -30,6 +30,7 @@ struct QGemmParams {
   int rqOffsetMinusLowest32, rqFastOK, rqFast32OK, rqFoldedOK, rqBiasedOK;
   // division by tilesM * tilesN and by 4 * tilesN as multiply-high and shift (filled by launchers whose kernel uses them)
   unsigned perBatchMagic, perBatchShift, bandMagic, bandShift;
+  int vectorStores;  // rows of C and Q start at multiples of four elements of theirs (filled by launchers of ragged products)
 };
 
 // x / d for any 32-bit x as (mulhi(x, magic) + x) >> shift, evaluated without overflow; shift 0 stands for d == 1.
