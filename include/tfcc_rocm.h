@@ -440,6 +440,25 @@ int tfcc_rocm_transpose_f32(void* stream, const float* in, const unsigned* shape
 int tfcc_rocm_lstm_cell_f32(void* stream, unsigned batch, unsigned units, const float* state_c,
                             const float* input_value, const float* state_h_value, const float* bias, float forget,
                             float* h, float* cs);
+/* A whole LSTM sequence (directions = 1), or both directions of a bidirectional one, in one go: the loop of
+ * tfcc/core/operations/tfcc_rnn.cpp:29-135 behind the products of the inputs.  Per direction: x [seq, batch, 4 units]
+ * (inputs times input kernel, gates i, c, f, o), kernel [units, 4 units], bias [4 units], h0 and c0 [batch, units]; out
+ * [seq, batch, units] in the order the steps are taken, h and c [batch, units] after the last one; backward: the steps
+ * run from the last row of x to the first.  1 to 16 rows, 1 to 1024 units (else the workspace size is 0).  The workspace
+ * needs no particular contents.  wait_us: how long the workgroups wait for one another before the sequence is computed
+ * in a single one. */
+typedef struct tfcc_rocm_lstm_sequence_desc {
+  unsigned seq, batch, units, directions;
+  const float *x[2], *kernel[2], *bias[2], *h0[2], *c0[2];
+  float *out[2], *h[2], *c[2];
+  int backward[2];
+  float forget;
+  void* workspace;
+  size_t workspace_bytes;
+  unsigned wait_us;
+} tfcc_rocm_lstm_sequence_desc;
+size_t tfcc_rocm_lstm_sequence_workspace(unsigned batch, unsigned units, unsigned directions);
+int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc* desc);
 /* One step of tfcc::rnn::lstm_forward / lstm_backward (tfcc/core/operations/tfcc_rnn.cpp:62-71) in one launch:
  * matmul(h_prev, state kernel) and the LSTM cell above on its sums.  batch <= 8.  The state kernel is passed with its
  * gates interleaved: element [k, 4 * u + g] = state_kernel[k, g * units + u], i.e. the [units, 4, units] view of the

@@ -1,0 +1,106 @@
+"""A whole LSTM sequence in one launch (tfcc_rocm_lstm_sequence_f32) against the oracle's recurrence: every configuration of
+the kernel at the edges of its range of units and rows, one and two directions, on several streams at once, and with a
+wait that is over at once, so that the launch behind it computes the sequence."""
+import ctypes as C
+import threading
+
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from conftest import rel_fro
+
+pytestmark = pytest.mark.gpu
+
+
+def setup(T, seq, batch, length, hidden, directions, seed=0):
+    rng = np.random.default_rng(seq * 100 + batch * 10 + hidden + seed)
+    u = lambda *s: (rng.uniform(-1, 1, s) / np.sqrt(hidden)).astype(np.float32)
+    x = rng.standard_normal((seq, batch, length)).astype(np.float32)
+    sets = [dict(ik=u(length, 4 * hidden), sk=u(hidden, 4 * hidden), bias=u(4 * hidden), ih=u(batch, hidden), ic=u(batch, hidden))
+            for _ in range(directions)]
+    return x, sets
+
+
+def launch(pkg, T, x, sets, backward, wait_us=20000, stream=None):
+    import torch
+    seq, batch, _ = x.shape
+    hidden = sets[0]["ih"].shape[1]
+    d = pkg.LstmSequenceDesc()
+    d.seq, d.batch, d.units, d.directions, d.forget, d.wait_us = seq, batch, hidden, len(sets), 0.0, wait_us
+    need = pkg.lib().tfcc_rocm_lstm_sequence_workspace(batch, hidden, len(sets))
+    keep = [torch.randint(0, 255, (need,), dtype=torch.uint8, device="cuda")]  # no particular contents
+    d.workspace, d.workspace_bytes = keep[0].data_ptr(), need
+    outs = []
+    for i, s in enumerate(sets):
+        dev = {k: T.t(v) for k, v in s.items()}
+        values = pkg.blas_matmul(T.t(x.reshape(seq * batch, -1)), dev["ik"])
+        out, h, c = torch.empty((seq, batch, hidden), device="cuda"), torch.empty((batch, hidden), device="cuda"), torch.empty((batch, hidden), device="cuda")
+        keep += [dev, values]
+        d.x[i], d.kernel[i], d.bias[i], d.h0[i], d.c0[i] = (t.data_ptr() for t in (values, dev["sk"], dev["bias"], dev["ih"], dev["ic"]))
+        d.out[i], d.h[i], d.c[i], d.backward[i] = out.data_ptr(), h.data_ptr(), c.data_ptr(), int(backward[i])
+        outs.append((out, h, c))
+    torch.cuda.synchronize()
+    pkg.check(pkg.lib().tfcc_rocm_lstm_sequence_f32(stream, C.byref(d)))
+    return outs, keep
+
+
+def compare(T, outs, x, sets, backward):
+    for (out, h, c), s, back in zip(outs, sets, backward):
+        want = O.lstm_sequence(x, s["ik"], s["sk"], s["bias"], s["ih"], s["ic"], back)
+        for got, w in zip((out, h, c), want):
+            assert rel_fro(T.n(got), w.astype(np.float64)) <= 1e-5
+
+
+@pytest.mark.parametrize("seq,batch,hidden,directions", [
+    (1, 1, 1, 1), (2, 1, 3, 2), (3, 2, 255, 2), (4, 3, 256, 2), (5, 4, 257, 2), (3, 5, 511, 1), (4, 8, 512, 2),   # rows 1 to 16, units
+    (3, 9, 513, 2), (3, 12, 700, 1), (3, 13, 1023, 2), (4, 16, 1024, 2), (64, 4, 512, 2), (7, 16, 200, 2), (9, 1, 1000, 2)])
+def test_sequence_against_the_oracle(pkg, T, seq, batch, hidden, directions):
+    print("lstm sequence", seq, batch, hidden, directions, flush=True)
+    x, sets = setup(T, seq, batch, 40, hidden, directions)
+    backward = (False, True)[:directions]
+    outs, keep = launch(pkg, T, x, sets, backward)
+    compare(T, outs, x, sets, backward)
+    again, keep2 = launch(pkg, T, x, sets, backward)
+    for a, b in zip(outs, again):
+        for p, q in zip(a, b):
+            assert np.array_equal(T.n(p), T.n(q))
+
+
+@pytest.mark.parametrize("seq,batch,hidden", [(5, 3, 96), (4, 12, 600)])
+def test_a_wait_that_is_over_at_once(pkg, T, seq, batch, hidden):
+    x, sets = setup(T, seq, batch, 24, hidden, 2)
+    outs, keep = launch(pkg, T, x, sets, (False, True), wait_us=0)
+    compare(T, outs, x, sets, (False, True))
+
+
+def test_limits(pkg, T):
+    lib = pkg.lib()
+    assert lib.tfcc_rocm_lstm_sequence_workspace(17, 64, 2) == 0 and lib.tfcc_rocm_lstm_sequence_workspace(1, 1025, 2) == 0
+    d = pkg.LstmSequenceDesc()
+    d.seq, d.batch, d.units, d.directions = 1, 1, 8, 1
+    assert lib.tfcc_rocm_lstm_sequence_f32(None, C.byref(d)) == 1
+
+
+def test_several_threads_and_streams(pkg, T):
+    import torch
+    x, sets = setup(T, 20, 4, 32, 512, 2)
+    errors = []
+
+    def work():
+        try:
+            for _ in range(5):
+                stream = torch.cuda.Stream()
+                outs, keep = launch(pkg, T, x, sets, (False, True), stream=stream.cuda_stream)
+                torch.cuda.synchronize()
+                compare(T, outs, x, sets, (False, True))
+                pkg.check(pkg.lib().tfcc_rocm_stream_release(stream.cuda_stream))
+        except BaseException as e:  # noqa: B036
+            errors.append(e)
+
+    threads = [threading.Thread(target=work) for _ in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors

@@ -70,6 +70,14 @@ class AttentionDesc(C.Structure):
     ]
 
 
+class LstmSequenceDesc(C.Structure):
+    """tfcc_rocm_lstm_sequence_desc"""
+    _fields_ = [("seq", C.c_uint), ("batch", C.c_uint), ("units", C.c_uint), ("directions", C.c_uint)] + \
+        [(n, C.c_void_p * 2) for n in ("x", "kernel", "bias", "h0", "c0", "out", "h", "c")] + \
+        [("backward", C.c_int * 2), ("forget", C.c_float), ("workspace", C.c_void_p), ("workspace_bytes", C.c_size_t),
+         ("wait_us", C.c_uint)]
+
+
 # name -> (restype, argtypes): every symbol include/tfcc_rocm.h declares
 _VP, _U64, _U, _I, _F, _D, _I64 = C.c_void_p, C.c_uint64, C.c_uint, C.c_int, C.c_float, C.c_double, C.c_int64
 SYMBOLS = {
@@ -146,6 +154,8 @@ SYMBOLS = {
     "tfcc_rocm_compare": (_I, [_VP, _I, _VP, _VP, _I, _I, C.POINTER(C.c_uint), C.POINTER(_U64), C.POINTER(_U64), _VP]),
     "tfcc_rocm_topk_f32": (_I, [_VP, _VP, _U64, _U, _U, _VP, _VP]),
     "tfcc_rocm_argmax_f32": (_I, [_VP, _VP, _U64, _U, _U64, _VP]),
+    "tfcc_rocm_lstm_sequence_workspace": (C.c_size_t, [_U, _U, _U]),
+    "tfcc_rocm_lstm_sequence_f32": (_I, [_VP, _VP]),
     "tfcc_rocm_lstm_step_f32": (_I, [_VP, _U, _U, _VP, _VP, _VP, _VP, _F, _VP, _VP, _VP]),
     "tfcc_rocm_gru_cell_gates_f32": (_I, [_VP, _U, _U, _U, _VP, _VP, _VP, _VP, _VP]),
     "tfcc_rocm_gru_cell_candidate_f32": (_I, [_VP, _U, _U, _VP, _VP, _VP, _VP, _VP, _VP]),

@@ -1,0 +1,396 @@
+// A whole LSTM sequence, or both directions of a bidirectional one, in one launch.
+//
+// The recurrence is a chain of small steps: [batch, units] times [units, 4 units], the cell, and every unit needs every
+// unit's result of the step before.  A launch per step costs 4.8 us (4 x 512) although its arithmetic takes 0.2 us,
+// because the state kernel is fetched again and the launch itself has to be paid.  Here a workgroup owns U units for the
+// whole sequence, keeps their columns of the state kernel in registers, and the workgroups hand their part of h to each
+// other through memory: 2.3 us per step, both directions at once.
+//
+// The exchange is made of 64-bit words of a value and the number of the step it belongs to, written and read as one
+// atomic each: a reader polls the word itself until the step is the one it waits for, so nothing is ordered by fences.
+// Two sets of words alternate; a workgroup writes step t + 2 only after it has read all of step t + 1, which every other
+// workgroup wrote after it had read all of step t, so no word is overwritten before its last reader is through.
+//
+// All workgroups have to run at the same time.  The launcher asks for at most one per CU, but other work may hold CUs, so
+// every wait is bounded: a workgroup that has waited `waitTicks` raises a flag and ends, the others see the flag and end,
+// and the launch behind this one, which does nothing otherwise, finds the flag and computes the sequence in one workgroup
+// per direction.
+//
+// Arithmetic: tfcc/core/operations/tfcc_rnn.cpp:29-135 with the cell of tfcc/mkl/kernel/tfcc_mklcellkernel.hpp:51-87.
+#include <mutex>
+
+#include "common.hpp"
+#include "lstm_sequence.hpp"
+
+namespace tfcc_rocm {
+namespace {
+
+struct Sequence {
+  const float* x;       // [seq, batch, 4 units]: products of the inputs, gates i, c, f, o
+  const float* kernel;  // [units, 4 units]
+  const float* bias;    // [4 units]
+  const float* h0;      // [batch, units]
+  const float* c0;
+  float* out;           // [seq, batch, units], in the order the steps are taken
+  float* h;             // [batch, units]
+  float* c;
+  int backward;
+};
+struct SequenceParams {
+  Sequence s[2];
+  unsigned seq, batch, units, directions;
+  float forget;
+  unsigned blocksPerDirection;
+  unsigned long long* words;  // [2 sets][direction][batch][pitch]: value in the low half, step in the high one
+  unsigned* failed;
+  unsigned long long waitTicks;
+};
+
+__device__ __forceinline__ float sigmoid_value(float v) { return 1.f / (1.f + expf(0.f - v)); }
+
+__device__ __forceinline__ unsigned long long word_of(float value, unsigned step) {
+  return ((unsigned long long)step << 32) | __builtin_bit_cast(unsigned, value);
+}
+
+// Step 0 reads the initial h as a word of step 1; the other set holds no step anybody waits for.
+__global__ __launch_bounds__(256) void lstm_exchange_init_kernel(SequenceParams p, unsigned pitch, unsigned total) {
+  const unsigned i = blockIdx.x * 256 + threadIdx.x;
+  if (i == 0) *p.failed = 0;
+  if (i >= total) return;
+  const unsigned u = i % pitch, b = i / pitch % p.batch, d = i / pitch / p.batch;
+  const float h = u < p.units ? p.s[d].h0[(size_t)b * p.units + u] : 0.f;
+  p.words[i] = word_of(h, 1);
+  p.words[(size_t)total + i] = 0;
+}
+
+// Sums v[0 .. N) over the lanes that differ in the bits MASK, MASK / 2, ..., U of their number.  While the count is
+// even, the two halves of a pair of lanes keep one half of the values each: a lane ends with the totals of the values
+// base .. base + left(N) - 1.
+template <int N, int MASK, int U>
+constexpr int values_left() {
+  if constexpr (MASK >= U) return values_left<(N % 2 == 0 ? N / 2 : N), MASK / 2, U>();
+  else return N;
+}
+template <int N, int MASK, int U, int TOTAL>
+__device__ __forceinline__ void sum_over_lanes(float (&v)[TOTAL], int lane, int& base) {
+  if constexpr (MASK >= U) {
+    if constexpr (N % 2 == 0) {
+      constexpr int HALF = N / 2;
+      const bool upper = (lane & MASK) != 0;
+#pragma unroll
+      for (int a = 0; a < HALF; ++a) {
+        if constexpr (MASK >= 16) {
+          const unsigned x = __builtin_bit_cast(unsigned, v[a]), y = __builtin_bit_cast(unsigned, v[a + HALF]);
+          unsigned r0, r1;
+          if constexpr (MASK == 32) {
+            const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+            r0 = (unsigned)r[0]; r1 = (unsigned)r[1];
+          } else {
+            const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+            r0 = (unsigned)r[0]; r1 = (unsigned)r[1];
+          }
+          v[a] = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+        } else {
+          const float mine = upper ? v[a + HALF] : v[a], theirs = upper ? v[a] : v[a + HALF];
+          float same, other;
+          butterfly_pair<MASK>(theirs, same, other);
+          v[a] = mine + other;
+        }
+      }
+      base += upper ? HALF : 0;
+      sum_over_lanes<HALF, MASK / 2, U>(v, lane, base);
+    } else {
+#pragma unroll
+      for (int a = 0; a < N; ++a) {
+        float x, y;
+        butterfly_pair<MASK>(v[a], x, y);
+        v[a] = x + y;
+      }
+      sum_over_lanes<N, MASK / 2, U>(v, lane, base);
+    }
+  }
+}
+
+// MB: rows of the batch, padded; U units per workgroup; T threads.  Thread (slice, unit) holds the four gates of its
+// unit for the rows 4 (g * slices + slice) .. + 3 of the state kernel, g < G.
+template <int MB, int U, int T, int G>
+__global__ __launch_bounds__(T) void lstm_sequence_kernel(SequenceParams p) {
+  constexpr int SLICES = T / U, PITCH = SLICES * 4 * G, WAVES = T / 64, N = 4 * MB;
+  constexpr int LEFT = values_left<N, 32, U>();
+  static_assert(N * U <= T, "a thread per gate, unit and row finishes a step");
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float* hs = lds;                // [MB][PITCH]
+  float* parts = lds + MB * PITCH;  // [WAVES][N][U]
+  __shared__ int gaveUp;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const unsigned units = p.units, batch = p.batch;
+  const unsigned d = blockIdx.x / p.blocksPerDirection, u0 = (blockIdx.x - d * p.blocksPerDirection) * U;
+  const Sequence& s = p.s[d];
+  const int unit = tid % U, slice = tid / U;
+
+  float w[G][4][4];  // [rows][gate]
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const unsigned row = 4 * (g * SLICES + slice) + r;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        w[g][r][q] = (row < units && u0 + unit < units) ? s.kernel[(size_t)row * 4 * units + q * units + u0 + unit] : 0.f;
+    }
+  for (int i = tid; i < MB * PITCH; i += T) hs[i] = 0.f;  // rows of the batch and units that do not exist stay zero
+  if (tid == 0) gaveUp = 0;
+
+  // thread (row m, unit, gate) finishes one gate; the four gates of a unit are neighbouring lanes
+  const unsigned fg = tid & 3, fu = u0 + (tid >> 2) % U, fm = tid / (4 * U);
+  const bool valid = fm < batch && fu < units;
+  const size_t fidx = (size_t)fm * units + fu;
+  float cPrev = 0.f, bv = 0.f, xin = 0.f;
+  auto inputOf = [&](unsigned step) {
+    const unsigned t = s.backward ? p.seq - 1 - step : step;
+    return s.x[((size_t)t * batch + fm) * 4 * units + (size_t)fg * units + fu];
+  };
+  if (valid) {
+    bv = s.bias[(size_t)fg * units + fu];
+    cPrev = s.c0[fidx];
+    xin = inputOf(0);
+  }
+  const size_t setSize = (size_t)p.directions * batch * PITCH;
+  unsigned long long* mine = p.words + (size_t)d * batch * PITCH;
+  __syncthreads();
+
+  for (unsigned step = 0; step < p.seq; ++step) {
+    // ---- h of the step before: every thread polls its words
+    const unsigned long long* words = mine + (step & 1u) * setSize;
+    const unsigned long long start = wall_clock64();
+    constexpr int PER = (MB * PITCH + T - 1) / T, CHUNK = PER < 8 ? PER : 8;
+#pragma unroll
+    for (int k0 = 0; k0 < PER; k0 += CHUNK) {
+      unsigned long long v[CHUNK];
+      bool wanted[CHUNK];
+#pragma unroll
+      for (int k = 0; k < CHUNK; ++k) {
+        const unsigned i = tid + (k0 + k) * T;
+        wanted[k] = i < batch * PITCH && i % PITCH < units;
+      }
+      for (unsigned tries = 0;; ++tries) {
+        bool ready = true;
+#pragma unroll
+        for (int k = 0; k < CHUNK; ++k) {
+          v[k] = wanted[k] ? __hip_atomic_load(words + tid + (k0 + k) * T, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+        }
+#pragma unroll
+        for (int k = 0; k < CHUNK; ++k) ready = ready && (!wanted[k] || (unsigned)(v[k] >> 32) == step + 1);
+        if (ready) break;
+        if ((tries & 15u) == 15u &&
+            (wall_clock64() - start > p.waitTicks ||
+             __hip_atomic_load(p.failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+          gaveUp = 1;
+          break;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < CHUNK; ++k)
+        if (wanted[k]) hs[tid + (k0 + k) * T] = __builtin_bit_cast(float, (unsigned)v[k]);
+    }
+    __syncthreads();
+    if (gaveUp) {  // the same for the whole workgroup
+      if (tid == 0) __hip_atomic_store(p.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+
+    // ---- this workgroup's columns of h times the state kernel
+    float v[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = 0.f;
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const float4 h4 = *reinterpret_cast<const float4*>(hs + m * PITCH + 4 * (g * SLICES + slice));
+        const float hv[4] = {h4.x, h4.y, h4.z, h4.w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) v[m * 4 + q] = fmaf(hv[r], w[g][r][q], v[m * 4 + q]);
+      }
+    int base = 0;
+    sum_over_lanes<N, 32, U>(v, lane, base);
+#pragma unroll
+    for (int a = 0; a < LEFT; ++a) parts[(wave * N + base + a) * U + unit] = v[a];
+    __syncthreads();
+
+    // ---- the cell
+    if (fm < (unsigned)MB) {
+      float sum = 0.f;
+#pragma unroll
+      for (int wv = 0; wv < WAVES; ++wv) sum += parts[(wv * N + fm * 4 + fg) * U + (tid >> 2) % U];
+      float pre = xin + sum + bv;
+      if (fg == 2) pre += p.forget;
+      const float act = fg == 1 ? tanhf(pre) : sigmoid_value(pre);
+      const int first = lane & ~3;
+      const float xi = __shfl(act, first, 64), xc = __shfl(act, first + 1, 64), xf = __shfl(act, first + 2, 64),
+                  xo = __shfl(act, first + 3, 64);
+      if (valid) {
+        const float c = __fadd_rn(__fmul_rn(xc, xi), __fmul_rn(cPrev, xf)), h = tanhf(c) * xo;
+        cPrev = c;
+        const bool last = step + 1 == p.seq;
+        if (fg == 0) {
+          if (!last)
+            __hip_atomic_store(mine + ((step + 1) & 1u) * setSize + (size_t)fm * PITCH + fu, word_of(h, step + 2),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          s.out[(size_t)step * batch * units + fidx] = h;
+          if (last) {
+            s.h[fidx] = h;
+            s.c[fidx] = c;
+          }
+        }
+        if (!last) xin = inputOf(step + 1);
+      }
+    }
+  }
+}
+
+// The sequence once more in one workgroup per direction, if the launch before it gave up.
+__global__ __launch_bounds__(1024) void lstm_repair_kernel(SequenceParams p) {
+  if (__hip_atomic_load(p.failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) return;
+  const Sequence& s = p.s[blockIdx.x];
+  const unsigned units = p.units, batch = p.batch, state = batch * units;
+  for (unsigned i = threadIdx.x; i < state; i += 1024) s.c[i] = s.c0[i];
+  for (unsigned step = 0; step < p.seq; ++step) {
+    const float* h = step == 0 ? s.h0 : s.out + (size_t)(step - 1) * state;
+    const unsigned t = s.backward ? p.seq - 1 - step : step;
+    for (unsigned i = threadIdx.x; i < state; i += 1024) {
+      const unsigned b = i / units, u = i - b * units;
+      float sum[4] = {0.f, 0.f, 0.f, 0.f};
+      for (unsigned r = 0; r < units; ++r)
+        for (int q = 0; q < 4; ++q) sum[q] = fmaf(h[(size_t)b * units + r], s.kernel[(size_t)r * 4 * units + q * units + u], sum[q]);
+      const float* x = s.x + ((size_t)t * batch + b) * 4 * units + u;
+      float pre[4];
+      for (int q = 0; q < 4; ++q) pre[q] = x[(size_t)q * units] + sum[q] + s.bias[(size_t)q * units + u];
+      const float xi = sigmoid_value(pre[0]), xc = tanhf(pre[1]), xf = sigmoid_value(pre[2] + p.forget), xo = sigmoid_value(pre[3]);
+      const float c = __fadd_rn(__fmul_rn(xc, xi), __fmul_rn(s.c[i], xf)), hn = tanhf(c) * xo;
+      s.c[i] = c;
+      s.out[(size_t)step * state + i] = hn;
+      if (step + 1 == p.seq) s.h[i] = hn;
+    }
+    __threadfence_block();
+    __syncthreads();
+  }
+}
+
+// Tile of a product: U units per workgroup so that both directions take at most 256 workgroups.
+struct Config { unsigned u, pitch; };
+Config config_of(unsigned units) { return units <= 256 ? Config{4, 256} : units <= 512 ? Config{4, 512} : Config{8, 1024}; }
+
+template <int MB, int U, int T, int G>
+int launch(hipStream_t stream, const SequenceParams& p) {
+  constexpr unsigned pitch = T / U * 4 * G;
+  constexpr size_t lds = ((size_t)MB * pitch + (size_t)(T / 64) * 4 * MB * U) * sizeof(float);
+  static_assert(lds <= 128 * 1024, "LDS budget");
+  auto kern = lstm_sequence_kernel<MB, U, T, G>;
+  static bool attrSet[16] = {};  // per device: the attribute belongs to the function on one device
+  int dev = 0;
+  TFCC_HIP_CHECK(hipGetDevice(&dev));
+  TFCC_REQUIRE(dev >= 0 && dev < 16, "device index %d", dev);
+  if (!attrSet[dev]) {
+    TFCC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    attrSet[dev] = true;
+  }
+  const unsigned total = p.directions * p.batch * pitch;
+  hipLaunchKernelGGL(lstm_exchange_init_kernel, dim3((total + 255) / 256), dim3(256), 0, stream, p, pitch, total);
+  hipLaunchKernelGGL(kern, dim3(p.blocksPerDirection * p.directions), dim3(T), lds, stream, p);
+  hipLaunchKernelGGL(lstm_repair_kernel, dim3(p.directions), dim3(1024), 0, stream, p);
+  return check_launch("lstm_sequence");
+}
+
+template <int U, int T, int G>
+int launch_rows(hipStream_t stream, const SequenceParams& p) {
+  if (p.batch == 1) return launch<1, U, T, G>(stream, p);
+  if (p.batch == 2) return launch<2, U, T, G>(stream, p);
+  if (p.batch <= 4) return launch<4, U, T, G>(stream, p);
+  if (p.batch <= 8) return launch<8, U, T, G>(stream, p);
+  if (p.batch <= 12) return launch<12, U, T, G>(stream, p);
+  return launch<16, U, T, G>(stream, p);
+}
+
+// Two of these launches at once would each hold CUs that the other waits for, until both give up: launches from different
+// streams of the process follow one another.  The event is recorded only when a second stream turns up.
+struct Turn {
+  std::mutex mtx;
+  hipStream_t last = nullptr;
+  hipEvent_t event = nullptr;
+  bool used = false;
+};
+Turn g_turns[16];
+
+}  // namespace
+
+void lstm_sequence_forget_stream(hipStream_t stream) {
+  for (Turn& t : g_turns) {
+    std::lock_guard<std::mutex> lk(t.mtx);
+    if (t.used && t.last == stream) t.used = false;  // the stream is idle
+  }
+}
+
+}  // namespace tfcc_rocm
+
+using namespace tfcc_rocm;
+
+extern "C" {
+
+size_t tfcc_rocm_lstm_sequence_workspace(unsigned batch, unsigned units, unsigned directions) {
+  if (batch < 1 || batch > 16 || units < 1 || units > 1024 || directions < 1 || directions > 2) return 0;
+  return (size_t)2 * directions * batch * config_of(units).pitch * 8 + 64;
+}
+
+int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc* q) {
+  TFCC_REQUIRE(q != nullptr, "lstm_sequence: null argument");
+  const size_t need = tfcc_rocm_lstm_sequence_workspace(q->batch, q->units, q->directions);
+  TFCC_REQUIRE(need != 0, "lstm_sequence: 1 to 16 rows, 1 to 1024 units and 1 or 2 directions, got %u, %u, %u", q->batch, q->units,
+               q->directions);
+  TFCC_REQUIRE(q->seq >= 1 && q->seq < 0xfffffff0u, "lstm_sequence: %u steps", q->seq);
+  TFCC_REQUIRE(q->workspace && (uintptr_t)q->workspace % 8 == 0 && q->workspace_bytes >= need,
+               "lstm_sequence: the workspace needs %zu bytes", need);
+  SequenceParams p{};
+  for (unsigned d = 0; d < q->directions; ++d) {
+    TFCC_REQUIRE(q->x[d] && q->kernel[d] && q->bias[d] && q->h0[d] && q->c0[d] && q->out[d] && q->h[d] && q->c[d],
+                 "lstm_sequence: null operand");
+    p.s[d] = Sequence{q->x[d], q->kernel[d], q->bias[d], q->h0[d], q->c0[d], q->out[d], q->h[d], q->c[d], q->backward[d]};
+  }
+  const Config c = config_of(q->units);
+  p.seq = q->seq; p.batch = q->batch; p.units = q->units; p.directions = q->directions;
+  p.forget = q->forget;
+  p.blocksPerDirection = (q->units + c.u - 1) / c.u;
+  p.words = static_cast<unsigned long long*>(q->workspace);
+  p.failed = reinterpret_cast<unsigned*>(static_cast<char*>(q->workspace) + need - 64);
+  p.waitTicks = (unsigned long long)q->wait_us * 100;  // of the 100 MHz clock
+  int dev = 0, cus = 0;
+  TFCC_HIP_CHECK(hipGetDevice(&dev));
+  TFCC_REQUIRE(dev >= 0 && dev < 16, "device index %d", dev);
+  TFCC_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  TFCC_REQUIRE((int)(p.blocksPerDirection * p.directions) <= cus, "lstm_sequence: needs %u CUs", p.blocksPerDirection * p.directions);
+  hipStream_t s = as_stream(stream);
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  TFCC_HIP_CHECK(hipStreamIsCapturing(s, &capturing));
+  Turn& turn = g_turns[dev];
+  std::unique_lock<std::mutex> lk(turn.mtx, std::defer_lock);
+  if (capturing == hipStreamCaptureStatusNone) {
+    lk.lock();
+    if (turn.used && turn.last != s) {
+      hipStreamCaptureStatus other = hipStreamCaptureStatusNone;
+      if (turn.event == nullptr) TFCC_HIP_CHECK(hipEventCreateWithFlags(&turn.event, hipEventDisableTiming));
+      if (hipStreamIsCapturing(turn.last, &other) == hipSuccess && other == hipStreamCaptureStatusNone) {
+        TFCC_HIP_CHECK(hipEventRecord(turn.event, turn.last));
+        TFCC_HIP_CHECK(hipStreamWaitEvent(s, turn.event, 0));
+      }
+    }
+    turn.used = true;
+    turn.last = s;
+  }
+  if (q->units <= 256) return launch_rows<4, 256, 1>(s, p);
+  if (q->units <= 512) return launch_rows<4, 512, 1>(s, p);
+  return launch_rows<8, 512, 4>(s, p);
+}
+
+}  // extern "C"

@@ -515,6 +515,22 @@ class ROCMBlasInterface : public BlasInterface<float> {
   Variable<float> matmul(const Tensor<float>& a, const Tensor<float>& b, const Tensor<float>& bias) override {
     return rocm_sgemm(a, b, &bias, nullptr, 0);
   }
+  std::vector<Variable<float>> matmulShared(const Tensor<float>& a, const std::vector<const Tensor<float>*>& b) override {
+    bool grouped = b.size() >= 2 && b.size() <= 4 && a.shape().size() == 2 && a.size() > 0;
+    for (const Tensor<float>* m : b) grouped = grouped && m->size() > 0 && m->shape() == b[0]->shape() && m->shape().size() == 2 && m->shape(0) == a.shape(1);
+    if (!grouped) return BlasInterface<float>::matmulShared(a, b);
+    const unsigned m = a.shape(0), k = a.shape(1), n = b[0]->shape(1);
+    std::vector<Variable<float>> r;
+    const float* bp[4];
+    float* cp[4];
+    for (size_t g = 0; g < b.size(); ++g) {
+      r.emplace_back(Shape({m, n}));
+      bp[g] = b[g]->data();
+      cp[g] = r.back().data();
+    }
+    check(tfcc_rocm_sgemm_grouped(current_stream(), a.data(), bp, nullptr, cp, static_cast<unsigned>(b.size()), m, n, k));
+    return r;
+  }
 };
 
 // ---- quantization --------------------------------------------------------------------------------
@@ -636,6 +652,36 @@ class ROCMCellInterface : public CellInterface<float> {
     check_lstm(stateC, inputValue, stateHValue, bias);
     check(tfcc_rocm_lstm_cell_f32(current_stream(), stateC.shape(0), stateC.shape(1), stateC.data(), inputValue.data(),
                                   stateHValue.data(), bias.data(), forget, h, cs));
+  }
+  void processLSTMSequences(const std::vector<LSTMSequence<float>>& sequences, unsigned seq, float forget) override {
+    tfcc_rocm_lstm_sequence_desc d{};
+    const unsigned batch = sequences[0].ih->shape(0), units = sequences[0].ih->shape(1);
+    const size_t bytes = tfcc_rocm_lstm_sequence_workspace(batch, units, static_cast<unsigned>(sequences.size()));
+    if (bytes == 0) throw NotImplementedError("LSTM sequence in one launch: 1 to 16 rows, at most 1024 units");
+    for (size_t i = 1; i < sequences.size(); ++i)
+      if (sequences[i].ih->shape() != sequences[0].ih->shape()) throw NotImplementedError("LSTM sequences of different shapes");
+    Variable<uint8_t> workspace({static_cast<unsigned>(bytes)});
+    d.seq = seq;
+    d.batch = batch;
+    d.units = units;
+    d.directions = static_cast<unsigned>(sequences.size());
+    for (size_t i = 0; i < sequences.size(); ++i) {
+      const LSTMSequence<float>& s = sequences[i];
+      d.x[i] = s.inputValues->data();
+      d.kernel[i] = s.stateKernel->data();
+      d.bias[i] = s.bias->data();
+      d.h0[i] = s.ih->data();
+      d.c0[i] = s.ic->data();
+      d.out[i] = s.out;
+      d.h[i] = s.h;
+      d.c[i] = s.c;
+      d.backward[i] = s.backward ? 1 : 0;
+    }
+    d.forget = forget;
+    d.workspace = workspace.data();
+    d.workspace_bytes = bytes;
+    d.wait_us = 20000;
+    check(tfcc_rocm_lstm_sequence_f32(current_stream(), &d));
   }
   // [units, 4 units] -> gates interleaved, [units, units, 4]: column 4 u + g is gate g of unit u
   Variable<float> prepareLSTMStateKernel(const Tensor<float>& stateKernel, unsigned batch) override {

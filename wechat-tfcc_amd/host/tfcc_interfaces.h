@@ -42,6 +42,12 @@ class BlasInterface {
   virtual Variable<T> matmul(const Tensor<T>&, const Tensor<T>&) { throw NotImplementedError(); }
   // c = a * b + bias, bias: [n]
   virtual Variable<T> matmul(const Tensor<T>&, const Tensor<T>&, const Tensor<T>&) { throw NotImplementedError(); }
+  // { a * b[g] }, a: [m, k], every b: [k, n]; devices with a launch for several products override it
+  virtual std::vector<Variable<T>> matmulShared(const Tensor<T>& a, const std::vector<const Tensor<T>*>& b) {
+    std::vector<Variable<T>> r;
+    for (const Tensor<T>* m : b) r.push_back(matmul(a, *m));
+    return r;
+  }
 };
 
 template <class T>
@@ -211,6 +217,12 @@ class TransformationInterface {
 // the memory of a whole sequence: the same step written into h and cs ([batch, units] each; cs may be
 // stateC's own memory), so that a sequence needs neither a copy nor a concat per step.
 template <class T>
+struct LSTMSequence {  // one direction; all of the shapes lstm_forward checks
+  const Tensor<T>*inputValues, *stateKernel, *bias, *ih, *ic;  // inputValues: [seq * batch, 4 units]
+  bool backward;
+  T *out, *h, *c;  // [seq, batch, units], [batch, units], [batch, units]
+};
+template <class T>
 class CellInterface {
  public:
   virtual ~CellInterface() {}
@@ -219,6 +231,11 @@ class CellInterface {
     throw NotImplementedError();
   }
   virtual void processLSTMCellInto(const Tensor<T>&, const Tensor<T>&, const Tensor<T>&, const Tensor<T>&, T, T*, T*) {
+    throw NotImplementedError();
+  }
+  // Whole sequences of one shape at once, for devices that have that.  NotImplementedError (the default, or for shapes
+  // the device does not take) sends the caller to the steps below.
+  virtual void processLSTMSequences(const std::vector<LSTMSequence<T>>& /*sequences*/, unsigned /*seq*/, T /*forget*/) {
     throw NotImplementedError();
   }
   // A whole time step in one launch, for devices that have one: the state kernel in the layout that launch wants
@@ -835,56 +852,86 @@ namespace rnn {
 namespace detail {
 // tfcc::rnn::lstm_forward / lstm_backward (tfcc/core/operations/tfcc_rnn.cpp:29-81, 83-135): the same checks,
 // gate layout, forget bias 0 and output order (outputs in the order the steps are taken).  The products of the
-// inputs with inputKernel do not depend on the recurrence, so all steps share one matmul of [seq * batch, length];
-// each step then costs one launch (the product with stateKernel and the cell together, where the device offers
-// that) or two (matmul, then a cell launch), and writes h straight into its row block of the result.
+// inputs with inputKernel do not depend on the recurrence, so all steps share one matmul of [seq * batch, length] per
+// direction; the steps then run in one go where the device offers that, or cost one launch each (the product with
+// stateKernel and the cell together) or two (matmul, then a cell launch) and write h straight into their row block of
+// the result.
 template <class T>
-std::tuple<Variable<T>, Variable<T>, Variable<T>> lstm_sequence(bool backward, const Tensor<T>& a,
-                                                                const Tensor<T>& inputKernel,
-                                                                const Tensor<T>& stateKernel, const Tensor<T>& bias,
-                                                                const Tensor<T>& ih, const Tensor<T>& ic) {
+struct LSTMInput {
+  const Tensor<T>*inputKernel, *stateKernel, *bias, *ih, *ic;
+  bool backward;
+};
+template <class T>
+using LSTMOutput = std::tuple<Variable<T>, Variable<T>, Variable<T>>;
+
+// Sequences over one input, of one shape: on a device that takes them, all in one go.
+template <class T>
+std::vector<LSTMOutput<T>> lstm_sequences(const Tensor<T>& a, const std::vector<LSTMInput<T>>& inputs) {
   if (a.shape().size() != 3) throw InvalidArgumentError("invalid input");
   const unsigned seq = a.shape(0), batch = a.shape(1), length = a.shape(2);
-  if (ih.shape() != ic.shape() || ih.shape().size() != 2 || ih.shape(0) != batch)
-    throw InvalidArgumentError("invalid ih or ic");
-  const unsigned hidden = ih.shape(1);
-  if (inputKernel.shape().size() != 2 || inputKernel.shape(0) != length || inputKernel.shape(1) != hidden * 4)
-    throw InvalidArgumentError("invalid input kernel");
-  if (stateKernel.shape().size() != 2 || stateKernel.shape(0) != hidden || stateKernel.shape(1) != hidden * 4)
-    throw InvalidArgumentError("invalid state kernel");
-  if (bias.shape().size() != 1 || bias.shape(0) != 4 * hidden) throw InvalidArgumentError("invalid bias");
-  if (a.size() == 0 || hidden == 0) throw InvalidArgumentError("invalid input");
+  for (const LSTMInput<T>& i : inputs) {
+    if (i.ih->shape() != i.ic->shape() || i.ih->shape().size() != 2 || i.ih->shape(0) != batch)
+      throw InvalidArgumentError("invalid ih or ic");
+    const unsigned hidden = i.ih->shape(1);
+    if (i.inputKernel->shape().size() != 2 || i.inputKernel->shape(0) != length || i.inputKernel->shape(1) != hidden * 4)
+      throw InvalidArgumentError("invalid input kernel");
+    if (i.stateKernel->shape().size() != 2 || i.stateKernel->shape(0) != hidden || i.stateKernel->shape(1) != hidden * 4)
+      throw InvalidArgumentError("invalid state kernel");
+    if (i.bias->shape().size() != 1 || i.bias->shape(0) != 4 * hidden) throw InvalidArgumentError("invalid bias");
+    if (a.size() == 0 || hidden == 0) throw InvalidArgumentError("invalid input");
+  }
+  const unsigned hidden = inputs[0].ih->shape(1);
+  const size_t state = static_cast<size_t>(batch) * hidden;
 
   Interface<T>& interface = Operation<T>::getCurrentInterface();
   View<T> flat(a, Shape({seq * batch, length}));
-  Variable<T> inputValues = interface.getBlasInterface().matmul(flat, inputKernel);  // [seq * batch, 4 hidden]
-  Variable<T> result({seq, batch, hidden});
-  Variable<T> c = interface.getDataInterface().copy(ic);
-  const size_t state = static_cast<size_t>(batch) * hidden;
-  View<T> h(ih);
-  Variable<T> prepared;  // the state kernel as the one-launch step wants it, where the device has such a step
-  bool oneLaunch = false;
+  std::vector<const Tensor<T>*> kernels;
+  for (const LSTMInput<T>& i : inputs) kernels.push_back(i.inputKernel);
+  // [seq * batch, 4 hidden] each
+  std::vector<Variable<T>> values = interface.getBlasInterface().matmulShared(flat, kernels);
+  std::vector<LSTMOutput<T>> outputs;
+  std::vector<LSTMSequence<T>> sequences;
+  for (size_t d = 0; d < inputs.size(); ++d) {
+    outputs.emplace_back(Variable<T>({seq, batch, hidden}), Variable<T>({batch, hidden}), Variable<T>({batch, hidden}));
+    sequences.push_back({&values[d], inputs[d].stateKernel, inputs[d].bias, inputs[d].ih, inputs[d].ic, inputs[d].backward,
+                         std::get<0>(outputs[d]).data(), std::get<1>(outputs[d]).data(), std::get<2>(outputs[d]).data()});
+  }
   try {
-    prepared = interface.getCellInterface().prepareLSTMStateKernel(stateKernel, batch);
-    oneLaunch = true;
+    interface.getCellInterface().processLSTMSequences(sequences, seq, static_cast<T>(0));
+    return outputs;
   } catch (const NotImplementedError&) {
   }
-  for (unsigned step = 0; step < seq; ++step) {
-    const unsigned t = backward ? seq - 1 - step : step;
-    View<T> x(inputValues, inputValues.shape(), t * batch, (t + 1) * batch);
-    if (oneLaunch) {
-      interface.getCellInterface().processLSTMStepInto(c, x, h, prepared, bias, static_cast<T>(0),
-                                                       result.data() + step * state, c.data());
-    } else {
-      Variable<T> stateValues = interface.getBlasInterface().matmul(h, stateKernel);
-      interface.getCellInterface().processLSTMCellInto(c, x, stateValues, bias, static_cast<T>(0),
-                                                       result.data() + step * state, c.data());
+  // step by step
+  for (size_t d = 0; d < inputs.size(); ++d) {
+    const LSTMInput<T>& in = inputs[d];
+    Variable<T>& result = std::get<0>(outputs[d]);
+    Variable<T> c = interface.getDataInterface().copy(*in.ic);
+    View<T> h(*in.ih);
+    Variable<T> prepared;  // the state kernel as the one-launch step wants it, where the device has such a step
+    bool oneLaunch = false;
+    try {
+      prepared = interface.getCellInterface().prepareLSTMStateKernel(*in.stateKernel, batch);
+      oneLaunch = true;
+    } catch (const NotImplementedError&) {
     }
-    h = View<T>(result, result.shape(), step, step + 1);
-    h.reshape(Shape({batch, hidden}));
+    for (unsigned step = 0; step < seq; ++step) {
+      const unsigned t = in.backward ? seq - 1 - step : step;
+      View<T> x(values[d], values[d].shape(), t * batch, (t + 1) * batch);
+      if (oneLaunch) {
+        interface.getCellInterface().processLSTMStepInto(c, x, h, prepared, *in.bias, static_cast<T>(0),
+                                                         result.data() + step * state, c.data());
+      } else {
+        Variable<T> stateValues = interface.getBlasInterface().matmul(h, *in.stateKernel);
+        interface.getCellInterface().processLSTMCellInto(c, x, stateValues, *in.bias, static_cast<T>(0),
+                                                         result.data() + step * state, c.data());
+      }
+      h = View<T>(result, result.shape(), step, step + 1);
+      h.reshape(Shape({batch, hidden}));
+    }
+    std::get<1>(outputs[d]) = interface.getDataInterface().copy(h);
+    std::get<2>(outputs[d]) = std::move(c);
   }
-  Variable<T> lastH = interface.getDataInterface().copy(h);
-  return std::make_tuple(std::move(result), std::move(lastH), std::move(c));
+  return outputs;
 }
 }  // namespace detail
 
@@ -892,14 +939,14 @@ template <class T>
 std::tuple<Variable<T>, Variable<T>, Variable<T>> lstm_forward(const Tensor<T>& a, const Tensor<T>& inputKernel,
                                                                const Tensor<T>& stateKernel, const Tensor<T>& bias,
                                                                const Tensor<T>& ih, const Tensor<T>& ic) {
-  return detail::lstm_sequence(false, a, inputKernel, stateKernel, bias, ih, ic);
+  return std::move(detail::lstm_sequences<T>(a, {{&inputKernel, &stateKernel, &bias, &ih, &ic, false}})[0]);
 }
 
 template <class T>
 std::tuple<Variable<T>, Variable<T>, Variable<T>> lstm_backward(const Tensor<T>& a, const Tensor<T>& inputKernel,
                                                                 const Tensor<T>& stateKernel, const Tensor<T>& bias,
                                                                 const Tensor<T>& ih, const Tensor<T>& ic) {
-  return detail::lstm_sequence(true, a, inputKernel, stateKernel, bias, ih, ic);
+  return std::move(detail::lstm_sequences<T>(a, {{&inputKernel, &stateKernel, &bias, &ih, &ic, true}})[0]);
 }
 
 }  // namespace rnn

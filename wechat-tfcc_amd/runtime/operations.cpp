@@ -1436,14 +1436,14 @@ class BidirectionalLSTM : public TypedOperation<T> {
     std::array<const Tensor<T>*, 6> i6{in[0], in[1], in[2], in[3], in[4], in[5]};
     std::array<Variable<T>*, 6> o6{out[0], out[1], out[2], out[3], out[4], out[5]};
     graph.addStep([i6, o6] {
-      for (unsigned d = 0; d < 2; ++d) {
-        for (int i = 1; i < 6; ++i)
-          if (i6[i]->shape().size() < 2 || i6[i]->shape(0) != 2) throw InvalidArgumentError("invalid shape");
-        View<T> ik = direction(*i6[1], d), sk = direction(*i6[2], d), bias = direction(*i6[3], d),
-                ih = direction(*i6[4], d), ic = direction(*i6[5], d);
-        std::tie(*o6[0 + d], *o6[2 + d], *o6[4 + d]) =
-            d == 0 ? rnn::lstm_forward(*i6[0], ik, sk, bias, ih, ic) : rnn::lstm_backward(*i6[0], ik, sk, bias, ih, ic);
-      }
+      for (int i = 1; i < 6; ++i)
+        if (i6[i]->shape().size() < 2 || i6[i]->shape(0) != 2) throw InvalidArgumentError("invalid shape");
+      std::vector<View<T>> v;
+      for (unsigned d = 0; d < 2; ++d)
+        for (int i = 1; i < 6; ++i) v.push_back(direction(*i6[i], d));
+      auto r = rnn::detail::lstm_sequences<T>(
+          *i6[0], {{&v[0], &v[1], &v[2], &v[3], &v[4], false}, {&v[5], &v[6], &v[7], &v[8], &v[9], true}});
+      for (unsigned d = 0; d < 2; ++d) std::tie(*o6[0 + d], *o6[2 + d], *o6[4 + d]) = std::move(r[d]);
     });
     return true;
   }
