@@ -2,9 +2,10 @@
 //
 // The recurrence is a chain of small steps: [batch, units] times [units, 4 units], the cell, and every unit needs every
 // unit's result of the step before.  A launch per step costs 4.8 us (4 x 512) although its arithmetic takes 0.2 us,
-// because the state kernel is fetched again and the launch itself has to be paid.  Here a workgroup owns U units for the
-// whole sequence, keeps their columns of the state kernel in registers, and the workgroups hand their part of h to each
-// other through memory: 2.3 us per step, both directions at once.
+// because the state kernel is fetched again and the launch itself has to be paid.  Here a workgroup owns eight units for
+// the whole sequence, keeps their columns of the state kernel in registers, and the workgroups hand their part of h to
+// each other through memory: 2.3 us per step, both directions at once (1.7 for 1 x 256, 3.8 for 4 x 1024).  What is left
+// is the way of h to memory and back and the polls that came too early.
 //
 // The exchange is made of 64-bit words of a value and the number of the step it belongs to, written and read as one
 // atomic each: a reader polls the word itself until the step is the one it waits for, so nothing is ordered by fences.
@@ -111,59 +112,94 @@ __device__ __forceinline__ void sum_over_lanes(float (&v)[TOTAL], int lane, int&
   }
 }
 
-// MB: rows of the batch, padded; U units per workgroup; T threads.  Thread (slice, unit) holds the four gates of its
-// unit for the rows 4 (g * slices + slice) .. + 3 of the state kernel, g < G.
-template <int MB, int U, int T, int G>
-__global__ __launch_bounds__(T) void lstm_sequence_kernel(SequenceParams p) {
-  constexpr int SLICES = T / U, PITCH = SLICES * 4 * G, WAVES = T / 64, N = 4 * MB;
-  constexpr int LEFT = values_left<N, 32, U>();
-  static_assert(N * U <= T, "a thread per gate, unit and row finishes a step");
-  extern __shared__ __attribute__((aligned(16))) float lds[];
-  float* hs = lds;                // [MB][PITCH]
-  float* parts = lds + MB * PITCH;  // [WAVES][N][U]
+typedef float lstm_v4f __attribute__((ext_vector_type(4)));
+
+// The cell's functions stand in the chain of every step, so they are written without branches and share an exponential:
+// sigmoid(v) = 1 / (1 + e^-v), tanh(v) = (1 - e^-2|v|) / (1 + e^-2|v|) with v's sign, and below 0.625, where 1 - e would
+// cancel, v + v^3 P(v^2) with P a least-squares fit of degree 4 weighted for the relative error (1.3 units in the last
+// place of a float).  The quotient is corrected once, to within a unit in the last place.
+__device__ __forceinline__ float sigmoid_or_tanh(float v, bool tanhWanted) {
+  const float y = __builtin_fabsf(v);
+  float t = tanhWanted ? -2.f * y : -v;
+  t = t > 88.f ? 88.f : t;
+  const float e = softmax_exp(t);
+  const float num = tanhWanted ? 1.f - e : 1.f, den = 1.f + e;
+  const float r = __builtin_amdgcn_rcpf(den);
+  float q = num * r;
+  q = fmaf(fmaf(-den, q, num), r, q);
+  const float s = v * v;
+  float p = -5.704978481e-03f;
+  p = fmaf(p, s, 2.063907869e-02f);
+  p = fmaf(p, s, -5.373971164e-02f);
+  p = fmaf(p, s, 1.333144158e-01f);
+  p = fmaf(p, s, -3.333328068e-01f);
+  const float small = fmaf(v * s, p, v);
+  return !tanhWanted ? q : y < 0.625f ? small : __builtin_copysignf(q, v);
+}
+
+// A wavefront owns a unit and sums its four gates over all of K = 64 KI rows of the state kernel for 4 Q rows of the
+// batch, with matrix ops of sixteen independent 4 x 4 x 1 blocks: block = lane / 4 takes the rows k = 64 i + 4 block + r,
+// the four columns are the gates, the four rows four rows of the batch.  Twice the rate of the vector unit, no rows or
+// columns of padding at four rows, and what remains, sixteen partial sums of 4 Q values, ends one value per lane with the
+// four gates of a unit side by side: the wavefront finishes its unit alone, and the only barrier of a step is the one
+// behind the exchange (on the vector unit, with the sums joined through LDS: 3.0 us per step against 2.3).
+template <int Q, int KI, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void lstm_sequence_kernel(SequenceParams p) {
+  constexpr int T = 64 * WAVES, K = 64 * KI, MB = 4 * Q, LP = K + 16;  // LP: four rows fall on different banks
+  constexpr int LEFT = values_left<MB, 32, 4>();
+  extern __shared__ __attribute__((aligned(16))) float hs[];  // [2][MB][LP]
   __shared__ int gaveUp;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const unsigned units = p.units, batch = p.batch;
-  const unsigned d = blockIdx.x / p.blocksPerDirection, u0 = (blockIdx.x - d * p.blocksPerDirection) * U;
+  const unsigned d = blockIdx.x / p.blocksPerDirection;
   const Sequence& s = p.s[d];
-  const int unit = tid % U, slice = tid / U;
-
-  float w[G][4][4];  // [rows][gate]
-#pragma unroll
-  for (int g = 0; g < G; ++g)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const unsigned row = 4 * (g * SLICES + slice) + r;
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        w[g][r][q] = (row < units && u0 + unit < units) ? s.kernel[(size_t)row * 4 * units + q * units + u0 + unit] : 0.f;
-    }
-  for (int i = tid; i < MB * PITCH; i += T) hs[i] = 0.f;  // rows of the batch and units that do not exist stay zero
+  const size_t setSize = (size_t)p.directions * batch * K;
+  unsigned long long* mine = p.words + (size_t)d * batch * K;
+  for (int i = tid; i < 2 * MB * LP; i += T) hs[i] = 0.f;  // rows of the batch and units that do not exist stay zero
   if (tid == 0) gaveUp = 0;
-
-  // thread (row m, unit, gate) finishes one gate; the four gates of a unit are neighbouring lanes
-  const unsigned fg = tid & 3, fu = u0 + (tid >> 2) % U, fm = tid / (4 * U);
-  const bool valid = fm < batch && fu < units;
-  const size_t fidx = (size_t)fm * units + fu;
-  float cPrev = 0.f, bv = 0.f, xin = 0.f;
-  auto inputOf = [&](unsigned step) {
-    const unsigned t = s.backward ? p.seq - 1 - step : step;
-    return s.x[((size_t)t * batch + fm) * 4 * units + (size_t)fg * units + fu];
-  };
-  if (valid) {
-    bv = s.bias[(size_t)fg * units + fu];
-    cPrev = s.c0[fidx];
-    xin = inputOf(0);
-  }
-  const size_t setSize = (size_t)p.directions * batch * PITCH;
-  unsigned long long* mine = p.words + (size_t)d * batch * PITCH;
   __syncthreads();
 
+  const unsigned u = (blockIdx.x - d * p.blocksPerDirection) * WAVES + wave;
+  const int gate = lane & 3, block = lane >> 2;
+  const bool exists = u < units;
+  float w[KI][4];
+#pragma unroll
+  for (int i = 0; i < KI; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const unsigned k = 64 * i + 4 * block + r;
+      w[i][r] = (k < units && exists) ? s.kernel[(size_t)k * 4 * units + (size_t)gate * units + u] : 0.f;
+    }
+  // the row of the batch whose values this lane finishes
+  int base = 0;
+  {
+    float none[MB] = {};
+    sum_over_lanes<MB, 32, 4>(none, lane, base);
+  }
+  // what the halving has not told apart are copies: the first LEFT of the lanes that hold the same values take one each
+  constexpr int COPIES = 16 / (MB / LEFT);  // lanes of a gate that hold the same LEFT values
+  const int copy = block & (COPIES - 1);
+  const unsigned fm = base + (LEFT > 1 ? copy : 0);
+  const bool valid = copy < LEFT && fm < batch && exists;
+  auto inputOf = [&](unsigned step) {
+    const unsigned t = s.backward ? p.seq - 1 - step : step;
+    return valid ? s.x[((size_t)t * batch + fm) * 4 * units + (size_t)gate * units + u] : 0.f;
+  };
+  const size_t at = (size_t)fm * units + u;
+  const float bv = valid ? s.bias[(size_t)gate * units + u] : 0.f;
+  float cPrev = valid ? s.c0[at] : 0.f, xin = inputOf(0);
+
   for (unsigned step = 0; step < p.seq; ++step) {
-    // ---- h of the step before: every thread polls its words
+    // ---- h of the step before: every thread polls its words.  (Two buffers in LDS: a slow wavefront may still read the
+    // last step's.)  A poll that comes too early costs a whole trip to memory before the next one, and the traffic holds
+    // up the words it waits for; that the polling wavefronts are the ones that have just finished a step is what keeps
+    // most first polls from coming too early (wavefronts that only poll: 4.9 us per step against 2.3).
+    float* h = hs + (step & 1u) * (MB * LP);
     const unsigned long long* words = mine + (step & 1u) * setSize;
+    if constexpr (KI > 8 || Q > 2) __builtin_amdgcn_s_sleep(2);  // with more words per step: 1024 units x 4 rows 4.15 -> 3.8 us
     const unsigned long long start = wall_clock64();
-    constexpr int PER = (MB * PITCH + T - 1) / T, CHUNK = PER < 8 ? PER : 8;
+    constexpr int PER = (MB * K + T - 1) / T, CHUNK = PER < 8 ? PER : 8;
 #pragma unroll
     for (int k0 = 0; k0 < PER; k0 += CHUNK) {
       unsigned long long v[CHUNK];
@@ -171,14 +207,13 @@ __global__ __launch_bounds__(T) void lstm_sequence_kernel(SequenceParams p) {
 #pragma unroll
       for (int k = 0; k < CHUNK; ++k) {
         const unsigned i = tid + (k0 + k) * T;
-        wanted[k] = i < batch * PITCH && i % PITCH < units;
+        wanted[k] = i < batch * K && i % K < units;
       }
       for (unsigned tries = 0;; ++tries) {
         bool ready = true;
 #pragma unroll
-        for (int k = 0; k < CHUNK; ++k) {
+        for (int k = 0; k < CHUNK; ++k)
           v[k] = wanted[k] ? __hip_atomic_load(words + tid + (k0 + k) * T, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
-        }
 #pragma unroll
         for (int k = 0; k < CHUNK; ++k) ready = ready && (!wanted[k] || (unsigned)(v[k] >> 32) == step + 1);
         if (ready) break;
@@ -190,8 +225,10 @@ __global__ __launch_bounds__(T) void lstm_sequence_kernel(SequenceParams p) {
         }
       }
 #pragma unroll
-      for (int k = 0; k < CHUNK; ++k)
-        if (wanted[k]) hs[tid + (k0 + k) * T] = __builtin_bit_cast(float, (unsigned)v[k]);
+      for (int k = 0; k < CHUNK; ++k) {
+        const unsigned i = tid + (k0 + k) * T;
+        if (wanted[k]) h[i / K * LP + i % K] = __builtin_bit_cast(float, (unsigned)v[k]);
+      }
     }
     __syncthreads();
     if (gaveUp) {  // the same for the whole workgroup
@@ -199,53 +236,58 @@ __global__ __launch_bounds__(T) void lstm_sequence_kernel(SequenceParams p) {
       return;
     }
 
-    // ---- this workgroup's columns of h times the state kernel
-    float v[N];
+    // ---- the wavefront's four columns of h times the state kernel; the next step's inputs are asked for now, because
+    // the words polled next can only return behind them
+    const bool last = step + 1 == p.seq;
+    const float xNext = last ? 0.f : inputOf(step + 1);
+    constexpr int CHAINS = Q == 1 ? 2 : 1;  // accumulators per sum: a matrix op waits for the one before it on its own
+    lstm_v4f acc[Q][CHAINS];
 #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = 0.f;
+    for (int q = 0; q < Q; ++q)
 #pragma unroll
-    for (int m = 0; m < MB; ++m)
+      for (int c = 0; c < CHAINS; ++c) acc[q][c] = lstm_v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const float4 h4 = *reinterpret_cast<const float4*>(hs + m * PITCH + 4 * (g * SLICES + slice));
-        const float hv[4] = {h4.x, h4.y, h4.z, h4.w};
+    for (int i = 0; i < KI; ++i)
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const lstm_v4f a = *reinterpret_cast<const lstm_v4f*>(h + (4 * q + gate) * LP + 64 * i + 4 * block);
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) v[m * 4 + q] = fmaf(hv[r], w[g][r][q], v[m * 4 + q]);
+          acc[q][r % CHAINS] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[r], w[i][r], acc[q][r % CHAINS], 0, 0, 0);
       }
-    int base = 0;
-    sum_over_lanes<N, 32, U>(v, lane, base);
+    float v[MB];
 #pragma unroll
-    for (int a = 0; a < LEFT; ++a) parts[(wave * N + base + a) * U + unit] = v[a];
-    __syncthreads();
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v[4 * q + r] = acc[q][0][r];
+#pragma unroll
+        for (int c = 1; c < CHAINS; ++c) v[4 * q + r] += acc[q][c][r];
+      }
+    int unused = 0;
+    sum_over_lanes<MB, 32, 4>(v, lane, unused);
+    float sum = v[0];
+#pragma unroll
+    for (int a = 1; a < LEFT; ++a) sum = copy == a ? v[a] : sum;
 
     // ---- the cell
-    if (fm < (unsigned)MB) {
-      float sum = 0.f;
-#pragma unroll
-      for (int wv = 0; wv < WAVES; ++wv) sum += parts[(wv * N + fm * 4 + fg) * U + (tid >> 2) % U];
-      float pre = xin + sum + bv;
-      if (fg == 2) pre += p.forget;
-      const float act = fg == 1 ? tanhf(pre) : sigmoid_value(pre);
-      const int first = lane & ~3;
-      const float xi = __shfl(act, first, 64), xc = __shfl(act, first + 1, 64), xf = __shfl(act, first + 2, 64),
-                  xo = __shfl(act, first + 3, 64);
-      if (valid) {
-        const float c = __fadd_rn(__fmul_rn(xc, xi), __fmul_rn(cPrev, xf)), h = tanhf(c) * xo;
-        cPrev = c;
-        const bool last = step + 1 == p.seq;
-        if (fg == 0) {
-          if (!last)
-            __hip_atomic_store(mine + ((step + 1) & 1u) * setSize + (size_t)fm * PITCH + fu, word_of(h, step + 2),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          s.out[(size_t)step * batch * units + fidx] = h;
-          if (last) {
-            s.h[fidx] = h;
-            s.c[fidx] = c;
-          }
-        }
-        if (!last) xin = inputOf(step + 1);
+    float pre = xin + sum + bv;
+    if (gate == 2) pre += p.forget;
+    const float act = sigmoid_or_tanh(pre, gate == 1);
+    const int first = lane & ~3;
+    const float xi = __shfl(act, first, 64), xc = __shfl(act, first + 1, 64), xf = __shfl(act, first + 2, 64),
+                xo = __shfl(act, first + 3, 64);
+    const float c = __fadd_rn(__fmul_rn(xc, xi), __fmul_rn(cPrev, xf)), hn = sigmoid_or_tanh(c, true) * xo;
+    cPrev = c;
+    xin = xNext;
+    if (valid && gate == 0) {
+      if (!last)
+        __hip_atomic_store(mine + ((step + 1) & 1u) * setSize + (size_t)fm * K + u, word_of(hn, step + 2), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      s.out[(size_t)step * batch * units + at] = hn;
+      if (last) {
+        s.h[at] = hn;
+        s.c[at] = c;
       }
     }
   }
@@ -279,39 +321,38 @@ __global__ __launch_bounds__(1024) void lstm_repair_kernel(SequenceParams p) {
   }
 }
 
-// Tile of a product: U units per workgroup so that both directions take at most 256 workgroups.
-struct Config { unsigned u, pitch; };
-Config config_of(unsigned units) { return units <= 256 ? Config{4, 256} : units <= 512 ? Config{4, 512} : Config{8, 1024}; }
+unsigned padded_units(unsigned units) { return units <= 256 ? 256 : units <= 512 ? 512 : 1024; }
 
-template <int MB, int U, int T, int G>
-int launch(hipStream_t stream, const SequenceParams& p) {
-  constexpr unsigned pitch = T / U * 4 * G;
-  constexpr size_t lds = ((size_t)MB * pitch + (size_t)(T / 64) * 4 * MB * U) * sizeof(float);
-  static_assert(lds <= 128 * 1024, "LDS budget");
-  auto kern = lstm_sequence_kernel<MB, U, T, G>;
-  static bool attrSet[16] = {};  // per device: the attribute belongs to the function on one device
-  int dev = 0;
+template <int Q, int KI, int WAVES>
+int launch(hipStream_t stream, SequenceParams p) {
+  constexpr unsigned pitch = 64 * KI, unitsPerBlock = WAVES;
+  constexpr size_t lds = (size_t)2 * 4 * Q * (pitch + 16) * sizeof(float);
+  static_assert(lds <= 140 * 1024, "LDS budget");
+  p.blocksPerDirection = (p.units + unitsPerBlock - 1) / unitsPerBlock;
+  int dev = 0, cus = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));
   TFCC_REQUIRE(dev >= 0 && dev < 16, "device index %d", dev);
+  TFCC_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  TFCC_REQUIRE((int)(p.blocksPerDirection * p.directions) <= cus, "lstm_sequence: needs %u CUs", p.blocksPerDirection * p.directions);
+  auto kern = lstm_sequence_kernel<Q, KI, WAVES>;
+  static bool attrSet[16] = {};  // per device: the attribute belongs to the function on one device
   if (!attrSet[dev]) {
     TFCC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attrSet[dev] = true;
   }
   const unsigned total = p.directions * p.batch * pitch;
   hipLaunchKernelGGL(lstm_exchange_init_kernel, dim3((total + 255) / 256), dim3(256), 0, stream, p, pitch, total);
-  hipLaunchKernelGGL(kern, dim3(p.blocksPerDirection * p.directions), dim3(T), lds, stream, p);
+  hipLaunchKernelGGL(kern, dim3(p.blocksPerDirection * p.directions), dim3(64 * WAVES), lds, stream, p);
   hipLaunchKernelGGL(lstm_repair_kernel, dim3(p.directions), dim3(1024), 0, stream, p);
   return check_launch("lstm_sequence");
 }
 
-template <int U, int T, int G>
+template <int KI, int WAVES>
 int launch_rows(hipStream_t stream, const SequenceParams& p) {
-  if (p.batch == 1) return launch<1, U, T, G>(stream, p);
-  if (p.batch == 2) return launch<2, U, T, G>(stream, p);
-  if (p.batch <= 4) return launch<4, U, T, G>(stream, p);
-  if (p.batch <= 8) return launch<8, U, T, G>(stream, p);
-  if (p.batch <= 12) return launch<12, U, T, G>(stream, p);
-  return launch<16, U, T, G>(stream, p);
+  if (p.batch <= 4) return launch<1, KI, WAVES>(stream, p);
+  if (p.batch <= 8) return launch<2, KI, WAVES>(stream, p);
+  if (p.batch <= 12) return launch<3, KI, WAVES>(stream, p);
+  return launch<4, KI, WAVES>(stream, p);
 }
 
 // Two of these launches at once would each hold CUs that the other waits for, until both give up: launches from different
@@ -341,7 +382,7 @@ extern "C" {
 
 size_t tfcc_rocm_lstm_sequence_workspace(unsigned batch, unsigned units, unsigned directions) {
   if (batch < 1 || batch > 16 || units < 1 || units > 1024 || directions < 1 || directions > 2) return 0;
-  return (size_t)2 * directions * batch * config_of(units).pitch * 8 + 64;
+  return (size_t)2 * directions * batch * padded_units(units) * 8 + 64;
 }
 
 int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc* q) {
@@ -358,18 +399,14 @@ int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc
                  "lstm_sequence: null operand");
     p.s[d] = Sequence{q->x[d], q->kernel[d], q->bias[d], q->h0[d], q->c0[d], q->out[d], q->h[d], q->c[d], q->backward[d]};
   }
-  const Config c = config_of(q->units);
   p.seq = q->seq; p.batch = q->batch; p.units = q->units; p.directions = q->directions;
   p.forget = q->forget;
-  p.blocksPerDirection = (q->units + c.u - 1) / c.u;
   p.words = static_cast<unsigned long long*>(q->workspace);
   p.failed = reinterpret_cast<unsigned*>(static_cast<char*>(q->workspace) + need - 64);
   p.waitTicks = (unsigned long long)q->wait_us * 100;  // of the 100 MHz clock
-  int dev = 0, cus = 0;
+  int dev = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));
   TFCC_REQUIRE(dev >= 0 && dev < 16, "device index %d", dev);
-  TFCC_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  TFCC_REQUIRE((int)(p.blocksPerDirection * p.directions) <= cus, "lstm_sequence: needs %u CUs", p.blocksPerDirection * p.directions);
   hipStream_t s = as_stream(stream);
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   TFCC_HIP_CHECK(hipStreamIsCapturing(s, &capturing));
@@ -388,9 +425,12 @@ int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc
     turn.used = true;
     turn.last = s;
   }
-  if (q->units <= 256) return launch_rows<4, 256, 1>(s, p);
-  if (q->units <= 512) return launch_rows<4, 512, 1>(s, p);
-  return launch_rows<8, 512, 4>(s, p);
+  // eight wavefronts, so eight units, per workgroup: with four, twice the workgroups poll; with twelve or sixteen, each of
+  // which reads all of h from LDS, that takes longer than the trip to memory (4 x 1024: 3.8, 5.8 and 7.0 us per step with
+  // eight, twelve and sixteen)
+  if (q->units <= 256) return launch_rows<4, 8>(s, p);
+  if (q->units <= 512) return launch_rows<8, 8>(s, p);
+  return launch_rows<16, 8>(s, p);
 }
 
 }  // extern "C"
