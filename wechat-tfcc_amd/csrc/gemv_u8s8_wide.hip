@@ -515,7 +515,8 @@ unsigned long long workspace_key(int dev, hipStream_t stream) {
 }
 int workspace_alloc(void** mem, size_t bytes) {
   if (hipMalloc(mem, bytes) != hipSuccess) return TFCC_ROCM_OUT_OF_MEMORY;
-  if (hipMemset(*mem, 0, bytes) != hipSuccess) {
+  // (the fill runs on the null stream, and the stream that is going to use the words need not wait for that one)
+  if (hipMemset(*mem, 0, bytes) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
     (void)hipFree(*mem);
     return TFCC_ROCM_HIP_ERROR;
   }
