@@ -1,0 +1,80 @@
+"""The edges of the quantization kernels: whole tensors in one launch and the launch behind its limit, elements behind the
+last 16-byte piece, rows that start at any address.  Whole numbers and one fixed expression of floats: exact."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+
+LIMIT = 128 * 1024  # elements a single launch quantizes
+
+
+@pytest.mark.parametrize("total", [1, 2, 3, 5, 4095, 4096, 4097, 32771, LIMIT - 1, LIMIT, LIMIT + 1, LIMIT + 4])
+@pytest.mark.parametrize("dtype", ["uint8", "int8"])
+@pytest.mark.parametrize("skip", [0, 1])
+def test_quantize_with_the_range_of_the_data(pkg, T, total, dtype, skip):
+    import torch
+    x = np.random.default_rng(total).normal(0.1, 2.0, total + skip).astype(np.float32)
+    x[skip + total // 2] = 17.0  # the extremes: inside, and the very last element
+    x[-1] = -31.0
+    q, mn, mx = pkg.quantize(T.t(x)[skip:], getattr(torch, dtype))  # skip: not on a 16-byte boundary
+    lo, hi = float(x[skip:].min()), float(x[skip:].max())
+    assert (float(T.n(mn)[0]), float(T.n(mx)[0])) == (lo, hi)
+    assert np.array_equal(T.n(q), O.quantize(x[skip:], lo, hi, dtype))
+
+
+@pytest.mark.parametrize("special", [[np.nan, 1.0, -2.0], [np.inf, 1.0, -2.0], [3.0, 3.0, 3.0], [np.nan] * 3, [-7.5, 0.3, 9.25]])
+@pytest.mark.parametrize("dtype", ["uint8", "int16", "int32"])
+def test_quantize_small_and_large_tensors_agree(pkg, T, special, dtype):
+    import torch
+    small = np.array(special, np.float32)
+    large = np.tile(small, LIMIT // 3 + 1)  # beyond the limit: the form in three launches
+    a, b = (pkg.quantize(T.t(v), getattr(torch, dtype)) for v in (small, large))
+    for v, w in zip(a[1:], b[1:]):
+        assert np.array_equal(T.n(v), T.n(w), equal_nan=True)
+    assert np.array_equal(np.tile(T.n(a[0]), LIMIT // 3 + 1), T.n(b[0]))
+
+
+@pytest.mark.parametrize("total", [1, 3, 4, 1023, 4097, 95249])
+def test_dequantize_behind_the_last_piece(pkg, T, total):
+    x = np.random.default_rng(total).integers(-2 ** 31, 2 ** 31, total, dtype=np.int64).astype(np.int32)
+    got = T.n(pkg.dequantize(T.t(x), T.f1(-3.25), T.f1(7.5)))
+    assert np.array_equal(got, O.dequantize(x, -3.25, 7.5))
+
+
+@pytest.mark.parametrize("col", [1, 15, 16, 17, 127, 1001, 8192, 8209])
+@pytest.mark.parametrize("dtype", ["uint8", "int8", "int16"])
+def test_row_sums_at_any_address(pkg, T, col, dtype):
+    info = np.iinfo(dtype)
+    a = np.random.default_rng(col).integers(info.min, info.max + 1, (7, col)).astype(dtype)
+    flat = T.t(np.concatenate([a[0, :1], a.ravel()]))
+    for t in (T.t(a), flat[1:].view(7, col)):
+        assert np.array_equal(T.n(pkg.reduce_sum(t, True)).ravel(), a.sum(1, dtype=np.int64).astype(np.int32))
+
+
+def test_quantize_on_several_streams_and_under_capture(pkg, T):
+    import torch
+    rng = np.random.default_rng(3)
+    xs = [rng.normal(0, 1 + i, 3 * LIMIT + i).astype(np.float32) for i in range(4)]
+    ts, streams = [T.t(x) for x in xs], [torch.cuda.Stream() for _ in xs]
+    torch.cuda.synchronize()
+    want = [O.quantize(x, float(x.min()), float(x.max()), "uint8") for x in xs]
+    outs = []
+    for _ in range(5):
+        for t, s in zip(ts, streams):
+            with torch.cuda.stream(s):
+                outs.append(pkg.quantize(t, torch.uint8)[0])
+    torch.cuda.synchronize()
+    for i, q in enumerate(outs):
+        assert np.array_equal(T.n(q), want[i % 4])
+    graph, static = torch.cuda.CUDAGraph(), ts[0].clone()
+    with torch.cuda.graph(graph):
+        q = pkg.quantize(static, torch.uint8)[0]
+    for i in (0, 0, 0):
+        static.copy_(ts[i])
+        graph.replay()
+        eager = pkg.quantize(ts[1], torch.uint8)[0]
+        torch.cuda.synchronize()
+        assert np.array_equal(T.n(q), want[0]) and np.array_equal(T.n(eager), want[1])
+        q.zero_()

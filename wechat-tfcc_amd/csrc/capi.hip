@@ -6,6 +6,7 @@
 #include "common.hpp"
 #include "gemv.hpp"
 #include "lstm_sequence.hpp"
+#include "quant_ops.hpp"
 
 namespace tfcc_rocm {
 
@@ -102,6 +103,7 @@ int tfcc_rocm_stream_release(void* stream) {
   // the stream's pending work may still use what is given back
   TFCC_HIP_CHECK(hipStreamSynchronize(as_stream(stream)));
   tfcc_rocm::lstm_sequence_forget_stream(as_stream(stream));
+  if (int e = tfcc_rocm::quantize_release_stream(as_stream(stream))) return e;
   return tfcc_rocm::gemv_wide_release_stream(as_stream(stream));
 }
 
