@@ -7,6 +7,7 @@
 #include "gemv.hpp"
 #include "lstm_sequence.hpp"
 #include "quant_ops.hpp"
+#include "sgemm_params.hpp"
 
 namespace tfcc_rocm {
 
@@ -104,6 +105,9 @@ int tfcc_rocm_stream_release(void* stream) {
   TFCC_HIP_CHECK(hipStreamSynchronize(as_stream(stream)));
   tfcc_rocm::lstm_sequence_forget_stream(as_stream(stream));
   if (int e = tfcc_rocm::quantize_release_stream(as_stream(stream))) return e;
+  int dev = 0;
+  TFCC_HIP_CHECK(hipGetDevice(&dev));
+  tfcc_rocm::sgemm_detail::sgemm_skinny_release_stream(dev, as_stream(stream));
   return tfcc_rocm::gemv_wide_release_stream(as_stream(stream));
 }
 

@@ -7,13 +7,9 @@
 // tfcc/mkl/kernel/tfcc_mklquantizationkernel.avx256.cpp:55-145 (the AVX2 kernels: nearest-even
 // rounding, fused multiply-add) and the branches of
 // tfcc/mkl/interfaces/tfcc_mklquantizationinterface.cpp:47-69,72-147,191-240,284-333.
-#include <map>
-#include <mutex>
-#include <utility>
-#include <vector>
-
 #include "common.hpp"
 #include "quant_ops.hpp"
+#include "stream_slots.hpp"
 
 namespace tfcc_rocm {
 namespace {
@@ -592,47 +588,9 @@ unsigned stream_grid(size_t total4) {
   return (unsigned)blocks;
 }
 
-// The word on which a stream's range reductions count their workgroups.  Launches on one stream run in order and share it;
-// streams that may overlap get one each.  A graph may replay beside its stream's own work, so a stream that is being
-// captured gets none, and neither does one that comes when all words are given out: those calls take the form with
-// atomics on the result.
-class ArrivalSlots {
- public:
-  bool of(int dev, hipStream_t stream, unsigned* slot) {
-    if (stream == hipStreamPerThread) return false;  // one handle, a stream per thread
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return false;
-    std::lock_guard<std::mutex> lock(mutex_);
-    const auto found = given_.find({dev, stream});
-    if (found != given_.end()) {
-      *slot = found->second;
-      return true;
-    }
-    if (free_.empty() && next_ == kArrivalSlots) return false;
-    if (free_.empty()) {
-      *slot = next_++;
-    } else {
-      *slot = free_.back();
-      free_.pop_back();
-    }
-    given_[{dev, stream}] = *slot;
-    return true;
-  }
-  void release(int dev, hipStream_t stream) {
-    std::lock_guard<std::mutex> lock(mutex_);
-    const auto found = given_.find({dev, stream});
-    if (found == given_.end()) return;
-    free_.push_back(found->second);
-    given_.erase(found);
-  }
-
- private:
-  std::mutex mutex_;
-  std::map<std::pair<int, hipStream_t>, unsigned> given_;
-  std::vector<unsigned> free_;
-  unsigned next_ = 0;
-};
-ArrivalSlots gArrivalSlots;
+// The word on which a stream's range reductions count their workgroups; calls that get none take the form with atomics on
+// the result.
+StreamSlots gArrivalSlots(kArrivalSlots);
 
 bool valid_type(int t) { return t >= TFCC_ROCM_S8 && t <= TFCC_ROCM_U32; }
 

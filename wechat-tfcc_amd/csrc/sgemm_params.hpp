@@ -66,5 +66,11 @@ int sgemm_wave96_launch(hipStream_t stream, SgemmParams p, int ksplit, int block
 bool sgemv_supported(const SgemmParams& p);
 int sgemv_launch(hipStream_t stream, const SgemmParams& p);
 
+// The kernel for few rows (sgemm_skinny.hip): one product, or the grouped form; any alignment, B as stored or transposed,
+// operands below 2^30 elements.
+bool sgemm_skinny_better(unsigned m, unsigned n, unsigned k);
+void sgemm_skinny_release_stream(int dev, hipStream_t stream);
+int sgemm_skinny_launch(hipStream_t stream, const SgemmParams& p, bool transB);
+
 }  // namespace sgemm_detail
 }  // namespace tfcc_rocm

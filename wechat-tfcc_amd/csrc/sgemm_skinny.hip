@@ -1,0 +1,225 @@
+// fp32 products whose tiles leave most of the chip idle: few rows, K long against N.  In 32-row tiles 32 x 3072 x 768 is
+// 24 workgroups of four wavefronts, each walking a quarter of K slab by slab; the matrix cores of 24 CUs and their loads
+// decide (19 us for 9 MB of B).
+//
+// A workgroup owns 16 rows x 16 columns and deals the steps of K (16 k each) among eight wavefronts; where the tiles leave
+// CUs without work, several workgroups share a tile's steps.  Nothing is shared before the partial tiles meet, so nothing
+// goes through LDS on the way in: a lane loads its operands of the 16x16x4 matrix op as they lie, four consecutive k of a
+// row of A in one load and the same four k of its column of B, with two batches of four steps under way.  Bound by what a
+// CU can have on its way from memory.  (Tiles of 16 x 32, whole lines of B, take twice as long: half the workgroups.)
+//
+// With weights from memory, against the tiles of 32 rows: 32 x 3072 x 768 19.6 -> 8.6 us, 9 x 4096 x 1024 24.3 -> 8.2,
+// 16 x 8192 x 2048 70 -> 26, 64 x 8192 x 300 50 -> 13, 32 x 768 x 768 6.3 -> 4.7, 48 x 1001 x 1237 8.2 -> 5.9.
+//
+// An element is the sum of its wavefronts' partial sums, added in the order of the wavefronts, then of the splits;
+// wavefront w of W has the steps w, w + W, ... in ascending order.  The shorter chains leave half the error (3072 k: 2e-7
+// against 5e-7).  B transposed and B as stored give the same bits, and so does a launch that may not use the memory in
+// which the splits meet: its workgroups play all splits one after the other.  Bias, residual and the erf-form GELU follow
+// as in the other kernels (tfcc/mkl/interfaces/tfcc_mklblasinterface.cpp:41-67, 69-78, 87-118).
+#include "common.hpp"
+#include "sgemm_params.hpp"
+#include "stream_slots.hpp"
+
+namespace tfcc_rocm {
+namespace {
+
+using sgemm_detail::SgemmParams;
+
+typedef float skinny_v4f __attribute__((ext_vector_type(4)));
+
+constexpr int kWaves = 8;  // two workgroups to a CU: tiles that are no multiple of the CUs even out
+constexpr int kBatch = 4;  // steps asked for at once
+
+constexpr unsigned kMaxParts = 1024, kMaxGroups = 4, kNoSlot = ~0u, kSlots = 8;  // kMaxParts: tiles x splits of a product
+constexpr unsigned kSlotTiles = kMaxParts * kMaxGroups, kSlotFloats = 256 * kSlotTiles;
+__device__ float skinnyPartials[(size_t)kSlots * kSlotFloats];
+__device__ unsigned skinnyCounts[kSlots * kSlotTiles];  // zero between launches: the workgroup that arrives last sees to it
+StreamSlots gSlots(kSlots);
+
+// Whether a product takes this kernel, and over how many workgroups a tile's K is split: from the sizes of one product
+// alone, so that it is summed the same way alone, in a group and with B transposed.  Nanoseconds as measured, launch aside:
+// a CU takes 2.8 per k of every tile it has; arriving and adding up costs 1300 and 200 more per split; the 32-row tiles with
+// four K groups take 5.1 per k while there is one for each CU.  (The line stands at 4.6, so that what is in doubt stays
+// where it was.)  Splits of less than 512 k end before their loads have paid for the arrival: 2048 -> 512 with 9 rows, 7.4
+// us in splits of 256 against 6.2.  Below 256 k nothing is split in the tiled kernels either, and a product keeps their
+// bits, which are those it has in a batch.
+struct Plan { unsigned splits; bool better; };
+Plan plan_of(unsigned m, unsigned n, unsigned k) {
+  const unsigned long long tiles = (unsigned long long)((m + 15) / 16) * ((n + 15) / 16);
+  if (m <= 8 || k < 256 || tiles > kMaxParts) return Plan{1, false};
+  Plan best{1, false};
+  unsigned long long bestCost = ~0ull;
+  for (unsigned s = 1; s == 1 || (s <= k / 512 && tiles * s <= kMaxParts); ++s) {
+    const unsigned long long perCu = (tiles * s + 255) / 256;
+    const unsigned long long cost = perCu * k * 28 / s + (s > 1 ? 13000 + 2000 * s : 0);
+    if (cost < bestCost) {
+      best.splits = s;
+      bestCost = cost;
+    }
+  }
+  best.better = bestCost < (unsigned long long)k * 46;
+  return best;
+}
+
+template <bool TRANSB>
+__global__ __launch_bounds__(64 * kWaves, 4) void sgemm_skinny_kernel(const float* hotA, const float* hotB, unsigned M,
+                                                                      unsigned N, unsigned K, unsigned lda, unsigned ldb,
+                                                                      unsigned tilesM, unsigned tilesTotal, unsigned chunk,
+                                                                      unsigned splits, unsigned slot, const SgemmParams p) {
+  __shared__ float part[kWaves][4][64];
+  __shared__ unsigned arrived;
+  const unsigned lane = threadIdx.x & 63;
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // each XCD gets a contiguous run of tiles, the row tiles of a column tile side by side: they read the same piece of B
+  const unsigned L = (blockIdx.x & 7u) * chunk + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= chunk || L >= tilesTotal) return;
+  const unsigned tn = L / tilesM, tm = L - tn * tilesM, group = blockIdx.y;
+  const unsigned m0 = tm * 16, n0 = tn * 16;
+  const float* A = hotA;
+  const float* B = p.groups ? p.groupB[group] : hotB;
+
+  // rows and columns past the edge read the last one, and their sums are dropped
+  const unsigned g = lane >> 4, edge = lane & 15u;
+  const unsigned row = min(m0 + edge, M - 1), col = min(n0 + edge, N - 1);
+  const unsigned aOff = (row * lda + 4 * g) * 4u;
+  unsigned bOff = (TRANSB ? col * ldb + 4 * g : 4 * g * ldb + col) * 4u;
+  struct Ops { float a[4], b[4]; };
+  asm volatile("" : "+v"(bOff));
+  // (the step's part of an address is the wavefront's, the lane's part one register)
+  auto at = [](const float* base, unsigned long long uniform, unsigned byte) __attribute__((always_inline)) {
+    return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base + uniform) + byte);
+  };
+  auto load = [&](Ops& o, unsigned step) __attribute__((always_inline)) {
+    __builtin_memcpy(o.a, at(A, step * 16u, aOff), 16);
+    if (TRANSB) {
+      __builtin_memcpy(o.b, at(B, step * 16u, bOff), 16);
+    } else {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) o.b[s] = *at(B, (unsigned long long)(step * 16u + s) * ldb, bOff);
+    }
+  };
+  const unsigned whole = K / 16, lanes = splits * kWaves;  // wavefronts that share the tile
+  const bool alone = slot == kNoSlot;
+  Ops ops[2][kBatch];
+  auto loadBatch = [&](int which, unsigned step) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      if (step + u * lanes < whole) load(ops[which][u], step + u * lanes);
+  };
+  const unsigned stride = kBatch * lanes;
+  const unsigned firstSplit = alone ? 0u : blockIdx.z, lastSplit = alone ? splits - 1 : blockIdx.z;
+  loadBatch(0, firstSplit * kWaves + wave);
+  loadBatch(1, firstSplit * kWaves + wave + stride);
+
+  // what the finish needs: thread t of the first 256 finishes value t / 64
+  const unsigned fe = (threadIdx.x >> 6) & 3u, grow = m0 + 4 * g + fe, gcol = n0 + edge;
+  const bool finisher = threadIdx.x < 256, mine = finisher && grow < M && gcol < N;
+  const float* bias = p.groups ? p.groupBias[group] : p.bias;
+  float bv = 0.f, rv = 0.f;
+  if (mine && bias) bv = bias[gcol];
+  if (mine && p.residual) rv = p.residual[(size_t)grow * N + gcol];
+
+  float v = 0.f;
+  for (unsigned split = firstSplit;; ++split) {
+    skinny_v4f acc = skinny_v4f{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const Ops& o) __attribute__((always_inline)) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[s], o.b[s], acc, 0, 0, 0);
+    };
+    auto multiplyBatch = [&](int which, unsigned step) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u)
+        if (step + u * lanes < whole) multiply(ops[which][u]);
+    };
+    const unsigned first = split * kWaves + wave;
+    for (unsigned step = first; step < whole; step += 2 * stride) {
+      multiplyBatch(0, step);
+      loadBatch(0, step + 2 * stride);
+      multiplyBatch(1, step + stride);
+      loadBatch(1, step + 3 * stride);
+    }
+    if (K % 16 != 0 && first == whole % lanes) {  // the step in which K ends
+      Ops o;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const bool in = whole * 16 + 4 * g + s < K;
+        o.a[s] = in ? *at(A, whole * 16u + s, aOff) : 0.f;
+        o.b[s] = in ? *at(B, TRANSB ? whole * 16u + s : (unsigned long long)(whole * 16u + s) * ldb, bOff) : 0.f;
+      }
+      multiply(o);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) part[wave][e][lane] = acc[e];
+    __syncthreads();
+    float sum = 0.f;
+    if (finisher) {
+      sum = part[0][fe][lane];
+#pragma unroll
+      for (int w = 1; w < kWaves; ++w) sum += part[w][fe][lane];
+    }
+    v = split == firstSplit ? sum : v + sum;
+    if (split == lastSplit) break;
+    __syncthreads();
+    loadBatch(0, first + kWaves);
+    loadBatch(1, first + kWaves + stride);
+  }
+
+  if (!alone && splits > 1) {
+    // The partial tile goes past the caches, and waiting for the store is all the order there has to be in front of the
+    // count; the workgroup that arrives last adds the partial tiles in the order of the splits.
+    const unsigned tile = group * tilesTotal + L;
+    float* mineAt = skinnyPartials + (size_t)slot * kSlotFloats + (size_t)tile * splits * 256;
+    unsigned* count = skinnyCounts + slot * kSlotTiles + tile;
+    if (finisher) __hip_atomic_store(mineAt + blockIdx.z * 256 + threadIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) arrived = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (arrived != splits - 1) return;
+    if (threadIdx.x == 0) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (finisher) {
+      v = __hip_atomic_load(mineAt + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (unsigned s = 1; s < splits; ++s)
+        v += __hip_atomic_load(mineAt + s * 256 + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  if (!mine) return;
+  v += bv;
+  if (p.residual) v += rv;
+  if (p.act == 1) v = gelu_erf_f32(v);
+  float* C = p.groups ? p.groupC[group] : p.C;
+  C[(size_t)grow * p.ldc + gcol] = v;
+}
+
+template <bool TRANSB>
+int launch_skinny(hipStream_t stream, SgemmParams p) {
+  const unsigned groups = p.groups ? p.groups : 1u;
+  p.batch = 1;
+  if (!sgemm_detail::set_tiles(p, 16, 16)) return set_error(TFCC_ROCM_INVALID_ARGUMENT, "sgemm: too many tiles");
+  const unsigned splits = plan_of(p.M, p.N, p.K).splits;
+  unsigned slot = kNoSlot;
+  int dev = 0;
+  if (splits > 1) {
+    TFCC_HIP_CHECK(hipGetDevice(&dev));
+    if (!gSlots.of(dev, stream, &slot)) slot = kNoSlot;
+  }
+  hipLaunchKernelGGL((sgemm_skinny_kernel<TRANSB>), dim3(p.chunk * 8, groups, slot == kNoSlot ? 1u : splits), dim3(64 * kWaves),
+                     0, stream, p.A, p.B, (unsigned)p.M, (unsigned)p.N, (unsigned)p.K, (unsigned)p.lda, (unsigned)p.ldb,
+                     p.tilesM, p.tilesTotal, p.chunk, splits, slot, p);
+  return check_launch("sgemm");
+}
+
+}  // namespace
+
+namespace sgemm_detail {
+
+bool sgemm_skinny_better(unsigned m, unsigned n, unsigned k) { return plan_of(m, n, k).better; }
+
+int sgemm_skinny_launch(hipStream_t stream, const SgemmParams& p, bool transB) {
+  return transB ? launch_skinny<true>(stream, p) : launch_skinny<false>(stream, p);
+}
+
+void sgemm_skinny_release_stream(int dev, hipStream_t stream) { gSlots.release(dev, stream); }
+
+}  // namespace sgemm_detail
+}  // namespace tfcc_rocm
