@@ -9,7 +9,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 # m, k, n
-SHAPES = [(9, 256, 1), (9, 257, 17), (16, 271, 16), (17, 272, 15), (9, 300, 130), (33, 511, 31), (64, 768, 768),
+SHAPES = [(1, 257, 3), (1, 3072, 768), (2, 1001, 1237), (4, 8192, 300), (5, 2048, 130), (8, 1537, 512), (9, 256, 1), (9, 257, 17), (16, 271, 16), (17, 272, 15), (9, 300, 130), (33, 511, 31), (64, 768, 768),
           (29, 1023, 1237), (9, 1024, 64), (16, 1537, 33), (48, 3072, 768), (31, 3079, 770), (9, 8192, 300), (200, 8191, 20),
           (2000, 300, 5), (15, 2560, 4096), (256, 288, 256)]
 
@@ -48,7 +48,7 @@ def test_few_rows(pkg, T, m, k, n):
         assert np.array_equal(T.n(captured), got)
 
 
-@pytest.mark.parametrize("m,k,n", [(29, 768, 130), (9, 2050, 64), (40, 3072, 257)])
+@pytest.mark.parametrize("m,k,n", [(3, 1001, 65), (8, 4096, 300), (29, 768, 130), (9, 2050, 64), (40, 3072, 257)])
 def test_few_rows_transposed_with_residual_and_gelu(pkg, T, m, k, n):
     a, b, bias = _operands(m, k, n)
     r = np.random.default_rng(1).normal(0, 1, (m, n)).astype(np.float32)

@@ -474,8 +474,8 @@ int k_groups_of_plain_product(unsigned m, unsigned n, unsigned k, unsigned fillB
 // count towards filling the chip (`fillBatch`), and launches.
 int dispatch(hipStream_t s, const SgemmParams& p, bool vec, bool small, bool tb, unsigned fillBatch) {
   const unsigned m = p.M, n = p.N, k = p.K;
-  // One product, or a few that share A, of more rows than the streaming kernel takes but too few for its tiles to occupy
-  // the chip.  (A true batch keeps the tiled kernels, see below.)
+  // One product, or a few that share A, of too few rows and columns for the kernels below to occupy the chip.  (A true
+  // batch keeps the tiled kernels, see below.)
   if (fillBatch == 1 && small && sgemm_detail::sgemm_skinny_better(m, n, k))
     return sgemm_detail::sgemm_skinny_launch(s, p, tb);
   if (tb) {

@@ -8,14 +8,16 @@
 // row of A in one load and the same four k of its column of B, with two batches of four steps under way.  Bound by what a
 // CU can have on its way from memory.  (Tiles of 16 x 32, whole lines of B, take twice as long: half the workgroups.)
 //
-// With weights from memory, against the tiles of 32 rows: 32 x 3072 x 768 19.6 -> 8.6 us, 9 x 4096 x 1024 24.3 -> 8.2,
+// With weights from memory, against the kernel that streams B under up to eight rows: 1 x 1001 x 1237 12.2 -> 5.1 us,
+// 8 x 3072 x 768 11.1 -> 6.9, 1 x 8192 x 2048 34 -> 20; and against the tiles of 32 rows: 32 x 3072 x 768 19.6 -> 8.6 us, 9 x 4096 x 1024 24.3 -> 8.2,
 // 16 x 8192 x 2048 70 -> 26, 64 x 8192 x 300 50 -> 13, 32 x 768 x 768 6.3 -> 4.7, 48 x 1001 x 1237 8.2 -> 5.9.
 //
 // An element is the sum of its wavefronts' partial sums, added in the order of the wavefronts, then of the splits;
-// wavefront w of W has the steps w, w + W, ... in ascending order.  The shorter chains leave half the error (3072 k: 2e-7
-// against 5e-7).  B transposed and B as stored give the same bits, and so does a launch that may not use the memory in
-// which the splits meet: its workgroups play all splits one after the other.  Bias, residual and the erf-form GELU follow
-// as in the other kernels (tfcc/mkl/interfaces/tfcc_mklblasinterface.cpp:41-67, 69-78, 87-118).
+// wavefront w of W has the steps w, w + W, ..., dealt in ascending order to four accumulators.  The short chains leave less
+// error against float64 than both other kernels (3072 k: 1.2e-7 against 2.0e-7 and 5.0e-7).  B transposed and B as stored
+// give the same bits, and so does a launch that may not use the memory in which the splits meet: its workgroups play all
+// splits one after the other.  Bias, residual and the erf-form GELU follow as in the other kernels
+// (tfcc/mkl/interfaces/tfcc_mklblasinterface.cpp:41-67, 69-78, 87-118).
 #include "common.hpp"
 #include "sgemm_params.hpp"
 #include "stream_slots.hpp"
@@ -40,13 +42,14 @@ StreamSlots gSlots(kSlots);
 // alone, so that it is summed the same way alone, in a group and with B transposed.  Nanoseconds as measured, launch aside:
 // a CU takes 2.8 per k of every tile it has; arriving and adding up costs 1300 and 200 more per split; the 32-row tiles with
 // four K groups take 5.1 per k while there is one for each CU.  (The line stands at 4.6, so that what is in doubt stays
-// where it was.)  Splits of less than 512 k end before their loads have paid for the arrival: 2048 -> 512 with 9 rows, 7.4
+// where it was.)  Up to eight rows the streaming kernel takes 2.4 to 2.9 per k, whatever N, on one CU for 32 columns, and
+// walks what K has beyond a multiple of 64 row by row, 7000 in all.  Splits of less than 512 k end before their loads have paid for the arrival: 2048 -> 512 with 9 rows, 7.4
 // us in splits of 256 against 6.2.  Below 256 k nothing is split in the tiled kernels either, and a product keeps their
 // bits, which are those it has in a batch.
 struct Plan { unsigned splits; bool better; };
 Plan plan_of(unsigned m, unsigned n, unsigned k) {
   const unsigned long long tiles = (unsigned long long)((m + 15) / 16) * ((n + 15) / 16);
-  if (m <= 8 || k < 256 || tiles > kMaxParts) return Plan{1, false};
+  if (k < 256 || tiles > kMaxParts) return Plan{1, false};
   Plan best{1, false};
   unsigned long long bestCost = ~0ull;
   for (unsigned s = 1; s == 1 || (s <= k / 512 && tiles * s <= kMaxParts); ++s) {
@@ -57,7 +60,8 @@ Plan plan_of(unsigned m, unsigned n, unsigned k) {
       bestCost = cost;
     }
   }
-  best.better = bestCost < (unsigned long long)k * 46;
+  const unsigned long long streaming = ((unsigned long long)k * (m <= 4 ? 24 : 29) + (k % 64 != 0 ? 70000 : 0)) * 9 / 10;
+  best.better = bestCost < (m > 8 ? (unsigned long long)k * 46 : streaming);
   return best;
 }
 
@@ -121,15 +125,17 @@ __global__ __launch_bounds__(64 * kWaves, 4) void sgemm_skinny_kernel(const floa
 
   float v = 0.f;
   for (unsigned split = firstSplit;; ++split) {
-    skinny_v4f acc = skinny_v4f{0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](const Ops& o) __attribute__((always_inline)) {
+    skinny_v4f acc[kBatch];  // one for each step of a batch: short chains, for the rounding and for the matrix ops' latency
 #pragma unroll
-      for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[s], o.b[s], acc, 0, 0, 0);
+    for (int u = 0; u < kBatch; ++u) acc[u] = skinny_v4f{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const Ops& o, int u) __attribute__((always_inline)) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[s], o.b[s], acc[u], 0, 0, 0);
     };
     auto multiplyBatch = [&](int which, unsigned step) __attribute__((always_inline)) {
 #pragma unroll
       for (int u = 0; u < kBatch; ++u)
-        if (step + u * lanes < whole) multiply(ops[which][u]);
+        if (step + u * lanes < whole) multiply(ops[which][u], u);
     };
     const unsigned first = split * kWaves + wave;
     for (unsigned step = first; step < whole; step += 2 * stride) {
@@ -146,10 +152,10 @@ __global__ __launch_bounds__(64 * kWaves, 4) void sgemm_skinny_kernel(const floa
         o.a[s] = in ? *at(A, whole * 16u + s, aOff) : 0.f;
         o.b[s] = in ? *at(B, TRANSB ? whole * 16u + s : (unsigned long long)(whole * 16u + s) * ldb, bOff) : 0.f;
       }
-      multiply(o);
+      multiply(o, 0);
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) part[wave][e][lane] = acc[e];
+    for (int e = 0; e < 4; ++e) part[wave][e][lane] = (acc[0][e] + acc[1][e]) + (acc[2][e] + acc[3][e]);
     __syncthreads();
     float sum = 0.f;
     if (finisher) {
