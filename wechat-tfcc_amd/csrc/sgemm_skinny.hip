@@ -9,8 +9,9 @@
 // CU can have on its way from memory.  (Tiles of 16 x 32, whole lines of B, take twice as long: half the workgroups.)
 //
 // With weights from memory, against the kernel that streams B under up to eight rows: 1 x 1001 x 1237 12.2 -> 5.1 us,
-// 8 x 3072 x 768 11.1 -> 6.9, 1 x 8192 x 2048 34 -> 20; and against the tiles of 32 rows: 32 x 3072 x 768 19.6 -> 8.6 us, 9 x 4096 x 1024 24.3 -> 8.2,
-// 16 x 8192 x 2048 70 -> 26, 64 x 8192 x 300 50 -> 13, 32 x 768 x 768 6.3 -> 4.7, 48 x 1001 x 1237 8.2 -> 5.9.
+// 8 x 3072 x 768 11.1 -> 6.9, 1 x 8192 x 2048 34 -> 20; and against the tiles of 32 rows: 32 x 3072 x 768 19.6 -> 8.6,
+// 9 x 4096 x 1024 24.3 -> 8.5, 16 x 8192 x 2048 70 -> 26, 64 x 8192 x 300 50 -> 12.4, 32 x 768 x 768 6.3 -> 4.8,
+// 48 x 1001 x 1237 8.2 -> 5.9.
 //
 // An element is the sum of its wavefronts' partial sums, added in the order of the wavefronts, then of the splits;
 // wavefront w of W has the steps w, w + W, ..., dealt in ascending order to four accumulators.  The short chains leave less

@@ -18,7 +18,11 @@ class StreamSlots {
   bool of(int dev, hipStream_t stream, unsigned* slot) {
     if (stream == hipStreamPerThread) return false;  // one handle, a stream per thread
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return false;
+    if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) {  // the null stream beside a capture
+      (void)hipGetLastError();
+      return false;
+    }
+    if (capturing != hipStreamCaptureStatusNone) return false;
     std::lock_guard<std::mutex> lock(mutex_);
     const auto found = given_.find({dev, stream});
     if (found != given_.end()) {
