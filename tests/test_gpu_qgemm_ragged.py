@@ -18,6 +18,8 @@ SHAPES = [
     (513, 1023, 1025, 1), (1000, 500, 2001, 1), (515, 257, 1030, 1), (100, 300, 200, 40),                        # 64 x 128, two K groups
     (1344, 959, 1948, 1), (2000, 400, 1999, 1),                                                                  # 128 x 128, two K groups
     (2000, 64, 2001, 1), (3000, 200, 3001, 1), (130, 100, 131, 70), (3584, 130, 3585, 1),                        # one K group
+    (4, 65, 1, 1), (16, 66, 1, 1), (9, 67, 1, 1), (40, 129, 1, 1), (300, 130, 1, 1), (2049, 193, 1, 1), (5, 257, 1, 1),  # one column
+    (3, 65, 2, 1), (7, 66, 3, 1), (33, 130, 2, 3), (4000, 65, 1, 1), (40, 130, 1, 40), (8, 4097, 1, 1),
     (256, 1024, 1024, 1), (32, 512, 4096, 1), (64, 64, 64, 6), (520, 512, 1024, 1),                              # aligned, both sides of the line
 ]
 
@@ -58,7 +60,8 @@ def test_ragged_quantized_products(pkg, T, m, k, n, batch):
             assert acc is None or np.array_equal(T.n(acc), want)
 
 
-@pytest.mark.parametrize("m,k,n", [(1, 1, 1), (2, 7, 5), (8, 2153, 897), (3, 1001, 12), (5, 64, 66), (7, 4095, 130), (8, 700, 3001)])
+@pytest.mark.parametrize("m,k,n", [(1, 1, 1), (2, 7, 5), (8, 2153, 897), (3, 1001, 12), (5, 64, 66), (7, 4095, 130), (8, 700, 3001),
+                                   (1, 65, 1), (4, 66, 1), (8, 129, 1), (3, 1025, 1), (2, 4098, 1), (5, 67, 1), (6, 130, 2)])
 def test_ragged_skinny_product_dequantized(pkg, T, m, k, n):
     rng = np.random.default_rng(m + k + n)
     a = rng.integers(0, 256, (m, k), dtype=np.uint8)

@@ -134,8 +134,10 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmPara
   int colsum[4] = {0, 0, 0, 0};
 
   // Every load is moved back far enough to end inside its operand.  That changes the bytes only of what crosses the end
-  // or lies behind it, which happens in the step in which K ends (and in the one behind it that evens out a pair): those
-  // are put right there.  (Rows of A past M and columns of B past N hold whatever they hold: they are not stored.)
+  // or lies behind it, and those are put right.  For A that is the step in which K ends (and the one behind it that evens
+  // out a pair).  A load of B crosses the end from the last three rows on if N is 1, from the last row on otherwise, so
+  // the step that holds row K - 3 counts too: with K = 64 i + 1 or 64 i + 2 it is the step before.  (Rows of A past M and
+  // columns of B past N hold whatever they hold: they are not stored.)
   const unsigned lastA = sizeA - 16, lastB = sizeB - 4;
   if (wave == WORKERS) prepare();
   else for (unsigned s = wave; s < steps; s += 2 * WORKERS) {
@@ -153,7 +155,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmPara
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const unsigned step = s + u * WORKERS;
-      if (step + 1 >= steps) {
+      if ((step + 1) * 64 + 3 > K) {
         unsigned ka = offA + step * 64, kb = offB + step * 64 * N;
         asm volatile("" : "+v"(ka), "+v"(kb));  // worked out again, instead of keeping every load's offset in a register
 #pragma unroll
