@@ -20,6 +20,8 @@ SHAPES = [
     (2000, 64, 2001, 1), (3000, 200, 3001, 1), (130, 100, 131, 70), (3584, 130, 3585, 1),                        # one K group
     (4, 65, 1, 1), (16, 66, 1, 1), (9, 67, 1, 1), (40, 129, 1, 1), (300, 130, 1, 1), (2049, 193, 1, 1), (5, 257, 1, 1),  # one column
     (3, 65, 2, 1), (7, 66, 3, 1), (33, 130, 2, 3), (4000, 65, 1, 1), (40, 130, 1, 40), (8, 4097, 1, 1),
+    (5000, 129, 1, 1), (5000, 258, 1, 1), (40, 130, 1, 70), (33000, 385, 1, 1), (5000, 131, 1, 1), (5000, 130, 3, 1),  # in slabs
+    (100000, 129, 1, 1), (40, 257, 2, 800),
     (256, 1024, 1024, 1), (32, 512, 4096, 1), (64, 64, 64, 6), (520, 512, 1024, 1),                              # aligned, both sides of the line
 ]
 

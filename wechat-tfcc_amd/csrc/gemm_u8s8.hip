@@ -128,8 +128,9 @@ __global__ __launch_bounds__(kThreads * KSPLIT) void qgemm_kernel(const QGemmPar
   // returns zero without a branch.  Bytes of A beyond K inside a row and columns of B beyond N read neighbouring data;
   // they only ever meet zero B rows or columns that are never stored.  A load may have any byte address; what its range
   // check cannot do is return the valid bytes of one that crosses the end of the operand.  So every load is moved back
-  // to end inside the operand, and in the slab in which K ends, where that can have changed something, the bytes are
-  // shifted to their places (1344 x 959 x 1948: 20 us against 120 when ragged operands were read byte by byte).
+  // to end inside the operand, and where that can have changed something - for A in the slab in which K ends, for B in
+  // every slab that reaches row K - 3, because with N = 1 the last three rows start too close to the end - the bytes
+  // are shifted to their places (1344 x 959 x 1948: 20 us against 120 when ragged operands were read byte by byte).
   const unsigned sizeA = M * K, sizeB = K * N, lastA = sizeA - 16, lastB = sizeB - 4;
   const __amdgpu_buffer_rsrc_t rsrcA =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(A), 0, (int)sizeA, 0x00020000);
@@ -163,7 +164,7 @@ __global__ __launch_bounds__(kThreads * KSPLIT) void qgemm_kernel(const QGemmPar
       for (int q = 0; q < 16; ++q)
         bReg[it][q] = __builtin_amdgcn_raw_buffer_load_b32(rsrcB, min(at + q * N, lastB), 0, 0);
     }
-    if (k0 + BK >= K) {
+    if (k0 + BK + 3 > K) {
       asm volatile("" ::: "memory");
 #pragma unroll
       for (int it = 0; it < B_ITEMS; ++it) {
