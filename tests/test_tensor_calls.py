@@ -82,3 +82,27 @@ def test_what_is_not_plain_is_left_to_the_python_form(pkg, dev):
         pkg.blas_matmul(x.double(), w)
     with pytest.raises(pkg.InvalidArgumentError):
         pkg.reduce_sum(a[:0], True)
+
+
+@pytest.mark.gpu
+def test_tensors_without_memory_raise(pkg, dev):
+    import torch
+    f, a, b = operands(torch, 8, 32, 24)
+    x3, w, one = f(3, 8, 32), f(32, 24), torch.tensor([1.0], device="cuda")
+    seen = []
+
+    def mapped(call):
+        def inner(t):
+            seen.append(call(pkg._native(), t))
+            return t
+        return inner
+
+    for x, call in ((x3, lambda n, t: n.blas_matmul(t, w, None)), (x3, lambda n, t: n.quantize(t, torch.uint8)),
+                    (a.expand(3, 8, 32).contiguous(), lambda n, t: n.reduce_sum(t, True)),
+                    (torch.ones((3, 8), dtype=torch.int32, device="cuda"), lambda n, t: n.dequantize(t, one, one))):
+        torch.vmap(mapped(call))(x)  # the compiled form declines
+    assert seen == [None] * 4
+    for x, call in ((x3, lambda t: pkg.blas_matmul(t, w)), (x3, lambda t: pkg.quantize(t, torch.uint8)[0])):
+        with pytest.raises(RuntimeError):  # and the Python form raises, as it cannot have their address
+            torch.vmap(call)(x)
+    assert torch.allclose(pkg.blas_matmul(x3, w), torch.matmul(x3, w), rtol=1e-5, atol=1e-4)  # and nothing is left behind

@@ -18,11 +18,12 @@ namespace {
 
 using at::Tensor;
 
-// The caller keeps the reference; nullptr: not a tensor this module takes.
+// The caller keeps the reference; nullptr: not a tensor this module takes (one without memory of its own, as inside
+// torch.func transforms, is none).
 const Tensor* plain(PyObject* o, at::ScalarType type, c10::DeviceIndex device) {
   if (!THPVariable_CheckExact(o)) return nullptr;
   const Tensor& t = THPVariable_Unpack(o);
-  if (!t.is_cuda() || t.layout() != at::kStrided || t.scalar_type() != type || t.get_device() != device || !t.is_contiguous()) return nullptr;
+  if (!t.is_cuda() || !t.has_storage() || t.layout() != at::kStrided || t.scalar_type() != type || t.get_device() != device || !t.is_contiguous()) return nullptr;
   return &t;
 }
 
@@ -53,14 +54,16 @@ struct Here {
   void* stream() const { return c10::hip::getCurrentHIPStream(device).stream(); }
 };
 
-// the launch itself runs without the interpreter lock, as through ctypes
+// The launch itself runs without the interpreter lock, as through ctypes.  What is thrown on the way - a data pointer
+// that cannot be had, memory of the library's own bookkeeping - becomes a Python error only with the lock held again.
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
 template <class F>
 int launch(F&& f) {
-  int status;
-  Py_BEGIN_ALLOW_THREADS
-  status = f();
-  Py_END_ALLOW_THREADS
-  return status;
+  Unlocked unlocked;
+  return f();
 }
 
 PyObject* wrap(Tensor t) { return THPVariable_Wrap(std::move(t)); }
