@@ -499,13 +499,15 @@ __global__ __launch_bounds__(256) void minmax_kernel(const float* in, size_t tot
 // The same reduction without atomics on the result, in one launch: every workgroup leaves its minimum and maximum in the
 // (not yet written) output buffer of the quantize call, and the workgroup that arrives last reduces those.  65536 atomics
 // on two words took 380 us for 16.7 M floats; this takes the time of reading them once.  A launch more for the last step
-// cost 3.7 us of the host's time and 1.8 us on the device.
+// cost 3.7 us of the host's time and 1.8 us on the device; a call that may not count on a word of its stream's (a graph
+// being recorded) makes it (131073 elements 7.1 us in a replay, 16.7 M 33; with the atomics 15 and 400).
 constexpr unsigned kArrivalSlots = 1024, kArrivalPitch = 16;
 __device__ unsigned arrivals[kArrivalSlots * kArrivalPitch];  // zero between launches: the last workgroup sees to it
 
-__global__ __launch_bounds__(1024) void minmax_arrival_kernel(const float* in, size_t total, float* partials, unsigned slot,
-                                                             float* mnOut, float* mxOut) {
-  __shared__ float shMn[16], shMx[16];
+template <int WAVES, bool COUNTED>
+__global__ __launch_bounds__(64 * WAVES) void minmax_partial_kernel(const float* in, size_t total, float* partials,
+                                                                    unsigned slot, float* mnOut, float* mxOut) {
+  __shared__ float shMn[WAVES], shMx[WAVES];
   __shared__ unsigned last;
   const size_t total4 = total / 4, step = (size_t)gridDim.x * blockDim.x;
   const float4* in4 = reinterpret_cast<const float4*>(in);
@@ -539,12 +541,19 @@ __global__ __launch_bounds__(1024) void minmax_arrival_kernel(const float* in, s
     }
     __syncthreads();
 #pragma unroll
-    for (int w = 0; w < 16; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       mn = fminf(mn, shMn[w]);
       mx = fmaxf(mx, shMx[w]);
     }
   };
   join();
+  if constexpr (!COUNTED) {
+    if (threadIdx.x == 0) {
+      partials[2 * blockIdx.x] = mn;
+      partials[2 * blockIdx.x + 1] = mx;
+    }
+    return;
+  }
   if (threadIdx.x == 0) {
     __hip_atomic_store(partials + 2 * blockIdx.x, mn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(partials + 2 * blockIdx.x + 1, mx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -556,7 +565,7 @@ __global__ __launch_bounds__(1024) void minmax_arrival_kernel(const float* in, s
   }
   __syncthreads();
   if (!last) return;
-  for (unsigned i = threadIdx.x; i < gridDim.x; i += 1024) {
+  for (unsigned i = threadIdx.x; i < gridDim.x; i += 64 * WAVES) {
     mn = fminf(mn, __hip_atomic_load(partials + 2 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     mx = fmaxf(mx, __hip_atomic_load(partials + 2 * i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
   }
@@ -565,6 +574,30 @@ __global__ __launch_bounds__(1024) void minmax_arrival_kernel(const float* in, s
     *mnOut = mn;
     *mxOut = mx;
     __hip_atomic_store(arrivals + slot * kArrivalPitch, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// The last step as a launch of its own.
+__global__ __launch_bounds__(256) void minmax_final_kernel(const float* partials, unsigned blocks, float* mnOut, float* mxOut) {
+  __shared__ float shMn[4], shMx[4];
+  float mn = 3.402823466e+38f, mx = -3.402823466e+38f;
+  for (unsigned i = threadIdx.x; i < blocks; i += 256) {
+    mn = fminf(mn, partials[2 * i]);
+    mx = fmaxf(mx, partials[2 * i + 1]);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    mn = fminf(mn, __shfl_down(mn, off, 64));
+    mx = fmaxf(mx, __shfl_down(mx, off, 64));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    shMn[threadIdx.x >> 6] = mn;
+    shMx[threadIdx.x >> 6] = mx;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    *mnOut = fminf(fminf(shMn[0], shMn[1]), fminf(shMn[2], shMn[3]));
+    *mxOut = fmaxf(fmaxf(shMx[0], shMx[1]), fmaxf(shMx[2], shMx[3]));
   }
 }
 
@@ -580,16 +613,19 @@ unsigned grid_for(size_t total, unsigned perThread = 1) {
   return (unsigned)blocks;
 }
 
-// the vector kernels: four 16-byte loads per thread per pass, at most 8 workgroups per CU
+// The vector kernels: four 16-byte loads per thread per pass, at most 8 workgroups per CU; one load per thread while that
+// still leaves CUs without work (131073 elements quantized: 32 workgroups against 129).
 unsigned stream_grid(size_t total4) {
   size_t blocks = (total4 + 1023) / 1024;
+  const size_t spread = (total4 + 255) / 256;
+  if (blocks < 256) blocks = spread < 256 ? spread : 256;
   if (blocks > 256u * 8u) blocks = 256u * 8u;
   if (blocks < 1) blocks = 1;
   return (unsigned)blocks;
 }
 
-// The word on which a stream's range reductions count their workgroups; calls that get none take the form with atomics on
-// the result.
+// The word on which a stream's range reductions count their workgroups; calls that get none reduce the partial results in a
+// launch of its own.
 StreamSlots gArrivalSlots(kArrivalSlots);
 
 bool valid_type(int t) { return t >= TFCC_ROCM_S8 && t <= TFCC_ROCM_U32; }
@@ -752,16 +788,24 @@ int tfcc_rocm_quantize_minmax(void* stream, const float* in, uint64_t total, voi
   }
   unsigned* mnWord = reinterpret_cast<unsigned*>(min_v);
   unsigned* mxWord = reinterpret_cast<unsigned*>(max_v);
-  // one workgroup per CU at most: every arrival costs an atomic on one word and a write-back (192 workgroups of 256
-  // threads for 786432 elements: 6 us, 48 of 1024: 5.6)
-  const unsigned blocks = total >= 256u * 16384u ? 256u : (unsigned)((total + 16383) / 16384);
   int dev = 0;
   unsigned slot = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));
-  if ((uintptr_t)in % 16 == 0 && (uintptr_t)out % 4 == 0 && gArrivalSlots.of(dev, s, &slot)) {
-    // partial results, eight bytes per 4096 elements, rest in the output buffer until the quantize pass overwrites it
-    hipLaunchKernelGGL(minmax_arrival_kernel, dim3(blocks), dim3(1024), 0, s, in, (size_t)total, static_cast<float*>(out), slot,
-                       min_v, max_v);
+  if ((uintptr_t)in % 16 == 0 && (uintptr_t)out % 4 == 0) {
+    // partial results, eight bytes per workgroup, rest in the output buffer until the quantize pass overwrites it
+    float* partials = static_cast<float*>(out);
+    if (gArrivalSlots.of(dev, s, &slot)) {
+      // one workgroup per CU at most: every arrival costs an atomic on one word and a write-back (192 workgroups of 256
+      // threads for 786432 elements: 6 us, 48 of 1024: 5.6)
+      const unsigned blocks = total >= 256u * 16384u ? 256u : (unsigned)((total + 16383) / 16384);
+      hipLaunchKernelGGL((minmax_partial_kernel<16, true>), dim3(blocks), dim3(1024), 0, s, in, (size_t)total, partials, slot,
+                         min_v, max_v);
+    } else {
+      const unsigned blocks = stream_grid(total / 4);
+      hipLaunchKernelGGL((minmax_partial_kernel<4, false>), dim3(blocks), dim3(256), 0, s, in, (size_t)total, partials, 0u,
+                         nullptr, nullptr);
+      hipLaunchKernelGGL(minmax_final_kernel, dim3(1), dim3(256), 0, s, partials, blocks, min_v, max_v);
+    }
   } else {
     hipLaunchKernelGGL(minmax_init_kernel, dim3(1), dim3(1), 0, s, mnWord, mxWord);
     hipLaunchKernelGGL(minmax_kernel, dim3(grid_for(total, 4)), dim3(256), 0, s, in, (size_t)total, mnWord, mxWord);
