@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 # m, k, n
 SHAPES = [(1, 257, 3), (1, 3072, 768), (2, 1001, 1237), (4, 8192, 300), (5, 2048, 130), (8, 1537, 512), (9, 256, 1), (9, 257, 17), (16, 271, 16), (17, 272, 15), (9, 300, 130), (33, 511, 31), (64, 768, 768),
           (29, 1023, 1237), (9, 1024, 64), (16, 1537, 33), (48, 3072, 768), (31, 3079, 770), (9, 8192, 300), (200, 8191, 20),
-          (2000, 300, 5), (15, 2560, 4096), (256, 288, 256)]
+          (2000, 300, 5), (15, 2560, 4096), (256, 288, 256),
+          (1, 1024, 16), (3, 1040, 33), (2, 16384 + 13, 64), (1, 65536, 16), (7, 5133, 20), (20, 2047, 40), (12, 3600, 96)]  # 2 to 64 splits
 
 
 def _within_bound(got, a, b, bias=None):
@@ -83,3 +84,41 @@ def test_few_rows_on_many_streams(pkg, T):
     torch.cuda.synchronize()
     for o in outs:
         assert np.array_equal(T.n(o), want)
+
+
+def test_few_rows_in_a_group_under_capture(pkg, T):
+    import torch
+    a, _, _ = _operands(12, 4100, 64)
+    ta = T.t(a)
+    rng = np.random.default_rng(2)
+    bs, biases = ([T.t(rng.normal(0, 1, s).astype(np.float32)) for _ in range(3)] for s in ((4100, 64), (64,)))
+    eager, graph = pkg.sgemm_grouped(ta, bs, biases), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        captured = pkg.sgemm_grouped(ta, bs, biases)
+    for _ in range(3):
+        for c in captured:
+            c.zero_()
+        graph.replay()
+        for c, e, b, bias in zip(captured, eager, bs, biases):
+            assert torch.equal(c, e)
+            assert torch.equal(e, pkg.blas_matmul(ta, b, bias))
+
+
+def test_memory_of_a_stream_is_given_back(pkg, T):
+    """more streams, one after the other, than the library gives memory to at once"""
+    import torch
+    lib = pkg.lib()
+    a, b, _ = _operands(24, 4096, 512)
+    ta, tb = T.t(a), T.t(b)
+    want, out = pkg.blas_matmul(ta, tb), T.t(np.zeros((24, 512), np.float32))
+    for _ in range(80):
+        stream = C.c_void_p()
+        pkg.check(lib.tfcc_rocm_stream_create(C.byref(stream)))
+        out.zero_()
+        torch.cuda.synchronize()
+        pkg.check(lib.tfcc_rocm_sgemm_strided_batched(stream, ta.data_ptr(), 0, tb.data_ptr(), 0, None, out.data_ptr(), 0, 24, 512,
+                                                      4096, 1))
+        pkg.check(lib.tfcc_rocm_stream_synchronize(stream))
+        assert np.array_equal(T.n(out), T.n(want))
+        pkg.check(lib.tfcc_rocm_stream_destroy(stream))

@@ -16,9 +16,13 @@
 // An element is the sum of its wavefronts' partial sums, added in the order of the wavefronts, then of the splits;
 // wavefront w of W has the steps w, w + W, ..., dealt in ascending order to four accumulators.  The short chains leave less
 // error against float64 than both other kernels (3072 k: 1.2e-7 against 2.0e-7 and 5.0e-7).  B transposed and B as stored
-// give the same bits, and so does a launch that may not use the memory in which the splits meet: its workgroups play all
-// splits one after the other.  Bias, residual and the erf-form GELU follow as in the other kernels
+// give the same bits, and so does a launch that may not use the memory in which the splits meet (a stream that is being
+// captured): its workgroups, of sixteen wavefronts, have all splits of a tile.  Replayed with weights from memory / in cache,
+// against the streaming kernel: 8 x 3072 x 768 16.9/10.4 -> 17.2/8.8 us, 1 x 8192 x 300 35/20 -> 28/18, 1 x 3072 x 768
+// 14.7/5.9 -> 14.8/8.5, 1 x 16384 x 64, four tiles, 26/20 -> 29/26.  Bias, residual and the erf-form GELU follow as in the other kernels
 // (tfcc/mkl/interfaces/tfcc_mklblasinterface.cpp:41-67, 69-78, 87-118).
+#include <type_traits>
+
 #include "common.hpp"
 #include "sgemm_params.hpp"
 #include "stream_slots.hpp"
@@ -33,19 +37,25 @@ typedef float skinny_v4f __attribute__((ext_vector_type(4)));
 constexpr int kWaves = 8;  // two workgroups to a CU: tiles that are no multiple of the CUs even out
 constexpr int kBatch = 4;  // steps asked for at once
 
-constexpr unsigned kMaxParts = 1024, kMaxGroups = 4, kNoSlot = ~0u, kSlots = 8;  // kMaxParts: tiles x splits of a product
-constexpr unsigned kSlotTiles = kMaxParts * kMaxGroups, kSlotFloats = 256 * kSlotTiles;
-__device__ float skinnyPartials[(size_t)kSlots * kSlotFloats];
-__device__ unsigned skinnyCounts[kSlots * kSlotTiles];  // zero between launches: the workgroup that arrives last sees to it
-StreamSlots gSlots(kSlots);
+// The memory in which the splits of a tile meet: a piece per stream, asked for by the first product that splits.
+constexpr unsigned kMaxParts = 1024, kMaxGroups = 4;  // kMaxParts: tiles x splits of a product
+constexpr unsigned kPieceTiles = kMaxParts * kMaxGroups;
+struct Meeting {
+  float partials[256 * (size_t)kPieceTiles];
+  unsigned counts[kPieceTiles];  // zero between launches: the workgroup that arrives last sees to it
+};
+int clear_counts(hipStream_t stream, void* piece) {
+  return tfcc_rocm_fill_async(stream, static_cast<Meeting*>(piece)->counts, 0, sizeof(unsigned), kPieceTiles);
+}
+StreamPieces gPieces(sizeof(Meeting), 64, clear_counts);  // 4 MB each
 
 // Whether a product takes this kernel, and over how many workgroups a tile's K is split: from the sizes of one product
 // alone, so that it is summed the same way alone, in a group and with B transposed.  Nanoseconds as measured, launch aside:
 // a CU takes 2.8 per k of every tile it has; arriving and adding up costs 1300 and 200 more per split; the 32-row tiles with
 // four K groups take 5.1 per k while there is one for each CU.  (The line stands at 4.6, so that what is in doubt stays
 // where it was.)  Up to eight rows the streaming kernel takes 2.4 to 2.9 per k, whatever N, on one CU for 32 columns, and
-// walks what K has beyond a multiple of 64 row by row, 7000 in all.  Splits of less than 512 k end before their loads have paid for the arrival: 2048 -> 512 with 9 rows, 7.4
-// us in splits of 256 against 6.2.  Below 256 k nothing is split in the tiled kernels either, and a product keeps their
+// walks what K has beyond a multiple of 64 row by row, 7000 in all.  Splits of less than 512 k end before their loads have
+// paid for the arrival: 2048 -> 512 with 9 rows, 7.4 us in splits of 256 against 6.2.  Below 256 k nothing is split in the tiled kernels either, and a product keeps their
 // bits, which are those it has in a batch.
 struct Plan { unsigned splits; bool better; };
 Plan plan_of(unsigned m, unsigned n, unsigned k) {
@@ -66,15 +76,26 @@ Plan plan_of(unsigned m, unsigned n, unsigned k) {
   return best;
 }
 
-template <bool TRANSB>
-__global__ __launch_bounds__(64 * kWaves, 4) void sgemm_skinny_kernel(const float* hotA, const float* hotB, unsigned M,
-                                                                      unsigned N, unsigned K, unsigned lda, unsigned ldb,
-                                                                      unsigned tilesM, unsigned tilesTotal, unsigned chunk,
-                                                                      unsigned splits, unsigned slot, const SgemmParams p) {
-  __shared__ float part[kWaves][4][64];
+// TEAMS teams of eight wavefronts.  One: the workgroup has the split blockIdx.z of its tile and meets the others in `meeting`
+// (null for a product that is not split).  Two, where there is no such memory: the workgroup has all splits, the teams
+// taking turns; a wavefront asks for the first steps of its next split as it ends one, and the partial tiles of six splits
+// wait in LDS before the workgroup meets.
+//
+// What is under way has to be the same on every path to a matrix op, or the compiler waits for every load before it uses the
+// first (with a condition in front of every load 1 x 16384 x 64 in a graph took 37 us instead of 26): whole batches are asked for without a condition, and the last 0 to 3 steps of a wavefront have code of their own
+// for each number.
+template <bool TRANSB, int TEAMS>
+__global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(const float* hotA, const float* hotB, unsigned M,
+                                                                              unsigned N, unsigned K, unsigned lda, unsigned ldb,
+                                                                              unsigned tilesM, unsigned tilesTotal, unsigned chunk,
+                                                                              unsigned splits, unsigned perWave, Meeting* meeting,
+                                                                              const SgemmParams p) {
+  constexpr unsigned ROUNDS = TEAMS == 1 ? 1 : 3, HELD = TEAMS * ROUNDS;  // splits that wait in LDS
+  __shared__ float part[HELD * kWaves][4][64];
   __shared__ unsigned arrived;
   const unsigned lane = threadIdx.x & 63;
-  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned waveInGroup = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned team = TEAMS == 1 ? 0u : waveInGroup / kWaves, wave = waveInGroup - team * kWaves;
   // each XCD gets a contiguous run of tiles, the row tiles of a column tile side by side: they read the same piece of B
   const unsigned L = (blockIdx.x & 7u) * chunk + (blockIdx.x >> 3);
   if ((blockIdx.x >> 3) >= chunk || L >= tilesTotal) return;
@@ -82,101 +103,164 @@ __global__ __launch_bounds__(64 * kWaves, 4) void sgemm_skinny_kernel(const floa
   const unsigned m0 = tm * 16, n0 = tn * 16;
   const float* A = hotA;
   const float* B = p.groups ? p.groupB[group] : hotB;
+  // (no range check: every offset below lies inside the operand)
+  const __amdgpu_buffer_rsrc_t rsrcA = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A), 0, -1, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrcB = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), 0, -1, 0x00020000);
 
   // rows and columns past the edge read the last one, and their sums are dropped
   const unsigned g = lane >> 4, edge = lane & 15u;
   const unsigned row = min(m0 + edge, M - 1), col = min(n0 + edge, N - 1);
   const unsigned aOff = (row * lda + 4 * g) * 4u;
-  unsigned bOff = (TRANSB ? col * ldb + 4 * g : 4 * g * ldb + col) * 4u;
+  const unsigned bOff = (TRANSB ? col * ldb + 4 * g : 4 * g * ldb + col) * 4u;
   struct Ops { float a[4], b[4]; };
-  asm volatile("" : "+v"(bOff));
-  // (the step's part of an address is the wavefront's, the lane's part one register)
-  auto at = [](const float* base, unsigned long long uniform, unsigned byte) __attribute__((always_inline)) {
-    return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base + uniform) + byte);
-  };
-  auto load = [&](Ops& o, unsigned step) __attribute__((always_inline)) {
-    __builtin_memcpy(o.a, at(A, step * 16u, aOff), 16);
+  auto load = [&](Ops& o, unsigned k) __attribute__((always_inline)) {
+    const auto a = __builtin_amdgcn_raw_buffer_load_b128(rsrcA, aOff, k * 4u, 0);
+    __builtin_memcpy(o.a, &a, 16);
     if (TRANSB) {
-      __builtin_memcpy(o.b, at(B, step * 16u, bOff), 16);
+      const auto b = __builtin_amdgcn_raw_buffer_load_b128(rsrcB, bOff, k * 4u, 0);
+      __builtin_memcpy(o.b, &b, 16);
     } else {
 #pragma unroll
-      for (int s = 0; s < 4; ++s) o.b[s] = *at(B, (unsigned long long)(step * 16u + s) * ldb, bOff);
+      for (unsigned s = 0; s < 4; ++s)
+        o.b[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrcB, bOff, (k + s) * ldb * 4u, 0));
     }
   };
   const unsigned whole = K / 16, lanes = splits * kWaves;  // wavefronts that share the tile
-  const bool alone = slot == kNoSlot;
   Ops ops[2][kBatch];
-  auto loadBatch = [&](int which, unsigned step) __attribute__((always_inline)) {
+  auto loadSteps = [&](int which, unsigned step, auto steps) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u)
-      if (step + u * lanes < whole) load(ops[which][u], step + u * lanes);
+    for (int u = 0; u < decltype(steps)::value; ++u) load(ops[which][u], (step + u * lanes) * 16u);
   };
-  const unsigned stride = kBatch * lanes;
-  const unsigned firstSplit = alone ? 0u : blockIdx.z, lastSplit = alone ? splits - 1 : blockIdx.z;
-  loadBatch(0, firstSplit * kWaves + wave);
-  loadBatch(1, firstSplit * kWaves + wave + stride);
+  unsigned split = TEAMS == 1 ? blockIdx.z : team;
+  unsigned first = split * kWaves + wave;
 
   // what the finish needs: thread t of the first 256 finishes value t / 64
   const unsigned fe = (threadIdx.x >> 6) & 3u, grow = m0 + 4 * g + fe, gcol = n0 + edge;
   const bool finisher = threadIdx.x < 256, mine = finisher && grow < M && gcol < N;
-  const float* bias = p.groups ? p.groupBias[group] : p.bias;
   float bv = 0.f, rv = 0.f;
-  if (mine && bias) bv = bias[gcol];
-  if (mine && p.residual) rv = p.residual[(size_t)grow * N + gcol];
+  auto loadFinish = [&]() __attribute__((always_inline)) {
+    const float* bias = p.groups ? p.groupBias[group] : p.bias;
+    if (mine && bias) bv = bias[gcol];
+    if (mine && p.residual) rv = p.residual[(size_t)grow * N + gcol];
+  };
 
-  float v = 0.f;
-  for (unsigned split = firstSplit;; ++split) {
-    skinny_v4f acc[kBatch];  // one for each step of a batch: short chains, for the rounding and for the matrix ops' latency
+  skinny_v4f acc[kBatch];  // one for each step of a batch: short chains, for the rounding and for the matrix ops' latency
+  auto multiply = [&](const Ops& o, int u) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[s], o.b[s], acc[u], 0, 0, 0);
+  };
+  auto multiplySteps = [&](int which, auto steps) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < decltype(steps)::value; ++u) multiply(ops[which][u], u);
+  };
+  const std::integral_constant<int, kBatch> batch;
+  auto with = [](unsigned steps, auto f) __attribute__((always_inline)) {  // 0 to 3
+    if (steps < 2) {
+      if (steps == 0) f(std::integral_constant<int, 0>{});
+      else f(std::integral_constant<int, 1>{});
+    } else {
+      if (steps == 2) f(std::integral_constant<int, 2>{});
+      else f(std::integral_constant<int, 3>{});
+    }
+  };
+  // The wavefront's steps of its split: first, first + lanes, ...; perWave of them, or one more.  Whoever shares a tile has
+  // at least four, and a first batch that has been asked for.
+  const unsigned oneMore = whole - perWave * lanes;
+  auto sumSplit = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) acc[u] = skinny_v4f{0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](const Ops& o, int u) __attribute__((always_inline)) {
-#pragma unroll
-      for (int s = 0; s < 4; ++s) acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[s], o.b[s], acc[u], 0, 0, 0);
-    };
-    auto multiplyBatch = [&](int which, unsigned step) __attribute__((always_inline)) {
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u)
-        if (step + u * lanes < whole) multiply(ops[which][u], u);
-    };
-    const unsigned first = split * kWaves + wave;
-    for (unsigned step = first; step < whole; step += 2 * stride) {
-      multiplyBatch(0, step);
-      loadBatch(0, step + 2 * stride);
-      multiplyBatch(1, step + stride);
-      loadBatch(1, step + 3 * stride);
+    const unsigned steps = perWave + (first < oneMore ? 1u : 0u);
+    if (TEAMS == 1 && steps < kBatch) {
+      with(steps, [&](auto few) {
+        loadSteps(0, first, few);
+        if (TEAMS == 1) loadFinish();
+        multiplySteps(0, few);
+      });
+      return;
     }
+    loadSteps(0, first, batch);
+    unsigned left = steps - kBatch, next = first + kBatch * lanes;  // what has not been asked for
+    for (; left >= 2 * kBatch; left -= 2 * kBatch, next += 2 * kBatch * lanes) {
+      loadSteps(1, next, batch);
+      multiplySteps(0, batch);
+      loadSteps(0, next + kBatch * lanes, batch);
+      multiplySteps(1, batch);
+    }
+    if (left >= kBatch) {
+      loadSteps(1, next, batch);
+      multiplySteps(0, batch);
+      with(left - kBatch, [&](auto few) {
+        loadSteps(0, next + kBatch * lanes, few);
+        if (TEAMS == 1) loadFinish();
+        multiplySteps(1, batch);
+        multiplySteps(0, few);
+      });
+    } else {
+      with(left, [&](auto few) {
+        loadSteps(1, next, few);
+        if (TEAMS == 1) loadFinish();
+        multiplySteps(0, batch);
+        multiplySteps(1, few);
+      });
+    }
+  };
+  auto keepSplit = [&](unsigned held) __attribute__((always_inline)) {
     if (K % 16 != 0 && first == whole % lanes) {  // the step in which K ends
       Ops o;
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
+      for (unsigned s = 0; s < 4; ++s) {
         const bool in = whole * 16 + 4 * g + s < K;
-        o.a[s] = in ? *at(A, whole * 16u + s, aOff) : 0.f;
-        o.b[s] = in ? *at(B, TRANSB ? whole * 16u + s : (unsigned long long)(whole * 16u + s) * ldb, bOff) : 0.f;
+        o.a[s] = in ? A[(size_t)row * lda + whole * 16 + 4 * g + s] : 0.f;
+        const size_t k = whole * 16 + 4 * g + s;
+        o.b[s] = in ? B[TRANSB ? (size_t)col * ldb + k : k * ldb + col] : 0.f;
       }
       multiply(o, 0);
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) part[wave][e][lane] = (acc[0][e] + acc[1][e]) + (acc[2][e] + acc[3][e]);
+    for (int e = 0; e < 4; ++e) part[held * kWaves + wave][e][lane] = (acc[0][e] + acc[1][e]) + (acc[2][e] + acc[3][e]);
+  };
+  float v = 0.f;
+  auto meet = [&](unsigned from, unsigned to) __attribute__((always_inline)) {  // adds the held splits from .. to - 1
     __syncthreads();
-    float sum = 0.f;
-    if (finisher) {
-      sum = part[0][fe][lane];
+    if (!finisher) return;
+    for (unsigned s = from; s < to; ++s) {
+      float sum = part[(s - from) * kWaves][fe][lane];
 #pragma unroll
-      for (int w = 1; w < kWaves; ++w) sum += part[w][fe][lane];
+      for (int w = 1; w < kWaves; ++w) sum += part[(s - from) * kWaves + w][fe][lane];
+      v = s == 0 || TEAMS == 1 ? sum : v + sum;
     }
-    v = split == firstSplit ? sum : v + sum;
-    if (split == lastSplit) break;
-    __syncthreads();
-    loadBatch(0, first + kWaves);
-    loadBatch(1, first + kWaves + stride);
+  };
+  if constexpr (TEAMS == 1) {
+    sumSplit();
+    keepSplit(0);
+    meet(split, split + 1);
+  } else {
+    unsigned met = 0;
+    for (;;) {
+      if (split < splits) {
+        sumSplit();
+        if (met == 0 && split == team) loadFinish();
+        keepSplit(split - met);
+      }
+      split += TEAMS;
+      first += TEAMS * kWaves;
+      const unsigned through = split - team;  // every split below it has been summed
+      if (through >= splits || through - met == HELD) {  // the same for the whole workgroup
+        const unsigned to = min(through, splits);
+        meet(met, to);
+        met = to;
+        if (met == splits) break;
+        __syncthreads();
+      }
+    }
   }
 
-  if (!alone && splits > 1) {
+  if (TEAMS == 1 && splits > 1) {
     // The partial tile goes past the caches, and waiting for the store is all the order there has to be in front of the
     // count; the workgroup that arrives last adds the partial tiles in the order of the splits.
     const unsigned tile = group * tilesTotal + L;
-    float* mineAt = skinnyPartials + (size_t)slot * kSlotFloats + (size_t)tile * splits * 256;
-    unsigned* count = skinnyCounts + slot * kSlotTiles + tile;
+    float* mineAt = meeting->partials + (size_t)tile * splits * 256;
+    unsigned* count = meeting->counts + tile;
     if (finisher) __hip_atomic_store(mineAt + blockIdx.z * 256 + threadIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -204,15 +288,17 @@ int launch_skinny(hipStream_t stream, SgemmParams p) {
   p.batch = 1;
   if (!sgemm_detail::set_tiles(p, 16, 16)) return set_error(TFCC_ROCM_INVALID_ARGUMENT, "sgemm: too many tiles");
   const unsigned splits = plan_of(p.M, p.N, p.K).splits;
-  unsigned slot = kNoSlot;
-  int dev = 0;
+  Meeting* meeting = nullptr;
   if (splits > 1) {
+    int dev = 0;
     TFCC_HIP_CHECK(hipGetDevice(&dev));
-    if (!gSlots.of(dev, stream, &slot)) slot = kNoSlot;
+    meeting = static_cast<Meeting*>(gPieces.of(dev, stream));
   }
-  hipLaunchKernelGGL((sgemm_skinny_kernel<TRANSB>), dim3(p.chunk * 8, groups, slot == kNoSlot ? 1u : splits), dim3(64 * kWaves),
-                     0, stream, p.A, p.B, (unsigned)p.M, (unsigned)p.N, (unsigned)p.K, (unsigned)p.lda, (unsigned)p.ldb,
-                     p.tilesM, p.tilesTotal, p.chunk, splits, slot, p);
+  const bool alone = splits > 1 && meeting == nullptr;
+  auto kern = alone ? sgemm_skinny_kernel<TRANSB, 2> : sgemm_skinny_kernel<TRANSB, 1>;
+  hipLaunchKernelGGL(kern, dim3(p.chunk * 8, groups, alone ? 1u : splits), dim3(64 * kWaves * (alone ? 2 : 1)), 0, stream, p.A, p.B,
+                     (unsigned)p.M, (unsigned)p.N, (unsigned)p.K, (unsigned)p.lda, (unsigned)p.ldb, p.tilesM, p.tilesTotal, p.chunk,
+                     splits, p.K / 16 / (splits * kWaves), meeting, p);
   return check_launch("sgemm");
 }
 
@@ -226,7 +312,7 @@ int sgemm_skinny_launch(hipStream_t stream, const SgemmParams& p, bool transB) {
   return transB ? launch_skinny<true>(stream, p) : launch_skinny<false>(stream, p);
 }
 
-void sgemm_skinny_release_stream(int dev, hipStream_t stream) { gSlots.release(dev, stream); }
+void sgemm_skinny_release_stream(int dev, hipStream_t stream) { gPieces.release(dev, stream); }
 
 }  // namespace sgemm_detail
 }  // namespace tfcc_rocm
