@@ -104,3 +104,56 @@ def test_several_threads_and_streams(pkg, T):
     for t in threads:
         t.join()
     assert not errors, errors
+
+
+def test_beside_a_capture_after_the_null_stream(pkg, T):
+    """The null stream may not be asked, waited for or recorded on while a graph is being recorded elsewhere."""
+    import torch
+    x, sets = setup(T, 6, 3, 16, 300, 2)
+    lib, prepared = pkg.lib(), []
+
+    class Held:  # launch() up to the call itself, which comes while the graph is being recorded
+        def __getattr__(self, name):
+            return (lambda stream, d: prepared.append(d) or 0) if name == "tfcc_rocm_lstm_sequence_f32" else getattr(lib, name)
+
+    class Package:
+        LstmSequenceDesc, blas_matmul, check, lib = pkg.LstmSequenceDesc, staticmethod(pkg.blas_matmul), staticmethod(pkg.check), staticmethod(Held)
+
+    runs = [launch(Package, T, x, sets, (False, True)) for _ in range(4)]
+    call, recorded, other, graph = lib.tfcc_rocm_lstm_sequence_f32, C.c_void_p(), C.c_void_p(), C.c_void_p()
+    for stream in (recorded, other):
+        pkg.check(lib.tfcc_rocm_stream_create(C.byref(stream)))
+    status = [call(other, prepared[0]), call(None, prepared[1])]  # the null stream had the last turn
+    torch.cuda.synchronize()
+    t = torch.zeros(64, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    pkg.check(lib.tfcc_rocm_stream_begin_capture(recorded))  # of a stream that the null stream waits for
+    pkg.check(lib.tfcc_rocm_fill_async(recorded, t.data_ptr(), 7, 1, 64))
+    status.append(call(other, prepared[2]))
+    pkg.check(lib.tfcc_rocm_stream_end_capture(recorded, C.byref(graph)))
+    torch.cuda.synchronize()
+    status.append(call(None, prepared[3]))
+    pkg.check(lib.tfcc_rocm_graph_launch(graph, recorded))
+    torch.cuda.synchronize()
+    assert (t == 7).all()
+    pkg.check(lib.tfcc_rocm_graph_destroy(graph))
+    for stream in (recorded, other):
+        pkg.check(lib.tfcc_rocm_stream_destroy(stream))
+    assert status == [0, 0, 0, 0], lib.tfcc_rocm_last_error_string()
+    for outs, keep in runs:
+        compare(T, outs, x, sets, (False, True))
+
+
+def test_after_a_stream_that_is_gone(pkg, T):
+    import torch
+    hip = C.CDLL("libamdhip64.so")
+    x, sets = setup(T, 5, 2, 16, 128, 2)
+    for _ in range(3):
+        raw = C.c_void_p()
+        assert hip.hipStreamCreate(C.byref(raw)) == 0
+        outs, keep = launch(pkg, T, x, sets, (False, True), stream=raw)
+        assert hip.hipStreamSynchronize(raw) == 0 and hip.hipStreamDestroy(raw) == 0  # not through the library
+        compare(T, outs, x, sets, (False, True))
+        outs, keep = launch(pkg, T, x, sets, (False, True))
+        torch.cuda.synchronize()
+        compare(T, outs, x, sets, (False, True))

@@ -5,7 +5,6 @@
 
 #include "common.hpp"
 #include "gemv.hpp"
-#include "lstm_sequence.hpp"
 #include "quant_ops.hpp"
 #include "sgemm_params.hpp"
 
@@ -103,7 +102,6 @@ int tfcc_rocm_stream_create(void** stream) {
 int tfcc_rocm_stream_release(void* stream) {
   // the stream's pending work may still use what is given back
   TFCC_HIP_CHECK(hipStreamSynchronize(as_stream(stream)));
-  tfcc_rocm::lstm_sequence_forget_stream(as_stream(stream));
   if (int e = tfcc_rocm::quantize_release_stream(as_stream(stream))) return e;
   int dev = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));

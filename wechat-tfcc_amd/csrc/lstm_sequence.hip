@@ -21,7 +21,6 @@
 #include <mutex>
 
 #include "common.hpp"
-#include "lstm_sequence.hpp"
 
 namespace tfcc_rocm {
 namespace {
@@ -355,24 +354,30 @@ int launch_rows(hipStream_t stream, const SequenceParams& p) {
   return launch<4, KI, WAVES>(stream, p);
 }
 
+int launch_units(hipStream_t stream, const SequenceParams& p) {
+  // eight wavefronts, so eight units, per workgroup: with four, twice the workgroups poll; with twelve or sixteen, each of
+  // which reads all of h from LDS, that takes longer than the trip to memory (4 x 1024: 3.8, 5.8 and 7.0 us per step with
+  // eight, twelve and sixteen)
+  if (p.units <= 256) return launch_rows<4, 8>(stream, p);
+  if (p.units <= 512) return launch_rows<8, 8>(stream, p);
+  return launch_rows<16, 8>(stream, p);
+}
+
 // Two of these launches at once would each hold CUs that the other waits for, until both give up: launches from different
-// streams of the process follow one another.  The event is recorded only when a second stream turns up.
+// streams of the process follow one another.  Once a second stream has turned up, each leaves an event on the stream that
+// ran it for the next one to wait for, so no stream is looked at that may be gone, or is being captured, by then.  (Before
+// that nothing is recorded, which a short sequence would feel: 2.7 us of 33 for 4 steps of 2 x 64.  The second stream's
+// first sequence may therefore meet the one before it.)
 struct Turn {
   std::mutex mtx;
-  hipStream_t last = nullptr;
+  hipStream_t first = nullptr;
+  bool used = false, several = false;
   hipEvent_t event = nullptr;
-  bool used = false;
+  bool recorded = false;
 };
 Turn g_turns[16];
 
 }  // namespace
-
-void lstm_sequence_forget_stream(hipStream_t stream) {
-  for (Turn& t : g_turns) {
-    std::lock_guard<std::mutex> lk(t.mtx);
-    if (t.used && t.last == stream) t.used = false;  // the stream is idle
-  }
-}
 
 }  // namespace tfcc_rocm
 
@@ -409,28 +414,21 @@ int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc
   TFCC_REQUIRE(dev >= 0 && dev < 16, "device index %d", dev);
   hipStream_t s = as_stream(stream);
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  TFCC_HIP_CHECK(hipStreamIsCapturing(s, &capturing));
+  if (hipStreamIsCapturing(s, &capturing) != hipSuccess) (void)hipGetLastError();  // the null stream beside a capture: it is not captured
+  if (capturing != hipStreamCaptureStatusNone) return launch_units(s, p);
   Turn& turn = g_turns[dev];
-  std::unique_lock<std::mutex> lk(turn.mtx, std::defer_lock);
-  if (capturing == hipStreamCaptureStatusNone) {
-    lk.lock();
-    if (turn.used && turn.last != s) {
-      hipStreamCaptureStatus other = hipStreamCaptureStatusNone;
-      if (turn.event == nullptr) TFCC_HIP_CHECK(hipEventCreateWithFlags(&turn.event, hipEventDisableTiming));
-      if (hipStreamIsCapturing(turn.last, &other) == hipSuccess && other == hipStreamCaptureStatusNone) {
-        TFCC_HIP_CHECK(hipEventRecord(turn.event, turn.last));
-        TFCC_HIP_CHECK(hipStreamWaitEvent(s, turn.event, 0));
-      }
-    }
-    turn.used = true;
-    turn.last = s;
-  }
-  // eight wavefronts, so eight units, per workgroup: with four, twice the workgroups poll; with twelve or sixteen, each of
-  // which reads all of h from LDS, that takes longer than the trip to memory (4 x 1024: 3.8, 5.8 and 7.0 us per step with
-  // eight, twelve and sixteen)
-  if (q->units <= 256) return launch_rows<4, 8>(s, p);
-  if (q->units <= 512) return launch_rows<8, 8>(s, p);
-  return launch_rows<16, 8>(s, p);
+  std::lock_guard<std::mutex> lk(turn.mtx);
+  if (!turn.used) turn.first = s;
+  turn.several = turn.several || (turn.used && turn.first != s) || s == hipStreamPerThread;
+  turn.used = true;
+  if (!turn.several) return launch_units(s, p);
+  if (turn.event == nullptr) TFCC_HIP_CHECK(hipEventCreateWithFlags(&turn.event, hipEventDisableTiming));
+  // (what cannot be waited for or recorded is done without: the sequences may then meet, and still end)
+  if (turn.recorded && hipStreamWaitEvent(s, turn.event, 0) != hipSuccess) (void)hipGetLastError();
+  const int status = launch_units(s, p);
+  turn.recorded = hipEventRecord(turn.event, s) == hipSuccess;
+  if (!turn.recorded) (void)hipGetLastError();
+  return status;
 }
 
 }  // extern "C"
