@@ -21,6 +21,7 @@
 #include <mutex>
 
 #include "common.hpp"
+#include "lstm_sequence_plan.hpp"
 
 namespace tfcc_rocm {
 namespace {
@@ -320,19 +321,16 @@ __global__ __launch_bounds__(1024) void lstm_repair_kernel(SequenceParams p) {
   }
 }
 
-unsigned padded_units(unsigned units) { return units <= 256 ? 256 : units <= 512 ? 512 : 1024; }
-
 template <int Q, int KI, int WAVES>
 int launch(hipStream_t stream, SequenceParams p) {
-  constexpr unsigned pitch = 64 * KI, unitsPerBlock = WAVES;
+  constexpr unsigned pitch = 64 * KI;
+  static_assert(WAVES == (int)lstm_plan::kUnitsPerWorkgroup, "a wavefront per unit");
   constexpr size_t lds = (size_t)2 * 4 * Q * (pitch + 16) * sizeof(float);
   static_assert(lds <= 140 * 1024, "LDS budget");
-  p.blocksPerDirection = (p.units + unitsPerBlock - 1) / unitsPerBlock;
-  int dev = 0, cus = 0;
+  p.blocksPerDirection = lstm_plan::workgroups(p.units, 1);
+  int dev = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));
   TFCC_REQUIRE(dev >= 0 && dev < 16, "device index %d", dev);
-  TFCC_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  TFCC_REQUIRE((int)(p.blocksPerDirection * p.directions) <= cus, "lstm_sequence: needs %u CUs", p.blocksPerDirection * p.directions);
   auto kern = lstm_sequence_kernel<Q, KI, WAVES>;
   static bool attrSet[16] = {};  // per device: the attribute belongs to the function on one device
   if (!attrSet[dev]) {
@@ -386,15 +384,19 @@ using namespace tfcc_rocm;
 extern "C" {
 
 size_t tfcc_rocm_lstm_sequence_workspace(unsigned batch, unsigned units, unsigned directions) {
-  if (batch < 1 || batch > 16 || units < 1 || units > 1024 || directions < 1 || directions > 2) return 0;
-  return (size_t)2 * directions * batch * padded_units(units) * 8 + 64;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return lstm_plan::workspace_bytes(batch, units, directions, cus);
 }
 
 int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc* q) {
   TFCC_REQUIRE(q != nullptr, "lstm_sequence: null argument");
   const size_t need = tfcc_rocm_lstm_sequence_workspace(q->batch, q->units, q->directions);
-  TFCC_REQUIRE(need != 0, "lstm_sequence: 1 to 16 rows, 1 to 1024 units and 1 or 2 directions, got %u, %u, %u", q->batch, q->units,
-               q->directions);
+  TFCC_REQUIRE(need != 0, "lstm_sequence: 1 to 16 rows, 1 to 1024 units, 1 or 2 directions and a CU for eight units of each, got %u, %u, %u",
+               q->batch, q->units, q->directions);
   TFCC_REQUIRE(q->seq >= 1 && q->seq < 0xfffffff0u, "lstm_sequence: %u steps", q->seq);
   TFCC_REQUIRE(q->workspace && (uintptr_t)q->workspace % 8 == 0 && q->workspace_bytes >= need,
                "lstm_sequence: the workspace needs %zu bytes", need);

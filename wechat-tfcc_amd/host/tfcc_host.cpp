@@ -657,7 +657,7 @@ class ROCMCellInterface : public CellInterface<float> {
     tfcc_rocm_lstm_sequence_desc d{};
     const unsigned batch = sequences[0].ih->shape(0), units = sequences[0].ih->shape(1);
     const size_t bytes = tfcc_rocm_lstm_sequence_workspace(batch, units, static_cast<unsigned>(sequences.size()));
-    if (bytes == 0) throw NotImplementedError("LSTM sequence in one launch: 1 to 16 rows, at most 1024 units");
+    if (bytes == 0) throw NotImplementedError("LSTM sequence in one launch: 1 to 16 rows, at most 1024 units, a CU for every eight");
     for (size_t i = 1; i < sequences.size(); ++i)
       if (sequences[i].ih->shape() != sequences[0].ih->shape()) throw NotImplementedError("LSTM sequences of different shapes");
     Variable<uint8_t> workspace({static_cast<unsigned>(bytes)});
