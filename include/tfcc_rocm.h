@@ -447,7 +447,7 @@ int tfcc_rocm_lstm_cell_f32(void* stream, unsigned batch, unsigned units, const 
  * run from the last row of x to the first.  1 to 16 rows, 1 to 1024 units, and at least a CU
  * of the current device for eight units of a direction (else the workspace size is 0).  The workspace needs no particular
  * contents; out, h and c may overlap no input.  wait_us: how long the workgroups wait for one another
- * before the sequence is computed in a single one.  Calls of a process on one GPU follow one another, whatever their
+ * before the sequence is computed in a single one per direction (0: always that).  Calls of a process on one GPU follow one another, whatever their
  * streams (from the second stream's second call on).  Sequences replayed from graphs do not: two at once that do not fit
  * on the GPU together, or one on a stream confined to fewer CUs than it has workgroups (one for eight units of a
  * direction), end through that wait - the results are the same, the time is not. */

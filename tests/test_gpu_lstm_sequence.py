@@ -45,6 +45,11 @@ def launch(pkg, T, x, sets, backward, wait_us=20000, stream=None):
     return outs, keep
 
 
+def gave_up(T, keep):
+    """the word by which the workgroups tell the launch behind them to compute the sequence"""
+    return int(T.n(keep[0])[-64:-60].view(np.uint32)[0])
+
+
 def compare(T, outs, x, sets, backward):
     for (out, h, c), s, back in zip(outs, sets, backward):
         want = O.lstm_sequence(x, s["ik"], s["sk"], s["bias"], s["ih"], s["ic"], back)
@@ -61,17 +66,20 @@ def test_sequence_against_the_oracle(pkg, T, seq, batch, hidden, directions):
     backward = (False, True)[:directions]
     outs, keep = launch(pkg, T, x, sets, backward)
     compare(T, outs, x, sets, backward)
+    assert gave_up(T, keep) == 0
     again, keep2 = launch(pkg, T, x, sets, backward)
+    assert gave_up(T, keep2) == 0
     for a, b in zip(outs, again):
         for p, q in zip(a, b):
             assert np.array_equal(T.n(p), T.n(q))
 
 
-@pytest.mark.parametrize("seq,batch,hidden", [(5, 3, 96), (4, 12, 600)])
+@pytest.mark.parametrize("seq,batch,hidden", [(5, 3, 96), (4, 12, 600), (1, 1, 5), (3, 16, 1024)])
 def test_a_wait_that_is_over_at_once(pkg, T, seq, batch, hidden):
     x, sets = setup(T, seq, batch, 24, hidden, 2)
     outs, keep = launch(pkg, T, x, sets, (False, True), wait_us=0)
     compare(T, outs, x, sets, (False, True))
+    assert gave_up(T, keep) == 1
 
 
 def test_limits(pkg, T):

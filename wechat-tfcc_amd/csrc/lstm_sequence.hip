@@ -157,7 +157,7 @@ __global__ __launch_bounds__(64 * WAVES) void lstm_sequence_kernel(SequenceParam
   const size_t setSize = (size_t)p.directions * batch * K;
   unsigned long long* mine = p.words + (size_t)d * batch * K;
   for (int i = tid; i < 2 * MB * LP; i += T) hs[i] = 0.f;  // rows of the batch and units that do not exist stay zero
-  if (tid == 0) gaveUp = 0;
+  if (tid == 0) gaveUp = p.waitTicks == 0;  // no wait at all: the launch behind this one has the sequence
   __syncthreads();
 
   const unsigned u = (blockIdx.x - d * p.blocksPerDirection) * WAVES + wave;
