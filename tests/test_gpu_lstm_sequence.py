@@ -165,3 +165,37 @@ def test_after_a_stream_that_is_gone(pkg, T):
         outs, keep = launch(pkg, T, x, sets, (False, True))
         torch.cuda.synchronize()
         compare(T, outs, x, sets, (False, True))
+
+
+@pytest.mark.parametrize("function,low,high", [("tanh", -0.65, 0.65), ("tanh", 0.5, 0.8), ("tanh", -4.0, 4.0), ("tanh", -12.0, 12.0), ("sigmoid", -1.0, 1.0),
+                                               ("sigmoid", -4.0, 4.0), ("sigmoid", 0.0, 20.0), ("sigmoid", -20.0, -4.0), ("sigmoid", -87.0, 0.0)])
+def test_functions_of_the_cell(pkg, T, function, low, high):
+    """One step with a state kernel of zeros leaves tanh(x) (gates i open, f shut) or sigmoid(x) (c gate 0, state 1) in c.  No
+    further from float64 than the step kernel with the library's functions, which the reference's formulas call."""
+    import torch
+    lib, batch, units = pkg.lib(), 16, 1024
+    v = np.random.default_rng(int(abs(high) * 8 + abs(low))).uniform(low, high, (batch, units)).astype(np.float32)
+    x = np.zeros((batch, 4, units), np.float32)
+    x[:, 0], x[:, 3] = 40.0, 40.0
+    x[:, 1], x[:, 2] = (v, -200.0) if function == "tanh" else (0.0, v)
+    t = {k: T.t(a) for k, a in dict(x=x.reshape(batch, -1), kernel=np.zeros((units, 4 * units), np.float32), bias=np.zeros(4 * units, np.float32),
+                                    h0=np.zeros((batch, units), np.float32), h=np.zeros((batch, 4 * units), np.float32),
+                                    c0=np.full((batch, units), 0.0 if function == "tanh" else 1.0, np.float32)).items()}
+    got, library, h, out = (torch.empty((batch, units), device="cuda") for _ in range(4))
+    d = pkg.LstmSequenceDesc()
+    d.seq, d.batch, d.units, d.directions, d.wait_us = 1, batch, units, 1, 20000
+    need = lib.tfcc_rocm_lstm_sequence_workspace(batch, units, 1)
+    workspace = torch.empty(need, dtype=torch.uint8, device="cuda")
+    d.workspace, d.workspace_bytes = workspace.data_ptr(), need
+    d.x[0], d.kernel[0], d.bias[0], d.h0[0], d.c0[0] = (t[k].data_ptr() for k in ("x", "kernel", "bias", "h0", "c0"))
+    d.out[0], d.h[0], d.c[0] = out.data_ptr(), h.data_ptr(), got.data_ptr()
+    pkg.check(lib.tfcc_rocm_lstm_sequence_f32(None, C.byref(d)))
+    pkg.check(lib.tfcc_rocm_lstm_cell_f32(None, batch, units, t["c0"].data_ptr(), t["x"].data_ptr(), t["h"].data_ptr(), t["bias"].data_ptr(), 0.0,
+                                          h.data_ptr(), library.data_ptr()))
+    wide = v.astype(np.float64)
+    want = np.tanh(wide) if function == "tanh" else 1.0 / (1.0 + np.exp(-wide))
+    unit = np.spacing(np.abs(want).astype(np.float32)).astype(np.float64)
+    ours, theirs = (np.abs(T.n(r).astype(np.float64) - want) / unit for r in (got, library))
+    print(function, low, high, "largest %.3f mean %.4f, library %.3f %.4f" % (ours.max(), ours.mean(), theirs.max(), theirs.mean()))
+    # (a hundredth for what the choice of inputs does to a mean, a tenth for the largest of 16384)
+    assert ours.max() <= theirs.max() + 0.1 and ours.mean() <= theirs.mean() + 0.01
