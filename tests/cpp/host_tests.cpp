@@ -1084,6 +1084,51 @@ static void test_attention_permuted() {
   CHECK_THROWS(tfcc::rocm::blas::attention_permuted(q, toHeads, k, toHeadsT, v, toHeads, toHeads, nullptr), tfcc::NotImplementedError);
 }
 
+static int g_blocksMade = 0, g_blocksDropped = 0;
+
+static void test_pinned_pool() {
+  tfcc::PinnedPool pool(
+      [](void** p, size_t bytes) {
+        *p = std::malloc(bytes);
+        ++g_blocksMade;
+        return *p ? 0 : 1;
+      },
+      [](void* p) {
+        std::free(p);
+        ++g_blocksDropped;
+        return 0;
+      });
+  pool.enter();
+  void* a = pool.take(5000);
+  pool.give(a);
+  // a session that comes and goes beside the first one leaves the kept block where it is
+  pool.enter();
+  pool.leave();
+  CHECK(g_blocksDropped == 0);
+  CHECK(pool.take(8192) == a);
+  CHECK(g_blocksMade == 1);
+  void* b = pool.take(1);
+  pool.give(b);
+  pool.leave();  // the last one: what is kept goes back
+  CHECK(g_blocksMade == 2);
+  CHECK(g_blocksDropped == 1);
+  pool.give(a);  // a result that outlived every session
+  CHECK(g_blocksDropped == 2);
+  // the bound: a kept block makes room for one of another size, blocks in use do not
+  pool.enter();
+  CHECK(pool.take(tfcc::PinnedPool::kMaxBlock + 1) == nullptr);
+  std::vector<void*> all;
+  for (size_t i = 0; i < tfcc::PinnedPool::kMaxTotal / tfcc::PinnedPool::kMaxBlock; ++i) all.push_back(pool.take(tfcc::PinnedPool::kMaxBlock));
+  CHECK(std::count(all.begin(), all.end(), nullptr) == 0);
+  CHECK(pool.take(1) == nullptr);
+  pool.give(all.back());
+  all.back() = pool.take(1);
+  CHECK(all.back() != nullptr);
+  for (void* p : all) pool.give(p);
+  pool.leave();
+  CHECK(g_blocksMade == g_blocksDropped);
+}
+
 static void test_two_sessions_on_two_threads() {
   int f1 = 0, f2 = 0;
   std::thread t1(thread_body, 11u, 12, &f1), t2(thread_body, 23u, 12, &f2);
@@ -1110,6 +1155,7 @@ int main(int argc, char** argv) {
   run("framework.squeeze", test_squeeze);
   run("framework.view_window", test_view_window);
   run("framework.flexallocator", test_flexallocator);
+  run("framework.pinned_pool", test_pinned_pool);
   run("framework.getdevicetype", [&] { test_device_identity(mode == "gpu" ? tfcc::DeviceType::ROCM : tfcc::DeviceType::HOST); });
   if (mode == "gpu") {
     run("blas.matmul_validation", test_matmul_validation);

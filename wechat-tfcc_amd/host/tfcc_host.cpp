@@ -1127,6 +1127,7 @@ ROCMSession::ROCMSession(ROCMDevice& device, std::unique_ptr<Allocator> allocato
     : Session(std::move(allocator)), _device(device), _stream(nullptr) {
   device.attach();
   check(tfcc_rocm_stream_create(&_stream));
+  PinnedPool::instance().enter();
   // session memory comes from the device allocator; a block only really goes back after the stream
   // has drained, because kernels still queued may be using it
   _allocator->setRealMalloc([this](size_t len) { return _device.malloc(len); });
@@ -1142,7 +1143,7 @@ ROCMSession::~ROCMSession() {
   if (_staging) PinnedPool::instance().give(_staging);
   if (_flag) PinnedPool::instance().give(_flag);
   if (_arrivals) _device.free(_arrivals);
-  PinnedPool::instance().trim();
+  PinnedPool::instance().leave();
   _allocator->releaseCache();
   tfcc_rocm_stream_destroy(_stream);
 }
@@ -1154,7 +1155,7 @@ void ROCMSession::sync() const {
 }
 
 PinnedPool& PinnedPool::instance() {
-  static PinnedPool* pool = new PinnedPool();  // never destroyed: results may outlive every static object
+  static PinnedPool* pool = new PinnedPool(tfcc_rocm_host_malloc, tfcc_rocm_host_free);  // never destroyed: results may outlive every static object
   return *pool;
 }
 
@@ -1170,7 +1171,7 @@ void* PinnedPool::take(size_t bytes) {
     _kept.erase(it);
   } else {
     if (_total + size > kMaxTotal) trimLocked();
-    if (_total + size > kMaxTotal || tfcc_rocm_host_malloc(&p, size) != TFCC_ROCM_OK) return nullptr;
+    if (_total + size > kMaxTotal || _make(&p, size) != 0) return nullptr;
     _total += size;
   }
   _live[p] = size;
@@ -1183,19 +1184,25 @@ void PinnedPool::give(void* block) {
   if (it == _live.end()) return;
   _kept.emplace(it->second, block);
   _live.erase(it);
+  if (_sessions == 0) trimLocked();
 }
 
 void PinnedPool::trimLocked() {
   for (auto& kv : _kept) {
-    tfcc_rocm_host_free(kv.second);
+    _drop(kv.second);
     _total -= kv.first;
   }
   _kept.clear();
 }
 
-void PinnedPool::trim() {
+void PinnedPool::enter() {
   std::lock_guard<std::mutex> lk(_mtx);
-  trimLocked();
+  ++_sessions;
+}
+
+void PinnedPool::leave() {
+  std::lock_guard<std::mutex> lk(_mtx);
+  if (--_sessions == 0) trimLocked();
 }
 
 HostBlock::HostBlock(size_t bytes, bool gpu) {

@@ -37,22 +37,27 @@ class ROCMDevice : public Device {
 };
 
 // Page-locked host blocks, shared by all sessions and threads of the process: a block costs the driver hundreds of
-// microseconds to make, so freed ones are kept for the next request of their size class (powers of two).  Blocks in use
-// and kept together never exceed kMaxTotal; trim() gives the kept ones back (every session does that when it ends).
+// microseconds to make, so freed ones are kept for the next request of their size class (powers of two) for as long as a
+// session lives: one that ends beside others takes nothing from them.  Blocks in use and kept together never exceed
+// kMaxTotal.
 class PinnedPool {
+  int (*const _make)(void**, size_t);
+  int (*const _drop)(void*);
   std::mutex _mtx;
   std::map<void*, size_t> _live;
   std::multimap<size_t, void*> _kept;
-  size_t _total = 0;
+  size_t _total = 0, _sessions = 0;
 
   void trimLocked();
 
  public:
   static constexpr size_t kMaxBlock = size_t(64) << 20, kMaxTotal = size_t(256) << 20;
   static PinnedPool& instance();
+  PinnedPool(int (*make)(void**, size_t), int (*drop)(void*)) : _make(make), _drop(drop) {}
+  void enter();  // a session begins
+  void leave();  // and ends: the last one gives back what is kept
   void* take(size_t bytes);  // nullptr: too large, the bound is reached, or there is no GPU
   void give(void* block);
-  void trim();
 };
 
 // Host memory of a result: from the pool where that has room, ordinary memory otherwise.
