@@ -1129,6 +1129,37 @@ static void test_pinned_pool() {
   CHECK(g_blocksMade == g_blocksDropped);
 }
 
+// Room for the output in the pool, none for the word the GPU raises: the copies are waited for in the stream instead.
+static void test_download_without_a_flag() {
+  auto& device = dynamic_cast<tfcc::ROCMDevice&>(*tfcc::Device::getThreadDefault());
+  tfcc::Session* before = tfcc::Session::getThreadDefault();
+  {
+    tfcc::ROCMSession session(device);
+    tfcc::Session::setThreadDefault(&session);
+    std::vector<float> want(1000);
+    for (size_t i = 0; i < want.size(); ++i) want[i] = static_cast<float>(i);
+    tfcc::PinnedPool& pool = tfcc::PinnedPool::instance();
+    std::vector<void*> others;
+    {
+      tfcc::Variable<float> v = tfcc::data::set(want, {1000});
+      float* out = static_cast<float*>(pool.take(4000));
+      CHECK(out != nullptr);
+      for (size_t size = tfcc::PinnedPool::kMaxBlock; out != nullptr && size >= 4096; size /= 2)
+        while (void* p = pool.take(size)) others.push_back(p);
+      if (out != nullptr) {
+        session.download({{v.data(), out, 4000}}, true);
+        CHECK(std::equal(want.begin(), want.end(), out));
+        for (void* p : others) pool.give(p);
+        std::fill(out, out + 1000, -1.f);
+        session.download({{v.data(), out, 4000}}, true);  // with the flag
+        CHECK(std::equal(want.begin(), want.end(), out));
+        pool.give(out);
+      }
+    }
+    tfcc::Session::setThreadDefault(before);
+  }
+}
+
 static void test_two_sessions_on_two_threads() {
   int f1 = 0, f2 = 0;
   std::thread t1(thread_body, 11u, 12, &f1), t2(thread_body, 23u, 12, &f2);
@@ -1160,6 +1191,7 @@ int main(int argc, char** argv) {
   if (mode == "gpu") {
     run("blas.matmul_validation", test_matmul_validation);
     run("data.set_get_copy", test_data);
+    run("data.download_without_a_flag", test_download_without_a_flag);
     run("blas.matmul", test_blas);
     run("blas.matmul_broadcast", test_matmul_broadcast);
     run("quantization.known_answers", test_dequantize_requantize_known_answers);

@@ -1279,26 +1279,30 @@ void ROCMSession::waitForFlag() {
   _stagingUsed = 0;  // everything before the download has run
 }
 
+bool ROCMSession::reserveFlag() {
+  if (_flag == nullptr) {
+    _flag = static_cast<unsigned*>(PinnedPool::instance().take(64));
+    if (_flag == nullptr) return false;
+    *_flag = _epoch;
+  }
+  if (_arrivals == nullptr) {
+    _arrivals = static_cast<unsigned*>(_device.malloc(64));
+    if (_arrivals == nullptr) return false;
+    check(tfcc_rocm_fill_async(_stream, _arrivals, 0, sizeof(unsigned), 1));
+  }
+  return true;
+}
+
 void ROCMSession::download(const std::vector<HostRead>& reads, bool pinned) {
   if (_recording) throw RuntimeError("download: not possible while the session's stream records a graph");
   std::vector<tfcc_rocm_copy_piece> pieces;
   for (const HostRead& r : reads)
     if (r.bytes > 0) pieces.push_back({r.device, r.host, r.bytes});
   if (pieces.empty()) return;
-  if (!pinned) {
+  if (!pinned || !reserveFlag()) {
     for (const tfcc_rocm_copy_piece& p : pieces) check(tfcc_rocm_memcpy_d2h(_stream, p.dst, p.src, p.bytes));
     _stagingUsed = 0;
     return;
-  }
-  if (_flag == nullptr) {
-    _flag = static_cast<unsigned*>(PinnedPool::instance().take(64));
-    if (_flag == nullptr) throw ResourceExhaustedError();
-    *_flag = _epoch;
-  }
-  if (_arrivals == nullptr) {
-    _arrivals = static_cast<unsigned*>(_device.malloc(64));
-    if (_arrivals == nullptr) throw ResourceExhaustedError();
-    check(tfcc_rocm_fill_async(_stream, _arrivals, 0, sizeof(unsigned), 1));
   }
   ++_epoch;
   const int status = tfcc_rocm_copy_to_pinned(_stream, pieces.data(), static_cast<unsigned>(pieces.size()), _arrivals, _flag, _epoch);

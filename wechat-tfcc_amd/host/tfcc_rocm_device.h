@@ -93,6 +93,7 @@ class ROCMSession : public Session {
   unsigned _epoch = 0;
 
   bool reserveStaging(size_t bytes);
+  bool reserveFlag();  // false: no room for what a download behind the flag needs
   void waitForFlag();
 
  public:
