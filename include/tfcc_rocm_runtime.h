@@ -41,9 +41,11 @@ int tfcc_rocm_runtime_model_run(void* model, const void* inputs, size_t len, voi
 int tfcc_rocm_runtime_buffer_free(void* buffer);
 
 /* Model::run without the messages: the inputs are read where they lie (dtype: DataType of
- * tfcc_runtime/proto/common.proto:5-20) and the outputs stay in one block of host memory that belongs to
+ * tfcc_runtime/proto/common.proto:5-20) and every output stays in host memory of its own that belongs to
  * the result, page-locked where the process-wide bound of 256 MB allows.  result_output describes output
- * `index`: its pointers are valid, and its data may be written, until result_free. */
+ * `index`: its pointers are valid, and its data may be written, until result_free.  result_detach moves
+ * output `index` into a result of one output, freed by itself, so that it can outlive the others; in
+ * `result` it is empty from then on. */
 typedef struct tfcc_rocm_runtime_array {
   const char* name;
   int dtype;
@@ -55,6 +57,7 @@ typedef struct tfcc_rocm_runtime_array {
 int tfcc_rocm_runtime_model_run_arrays(void* model, const tfcc_rocm_runtime_array* inputs, size_t count,
                                        void** result, size_t* outputs);
 int tfcc_rocm_runtime_result_output(void* result, size_t index, tfcc_rocm_runtime_array* output);
+int tfcc_rocm_runtime_result_detach(void* result, size_t index, void** detached);
 int tfcc_rocm_runtime_result_free(void* result);
 
 /* Model::test(npz, stream), model.cpp:185-280: runs the entrance graph on the arrays of an .npz and

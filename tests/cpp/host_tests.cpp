@@ -1147,11 +1147,13 @@ static void test_download_without_a_flag() {
       for (size_t size = tfcc::PinnedPool::kMaxBlock; out != nullptr && size >= 4096; size /= 2)
         while (void* p = pool.take(size)) others.push_back(p);
       if (out != nullptr) {
-        session.download({{v.data(), out, 4000}}, true);
+        float ordinary[10];
+        session.download({{v.data(), out, 4000, true}, {v.data(), ordinary, 40, false}});
+        CHECK(std::equal(ordinary, ordinary + 10, want.begin()));
         CHECK(std::equal(want.begin(), want.end(), out));
         for (void* p : others) pool.give(p);
         std::fill(out, out + 1000, -1.f);
-        session.download({{v.data(), out, 4000}}, true);  // with the flag
+        session.download({{v.data(), out, 4000, true}});  // with the flag
         CHECK(std::equal(want.begin(), want.end(), out));
         pool.give(out);
       }

@@ -81,6 +81,36 @@ def test_sizes_where_the_transfers_change(mf, rt, dev, shapes):
     round_trip(mf, rt, shapes, False)
 
 
+def test_a_kept_output_does_not_hold_the_others(mf, rt):
+    # a run hands out 64 MB beside three numbers; sixteen of the small ones together hold none of the large
+    def resident():
+        with open("/proc/self/statm") as f:
+            return int(f.read().split()[1]) * 4096
+    n = 16 << 20
+    model = copies(mf, rt, [(mf.FLOAT, (n,)), (mf.FLOAT, (3,))], True)
+    inputs = {"x0": np.ones(n, np.float32), "x1": np.arange(3, dtype=np.float32)}
+    held = [model.run(inputs)["y1"]]
+    before = resident()
+    for _ in range(16):
+        held.append(model.run(inputs)["y1"])
+    assert resident() - before < 4 * inputs["x0"].nbytes
+    model.close()
+    assert all((h == [0, 1, 2]).all() for h in held)
+
+
+@pytest.mark.gpu
+def test_pinned_outputs_kept_alone_leave_the_bound_to_others(mf, rt, dev):
+    # 40 MB beside three numbers: blocks of 64 MB, of which the process-wide bound admits four
+    n = 10 << 20
+    model = copies(mf, rt, [(mf.FLOAT, (n,)), (mf.FLOAT, (3,))], False)
+    held = []
+    for i in range(8):
+        out = model.run({"x0": np.full(n, i, np.float32), "x1": np.full(3, i, np.float32)})
+        assert (out["y0"] == i).all()
+        held.append(out["y1"])
+    assert all((h == i).all() for i, h in enumerate(held))
+
+
 @pytest.mark.gpu
 def test_outputs_outlive_the_model_and_later_runs(mf, rt, dev):
     # 9 MB each: blocks of 16 MB, of which the process-wide bound admits sixteen; the runs beyond it get ordinary memory

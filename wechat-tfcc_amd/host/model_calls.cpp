@@ -1,6 +1,6 @@
 // CPython module behind runtime_api.Model.run: numpy arrays in, numpy arrays out, over the C ABI of
-// tfcc_rocm_runtime.h.  Inputs are read where numpy holds them; the outputs of a run are arrays over the run's one
-// block of host memory, which goes back when the last of them does.
+// tfcc_rocm_runtime.h.  Inputs are read where numpy holds them; every output is an array over a block of host memory of
+// its own, which goes back with it.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #define NPY_NO_DEPRECATED_API NPY_1_7_API_VERSION
@@ -126,20 +126,23 @@ PyObject* run(PyObject*, PyObject* args) {
     Py_XDECREF(message);
     return nullptr;
   }
-  PyObject* owner = PyCapsule_New(result, nullptr, free_result);
-  if (owner == nullptr) {
-    tfcc_rocm_runtime_result_free(result);
-    return nullptr;
-  }
   PyObject* outputs = PyDict_New();
   for (size_t i = 0; outputs && i < count; ++i) {
-    tfcc_rocm_runtime_array o;
-    tfcc_rocm_runtime_result_output(result, i, &o);
-    PyObject* a = output_array(o, owner);
-    if (a == nullptr || PyDict_SetItemString(outputs, o.name, a) < 0) Py_CLEAR(outputs);
+    void* part = nullptr;
+    PyObject *owner = nullptr, *a = nullptr;
+    if (tfcc_rocm_runtime_result_detach(result, i, &part) != 0) PyErr_NoMemory();
+    else if ((owner = PyCapsule_New(part, nullptr, free_result)) == nullptr) tfcc_rocm_runtime_result_free(part);
+    if (owner) {
+      tfcc_rocm_runtime_array o;
+      tfcc_rocm_runtime_result_output(part, 0, &o);
+      a = output_array(o, owner);
+      if (a == nullptr || PyDict_SetItemString(outputs, o.name, a) < 0) Py_CLEAR(a);
+      Py_DECREF(owner);
+    }
+    if (a == nullptr) Py_CLEAR(outputs);
     Py_XDECREF(a);
   }
-  Py_DECREF(owner);
+  tfcc_rocm_runtime_result_free(result);
   return outputs;
 }
 

@@ -1293,17 +1293,20 @@ bool ROCMSession::reserveFlag() {
   return true;
 }
 
-void ROCMSession::download(const std::vector<HostRead>& reads, bool pinned) {
+void ROCMSession::download(const std::vector<HostRead>& reads) {
   if (_recording) throw RuntimeError("download: not possible while the session's stream records a graph");
   std::vector<tfcc_rocm_copy_piece> pieces;
-  for (const HostRead& r : reads)
-    if (r.bytes > 0) pieces.push_back({r.device, r.host, r.bytes});
-  if (pieces.empty()) return;
-  if (!pinned || !reserveFlag()) {
-    for (const tfcc_rocm_copy_piece& p : pieces) check(tfcc_rocm_memcpy_d2h(_stream, p.dst, p.src, p.bytes));
+  const bool byKernel = std::any_of(reads.begin(), reads.end(), [](const HostRead& r) { return r.pinned && r.bytes > 0; }) && reserveFlag();
+  for (const HostRead& r : reads) {
+    if (r.bytes == 0) continue;
+    if (byKernel && r.pinned) {
+      pieces.push_back({r.device, r.host, r.bytes});
+      continue;
+    }
+    check(tfcc_rocm_memcpy_d2h(_stream, r.host, r.device, r.bytes));
     _stagingUsed = 0;
-    return;
   }
+  if (pieces.empty()) return;
   ++_epoch;
   const int status = tfcc_rocm_copy_to_pinned(_stream, pieces.data(), static_cast<unsigned>(pieces.size()), _arrivals, _flag, _epoch);
   if (status != TFCC_ROCM_OK) {

@@ -101,11 +101,12 @@ class ROCMSession : public Session {
     const void* device;
     void* host;
     size_t bytes;
+    bool pinned;  // the host address lies in a block of PinnedPool
   };
   // device <- host memory that may be changed as soon as the call returns; the copy itself is ordered on the stream
   void upload(void* device, const void* host, size_t bytes);
-  // host <- device, complete when the call returns.  pinned: the host addresses lie in blocks of PinnedPool.
-  void download(const std::vector<HostRead>& reads, bool pinned);
+  // host <- device, complete when the call returns
+  void download(const std::vector<HostRead>& reads);
 
   explicit ROCMSession(ROCMDevice& device);
   ROCMSession(ROCMDevice& device, std::unique_ptr<Allocator> allocator);

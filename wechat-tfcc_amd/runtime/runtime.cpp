@@ -703,16 +703,16 @@ void describe_output(Graph& graph, const std::string& name, RunResult::Output& o
 }
 
 template <class T>
-void get_output(Graph& graph, const RunResult::Output& out, char* host, bool rocm, std::vector<ROCMSession::HostRead>& reads) {
+void get_output(Graph& graph, RunResult::Output& out, bool rocm, std::vector<ROCMSession::HostRead>& reads) {
   if (out.bytes == 0) return;
   if (is_value(graph.getSymbolManager().getSymbolInfo(out.name).stype)) {
     const T v = graph.getValue(out.name, T());
-    std::memcpy(host, &v, sizeof(T));
+    std::memcpy(out.block.data(), &v, sizeof(T));
     return;
   }
   const Tensor<T>& tensor = graph.getTensor(out.name, T());
-  if (rocm) reads.push_back({tensor.data(), host, out.bytes});
-  else ::tfcc::Operation<T>::getCurrentInterface().getDataInterface().get(tensor, reinterpret_cast<T*>(host));
+  if (rocm) reads.push_back({tensor.data(), out.block.data(), out.bytes, out.block.pinned()});
+  else ::tfcc::Operation<T>::getCurrentInterface().getDataInterface().get(tensor, reinterpret_cast<T*>(out.block.data()));
 }
 }  // namespace
 
@@ -731,11 +731,12 @@ RunResult Model::run(const std::vector<proto::InputView>& inputs) {
   }
   graph.process();
   RunResult result;
-  size_t total = 0;
   for (const std::string& name : graph.getOutputs()) {
     const DataType dtype = graph.getSymbolManager().getSymbolInfo(name).dtype;
-    result.outputs.push_back({name, dtype, {}, total, 0});
+    result.outputs.emplace_back();
     RunResult::Output& out = result.outputs.back();
+    out.name = name;
+    out.dtype = dtype;
     switch (dtype) {
 #define TFCC_RUNTIME_DESCRIBE(T, E) \
   case E: describe_output<T>(graph, name, out); break;
@@ -744,22 +745,20 @@ RunResult Model::run(const std::vector<proto::InputView>& inputs) {
       case BOOL: describe_output<uint8_t>(graph, name, out); break;
       default: throw RuntimeError("Invalid output type");
     }
-    total += (out.bytes + 255) / 256 * 256;
+    out.block = HostBlock(out.bytes, rocm != nullptr && !is_value(graph.getSymbolManager().getSymbolInfo(name).stype));
   }
-  result.block = HostBlock(total, rocm != nullptr);
   std::vector<ROCMSession::HostRead> reads;
-  for (const RunResult::Output& out : result.outputs) {
-    char* host = result.block.data() + out.offset;
+  for (RunResult::Output& out : result.outputs) {
     switch (out.dtype) {
 #define TFCC_RUNTIME_OUTPUT(T, E) \
-  case E: get_output<T>(graph, out, host, rocm != nullptr, reads); break;
+  case E: get_output<T>(graph, out, rocm != nullptr, reads); break;
       TFCC_RUNTIME_FOR_ALL_TYPES(TFCC_RUNTIME_OUTPUT)
 #undef TFCC_RUNTIME_OUTPUT
-      case BOOL: get_output<uint8_t>(graph, out, host, rocm != nullptr, reads); break;
+      case BOOL: get_output<uint8_t>(graph, out, rocm != nullptr, reads); break;
       default: throw RuntimeError("Invalid output type");
     }
   }
-  if (rocm) rocm->download(reads, result.block.pinned());
+  if (rocm) rocm->download(reads);
   return result;
 }
 
@@ -769,7 +768,7 @@ void Model::run(const std::vector<proto::DataItem>& inputs, std::vector<proto::D
     views.push_back({item.name, item.dtype, item.shape, item.data.data(), item.data.size()});
   const RunResult result = run(views);
   for (const RunResult::Output& out : result.outputs)
-    outputs.push_back({out.name, out.dtype, out.shape, std::string(result.block.data() + out.offset, out.bytes)});
+    outputs.push_back({out.name, out.dtype, out.shape, std::string(out.block.data() ? out.block.data() : "", out.bytes)});
 }
 
 void Model::run(const std::string& inputs, std::string& outputs) {
@@ -782,7 +781,7 @@ void Model::run(const std::string& inputs, std::string& outputs) {
   const RunResult result = run(in);
   std::vector<proto::DataItem> out;
   for (const RunResult::Output& o : result.outputs)
-    out.push_back({o.name, o.dtype, o.shape, std::string(result.block.data() + o.offset, o.bytes)});
+    out.push_back({o.name, o.dtype, o.shape, std::string(o.block.data() ? o.block.data() : "", o.bytes)});
   outputs = proto::serialize_outputs(out);
 }
 

@@ -380,15 +380,15 @@ class Graph {
   static bool isRecordDetailError() { return _recordDetailError; }
 };
 
-// The graph outputs of one run in one block of host memory.
+// The graph outputs of one run, each in host memory of its own: one that is kept holds no other's.
 struct RunResult {
   struct Output {
     std::string name;
     DataType dtype;
     std::vector<unsigned> shape;
-    size_t offset, bytes;
+    size_t bytes = 0;
+    HostBlock block;
   };
-  HostBlock block;
   std::vector<Output> outputs;
 };
 

@@ -106,7 +106,20 @@ int tfcc_rocm_runtime_result_output(void* result, size_t index, tfcc_rocm_runtim
     if (result == nullptr || output == nullptr) throw tfcc::InvalidArgumentError("null argument");
     auto& r = *static_cast<tfcc::runtime::RunResult*>(result);
     const tfcc::runtime::RunResult::Output& o = r.outputs.at(index);
-    *output = {o.name.c_str(), static_cast<int>(o.dtype), o.shape.data(), o.shape.size(), r.block.data() + o.offset, o.bytes};
+    *output = {o.name.c_str(), static_cast<int>(o.dtype), o.shape.data(), o.shape.size(), o.block.data(), o.bytes};
+  });
+}
+
+int tfcc_rocm_runtime_result_detach(void* result, size_t index, void** detached) {
+  return guarded([&] {
+    if (result == nullptr || detached == nullptr) throw tfcc::InvalidArgumentError("null argument");
+    auto& r = *static_cast<tfcc::runtime::RunResult*>(result);
+    tfcc::runtime::RunResult::Output& o = r.outputs.at(index);
+    std::unique_ptr<tfcc::runtime::RunResult> d(new tfcc::runtime::RunResult());
+    d->outputs.push_back({o.name, o.dtype, o.shape, o.bytes, {}});
+    std::swap(d->outputs[0].block, o.block);
+    o.bytes = 0;
+    *detached = d.release();
   });
 }
 

@@ -19,6 +19,7 @@ SYMBOLS = {
     "tfcc_rocm_runtime_buffer_free": (C.c_int, [_VP]),
     "tfcc_rocm_runtime_model_run_arrays": (C.c_int, [_VP, _VP, C.c_size_t, C.POINTER(_VP), C.POINTER(C.c_size_t)]),
     "tfcc_rocm_runtime_result_output": (C.c_int, [_VP, C.c_size_t, _VP]),
+    "tfcc_rocm_runtime_result_detach": (C.c_int, [_VP, C.c_size_t, C.POINTER(_VP)]),
     "tfcc_rocm_runtime_result_free": (C.c_int, [_VP]),
     "tfcc_rocm_runtime_model_test": (C.c_int, [_VP, _VP, C.c_size_t, C.POINTER(C.c_int), C.POINTER(_VP)]),
     "tfcc_rocm_runtime_set_fusion": (C.c_int, [C.c_int]),
