@@ -1,7 +1,9 @@
 """Model.run on numpy arrays: what it takes and returns equals the message form (run_serialized), at the sizes where its
 transfers change course, and its outputs stay valid for as long as they are held."""
+import collections
 import gc
 import importlib
+import types
 
 import numpy as np
 import pytest
@@ -79,6 +81,29 @@ def test_what_is_not_an_input_raises(mf, rt):
 ])
 def test_sizes_where_the_transfers_change(mf, rt, dev, shapes):
     round_trip(mf, rt, shapes, False)
+
+
+def test_any_mapping_is_taken(mf, rt):
+    model = copies(mf, rt, [(mf.FLOAT, (2,)), (mf.INT32, (3,))], True)
+    want = {"x0": np.array([1, 2], np.float32), "x1": np.array([3, 4, 5], np.int32)}
+
+    class Items:
+        def items(self):
+            return ([k, v] for k, v in want.items())
+
+    for arrays in (want, collections.OrderedDict(want), types.MappingProxyType(want), collections.UserDict(want),
+                   collections.ChainMap({"x0": want["x0"]}, {"x1": want["x1"]}), Items()):
+        out = model.run(arrays)
+        assert np.array_equal(out["y0"], want["x0"]) and np.array_equal(out["y1"], want["x1"])
+    with pytest.raises(AttributeError):
+        model.run([("x0", want["x0"])])
+
+    class Pairs:
+        def items(self):
+            return [("x0",)]
+
+    with pytest.raises(ValueError):
+        model.run(Pairs())
 
 
 def test_a_kept_output_does_not_hold_the_others(mf, rt):

@@ -93,19 +93,25 @@ PyObject* output_array(const tfcc_rocm_runtime_array& o, PyObject* owner) {
   return a;
 }
 
-// run(model handle, {name: array}, exception class) -> {name: array}
+// run(model handle, {name: array}, exception class) -> {name: array}.  The arrays are read with the interpreter lock
+// released: another thread that writes to one meanwhile changes what the run sees.
 PyObject* run(PyObject*, PyObject* args) {
   unsigned long long handle = 0;
   PyObject *arrays = nullptr, *error = nullptr;
-  if (!PyArg_ParseTuple(args, "KO!O", &handle, &PyDict_Type, &arrays, &error)) return nullptr;
-  std::vector<Input> inputs(static_cast<size_t>(PyDict_Size(arrays)));
-  // converting a value may run code of its own, so the dict is walked through a list of its items
-  PyObject* items = PyDict_Items(arrays);
+  if (!PyArg_ParseTuple(args, "KOO", &handle, &arrays, &error)) return nullptr;
+  // converting a value may run code of its own, so what is walked is a list; as `for name, a in arrays.items()`, any
+  // mapping with such a method will do
+  PyObject* pairs = PyDict_CheckExact(arrays) ? PyDict_Items(arrays) : PyObject_CallMethod(arrays, "items", nullptr);
+  PyObject* items = pairs ? PySequence_List(pairs) : nullptr;
+  Py_XDECREF(pairs);
   if (items == nullptr) return nullptr;
+  std::vector<Input> inputs(static_cast<size_t>(PyList_GET_SIZE(items)));
   bool fine = true;
   for (size_t i = 0; i < inputs.size() && fine; ++i) {
-    PyObject* item = PyList_GET_ITEM(items, static_cast<Py_ssize_t>(i));
-    fine = read_input(PyTuple_GET_ITEM(item, 0), PyTuple_GET_ITEM(item, 1), inputs[i]);
+    PyObject* item = PySequence_Tuple(PyList_GET_ITEM(items, static_cast<Py_ssize_t>(i)));
+    if (item && PyTuple_GET_SIZE(item) != 2) PyErr_SetString(PyExc_ValueError, "items() gives something else than (name, array)");
+    fine = item && PyTuple_GET_SIZE(item) == 2 && read_input(PyTuple_GET_ITEM(item, 0), PyTuple_GET_ITEM(item, 1), inputs[i]);
+    Py_XDECREF(item);
   }
   Py_DECREF(items);
   if (!fine) return nullptr;

@@ -105,7 +105,9 @@ class Model:
             lib().tfcc_rocm_runtime_buffer_free(out)
 
     def run(self, arrays):
-        """{name: ndarray} -> {name: ndarray}: what run_serialized does with the messages of modelfile, without them"""
+        """{name: ndarray} -> {name: ndarray}: what run_serialized does with the messages of modelfile, without them.
+        `arrays` is any mapping with items().  C-contiguous arrays are read where they lie and without the interpreter
+        lock, so no other thread may write to them until the call returns; other layouts are copied first."""
         return _calls().run(self._h.value or 0, arrays, RuntimeError_)
 
     def test(self, npz_bytes):
