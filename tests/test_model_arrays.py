@@ -65,6 +65,8 @@ def test_what_is_not_an_input_raises(mf, rt):
         model.run({"x0": np.zeros((2, 2), ">f4")})
     with pytest.raises(rt.RuntimeError_):
         model.run({"nobody": np.zeros((2, 2), np.float32)})
+    with pytest.raises(rt.RuntimeError_):
+        model.run({"x0\0": np.zeros((2, 2), np.float32)})
     with pytest.raises(rt.RuntimeError_, match="type not match"):
         model.run({"x0": np.zeros((2, 2), np.float64)})
     view = np.arange(8, dtype=np.float32).reshape(4, 2)[::2]  # not contiguous

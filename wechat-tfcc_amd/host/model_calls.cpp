@@ -49,7 +49,7 @@ struct Input {
   ~Input() { Py_XDECREF(array); }
 };
 
-bool read_input(PyObject* key, PyObject* value, Input& in) {
+bool read_input(PyObject* key, PyObject* value, PyObject* error, Input& in) {
   Py_ssize_t len = 0;
   if (PyUnicode_Check(key)) {
     const char* text = PyUnicode_AsUTF8AndSize(key, &len);
@@ -59,6 +59,11 @@ bool read_input(PyObject* key, PyObject* value, Input& in) {
     char* text = nullptr;
     if (PyBytes_AsStringAndSize(key, &text, &len) < 0) return false;
     in.name.assign(text, static_cast<size_t>(len));
+  }
+  // the C ABI ends a name at its first zero: what follows would be dropped, and another input might answer to the rest
+  if (in.name.find('\0') != std::string::npos) {
+    PyErr_Format(error, "invalid input name %R", key);
+    return false;
   }
   in.array = reinterpret_cast<PyArrayObject*>(PyArray_FromAny(value, nullptr, 0, 0, NPY_ARRAY_C_CONTIGUOUS, nullptr));
   if (in.array == nullptr) return false;
@@ -110,7 +115,7 @@ PyObject* run(PyObject*, PyObject* args) {
   for (size_t i = 0; i < inputs.size() && fine; ++i) {
     PyObject* item = PySequence_Tuple(PyList_GET_ITEM(items, static_cast<Py_ssize_t>(i)));
     if (item && PyTuple_GET_SIZE(item) != 2) PyErr_SetString(PyExc_ValueError, "items() gives something else than (name, array)");
-    fine = item && PyTuple_GET_SIZE(item) == 2 && read_input(PyTuple_GET_ITEM(item, 0), PyTuple_GET_ITEM(item, 1), inputs[i]);
+    fine = item && PyTuple_GET_SIZE(item) == 2 && read_input(PyTuple_GET_ITEM(item, 0), PyTuple_GET_ITEM(item, 1), error, inputs[i]);
     Py_XDECREF(item);
   }
   Py_DECREF(items);
