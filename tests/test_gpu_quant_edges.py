@@ -24,6 +24,17 @@ def test_quantize_with_the_range_of_the_data(pkg, T, total, dtype, skip):
     assert np.array_equal(T.n(q), O.quantize(x[skip:], lo, hi, dtype))
 
 
+@pytest.mark.parametrize("total", [5, 4095, 40001, LIMIT + 4])
+def test_quantize_over_its_own_input(pkg, T, total):
+    import torch
+    x = np.random.default_rng(total).normal(0.1, 2.0, total).astype(np.float32)
+    data, lo, hi = T.t(x), T.f1(0.0), T.f1(0.0)
+    pkg.check(pkg.lib().tfcc_rocm_quantize_minmax(pkg._stream(), pkg._ptr(data), total, pkg._ptr(data), pkg._type_code(torch.int32),
+                                                  pkg._ptr(lo), pkg._ptr(hi)))
+    assert (float(T.n(lo)[0]), float(T.n(hi)[0])) == (float(x.min()), float(x.max()))
+    assert np.array_equal(T.n(data).view(np.int32), T.n(pkg.quantize(T.t(x), torch.int32, lo, hi)))
+
+
 @pytest.mark.parametrize("special", [[np.nan, 1.0, -2.0], [np.inf, 1.0, -2.0], [3.0, 3.0, 3.0], [np.nan] * 3, [-7.5, 0.3, 9.25]])
 @pytest.mark.parametrize("dtype", ["uint8", "int16", "int32"])
 def test_quantize_small_and_large_tensors_agree(pkg, T, special, dtype):

@@ -781,7 +781,11 @@ int tfcc_rocm_quantize_minmax(void* stream, const float* in, uint64_t total, voi
   TFCC_REQUIRE(total > 0, "quantize: empty tensor");
   TFCC_REQUIRE(valid_type(out_type), "quantize: bad type code");
   hipStream_t s = as_stream(stream);
-  if (total <= kWholeLimit) {
+  // In place (a four-byte type over its own input): only the form that writes nothing before the range is known, and then
+  // every element where it was read.
+  const uintptr_t inAt = (uintptr_t)in, outAt = (uintptr_t)out;
+  const bool apart = inAt + 4 * total <= outAt || outAt + total * (int_range(out_type).bits / 8) <= inAt;
+  if (apart && total <= kWholeLimit) {
     hipLaunchKernelGGL(quantize_whole_kernel, dim3((unsigned)((total + 4095) / 4096)), dim3(1024), 0, s, in, (unsigned)total,
                        out, out_type, min_v, max_v);
     return check_launch("quantize");
@@ -791,7 +795,7 @@ int tfcc_rocm_quantize_minmax(void* stream, const float* in, uint64_t total, voi
   int dev = 0;
   unsigned slot = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));
-  if ((uintptr_t)in % 16 == 0 && (uintptr_t)out % 4 == 0) {
+  if (apart && (uintptr_t)in % 16 == 0 && (uintptr_t)out % 4 == 0) {
     // partial results, eight bytes per workgroup, rest in the output buffer until the quantize pass overwrites it
     float* partials = static_cast<float*>(out);
     if (gArrivalSlots.of(dev, s, &slot)) {
