@@ -401,4 +401,17 @@ __host__ __device__ static inline RequantScalars make_requant_scalars(int inType
   return s;
 }
 
+// 4x4 byte transpose: in r[q] = bytes (n0..n3) of k-row q; out c[j] = bytes (k0..k3) of column j
+// v_perm_b32(hi, lo, sel): selector bytes 0-3 pick from lo, 4-7 from hi
+__device__ __forceinline__ void transpose4x4(const unsigned r[4], unsigned c[4]) {
+  const unsigned t0 = __builtin_amdgcn_perm(r[1], r[0], 0x05010400u);  // r0.b0 r1.b0 r0.b1 r1.b1
+  const unsigned t1 = __builtin_amdgcn_perm(r[1], r[0], 0x07030602u);  // r0.b2 r1.b2 r0.b3 r1.b3
+  const unsigned t2 = __builtin_amdgcn_perm(r[3], r[2], 0x05010400u);
+  const unsigned t3 = __builtin_amdgcn_perm(r[3], r[2], 0x07030602u);
+  c[0] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);  // t0.lo16 t2.lo16
+  c[1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);  // t0.hi16 t2.hi16
+  c[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
+  c[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
+}
+
 }  // namespace tfcc_rocm

@@ -75,17 +75,6 @@ struct GemvWideParams {
 // The workspace of the entry point that must not allocate: one per GPU, inside the library's image.
 __device__ __align__(256) unsigned long long scratch[kMaxStaticBlocks * kMaxM * kCols];
 
-__device__ __forceinline__ void transpose4x4(const unsigned r[4], unsigned c[4]) {
-  unsigned t0 = __builtin_amdgcn_perm(r[1], r[0], 0x05010400u);
-  unsigned t1 = __builtin_amdgcn_perm(r[1], r[0], 0x07030602u);
-  unsigned t2 = __builtin_amdgcn_perm(r[3], r[2], 0x05010400u);
-  unsigned t3 = __builtin_amdgcn_perm(r[3], r[2], 0x07030602u);
-  c[0] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
-  c[1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
-  c[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
-  c[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
-}
-
 // Rows r0 .. r0 + RPT - 1 of column egn (ec within the block) of this workgroup's partial tile, in sum[]: joins them
 // with the other parts of K through the workspace and, for the elements this thread completes, applies the offset
 // terms and writes the results.

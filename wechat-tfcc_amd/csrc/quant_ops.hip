@@ -137,15 +137,6 @@ __device__ __forceinline__ float4 load_streamed(const float4* p) {
 // rows four at a time, transposes each 4 x 4 byte block in registers so that a word holds one column's four rows,
 // and adds those with one dot-product instruction; the four row lanes meet in LDS and the slab's sums go to the
 // (zeroed) result with integer atomics, whose order does not matter.
-__device__ __forceinline__ void transpose_bytes_4x4(const unsigned r[4], unsigned c[4]) {
-  const unsigned t0 = __builtin_amdgcn_perm(r[1], r[0], 0x05010400u), t1 = __builtin_amdgcn_perm(r[1], r[0], 0x07030602u);
-  const unsigned t2 = __builtin_amdgcn_perm(r[3], r[2], 0x05010400u), t3 = __builtin_amdgcn_perm(r[3], r[2], 0x07030602u);
-  c[0] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
-  c[1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
-  c[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
-  c[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
-}
-
 template <class T>
 __global__ __launch_bounds__(256) void reduce_cols_wide_kernel(const T* a, unsigned row, unsigned col,
                                                                unsigned rowsPerSlab, int* out) {
@@ -172,7 +163,7 @@ __global__ __launch_bounds__(256) void reduce_cols_wide_kernel(const T* a, unsig
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
         unsigned c[4];
-        transpose_bytes_4x4(w[d], c);
+        transpose4x4(w[d], c);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           s[4 * d + e] = kSigned ? __builtin_amdgcn_sdot4((int)c[e], 0x01010101, s[4 * d + e], false)

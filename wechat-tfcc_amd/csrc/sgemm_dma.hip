@@ -402,10 +402,6 @@ int launch(hipStream_t stream, const SgemmParams& p) {
 
 namespace sgemm_detail {
 
-bool sgemm_dma_available(int config, int ksplit) {
-  return (config >= 0 && config <= 3 && (ksplit == 1 || ksplit == 2)) || (config == 5 && ksplit == 2);
-}
-
 // Two stages everywhere: more workgroups per CU beat a deeper ring (measured 42.3 against 43.9 us with
 // three stages, 1024 x 3072 x 768 in 64x64 tiles).
 int sgemm_dma_launch(hipStream_t stream, SgemmParams p, int config, int ksplit, bool serialGroups) {

@@ -50,7 +50,6 @@ inline bool set_tiles(SgemmParams& p, unsigned bm, unsigned bn) {
 // 5 = 128x96 (serial groups only); ksplit 1 or 2 groups of wavefronts on one tile (four K groups run on the
 // kernels of sgemm_wave96.hip).
 // Requires B not transposed and operands below 2^30 elements.
-bool sgemm_dma_available(int config, int ksplit);
 // serialGroups: one group of wavefronts per tile does the work of the `ksplit` groups one slab after the other
 // (same additions, same result) - for launches that fill the chip anyway.
 int sgemm_dma_launch(hipStream_t stream, SgemmParams p, int config, int ksplit, bool serialGroups);
