@@ -444,11 +444,11 @@ int tfcc_rocm_lstm_cell_f32(void* stream, unsigned batch, unsigned units, const 
  * tfcc/core/operations/tfcc_rnn.cpp:29-135 behind the products of the inputs.  Per direction: x [seq, batch, 4 units]
  * (inputs times input kernel, gates i, c, f, o), kernel [units, 4 units], bias [4 units], h0 and c0 [batch, units]; out
  * [seq, batch, units] in the order the steps are taken, h and c [batch, units] after the last one; backward: the steps
- * run from the last row of x to the first.  1 to 16 rows, 1 to 1024 units, and at least a CU
- * of the current device for eight units of a direction (else the workspace size is 0).  The workspace needs no particular
- * contents; out, h and c may overlap no input.  wait_us: how long the workgroups wait for one another
- * before the sequence is computed in a single one per direction (0: always that).  Calls of a process on one GPU follow one another, whatever their
- * streams (from the second stream's second call on).  Sequences replayed from graphs do not: two at once that do not fit
+ * run from the last row of x to the first.  1 to 16 rows, 1 to 1024 units, and at least a CU of the current device for eight
+ * units of a direction (else the workspace size is 0).  The workspace needs no particular contents; out, h and c may overlap
+ * no input.  wait_us: how long the workgroups wait for one another before the sequence is computed in a single one per
+ * direction (0: always that).  Calls of a process on one GPU follow one another, whatever their streams (from the second
+ * stream's second call on).  Sequences replayed from graphs do not: two at once that do not fit
  * on the GPU together, or one on a stream confined to fewer CUs than it has workgroups (one for eight units of a
  * direction), end through that wait - the results are the same, the time is not. */
 typedef struct tfcc_rocm_lstm_sequence_desc {
