@@ -1,0 +1,803 @@
+// fp32 matrix product on the bf16 matrix cores: every operand is split into three bf16 numbers that add up to it exactly.
+//
+// The fp32 matrix ops deliver 157 TFLOP/s, the bf16 ones sixteen times that.  A float's 24 bits are three bf16 numbers of
+// eight: x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1, all exact (rounding to nearest halves what is left each time, so
+// the third has room for the rest).  Of the nine products of pieces the six down to 2^-18 of the first are formed, a2 b0,
+// a1 b0, a0 b0, a1 b1, a0 b1, a0 b2; the three left out are below 2^-25 of a b, with either sign.  A matrix op adds sixteen
+// products to its accumulator at once, so even with six times as many of them the sum is rounded less often than by the fp32
+// ops, which take two at a time, and the result is closer to the exact one.  Against 64 bits, relative 2-norm, normal
+// operands: 4096^3 10.1e-7 (fp32 ops 11.5e-7), 1024 x 768 x 3072 1.5e-7 to 2.1e-7 (5.0e-7), 1024 x 3072 x 768 3.0e-7 to 4.3e-7
+// (5.0e-7); operands of one sign behave alike.
+//
+// What the split cannot represent is found and done again.  Infinities, NaN and values that round up to infinity make the
+// results they enter NaN or infinite; operands below 2^-109 leave bits of x2 outside bf16's range, which matters next to a very
+// large partner or in a very small result; products below 2^-126 round where the fp32 op would not.  So every thread keeps the
+// largest magnitude it split (one instruction for two values), and looks at its results: one that is not finite has the
+// workgroup compute its tile again with the fp32 matrix ops; a few below 2^-64, which happens by chance (a sum that cancels to
+// zero, in one product of ten), are summed again one by one; if there are many (a row of zeros), or a magnitude was 2^30 or
+// more, the tile's operands are read once more for their smallest, and that decides.
+//
+// Two kernels.  What they have in common is that vector instructions run under bf16 matrix ops: up to six of them between
+// two of 32 cycles cost next to nothing, if they stand there; a wavefront that issues matrix ops back to back keeps the
+// others' vector instructions waiting.  The order of both loops is therefore written down.
+#include <type_traits>
+
+#include "common.hpp"
+#include "lds_dma.hpp"
+#include "sgemm_params.hpp"
+
+namespace tfcc_rocm {
+
+using sgemm_detail::SgemmParams;
+
+namespace {
+
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+
+// a byte offset that fails the range check of any operand here (below 2^31 bytes, the dispatcher sees to it), also with a
+// tile's rows of one added
+constexpr unsigned kOutside = 0x80000000u;
+
+// f(FROM), f(FROM + 1), ..., f(TO - 1) with the index a constant
+template <int FROM, int TO, class F>
+__device__ __forceinline__ void each(F&& f) {
+  if constexpr (FROM < TO) {
+    f(std::integral_constant<int, FROM>{});
+    each<FROM + 1, TO>(f);
+  }
+}
+
+// Eight consecutive k of a row or column on their way to three operand pieces, in 48 instructions that are dealt out
+// between the matrix ops, few of which need a result of the three before them.
+struct Splitting {
+  v4u piece[3];
+  float e[4];
+};
+constexpr int kSplitOps = 48;
+
+// the piece that is complete, and can be written to LDS, a little before this operation; or -1
+constexpr int written(int op) { return op == 10 ? 0 : op == 30 ? 1 : op == kSplitOps - 1 ? 2 : -1; }
+
+template <int op>
+__device__ __forceinline__ void split_op(float (&x)[8], Splitting& t, float& largest) {
+  if constexpr (op < 8 && op % 2 == 1) {  // (a conversion between two of the magnitudes, which depend on one another)
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(largest) : "v"(x[op - 1]), "v"(x[op]));
+  } else {
+    constexpr int o = op < 8 ? op / 2 : op - 4, stage = o / 20, in = o % 20;  // 4 conversions, then 2 x (4 widened, 4 subtracted)
+    if constexpr (in < 4) {
+      unsigned pair = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f{x[2 * in], x[2 * in + 1]}), v2bf));
+      asm("" : "+v"(pair));  // or the compiler works parts of it out again where they are used
+      t.piece[stage][in] = pair;
+    } else {
+      constexpr int v = (in - 4) / 8 * 4 + (in - 4) % 4;  // the value
+      const unsigned p = t.piece[stage][v / 2];
+      if constexpr ((in - 4) % 8 < 4) t.e[v & 3] = __builtin_bit_cast(float, v & 1 ? p & 0xffff0000u : p << 16);
+      else x[v] -= t.e[v & 3];
+    }
+  }
+}
+
+// the six terms of a product: the pieces of A and of B
+constexpr int kTermA[6] = {2, 1, 0, 1, 0, 0}, kTermB[6] = {0, 0, 0, 1, 1, 2};
+
+__device__ __forceinline__ v16f product(v4u a, v4u b, v16f c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+}
+
+// A tile of the launch and its operands.
+struct Tile {
+  unsigned m0, n0, bi;
+  const float *A, *B, *bias, *R;
+  float* C;
+  unsigned bytesA, bytesB;
+  bool exists;
+};
+template <int BM, int BN, bool TRANSB>
+__device__ __forceinline__ Tile tile_of(const SgemmParams& p) {
+  Tile t;
+  // consecutive workgroup ids land on different XCDs: hand each XCD a contiguous run of tiles
+  const unsigned xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3, L = xcd * p.chunk + slot;
+  t.exists = slot < p.chunk && L < p.tilesTotal;
+  t.bi = udiv_apply(L, p.perBatchMagic, p.perBatchShift);
+  const unsigned w = L - t.bi * p.tilesM * p.tilesN, band = 4u * p.tilesN, b = udiv_apply(w, p.bandMagic, p.bandShift);
+  const unsigned rows = min(4u, p.tilesM - b * 4u), r = w - b * band, q = rows == 4u ? r >> 2 : r / rows;
+  t.m0 = (b * 4u + (r - q * rows)) * BM;
+  t.n0 = q * BN;
+  const unsigned bo = udiv_apply(t.bi, p.innerMagic, p.innerShift), bn = t.bi - bo * p.batchInner;
+  t.A = p.A + (size_t)bo * p.strideA + (size_t)bn * p.innerA;
+  t.B = p.B + (size_t)bo * p.strideB + (size_t)bn * p.innerB;
+  t.bias = p.bias;
+  t.C = p.C + (size_t)bo * p.strideC + (size_t)bn * p.innerC;
+  if (p.groups) {  // selects, not indexing: the argument block stays in scalar registers
+    t.A = p.A;
+    t.B = t.bi == 0 ? p.groupB[0] : t.bi == 1 ? p.groupB[1] : t.bi == 2 ? p.groupB[2] : p.groupB[3];
+    t.bias = t.bi == 0 ? p.groupBias[0] : t.bi == 1 ? p.groupBias[1] : t.bi == 2 ? p.groupBias[2] : p.groupBias[3];
+    t.C = t.bi == 0 ? p.groupC[0] : t.bi == 1 ? p.groupC[1] : t.bi == 2 ? p.groupC[2] : p.groupC[3];
+  }
+  t.R = p.residual ? p.residual + (size_t)t.bi * p.strideR : nullptr;  // dense, flat batch
+  t.bytesA = ((p.M - 1) * p.lda + p.K) * 4u;
+  t.bytesB = TRANSB ? ((p.N - 1) * p.ldb + p.K) * 4u : ((p.K - 1) * p.ldb + p.N) * 4u;
+  return t;
+}
+
+// The smallest magnitude in `rows` rows of `n` floats, as twice its bits less one: zero counts as the largest.
+__device__ __forceinline__ unsigned smallest_of(const float* x, unsigned rows, unsigned n, unsigned ld) {
+  const __amdgpu_buffer_rsrc_t d =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), 0, (int)(((rows - 1) * ld + n) * 4u), 0x00020000);
+  const unsigned pieces = (n + 3) / 4, total = rows * pieces;
+  unsigned least = 0xffffffffu;
+  for (unsigned i = threadIdx.x; i < total; i += 8 * blockDim.x) {
+    v4f v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const unsigned at = i + u * blockDim.x, r = at / pieces;
+      v[u] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(d, at < total ? (r * ld + 4 * (at - r * pieces)) * 4u : kOutside, 0, 0));
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const unsigned at = i + u * blockDim.x, k = 4 * (at - at / pieces * pieces);
+#pragma unroll
+      for (unsigned e = 0; e < 4; ++e)
+        if (k + e < n) least = min(least, (__builtin_bit_cast(unsigned, v[u][e]) << 1) - 1u);
+    }
+  }
+  return least;
+}
+
+// Results that are summed again one by one.
+constexpr unsigned kMostRepairs = 32;
+struct Repairs {
+  unsigned count, at[kMostRepairs];  // row of the tile * 256 + column
+  unsigned least[2];                 // the smallest operands of A and of B
+  float value[kMostRepairs], part[8];
+};
+
+// Whether the workgroup has to compute its tile with the fp32 matrix ops.  Every thread's `largest` operand, whether its
+// results are all finite, and the smallest magnitude among those inside the matrix; list(): adds its results below 2^-64 to
+// `repairs`.  If they are few, their values are there afterwards, for repair_results.
+template <int BM, int BN, bool TRANSB, class List>
+__device__ __forceinline__ bool split_failed(const SgemmParams& p, const Tile& t, float largest, bool finite, float smallestResult,
+                                             Repairs& repairs, List&& list) {
+  if (threadIdx.x == 0) repairs.count = 0;
+  if (threadIdx.x < 2) repairs.least[threadIdx.x] = 0xffffffffu;
+  if (!__syncthreads_or(!finite || largest >= 0x1p30f || smallestResult < 0x1p-64f)) return false;
+  if (__syncthreads_or(!finite)) return true;
+  const bool large = __syncthreads_or(largest >= 0x1p30f) != 0;
+  if (smallestResult < 0x1p-64f) list();
+  __syncthreads();
+  if (large || repairs.count > kMostRepairs) {
+    const unsigned rows = min((unsigned)BM, p.M - t.m0), cols = min((unsigned)BN, p.N - t.n0);
+    const unsigned la = smallest_of(t.A + (size_t)t.m0 * p.lda, rows, p.K, p.lda);
+    const unsigned lb = TRANSB ? smallest_of(t.B + (size_t)t.n0 * p.ldb, cols, p.K, p.ldb) : smallest_of(t.B + t.n0, p.K, cols, p.ldb);
+    __hip_atomic_fetch_min(&repairs.least[0], la, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_min(&repairs.least[1], lb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __syncthreads();
+    if (threadIdx.x == 0) repairs.count = 0;
+    const int ea = (int)(repairs.least[0] >> 24) - 127, eb = (int)(repairs.least[1] >> 24) - 127;  // their exponents
+    return __syncthreads_or(ea < -100 || eb < -100 || (ea + eb < -100 && smallestResult < 0x1p-90f)) != 0;
+  }
+  for (unsigned i = 0; i < repairs.count; ++i) {
+    const unsigned row = t.m0 + (repairs.at[i] >> 8), col = t.n0 + (repairs.at[i] & 255u);
+    float sum = 0.f;
+    for (unsigned k = threadIdx.x; k < p.K; k += blockDim.x)
+      sum = fmaf(t.A[(size_t)row * p.lda + k], TRANSB ? t.B[(size_t)col * p.ldb + k] : t.B[(size_t)k * p.ldb + col], sum);
+    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d);
+    if ((threadIdx.x & 63) == 0) repairs.part[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (unsigned w = 1; w < blockDim.x >> 6; ++w) sum += repairs.part[w];
+      if (t.bias) sum += t.bias[col];
+      if (t.R) sum += t.R[(size_t)row * p.N + col];
+      repairs.value[i] = p.act == 1 ? gelu_erf_f32(sum) : sum;
+    }
+    __syncthreads();
+  }
+  return false;
+}
+
+// Behind the tile store: the whole workgroup.
+__device__ __forceinline__ void repair_results(const SgemmParams& p, const Tile& t, const Repairs& repairs) {
+  if (repairs.count == 0) return;
+  __threadfence_block();
+  __syncthreads();  // the stores of the tile have been made
+  if (threadIdx.x < repairs.count)
+    t.C[(size_t)(t.m0 + (repairs.at[threadIdx.x] >> 8)) * p.ldc + t.n0 + (repairs.at[threadIdx.x] & 255u)] = repairs.value[threadIdx.x];
+}
+
+// ---- large products ------------------------------------------------------------------------------------------------------
+// A workgroup of WGM x WGN wavefronts, a wavefront (32 MI) x (32 NI) outputs.  K goes in slabs of sixteen, one matrix op
+// deep: a thread loads eight values of a row of A and eight of a column of B and splits them on the way from its registers
+// to LDS, once for the workgroup; the wavefronts read the pieces in operand order.  TWO: the five small terms have an
+// accumulator of their own, which brings the error down to 4e-7 at K = 4096, where there are registers for it.
+//
+// Bound by power and the matrix cores: 4096^3 in 256 x 256 tiles 918 -> 561 to 601 us by the box, 229 to 245 TFLOP/s; these matrix ops alone, from
+// registers on the same operands, sustain 302.  In the loop 88 % of the time of its matrix ops alone; without the splitting
+// 92 %, without the writes 94 %, without the barrier 92 %.  (A wavefront for each SIMD on 128 x 128, more slabs on their
+// way, two K groups of such tiles: all slower.)
+template <int MI, int NI, int WGM, int WGN, bool TWO, bool TRANSB>
+__global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const SgemmParams p) {
+  constexpr int BM = 32 * MI * WGM, BN = 32 * NI * WGN, BK = 16, T = 64 * WGM * WGN;
+  static_assert(2 * BM == T && 2 * BN == T, "a thread loads eight values of each operand");
+  // [piece][eight k][row or column] of 16 bytes; 64 bytes between the halves of k put a thread pair's writes on
+  // different banks
+  constexpr int HALF = BM * 16 + 64, PIECE = 2 * HALF, OPERAND = 3 * PIECE, STAGE = 2 * OPERAND;
+
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ Repairs repairs;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wm = wv / WGN, wn = wv - wm * WGN;  // wave-uniform
+  const int tid = threadIdx.x, lane = tid & 63, lrow = lane & 31, g = lane >> 5;
+  const Tile tile = tile_of<BM, BN, TRANSB>(p);
+  if (!tile.exists) return;
+  const unsigned m0 = tile.m0, n0 = tile.n0, M = p.M, N = p.N, K = p.K, lda = p.lda, ldb = p.ldb;
+  const float *A = tile.A, *B = tile.B;
+
+  // ---- loads.  Rows of A (and of B given transposed): two threads to a row, eight k each.  B as stored: a thread to a
+  // column, eight rows.  Past the operands' ends lie zeros (the range check looks at the lane's offset, so the slab's k
+  // is in the descriptor); past the end of a row of A lies the next one, which the last slab masks.
+  const int arow = tid >> 1, ahalf = tid & 1, brow = TRANSB ? tid >> 1 : tid & (BN - 1), bhalf = TRANSB ? tid & 1 : tid / BN;
+  const unsigned aOff = m0 + arow < M ? ((m0 + arow) * lda + 8 * ahalf) * 4u : kOutside;
+  const unsigned bOff = n0 + brow >= N ? kOutside : TRANSB ? ((n0 + brow) * ldb + 8 * bhalf) * 4u : (8 * bhalf * ldb + n0 + brow) * 4u;
+  const unsigned slabs = (K + BK - 1) / BK;
+  struct Raw { float a[8], b[8]; };
+  // the operand from its k `k0` on, `step` bytes to a k: 32-bit scalar arithmetic (a 64-bit comparison would be made on the
+  // vector unit, and the descriptor then read back lane by lane)
+  auto descriptor = [&](const float* base, unsigned k0, unsigned step, unsigned bytes) {
+    const unsigned skip = k0 < K ? k0 * step : 0u;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base) + skip / 4, 0, k0 < K ? (int)(bytes - skip) : 0, 0x00020000);
+  };
+  // one of the ten loads of slab s (TRANSB: four): 0 and 1 are A's
+  auto load = [&](Raw& r, unsigned s, int which) __attribute__((always_inline)) {
+    const unsigned k0 = s * BK;
+    auto quad = [&](float (&x)[8], __amdgpu_buffer_rsrc_t d, unsigned off, int h) {
+      const v4f v = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(d, off + 16 * h, 0, 0));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[4 * h + e] = v[e];
+    };
+    if (which < 2)
+      quad(r.a, descriptor(A, k0, 4u, tile.bytesA), aOff, which);
+    else if (TRANSB)
+      quad(r.b, descriptor(B, k0, 4u, tile.bytesB), bOff, which - 2);
+    else  // (a scalar offset is not range-checked)
+      r.b[which - 2] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(descriptor(B, k0, ldb * 4u, tile.bytesB),
+                                                                                      bOff + (which - 2) * ldb * 4u, 0, 0));
+  };
+  constexpr int LOADS = TRANSB ? 4 : 10;
+  auto mask = [&](Raw& r, unsigned s) {  // the slab in which K ends, or one behind it
+    const int left = (int)K - (int)(s * BK);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      r.a[e] = 8 * ahalf + e < left ? r.a[e] : 0.f;
+      r.b[e] = 8 * bhalf + e < left ? r.b[e] : 0.f;
+    }
+  };
+  float largest = 0.f;
+  unsigned char* const aTo = smem + ahalf * HALF + arow * 16;
+  unsigned char* const bTo = smem + OPERAND + bhalf * HALF + brow * 16;
+
+  v16f main[MI][NI], rest[TWO ? MI : 1][TWO ? NI : 1];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        main[i][j][r] = 0.f;
+        if constexpr (TWO) rest[i][j][r] = 0.f;
+      }
+
+  const unsigned char* const aFrom = smem + g * HALF + (wm * 32 * MI + lrow) * 16;
+  const unsigned char* const bFrom = smem + OPERAND + g * HALF + (wn * 32 * NI + lrow) * 16;
+  Raw raw;
+  Splitting sp;
+  v4u a[3][MI], b[3][NI];
+  // the instructions that split a thread's values: A's, then B's
+  auto splitOp = [&](Raw& r, auto op) __attribute__((always_inline)) {
+    if constexpr (op < kSplitOps) split_op<op>(r.a, sp, largest);
+    else split_op<op - kSplitOps>(r.b, sp, largest);
+  };
+  // each piece is written when it is there, a while before the next: three writes in a row hold the wavefront up
+  // (326 -> 298 us for 192 slabs of 256 x 256)
+  auto put = [&](unsigned char* to, unsigned stage, int i) __attribute__((always_inline)) {
+    *reinterpret_cast<v4u*>(to + stage + i * PIECE) = sp.piece[i];
+  };
+  auto readA = [&](int i, int j, unsigned stage) __attribute__((always_inline)) {
+    a[i][j] = *reinterpret_cast<const v4u*>(aFrom + stage + i * PIECE + j * 512);
+  };
+  auto readB = [&](int i, int j, unsigned stage) __attribute__((always_inline)) {
+    b[i][j] = *reinterpret_cast<const v4u*>(bFrom + stage + i * PIECE + j * 512);
+  };
+
+  // ---- slabs 0 and 1 in LDS, slab 2 on its way, the first operands in registers
+  Raw ahead[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int w = 0; w < LOADS; ++w) {
+      load(ahead[s], s, w);
+      __builtin_amdgcn_sched_barrier(0);  // in the order of the loop, whose waits count on it
+    }
+#pragma unroll
+  for (int w = 0; w < LOADS; ++w) {
+    load(raw, 2, w);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    if ((unsigned)(s + 1) * BK > K) mask(ahead[s], s);
+    each<0, 2 * kSplitOps>([&](auto o) __attribute__((always_inline)) {
+      splitOp(ahead[s], o);
+      if constexpr (written(o % kSplitOps) >= 0) put(o < kSplitOps ? aTo : bTo, s * STAGE, written(o % kSplitOps));
+    });
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < MI; ++i) readA(2, i, 0);
+#pragma unroll
+  for (int j = 0; j < NI; ++j) readB(0, j, 0);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < MI; ++i) readA(1, i, 0);
+#pragma unroll
+  for (int j = 0; j < NI; ++j) readB(1, j, 0);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- A slab is six terms of MI NI matrix ops.  Their order, a2 b0, a1 b0, a0 b0, a1 b1, a0 b1, a0 b2, lets every operand
+  // be read again, for the next slab, well before its first use there; only a0 and b2 are read in their own slab.  Between
+  // the matrix ops the values of the slab after the next are split and written, and the one behind that is asked for.  Of
+  // the three stages one is read, one is complete, one is written, so a single barrier in a slab is enough.
+  constexpr int PT = MI * NI, TOTAL = 6 * PT, SPREAD = 5 * PT;  // SPREAD: matrix ops that the splitting is dealt out behind
+  unsigned st0 = 0, st1 = STAGE, st2 = 2 * STAGE;               // stages of slabs s, s + 1, s + 2
+  for (unsigned s = 0; s < slabs; ++s) {
+    if ((s + 3) * BK > K) mask(raw, s + 2);
+    each<0, TOTAL>([&](auto mc) __attribute__((always_inline)) {
+      constexpr int m = mc, t = m / PT, i = m % PT / NI, j = m % NI;
+      if constexpr (TWO && t != 2)
+        rest[TWO ? i : 0][TWO ? j : 0] = product(a[kTermA[t]][i], b[kTermB[t]][j], rest[TWO ? i : 0][TWO ? j : 0]);
+      else
+        main[i][j] = product(a[kTermA[t]][i], b[kTermB[t]][j], main[i][j]);
+      if (m == 0) __syncthreads();
+      if (m >= 1 && m <= MI) readA(0, m - 1, st0);
+      if (m > MI && m <= MI + NI) readB(2, m - MI - 1, st0);
+      constexpr int from = m < SPREAD ? m * 2 * kSplitOps / SPREAD : 2 * kSplitOps, to = m < SPREAD ? (m + 1) * 2 * kSplitOps / SPREAD : from;
+      each<from, to>([&](auto o) __attribute__((always_inline)) {
+        splitOp(raw, o);
+        if constexpr (written(o % kSplitOps) >= 0) put(o < kSplitOps ? aTo : bTo, st2, written(o % kSplitOps));
+        if constexpr (o == kSplitOps + 3) load(raw, s + 3, 0);
+        if constexpr (o == kSplitOps + 7) load(raw, s + 3, 1);
+      });
+      if (m >= SPREAD && m - SPREAD < (LOADS - 2 + 1) / 2) {
+        load(raw, s + 3, 2 + 2 * (m - SPREAD));
+        load(raw, s + 3, 3 + 2 * (m - SPREAD));
+      }
+      if (m >= 2 * PT && m < 2 * PT + MI) readA(2, m - 2 * PT, st1);
+      if (m >= 3 * PT && m < 3 * PT + NI) readB(0, m - 3 * PT, st1);
+      if (m >= 4 * PT && m < 4 * PT + MI) readA(1, m - 4 * PT, st1);
+      if (m >= 5 * PT && m < 5 * PT + NI) readB(1, m - 5 * PT, st1);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    const unsigned done = st0;
+    st0 = st1;
+    st1 = st2;
+    st2 = done;
+  }
+  if constexpr (TWO) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) main[i][j][r] += rest[i][j][r];
+  }
+
+  // ---- what the split may have got wrong
+  const unsigned rowBase = m0 + wm * MI * 32, colBase = n0 + wn * NI * 32;
+  float notFinite = 0.f, low = 1.f;
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        notFinite = fmaf(main[i][j][r], 0.f, notFinite);
+        low = fminf(low, __builtin_fabsf(main[i][j][r]));
+      }
+  if (rowBase + 32 * MI > M || colBase + 32 * NI > N) {  // the zeros outside the matrix do not count
+    low = 1.f;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (rowBase + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3) < M && colBase + 32 * j + lrow < N)
+            low = fminf(low, __builtin_fabsf(main[i][j][r]));
+  }
+  auto list = [&]() {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const unsigned row = rowBase + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3), col = colBase + 32 * j + lrow;
+          if (__builtin_fabsf(main[i][j][r]) < 0x1p-64f && row < M && col < N) {
+            const unsigned at = atomicAdd(&repairs.count, 1u);
+            if (at < kMostRepairs) repairs.at[at] = (row - m0) << 8 | (col - n0);
+          }
+        }
+  };
+  if (split_failed<BM, BN, TRANSB>(p, tile, largest, notFinite == 0.f, low, repairs, list)) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) main[i][j][r] = 0.f;
+    for (unsigned k = 0; k < K; k += 8) {
+      float x[4][MI], y[4][NI];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const unsigned kk = k + 2 * e + g;
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+          const unsigned row = rowBase + 32 * i + lrow;
+          x[e][i] = kk < K && row < M ? A[(size_t)row * lda + kk] : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          const unsigned col = colBase + 32 * j + lrow;
+          y[e][j] = kk < K && col < N ? TRANSB ? B[(size_t)col * ldb + kk] : B[(size_t)kk * ldb + col] : 0.f;
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; ++j) main[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e][i], y[e][j], main[i][j], 0, 0, 0);
+    }
+  }
+
+  // ---- tile store: + bias, + residual, GELU; rows past M and columns past N fail the range check
+  const bool inside = rowBase < M && colBase < N;
+  const unsigned ldc = p.ldc, rows = inside ? min(M - rowBase, 32u * MI) : 1u;
+  const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(tile.C + (size_t)rowBase * ldc + colBase, 0,
+                                                                      (int)(((rows - 1) * ldc + N - colBase) * 4u), 0x00020000);
+  const float* R = tile.R ? tile.R + (size_t)rowBase * N + colBase : nullptr;
+  float bv[NI];
+  unsigned to[NI], from[NI];
+#pragma unroll
+  for (int j = 0; j < NI; ++j) {
+    const bool in = colBase + 32 * j + lrow < N;
+    bv[j] = tile.bias && in ? tile.bias[colBase + 32 * j + lrow] : 0.f;
+    to[j] = in ? ((4 * g) * ldc + 32 * j + lrow) * 4u : kOutside;
+    from[j] = in ? ((4 * g) * N + 32 * j + lrow) * 4u : kOutside;
+  }
+  auto store_all = [&](bool residual, bool gelu) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t rr =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(R), 0, (int)(((rows - 1) * N + N - colBase) * 4u), 0x00020000);
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const unsigned row = 32 * i + 8 * (r >> 2) + (r & 3);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          float v = main[i][j][r] + bv[j];
+          if (residual) v += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rr, from[j] + row * N * 4u, 0, 0));
+          // same expression as the stand-alone GELU kernel, so that fusing changes no bit
+          if (gelu) v = gelu_erf_f32(v);
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rc, to[j] + row * ldc * 4u, 0, 0);
+        }
+      }
+  };
+  if (inside) {
+    if (p.act == 1) store_all(R != nullptr, true);
+    else store_all(R != nullptr, false);
+  }
+  repair_results(p, tile, repairs);
+}
+
+// ---- products of a few dozen to a few hundred tiles ------------------------------------------------------------------
+// KG wavefronts own 64 x 64 outputs; wavefront q sums the slabs of 32 k q, q + KG, ... for all of them.  Copies go straight to
+// a ring in LDS that belongs to the wavefront, so there is no barrier until the partial tiles meet; a wavefront splits what it
+// multiplies by itself, twice the splitting of a 128 x 128 tile shared by four, and the vector unit bounds the loop: eight of
+// its instructions to a matrix op, 1250 cycles for the 768 that a step's matrix ops take.  (Operands fetched straight to
+// registers: the address unit is the bound, 38 us against 33.5 for 1024 x 3072 x 768.)
+template <int KG, bool TRANSB>
+__global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmParams p) {
+  constexpr int BM = 64, BN = 64, BK = 16, STAGES = 2;
+  constexpr int A_BYTES = BM * BK * 4, B_BYTES = BK * BN * 4, STAGE = A_BYTES + B_BYTES, COPIES = STAGE / 1024;
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ Repairs repairs;
+  const int grp = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63, lrow = lane & 31, g = lane >> 5;
+  unsigned char* gsm = smem + grp * STAGES * STAGE;
+  const unsigned ldsGroup = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)gsm;
+  const Tile tile = tile_of<BM, BN, TRANSB>(p);
+  if (!tile.exists) return;
+  const unsigned m0 = tile.m0, n0 = tile.n0, M = p.M, N = p.N, K = p.K, lda = p.lda, ldb = p.ldb;
+
+  // ---- copies of 1 KB.  Rows of A (and of B given transposed): 64 bytes each, chunk c of 16 bytes of row r at chunk
+  // c ^ (r / 4 & 3); B as stored: k rows of 256 bytes.  The slab's k goes into the descriptor, so what is left of the operand
+  // is what a lane's offset is checked against.
+  const lds_dma_v4i rsrcA = make_rsrc(tile.A, tile.bytesA), rsrcB = make_rsrc(tile.B, tile.bytesB);
+  constexpr int A_COPIES = A_BYTES / 1024, B_COPIES = B_BYTES / 1024;
+  unsigned aOff[A_COPIES], bOff[B_COPIES];
+#pragma unroll
+  for (int u = 0; u < A_COPIES; ++u) {
+    const unsigned r = 16 * u + lane / 4, c = (lane & 3) ^ ((r >> 2) & 3);
+    aOff[u] = m0 + r < M ? ((m0 + r) * lda + 4 * c) * 4u : kOutside;
+    if constexpr (TRANSB) {
+      bOff[u] = n0 + r < N ? ((n0 + r) * ldb + 4 * c) * 4u : kOutside;
+    } else {
+      const unsigned k = 4 * u + lane / 16, col = n0 + 4 * (lane & 15);
+      bOff[u] = col < N ? (k * ldb + col) * 4u : kOutside;
+    }
+  }
+  const unsigned slabs = (K + 31) / 32, steps = 2 * ((slabs + KG - 1) / KG);
+  auto firstK = [&](unsigned s) { return ((s >> 1) * KG + grp) * 32u + (s & 1u) * BK; };
+  auto copy = [&](unsigned s, unsigned stage, int u) __attribute__((always_inline)) {
+    const unsigned k0 = firstK(s);
+    const bool live = k0 < K, isA = u < A_COPIES;
+    const unsigned so = live ? isA || TRANSB ? k0 * 4u : k0 * ldb * 4u : 0u;
+    lds_dma_v4i rsrc = isA ? rsrcA : rsrcB;
+    const unsigned long long base = (((unsigned long long)(unsigned)rsrc[1] << 32) | (unsigned)rsrc[0]) + so;
+    rsrc[0] = (int)(unsigned)base;
+    rsrc[1] = (int)(unsigned)(base >> 32);
+    rsrc[2] = live ? rsrc[2] - (int)so : 0;
+    dma16s(rsrc, ldsGroup + stage * STAGE + u * 1024, isA ? aOff[u] : bOff[u - A_COPIES], 0u);
+  };
+#pragma unroll
+  for (int s = 0; s < STAGES; ++s)
+#pragma unroll
+    for (int u = 0; u < COPIES; ++u) copy(s, s, u);
+
+  // Lane (c, g) holds rows c and 32 + c, columns 2 c and 2 c + 1, and of a slab the k 8 g .. 8 g + 7.
+  struct Raw { float a[2][8], b[2][8]; };
+  auto rowValues = [&](float (&x)[8], const unsigned char* image, int row, int h) __attribute__((always_inline)) {
+    const v4f v = *reinterpret_cast<const v4f*>(image + row * 64 + (((2 * g + h) ^ ((row >> 2) & 3)) << 4));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[4 * h + e] = v[e];
+  };
+  // one of the twelve reads of a slab's values (TRANSB: eight): 0 .. 3 are A's
+  constexpr int READS = TRANSB ? 8 : 12;
+  auto read = [&](Raw& r, unsigned stage, int w) __attribute__((always_inline)) {
+    const unsigned char* st = gsm + stage * STAGE;
+    if (w < 4) {
+      rowValues(r.a[w >> 1], st, 32 * (w >> 1) + lrow, w & 1);
+    } else if (TRANSB) {
+      rowValues(r.b[(w - 4) >> 1], st + A_BYTES, 2 * lrow + ((w - 4) >> 1), w & 1);
+    } else {
+      const v2f v = *reinterpret_cast<const v2f*>(st + A_BYTES + (8 * g + w - 4) * 256 + lrow * 8);
+      r.b[0][w - 4] = v[0];
+      r.b[1][w - 4] = v[1];
+    }
+  };
+  auto mask = [&](Raw& r, unsigned s) __attribute__((always_inline)) {  // the slab in which K ends, or one behind it
+    const int left = (int)K - (int)firstK(s) - 8 * g;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        r.a[i][e] = e < left ? r.a[i][e] : 0.f;
+        if constexpr (TRANSB) r.b[i][e] = e < left ? r.b[i][e] : 0.f;
+      }
+  };
+
+  v16f acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  float largest = 0.f;
+  // Two sets of operands: the matrix ops of a step run on one while the next step's values are split into the other, and
+  // the values of the step after that are read as their registers fall free.
+  Raw raw;
+  Splitting a[2][2], b[2][2];
+  auto splitOp = [&](int set, auto op) __attribute__((always_inline)) {
+    constexpr int o = op % kSplitOps, which = op / kSplitOps;
+    if constexpr (which < 2) split_op<o>(raw.a[which], a[set][which], largest);
+    else split_op<o>(raw.b[which - 2], b[set][which - 2], largest);
+  };
+  wait_vmcnt<COPIES*(STAGES - 1)>();
+#pragma unroll
+  for (int w = 0; w < READS; ++w) read(raw, 0, w);
+  if (firstK(0) + BK > K) mask(raw, 0);
+  each<0, 4 * kSplitOps>([&](auto o) __attribute__((always_inline)) { splitOp(0, o); });
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the reads of slab 0 have returned
+#pragma unroll
+  for (int u = 0; u < COPIES; ++u) copy(2, 0, u);
+  wait_vmcnt<COPIES*(STAGES - 1)>();
+#pragma unroll
+  for (int w = 0; w < READS; ++w) read(raw, 1, w);
+  auto step = [&](unsigned s, auto set) __attribute__((always_inline)) {
+    constexpr int cur = set, nxt = 1 - set;
+    // slab s + 1 is in registers, s + 2 in stage `cur`, s + 3 goes to stage `nxt`
+    if (firstK(s + 1) + BK > K) mask(raw, s + 1);
+    each<0, 24>([&](auto m) __attribute__((always_inline)) {
+      constexpr int t = m / 4, i = m / 2 % 2, j = m % 2;
+      acc[i][j] = product(a[cur][i].piece[kTermA[t]], b[cur][j].piece[kTermB[t]], acc[i][j]);
+      each<8 * m, 8 * m + 8>([&](auto o) __attribute__((always_inline)) { splitOp(nxt, o); });
+      if constexpr (m == 4) __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the reads of slab s + 1 have returned
+      if constexpr (m >= 4 && m <= 7) {
+        copy(s + 3, nxt, 2 * (m - 4));
+        copy(s + 3, nxt, 2 * (m - 4) + 1);
+      }
+      if constexpr (m == 8) wait_vmcnt<COPIES>();
+      if constexpr (m == 8 || m == 9) read(raw, cur, m - 8);     // A's first block is through with operation 47
+      if constexpr (m == 12 || m == 13) read(raw, cur, m - 10);  // its second one with 95
+      if constexpr (m == 23) {
+#pragma unroll
+        for (int w = 4; w < READS; ++w) read(raw, cur, w);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  for (unsigned s = 0; s < steps; s += 2) {  // an even number: two to a slab of 32 k
+    step(s, std::integral_constant<int, 0>{});
+    step(s + 1, std::integral_constant<int, 1>{});
+  }
+  wait_vmcnt<0>();
+  __syncthreads();
+
+  // ---- the partial tiles meet: registers 4 c .. 4 c + 3 of block (i, j) as one quad, in the order of i, c, j; wavefront w
+  // finishes the quads from w QPW on, rows of two neighbouring columns
+  constexpr int QPW = 16 / KG;
+  v4f* meetings = reinterpret_cast<v4f*>(smem);
+  v4f sum[QPW];
+  auto meet = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int i = q >> 3, c = (q >> 1) & 3, j = q & 1;
+      meetings[(grp * 16 + q) * 64 + lane] = v4f{acc[i][j][4 * c], acc[i][j][4 * c + 1], acc[i][j][4 * c + 2], acc[i][j][4 * c + 3]};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < QPW; ++q) {
+      sum[q] = meetings[(grp * QPW + q) * 64 + lane];
+#pragma unroll
+      for (int o = 1; o < KG; ++o) {
+        const v4f w = meetings[(o * 16 + grp * QPW + q) * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[q][e] += w[e];
+      }
+    }
+  };
+  meet();
+  const unsigned ldc = p.ldc, col = n0 + 2 * lrow;
+  auto rowOf = [&](int x, int e) {  // of quads 2 x and 2 x + 1
+    const int q = grp * QPW + 2 * x;
+    return m0 + 32 * (q >> 3) + 8 * ((q >> 1) & 3) + 4 * g + e;
+  };
+  float notFinite = 0.f, low = 1.f;
+#pragma unroll
+  for (int x = 0; x < QPW / 2; ++x)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        notFinite = fmaf(sum[2 * x + j][e], 0.f, notFinite);
+        low = rowOf(x, e) < M && col + j < N ? fminf(low, __builtin_fabsf(sum[2 * x + j][e])) : low;
+      }
+  auto list = [&]() {
+#pragma unroll
+    for (int x = 0; x < QPW / 2; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          if (__builtin_fabsf(sum[2 * x + j][e]) < 0x1p-64f && rowOf(x, e) < M && col + j < N) {
+            const unsigned at = atomicAdd(&repairs.count, 1u);
+            if (at < kMostRepairs) repairs.at[at] = (rowOf(x, e) - m0) << 8 | (col + j - n0);
+          }
+  };
+  if (split_failed<BM, BN, TRANSB>(p, tile, largest, notFinite == 0.f, low, repairs, list)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    for (unsigned s = 0; s < steps; ++s) {
+      float x[8][2], y[8][2];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const unsigned kk = firstK(s) + 2 * e + g;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const unsigned row = m0 + 32 * i + lrow, c = col + i;
+          x[e][i] = kk < K && row < M ? tile.A[(size_t)row * lda + kk] : 0.f;
+          y[e][i] = kk < K && c < N ? TRANSB ? tile.B[(size_t)c * ldb + kk] : tile.B[(size_t)kk * ldb + c] : 0.f;
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e][i], y[e][j], acc[i][j], 0, 0, 0);
+    }
+    __syncthreads();
+    meet();
+  }
+
+  // ---- tile store: + bias, + residual, GELU
+  float bv[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) bv[j] = tile.bias && col + j < N ? tile.bias[col + j] : 0.f;
+#pragma unroll
+  for (int x = 0; x < QPW / 2; ++x)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const unsigned row = rowOf(x, e);
+      if (row >= M) continue;
+      float v[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        v[j] = sum[2 * x + j][e] + bv[j];
+        if (tile.R && col + j < N) v[j] += tile.R[(size_t)row * N + col + j];
+        // same expression as the stand-alone GELU kernel, so that fusing changes no bit
+        if (p.act == 1) v[j] = gelu_erf_f32(v[j]);
+      }
+      float* to = tile.C + (size_t)row * ldc + col;
+      if (col + 1 < N && ((uintptr_t)to & 7) == 0) *reinterpret_cast<v2f*>(to) = v2f{v[0], v[1]};
+      else
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          if (col + j < N) to[j] = v[j];
+    }
+  repair_results(p, tile, repairs);
+}
+
+template <class Kernel>
+int launch(hipStream_t stream, SgemmParams& p, Kernel kern, bool (&attrSet)[16], int bm, int bn, int threads, size_t lds) {
+  if (!sgemm_detail::set_tiles(p, bm, bn)) return set_error(TFCC_ROCM_INVALID_ARGUMENT, "sgemm: too many tiles");
+  int dev = 0;
+  TFCC_HIP_CHECK(hipGetDevice(&dev));
+  TFCC_REQUIRE(dev >= 0 && dev < 16, "device index %d", dev);
+  if (!attrSet[dev]) {  // per device: the attribute belongs to the function on one device
+    TFCC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    attrSet[dev] = true;
+  }
+  hipLaunchKernelGGL(kern, dim3(p.chunk * 8), dim3(threads), lds, stream, p);
+  return check_launch("sgemm");
+}
+
+template <int MI, int NI, int WGM, int WGN, bool TWO, bool TRANSB>
+int launch_shared(hipStream_t stream, SgemmParams p) {
+  constexpr int BM = 32 * MI * WGM, BN = 32 * NI * WGN;
+  constexpr size_t lds = (size_t)3 * (2 * 3 * 2 * (BM * 16 + 64));
+  static_assert(lds <= 159 * 1024, "LDS budget");
+  static bool attrSet[16] = {};
+  return launch(stream, p, sgemm_split_kernel<MI, NI, WGM, WGN, TWO, TRANSB>, attrSet, BM, BN, 64 * WGM * WGN, lds);
+}
+
+template <int KG, bool TRANSB>
+int launch64(hipStream_t stream, SgemmParams p) {
+  static bool attrSet[16] = {};
+  return launch(stream, p, sgemm_split64_kernel<KG, TRANSB>, attrSet, 64, 64, 64 * KG, (size_t)KG * 64 * 64 * 4);
+}
+
+}  // namespace
+
+namespace sgemm_detail {
+
+int sgemm_split_launch(hipStream_t stream, const SgemmParams& p, int config, bool transB) {
+  switch (config) {
+    case 0: return transB ? launch_shared<4, 2, 2, 4, false, true>(stream, p) : launch_shared<4, 2, 2, 4, false, false>(stream, p);
+    case 1: return transB ? launch_shared<2, 2, 2, 2, true, true>(stream, p) : launch_shared<2, 2, 2, 2, true, false>(stream, p);
+    default: return transB ? launch64<4, true>(stream, p) : launch64<4, false>(stream, p);
+  }
+}
+
+}  // namespace sgemm_detail
+}  // namespace tfcc_rocm
