@@ -8,6 +8,9 @@
 // row, loaded as it lies, and a lane turns its 16(k) x 4(n) bytes of B into operand order with byte permutes.  The
 // partial tiles are added in LDS (integer adds: any order gives the same sum) and every thread finishes four columns.
 //
+// With a long K and few tiles one workgroup would make trip after trip to memory while most CUs have nothing to do (3 x
+// 11304 x 910, fifteen tiles: 27 us): several workgroups share the tile's steps then, and add up in memory.
+//
 // Any K, N and alignment: buffer loads take any byte address, and those that would cross the end of an operand are moved
 // back to end with it.  Arithmetic and epilogue
 // are those of gemm_u8s8.hip (tfcc/mkl/operations/tfcc_mklquantization.cpp:33-69,176-201).
@@ -15,6 +18,7 @@
 #include "gemv.hpp"
 #include "qgemm_params.hpp"
 #include "qgemm_small.hpp"
+#include "stream_slots.hpp"
 
 namespace tfcc_rocm {
 
@@ -24,6 +28,12 @@ namespace {
 
 constexpr int kCols = 64;    // columns of a tile
 constexpr int kPitch = 68;   // words per tile row in LDS: the four row groups of a store fall on different banks
+
+// The memory in which the workgroups that share a tile's K meet: a piece per stream, asked for by the first product that
+// is split.  A word per result, the sum in its high half, how many have added to it in the low one; zero between launches.
+constexpr unsigned kMaxResults = 1u << 19;
+int clear_words(hipStream_t stream, void* piece) { return tfcc_rocm_fill_async(stream, piece, 0, 8, kMaxResults); }
+StreamPieces gPieces(kMaxResults * 8, 64, clear_words);  // 4 MB each
 
 // The requantize scalars of the launch; the values themselves where the ranges lie in device memory.
 __device__ __forceinline__ RequantScalars requant_scalars(const QGemmParams& p, float minC, float maxC) {
@@ -76,7 +86,8 @@ __global__ __launch_bounds__(256) void qgemm_tiny_kernel(const QGemmParams p, co
 }
 
 template <int BM, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmParams p, const QSmallOutputs o) {
+__global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmParams p, const QSmallOutputs o, unsigned splits,
+                                                                 unsigned long long* meeting) {
   constexpr int kThreads = WAVES * 64, RB = BM / 16, WORKERS = WAVES - 1;
   __shared__ int tile[BM * kPitch];
   __shared__ int sums[kCols];
@@ -87,12 +98,13 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmPara
   for (int i = tid; i < BM * kPitch; i += kThreads) tile[i] = 0;
   if (tid < kCols) sums[tid] = 0;
 
-  unsigned tm, tn, bi;
+  unsigned tm, tn, bi, tileIndex;
   {
     // each XCD a contiguous run of tiles, the tiles of one column block next to each other: B is the larger operand
     const unsigned xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
     const unsigned L = xcd * p.chunk + slot;
     if (slot >= p.chunk || L >= p.tilesTotal) return;
+    tileIndex = L;
     bi = udiv_apply(L, p.perBatchMagic, p.perBatchShift);
     const unsigned t = L - bi * (p.tilesM * p.tilesN);
     tn = udiv_apply(t, p.bandMagic, p.bandShift);  // here: division by tilesM
@@ -113,7 +125,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmPara
   auto prepare = [&]() __attribute__((always_inline)) {
     int oA, oB;
     float minC, maxC;
-    offsets_and_range(p, blockIdx.x == 0 && lane == 0, oA, oB, minC, maxC);
+    offsets_and_range(p, (blockIdx.x | blockIdx.y) == 0 && lane == 0, oA, oB, minC, maxC);
     if (lane == 0) {
       shared.offsetA = oA;
       shared.offsetB = oB;
@@ -124,7 +136,8 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmPara
     }
   };
 
-  const unsigned steps = (K + 63) / 64;
+  // the workers of all workgroups that share the tile deal its steps among themselves
+  const unsigned steps = (K + 63) / 64, workers = splits * WORKERS, first = blockIdx.y * WORKERS + wave;
   const unsigned offA = (m0 + j) * K + kg * 16, offB = kg * 16 * N + n0 + j * 4;
   v4i acc[RB][4];
 #pragma unroll
@@ -140,12 +153,12 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmPara
   // columns of B past N hold whatever they hold: they are not stored.)
   const unsigned lastA = sizeA - 16, lastB = sizeB - 4;
   if (wave == WORKERS) prepare();
-  else for (unsigned s = wave; s < steps; s += 2 * WORKERS) {
+  else for (unsigned s = first; s < steps; s += 2 * workers) {
     v4i a[2][RB];
     unsigned b[2][16];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const unsigned ka = offA + (s + u * WORKERS) * 64, kb = offB + (s + u * WORKERS) * 64 * N;
+      const unsigned ka = offA + (s + u * workers) * 64, kb = offB + (s + u * workers) * 64 * N;
 #pragma unroll
       for (int q = 0; q < 16; ++q) b[u][q] = __builtin_amdgcn_raw_buffer_load_b32(rsrcB, min(kb + q * N, lastB), 0, 0);
 #pragma unroll
@@ -154,7 +167,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmPara
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const unsigned step = s + u * WORKERS;
+      const unsigned step = s + u * workers;
       if ((step + 1) * 64 + 3 > K) {
         unsigned ka = offA + step * 64, kb = offB + step * 64 * N;
         asm volatile("" : "+v"(ka), "+v"(kb));  // worked out again, instead of keeping every load's offset in a register
@@ -187,7 +200,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmPara
   }
 
   // lane (j, kg) holds rows 16 i + 4 kg + r of column 4 j + e; column 4 j + e lies at word e * 16 + j of its tile row
-  if (wave < (int)min(steps, (unsigned)WORKERS)) {
+  if (wave < WORKERS && first < steps) {
 #pragma unroll
     for (int i = 0; i < RB; ++i)
 #pragma unroll
@@ -211,25 +224,48 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmPara
     const unsigned rt = global + (unsigned)rowsumA[grow] * offsetB;
     const size_t at = (size_t)bi * p.strideC + (size_t)grow * N + gcol;
     const unsigned left = N - gcol;
-    int v[4];
+    unsigned cs[4], sum[4];
+    bool mine[4];  // the results that this thread finishes
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const unsigned cs = e < (int)left ? (unsigned)colsumB[gcol + e] : 0u;
-      const unsigned own = p.colsumExact ? cs : (unsigned)sums[e * 16 + c];
-      v[e] = (int)((unsigned)tile[row * kPitch + e * 16 + c] + 128u * own + cs * offsetA + rt);
+      mine[e] = e < (int)left;
+      cs[e] = mine[e] ? (unsigned)colsumB[gcol + e] : 0u;
+      sum[e] = (unsigned)tile[row * kPitch + e * 16 + c] + (p.colsumExact ? 0u : 128u * (unsigned)sums[e * 16 + c]);
     }
-    const bool four = left >= 4 && p.vectorStores;
+    if (splits > 1) {
+      // One trip to memory and back, no fences: what an addition returns says whether it was the last one, and then it
+      // holds the sum of the others (whole numbers: in any order the same).
+      unsigned long long* const words = meeting + (size_t)tileIndex * (BM * kCols) + idx;
+      unsigned long long before[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (mine[e])
+          before[e] = __hip_atomic_fetch_add(words + e * (BM * 16), ((unsigned long long)sum[e] << 32) | 1ull, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        mine[e] = mine[e] && (unsigned)before[e] == splits - 1;
+        if (!mine[e]) continue;
+        sum[e] += (unsigned)(before[e] >> 32);
+        __hip_atomic_store(words + e * (BM * 16), 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      if (!(mine[0] | mine[1] | mine[2] | mine[3])) continue;
+    }
+    int v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (int)(sum[e] + (p.colsumExact ? 128u * cs[e] : 0u) + cs[e] * offsetA + rt);
+    const bool four = (mine[0] & mine[1] & mine[2] & mine[3]) && p.vectorStores;
     if (p.C) {
       if (four) *reinterpret_cast<v4i*>(p.C + at) = v4i{v[0], v[1], v[2], v[3]};
       else
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (e < (int)left) p.C[at + e] = v[e];
+          if (mine[e]) p.C[at + e] = v[e];
     }
     if (o.f32Out) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (e < (int)left) o.f32Out[at + e] = (float)((double)v[e] * ((double)o.scaleA * (double)o.scaleB[gcol + e]));
+        if (mine[e]) o.f32Out[at + e] = (float)((double)v[e] * ((double)o.scaleA * (double)o.scaleB[gcol + e]));
     }
     if (p.Q) {
       const RequantScalars& rq = shared.rq;
@@ -240,13 +276,13 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmPara
       else
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (e < (int)left) p.Q[at + e] = (unsigned char)q[e];
+          if (mine[e]) p.Q[at + e] = (unsigned char)q[e];
     }
   }
 }
 
 template <int BM, int WAVES>
-int launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o) {
+int launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o, unsigned splits = 1, unsigned long long* meeting = nullptr) {
   p.tilesM = (p.M + BM - 1) / BM;
   p.tilesN = (p.N + kCols - 1) / kCols;
   const unsigned long long total = (unsigned long long)p.tilesM * p.tilesN * p.batch;
@@ -256,14 +292,8 @@ int launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o) {
   const UDiv perBatch = udiv_prepare(p.tilesM * p.tilesN), rows = udiv_prepare(p.tilesM);
   p.perBatchMagic = perBatch.magic; p.perBatchShift = perBatch.shift;
   p.bandMagic = rows.magic; p.bandShift = rows.shift;
-  hipLaunchKernelGGL((qgemm_small_kernel<BM, WAVES>), dim3(p.chunk * 8), dim3(WAVES * 64), 0, stream, p, o);
+  hipLaunchKernelGGL((qgemm_small_kernel<BM, WAVES>), dim3(p.chunk * 8, splits), dim3(WAVES * 64), 0, stream, p, o, splits, meeting);
   return check_launch("quantized matmul (small)");
-}
-
-}  // namespace
-
-bool qgemm_small_supported(const QGemmParams& p) {
-  return ((unsigned long long)p.M + 64) * p.K + 4096 < (1ull << 31) && ((unsigned long long)p.K + 4160) * p.N + 4096 < (1ull << 31);
 }
 
 // Rows per tile and wavefronts by the amount of work, in steps of 16 rows x 64 columns x 64 k (measured, us):
@@ -275,6 +305,64 @@ bool qgemm_small_supported(const QGemmParams& p) {
 // Wavefronts: 4 for at most six steps of k, or when 8 of each tile would be more than eight per CU (1024 x 768 x 768 in 32
 // rows: 8.1 with 4, 10.8 with 8); 16 on the smallest tiles when they are few and K is long (32 x 3292 x 704: 8.4 against
 // 8.7 and 10.7 with 8 and 4); 8 otherwise.
+//
+// A tile's steps go to several workgroups where that saves more trips to memory than the meeting costs.  Microseconds as
+// measured: a pair of steps of every worker is a trip, and a launch takes 3.0 + 1.2 for each trip of four wavefronts, 3.8 +
+// 1.8 of eight, 4.2 + 3 of sixteen, 4 + 2.1 (1.7) in 32 rows of eight (four); the meeting takes 2.4 as long as there are
+// at most eight wavefronts on a CU.  Asked for is 0.7 on top, and more than
+// 20 steps: with the operands in cache 8 x 920 x 552 takes 6.1 in one piece and 6.5 in three.  3 x 11304 x 910 27.3 -> 9.3, 32 x 8192 x 512 18.5 -> 7.8,
+// 92 x 4184 x 115 11.6 -> 7.0, 1 x 3643 x 2512 11.2 -> 7.4, 99 x 3481 x 512 11.7 -> 7.8; 77 x 1001 x 1237 (two trips)
+// would go from 7.0 to 7.8 and is not split.
+struct Plan {
+  unsigned rows, waves;         // of a workgroup that has all of K
+  unsigned splits, splitWaves;  // of tiles of 16 rows; splits 1: not better
+  unsigned cost, splitCost;     // hundredths of a microsecond
+};
+Plan plan_of(unsigned m, unsigned n, unsigned k, unsigned batch) {
+  const unsigned steps = (k + 63) / 64;
+  const unsigned long long columns = (unsigned long long)((n + 63) / 64) * batch;
+  const unsigned long long tiles16 = (m + 15) / 16 * columns, tiles32 = (m + 31) / 32 * columns, tiles64 = (m + 63) / 64 * columns;
+  const unsigned long long work = tiles16 * steps;
+  Plan p{16, 8, 1, 0, 0, ~0u};
+  if (work > 12000 && tiles64 >= 128) p.rows = 64, p.waves = steps <= 6 ? 4 : 8;
+  else if (work > 4096 && m > 16) p.rows = 32, p.waves = steps <= 6 || tiles32 * 8 > 2048 ? 4 : 8;
+  else if (steps <= 6 || tiles16 * 8 > 2048) p.waves = 4;
+  else if (tiles16 <= 128 && steps >= 30) p.waves = 16;
+  auto trips = [&](unsigned waves) { return (steps + 2 * (waves - 1) - 1) / (2 * (waves - 1)); };
+  p.cost = p.rows == 32 ? 400 + (p.waves == 4 ? 170 : 210) * trips(p.waves)
+                        : p.waves == 4 ? 300 + 120 * trips(4) : p.waves == 8 ? 380 + 180 * trips(8) : 420 + 300 * trips(16);
+  if (steps <= 20 || p.rows == 64 || tiles16 * 16 * kCols > kMaxResults) return p;
+  for (unsigned waves = 4; waves <= 8; waves += 4)
+    for (unsigned want = 1; want <= 3; ++want) {  // trips
+      const unsigned splits = (steps + 2 * (waves - 1) * want - 1) / (2 * (waves - 1) * want);
+      const unsigned cost = (waves == 4 ? 300 + 120 * want : 380 + 180 * want) + 240;
+      if (splits < 2 || splits > 32 || tiles16 * splits * waves > 2048 || cost + 70 > p.cost || cost >= p.splitCost) continue;
+      p.splits = splits;
+      p.splitWaves = waves;
+      p.splitCost = cost;
+    }
+  return p;
+}
+
+unsigned long long* meeting_of(hipStream_t stream) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+  return static_cast<unsigned long long*>(gPieces.of(dev, stream));
+}
+
+}  // namespace
+
+void qgemm_small_release_stream(int dev, hipStream_t stream) { gPieces.release(dev, stream); }
+
+bool qgemm_small_supported(const QGemmParams& p) {
+  return ((unsigned long long)p.M + 64) * p.K + 4096 < (1ull << 31) && ((unsigned long long)p.K + 4160) * p.N + 4096 < (1ull << 31);
+}
+
+bool qgemm_small_splits(hipStream_t stream, unsigned m, unsigned n, unsigned k, unsigned instead) {
+  const Plan plan = plan_of(m, n, k, 1);
+  return plan.splits > 1 && plan.splitCost + 70 <= instead && meeting_of(stream) != nullptr;
+}
+
 int qgemm_small_launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o) {
   if ((unsigned long long)p.M * p.K < 16 || (unsigned long long)p.K * p.N < 4) {
     const unsigned long long total = (unsigned long long)p.M * p.N * p.batch;
@@ -283,15 +371,12 @@ int qgemm_small_launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o
     return check_launch("quantized matmul (tiny)");
   }
   p.vectorStores = p.N % 4 == 0 && p.strideC % 4 == 0 && (uintptr_t)p.C % 16 == 0 && (uintptr_t)p.Q % 4 == 0;
-  const unsigned steps = (p.K + 63) / 64;
-  const unsigned long long columns = (unsigned long long)((p.N + 63) / 64) * p.batch;
-  const unsigned long long tiles16 = (p.M + 15) / 16 * columns, tiles32 = (p.M + 31) / 32 * columns, tiles64 = (p.M + 63) / 64 * columns;
-  const unsigned long long work = tiles16 * steps;
-  if (work > 12000 && tiles64 >= 128) return steps <= 6 ? launch<64, 4>(stream, p, o) : launch<64, 8>(stream, p, o);
-  if (work > 4096 && p.M > 16)
-    return steps <= 6 || tiles32 * 8 > 2048 ? launch<32, 4>(stream, p, o) : launch<32, 8>(stream, p, o);
-  if (steps <= 6 || tiles16 * 8 > 2048) return launch<16, 4>(stream, p, o);
-  return tiles16 <= 128 && steps >= 30 ? launch<16, 16>(stream, p, o) : launch<16, 8>(stream, p, o);
+  const Plan plan = plan_of(p.M, p.N, p.K, p.batch);
+  if (unsigned long long* const meeting = plan.splits > 1 ? meeting_of(stream) : nullptr)
+    return plan.splitWaves == 4 ? launch<16, 4>(stream, p, o, plan.splits, meeting) : launch<16, 8>(stream, p, o, plan.splits, meeting);
+  if (plan.rows == 64) return plan.waves == 4 ? launch<64, 4>(stream, p, o) : launch<64, 8>(stream, p, o);
+  if (plan.rows == 32) return plan.waves == 4 ? launch<32, 4>(stream, p, o) : launch<32, 8>(stream, p, o);
+  return plan.waves == 4 ? launch<16, 4>(stream, p, o) : plan.waves == 8 ? launch<16, 8>(stream, p, o) : launch<16, 16>(stream, p, o);
 }
 
 }  // namespace tfcc_rocm

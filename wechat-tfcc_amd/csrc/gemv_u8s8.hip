@@ -322,6 +322,19 @@ int gemv_launch(hipStream_t stream, const unsigned char* a, const signed char* b
   if (gemv_wide_supported(a, b, m, n, k))
     return gemv_wide_launch(stream, false, a, b, rowsumA, colsumB, offsetA, offsetB, ranges, rangeOut, m, n, k, accOut,
                             scaleA, scaleB, f32Out, colsumExact);
+  // The one-pass kernel's workgroups have all of K: 3 us and 0.11 more for every 64 k (8 x 12288 x 512: 24.3 us).  A long
+  // K goes to tiles that several workgroups share (8.4 us), where those may have memory to meet in.
+  QGemmParams q{};
+  q.A = a; q.B = b; q.rowsumA = rowsumA; q.colsumB = colsumB; q.C = accOut;
+  q.strideC = (uint64_t)m * n;
+  q.M = m; q.N = n; q.K = k; q.batch = 1;
+  q.offsetA = offsetA; q.offsetB = offsetB; q.colsumExact = colsumExact ? 1 : 0;
+  if (ranges && ranges[0]) {
+    q.minA = ranges[0]; q.maxA = ranges[1]; q.minB = ranges[2]; q.maxB = ranges[3];
+    if (rangeOut) { q.minC = rangeOut[0]; q.maxC = rangeOut[1]; }
+  }
+  if (qgemm_small_supported(q) && qgemm_small_splits(stream, m, n, k, 300 + 11 * (k / 64)))
+    return qgemm_small_launch(stream, q, QSmallOutputs{f32Out, scaleB, scaleA});
   return gemv_onepass_launch(stream, a, b, rowsumA, colsumB, offsetA, offsetB, ranges, rangeOut, m, n, k, accOut, scaleA,
                              scaleB, f32Out);
 }

@@ -31,5 +31,10 @@ struct QSmallOutputs {
 // Any shape and alignment; operands well below 2^31 bytes.
 bool qgemm_small_supported(const QGemmParams& p);
 int qgemm_small_launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o);
+// Whether the product would be split over several workgroups per tile, and be faster than a kernel that takes `instead`
+// hundredths of a microsecond.
+bool qgemm_small_splits(hipStream_t stream, unsigned m, unsigned n, unsigned k, unsigned instead);
+// Gives back what is kept for `stream` on the device (the stream must be idle).
+void qgemm_small_release_stream(int dev, hipStream_t stream);
 
 }  // namespace tfcc_rocm
