@@ -199,3 +199,19 @@ def test_functions_of_the_cell(pkg, T, function, low, high):
     print(function, low, high, "largest %.3f mean %.4f, library %.3f %.4f" % (ours.max(), ours.mean(), theirs.max(), theirs.mean()))
     # (a hundredth for what the choice of inputs does to a mean, a tenth for the largest of 16384)
     assert ours.max() <= theirs.max() + 0.1 and ours.mean() <= theirs.mean() + 0.01
+
+
+@pytest.mark.parametrize("seq,batch,hidden", [(9, 2, 257), (11, 6, 510), (10, 12, 512), (9, 12, 1024), (13, 5, 601), (70, 4, 514)])
+def test_words_without_a_number(pkg, T, seq, batch, hidden):
+    """more than 256 units: the four sets of words in turn, and values that look like a word nobody has written"""
+    x, sets = setup(T, seq, batch, 40, hidden, 2)
+    outs, keep = launch(pkg, T, x, sets, (False, True))
+    compare(T, outs, x, sets, (False, True))
+    assert gave_up(T, keep) == 0
+    sets[0]["ih"].view(np.uint32)[-1, :] = 0xffffffff
+    outs, keep = launch(pkg, T, x, sets, (False, True))
+    assert gave_up(T, keep) == 0
+    assert np.isnan(T.n(outs[0][0])[:, -1]).all()
+    want = O.lstm_sequence(x[:, :-1], sets[0]["ik"], sets[0]["sk"], sets[0]["bias"], sets[0]["ih"][:-1], sets[0]["ic"][:-1], False)
+    for got, w in zip(outs[0], want):
+        assert rel_fro(T.n(got)[..., :-1, :], w.astype(np.float64)) <= 1e-5

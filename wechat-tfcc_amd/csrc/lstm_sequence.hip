@@ -7,10 +7,17 @@
 // each other through memory: 2.3 us per step, both directions at once (1.7 for 1 x 256, 3.8 for 4 x 1024).  What is left
 // is the way of h to memory and back and the polls that came too early.
 //
-// The exchange is made of 64-bit words of a value and the number of the step it belongs to, written and read as one
-// atomic each: a reader polls the word itself until the step is the one it waits for, so nothing is ordered by fences.
-// Two sets of words alternate; a workgroup writes step t + 2 only after it has read all of step t + 1, which every other
-// workgroup wrote after it had read all of step t, so no word is overwritten before its last reader is through.
+// The exchange is made of words that a reader polls themselves, so nothing is ordered by fences.  There are two kinds:
+//   Up to 256 units 64-bit words of a value and the number of the step it belongs to: a reader waits for its step.  Two
+//   sets of words alternate; a workgroup writes step t + 2 only after it has read all of step t + 1, which every other
+//   workgroup wrote after it had read all of step t, so no word is overwritten before its last reader is through.
+//   With more units half the bytes, and a quarter of the loads, make up for one more store: 32-bit words, a value each,
+//   four to a load.  One that has not been written holds kUnwritten.  Four sets take turns.  A workgroup that has read all
+//   of step t knows that everyone has read all of step t - 1; behind its results for step t + 1 it clears its words of step
+//   t - 1, has seen that clearing done before it stores its results for step t + 2, and those are what a reader has to have
+//   before it looks at the cleared words again, for step t + 3.
+// Served bidirectional sequences, us, all in 64-bit words before: 64 of 4 x 512 218 -> 213, 31 of 7 x 600 206 -> 183, 64 of
+// 4 x 1024 327 -> 301, 32 of 12 x 1024 448 -> 345; in 32-bit words 64 of 1 x 256 take 141 against 131.
 //
 // All workgroups have to run at the same time.  The launcher asks for at most one per CU, but other work may hold CUs, so
 // every wait is bounded: a workgroup that has waited `waitTicks` raises a flag and ends, the others see the flag and end,
@@ -42,26 +49,40 @@ struct SequenceParams {
   unsigned seq, batch, units, directions;
   float forget;
   unsigned blocksPerDirection;
-  unsigned long long* words;  // [2 sets][direction][batch][pitch]: value in the low half, step in the high one
+  unsigned* words;  // [set][direction][batch][pitch]
   unsigned* failed;
   unsigned long long waitTicks;
+  int naps;  // before the first poll of a step
 };
 
 __device__ __forceinline__ float sigmoid_value(float v) { return 1.f / (1.f + expf(0.f - v)); }
 
-__device__ __forceinline__ unsigned long long word_of(float value, unsigned step) {
-  return ((unsigned long long)step << 32) | __builtin_bit_cast(unsigned, value);
+constexpr unsigned kUnwritten = 0xffffffffu;  // (a NaN; another one goes in its place where a value is just this)
+__device__ __forceinline__ unsigned word_of(float value) {
+  const unsigned bits = __builtin_bit_cast(unsigned, value);
+  return bits == kUnwritten ? 0x7fc00000u : bits;
 }
 
-// Step 0 reads the initial h as a word of step 1; the other set holds no step anybody waits for.
+__device__ __forceinline__ unsigned long long numbered_word(float value, unsigned step) {
+  return ((unsigned long long)step << 32) | __builtin_bit_cast(unsigned, value);
+}
+constexpr bool numbered(unsigned pitch) { return pitch <= 256; }  // 64-bit words, with the number of the step
+
+// Step 0 reads the initial h from the first set (as words of step 1); the others hold nothing anybody waits for.  Units that
+// do not exist are zeros in every set.
 __global__ __launch_bounds__(256) void lstm_exchange_init_kernel(SequenceParams p, unsigned pitch, unsigned total) {
   const unsigned i = blockIdx.x * 256 + threadIdx.x;
   if (i == 0) *p.failed = 0;
   if (i >= total) return;
   const unsigned u = i % pitch, b = i / pitch % p.batch, d = i / pitch / p.batch;
   const float h = u < p.units ? p.s[d].h0[(size_t)b * p.units + u] : 0.f;
-  p.words[i] = word_of(h, 1);
-  p.words[(size_t)total + i] = 0;
+  if (numbered(pitch)) {
+    reinterpret_cast<unsigned long long*>(p.words)[i] = numbered_word(h, 1);
+    reinterpret_cast<unsigned long long*>(p.words)[(size_t)total + i] = 0;
+    return;
+  }
+  p.words[i] = word_of(h);
+  for (unsigned set = 1; set < 4; ++set) p.words[(size_t)set * total + i] = u < p.units ? kUnwritten : 0u;
 }
 
 // Sums v[0 .. N) over the lanes that differ in the bits MASK, MASK / 2, ..., U of their number.  While the count is
@@ -120,6 +141,10 @@ __device__ __forceinline__ float of_quad(float v) {
 }
 
 typedef float lstm_v4f __attribute__((ext_vector_type(4)));
+typedef unsigned lstm_v4u __attribute__((ext_vector_type(4)));
+
+constexpr unsigned kNothing = 0x80000000u;  // an offset past every set: reads zeros without a trip to memory
+constexpr int kDeviceScope = 16;            // sc1, as a load of an atomic at device scope has it
 
 // The cell's functions stand in the chain of every step, so they are written without branches and share an exponential and
 // a quotient: with e = e^-|v|, sigmoid(v) = 1 / (1 + e), or e / (1 + e) for negative v, and with e = e^-2|v|, tanh(v) =
@@ -172,8 +197,10 @@ __global__ __launch_bounds__(64 * WAVES) void lstm_sequence_kernel(SequenceParam
   const unsigned units = p.units, batch = p.batch;
   const unsigned d = blockIdx.x / p.blocksPerDirection;
   const Sequence& s = p.s[d];
-  const size_t setSize = (size_t)p.directions * batch * K;
-  unsigned long long* mine = p.words + (size_t)d * batch * K;
+  constexpr bool NUMBERED = numbered(K);
+  constexpr unsigned SIZE = NUMBERED ? 2 : 1;  // of a word, in 32 bits
+  const size_t setSize = (size_t)p.directions * batch * K * SIZE;
+  unsigned* const mine = p.words + (size_t)d * batch * K * SIZE;
   for (int i = tid; i < 2 * MB * LP; i += T) hs[i] = 0.f;  // rows of the batch and units that do not exist stay zero
   if (tid == 0) gaveUp = p.waitTicks == 0;  // no wait at all: the launch behind this one has the sequence
   __syncthreads();
@@ -215,26 +242,25 @@ __global__ __launch_bounds__(64 * WAVES) void lstm_sequence_kernel(SequenceParam
     // up the words it waits for; that the polling wavefronts are the ones that have just finished a step is what keeps
     // most first polls from coming too early (wavefronts that only poll: 4.9 us per step against 2.3).
     float* h = hs + (step & 1u) * (MB * LP);
-    const unsigned long long* words = mine + (step & 1u) * setSize;
-    if constexpr (KI > 8 || Q > 2) __builtin_amdgcn_s_sleep(2);  // with more words per step: 1024 units x 4 rows 4.15 -> 3.8 us
-    const unsigned long long start = wall_clock64();
-    constexpr int PER = (MB * K + T - 1) / T, CHUNK = PER < 8 ? PER : 8;
+    if constexpr (NUMBERED) {
+      const unsigned long long* words = reinterpret_cast<const unsigned long long*>(mine) + (step & 1u) * (setSize / 2);
+      if constexpr (Q > 2) __builtin_amdgcn_s_sleep(2);
+      const unsigned long long start = wall_clock64();
+      constexpr int PER = (MB * K + T - 1) / T;
+      unsigned long long v[PER];
+      bool wanted[PER];
 #pragma unroll
-    for (int k0 = 0; k0 < PER; k0 += CHUNK) {
-      unsigned long long v[CHUNK];
-      bool wanted[CHUNK];
-#pragma unroll
-      for (int k = 0; k < CHUNK; ++k) {
-        const unsigned i = tid + (k0 + k) * T;
+      for (int k = 0; k < PER; ++k) {
+        const unsigned i = tid + k * T;
         wanted[k] = i < batch * K && i % K < units;
       }
       for (unsigned tries = 0;; ++tries) {
         bool ready = true;
 #pragma unroll
-        for (int k = 0; k < CHUNK; ++k)
-          v[k] = wanted[k] ? __hip_atomic_load(words + tid + (k0 + k) * T, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+        for (int k = 0; k < PER; ++k)
+          v[k] = wanted[k] ? __hip_atomic_load(words + tid + k * T, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
 #pragma unroll
-        for (int k = 0; k < CHUNK; ++k) ready = ready && (!wanted[k] || (unsigned)(v[k] >> 32) == step + 1);
+        for (int k = 0; k < PER; ++k) ready = ready && (!wanted[k] || (unsigned)(v[k] >> 32) == step + 1);
         if (ready) break;
         if ((tries & 15u) == 15u &&
             (wall_clock64() - start > p.waitTicks ||
@@ -244,10 +270,48 @@ __global__ __launch_bounds__(64 * WAVES) void lstm_sequence_kernel(SequenceParam
         }
       }
 #pragma unroll
-      for (int k = 0; k < CHUNK; ++k) {
-        const unsigned i = tid + (k0 + k) * T;
+      for (int k = 0; k < PER; ++k) {
+        const unsigned i = tid + k * T;
         if (wanted[k]) h[i / K * LP + i % K] = __builtin_bit_cast(float, (unsigned)v[k]);
       }
+    } else {
+      const unsigned* set = mine + (step & 3u) * setSize;
+      for (int i = 0; i < p.naps; ++i) __builtin_amdgcn_s_sleep(2);
+      const unsigned long long start = wall_clock64();
+      const __amdgpu_buffer_rsrc_t words = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned*>(set), 0, (int)(batch * K * 4), 0x00020000);
+      constexpr int PER = (MB * K / 4 + T - 1) / T;
+      unsigned wanted[PER];  // byte offsets; kNothing: there, or never wanted
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const unsigned i = 4 * (tid + k * T);
+        wanted[k] = i < batch * K && i % K < units ? i * 4u : kNothing;
+      }
+      for (unsigned tries = 0;; ++tries) {
+        asm volatile("" ::: "memory");  // every try asks memory again
+        lstm_v4u v[PER];
+#pragma unroll
+        for (int k = 0; k < PER; ++k)
+          v[k] = __builtin_bit_cast(lstm_v4u, __builtin_amdgcn_raw_buffer_load_b128(words, wanted[k], 0, kDeviceScope));
+        bool ready = true;
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+          const unsigned i = 4 * (tid + k * T);
+          const bool written = v[k][0] != kUnwritten && v[k][1] != kUnwritten && v[k][2] != kUnwritten && v[k][3] != kUnwritten;
+          if (wanted[k] != kNothing && written) {
+            *reinterpret_cast<lstm_v4u*>(h + i / K * LP + i % K) = v[k];
+            wanted[k] = kNothing;
+          }
+          ready = ready && wanted[k] == kNothing;
+        }
+        if (ready) break;
+        if ((tries & 15u) == 15u &&
+            (wall_clock64() - start > p.waitTicks ||
+             __hip_atomic_load(p.failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+          gaveUp = 1;
+          break;
+        }
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's stores of the step before are done
     }
     __syncthreads();
     if (gaveUp) {  // the same for the whole workgroup
@@ -298,9 +362,15 @@ __global__ __launch_bounds__(64 * WAVES) void lstm_sequence_kernel(SequenceParam
     cPrev = c;
     xin = xNext;
     if (valid && gate == 0) {
-      if (!last)
-        __hip_atomic_store(mine + ((step + 1) & 1u) * setSize + (size_t)fm * K + u, word_of(hn, step + 2), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+      if constexpr (NUMBERED) {
+        if (!last)
+          __hip_atomic_store(reinterpret_cast<unsigned long long*>(mine) + ((step + 1) & 1u) * (setSize / 2) + (size_t)fm * K + u,
+                             numbered_word(hn, step + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      } else {
+        unsigned* const word = mine + (size_t)fm * K + u;
+        if (!last) __hip_atomic_store(word + ((step + 1) & 3u) * setSize, word_of(hn), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (step > 0) __hip_atomic_store(word + ((step - 1) & 3u) * setSize, kUnwritten, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
       s.out[(size_t)step * batch * units + at] = hn;
       if (last) {
         s.h[at] = hn;
@@ -345,6 +415,11 @@ int launch(hipStream_t stream, SequenceParams p) {
   constexpr size_t lds = (size_t)2 * 4 * Q * (pitch + 16) * sizeof(float);
   static_assert(lds <= 140 * 1024, "LDS budget");
   p.blocksPerDirection = lstm_plan::workgroups(p.units, 1);
+  // The more words there are, the longer a poll takes, and one that comes too early holds up the words it waits for.  Us
+  // with 0, 1, 4, 9 and 12 naps of 128 cycles: 32 steps of 12 x 1024 436, 429, 410, 344, 345; 40 of 8 x 1000 391, 373, 292,
+  // 298, 302; 40 of 12 x 512 294, 286, 256, 256, 261; 40 of 5 x 600 211, 201, 204, 211, 218; 64 of 4 x 512 215, 217, 223, 238.
+  const unsigned words = p.batch * pitch;
+  p.naps = words <= 2048 ? 0 : words <= 4096 ? 1 : words <= 8192 ? 4 : 9;
   int dev = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));
   TFCC_REQUIRE(dev >= 0 && dev < 16, "device index %d", dev);
@@ -425,7 +500,7 @@ int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc
   }
   p.seq = q->seq; p.batch = q->batch; p.units = q->units; p.directions = q->directions;
   p.forget = q->forget;
-  p.words = static_cast<unsigned long long*>(q->workspace);
+  p.words = static_cast<unsigned*>(q->workspace);
   p.failed = reinterpret_cast<unsigned*>(static_cast<char*>(q->workspace) + need - 64);
   p.waitTicks = (unsigned long long)q->wait_us * 100;  // of the 100 MHz clock
   int dev = 0;
