@@ -35,7 +35,8 @@ def test_against_float64_and_the_transposed_form(pkg, dev, m, n, k):
     assert torch.equal(c[:, :n], out) and bool(torch.isnan(c[:, n:]).all())
 
 
-@pytest.mark.parametrize("m,n,k", [(2048, 2052, 200), (1100, 2700, 300), (600, 1500, 1100), (4096, 4000, 160)])
+@pytest.mark.parametrize("m,n,k", [(2048, 2052, 200), (1100, 2700, 300), (600, 1500, 1100), (4096, 4000, 160), (4000, 4095, 512),
+                                   (2048, 2047, 1024), (1024, 1025, 2050)])
 def test_bias_residual_and_gelu(pkg, dev, m, n, k):
     import torch
     gen = torch.Generator(device=dev).manual_seed(m)

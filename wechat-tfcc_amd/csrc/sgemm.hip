@@ -476,7 +476,10 @@ int k_groups_of_plain_product(unsigned m, unsigned n, unsigned k, unsigned fillB
 // for a k with one, two, ... tiles on it (two 128 x 128 tiles side by side take as long as 1.9, 64 x 64 tiles are multiple); the
 // kernels below reach some 115 TFLOP/s, 105 where a K or an N is no multiple of their pieces.  With an eighth asked for on
 // top, 113 of the 420 come here, 1.33 times as fast on the average, none more than 2 % slower (128 x 128 tiles up to 1.8 times
-// as fast, 64 x 64 up to 2.1, 256 x 256 1.4 to 1.7: 4096^3 911 -> 561 us).  A true batch of short products keeps the kernels
+// as fast, 64 x 64 up to 2.1, 256 x 256 1.4 to 1.7: 4096^3 911 -> 561 us).  A product with an activation, which stands inside
+// a layer, has to be faster by a quarter: 1024 x 768 x 3072 with GELU takes 38.7 us here and 41.8 below, yet the layer
+// around it 326 and 320 (its other products each run a microsecond or two longer behind it), 750 x 1024 x 4096 407 and 402.
+// A true batch of short products keeps the kernels
 // whose sums the attention kernel reproduces.
 int split_configuration(const SgemmParams& p, bool tb, unsigned fillBatch) {
   const unsigned long long m = p.M, n = p.N, k = p.K;
@@ -495,7 +498,7 @@ int split_configuration(const SgemmParams& p, bool tb, unsigned fillBatch) {
   const double costs[3] = {cost256(), cost128(), cost64()};
   const int best = costs[0] <= costs[1] && costs[0] <= costs[2] ? 0 : costs[1] <= costs[2] ? 1 : 2;
   const double rate = k % 32 != 0 || n % 4 != 0 ? 105e6 : 115e6;  // operations in a microsecond
-  return costs[best] < .87 * (4 + 2. * m * n * k * fillBatch / rate) ? best : -1;
+  return costs[best] < (p.act ? .75 : .87) * (4 + 2. * m * n * k * fillBatch / rate) ? best : -1;
 }
 
 // Picks the tile configuration from the shape of one product and the number of batch entries that
