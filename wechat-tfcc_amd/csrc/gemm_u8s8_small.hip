@@ -85,7 +85,7 @@ __global__ __launch_bounds__(256) void qgemm_tiny_kernel(const QGemmParams p, co
   if (p.Q) p.Q[at] = (unsigned char)requantized((int)sum, requant_scalars(p, minC, maxC));
 }
 
-template <int BM, int WAVES>
+template <int BM, int WAVES, bool SHARED>
 __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmParams p, const QSmallOutputs o, unsigned splits,
                                                                  unsigned long long* meeting) {
   constexpr int kThreads = WAVES * 64, RB = BM / 16, WORKERS = WAVES - 1;
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmPara
   auto prepare = [&]() __attribute__((always_inline)) {
     int oA, oB;
     float minC, maxC;
-    offsets_and_range(p, (blockIdx.x | blockIdx.y) == 0 && lane == 0, oA, oB, minC, maxC);
+    offsets_and_range(p, blockIdx.x == 0 && (!SHARED || blockIdx.y == 0) && lane == 0, oA, oB, minC, maxC);
     if (lane == 0) {
       shared.offsetA = oA;
       shared.offsetB = oB;
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmPara
   };
 
   // the workers of all workgroups that share the tile deal its steps among themselves
-  const unsigned steps = (K + 63) / 64, workers = splits * WORKERS, first = blockIdx.y * WORKERS + wave;
+  const unsigned steps = (K + 63) / 64, workers = SHARED ? splits * WORKERS : WORKERS, first = (SHARED ? blockIdx.y * WORKERS : 0u) + wave;
   const unsigned offA = (m0 + j) * K + kg * 16, offB = kg * 16 * N + n0 + j * 4;
   v4i acc[RB][4];
 #pragma unroll
@@ -232,7 +232,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmPara
       cs[e] = mine[e] ? (unsigned)colsumB[gcol + e] : 0u;
       sum[e] = (unsigned)tile[row * kPitch + e * 16 + c] + (p.colsumExact ? 0u : 128u * (unsigned)sums[e * 16 + c]);
     }
-    if (splits > 1) {
+    if constexpr (SHARED) {
       // One trip to memory and back, no fences: what an addition returns says whether it was the last one, and then it
       // holds the sum of the others (whole numbers: in any order the same).
       unsigned long long* const words = meeting + (size_t)tileIndex * (BM * kCols) + idx;
@@ -281,7 +281,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(const QGemmPara
   }
 }
 
-template <int BM, int WAVES>
+template <int BM, int WAVES, bool SHARED = false>
 int launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o, unsigned splits = 1, unsigned long long* meeting = nullptr) {
   p.tilesM = (p.M + BM - 1) / BM;
   p.tilesN = (p.N + kCols - 1) / kCols;
@@ -292,7 +292,7 @@ int launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o, unsigned s
   const UDiv perBatch = udiv_prepare(p.tilesM * p.tilesN), rows = udiv_prepare(p.tilesM);
   p.perBatchMagic = perBatch.magic; p.perBatchShift = perBatch.shift;
   p.bandMagic = rows.magic; p.bandShift = rows.shift;
-  hipLaunchKernelGGL((qgemm_small_kernel<BM, WAVES>), dim3(p.chunk * 8, splits), dim3(WAVES * 64), 0, stream, p, o, splits, meeting);
+  hipLaunchKernelGGL((qgemm_small_kernel<BM, WAVES, SHARED>), dim3(p.chunk * 8, splits), dim3(WAVES * 64), 0, stream, p, o, splits, meeting);
   return check_launch("quantized matmul (small)");
 }
 
@@ -373,7 +373,7 @@ int qgemm_small_launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o
   p.vectorStores = p.N % 4 == 0 && p.strideC % 4 == 0 && (uintptr_t)p.C % 16 == 0 && (uintptr_t)p.Q % 4 == 0;
   const Plan plan = plan_of(p.M, p.N, p.K, p.batch);
   if (unsigned long long* const meeting = plan.splits > 1 ? meeting_of(stream) : nullptr)
-    return plan.splitWaves == 4 ? launch<16, 4>(stream, p, o, plan.splits, meeting) : launch<16, 8>(stream, p, o, plan.splits, meeting);
+    return plan.splitWaves == 4 ? launch<16, 4, true>(stream, p, o, plan.splits, meeting) : launch<16, 8, true>(stream, p, o, plan.splits, meeting);
   if (plan.rows == 64) return plan.waves == 4 ? launch<64, 4>(stream, p, o) : launch<64, 8>(stream, p, o);
   if (plan.rows == 32) return plan.waves == 4 ? launch<32, 4>(stream, p, o) : launch<32, 8>(stream, p, o);
   return plan.waves == 4 ? launch<16, 4>(stream, p, o) : plan.waves == 8 ? launch<16, 8>(stream, p, o) : launch<16, 16>(stream, p, o);
