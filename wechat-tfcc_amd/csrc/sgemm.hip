@@ -475,10 +475,11 @@ int k_groups_of_plain_product(unsigned m, unsigned n, unsigned k, unsigned fillB
 // rows and 64 .. 8192 for K and N, are met within a fifth by a constant, one per round of tiles, and K times what a CU takes
 // for a k with one, two, ... tiles on it (two 128 x 128 tiles side by side take as long as 1.9, 64 x 64 tiles are multiple); the
 // kernels below reach some 115 TFLOP/s, 105 where a K or an N is no multiple of their pieces.  With an eighth asked for on
-// top, 113 of the 420 come here, 1.33 times as fast on the average, none more than 2 % slower (128 x 128 tiles up to 1.8 times
-// as fast, 64 x 64 up to 2.1, 256 x 256 1.4 to 1.7: 4096^3 911 -> 561 us).  A product with an activation, which stands inside
-// a layer, has to be faster by a quarter: 1024 x 768 x 3072 with GELU takes 38.7 us here and 41.8 below, yet the layer
-// around it 326 and 320 (its other products each run a microsecond or two longer behind it), 750 x 1024 x 4096 407 and 402.
+// top a quarter of them comes here, 1.3 times as fast on the average (128 x 128 tiles up to 1.8 times
+// as fast, 64 x 64 up to 2.1, 256 x 256 1.4 to 1.7: 4096^3 911 -> 561 us).  64 x 64 tiles have to be
+// faster by a quarter where the product below takes less than 60 us: those that are not gain 6 % on the average and lose up to
+// 7 (704 x 2847 x 455), and in a layer of other products less than nothing, because these run a microsecond or two longer
+// behind them (1024 x 768 x 3072 with GELU 38.7 us here and 41.8 below, the layer around it 326 and 320).
 // A true batch of short products keeps the kernels
 // whose sums the attention kernel reproduces.
 int split_configuration(const SgemmParams& p, bool tb, unsigned fillBatch) {
@@ -498,7 +499,8 @@ int split_configuration(const SgemmParams& p, bool tb, unsigned fillBatch) {
   const double costs[3] = {cost256(), cost128(), cost64()};
   const int best = costs[0] <= costs[1] && costs[0] <= costs[2] ? 0 : costs[1] <= costs[2] ? 1 : 2;
   const double rate = k % 32 != 0 || n % 4 != 0 ? 105e6 : 115e6;  // operations in a microsecond
-  return costs[best] < (p.act ? .75 : .87) * (4 + 2. * m * n * k * fillBatch / rate) ? best : -1;
+  const double below = 4 + 2. * m * n * k * fillBatch / rate;
+  return costs[best] < (best == 2 && below < 60 ? .75 : .87) * below ? best : -1;
 }
 
 // Picks the tile configuration from the shape of one product and the number of batch entries that
