@@ -439,6 +439,13 @@ int qgemm_dma_launch(hipStream_t stream, const QGemmParams& p, bool requant) {
     if (qgemm_w4_supported(p)) return qgemm_w4_launch(stream, p, requant);
     return launch_for_outputs<256, 256, 2, 4, 2>(stream, p, requant);
   }
+  // At most one 64x128 tile for each CU: with a CU to itself a workgroup waits for its slabs, not for the matrix cores (a
+  // slab of 128 k every 0.53 us with one on its way, 0.41 with three), so its ring takes four stages.  us, two -> four: 256 x
+  // 4096 x 4096 21.0 -> 17.2, 640 x 4096 x 1024 20.6 -> 17.0, 1024 x 4096 x 2048 24.8 (in 128x128) -> 18.4, 2048 x 1024 x
+  // 1024 11.1 -> 9.3; six stages 19.4, 19.2, 20.7, 10.2.  Up to 768 k there is no difference (1024 x 768 x 768 7.2), and
+  // with more tiles, which then run one after another, four are slower (1024 x 768 x 3072 11.5 against 14.7).
+  const unsigned long long narrow = (unsigned long long)((p.M + 63) / 64) * ((p.N + 127) / 128) * p.batch;
+  if (narrow <= 256 && p.K > 768) return launch_for_outputs<64, 128, 1, 4, 4>(stream, p, requant);
   // fewer than half a chip of 128x128 tiles: 64x128 tiles (four wavefronts side by side) put twice as many CUs to work
   const unsigned long long mid = (unsigned long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
   if (mid < 128) return launch_for_outputs<64, 128, 1, 4, 2>(stream, p, requant);
