@@ -100,3 +100,21 @@ def test_results_that_cancel(pkg, dev):
     out = pkg.blas_matmul(a, b, bias)
     assert out[100, 40] == bias[40]
     assert rel(out, a.double() @ b.double() + bias.double()) <= bound(k)
+
+
+@pytest.mark.parametrize("place", [0, 5, 134, 255])
+@pytest.mark.parametrize("m,n,k", [(2048, 2048, 256), (1020, 1022, 2050)])
+def test_an_operand_below_the_pieces_range_at_any_place(pkg, dev, m, n, k, place):
+    """One subnormal operand, wherever it lies in its four, next to a large partner: the only thing wrong with its tile."""
+    import torch
+    gen = torch.Generator(device=dev).manual_seed(place)
+    a, b = torch.randn(m, k, device=dev, generator=gen), torch.randn(k, n, device=dev, generator=gen)
+    a[:, place], b[place, :] = 0.0, 2.0 ** 100
+    a[200] = 0.0
+    a[200, place] = 2.0 ** -140
+    assert torch.equal(pkg.blas_matmul(a, b)[200], torch.full((n,), 2.0 ** -40, device=dev))
+    a, b = b.t().contiguous(), a.t().contiguous()  # and in B, as stored and transposed
+    assert torch.equal(pkg.blas_matmul(a, b)[:, 200], torch.full((n,), 2.0 ** -40, device=dev))
+    c = torch.empty(n, m, device=dev)
+    pkg.sgemm_general(a, b.t().contiguous(), c, n, m, k, k, k, m, trans_b=True)
+    assert torch.equal(c[:, 200], torch.full((n,), 2.0 ** -40, device=dev))

@@ -132,18 +132,18 @@ __device__ __forceinline__ unsigned smallest_of(const float* x, unsigned rows, u
   const unsigned pieces = (n + 3) / 4, total = rows * pieces;
   unsigned least = 0xffffffffu;
   for (unsigned i = threadIdx.x; i < total; i += 8 * blockDim.x) {
-    v4f v[8];
+    v4u v[8];  // whole numbers from the start: a bit_cast of a vector's element reads its first one
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const unsigned at = i + u * blockDim.x, r = at / pieces;
-      v[u] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(d, at < total ? (r * ld + 4 * (at - r * pieces)) * 4u : kOutside, 0, 0));
+      v[u] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(d, at < total ? (r * ld + 4 * (at - r * pieces)) * 4u : kOutside, 0, 0));
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const unsigned at = i + u * blockDim.x, k = 4 * (at - at / pieces * pieces);
 #pragma unroll
       for (unsigned e = 0; e < 4; ++e)
-        if (k + e < n) least = min(least, (__builtin_bit_cast(unsigned, v[u][e]) << 1) - 1u);
+        if (k + e < n) least = min(least, (v[u][e] << 1) - 1u);
     }
   }
   return least;
