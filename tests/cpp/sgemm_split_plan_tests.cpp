@@ -1,0 +1,45 @@
+// The rule that sends fp32 products to the kernels on the bf16 matrix cores (wechat-tfcc_amd/csrc/sgemm_split_plan.hpp), on the
+// host.  Without arguments: its limits.  With some, groups of m n k batch: prints the kernel that takes each product.  No GPU.
+#include <cstdio>
+#include <cstdlib>
+#include <initializer_list>
+
+#include "sgemm_split_plan.hpp"
+
+using namespace tfcc_rocm::sgemm_split_plan;
+
+static int failures = 0;
+#define EXPECT(cond)                                         \
+  do {                                                       \
+    if (!(cond)) {                                           \
+      ++failures;                                            \
+      std::printf("FAIL line %d: %s\n", __LINE__, #cond);    \
+    }                                                        \
+  } while (0)
+
+static int plain(unsigned m, unsigned n, unsigned k, unsigned batch = 1, bool transB = false) {
+  return kernel_of(m, n, k, k, transB ? k : n, n, transB, batch);
+}
+
+int main(int argc, char** argv) {
+  if (argc > 1) {
+    for (int i = 1; i + 3 < argc; i += 4)
+      std::printf("%d\n", plain(std::atoi(argv[i]), std::atoi(argv[i + 1]), std::atoi(argv[i + 2]), std::atoi(argv[i + 3])));
+    return 0;
+  }
+  EXPECT(plain(4096, 4096, 4096) == kWide && plain(2048, 2048, 2048) == k128 && plain(1024, 1024, 2048) == k64);
+  for (unsigned m : {1u, 8u, 47u, 4096u})  // few rows, few columns, short K, few tiles: the fp32 matrix ops
+    EXPECT(plain(m, 47, 4096) == kNone && plain(47, m, 4096) == kNone && plain(m, 4096, 127) == kNone && plain(m, 64, 4096) == kNone);
+  EXPECT(plain(64, 127 * 64, 8192) == kNone && plain(512, 512, 191, 64) == kNone);
+  // the reach of the kernels' 32-bit byte offsets
+  EXPECT(kernel_of(4096, 4096, 4096, (1u << 29) / (4096 + 256) + 1, 4096, 4096, false, 1) == kNone);
+  EXPECT(kernel_of(4096, 4096, 4096, 4096, (1u << 29) / (4096 + 256) + 1, 4096, false, 1) == kNone);
+  EXPECT(kernel_of(4096, 4096, 4096, 4096, (1u << 29) / (4096 + 256) + 1, 4096, true, 1) == kNone);
+  EXPECT(kernel_of(4096, 4096, 4096, 4096, 4096, 1u << 21, false, 1) == kNone);
+  // B given transposed is summed as B as stored, so the same kernel has to take it
+  for (unsigned m = 48; m <= 6000; m = m * 5 / 4 + 1)
+    for (unsigned n = 48; n <= 9000; n = n * 5 / 4 + 1)
+      for (unsigned k = 128; k <= 9000; k = k * 4 / 3 + 1) EXPECT(plain(m, n, k) == plain(m, n, k, 1, true));
+  if (failures == 0) std::printf("sgemm split plan: all passed\n");
+  return failures != 0;
+}

@@ -15,6 +15,7 @@
 // wavefront's column range) so that a lane owns NI consecutive output columns.
 #include "common.hpp"
 #include "sgemm_params.hpp"
+#include "sgemm_split_plan.hpp"
 
 namespace tfcc_rocm {
 
@@ -470,39 +471,6 @@ int k_groups_of_plain_product(unsigned m, unsigned n, unsigned k, unsigned fillB
   return ksplit;
 }
 
-// Which of the kernels of sgemm_split.hip takes the product: 0 for 256 x 256 tiles, 1 for 128 x 128, 2 for 64 x 64 with four K
-// groups, or -1: the ones below are as fast or faster.  Measured times of 420 shapes, even over the logarithm of 64 .. 4096
-// rows and 64 .. 8192 for K and N, are met within a fifth by a constant, one per round of tiles, and K times what a CU takes
-// for a k with one, two, ... tiles on it (two 128 x 128 tiles side by side take as long as 1.9, 64 x 64 tiles are multiple); the
-// kernels below reach some 115 TFLOP/s, 105 where a K or an N is no multiple of their pieces.  With an eighth asked for on
-// top a quarter of them comes here, 1.3 times as fast on the average (128 x 128 tiles up to 1.8 times
-// as fast, 64 x 64 up to 2.1, 256 x 256 1.4 to 1.7: 4096^3 911 -> 561 us).  64 x 64 tiles have to be
-// faster by a quarter where the product below takes less than 60 us: those that are not gain 6 % on the average and lose up to
-// 7 (704 x 2847 x 455), and in a layer of other products less than nothing, because these run a microsecond or two longer
-// behind them (1024 x 768 x 3072 with GELU 38.7 us here and 41.8 below, the layer around it 326 and 320).
-// A true batch of short products keeps the kernels
-// whose sums the attention kernel reproduces.
-int split_configuration(const SgemmParams& p, bool tb, unsigned fillBatch) {
-  const unsigned long long m = p.M, n = p.N, k = p.K;
-  if (m < 48 || n < 48 || k < (fillBatch > 1 ? 192 : 128)) return -1;
-  // byte offsets of whole operands and of a tile's rows of the result fit 31 and 30 bits
-  if ((m + 256) * p.lda >= (1u << 29) || ((tb ? n : k) + 256) * p.ldb >= (1u << 29) || p.ldc >= (1u << 21)) return -1;
-  auto tiles = [&](unsigned b) { return ((m + b - 1) / b) * ((n + b - 1) / b) * fillBatch; };
-  const unsigned long long t64 = tiles(64), t128 = tiles(128), t256 = tiles(256);
-  if (t64 < 128) return -1;
-  auto cost256 = [&] { const unsigned long long r = t256 % 256; return 8 + k * (t256 / 256 * .1406 + (r ? .0906 + r * .000195 : 0)); };
-  auto cost128 = [&] {
-    const unsigned long long r = t128 % 512;
-    return 9 + k * (t128 / 512 * .0813 + (r == 0 ? 0 : r <= 256 ? .0403 : .0403 + (r - 256) * .000151));
-  };
-  auto cost64 = [&] { return 4 + 4.5 * ((t64 + 511) / 512) + k * .0108 * ((t64 + 255) / 256); };
-  const double costs[3] = {cost256(), cost128(), cost64()};
-  const int best = costs[0] <= costs[1] && costs[0] <= costs[2] ? 0 : costs[1] <= costs[2] ? 1 : 2;
-  const double rate = k % 32 != 0 || n % 4 != 0 ? 105e6 : 115e6;  // operations in a microsecond
-  const double below = 4 + 2. * m * n * k * fillBatch / rate;
-  return costs[best] < (best == 2 && below < 60 ? .75 : .87) * below ? best : -1;
-}
-
 // Picks the tile configuration from the shape of one product and the number of batch entries that
 // count towards filling the chip (`fillBatch`), and launches.
 int dispatch(hipStream_t s, const SgemmParams& p, bool vec, bool small, bool tb, unsigned fillBatch) {
@@ -512,8 +480,8 @@ int dispatch(hipStream_t s, const SgemmParams& p, bool vec, bool small, bool tb,
   if (fillBatch == 1 && small && sgemm_detail::sgemm_skinny_better(m, n, k))
     return sgemm_detail::sgemm_skinny_launch(s, p, tb);
   if (small) {
-    const int split = split_configuration(p, tb, fillBatch);
-    if (split >= 0) return sgemm_detail::sgemm_split_launch(s, p, split, tb);
+    const int split = sgemm_split_plan::kernel_of(m, n, k, p.lda, p.ldb, p.ldc, tb, fillBatch);
+    if (split != sgemm_split_plan::kNone) return sgemm_detail::sgemm_split_launch(s, p, split, tb);
   }
   if (tb) {
     const int groups = k_groups_of_plain_product(m, n, k, fillBatch);

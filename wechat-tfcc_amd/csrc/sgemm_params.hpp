@@ -61,10 +61,10 @@ int sgemm_dma_launch(hipStream_t stream, SgemmParams p, int config, int ksplit, 
 // (blocks 3 or 4).  Same requirements and the same bits as the kernels above for the same number of K groups.
 int sgemm_wave96_launch(hipStream_t stream, SgemmParams p, int ksplit, int blocks = 3, int rowBlocks = 0);
 
-// The kernels on the bf16 matrix cores (sgemm_split.hip), operands split into three exact parts: tiles of 256 x 256
-// (config 0), 128 x 128 (1), 64 x 64 with four K groups (2).  Any alignment, B as stored or transposed (the same bits); operands
+// The kernels on the bf16 matrix cores (sgemm_split.hip), operands split into three exact parts.  `kernel`: one of
+// sgemm_split_plan.hpp.  Any alignment, B as stored or transposed (the same bits); operands
 // below 2^29 elements, rows of C below 2^21.
-int sgemm_split_launch(hipStream_t stream, const SgemmParams& p, int config, bool transB);
+int sgemm_split_launch(hipStream_t stream, const SgemmParams& p, int kernel, bool transB);
 
 // The streaming kernel for up to eight rows of A (sgemv.hip): any K, N, strides and alignment; B not transposed.
 bool sgemv_supported(const SgemmParams& p);

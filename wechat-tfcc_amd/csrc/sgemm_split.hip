@@ -2,12 +2,21 @@
 //
 // The fp32 matrix ops deliver 157 TFLOP/s, the bf16 ones sixteen times that.  A float's 24 bits are three bf16 numbers of
 // eight: x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1, all exact (rounding to nearest halves what is left each time, so
-// the third has room for the rest).  Of the nine products of pieces the six down to 2^-18 of the first are formed, a2 b0,
-// a1 b0, a0 b0, a1 b1, a0 b1, a0 b2; the three left out are below 2^-25 of a b, with either sign.  A matrix op adds sixteen
-// products to its accumulator at once, so even with six times as many of them the sum is rounded less often than by the fp32
-// ops, which take two at a time, and the result is closer to the exact one.  Against 64 bits, relative 2-norm, normal
-// operands: 4096^3 10.1e-7 (fp32 ops 11.5e-7), 1024 x 768 x 3072 1.5e-7 to 2.1e-7 (5.0e-7), 1024 x 3072 x 768 3.0e-7 to 4.3e-7
-// (5.0e-7); operands of one sign behave alike.
+// the third has room for the rest).  Of the nine products of pieces the six largest are formed, a2 b0, a1 b0, a0 b0, a1 b1,
+// a0 b1, a0 b2.  The three left out come to 2^-24.2 of a b at most (2^-28 on the average, with either sign), so a product
+// by itself may be off by one unit in the last place instead of half a one.
+//
+// a0 b0 has an accumulator of its own.  Its products have sixteen bits, so their sums are exact or nearly so, and the
+// five small terms meet in a second one 2^8 below; the two are added once, at the end.  (All six in one accumulator take half
+// the registers, but there the small terms are rounded at the size of the result: fewer roundings than in the fp32 ops for
+// dense operands, which take two k at a time, but more for sparse ones, where an fp32 op adds one product or none.)
+// Against 64 bits, relative 2-norm in 1e-8, here, in one accumulator, and with the fp32 ops:
+//                  4096^3, 128 x 256 tiles   1024 x 1024 x 2048, 64 x 64   2048^3, 128 x 128 (always in two)
+//   normal           40   101   115             13.4   35.2   57.5            27.2   80.9
+//   relu(normal)     32    94    81             10.6   33.7   40.5            21.6   57.7
+//   10 % dense       14    64    36              6.6   24.5   18.5             9.6   25.7
+//   2 % dense         6.4  34    16              5.1   13.8    8.9             4.8   11.7
+//   one in a row      2.6   5.4   2.5            2.6    5.4    2.5             2.6    2.5
 //
 // What the split cannot represent is found and done again.  Infinities, NaN and values that round up to infinity make the
 // results they enter NaN or infinite; operands below 2^-109 leave bits of x2 outside bf16's range, which matters next to a very
@@ -25,6 +34,7 @@
 #include "common.hpp"
 #include "lds_dma.hpp"
 #include "sgemm_params.hpp"
+#include "sgemm_split_plan.hpp"
 
 namespace tfcc_rocm {
 
@@ -35,6 +45,7 @@ namespace {
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
@@ -52,31 +63,33 @@ __device__ __forceinline__ void each(F&& f) {
   }
 }
 
-// Eight consecutive k of a row or column on their way to three operand pieces, in 48 instructions that are dealt out
-// between the matrix ops, few of which need a result of the three before them.
+// V (four or eight) consecutive k of a row or column on their way to three operand pieces, in 6 V instructions that are dealt
+// out between the matrix ops, few of which need a result of the three before them.
+template <int V>
 struct Splitting {
-  v4u piece[3];
+  unsigned piece[3][V / 2];
   float e[4];
 };
-constexpr int kSplitOps = 48;
 
 // the piece that is complete, and can be written to LDS, a little before this operation; or -1
-constexpr int written(int op) { return op == 10 ? 0 : op == 30 ? 1 : op == kSplitOps - 1 ? 2 : -1; }
+template <int V>
+constexpr int written(int op) { return op == V + 2 ? 0 : op == V / 2 * 7 + 2 ? 1 : op == 6 * V - 1 ? 2 : -1; }
 
-template <int op>
-__device__ __forceinline__ void split_op(float (&x)[8], Splitting& t, float& largest) {
-  if constexpr (op < 8 && op % 2 == 1) {  // (a conversion between two of the magnitudes, which depend on one another)
+template <int V, int op>
+__device__ __forceinline__ void split_op(float (&x)[V], Splitting<V>& t, float& largest) {
+  if constexpr (op < V && op % 2 == 1) {  // (a conversion between two of the magnitudes, which depend on one another)
     asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(largest) : "v"(x[op - 1]), "v"(x[op]));
   } else {
-    constexpr int o = op < 8 ? op / 2 : op - 4, stage = o / 20, in = o % 20;  // 4 conversions, then 2 x (4 widened, 4 subtracted)
-    if constexpr (in < 4) {
+    // V / 2 conversions, then twice: V widened and subtracted, four at a time, and V / 2 conversions
+    constexpr int H = V / 2, o = op < V ? op / 2 : op - H, stage = o / (5 * H), in = o % (5 * H);
+    if constexpr (in < H) {
       unsigned pair = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f{x[2 * in], x[2 * in + 1]}), v2bf));
       asm("" : "+v"(pair));  // or the compiler works parts of it out again where they are used
       t.piece[stage][in] = pair;
     } else {
-      constexpr int v = (in - 4) / 8 * 4 + (in - 4) % 4;  // the value
+      constexpr int v = (in - H) / 8 * 4 + (in - H) % 4;  // the value
       const unsigned p = t.piece[stage][v / 2];
-      if constexpr ((in - 4) % 8 < 4) t.e[v & 3] = __builtin_bit_cast(float, v & 1 ? p & 0xffff0000u : p << 16);
+      if constexpr ((in - H) % 8 < 4) t.e[v & 3] = __builtin_bit_cast(float, v & 1 ? p & 0xffff0000u : p << 16);
       else x[v] -= t.e[v & 3];
     }
   }
@@ -84,10 +97,11 @@ __device__ __forceinline__ void split_op(float (&x)[8], Splitting& t, float& lar
 
 // the six terms of a product: the pieces of A and of B
 constexpr int kTermA[6] = {2, 1, 0, 1, 0, 0}, kTermB[6] = {0, 0, 0, 1, 1, 2};
-
 __device__ __forceinline__ v16f product(v4u a, v4u b, v16f c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
 }
+
+__device__ __forceinline__ v4u operand(const unsigned (&x)[4]) { return v4u{x[0], x[1], x[2], x[3]}; }
 
 // A tile of the launch and its operands.
 struct Tile {
@@ -211,21 +225,30 @@ __device__ __forceinline__ void repair_results(const SgemmParams& p, const Tile&
 
 // ---- large products ------------------------------------------------------------------------------------------------------
 // A workgroup of WGM x WGN wavefronts, a wavefront (32 MI) x (32 NI) outputs.  K goes in slabs of sixteen, one matrix op
-// deep: a thread loads eight values of a row of A and eight of a column of B and splits them on the way from its registers
-// to LDS, once for the workgroup; the wavefronts read the pieces in operand order.  TWO: the five small terms have an
-// accumulator of their own, which brings the error down to 4e-7 at K = 4096, where there are registers for it.
+// deep: a thread loads four or eight values of a row of A and eight of a column of B and splits them on the way from its
+// registers to LDS, once for the workgroup; the wavefronts read the pieces in operand order.
 //
-// Bound by power and the matrix cores: 4096^3 in 256 x 256 tiles 918 -> 561 to 601 us by the box, 229 to 245 TFLOP/s; these matrix ops alone, from
-// registers on the same operands, sustain 302.  In the loop 88 % of the time of its matrix ops alone; without the splitting
-// 92 %, without the writes 94 %, without the barrier 92 %.  (A wavefront for each SIMD on 128 x 128, more slabs on their
-// way, two K groups of such tiles: all slower.)
-template <int MI, int NI, int WGM, int WGN, bool TWO, bool TRANSB>
-__global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const SgemmParams p) {
-  constexpr int BM = 32 * MI * WGM, BN = 32 * NI * WGN, BK = 16, T = 64 * WGM * WGN;
-  static_assert(2 * BM == T && 2 * BN == T, "a thread loads eight values of each operand");
+// Bound by power, the matrix cores and the splitting: 4096^3 in 128 x 256 tiles 915 -> 623 us, 221 TFLOP/s; the matrix ops
+// alone, from registers on the same operands, sustain 302.  (128 x 128 tiles, two to a CU, split four values to six
+// matrix ops' worth instead of three: 669 us.  256 x 256 tiles, two values: 600, but there are registers for one
+// accumulator only; with a block's six terms summed from zero, smallest first, and then added to it 635, and one
+// product in a row still 3.5e-8.  A wavefront for each SIMD on 128 x 128, more slabs on their way, two K groups
+// of such tiles: all slower.)
+template <int BM, int BN>
+struct SharedLayout {
   // [piece][eight k][row or column] of 16 bytes; 64 bytes between the halves of k put a thread pair's writes on
   // different banks
-  constexpr int HALF = BM * 16 + 64, PIECE = 2 * HALF, OPERAND = 3 * PIECE, STAGE = 2 * OPERAND;
+  static constexpr int HALF_A = BM * 16 + 64, HALF_B = BN * 16 + 64, PIECE_A = 2 * HALF_A, PIECE_B = 2 * HALF_B,
+                       STAGE = 3 * (PIECE_A + PIECE_B);
+};
+
+template <int MI, int NI, int WGM, int WGN, bool TRANSB>
+__global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const SgemmParams p) {
+  constexpr int BM = 32 * MI * WGM, BN = 32 * NI * WGN, BK = 16, T = 64 * WGM * WGN;
+  constexpr int VA = BM * BK / T, VB = BN * BK / T, OPS_A = 6 * VA, OPS = OPS_A + 6 * VB;  // values per thread
+  static_assert((VA == 4 || VA == 8) && VB == 8, "a thread has four or eight values of A and eight of B");
+  using L = SharedLayout<BM, BN>;
+  constexpr int STAGE = L::STAGE;
 
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ Repairs repairs;
@@ -237,80 +260,84 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
   const unsigned m0 = tile.m0, n0 = tile.n0, M = p.M, N = p.N, K = p.K, lda = p.lda, ldb = p.ldb;
   const float *A = tile.A, *B = tile.B;
 
-  // ---- loads.  Rows of A (and of B given transposed): two threads to a row, eight k each.  B as stored: a thread to a
-  // column, eight rows.  Past the operands' ends lie zeros (the range check looks at the lane's offset, so the slab's k
+  // ---- loads.  Rows of A (and of B given transposed): two threads to a row, eight k each, or four, four k each.  B as
+  // stored: a thread to a column, eight rows.  Past the operands' ends lie zeros (the range check looks at the lane's offset, so the slab's k
   // is in the descriptor); past the end of a row of A lies the next one, which the last slab masks.
-  const int arow = tid >> 1, ahalf = tid & 1, brow = TRANSB ? tid >> 1 : tid & (BN - 1), bhalf = TRANSB ? tid & 1 : tid / BN;
-  const unsigned aOff = m0 + arow < M ? ((m0 + arow) * lda + 8 * ahalf) * 4u : kOutside;
+  const int arow = tid / (BK / VA), ak = tid % (BK / VA) * VA;
+  const int brow = TRANSB ? tid >> 1 : tid & (BN - 1), bhalf = TRANSB ? tid & 1 : tid / BN;
+  const unsigned aOff = m0 + arow < M ? ((m0 + arow) * lda + ak) * 4u : kOutside;
   const unsigned bOff = n0 + brow >= N ? kOutside : TRANSB ? ((n0 + brow) * ldb + 8 * bhalf) * 4u : (8 * bhalf * ldb + n0 + brow) * 4u;
   const unsigned slabs = (K + BK - 1) / BK;
-  struct Raw { float a[8], b[8]; };
+  struct Raw { float a[VA], b[VB]; };
   // the operand from its k `k0` on, `step` bytes to a k: 32-bit scalar arithmetic (a 64-bit comparison would be made on the
   // vector unit, and the descriptor then read back lane by lane)
   auto descriptor = [&](const float* base, unsigned k0, unsigned step, unsigned bytes) {
     const unsigned skip = k0 < K ? k0 * step : 0u;
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base) + skip / 4, 0, k0 < K ? (int)(bytes - skip) : 0, 0x00020000);
   };
-  // one of the ten loads of slab s (TRANSB: four): 0 and 1 are A's
+  // one of the loads of slab s, A's first
+  constexpr int LOADS_A = VA / 4, LOADS = LOADS_A + (TRANSB ? 2 : 8);
   auto load = [&](Raw& r, unsigned s, int which) __attribute__((always_inline)) {
     const unsigned k0 = s * BK;
-    auto quad = [&](float (&x)[8], __amdgpu_buffer_rsrc_t d, unsigned off, int h) {
-      const v4f v = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(d, off + 16 * h, 0, 0));
+    auto quad = [&](float* x, __amdgpu_buffer_rsrc_t d, unsigned off) __attribute__((always_inline)) {
+      const v4f v = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(d, off, 0, 0));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[4 * h + e] = v[e];
+      for (int e = 0; e < 4; ++e) x[e] = v[e];
     };
-    if (which < 2)
-      quad(r.a, descriptor(A, k0, 4u, tile.bytesA), aOff, which);
+    const int ofB = which - LOADS_A;
+    if (ofB < 0)
+      quad(r.a + 4 * which, descriptor(A, k0, 4u, tile.bytesA), aOff + 16 * which);
     else if (TRANSB)
-      quad(r.b, descriptor(B, k0, 4u, tile.bytesB), bOff, which - 2);
+      quad(r.b + 4 * ofB, descriptor(B, k0, 4u, tile.bytesB), bOff + 16 * ofB);
     else  // (a scalar offset is not range-checked)
-      r.b[which - 2] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(descriptor(B, k0, ldb * 4u, tile.bytesB),
-                                                                                      bOff + (which - 2) * ldb * 4u, 0, 0));
+      r.b[ofB] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(descriptor(B, k0, ldb * 4u, tile.bytesB),
+                                                                               bOff + ofB * ldb * 4u, 0, 0));
   };
-  constexpr int LOADS = TRANSB ? 4 : 10;
   auto mask = [&](Raw& r, unsigned s) {  // the slab in which K ends, or one behind it
     const int left = (int)K - (int)(s * BK);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      r.a[e] = 8 * ahalf + e < left ? r.a[e] : 0.f;
-      r.b[e] = 8 * bhalf + e < left ? r.b[e] : 0.f;
-    }
+    for (int e = 0; e < VA; ++e) r.a[e] = ak + e < left ? r.a[e] : 0.f;
+#pragma unroll
+    for (int e = 0; e < VB; ++e) r.b[e] = 8 * bhalf + e < left ? r.b[e] : 0.f;
   };
   float largest = 0.f;
-  unsigned char* const aTo = smem + ahalf * HALF + arow * 16;
-  unsigned char* const bTo = smem + OPERAND + bhalf * HALF + brow * 16;
+  unsigned char* const aTo = smem + ak / 8 * L::HALF_A + arow * 16 + ak % 8 * 2;
+  unsigned char* const bTo = smem + 3 * L::PIECE_A + bhalf * L::HALF_B + brow * 16;
 
-  v16f main[MI][NI], rest[TWO ? MI : 1][TWO ? NI : 1];
+  v16f main[MI][NI], rest[MI][NI];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < NI; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        main[i][j][r] = 0.f;
-        if constexpr (TWO) rest[i][j][r] = 0.f;
-      }
+    for (int j = 0; j < NI; ++j) main[i][j] = rest[i][j] = v16f{};
 
-  const unsigned char* const aFrom = smem + g * HALF + (wm * 32 * MI + lrow) * 16;
-  const unsigned char* const bFrom = smem + OPERAND + g * HALF + (wn * 32 * NI + lrow) * 16;
+  const unsigned char* const aFrom = smem + g * L::HALF_A + (wm * 32 * MI + lrow) * 16;
+  const unsigned char* const bFrom = smem + 3 * L::PIECE_A + g * L::HALF_B + (wn * 32 * NI + lrow) * 16;
   Raw raw;
-  Splitting sp;
+  Splitting<VA> ofA;
+  Splitting<VB> ofB;
   v4u a[3][MI], b[3][NI];
-  // the instructions that split a thread's values: A's, then B's
-  auto splitOp = [&](Raw& r, auto op) __attribute__((always_inline)) {
-    if constexpr (op < kSplitOps) split_op<op>(r.a, sp, largest);
-    else split_op<op - kSplitOps>(r.b, sp, largest);
-  };
-  // each piece is written when it is there, a while before the next: three writes in a row hold the wavefront up
-  // (326 -> 298 us for 192 slabs of 256 x 256)
-  auto put = [&](unsigned char* to, unsigned stage, int i) __attribute__((always_inline)) {
-    *reinterpret_cast<v4u*>(to + stage + i * PIECE) = sp.piece[i];
+  // The instructions that split a thread's values, A's, then B's.  Each piece is written when it is there, a while before
+  // the next: three writes in a row hold the wavefront up (by a tenth, in 256 x 256 tiles).
+  auto splitOp = [&](Raw& r, unsigned stage, auto op) __attribute__((always_inline)) {
+    if constexpr (op < OPS_A) {
+      split_op<VA, op>(r.a, ofA, largest);
+      constexpr int w = written<VA>(op);
+      if constexpr (w >= 0 && VA == 8)
+        *reinterpret_cast<v4u*>(aTo + stage + w * L::PIECE_A) = v4u{ofA.piece[w][0], ofA.piece[w][1], ofA.piece[w][VA / 2 - 2], ofA.piece[w][VA / 2 - 1]};
+      else if constexpr (w >= 0)
+        *reinterpret_cast<v2u*>(aTo + stage + w * L::PIECE_A) = v2u{ofA.piece[w][0], ofA.piece[w][1]};
+    } else {
+      split_op<VB, op - OPS_A>(r.b, ofB, largest);
+      constexpr int w = written<VB>(op - OPS_A);
+      if constexpr (w >= 0)
+        *reinterpret_cast<v4u*>(bTo + stage + w * L::PIECE_B) = v4u{ofB.piece[w][0], ofB.piece[w][1], ofB.piece[w][2], ofB.piece[w][3]};
+    }
   };
   auto readA = [&](int i, int j, unsigned stage) __attribute__((always_inline)) {
-    a[i][j] = *reinterpret_cast<const v4u*>(aFrom + stage + i * PIECE + j * 512);
+    a[i][j] = *reinterpret_cast<const v4u*>(aFrom + stage + i * L::PIECE_A + j * 512);
   };
   auto readB = [&](int i, int j, unsigned stage) __attribute__((always_inline)) {
-    b[i][j] = *reinterpret_cast<const v4u*>(bFrom + stage + i * PIECE + j * 512);
+    b[i][j] = *reinterpret_cast<const v4u*>(bFrom + stage + i * L::PIECE_B + j * 512);
   };
 
   // ---- slabs 0 and 1 in LDS, slab 2 on its way, the first operands in registers
@@ -330,10 +357,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     if ((unsigned)(s + 1) * BK > K) mask(ahead[s], s);
-    each<0, 2 * kSplitOps>([&](auto o) __attribute__((always_inline)) {
-      splitOp(ahead[s], o);
-      if constexpr (written(o % kSplitOps) >= 0) put(o < kSplitOps ? aTo : bTo, s * STAGE, written(o % kSplitOps));
-    });
+    each<0, OPS>([&](auto o) __attribute__((always_inline)) { splitOp(ahead[s], s * STAGE, o); });
   }
   __syncthreads();
 #pragma unroll
@@ -357,23 +381,20 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
     if ((s + 3) * BK > K) mask(raw, s + 2);
     each<0, TOTAL>([&](auto mc) __attribute__((always_inline)) {
       constexpr int m = mc, t = m / PT, i = m % PT / NI, j = m % NI;
-      if constexpr (TWO && t != 2)
-        rest[TWO ? i : 0][TWO ? j : 0] = product(a[kTermA[t]][i], b[kTermB[t]][j], rest[TWO ? i : 0][TWO ? j : 0]);
-      else
-        main[i][j] = product(a[kTermA[t]][i], b[kTermB[t]][j], main[i][j]);
+      v16f& sum = t == 2 ? main[i][j] : rest[i][j];
+      sum = product(a[kTermA[t]][i], b[kTermB[t]][j], sum);
       if (m == 0) __syncthreads();
       if (m >= 1 && m <= MI) readA(0, m - 1, st0);
       if (m > MI && m <= MI + NI) readB(2, m - MI - 1, st0);
-      constexpr int from = m < SPREAD ? m * 2 * kSplitOps / SPREAD : 2 * kSplitOps, to = m < SPREAD ? (m + 1) * 2 * kSplitOps / SPREAD : from;
+      constexpr int from = m < SPREAD ? m * OPS / SPREAD : OPS, to = m < SPREAD ? (m + 1) * OPS / SPREAD : from;
       each<from, to>([&](auto o) __attribute__((always_inline)) {
-        splitOp(raw, o);
-        if constexpr (written(o % kSplitOps) >= 0) put(o < kSplitOps ? aTo : bTo, st2, written(o % kSplitOps));
-        if constexpr (o == kSplitOps + 3) load(raw, s + 3, 0);
-        if constexpr (o == kSplitOps + 7) load(raw, s + 3, 1);
+        splitOp(raw, st2, o);
+        if constexpr (o == OPS_A + 3) load(raw, s + 3, 0);
+        if constexpr (o == OPS_A + 7 && LOADS_A == 2) load(raw, s + 3, 1);
       });
-      if (m >= SPREAD && m - SPREAD < (LOADS - 2 + 1) / 2) {
-        load(raw, s + 3, 2 + 2 * (m - SPREAD));
-        load(raw, s + 3, 3 + 2 * (m - SPREAD));
+      if (m >= SPREAD && m - SPREAD < (LOADS - LOADS_A) / 2) {
+        load(raw, s + 3, LOADS_A + 2 * (m - SPREAD));
+        load(raw, s + 3, LOADS_A + 1 + 2 * (m - SPREAD));
       }
       if (m >= 2 * PT && m < 2 * PT + MI) readA(2, m - 2 * PT, st1);
       if (m >= 3 * PT && m < 3 * PT + NI) readB(0, m - 3 * PT, st1);
@@ -386,14 +407,12 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
     st1 = st2;
     st2 = done;
   }
-  if constexpr (TWO) {
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < NI; ++j)
+    for (int j = 0; j < NI; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) main[i][j][r] += rest[i][j][r];
-  }
+      for (int r = 0; r < 16; ++r) main[i][j][r] += rest[i][j][r];
 
   // ---- what the split may have got wrong
   const unsigned rowBase = m0 + wm * MI * 32, colBase = n0 + wn * NI * 32;
@@ -508,7 +527,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
 // KG wavefronts own 64 x 64 outputs; wavefront q sums the slabs of 32 k q, q + KG, ... for all of them.  Copies go straight to
 // a ring in LDS that belongs to the wavefront, so there is no barrier until the partial tiles meet; a wavefront splits what it
 // multiplies by itself, twice the splitting of a 128 x 128 tile shared by four, and the vector unit bounds the loop: eight of
-// its instructions to a matrix op, 1250 cycles for the 768 that a step's matrix ops take.  (Operands fetched straight to
+// its instructions to a matrix op, 1250 cycles for the 768 that a step's matrix ops take.  The second accumulator costs it
+// nothing, 31.8 us for 1024 x 1024 x 2048 with and without.  (Operands fetched straight to
 // registers: the address unit is the bound, 38 us against 33.5 for 1024 x 3072 x 768.)
 template <int KG, bool TRANSB>
 __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmParams p) {
@@ -591,28 +611,27 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
       }
   };
 
-  v16f acc[2][2];
+  v16f acc[2][2], rest[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    for (int j = 0; j < 2; ++j) acc[i][j] = rest[i][j] = v16f{};
   float largest = 0.f;
   // Two sets of operands: the matrix ops of a step run on one while the next step's values are split into the other, and
   // the values of the step after that are read as their registers fall free.
   Raw raw;
-  Splitting a[2][2], b[2][2];
+  Splitting<8> a[2][2], b[2][2];
+  constexpr int OPS = 48;  // of one of them
   auto splitOp = [&](int set, auto op) __attribute__((always_inline)) {
-    constexpr int o = op % kSplitOps, which = op / kSplitOps;
-    if constexpr (which < 2) split_op<o>(raw.a[which], a[set][which], largest);
-    else split_op<o>(raw.b[which - 2], b[set][which - 2], largest);
+    constexpr int o = op % OPS, which = op / OPS;
+    if constexpr (which < 2) split_op<8, o>(raw.a[which], a[set][which], largest);
+    else split_op<8, o>(raw.b[which - 2], b[set][which - 2], largest);
   };
   wait_vmcnt<COPIES*(STAGES - 1)>();
 #pragma unroll
   for (int w = 0; w < READS; ++w) read(raw, 0, w);
   if (firstK(0) + BK > K) mask(raw, 0);
-  each<0, 4 * kSplitOps>([&](auto o) __attribute__((always_inline)) { splitOp(0, o); });
+  each<0, 4 * OPS>([&](auto o) __attribute__((always_inline)) { splitOp(0, o); });
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the reads of slab 0 have returned
 #pragma unroll
   for (int u = 0; u < COPIES; ++u) copy(2, 0, u);
@@ -625,7 +644,8 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
     if (firstK(s + 1) + BK > K) mask(raw, s + 1);
     each<0, 24>([&](auto m) __attribute__((always_inline)) {
       constexpr int t = m / 4, i = m / 2 % 2, j = m % 2;
-      acc[i][j] = product(a[cur][i].piece[kTermA[t]], b[cur][j].piece[kTermB[t]], acc[i][j]);
+      v16f& sum = t == 2 ? acc[i][j] : rest[i][j];
+      sum = product(operand(a[cur][i].piece[kTermA[t]]), operand(b[cur][j].piece[kTermB[t]]), sum);
       each<8 * m, 8 * m + 8>([&](auto o) __attribute__((always_inline)) { splitOp(nxt, o); });
       if constexpr (m == 4) __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the reads of slab s + 1 have returned
       if constexpr (m >= 4 && m <= 7) {
@@ -648,6 +668,12 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
   }
   wait_vmcnt<0>();
   __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] += rest[i][j][r];
 
   // ---- the partial tiles meet: registers 4 c .. 4 c + 3 of block (i, j) as one quad, in the order of i, c, j; wavefront w
   // finishes the quads from w QPW on, rows of two neighbouring columns
@@ -772,13 +798,13 @@ int launch(hipStream_t stream, SgemmParams& p, Kernel kern, bool (&attrSet)[16],
   return check_launch("sgemm");
 }
 
-template <int MI, int NI, int WGM, int WGN, bool TWO, bool TRANSB>
+template <int MI, int NI, int WGM, int WGN, bool TRANSB>
 int launch_shared(hipStream_t stream, SgemmParams p) {
   constexpr int BM = 32 * MI * WGM, BN = 32 * NI * WGN;
-  constexpr size_t lds = (size_t)3 * (2 * 3 * 2 * (BM * 16 + 64));
+  constexpr size_t lds = 3 * SharedLayout<BM, BN>::STAGE;
   static_assert(lds <= 159 * 1024, "LDS budget");
   static bool attrSet[16] = {};
-  return launch(stream, p, sgemm_split_kernel<MI, NI, WGM, WGN, TWO, TRANSB>, attrSet, BM, BN, 64 * WGM * WGN, lds);
+  return launch(stream, p, sgemm_split_kernel<MI, NI, WGM, WGN, TRANSB>, attrSet, BM, BN, 64 * WGM * WGN, lds);
 }
 
 template <int KG, bool TRANSB>
@@ -791,10 +817,10 @@ int launch64(hipStream_t stream, SgemmParams p) {
 
 namespace sgemm_detail {
 
-int sgemm_split_launch(hipStream_t stream, const SgemmParams& p, int config, bool transB) {
-  switch (config) {
-    case 0: return transB ? launch_shared<4, 2, 2, 4, false, true>(stream, p) : launch_shared<4, 2, 2, 4, false, false>(stream, p);
-    case 1: return transB ? launch_shared<2, 2, 2, 2, true, true>(stream, p) : launch_shared<2, 2, 2, 2, true, false>(stream, p);
+int sgemm_split_launch(hipStream_t stream, const SgemmParams& p, int kernel, bool transB) {
+  switch (kernel) {
+    case sgemm_split_plan::kWide: return transB ? launch_shared<2, 2, 2, 4, true>(stream, p) : launch_shared<2, 2, 2, 4, false>(stream, p);
+    case sgemm_split_plan::k128: return transB ? launch_shared<2, 2, 2, 2, true>(stream, p) : launch_shared<2, 2, 2, 2, false>(stream, p);
     default: return transB ? launch64<4, true>(stream, p) : launch64<4, false>(stream, p);
   }
 }
