@@ -21,10 +21,17 @@
 // What the split cannot represent is found and done again.  Infinities, NaN and values that round up to infinity make the
 // results they enter NaN or infinite; operands below 2^-109 leave bits of x2 outside bf16's range, which matters next to a very
 // large partner or in a very small result; products below 2^-126 round where the fp32 op would not.  So every thread keeps the
-// largest magnitude it split (one instruction for two values), and looks at its results: one that is not finite has the
-// workgroup compute its tile again with the fp32 matrix ops; a few below 2^-64, which happens by chance (a sum that cancels to
-// zero, in one product of ten), are summed again one by one; if there are many (a row of zeros), or a magnitude was 2^30 or
-// more, the tile's operands are read once more for their smallest, and that decides.
+// largest magnitude it split of A and of B (one instruction for two values), and looks at its results: one that is not
+// finite has the tile formed with the fp32 matrix ops; those below 2^-64 are right if their row or column holds nothing but zeros,
+// which the magnitudes tell; a few others, which happens by chance (a sum that cancels to zero, in one product of ten), are
+// summed again one by one; if there are many (sparse operands on both sides), or a magnitude was 2^30 or more, the tile's
+// operands are read once more for their smallest, row by row and column by column, and that decides.
+//
+// What that costs, us, in order: normal operands; one row of zeros; the last quarter of the rows; one value in a hundred in
+// both operands; one value of 2^31; one NaN; and normal operands on the fp32 ops:
+//   4096^3, 128 x 256 tiles        640   640   612   595   689   4497   915
+//   2048^3, 128 x 128               99   110    99   129   131     569   125
+//   1024 x 1024 x 2048, 64 x 64     31    32    31    46    48     107    35
 //
 // Two kernels.  What they have in common is that vector instructions run under bf16 matrix ops: up to six of them between
 // two of 32 cycles cost next to nothing, if they stand there; a wavefront that issues matrix ops back to back keeps the
@@ -53,6 +60,9 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 // a byte offset that fails the range check of any operand here (below 2^31 bytes, the dispatcher sees to it), also with a
 // tile's rows of one added
 constexpr unsigned kOutside = 0x80000000u;
+
+// magnitudes, as their bits: infinity, 2^30, 2^-64, 2^-90
+constexpr unsigned kInfinite = 0x7f800000u, kLarge = 0x4e800000u, kSmall = 0x1f800000u, kVerySmall = 0x12800000u;
 
 // f(FROM), f(FROM + 1), ..., f(TO - 1) with the index a constant
 template <int FROM, int TO, class F>
@@ -139,83 +149,168 @@ __device__ __forceinline__ Tile tile_of(const SgemmParams& p) {
   return t;
 }
 
-// The smallest magnitude in `rows` rows of `n` floats, as twice its bits less one: zero counts as the largest.
-__device__ __forceinline__ unsigned smallest_of(const float* x, unsigned rows, unsigned n, unsigned ld) {
-  const __amdgpu_buffer_rsrc_t d =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), 0, (int)(((rows - 1) * ld + n) * 4u), 0x00020000);
-  const unsigned pieces = (n + 3) / 4, total = rows * pieces;
-  unsigned least = 0xffffffffu;
-  for (unsigned i = threadIdx.x; i < total; i += 8 * blockDim.x) {
-    v4u v[8];  // whole numbers from the start: a bit_cast of a vector's element reads its first one
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const unsigned at = i + u * blockDim.x, r = at / pieces;
-      v[u] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(d, at < total ? (r * ld + 4 * (at - r * pieces)) * 4u : kOutside, 0, 0));
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const unsigned at = i + u * blockDim.x, k = 4 * (at - at / pieces * pieces);
-#pragma unroll
-      for (unsigned e = 0; e < 4; ++e)
-        if (k + e < n) least = min(least, (v[u][e] << 1) - 1u);
-    }
-  }
-  return least;
+// The smallest of the sixteen lanes' values, in all of them.
+__device__ __forceinline__ unsigned least_of_sixteen(unsigned x) {
+  x = min(x, (unsigned)__builtin_amdgcn_mov_dpp((int)x, 0xb1, 0xf, 0xf, true));   // quad_perm 1, 0, 3, 2
+  x = min(x, (unsigned)__builtin_amdgcn_mov_dpp((int)x, 0x4e, 0xf, 0xf, true));   // quad_perm 2, 3, 0, 1
+  x = min(x, (unsigned)__builtin_amdgcn_mov_dpp((int)x, 0x141, 0xf, 0xf, true));  // row_half_mirror
+  return min(x, (unsigned)__builtin_amdgcn_mov_dpp((int)x, 0x140, 0xf, 0xf, true));  // row_mirror
 }
 
-// Results that are summed again one by one.
+// The smallest magnitude other than zero in every one of `rows` (at most ROWS) rows of `n` floats, by T threads, or of all of
+// them in every one of `n` (at most COLS) columns, as twice its bits less one: zero counts as the largest.  (Loaded as whole
+// numbers: a bit_cast of a vector's element reads its first one.)
+template <int ROWS, int T>
+__device__ __forceinline__ void least_of_rows(const float* x, unsigned rows, unsigned n, unsigned ld, unsigned* least) {
+  constexpr int EACH = ROWS * 16 / T, CHUNKS = 8 / EACH;  // sixteen lanes to a row
+  const __amdgpu_buffer_rsrc_t d =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), 0, (int)(((rows - 1) * ld + n) * 4u), 0x00020000);
+  const unsigned lane = threadIdx.x & 15, row = threadIdx.x >> 4;
+  unsigned smallest[EACH];
+#pragma unroll
+  for (int u = 0; u < EACH; ++u) smallest[u] = ~0u;
+  for (unsigned first = 4 * lane; first < n; first += 64 * CHUNKS) {
+    v4u v[EACH][CHUNKS];
+#pragma unroll
+    for (int u = 0; u < EACH; ++u)
+#pragma unroll
+      for (int k = 0; k < CHUNKS; ++k) {
+        const unsigned r = row + u * (T / 16), c = first + 64 * k;
+        v[u][k] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(d, c < n && r < rows ? (r * ld + c) * 4u : kOutside, 0, 0));
+      }
+#pragma unroll
+    for (int u = 0; u < EACH; ++u)
+#pragma unroll
+      for (int k = 0; k < CHUNKS; ++k)
+#pragma unroll
+        for (unsigned e = 0; e < 4; ++e) smallest[u] = min(smallest[u], first + 64 * k + e < n ? (v[u][k][e] << 1) - 1u : ~0u);
+  }
+#pragma unroll
+  for (int u = 0; u < EACH; ++u) {
+    const unsigned value = least_of_sixteen(smallest[u]);
+    if (lane == 0) least[row + u * (T / 16)] = value;
+  }
+}
+template <int COLS, int T>
+__device__ __forceinline__ void least_of_columns(const float* x, unsigned rows, unsigned n, unsigned ld, unsigned* least) {
+  const __amdgpu_buffer_rsrc_t d =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), 0, (int)(((rows - 1) * ld + n) * 4u), 0x00020000);
+  constexpr int STEP = T / (COLS / 4);  // rows at a time
+  const unsigned c = 4 * (threadIdx.x % (COLS / 4));
+  v4u smallest = {~0u, ~0u, ~0u, ~0u};
+  for (unsigned r = threadIdx.x / (COLS / 4); r < rows; r += 8 * STEP) {
+    v4u v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      v[u] = __builtin_bit_cast(
+          v4u, __builtin_amdgcn_raw_buffer_load_b128(d, c < n && r + u * STEP < rows ? ((r + u * STEP) * ld + c) * 4u : kOutside, 0, 0));
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) smallest[e] = min(smallest[e], (v[u][e] << 1) - 1u);
+  }
+#pragma unroll
+  for (unsigned e = 0; e < 4; ++e)
+    if (c + e < n) __hip_atomic_fetch_min(least + c + e, smallest[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// What a workgroup finds out about its tile when a result or an operand looks as if the split may have got something wrong.
 constexpr unsigned kMostRepairs = 32;
+template <int BM, int BN>
 struct Repairs {
-  unsigned count, at[kMostRepairs];  // row of the tile * 256 + column
-  unsigned least[2];                 // the smallest operands of A and of B
+  unsigned count, at[kMostRepairs];  // results that are summed again one by one: row of the tile * 256 + column
+  unsigned largest[BM + BN];         // the largest magnitude of every row of A, then of every column of B, as its bits
+  unsigned least[BM + BN];           // the smallest but zero, as twice its bits less one, if they were asked for
   float value[kMostRepairs], part[8];
 };
 
-// Whether the workgroup has to compute its tile with the fp32 matrix ops.  Every thread's `largest` operand, whether its
-// results are all finite, and the smallest magnitude among those inside the matrix; list(): adds its results below 2^-64 to
-// `repairs`.  If they are few, their values are there afterwards, for repair_results.
-template <int BM, int BN, bool TRANSB, class List>
-__device__ __forceinline__ bool split_failed(const SgemmParams& p, const Tile& t, float largest, bool finite, float smallestResult,
-                                             Repairs& repairs, List&& list) {
+// Whether there are results in the tile that have to be formed again with the fp32 matrix ops, and which of the thread's:
+// a bit of `again` for each of its BLOCKS x 16.  value(block, i): one of them; where(block, i, row, column): its place in the
+// tile.  `suspicious`: one of them is not finite or below 2^-64, or the thread has split a value of 2^30 or more.  raise(): puts
+// the magnitudes that the thread has split into `largest`.
+// A result that is not finite has to be formed again, and the tile with it.  One of a row or a column of zeros is right (which goes for those outside the
+// matrix, too).  Others below 2^-64 are summed one by one if they are few, and their values are there afterwards, for
+// repair_results.  If they are many, or there is a magnitude of 2^30 or more, the operands are read once more: those results,
+// and the ones that a large value enters, have to be formed again if their own row or column has a value that is too small for
+// them.
+template <int BM, int BN, int T, bool TRANSB, int BLOCKS, class Value, class Where, class Raise>
+__device__ __forceinline__ bool split_failed(const SgemmParams& p, const Tile& t, bool suspicious, Repairs<BM, BN>& repairs,
+                                             unsigned (&again)[BLOCKS], Value&& value, Where&& where, Raise&& raise) {
   if (threadIdx.x == 0) repairs.count = 0;
-  if (threadIdx.x < 2) repairs.least[threadIdx.x] = 0xffffffffu;
-  if (!__syncthreads_or(!finite || largest >= 0x1p30f || smallestResult < 0x1p-64f)) return false;
-  if (__syncthreads_or(!finite)) return true;
-  const bool large = __syncthreads_or(largest >= 0x1p30f) != 0;
-  if (smallestResult < 0x1p-64f) list();
+  if (!__syncthreads_or(suspicious)) return false;
+  for (unsigned i = threadIdx.x; i < BM + BN; i += T) {
+    repairs.largest[i] = 0;
+    repairs.least[i] = ~0u;
+  }
   __syncthreads();
-  if (large || repairs.count > kMostRepairs) {
+  raise();
+  __syncthreads();
+  bool large = false;
+  for (unsigned i = threadIdx.x; i < BM + BN; i += T) large = large || repairs.largest[i] >= kLarge;
+  unsigned any = 0;
+  // (without branches: 64 results are looked at in 1 us)
+  each<0, BLOCKS>([&](auto b) __attribute__((always_inline)) {
+    unsigned wrong = 0, small = 0;
+    each<0, 16>([&](auto i) __attribute__((always_inline)) {
+      unsigned row, col;
+      where(b, i, row, col);
+      const unsigned size = __builtin_bit_cast(unsigned, value(b, i)) & 0x7fffffffu;
+      wrong |= (unsigned)(size >= kInfinite) << i;
+      small |= (unsigned)((size < kSmall) & (repairs.largest[row] != 0) & (repairs.largest[BM + col] != 0)) << i;
+    });
+    again[b] = wrong;
+    any |= wrong;
+    for (; small != 0; small &= small - 1) {
+      unsigned row, col;
+      where(b, __builtin_ctz(small), row, col);
+      const unsigned at = atomicAdd(&repairs.count, 1u);
+      if (at < kMostRepairs) repairs.at[at] = row << 8 | col;
+    }
+  });
+  large = __syncthreads_or(large) != 0;
+  const bool many = large || repairs.count > kMostRepairs;
+  __syncthreads();
+  if (many) {
     const unsigned rows = min((unsigned)BM, p.M - t.m0), cols = min((unsigned)BN, p.N - t.n0);
-    const unsigned la = smallest_of(t.A + (size_t)t.m0 * p.lda, rows, p.K, p.lda);
-    const unsigned lb = TRANSB ? smallest_of(t.B + (size_t)t.n0 * p.ldb, cols, p.K, p.ldb) : smallest_of(t.B + t.n0, p.K, cols, p.ldb);
-    __hip_atomic_fetch_min(&repairs.least[0], la, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __hip_atomic_fetch_min(&repairs.least[1], lb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __syncthreads();
+    least_of_rows<BM, T>(t.A + (size_t)t.m0 * p.lda, rows, p.K, p.lda, repairs.least);
+    if constexpr (TRANSB) least_of_rows<BN, T>(t.B + (size_t)t.n0 * p.ldb, cols, p.K, p.ldb, repairs.least + BM);
+    else least_of_columns<BN, T>(t.B + t.n0, p.K, cols, p.ldb, repairs.least + BM);
     if (threadIdx.x == 0) repairs.count = 0;
-    const int ea = (int)(repairs.least[0] >> 24) - 127, eb = (int)(repairs.least[1] >> 24) - 127;  // their exponents
-    return __syncthreads_or(ea < -100 || eb < -100 || (ea + eb < -100 && smallestResult < 0x1p-90f)) != 0;
+    __syncthreads();
+    each<0, BLOCKS>([&](auto b) __attribute__((always_inline)) {
+      each<0, 16>([&](auto i) __attribute__((always_inline)) {
+        unsigned row, col;
+        where(b, i, row, col);
+        const unsigned size = __builtin_bit_cast(unsigned, value(b, i)) & 0x7fffffffu;
+        const bool candidate = (size < kSmall) | (repairs.largest[row] >= kLarge) | (repairs.largest[BM + col] >= kLarge);
+        const int x = (int)(repairs.least[row] >> 24) - 127, y = (int)(repairs.least[BM + col] >> 24) - 127;  // exponents
+        again[b] |= (unsigned)(candidate & ((x < -100) | (y < -100) | ((x + y < -100) & (size < kVerySmall)))) << i;
+      });
+      any |= again[b];
+    });
   }
   for (unsigned i = 0; i < repairs.count; ++i) {
     const unsigned row = t.m0 + (repairs.at[i] >> 8), col = t.n0 + (repairs.at[i] & 255u);
     float sum = 0.f;
-    for (unsigned k = threadIdx.x; k < p.K; k += blockDim.x)
+    for (unsigned k = threadIdx.x; k < p.K; k += T)
       sum = fmaf(t.A[(size_t)row * p.lda + k], TRANSB ? t.B[(size_t)col * p.ldb + k] : t.B[(size_t)k * p.ldb + col], sum);
     for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d);
     if ((threadIdx.x & 63) == 0) repairs.part[threadIdx.x >> 6] = sum;
     __syncthreads();
     if (threadIdx.x == 0) {
-      for (unsigned w = 1; w < blockDim.x >> 6; ++w) sum += repairs.part[w];
+      for (unsigned w = 1; w < T >> 6; ++w) sum += repairs.part[w];
       if (t.bias) sum += t.bias[col];
       if (t.R) sum += t.R[(size_t)row * p.N + col];
       repairs.value[i] = p.act == 1 ? gelu_erf_f32(sum) : sum;
     }
     __syncthreads();
   }
-  return false;
+  return __syncthreads_or(any != 0) != 0;
 }
 
 // Behind the tile store: the whole workgroup.
-__device__ __forceinline__ void repair_results(const SgemmParams& p, const Tile& t, const Repairs& repairs) {
+template <int BM, int BN>
+__device__ __forceinline__ void repair_results(const SgemmParams& p, const Tile& t, const Repairs<BM, BN>& repairs) {
   if (repairs.count == 0) return;
   __threadfence_block();
   __syncthreads();  // the stores of the tile have been made
@@ -251,7 +346,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
   constexpr int STAGE = L::STAGE;
 
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ Repairs repairs;
+  __shared__ Repairs<BM, BN> repairs;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int wm = wv / WGN, wn = wv - wm * WGN;  // wave-uniform
   const int tid = threadIdx.x, lane = tid & 63, lrow = lane & 31, g = lane >> 5;
@@ -300,7 +395,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
 #pragma unroll
     for (int e = 0; e < VB; ++e) r.b[e] = 8 * bhalf + e < left ? r.b[e] : 0.f;
   };
-  float largest = 0.f;
+  float largestA = 0.f, largestB = 0.f;
   unsigned char* const aTo = smem + ak / 8 * L::HALF_A + arow * 16 + ak % 8 * 2;
   unsigned char* const bTo = smem + 3 * L::PIECE_A + bhalf * L::HALF_B + brow * 16;
 
@@ -320,14 +415,14 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
   // the next: three writes in a row hold the wavefront up (by a tenth, in 256 x 256 tiles).
   auto splitOp = [&](Raw& r, unsigned stage, auto op) __attribute__((always_inline)) {
     if constexpr (op < OPS_A) {
-      split_op<VA, op>(r.a, ofA, largest);
+      split_op<VA, op>(r.a, ofA, largestA);
       constexpr int w = written<VA>(op);
       if constexpr (w >= 0 && VA == 8)
         *reinterpret_cast<v4u*>(aTo + stage + w * L::PIECE_A) = v4u{ofA.piece[w][0], ofA.piece[w][1], ofA.piece[w][VA / 2 - 2], ofA.piece[w][VA / 2 - 1]};
       else if constexpr (w >= 0)
         *reinterpret_cast<v2u*>(aTo + stage + w * L::PIECE_A) = v2u{ofA.piece[w][0], ofA.piece[w][1]};
     } else {
-      split_op<VB, op - OPS_A>(r.b, ofB, largest);
+      split_op<VB, op - OPS_A>(r.b, ofB, largestB);
       constexpr int w = written<VB>(op - OPS_A);
       if constexpr (w >= 0)
         *reinterpret_cast<v4u*>(bTo + stage + w * L::PIECE_B) = v4u{ofB.piece[w][0], ofB.piece[w][1], ofB.piece[w][2], ofB.piece[w][3]};
@@ -437,50 +532,41 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
           if (rowBase + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3) < M && colBase + 32 * j + lrow < N)
             low = fminf(low, __builtin_fabsf(main[i][j][r]));
   }
-  auto list = [&]() {
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int j = 0; j < NI; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const unsigned row = rowBase + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3), col = colBase + 32 * j + lrow;
-          if (__builtin_fabsf(main[i][j][r]) < 0x1p-64f && row < M && col < N) {
-            const unsigned at = atomicAdd(&repairs.count, 1u);
-            if (at < kMostRepairs) repairs.at[at] = (row - m0) << 8 | (col - n0);
-          }
-        }
+  auto raise = [&]() {
+    __hip_atomic_fetch_max(&repairs.largest[arow], __builtin_bit_cast(unsigned, largestA), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_max(&repairs.largest[BM + brow], __builtin_bit_cast(unsigned, largestB), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
-  if (split_failed<BM, BN, TRANSB>(p, tile, largest, notFinite == 0.f, low, repairs, list)) {
+  auto value = [&](auto block, auto r) __attribute__((always_inline)) -> float {
+    const float v = main[block / NI][block % NI][(int)r];  // (a copy: a bit_cast of a vector's element reads its first one)
+    return v;
+  };
+  auto where = [&](int block, int r, unsigned& row, unsigned& col) __attribute__((always_inline)) {
+    row = wm * MI * 32 + 32 * (block / NI) + 8 * (r >> 2) + 4 * g + (r & 3);
+    col = wn * NI * 32 + 32 * (block % NI) + lrow;
+  };
+  unsigned again[PT];
+  const bool suspicious = notFinite != 0.f || low < 0x1p-64f || largestA >= 0x1p30f || largestB >= 0x1p30f;
+  if (split_failed<BM, BN, T, TRANSB, PT>(p, tile, suspicious, repairs, again, value, where, raise)) {
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < NI; ++j)
+      for (int j = 0; j < NI; ++j) {
+        const unsigned arow = rowBase + 32 * i + lrow, bcol = colBase + 32 * j + lrow;
+        v16f sum = {};
+        for (unsigned k = 0; k < K; k += 32) {
+          float x[16], y[16];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) main[i][j][r] = 0.f;
-    for (unsigned k = 0; k < K; k += 8) {
-      float x[4][MI], y[4][NI];
+          for (int e = 0; e < 16; ++e) {
+            const unsigned kk = k + 2 * e + g;
+            x[e] = kk < K && arow < M ? A[(size_t)arow * lda + kk] : 0.f;
+            y[e] = kk < K && bcol < N ? TRANSB ? B[(size_t)bcol * ldb + kk] : B[(size_t)kk * ldb + bcol] : 0.f;
+          }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const unsigned kk = k + 2 * e + g;
-#pragma unroll
-        for (int i = 0; i < MI; ++i) {
-          const unsigned row = rowBase + 32 * i + lrow;
-          x[e][i] = kk < K && row < M ? A[(size_t)row * lda + kk] : 0.f;
+          for (int e = 0; e < 16; ++e) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], sum, 0, 0, 0);
         }
 #pragma unroll
-        for (int j = 0; j < NI; ++j) {
-          const unsigned col = colBase + 32 * j + lrow;
-          y[e][j] = kk < K && col < N ? TRANSB ? B[(size_t)col * ldb + kk] : B[(size_t)kk * ldb + col] : 0.f;
-        }
+        for (int r = 0; r < 16; ++r) main[i][j][r] = sum[r];
       }
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int j = 0; j < NI; ++j) main[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e][i], y[e][j], main[i][j], 0, 0, 0);
-    }
   }
 
   // ---- tile store: + bias, + residual, GELU; rows past M and columns past N fail the range check
@@ -535,7 +621,7 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
   constexpr int BM = 64, BN = 64, BK = 16, STAGES = 2;
   constexpr int A_BYTES = BM * BK * 4, B_BYTES = BK * BN * 4, STAGE = A_BYTES + B_BYTES, COPIES = STAGE / 1024;
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ Repairs repairs;
+  __shared__ Repairs<BM, BN> repairs;
   const int grp = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63, lrow = lane & 31, g = lane >> 5;
   unsigned char* gsm = smem + grp * STAGES * STAGE;
@@ -616,7 +702,7 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = rest[i][j] = v16f{};
-  float largest = 0.f;
+  float largest[4] = {};  // of the two rows and of the two columns
   // Two sets of operands: the matrix ops of a step run on one while the next step's values are split into the other, and
   // the values of the step after that are read as their registers fall free.
   Raw raw;
@@ -624,8 +710,8 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
   constexpr int OPS = 48;  // of one of them
   auto splitOp = [&](int set, auto op) __attribute__((always_inline)) {
     constexpr int o = op % OPS, which = op / OPS;
-    if constexpr (which < 2) split_op<8, o>(raw.a[which], a[set][which], largest);
-    else split_op<8, o>(raw.b[which - 2], b[set][which - 2], largest);
+    if constexpr (which < 2) split_op<8, o>(raw.a[which], a[set][which], largest[which]);
+    else split_op<8, o>(raw.b[which - 2], b[set][which - 2], largest[which]);
   };
   wait_vmcnt<COPIES*(STAGES - 1)>();
 #pragma unroll
@@ -679,8 +765,7 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
   // finishes the quads from w QPW on, rows of two neighbouring columns
   constexpr int QPW = 16 / KG;
   v4f* meetings = reinterpret_cast<v4f*>(smem);
-  v4f sum[QPW];
-  auto meet = [&]() __attribute__((always_inline)) {
+  auto meet = [&](v4f (&sum)[QPW]) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
       const int i = q >> 3, c = (q >> 1) & 3, j = q & 1;
@@ -698,7 +783,8 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
       }
     }
   };
-  meet();
+  v4f sum[QPW];
+  meet(sum);
   const unsigned ldc = p.ldc, col = n0 + 2 * lrow;
   auto rowOf = [&](int x, int e) {  // of quads 2 x and 2 x + 1
     const int q = grp * QPW + 2 * x;
@@ -714,25 +800,28 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
         notFinite = fmaf(sum[2 * x + j][e], 0.f, notFinite);
         low = rowOf(x, e) < M && col + j < N ? fminf(low, __builtin_fabsf(sum[2 * x + j][e])) : low;
       }
-  auto list = [&]() {
-#pragma unroll
-    for (int x = 0; x < QPW / 2; ++x)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          if (__builtin_fabsf(sum[2 * x + j][e]) < 0x1p-64f && rowOf(x, e) < M && col + j < N) {
-            const unsigned at = atomicAdd(&repairs.count, 1u);
-            if (at < kMostRepairs) repairs.at[at] = (rowOf(x, e) - m0) << 8 | (col + j - n0);
-          }
+  constexpr int MINE = QPW / 4;  // the thread's results, in sixteens
+  auto value = [&](auto block, auto r) __attribute__((always_inline)) -> float {
+    const float v = sum[4 * block + r / 4][(int)(r % 4)];  // (a copy: a bit_cast of a vector's element reads its first one)
+    return v;
   };
-  if (split_failed<BM, BN, TRANSB>(p, tile, largest, notFinite == 0.f, low, repairs, list)) {
+  auto where = [&](int block, int r, unsigned& row, unsigned& column) __attribute__((always_inline)) {
+    row = rowOf((4 * block + r / 4) / 2, r % 4) - m0;
+    column = 2 * lrow + (r / 4) % 2;
+  };
+  unsigned again[MINE];
+  auto raise = [&]() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __hip_atomic_fetch_max(&repairs.largest[i < 2 ? 32 * i + lrow : BM + 2 * lrow + i - 2], __builtin_bit_cast(unsigned, largest[i]),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  const bool suspicious = notFinite != 0.f || low < 0x1p-64f || fmaxf(fmaxf(largest[0], largest[1]), fmaxf(largest[2], largest[3])) >= 0x1p30f;
+  if (split_failed<BM, BN, 64 * KG, TRANSB, MINE>(p, tile, suspicious, repairs, again, value, where, raise)) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+      for (int j = 0; j < 2; ++j) acc[i][j] = v16f{};
     for (unsigned s = 0; s < steps; ++s) {
       float x[8][2], y[8][2];
 #pragma unroll
@@ -753,7 +842,12 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
           for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e][i], y[e][j], acc[i][j], 0, 0, 0);
     }
     __syncthreads();
-    meet();
+    v4f exact[QPW];
+    meet(exact);
+#pragma unroll
+    for (int q = 0; q < QPW; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[q][e] = exact[q][e];
   }
 
   // ---- tile store: + bias, + residual, GELU
