@@ -226,3 +226,27 @@ def test_zeros_cost_nothing(pkg, dev, kernel, m, n, k):
             best[i] = min(best[i], start.elapsed_time(end))
     print(kernel, best, best[1] / best[0])
     assert best[1] <= 1.2 * best[0]
+
+
+@pytest.mark.parametrize("kernel,m,n,k", ONE_OF_EACH)
+def test_other_rows_and_columns_do_not_matter(pkg, dev, kernel, m, n, k):
+    """A row's results have the same bits whatever its neighbours hold: infinities, NaN, large, tiny and zero ones."""
+    import torch
+    assert kernel_of(m, n, k) == kernel
+    gen = torch.Generator(device=dev).manual_seed(k)
+    a, b = torch.randn(m, k, device=dev, generator=gen), torch.randn(k, n, device=dev, generator=gen)
+    plain = pkg.blas_matmul(a, b)
+    x, y = a.clone(), b.clone()
+    x[5, 3], x[40, k - 1], x[77] = float("inf"), float("nan"), 0.0
+    x[300], x[333, 7] = a[300] * 2.0 ** -125, 2.0 ** 100
+    y[9, 70], y[:, 200] = -float("inf"), b[:, 200] * 2.0 ** 40
+    rows = [i for i in range(m) if i not in (5, 40, 77, 300, 333)]
+    cols = [j for j in range(n) if j not in (70, 200)]
+    out = pkg.blas_matmul(x, y)
+    assert torch.equal(out[rows][:, cols], plain[rows][:, cols])
+    assert torch.equal(torch.isnan(out), torch.isnan(x.double() @ y.double())) and not bool(out[77][cols].any())
+    c = torch.empty(m, n, device=dev)
+    pkg.sgemm_general(x, y.t().contiguous(), c, m, n, k, k, k, n, trans_b=True)
+    assert torch.equal(c[rows][:, cols], plain[rows][:, cols])
+    want = x[300].double() @ y[:, cols].double()
+    assert rel(out[300][cols], want) <= bound_fp32(k)

@@ -21,17 +21,17 @@
 // What the split cannot represent is found and done again.  Infinities, NaN and values that round up to infinity make the
 // results they enter NaN or infinite; operands below 2^-109 leave bits of x2 outside bf16's range, which matters next to a very
 // large partner or in a very small result; products below 2^-126 round where the fp32 op would not.  So every thread keeps the
-// largest magnitude it split of A and of B (one instruction for two values), and looks at its results: one that is not
-// finite has the tile formed with the fp32 matrix ops; those below 2^-64 are right if their row or column holds nothing but zeros,
+// largest magnitude it split of A and of B (one instruction for two values), and looks at its results: those that are not
+// finite are formed with the fp32 matrix ops; those below 2^-64 are right if their row or column holds nothing but zeros,
 // which the magnitudes tell; a few others, which happens by chance (a sum that cancels to zero, in one product of ten), are
 // summed again one by one; if there are many (sparse operands on both sides), or a magnitude was 2^30 or more, the tile's
 // operands are read once more for their smallest, row by row and column by column, and that decides.
 //
 // What that costs, us, in order: normal operands; one row of zeros; the last quarter of the rows; one value in a hundred in
 // both operands; one value of 2^31; one NaN; and normal operands on the fp32 ops:
-//   4096^3, 128 x 256 tiles        640   640   612   595   689   4497   915
-//   2048^3, 128 x 128               99   110    99   129   131     569   125
-//   1024 x 1024 x 2048, 64 x 64     31    32    31    46    48     107    35
+//   4096^3, 128 x 256 tiles        640   640   612   595   689   1486   915
+//   2048^3, 128 x 128               99   110    99   129   131     304   125
+//   1024 x 1024 x 2048, 64 x 64     31    32    31    46    48     110    35
 //
 // Two kernels.  What they have in common is that vector instructions run under bf16 matrix ops: up to six of them between
 // two of 32 cycles cost next to nothing, if they stand there; a wavefront that issues matrix ops back to back keeps the
@@ -228,11 +228,11 @@ struct Repairs {
 // a bit of `again` for each of its BLOCKS x 16.  value(block, i): one of them; where(block, i, row, column): its place in the
 // tile.  `suspicious`: one of them is not finite or below 2^-64, or the thread has split a value of 2^30 or more.  raise(): puts
 // the magnitudes that the thread has split into `largest`.
-// A result that is not finite has to be formed again, and the tile with it.  One of a row or a column of zeros is right (which goes for those outside the
+// A result that is not finite is formed again.  One of a row or a column of zeros is right (which goes for those outside the
 // matrix, too).  Others below 2^-64 are summed one by one if they are few, and their values are there afterwards, for
 // repair_results.  If they are many, or there is a magnitude of 2^30 or more, the operands are read once more: those results,
-// and the ones that a large value enters, have to be formed again if their own row or column has a value that is too small for
-// them.
+// and the ones that a large value enters, are formed again if their own row or column has a value that is too small for
+// them.  Whether a result is formed again therefore does not depend on what other rows and columns hold.
 template <int BM, int BN, int T, bool TRANSB, int BLOCKS, class Value, class Where, class Raise>
 __device__ __forceinline__ bool split_failed(const SgemmParams& p, const Tile& t, bool suspicious, Repairs<BM, BN>& repairs,
                                              unsigned (&again)[BLOCKS], Value&& value, Where&& where, Raise&& raise) {
@@ -551,6 +551,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
     for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int j = 0; j < NI; ++j) {
+        if (!__any(again[i * NI + j] != 0)) continue;
         const unsigned arow = rowBase + 32 * i + lrow, bcol = colBase + 32 * j + lrow;
         v16f sum = {};
         for (unsigned k = 0; k < K; k += 32) {
@@ -565,7 +566,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
           for (int e = 0; e < 16; ++e) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], sum, 0, 0, 0);
         }
 #pragma unroll
-        for (int r = 0; r < 16; ++r) main[i][j][r] = sum[r];
+        for (int r = 0; r < 16; ++r) main[i][j][r] = again[i * NI + j] >> r & 1 ? sum[r] : main[i][j][r];
       }
   }
 
@@ -847,7 +848,7 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
 #pragma unroll
     for (int q = 0; q < QPW; ++q)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) sum[q][e] = exact[q][e];
+      for (int e = 0; e < 4; ++e) sum[q][e] = again[q / 4] >> (4 * (q % 4) + e) & 1 ? exact[q][e] : sum[q][e];
   }
 
   // ---- tile store: + bias, + residual, GELU
