@@ -250,3 +250,24 @@ def test_other_rows_and_columns_do_not_matter(pkg, dev, kernel, m, n, k):
     assert torch.equal(c[rows][:, cols], plain[rows][:, cols])
     want = x[300].double() @ y[:, cols].double()
     assert rel(out[300][cols], want) <= bound_fp32(k)
+
+
+@pytest.mark.parametrize("n", [961, 962, 963])
+@pytest.mark.parametrize("row", [70, 1019])
+def test_tiny_results_in_the_last_columns_stay_in_their_row(pkg, dev, n, row):
+    """One tiny row and one to three columns in the last 64 x 64 tiles: few results to look at again, next to the columns that a
+    load of four has beyond N.  The next row, the columns behind N of a wider result, and what lies behind the last row stay."""
+    import torch
+    m, k = 1020, 2050
+    assert kernel_of(m, n, k) == K64
+    gen = torch.Generator(device=dev).manual_seed(n + row)
+    a, b = torch.randn(m, k, device=dev, generator=gen), torch.randn(k, n, device=dev, generator=gen)
+    plain = pkg.blas_matmul(a, b)
+    a[row] *= 2.0 ** -80
+    rest = [i for i in range(m) if i != row]
+    for ldc in (n, n + 5):
+        c = torch.full((m * ldc + 8,), 7.0, device=dev)
+        pkg.sgemm_general(a, b, c, m, n, k, k, n, ldc)
+        out = c[:m * ldc].view(m, ldc)
+        assert torch.equal(out[rest, :n], plain[rest]) and bool((c[m * ldc:] == 7).all()) and bool((out[:, n:] == 7).all())
+        assert rel(out[row, :n], a[row].double() @ b.double()) <= bound_fp32(k)

@@ -228,8 +228,8 @@ struct Repairs {
 // a bit of `again` for each of its BLOCKS x 16.  value(block, i): one of them; where(block, i, row, column): its place in the
 // tile.  `suspicious`: one of them is not finite or below 2^-64, or the thread has split a value of 2^30 or more.  raise(): puts
 // the magnitudes that the thread has split into `largest`.
-// A result that is not finite is formed again.  One of a row or a column of zeros is right (which goes for those outside the
-// matrix, too).  Others below 2^-64 are summed one by one if they are few, and their values are there afterwards, for
+// A result that is not finite is formed again.  One of a row or a column of zeros is right, and raise() leaves those outside the
+// matrix at zero, so that they are never listed: a listed one is stored.  Others below 2^-64 are summed one by one if they are few, and their values are there afterwards, for
 // repair_results.  If they are many, or there is a magnitude of 2^30 or more, the operands are read once more: those results,
 // and the ones that a large value enters, are formed again if their own row or column has a value that is too small for
 // them.  Whether a result is formed again therefore does not depend on what other rows and columns hold.
@@ -813,9 +813,10 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
   unsigned again[MINE];
   auto raise = [&]() {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      __hip_atomic_fetch_max(&repairs.largest[i < 2 ? 32 * i + lrow : BM + 2 * lrow + i - 2], __builtin_bit_cast(unsigned, largest[i]),
-                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    for (int i = 0; i < 4; ++i)  // (a load of four columns that N cuts holds values of the next row: no columns of the matrix)
+      if (i < 2 || col + i - 2 < N)
+        __hip_atomic_fetch_max(&repairs.largest[i < 2 ? 32 * i + lrow : BM + 2 * lrow + i - 2], __builtin_bit_cast(unsigned, largest[i]),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
   const bool suspicious = notFinite != 0.f || low < 0x1p-64f || fmaxf(fmaxf(largest[0], largest[1]), fmaxf(largest[2], largest[3])) >= 0x1p30f;
   if (split_failed<BM, BN, 64 * KG, TRANSB, MINE>(p, tile, suspicious, repairs, again, value, where, raise)) {
