@@ -160,7 +160,7 @@ def test_values_the_split_cannot_represent(pkg, dev, m, n, k):
 
 
 def test_results_that_cancel(pkg, dev):
-    """A few results that are zero among large ones are summed again, with their bias and activation."""
+    """A few results that are zero among large ones, which the kernel looks at again."""
     import torch
     m, n, k = 2048, 2048, 256
     gen = torch.Generator(device=dev).manual_seed(3)
@@ -271,3 +271,23 @@ def test_tiny_results_in_the_last_columns_stay_in_their_row(pkg, dev, n, row):
         out = c[:m * ldc].view(m, ldc)
         assert torch.equal(out[rest, :n], plain[rest]) and bool((c[m * ldc:] == 7).all()) and bool((out[:, n:] == 7).all())
         assert rel(out[row, :n], a[row].double() @ b.double()) <= bound_fp32(k)
+
+
+@pytest.mark.parametrize("kernel,m,n,k", [(WIDE, 3969, 3841, 600), (K128, 2047, 1921, 1009), (K64, 1020, 962, 2050)])
+def test_tiny_results_have_the_bits_of_large_ones(pkg, dev, kernel, m, n, k):
+    """Rows scaled by 2^-75, one of them or many together, in tiles that are full and in the last ones, of one or two columns: the
+    results are those of the rows as they were, scaled, however many of a tile's are small."""
+    import torch
+    assert kernel_of(m, n, k) == kernel
+    gen = torch.Generator(device=dev).manual_seed(m)
+    a, b = torch.randn(m, k, device=dev, generator=gen), torch.randn(k, n, device=dev, generator=gen)
+    bt = b.t().contiguous()
+    plain = pkg.blas_matmul(a, b)
+    for rows in ([70], list(range(64, 128))):
+        x, want = a.clone(), plain.clone()
+        x[rows] *= 2.0 ** -75
+        want[rows] *= 2.0 ** -75
+        assert torch.equal(pkg.blas_matmul(x, b), want)
+        c = torch.empty(m, n, device=dev)
+        pkg.sgemm_general(x, bt, c, m, n, k, k, k, n, trans_b=True)
+        assert torch.equal(c, want)

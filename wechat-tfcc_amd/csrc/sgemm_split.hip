@@ -23,9 +23,9 @@
 // large partner or in a very small result; products below 2^-126 round where the fp32 op would not.  So every thread keeps the
 // largest magnitude it split of A and of B (one instruction for two values), and looks at its results: those that are not
 // finite are formed with the fp32 matrix ops; those below 2^-64 are right if their row or column holds nothing but zeros,
-// which the magnitudes tell; a few others, which happens by chance (a sum that cancels to zero, in one product of ten), are
-// summed again one by one; if there are many (sparse operands on both sides), or a magnitude was 2^30 or more, the tile's
-// operands are read once more for their smallest, row by row and column by column, and that decides.
+// which the magnitudes tell; about the others the smallest operands of their rows and columns decide, for which those of a few
+// results, which happens by chance (a sum that cancels to zero, in one product of ten), are read once more, and all of the
+// tile's if there are many (sparse operands on both sides) or a magnitude was 2^30 or more.
 //
 // What that costs, us, in order: normal operands; one row of zeros; the last quarter of the rows; one value in a hundred in
 // both operands; one value of 2^31; one NaN; and normal operands on the fp32 ops:
@@ -215,13 +215,12 @@ __device__ __forceinline__ void least_of_columns(const float* x, unsigned rows, 
 }
 
 // What a workgroup finds out about its tile when a result or an operand looks as if the split may have got something wrong.
-constexpr unsigned kMostRepairs = 32;
+constexpr unsigned kMostListed = 32;
 template <int BM, int BN>
-struct Repairs {
-  unsigned count, at[kMostRepairs];  // results that are summed again one by one: row of the tile * 256 + column
-  unsigned largest[BM + BN];         // the largest magnitude of every row of A, then of every column of B, as its bits
-  unsigned least[BM + BN];           // the smallest but zero, as twice its bits less one, if they were asked for
-  float value[kMostRepairs], part[8];
+struct Findings {
+  unsigned count, at[kMostListed];  // results below 2^-64: row of the tile * 256 + column
+  unsigned largest[BM + BN];        // the largest magnitude of every row of A, then of every column of B, as its bits
+  unsigned least[BM + BN];          // the smallest but zero, as twice its bits less one, of those that were asked for
 };
 
 // Whether there are results in the tile that have to be formed again with the fp32 matrix ops, and which of the thread's:
@@ -229,24 +228,24 @@ struct Repairs {
 // tile.  `suspicious`: one of them is not finite or below 2^-64, or the thread has split a value of 2^30 or more.  raise(): puts
 // the magnitudes that the thread has split into `largest`.
 // A result that is not finite is formed again.  One of a row or a column of zeros is right, and raise() leaves those outside the
-// matrix at zero, so that they are never listed: a listed one is stored.  Others below 2^-64 are summed one by one if they are few, and their values are there afterwards, for
-// repair_results.  If they are many, or there is a magnitude of 2^30 or more, the operands are read once more: those results,
-// and the ones that a large value enters, are formed again if their own row or column has a value that is too small for
-// them.  Whether a result is formed again therefore does not depend on what other rows and columns hold.
+// matrix at zero, so that they are never listed: a listed one's row and column are read.  Others below 2^-64, and those that a
+// value of 2^30 or more enters, are formed again if their own row or column has a value that is too small for them.  For a few
+// such results their rows and columns are searched for it, for many, or next to a large value, all of the tile's.  Whether
+// a result is formed again therefore depends on its own row and column alone.
 template <int BM, int BN, int T, bool TRANSB, int BLOCKS, class Value, class Where, class Raise>
-__device__ __forceinline__ bool split_failed(const SgemmParams& p, const Tile& t, bool suspicious, Repairs<BM, BN>& repairs,
+__device__ __forceinline__ bool split_failed(const SgemmParams& p, const Tile& t, bool suspicious, Findings<BM, BN>& found,
                                              unsigned (&again)[BLOCKS], Value&& value, Where&& where, Raise&& raise) {
-  if (threadIdx.x == 0) repairs.count = 0;
   if (!__syncthreads_or(suspicious)) return false;
+  if (threadIdx.x == 0) found.count = 0;
   for (unsigned i = threadIdx.x; i < BM + BN; i += T) {
-    repairs.largest[i] = 0;
-    repairs.least[i] = ~0u;
+    found.largest[i] = 0;
+    found.least[i] = ~0u;
   }
   __syncthreads();
   raise();
   __syncthreads();
   bool large = false;
-  for (unsigned i = threadIdx.x; i < BM + BN; i += T) large = large || repairs.largest[i] >= kLarge;
+  for (unsigned i = threadIdx.x; i < BM + BN; i += T) large = large || found.largest[i] >= kLarge;
   unsigned any = 0;
   // (without branches: 64 results are looked at in 1 us)
   each<0, BLOCKS>([&](auto b) __attribute__((always_inline)) {
@@ -256,66 +255,55 @@ __device__ __forceinline__ bool split_failed(const SgemmParams& p, const Tile& t
       where(b, i, row, col);
       const unsigned size = __builtin_bit_cast(unsigned, value(b, i)) & 0x7fffffffu;
       wrong |= (unsigned)(size >= kInfinite) << i;
-      small |= (unsigned)((size < kSmall) & (repairs.largest[row] != 0) & (repairs.largest[BM + col] != 0)) << i;
+      small |= (unsigned)((size < kSmall) & (found.largest[row] != 0) & (found.largest[BM + col] != 0)) << i;
     });
     again[b] = wrong;
     any |= wrong;
     for (; small != 0; small &= small - 1) {
       unsigned row, col;
       where(b, __builtin_ctz(small), row, col);
-      const unsigned at = atomicAdd(&repairs.count, 1u);
-      if (at < kMostRepairs) repairs.at[at] = row << 8 | col;
+      const unsigned at = atomicAdd(&found.count, 1u);
+      if (at < kMostListed) found.at[at] = row << 8 | col;
     }
   });
   large = __syncthreads_or(large) != 0;
-  const bool many = large || repairs.count > kMostRepairs;
-  __syncthreads();
-  if (many) {
+  if (large || found.count > kMostListed) {
     const unsigned rows = min((unsigned)BM, p.M - t.m0), cols = min((unsigned)BN, p.N - t.n0);
-    least_of_rows<BM, T>(t.A + (size_t)t.m0 * p.lda, rows, p.K, p.lda, repairs.least);
-    if constexpr (TRANSB) least_of_rows<BN, T>(t.B + (size_t)t.n0 * p.ldb, cols, p.K, p.ldb, repairs.least + BM);
-    else least_of_columns<BN, T>(t.B + t.n0, p.K, cols, p.ldb, repairs.least + BM);
-    if (threadIdx.x == 0) repairs.count = 0;
-    __syncthreads();
-    each<0, BLOCKS>([&](auto b) __attribute__((always_inline)) {
-      each<0, 16>([&](auto i) __attribute__((always_inline)) {
-        unsigned row, col;
-        where(b, i, row, col);
-        const unsigned size = __builtin_bit_cast(unsigned, value(b, i)) & 0x7fffffffu;
-        const bool candidate = (size < kSmall) | (repairs.largest[row] >= kLarge) | (repairs.largest[BM + col] >= kLarge);
-        const int x = (int)(repairs.least[row] >> 24) - 127, y = (int)(repairs.least[BM + col] >> 24) - 127;  // exponents
-        again[b] |= (unsigned)(candidate & ((x < -100) | (y < -100) | ((x + y < -100) & (size < kVerySmall)))) << i;
-      });
-      any |= again[b];
-    });
-  }
-  for (unsigned i = 0; i < repairs.count; ++i) {
-    const unsigned row = t.m0 + (repairs.at[i] >> 8), col = t.n0 + (repairs.at[i] & 255u);
-    float sum = 0.f;
-    for (unsigned k = threadIdx.x; k < p.K; k += T)
-      sum = fmaf(t.A[(size_t)row * p.lda + k], TRANSB ? t.B[(size_t)col * p.ldb + k] : t.B[(size_t)k * p.ldb + col], sum);
-    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d);
-    if ((threadIdx.x & 63) == 0) repairs.part[threadIdx.x >> 6] = sum;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      for (unsigned w = 1; w < T >> 6; ++w) sum += repairs.part[w];
-      if (t.bias) sum += t.bias[col];
-      if (t.R) sum += t.R[(size_t)row * p.N + col];
-      repairs.value[i] = p.act == 1 ? gelu_erf_f32(sum) : sum;
+    least_of_rows<BM, T>(t.A + (size_t)t.m0 * p.lda, rows, p.K, p.lda, found.least);
+    if constexpr (TRANSB) least_of_rows<BN, T>(t.B + (size_t)t.n0 * p.ldb, cols, p.K, p.ldb, found.least + BM);
+    else least_of_columns<BN, T>(t.B + t.n0, p.K, cols, p.ldb, found.least + BM);
+  } else {
+    for (unsigned i = 0; i < found.count; ++i) {
+      const unsigned row = found.at[i] >> 8, col = found.at[i] & 255u;
+      unsigned x = ~0u, y = ~0u;
+      for (unsigned k = threadIdx.x; k < p.K; k += T) {
+        const float ofA = t.A[(size_t)(t.m0 + row) * p.lda + k];
+        const float ofB = TRANSB ? t.B[(size_t)(t.n0 + col) * p.ldb + k] : t.B[(size_t)k * p.ldb + t.n0 + col];
+        x = min(x, (__builtin_bit_cast(unsigned, ofA) << 1) - 1u);
+        y = min(y, (__builtin_bit_cast(unsigned, ofB) << 1) - 1u);
+      }
+      x = least_of_sixteen(x);
+      y = least_of_sixteen(y);
+      if ((threadIdx.x & 15) == 0) {
+        __hip_atomic_fetch_min(&found.least[row], x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_min(&found.least[BM + col], y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
     }
-    __syncthreads();
   }
+  if (!large && found.count == 0) return __syncthreads_or(any != 0) != 0;
+  __syncthreads();
+  each<0, BLOCKS>([&](auto b) __attribute__((always_inline)) {
+    each<0, 16>([&](auto i) __attribute__((always_inline)) {
+      unsigned row, col;
+      where(b, i, row, col);
+      const unsigned size = __builtin_bit_cast(unsigned, value(b, i)) & 0x7fffffffu;
+      const bool candidate = (size < kSmall) | (found.largest[row] >= kLarge) | (found.largest[BM + col] >= kLarge);
+      const int x = (int)(found.least[row] >> 24) - 127, y = (int)(found.least[BM + col] >> 24) - 127;  // exponents
+      again[b] |= (unsigned)(candidate & ((x < -100) | (y < -100) | ((x + y < -100) & (size < kVerySmall)))) << i;
+    });
+    any |= again[b];
+  });
   return __syncthreads_or(any != 0) != 0;
-}
-
-// Behind the tile store: the whole workgroup.
-template <int BM, int BN>
-__device__ __forceinline__ void repair_results(const SgemmParams& p, const Tile& t, const Repairs<BM, BN>& repairs) {
-  if (repairs.count == 0) return;
-  __threadfence_block();
-  __syncthreads();  // the stores of the tile have been made
-  if (threadIdx.x < repairs.count)
-    t.C[(size_t)(t.m0 + (repairs.at[threadIdx.x] >> 8)) * p.ldc + t.n0 + (repairs.at[threadIdx.x] & 255u)] = repairs.value[threadIdx.x];
 }
 
 // ---- large products ------------------------------------------------------------------------------------------------------
@@ -346,7 +334,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
   constexpr int STAGE = L::STAGE;
 
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ Repairs<BM, BN> repairs;
+  __shared__ Findings<BM, BN> found;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int wm = wv / WGN, wn = wv - wm * WGN;  // wave-uniform
   const int tid = threadIdx.x, lane = tid & 63, lrow = lane & 31, g = lane >> 5;
@@ -533,8 +521,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
             low = fminf(low, __builtin_fabsf(main[i][j][r]));
   }
   auto raise = [&]() {
-    __hip_atomic_fetch_max(&repairs.largest[arow], __builtin_bit_cast(unsigned, largestA), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __hip_atomic_fetch_max(&repairs.largest[BM + brow], __builtin_bit_cast(unsigned, largestB), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_max(&found.largest[arow], __builtin_bit_cast(unsigned, largestA), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_max(&found.largest[BM + brow], __builtin_bit_cast(unsigned, largestB), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
   auto value = [&](auto block, auto r) __attribute__((always_inline)) -> float {
     const float v = main[block / NI][block % NI][(int)r];  // (a copy: a bit_cast of a vector's element reads its first one)
@@ -546,7 +534,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
   };
   unsigned again[PT];
   const bool suspicious = notFinite != 0.f || low < 0x1p-64f || largestA >= 0x1p30f || largestB >= 0x1p30f;
-  if (split_failed<BM, BN, T, TRANSB, PT>(p, tile, suspicious, repairs, again, value, where, raise)) {
+  if (split_failed<BM, BN, T, TRANSB, PT>(p, tile, suspicious, found, again, value, where, raise)) {
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -607,7 +595,6 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
     if (p.act == 1) store_all(R != nullptr, true);
     else store_all(R != nullptr, false);
   }
-  repair_results(p, tile, repairs);
 }
 
 // ---- products of a few dozen to a few hundred tiles ------------------------------------------------------------------
@@ -622,7 +609,7 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
   constexpr int BM = 64, BN = 64, BK = 16, STAGES = 2;
   constexpr int A_BYTES = BM * BK * 4, B_BYTES = BK * BN * 4, STAGE = A_BYTES + B_BYTES, COPIES = STAGE / 1024;
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ Repairs<BM, BN> repairs;
+  __shared__ Findings<BM, BN> found;
   const int grp = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63, lrow = lane & 31, g = lane >> 5;
   unsigned char* gsm = smem + grp * STAGES * STAGE;
@@ -815,11 +802,11 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
 #pragma unroll
     for (int i = 0; i < 4; ++i)  // (a load of four columns that N cuts holds values of the next row: no columns of the matrix)
       if (i < 2 || col + i - 2 < N)
-        __hip_atomic_fetch_max(&repairs.largest[i < 2 ? 32 * i + lrow : BM + 2 * lrow + i - 2], __builtin_bit_cast(unsigned, largest[i]),
+        __hip_atomic_fetch_max(&found.largest[i < 2 ? 32 * i + lrow : BM + 2 * lrow + i - 2], __builtin_bit_cast(unsigned, largest[i]),
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
   const bool suspicious = notFinite != 0.f || low < 0x1p-64f || fmaxf(fmaxf(largest[0], largest[1]), fmaxf(largest[2], largest[3])) >= 0x1p30f;
-  if (split_failed<BM, BN, 64 * KG, TRANSB, MINE>(p, tile, suspicious, repairs, again, value, where, raise)) {
+  if (split_failed<BM, BN, 64 * KG, TRANSB, MINE>(p, tile, suspicious, found, again, value, where, raise)) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -877,7 +864,6 @@ __global__ __launch_bounds__(64 * KG, 2) void sgemm_split64_kernel(const SgemmPa
         for (int j = 0; j < 2; ++j)
           if (col + j < N) to[j] = v[j];
     }
-  repair_results(p, tile, repairs);
 }
 
 template <class Kernel>
