@@ -211,13 +211,14 @@ def test_sgemm_on_128x96_workgroups(pkg, T, m, n, k, batch):
 @pytest.mark.parametrize("m,n,k", [
     # the same hand-scheduled kernel with other numbers of 32-column blocks per wavefront: 32 x 64 tiles and four K
     # groups (the first BASELINE config; ragged), 32 x 32 tiles and four K groups (whole and ragged), 128 x 128 tiles
-    # for products of 512 tiles and more (whole; ragged rows and columns; a single 32-k slab)
+    # for products of 512 tiles and more: a single 32-k slab (the two before it take 128 x 128 tiles on the bf16 matrix
+    # cores, for B as stored and transposed)
     (128, 3072, 768), (100, 3000, 800), (512, 512, 512), (500, 500, 544), (2048, 4096, 256), (2050, 4100, 320),
     (4096, 2048, 32),
     # two K groups: two pairs of wavefronts on 64 x 64 tiles (whole; ragged, an odd number of 32-k slabs), two
     # wavefronts on 32 x 32 tiles
     (1024, 1024, 1024), (1000, 1000, 992), (400, 400, 256), (1111, 996, 320),
-    # 128 x 128 workgroups below 512 tiles, where they fill the CUs and 128 x 96 tiles do not
+    # on the bf16 matrix cores, for B as stored and transposed
     (2048, 2048, 512), (1920, 2040, 544),
     # 64 x 64 tiles with four K groups: four pairs of wavefronts
     (960, 1024, 2048), (1270, 636, 544),
@@ -243,6 +244,31 @@ def test_sgemm_wavefront_kernel_with_one_two_and_four_column_blocks(pkg, T, m, n
                                               tres.data_ptr(), 0, out.data_ptr(), 0, m, n, k, 1, 1))
     separate = T.n(pkg.gelu_accurate(pkg.add(pkg.blas_matmul(ta, tb, tbias), tres)))
     assert np.array_equal(T.n(out), separate)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,batch", [
+    # 128 x 128 workgroups of four hand-scheduled wavefronts below 512 tiles, where they fill the CUs and 128 x 96 tiles do not
+    (425, 6974, 628, 1), (68, 2432, 752, 12), (132, 2567, 689, 6),
+    # and from 512 tiles on, with many slabs and with few
+    (2412, 200, 515, 14), (399, 2847, 617, 6), (2860, 3798, 41, 1),
+])
+def test_sgemm_on_128x128_workgroups(pkg, T, m, n, k, batch):
+    """What the rule does not send to the bf16 matrix cores: the same bits as the register-staged kernel (reached through a
+    transposed B), float64 within the fp32 tolerance."""
+    import torch
+    from test_gpu_sgemm_split import NONE, kernel_of
+    print("sgemm 128x128 workgroups", m, n, k, batch, flush=True)
+    assert kernel_of(m, n, k, batch) == NONE
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, b = torch.randn(batch, m, k, device="cuda", generator=gen), torch.randn(batch, k, n, device="cuda", generator=gen)
+    plain = pkg.blas_matmul(a, b)
+    want = torch.stack([x.double() @ y.double() for x, y in zip(a, b)])
+    assert rel_fro(T.n(plain), T.n(want)) <= FP32_TOL
+    c = torch.empty(batch, m, n, device="cuda")
+    pkg.sgemm_general(a, b.transpose(1, 2).contiguous(), c, m, n, k, k, k, n, trans_b=True, batch_outer=batch,
+                      strides=(m * k, n * k, m * n))
+    assert torch.equal(c, plain)
 
 
 @pytest.mark.gpu

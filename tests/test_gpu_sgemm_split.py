@@ -291,3 +291,110 @@ def test_tiny_results_have_the_bits_of_large_ones(pkg, dev, kernel, m, n, k):
         c = torch.empty(m, n, device=dev)
         pkg.sgemm_general(x, bt, c, m, n, k, k, k, n, trans_b=True)
         assert torch.equal(c, want)
+
+
+# a batch of each: true batches, every entry with its own operands
+BATCHED = [(WIDE, 1021, 1030, 769, 6), (K128, 650, 770, 515, 12), (K64, 251, 510, 1565, 8)]
+
+
+@pytest.mark.parametrize("kernel,m,n,k,batch", BATCHED + [(kind, m, n, k, 1) for kind, m, n, k in ONE_OF_EACH])
+def test_fused_epilogues_have_the_bits_of_separate_steps(pkg, dev, kernel, m, n, k, batch):
+    import torch
+    assert kernel_of(m, n, k, batch) == kernel
+    gen = torch.Generator(device=dev).manual_seed(m)
+    a, b, r = (torch.randn(*s, device=dev, generator=gen) for s in ((batch, m, k), (batch, k, n), (batch, m, n)))
+    bias = torch.randn(n, device=dev, generator=gen)
+    plain = pkg.blas_matmul(a, b)
+    for act in (0, 1):
+        out = torch.empty(batch, m, n, device=dev)
+        pkg.check(pkg.lib().tfcc_rocm_sgemm_fused(None, a.data_ptr(), m * k, b.data_ptr(), k * n, bias.data_ptr(), r.data_ptr(),
+                                                  m * n, out.data_ptr(), m * n, m, n, k, batch, act))
+        want = plain + bias + r
+        assert torch.equal(out, pkg.gelu_accurate(want) if act else want)
+
+
+@pytest.mark.parametrize("kernel,m,n,k", ONE_OF_EACH)
+def test_products_that_share_a_have_the_bits_of_single_ones(pkg, dev, kernel, m, n, k):
+    import torch
+    assert kernel_of(m, n, k) == kernel
+    gen = torch.Generator(device=dev).manual_seed(n)
+    a = torch.randn(m, k, device=dev, generator=gen)
+    a[m - 1] *= 2.0 ** -120  # formed again with the fp32 matrix ops
+    for groups in (2, 4):
+        bs = [torch.randn(k * n + g, device=dev, generator=gen)[g:].view(k, n) for g in range(groups)]
+        biases = [torch.randn(n, device=dev, generator=gen) for _ in bs]
+        for got, b, bias in zip(pkg.sgemm_grouped(a, bs, biases), bs, biases):
+            assert torch.equal(got, pkg.blas_matmul(a, b, bias))
+
+
+@pytest.mark.parametrize("kernel,m,n,k,batch", BATCHED)
+def test_batches_of_padded_matrices_with_special_values_in_each(pkg, dev, kernel, m, n, k, batch):
+    """Two-level batches, rows with padding behind them, and in every entry other rows that have to be formed again (for which
+    the operands are read from where the entry's lie), with bias and GELU on top; B as stored and transposed."""
+    import torch
+    assert kernel_of(m, n, k, batch) == kernel
+    gen = torch.Generator(device=dev).manual_seed(k)
+    lda, ldb, ldt, ldc = k + 3, n + 1, k + 2, n + 5
+    a, b = torch.randn(batch, m, lda, device=dev, generator=gen), torch.randn(batch, k, ldb, device=dev, generator=gen)
+    bias = torch.randn(n, device=dev, generator=gen)
+    for i in range(batch):
+        a[i, 3 * i + 1, 7 * i] = float("inf")
+        a[i, 64 + i, :k] *= 2.0 ** -120
+        a[i, 140 + i, :k] = 0.0
+        a[i, 140 + i, 5 + i] = 2.0 ** -135
+        b[i, 5 + i, :n] = 2.0 ** 110
+        a[i, :140 + i, 5 + i] = 0.0
+        a[i, 141 + i:, 5 + i] = 0.0
+    bt = torch.zeros(batch, n, ldt, device=dev)
+    bt[:, :, :k] = b[:, :, :n].transpose(1, 2)
+    outer, inner = batch // 2, 2
+    x, y = a[:, :, :k], b[:, :, :n]
+    want = torch.stack([x[i].double() @ y[i].double() for i in range(batch)]) + bias.double()
+    outs = []
+    for tb, act in ((False, 0), (True, 0), (False, 1), (True, 1)):
+        c = torch.full((batch, m, ldc), 7.0, device=dev)
+        right, ld, size = (bt, ldt, n * ldt) if tb else (b, ldb, k * ldb)
+        pkg.sgemm_general(a, right, c, m, n, k, lda, ld, ldc, trans_b=tb, batch_outer=outer, batch_inner=inner,
+                          strides=(2 * m * lda, 2 * size, 2 * m * ldc), inner_strides=(m * lda, size, m * ldc), bias=bias, activation=act)
+        assert bool((c[:, :, n:] == 7).all())
+        outs.append(c[:, :, :n].contiguous())
+    assert torch.equal(outs[0].nan_to_num(), outs[1].nan_to_num()) and torch.equal(outs[2].nan_to_num(), outs[3].nan_to_num())
+    assert torch.equal(outs[2].nan_to_num(), pkg.gelu_accurate(outs[0]).nan_to_num())
+    finite = torch.isfinite(want)
+    assert torch.equal(torch.isfinite(outs[0]), finite)
+    for i in range(batch):
+        assert torch.equal(outs[0][i, 140 + i], (bias.double() + 2.0 ** -25).float())
+        rows = [j for j in range(m) if j != 3 * i + 1]
+        assert rel(outs[0][i, rows], want[i, rows]) <= bound_fp32(k)
+
+
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("kernel,m,n,k", [(WIDE, 3969, 3841, 600), (K128, 2047, 1921, 1009), (K64, 1020, 962, 2050)])
+def test_a_few_results_that_the_split_gets_wrong(pkg, dev, kernel, m, n, k, trans_b):
+    """Single results that are small next to a small operand, fewer than a tile lists, in full tiles and in the last ones: as the
+    fp32 matrix ops have them, bias and GELU on top, and nothing else is touched."""
+    import torch
+    assert kernel_of(m, n, k) == kernel
+    gen = torch.Generator(device=dev).manual_seed(m)
+    a, b = torch.randn(m, k, device=dev, generator=gen), torch.randn(k, n, device=dev, generator=gen)
+    a[:, 9] = 0.0
+    plain = product(pkg, a, b, trans_b)
+    row, cols = 70, [3, 40, 500, n - 1]
+    a[row] = 0.0
+    a[row, 9] = 1.2345678 * 2.0 ** -115  # the third part of it lies outside bf16's range
+    b[9] = 0.0
+    b[9, cols] = torch.tensor([1.0, -1.5, 3.0, 0.5], device=dev)
+    want = torch.zeros(n, dtype=torch.double, device=dev)
+    want[cols] = a[row, 9].double() * b[9, cols].double()
+    out = product(pkg, a, b, trans_b)
+    assert torch.equal(out[row].double(), want.float().double())
+    rest = [i for i in range(m) if i != row]
+    assert torch.equal(out[rest], plain[rest])
+
+
+def product(pkg, a, b, trans_b):
+    import torch
+    (m, k), n = a.shape, b.shape[1]
+    if not trans_b:
+        return pkg.blas_matmul(a, b)
+    return pkg.sgemm_general(a, b.t().contiguous(), torch.empty(m, n, device=a.device), m, n, k, k, k, n, trans_b=True)

@@ -506,10 +506,11 @@ int dispatch(hipStream_t s, const SgemmParams& p, bool vec, bool small, bool tb,
     return launch<2, 2, 1, 1, false>(s, p);
   }
   // Everything else runs on the kernels that copy K slabs straight into LDS, whatever its alignment (333 x 1003 x 517:
-  // 8.8 us against 64.7 for register-staged slabs fetched word by word, 2000 x 1501 x 3003: 138 against 350).
+  // 8.8 us against 64.7 for register-staged slabs fetched word by word).
   // 128x128 tiles once there are enough of them to fill the 256 CUs twice over: four hand-scheduled wavefronts of
-  // 32 x 128 on a shared ring, two workgroups per CU - 4096^3: 150 TFLOP/s against 141 for the same tiles scheduled by
-  // the compiler.
+  // 32 x 128 on a shared ring, two workgroups per CU.  (Measured on 4096^3, which the bf16 matrix cores have taken since:
+  // 150 TFLOP/s against 141 for the same tiles scheduled by the compiler.  Products of up to 128 k, and batches whose
+  // entries fill their tiles badly, still come here.)
   if (takes_128_tiles(m, n, fillBatch)) return sgemm_detail::sgemm_wave96_launch(s, p, 1, 4);
   int best, ksplit;
   unsigned long long bestTiles;
@@ -534,8 +535,8 @@ int dispatch(hipStream_t s, const SgemmParams& p, bool vec, bool small, bool tb,
   if (ksplit == 2 && kTiles[best].config == 3) return sgemm_detail::sgemm_wave96_launch(s, p, 2, 1, 1);
   // ... and without K groups the products whose 128 x 96 tiles fill at least 70 % of the CUs in each of their
   // rounds (or 128 x 128 tiles 85 %), K >= 512: four wavefronts of 32 x 96 (32 x 128) share each copy of B
-  // (1024 x 3072 x 768 with GELU: 39.3 against 42.4 us in 64 x 64 tiles, 1536^3: 69 against 80, 2048^3 in
-  // 128 x 128 tiles: 120 against 136; below those fills, or with a short K, the tiles of the table win).  The
+  // (1024 x 3072 x 768 with GELU: 39.3 against 42.4 us in 64 x 64 tiles, 1536^3: 69 against 80; in 128 x 128 tiles
+  // 2048^3, now on the bf16 matrix cores, 120 against 136; below those fills, or with a short K, the table's win).  The
   // sums are the same in every case: the K groups of the table, ascending k inside a group.
   if (ksplit == 1 && k >= 512) {
     const unsigned long long wide = (unsigned long long)((m + 127) / 128) * ((n + 95) / 96) * fillBatch;
