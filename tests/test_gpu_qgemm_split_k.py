@@ -1,12 +1,27 @@
 """Small quantized products whose K is shared by several workgroups per tile: the edges of the rule and of the tiles, K that
 ends inside a step, operands at odd addresses, batches; several calls in a row (the memory the workgroups meet in has to be
 zero again), on streams of their own and under capture, bit for bit against the oracle."""
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
 import oracle_lib as O
 
 pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def shared_by(m, k, n, batch=1):
+    """The workgroups that share a tile by the launcher's own rule (tests/cpp/qgemm_small_plan_tests.cpp)."""
+    host = os.path.join(ROOT, "wechat-tfcc_amd", "host")
+    exe = os.path.join(host, "build", "qgemm_small_plan_tests")
+    if not os.path.exists(exe):
+        subprocess.check_call(["make", "-C", host, "build/qgemm_small_plan_tests"])
+    return int(subprocess.check_output([exe] + [str(v) for v in (m, n, k, batch)]))
+
 
 # m, k, n, batch
 SHAPES = [(1, 1345, 1, 1), (3, 11304, 910, 1), (16, 1473, 65, 1), (17, 2049, 63, 1), (8, 12288, 512, 1), (92, 4184, 115, 1),
@@ -23,6 +38,7 @@ def _case(m, k, n, batch):
 
 @pytest.mark.parametrize("m,k,n,batch", SHAPES)
 def test_products_whose_k_is_shared(pkg, T, m, k, n, batch):
+    assert shared_by(m, k, n, batch) > 1
     a, b, rs, cs = _case(m, k, n, batch)
     ranges = (-100.0, 155.0, -117.0, 138.0)
     want = O.qgemm(a, b, *O.qmatmul_offsets(*ranges), rs, cs)
@@ -68,3 +84,14 @@ def test_dequantized_on_streams_and_under_capture(pkg, T, m, k, n):
     torch.cuda.synchronize()
     for f, acc in outs:
         assert np.array_equal(T.n(acc), want) and np.array_equal(T.n(f).view(np.uint32), want_f.view(np.uint32))
+
+
+@pytest.mark.parametrize("m,k,n,shared", [(133, 2187, 1144, 3), (105, 2452, 25, 7), (36, 2486, 467, 7), (526, 1832, 400, 1),
+                                          (1869, 1824, 32, 1), (250, 1624, 200, 1), (48, 1920, 4992, 1)])
+def test_both_sides_of_the_line(pkg, T, m, k, n, shared):
+    assert shared_by(m, k, n) == shared
+    a, b, rs, cs = _case(m, k, n, 1)
+    ranges = (-100.0, 155.0, -117.0, 138.0)
+    r = [T.f1(v) for v in ranges]
+    got, _, _ = pkg.quantization_matmul(T.t(a), T.t(rs), r[0], r[1], T.t(b), T.t(cs), r[2], r[3])
+    assert np.array_equal(T.n(got), O.qgemm(a, b, *O.qmatmul_offsets(*ranges), rs, cs))

@@ -136,3 +136,13 @@ def test_which_fp32_products_run_on_the_bf16_matrix_cores():
         subprocess.check_call(["make", "-C", os.path.join(ROOT, "wechat-tfcc_amd", "host"), "build/sgemm_split_plan_tests"])
     res = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
     assert res.returncode == 0 and "all passed" in res.stdout, res.stdout[-2000:]
+
+
+def test_which_small_quantized_products_are_shared():
+    """The limits of the rule (tests/cpp/qgemm_small_plan_tests.cpp): both sides of its line as measured, and that the memory the
+    workgroups meet in is large enough for whatever they share."""
+    exe = os.path.join(ROOT, "wechat-tfcc_amd", "host", "build", "qgemm_small_plan_tests")
+    if not os.path.exists(exe):
+        subprocess.check_call(["make", "-C", os.path.join(ROOT, "wechat-tfcc_amd", "host"), "build/qgemm_small_plan_tests"])
+    res = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert res.returncode == 0 and "all passed" in res.stdout, res.stdout[-2000:]

@@ -18,6 +18,7 @@
 #include "gemv.hpp"
 #include "qgemm_params.hpp"
 #include "qgemm_small.hpp"
+#include "qgemm_small_plan.hpp"
 #include "stream_slots.hpp"
 
 namespace tfcc_rocm {
@@ -26,12 +27,14 @@ typedef qgemm_v4i v4i;
 
 namespace {
 
-constexpr int kCols = 64;    // columns of a tile
+using qgemm_small_plan::kCols;
+using qgemm_small_plan::kMaxResults;
+using qgemm_small_plan::Plan;
+using qgemm_small_plan::plan_of;
 constexpr int kPitch = 68;   // words per tile row in LDS: the four row groups of a store fall on different banks
 
 // The memory in which the workgroups that share a tile's K meet: a piece per stream, asked for by the first product that
 // is split.  A word per result, the sum in its high half, how many have added to it in the low one; zero between launches.
-constexpr unsigned kMaxResults = 1u << 19;
 int clear_words(hipStream_t stream, void* piece) { return tfcc_rocm_fill_async(stream, piece, 0, 8, kMaxResults); }
 StreamPieces gPieces(kMaxResults * 8, 64, clear_words);  // 4 MB each
 
@@ -296,54 +299,6 @@ int launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o, unsigned s
   return check_launch("quantized matmul (small)");
 }
 
-// Rows per tile and wavefronts by the amount of work, in steps of 16 rows x 64 columns x 64 k (measured, us):
-//   up to 4096 steps, or at most 16 rows, tiles of 16 rows: there latency is all there is, and the most workgroups share
-//     it (77 x 1001 x 1237: 7.1 in 16 rows, 8.2 in 32, 11.3 in 64);
-//   from there tiles of 32 rows, which load half as much of B per product (128 x 768 x 3072: 6.3 against 6.9);
-//   above 12000 steps tiles of 64 rows while there are 128 of them (700 x 2001 x 803: 18.6 against 21.2 and 22.7; 100 x
-//     4001 x 4003, 126 tiles: 34 against 22 in 32 rows).
-// Wavefronts: 4 for at most six steps of k, or when 8 of each tile would be more than eight per CU (1024 x 768 x 768 in 32
-// rows: 8.1 with 4, 10.8 with 8); 16 on the smallest tiles when they are few and K is long (32 x 3292 x 704: 8.4 against
-// 8.7 and 10.7 with 8 and 4); 8 otherwise.
-//
-// A tile's steps go to several workgroups where that saves more trips to memory than the meeting costs.  Microseconds as
-// measured: a pair of steps of every worker is a trip, and a launch takes 3.0 + 1.2 for each trip of four wavefronts, 3.8 +
-// 1.8 of eight, 4.2 + 3 of sixteen, 4 + 2.1 (1.7) in 32 rows of eight (four); the meeting takes 2.4 as long as there are
-// at most eight wavefronts on a CU.  Asked for is 0.7 on top, and more than
-// 20 steps: with the operands in cache 8 x 920 x 552 takes 6.1 in one piece and 6.5 in three.  3 x 11304 x 910 27.3 -> 9.3, 32 x 8192 x 512 18.5 -> 7.8,
-// 92 x 4184 x 115 11.6 -> 7.0, 1 x 3643 x 2512 11.2 -> 7.4, 99 x 3481 x 512 11.7 -> 7.8; 77 x 1001 x 1237 (two trips)
-// would go from 7.0 to 7.8 and is not split.
-struct Plan {
-  unsigned rows, waves;         // of a workgroup that has all of K
-  unsigned splits, splitWaves;  // of tiles of 16 rows; splits 1: not better
-  unsigned cost, splitCost;     // hundredths of a microsecond
-};
-Plan plan_of(unsigned m, unsigned n, unsigned k, unsigned batch) {
-  const unsigned steps = (k + 63) / 64;
-  const unsigned long long columns = (unsigned long long)((n + 63) / 64) * batch;
-  const unsigned long long tiles16 = (m + 15) / 16 * columns, tiles32 = (m + 31) / 32 * columns, tiles64 = (m + 63) / 64 * columns;
-  const unsigned long long work = tiles16 * steps;
-  Plan p{16, 8, 1, 0, 0, ~0u};
-  if (work > 12000 && tiles64 >= 128) p.rows = 64, p.waves = steps <= 6 ? 4 : 8;
-  else if (work > 4096 && m > 16) p.rows = 32, p.waves = steps <= 6 || tiles32 * 8 > 2048 ? 4 : 8;
-  else if (steps <= 6 || tiles16 * 8 > 2048) p.waves = 4;
-  else if (tiles16 <= 128 && steps >= 30) p.waves = 16;
-  auto trips = [&](unsigned waves) { return (steps + 2 * (waves - 1) - 1) / (2 * (waves - 1)); };
-  p.cost = p.rows == 32 ? 400 + (p.waves == 4 ? 170 : 210) * trips(p.waves)
-                        : p.waves == 4 ? 300 + 120 * trips(4) : p.waves == 8 ? 380 + 180 * trips(8) : 420 + 300 * trips(16);
-  if (steps <= 20 || p.rows == 64 || tiles16 * 16 * kCols > kMaxResults) return p;
-  for (unsigned waves = 4; waves <= 8; waves += 4)
-    for (unsigned want = 1; want <= 3; ++want) {  // trips
-      const unsigned splits = (steps + 2 * (waves - 1) * want - 1) / (2 * (waves - 1) * want);
-      const unsigned cost = (waves == 4 ? 300 + 120 * want : 380 + 180 * want) + 240;
-      if (splits < 2 || splits > 32 || tiles16 * splits * waves > 2048 || cost + 70 > p.cost || cost >= p.splitCost) continue;
-      p.splits = splits;
-      p.splitWaves = waves;
-      p.splitCost = cost;
-    }
-  return p;
-}
-
 unsigned long long* meeting_of(hipStream_t stream) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return nullptr;
@@ -363,7 +318,7 @@ bool qgemm_small_splits(hipStream_t stream, unsigned m, unsigned n, unsigned k, 
   return plan.splits > 1 && plan.splitCost + 70 <= instead && meeting_of(stream) != nullptr;
 }
 
-int qgemm_small_launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o) {
+int qgemm_small_launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o, bool split) {
   if ((unsigned long long)p.M * p.K < 16 || (unsigned long long)p.K * p.N < 4) {
     const unsigned long long total = (unsigned long long)p.M * p.N * p.batch;
     if ((total + 255) / 256 > 0x7fffffffull) return set_error(TFCC_ROCM_INVALID_ARGUMENT, "quantized matmul: too many results");
@@ -372,7 +327,7 @@ int qgemm_small_launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o
   }
   p.vectorStores = p.N % 4 == 0 && p.strideC % 4 == 0 && (uintptr_t)p.C % 16 == 0 && (uintptr_t)p.Q % 4 == 0;
   const Plan plan = plan_of(p.M, p.N, p.K, p.batch);
-  if (unsigned long long* const meeting = plan.splits > 1 ? meeting_of(stream) : nullptr)
+  if (unsigned long long* const meeting = plan.splits > 1 && (split || plan.better) ? meeting_of(stream) : nullptr)
     return plan.splitWaves == 4 ? launch<16, 4, true>(stream, p, o, plan.splits, meeting) : launch<16, 8, true>(stream, p, o, plan.splits, meeting);
   if (plan.rows == 64) return plan.waves == 4 ? launch<64, 4>(stream, p, o) : launch<64, 8>(stream, p, o);
   if (plan.rows == 32) return plan.waves == 4 ? launch<32, 4>(stream, p, o) : launch<32, 8>(stream, p, o);

@@ -30,7 +30,8 @@ struct QSmallOutputs {
 
 // Any shape and alignment; operands well below 2^31 bytes.
 bool qgemm_small_supported(const QGemmParams& p);
-int qgemm_small_launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o);
+// split: by several workgroups per tile where qgemm_small_splits says so, whether or not that beats one workgroup per tile.
+int qgemm_small_launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o, bool split = false);
 // Whether the product would be split over several workgroups per tile, and be faster than a kernel that takes `instead`
 // hundredths of a microsecond.
 bool qgemm_small_splits(hipStream_t stream, unsigned m, unsigned n, unsigned k, unsigned instead);
