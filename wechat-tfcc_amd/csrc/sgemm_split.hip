@@ -27,11 +27,11 @@
 // results, which happens by chance (a sum that cancels to zero, in one product of ten), are read once more, and all of the
 // tile's if there are many (sparse operands on both sides) or a magnitude was 2^30 or more.
 //
-// What that costs, us, in order: normal operands; one row of zeros; the last quarter of the rows; one value in a hundred in
-// both operands; one value of 2^31; one NaN; and normal operands on the fp32 ops:
-//   4096^3, 128 x 256 tiles        640   640   612   595   689   1486   915
-//   2048^3, 128 x 128               99   110    99   129   131     304   125
-//   1024 x 1024 x 2048, 64 x 64     31    32    31    46    48     110    35
+// What that costs, us, in order, on one card: normal operands; one row of zeros; the last quarter of the rows; one value in a
+// hundred in both operands; one value of 2^31; one NaN; two results that cancel; and any operands on the fp32 ops:
+//   4096^3, 128 x 256 tiles        602   602   589   583   683   1459   595   910
+//   2048^3, 128 x 128               93    96    91   128   126    301    96   120
+//   1024 x 1024 x 2048, 64 x 64     30    31    30    45    47    106    31    33
 //
 // Two kernels.  What they have in common is that vector instructions run under bf16 matrix ops: up to six of them between
 // two of 32 cycles cost next to nothing, if they stand there; a wavefront that issues matrix ops back to back keeps the
@@ -311,8 +311,9 @@ __device__ __forceinline__ bool split_failed(const SgemmParams& p, const Tile& t
 // deep: a thread loads four or eight values of a row of A and eight of a column of B and splits them on the way from its
 // registers to LDS, once for the workgroup; the wavefronts read the pieces in operand order.
 //
-// Bound by power, the matrix cores and the splitting: 4096^3 in 128 x 256 tiles 915 -> 623 us, 221 TFLOP/s; the matrix ops
-// alone, from registers on the same operands, sustain 302.  (128 x 128 tiles, two to a CU, split four values to six
+// Bound by power, the matrix cores and the splitting: 4096^3 in 128 x 256 tiles 910 -> 602 us, 228 TFLOP/s (214 to 228 by the
+// card); the matrix ops alone, from registers on the same operands, sustain 302.  Times against 623 on another card:
+// (128 x 128 tiles, two to a CU, split four values to six
 // matrix ops' worth instead of three: 669 us.  256 x 256 tiles, two values: 600, but there are registers for one
 // accumulator only; with a block's six terms summed from zero, smallest first, and then added to it 635, and one
 // product in a row still 3.5e-8.  A wavefront for each SIMD on 128 x 128, more slabs on their way, two K groups

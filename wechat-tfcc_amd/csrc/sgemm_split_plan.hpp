@@ -12,7 +12,8 @@ enum Kernel { kNone = -1, kWide = 0, k128 = 1, k64 = 2 };  // tiles of 128 x 256
 // tiles all of it takes three quarters of what it takes when all have two; 64 x 64 tiles are multiple); the kernels on the
 // fp32 matrix ops reach some 115 TFLOP/s, 105 where a K or an N is no multiple of their pieces, and more on large products,
 // which have the most to gain here.  Of 420 shapes, even over the logarithm of 64 .. 4096 rows and 64 .. 8192 for K and N, up to
-// 2^35 products, 60 come here, 1.43 times as fast on the average and none slower (4096^3: 915 -> 623 us).  The larger tiles take
+// 2^35 products, 60 come here, 1.43 times as fast on the average and none slower; 150 others that come here take 0.70 of their
+// time, one of them 1.02 (4096^3: 910 -> 602 us, to 641 by the card).  The larger tiles take
 // what they are thought to be faster at: 38 shapes within a tenth of that line take 1.0 to 1.9 times as long on the fp32 ops up
 // to it, and 0.98 to 1.5 times from it on.  64 x 64 tiles have to be
 // faster by an eighth, and by a quarter where the product takes less than 60 us otherwise: those that are not gain 6 % on the average and lose up to
