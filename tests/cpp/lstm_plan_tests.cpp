@@ -30,6 +30,19 @@ int main() {
           for (unsigned u = 0; u < units; u += 8) ++needed;
         EXPECT((workspace_bytes(4, units, directions, cus) != 0) == (cus > 0 && needed <= (unsigned)cus));
       }
+  for (unsigned directions = 1; directions <= 2; ++directions)
+    for (unsigned batch = 1; batch <= 16; ++batch)
+      for (unsigned units = 1; units <= 1024; ++units) {
+        const unsigned rows = rows_of_xcd(batch, units, directions, 256);
+        EXPECT((rows != 0) == (units <= 768));
+        EXPECT(rows_of_xcd(batch, units, directions, 128) == 0);
+        if (rows == 0) continue;
+        const unsigned groups = (batch + rows - 1) / rows, each = 8 * ((units + 255) / 256);
+        EXPECT(rows <= 4 && groups * directions <= kXcds && (units + each - 1) / each <= kCusOfXcd);
+        // two sets of 64-bit words with this form's pitch fit in front of the flag
+        const size_t pitch = (units + 255) / 256 * 256;
+        EXPECT(2 * directions * batch * pitch * 8 + 64 <= workspace_bytes(batch, units, directions, 256));
+      }
   if (failures == 0) std::printf("lstm plan: all passed\n");
   return failures != 0;
 }

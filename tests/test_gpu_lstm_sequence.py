@@ -74,6 +74,24 @@ def test_sequence_against_the_oracle(pkg, T, seq, batch, hidden, directions):
             assert np.array_equal(T.n(p), T.n(q))
 
 
+@pytest.mark.parametrize("seq,batch,hidden,directions", [
+    (1, 4, 256, 2), (2, 5, 257, 2), (3, 7, 512, 2), (4, 9, 513, 2), (5, 13, 768, 2), (6, 16, 767, 1), (9, 15, 249, 2),
+    (11, 8, 505, 1), (8, 9, 769, 1), (13, 11, 745, 2), (7, 1, 768, 1), (10, 10, 8, 1)])
+def test_rows_dealt_out_to_xcds(pkg, T, seq, batch, hidden, directions):
+    """up to 768 units: one to four rows to an XCD with fewer in the last group, units that do not fill a workgroup or a
+    lane's four k, sequences around the four steps whose inputs are fetched together; twice, with the same bits"""
+    print("lstm rows", seq, batch, hidden, directions, flush=True)
+    x, sets = setup(T, seq, batch, 24, hidden, directions)
+    backward = (True, False)[:directions]
+    outs, keep = launch(pkg, T, x, sets, backward)
+    compare(T, outs, x, sets, backward)
+    assert gave_up(T, keep) == 0
+    again, keep = launch(pkg, T, x, sets, backward)
+    for a, b in zip(outs, again):
+        for p, q in zip(a, b):
+            assert np.array_equal(T.n(p), T.n(q))
+
+
 @pytest.mark.parametrize("seq,batch,hidden", [(5, 3, 96), (4, 12, 600), (1, 1, 5), (3, 16, 1024)])
 def test_a_wait_that_is_over_at_once(pkg, T, seq, batch, hidden):
     x, sets = setup(T, seq, batch, 24, hidden, 2)

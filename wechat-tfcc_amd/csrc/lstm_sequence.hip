@@ -4,20 +4,22 @@
 // unit's result of the step before.  A launch per step costs 4.8 us (4 x 512) although its arithmetic takes 0.2 us,
 // because the state kernel is fetched again and the launch itself has to be paid.  Here a workgroup owns eight units for
 // the whole sequence, keeps their columns of the state kernel in registers, and the workgroups hand their part of h to
-// each other through memory: 2.3 us per step, both directions at once (1.7 for 1 x 256, 3.8 for 4 x 1024).  What is left
-// is the way of h to memory and back and the polls that came too early.
+// each other through memory: 2.1 us per step of 4 x 512, both directions at once (3.0 for 4 x 1024).  What is left is
+// the way of h to memory and back and the polls that came too early.  Up to 768 units a second form keeps h inside an XCD:
+// 1.5 us per step (lstm_xcd_kernel, below); the first one then takes what is recorded in a
+// graph, and what a part of a partitioned GPU gets.
 //
 // The exchange is made of words that a reader polls themselves, so nothing is ordered by fences.  There are two kinds:
-//   Up to 256 units 64-bit words of a value and the number of the step it belongs to: a reader waits for its step.  Two
-//   sets of words alternate; a workgroup writes step t + 2 only after it has read all of step t + 1, which every other
+//   Up to 256 units, and in the second form, 64-bit words of a value and the number of the step it belongs to: a reader waits
+//   for its step.  Two sets of words alternate; a workgroup writes step t + 2 only after it has read all of step t + 1, which every other
 //   workgroup wrote after it had read all of step t, so no word is overwritten before its last reader is through.
 //   With more units half the bytes, and a quarter of the loads, make up for one more store: 32-bit words, a value each,
 //   four to a load.  One that has not been written holds kUnwritten.  Four sets take turns.  A workgroup that has read all
 //   of step t knows that everyone has read all of step t - 1; behind its results for step t + 1 it clears its words of step
 //   t - 1, has seen that clearing done before it stores its results for step t + 2, and those are what a reader has to have
 //   before it looks at the cleared words again, for step t + 3.
-// Served bidirectional sequences, us, all in 64-bit words before: 64 of 4 x 512 218 -> 213, 31 of 7 x 600 206 -> 183, 64 of
-// 4 x 1024 327 -> 301, 32 of 12 x 1024 448 -> 345; in 32-bit words 64 of 1 x 256 take 141 against 131.
+// Served bidirectional sequences in the first form, us, all in 64-bit words before: 64 of 4 x 512 218 -> 213, 31 of 7 x 600
+// 206 -> 183, 64 of 4 x 1024 327 -> 301, 32 of 12 x 1024 448 -> 345; in 32-bit words 64 of 1 x 256 take 141 against 131.
 //
 // All workgroups have to run at the same time.  The launcher asks for at most one per CU, but other work may hold CUs, so
 // every wait is bounded: a workgroup that has waited `waitTicks` raises a flag and ends, the others see the flag and end,
@@ -26,6 +28,7 @@
 //
 // Arithmetic: tfcc/core/operations/tfcc_rnn.cpp:29-135 with the cell of tfcc/mkl/kernel/tfcc_mklcellkernel.hpp:51-87.
 #include <mutex>
+#include <type_traits>
 
 #include "common.hpp"
 #include "lstm_sequence_plan.hpp"
@@ -49,6 +52,7 @@ struct SequenceParams {
   unsigned seq, batch, units, directions;
   float forget;
   unsigned blocksPerDirection;
+  unsigned groups, rowsPerGroup;  // of the form with an XCD for a group of rows; none: the other one
   unsigned* words;  // [set][direction][batch][pitch]
   unsigned* failed;
   unsigned long long waitTicks;
@@ -66,17 +70,19 @@ __device__ __forceinline__ unsigned word_of(float value) {
 __device__ __forceinline__ unsigned long long numbered_word(float value, unsigned step) {
   return ((unsigned long long)step << 32) | __builtin_bit_cast(unsigned, value);
 }
+constexpr unsigned kStepMask = 0x0fffffffu;  // where the words of a step carry the XCD they come from above it
+using lstm_plan::kXcds;
 constexpr bool numbered(unsigned pitch) { return pitch <= 256; }  // 64-bit words, with the number of the step
 
 // Step 0 reads the initial h from the first set (as words of step 1); the others hold nothing anybody waits for.  Units that
 // do not exist are zeros in every set.
-__global__ __launch_bounds__(256) void lstm_exchange_init_kernel(SequenceParams p, unsigned pitch, unsigned total) {
+__global__ __launch_bounds__(256) void lstm_exchange_init_kernel(SequenceParams p, unsigned pitch, unsigned total, bool withNumbers) {
   const unsigned i = blockIdx.x * 256 + threadIdx.x;
   if (i == 0) *p.failed = 0;
   if (i >= total) return;
   const unsigned u = i % pitch, b = i / pitch % p.batch, d = i / pitch / p.batch;
   const float h = u < p.units ? p.s[d].h0[(size_t)b * p.units + u] : 0.f;
-  if (numbered(pitch)) {
+  if (withNumbers) {
     reinterpret_cast<unsigned long long*>(p.words)[i] = numbered_word(h, 1);
     reinterpret_cast<unsigned long long*>(p.words)[(size_t)total + i] = 0;
     return;
@@ -380,6 +386,200 @@ __global__ __launch_bounds__(64 * WAVES) void lstm_sequence_kernel(SequenceParam
   }
 }
 
+// The XCD that a wavefront runs on: four bits of the register XCC_ID.
+__device__ __forceinline__ unsigned xcd_id() { return __builtin_amdgcn_s_getreg(20 | (3 << 11)); }
+
+// The form for up to 768 units on a whole GPU: the state kernel of a direction fits the registers of one XCD's 32 CUs, 16, 64
+// or 144 of a lane, so nothing has to leave the XCD between two steps, and the rows of the batch, which do not need one
+// another, are dealt out to the XCDs, four groups of them to each of two directions, eight to one.  A store that stops in the XCD's L2
+// and a load at device scope, which looks there first, take 0.78 us from all to all of 32 workgroups with 32 words each,
+// where a store to memory takes 1.16, and 1.38 with the workgroups on eight XCDs.
+//
+// That the workgroups of a group share an XCD is what the dispatch of workgroups to XCDs in turn gives; nothing depends on
+// it but time.  The words of the first step go through to memory and carry the XCD they come from; everyone reads all of them,
+// so everyone knows whether they are all from one, and if not, h goes through to memory in all steps.
+//
+// A wavefront owns UPW units.  A lane takes four k in 256 of all their gates, so a row of h is KQ loads from LDS, and
+// the products are on the vector unit: one row leaves three of the four rows of a 4 x 4 x 1 matrix op empty, and with four the
+// time is the same.  Us per step, 100 steps with both directions, the form below -> this one: 4 x 256 1.75 -> 1.22, 16 x 256 4.9
+// -> 1.7, 4 x 512 2.13 -> 1.53, 8 x 512 2.75 -> 1.86, 16 x 512 4.9 -> 2.56, 4 x 768 2.64 -> 2.20, 12 x 700 4.4 -> 3.4.  Of the 1.53,
+// without it: the products 0.26, the cell's functions 0.28, inputs and results 0.15; the exchange and the rest is 0.88.  (The
+// form below on one XCD, all rows in each: 4 x 512 1.98, 8 x 512 2.71, 4 x 768 3.35.  Words that have arrived not asked for again:
+// 16 x 512 2.85.  Results stored a step later: 2.63; inputs fetched one step at a time, not four: 2.61.)
+template <int ROWS, int KQ>
+__global__ __launch_bounds__(512) void lstm_xcd_kernel(SequenceParams p) {
+  constexpr int WAVES = 8, T = 64 * WAVES, K = 256 * KQ, UPW = KQ, SUMS = UPW * ROWS;
+  constexpr int LEFT = values_left<SUMS, 32, 4>(), COPIES = 16 / (SUMS / LEFT);
+  static_assert(LEFT <= COPIES, "a lane finishes one value");
+  __shared__ __attribute__((aligned(16))) float hs[2][ROWS][K];
+  __shared__ int gaveUp, apart;
+  const unsigned turn = blockIdx.x % kXcds, d = turn / p.groups, group = turn - d * p.groups;
+  if (d >= p.directions) return;  // nothing for this XCD
+  const int tid = threadIdx.x, lane = tid & 63, gate = lane & 3;
+  const unsigned xcd = xcd_id();
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const unsigned units = p.units, row0 = group * p.rowsPerGroup, rows = min(p.rowsPerGroup, p.batch - row0);
+  const Sequence& s = p.s[d];
+  const size_t setSize = (size_t)p.directions * p.batch * K;
+  unsigned long long* const mine = reinterpret_cast<unsigned long long*>(p.words) + ((size_t)d * p.batch + row0) * K;
+  for (int i = tid; i < 2 * ROWS * K; i += T) (&hs[0][0][0])[i] = 0.f;  // rows and units that do not exist stay zero
+  if (tid == 0) {
+    gaveUp = p.waitTicks == 0;  // no wait at all: the launch behind this one has the sequence
+    apart = 0;
+  }
+  __syncthreads();
+
+  const unsigned u0 = (blockIdx.x / kXcds * WAVES + wave) * UPW;
+  float w[KQ][4][4][UPW];  // [.][k][gate][unit]
+#pragma unroll
+  for (int i = 0; i < KQ; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const unsigned k = 256 * i + 4 * lane + e;
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int n = 0; n < UPW; ++n)
+          w[i][e][g][n] = k < units && u0 + n < units ? s.kernel[(size_t)k * 4 * units + (size_t)g * units + u0 + n] : 0.f;
+    }
+  // the unit and the row whose sum this lane ends with, as in the other form
+  int base = 0;
+  {
+    float none[SUMS] = {};
+    sum_over_lanes<SUMS, 32, 4>(none, lane, base);
+  }
+  const int copy = (lane >> 2) & (COPIES - 1);
+  const unsigned finished = base + (LEFT > 1 ? copy : 0);  // [unit][row]
+  const unsigned u = u0 + finished / ROWS, r = finished % ROWS, fm = row0 + r;
+  const bool valid = copy < LEFT && r < rows && u < units;
+  auto inputOf = [&](unsigned step) {
+    const unsigned t = s.backward ? p.seq - 1 - step : step;
+    return valid ? s.x[((size_t)t * p.batch + fm) * 4 * units + (size_t)gate * units + u] : 0.f;
+  };
+  const size_t at = (size_t)fm * units + u;
+  const float bv = valid ? s.bias[(size_t)gate * units + u] : 0.f;
+  float cPrev = valid ? s.c0[at] : 0.f;
+  const float forget = gate == 2 ? p.forget : -0.f;  // (adding -0 changes nothing)
+  constexpr int AHEAD = 4;
+  float xin[AHEAD], xNext[AHEAD];
+#pragma unroll
+  for (int q = 0; q < AHEAD; ++q) xin[q] = (unsigned)q < p.seq ? inputOf(q) : 0.f;
+
+  // false: someone has waited too long
+  auto take = [&](unsigned step, auto q) __attribute__((always_inline)) -> bool {
+    float (*h)[K] = hs[step & 1u];
+    const unsigned long long* words = mine + (step & 1u) * setSize;
+    const unsigned long long start = wall_clock64();
+    constexpr int PER = (ROWS * K + T - 1) / T;
+    unsigned long long v[PER];
+    bool wanted[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const unsigned i = tid + k * T;
+      wanted[k] = i < rows * K && i % K < units;
+    }
+    for (unsigned tries = 0;; ++tries) {
+      bool ready = true;
+#pragma unroll
+      for (int k = 0; k < PER; ++k)
+        v[k] = wanted[k] ? __hip_atomic_load(words + tid + k * T, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+#pragma unroll
+      for (int k = 0; k < PER; ++k) ready = ready && (!wanted[k] || ((unsigned)(v[k] >> 32) & kStepMask) == step + 1);
+      if (ready) break;
+      if ((tries & 15u) == 15u &&
+          (wall_clock64() - start > p.waitTicks ||
+           __hip_atomic_load(p.failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+        gaveUp = 1;
+        break;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const unsigned i = tid + k * T;
+      if (wanted[k]) h[i / K][i % K] = __builtin_bit_cast(float, (unsigned)v[k]);
+      if (step == 1 && wanted[k] && (unsigned)(v[k] >> 60) != xcd) apart = 1;
+    }
+    __syncthreads();
+    if (gaveUp) {  // the same for the whole workgroup
+      if (tid == 0) __hip_atomic_store(p.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return false;
+    }
+    const bool last = step + 1 == p.seq;
+    if (q == 0) {
+#pragma unroll
+      for (unsigned n = 0; n < AHEAD; ++n) xNext[n] = step + AHEAD + n < p.seq ? inputOf(step + AHEAD + n) : 0.f;
+    }
+
+    float sum[4][SUMS];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int n = 0; n < SUMS; ++n) sum[g][n] = 0.f;
+#pragma unroll
+    for (int i = 0; i < KQ; ++i)
+#pragma unroll
+      for (int b = 0; b < ROWS; ++b) {
+        const lstm_v4f a = *reinterpret_cast<const lstm_v4f*>(&h[b][256 * i + 4 * lane]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int n = 0; n < UPW; ++n) sum[g][ROWS * n + b] = fmaf(a[e], w[i][e][g][n], sum[g][ROWS * n + b]);
+      }
+    // the four gates to the four lanes of a quad
+    float half[2][SUMS], v1[SUMS];
+    const bool odd = (lane & 1) != 0, upper = (lane & 2) != 0;
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int n = 0; n < SUMS; ++n) {
+        float same, other;
+        butterfly_pair<2>(upper ? sum[g][n] : sum[g + 2][n], same, other);
+        half[g][n] = (upper ? sum[g + 2][n] : sum[g][n]) + other;
+      }
+#pragma unroll
+    for (int n = 0; n < SUMS; ++n) {
+      float same, other;
+      butterfly_pair<1>(odd ? half[0][n] : half[1][n], same, other);
+      v1[n] = (odd ? half[1][n] : half[0][n]) + other;
+    }
+    int unused = 0;
+    sum_over_lanes<SUMS, 32, 4>(v1, lane, unused);
+    float total = v1[0];
+#pragma unroll
+    for (int a = 1; a < LEFT; ++a) total = copy == a ? v1[a] : total;
+
+    // ---- the cell
+    const float act = sigmoid_or_tanh(xin[q] + total + bv + forget, gate == 1);
+    const float xi = of_quad<0>(act), xc = of_quad<1>(act), xf = of_quad<2>(act), xo = of_quad<3>(act);
+    const float c = __fadd_rn(__fmul_rn(xc, xi), __fmul_rn(cPrev, xf)), hn = sigmoid_or_tanh(c, true) * xo;
+    cPrev = c;
+    if (valid && gate == 0) {
+      unsigned long long* const word = mine + ((step + 1) & 1u) * setSize + (size_t)r * K + u;
+      if (!last) {
+        const unsigned long long v = numbered_word(hn, step + 2) | (step == 0 ? (unsigned long long)xcd << 60 : 0ull);
+        if (step == 0 || apart) __hip_atomic_store(word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else __hip_atomic_store(word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      s.out[(size_t)step * p.batch * units + at] = hn;
+      if (last) {
+        s.h[at] = hn;
+        s.c[at] = c;
+      }
+    }
+    return true;
+  };
+  for (unsigned step = 0; step < p.seq; step += AHEAD) {
+    if (!take(step, std::integral_constant<int, 0>{})) return;
+    if (step + 1 >= p.seq || !take(step + 1, std::integral_constant<int, 1>{})) return;
+    if (step + 2 >= p.seq || !take(step + 2, std::integral_constant<int, 2>{})) return;
+    if (step + 3 >= p.seq || !take(step + 3, std::integral_constant<int, 3>{})) return;
+#pragma unroll
+    for (int n = 0; n < AHEAD; ++n) xin[n] = xNext[n];
+  }
+}
+
 // The sequence once more in one workgroup per direction, if the launch before it gave up.
 __global__ __launch_bounds__(1024) void lstm_repair_kernel(SequenceParams p) {
   if (__hip_atomic_load(p.failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) return;
@@ -430,10 +630,27 @@ int launch(hipStream_t stream, SequenceParams p) {
     attrSet[dev] = true;
   }
   const unsigned total = p.directions * p.batch * pitch;
-  hipLaunchKernelGGL(lstm_exchange_init_kernel, dim3((total + 255) / 256), dim3(256), 0, stream, p, pitch, total);
+  hipLaunchKernelGGL(lstm_exchange_init_kernel, dim3((total + 255) / 256), dim3(256), 0, stream, p, pitch, total, numbered(pitch));
   hipLaunchKernelGGL(kern, dim3(p.blocksPerDirection * p.directions), dim3(64 * WAVES), lds, stream, p);
   hipLaunchKernelGGL(lstm_repair_kernel, dim3(p.directions), dim3(1024), 0, stream, p);
   return check_launch("lstm_sequence");
+}
+
+template <int ROWS, int KQ>
+int launch_xcd(hipStream_t stream, const SequenceParams& p) {
+  constexpr unsigned pitch = 256 * KQ;
+  const unsigned total = p.directions * p.batch * pitch, workgroups = (p.units + 8 * KQ - 1) / (8 * KQ);
+  hipLaunchKernelGGL(lstm_exchange_init_kernel, dim3((total + 255) / 256), dim3(256), 0, stream, p, pitch, total, true);
+  hipLaunchKernelGGL((lstm_xcd_kernel<ROWS, KQ>), dim3(kXcds * workgroups), dim3(512), 0, stream, p);
+  hipLaunchKernelGGL(lstm_repair_kernel, dim3(p.directions), dim3(1024), 0, stream, p);
+  return check_launch("lstm_sequence");
+}
+template <int KQ>
+int launch_xcd_rows(hipStream_t stream, const SequenceParams& p) {
+  if (p.rowsPerGroup == 1) return launch_xcd<1, KQ>(stream, p);
+  if (p.rowsPerGroup == 2) return launch_xcd<2, KQ>(stream, p);
+  if (p.rowsPerGroup == 3) return launch_xcd<3, KQ>(stream, p);
+  return launch_xcd<4, KQ>(stream, p);
 }
 
 template <int KI, int WAVES>
@@ -445,6 +662,11 @@ int launch_rows(hipStream_t stream, const SequenceParams& p) {
 }
 
 int launch_units(hipStream_t stream, const SequenceParams& p) {
+  if (p.rowsPerGroup != 0) {
+    if (p.units <= 256) return launch_xcd_rows<1>(stream, p);
+    if (p.units <= 512) return launch_xcd_rows<2>(stream, p);
+    return launch_xcd_rows<3>(stream, p);
+  }
   // eight wavefronts, so eight units, per workgroup: with four, twice the workgroups poll; with twelve or sixteen, each of
   // which reads all of h from LDS, that takes longer than the trip to memory (4 x 1024: 3.8, 5.8 and 7.0 us per step with
   // eight, twelve and sixteen)
@@ -467,6 +689,16 @@ struct Turn {
 };
 Turn g_turns[16];
 
+// of the current device; 0: unknown
+int compute_units() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return cus;
+}
+
 }  // namespace
 
 }  // namespace tfcc_rocm
@@ -476,12 +708,7 @@ using namespace tfcc_rocm;
 extern "C" {
 
 size_t tfcc_rocm_lstm_sequence_workspace(unsigned batch, unsigned units, unsigned directions) {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-    (void)hipGetLastError();
-    return 0;
-  }
-  return lstm_plan::workspace_bytes(batch, units, directions, cus);
+  return lstm_plan::workspace_bytes(batch, units, directions, compute_units());
 }
 
 int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc* q) {
@@ -500,6 +727,9 @@ int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc
   }
   p.seq = q->seq; p.batch = q->batch; p.units = q->units; p.directions = q->directions;
   p.forget = q->forget;
+  p.rowsPerGroup = lstm_plan::rows_of_xcd(q->batch, q->units, q->directions, compute_units());
+  if (q->seq > kStepMask - 2) p.rowsPerGroup = 0;  // (the words' number has 28 bits)
+  p.groups = p.rowsPerGroup ? (q->batch + p.rowsPerGroup - 1) / p.rowsPerGroup : 0;
   p.words = static_cast<unsigned*>(q->workspace);
   p.failed = reinterpret_cast<unsigned*>(static_cast<char*>(q->workspace) + need - 64);
   p.waitTicks = (unsigned long long)q->wait_us * 100;  // of the 100 MHz clock
@@ -509,7 +739,10 @@ int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc
   hipStream_t s = as_stream(stream);
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &capturing) != hipSuccess) (void)hipGetLastError();  // the null stream beside a capture: it is not captured
-  if (capturing != hipStreamCaptureStatusNone) return launch_units(s, p);
+  if (capturing != hipStreamCaptureStatusNone) {
+    p.rowsPerGroup = 0;  // replays are not ordered among one another; two of the first form fit side by side up to 512 units
+    return launch_units(s, p);
+  }
   Turn& turn = g_turns[dev];
   std::lock_guard<std::mutex> lk(turn.mtx);
   if (!turn.used) turn.first = s;

@@ -23,5 +23,15 @@ inline size_t workspace_bytes(unsigned batch, unsigned units, unsigned direction
   return (size_t)2 * directions * batch * padded_units(units) * 8 + 64;
 }
 
+constexpr unsigned kXcds = 8, kCusOfXcd = 32;  // of a whole GPU; workgroups are dispatched to the XCDs in turn
+
+// Rows of the batch that the workgroups of one XCD take, where a direction's state kernel fits the registers of one; 0: it does
+// not, or the GPU is a part of one.  Beyond 768 units it would take all of them.
+inline unsigned rows_of_xcd(unsigned batch, unsigned units, unsigned directions, int cus) {
+  if (units > 768 || cus < (int)(kXcds * kCusOfXcd)) return 0;
+  const unsigned groups = kXcds / directions;
+  return (batch + groups - 1) / groups;
+}
+
 }  // namespace lstm_plan
 }  // namespace tfcc_rocm
