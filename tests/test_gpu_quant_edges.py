@@ -24,6 +24,21 @@ def test_quantize_with_the_range_of_the_data(pkg, T, total, dtype, skip):
     assert np.array_equal(T.n(q), O.quantize(x[skip:], lo, hi, dtype))
 
 
+@pytest.mark.parametrize("total", [32768, 32769, 36864, (1 << 20) - 3, (1 << 20) + 1, (2 << 20) + 2, (4 << 20) + 3, 8 << 20, (8 << 20) + 1])
+@pytest.mark.parametrize("dtype,middle", [("uint8", 0.1), ("int8", -300.0), ("int16", 1.0), ("int32", 0.0), ("uint8", 3e6)])
+def test_quantize_in_workgroups_that_agree_on_the_range(pkg, T, total, dtype, middle):
+    """one, two, four and eight pieces to a thread, whole numbers that fit 32 bits and that do not, a NaN and the extremes in
+    the first and the last workgroup"""
+    import torch
+    x = np.random.default_rng(total).normal(middle, 2.0, total).astype(np.float32)
+    x[3], x[-1], x[total // 3] = middle + 17.0, middle - 31.0, np.nan
+    q, mn, mx = pkg.quantize(T.t(x), getattr(torch, dtype))
+    lo, hi = float(np.nanmin(x)), float(np.nanmax(x))
+    assert (float(T.n(mn)[0]), float(T.n(mx)[0])) == (lo, hi)
+    given = O.quantize(x, lo, hi, dtype) if "int8" in dtype else T.n(pkg.quantize(T.t(x), getattr(torch, dtype), T.f1(lo), T.f1(hi)))
+    assert np.array_equal(T.n(q), given)
+
+
 @pytest.mark.parametrize("total", [5, 4095, 40001, LIMIT + 4])
 def test_quantize_over_its_own_input(pkg, T, total):
     import torch

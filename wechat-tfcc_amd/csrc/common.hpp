@@ -243,6 +243,16 @@ __device__ __forceinline__ float wave_sum(float v) {
   butterfly_pair<1>(v, a, b); v = a + b;
   return v;
 }
+__device__ __forceinline__ float wave_min(float v) {
+  float a, b;
+  butterfly_pair<32>(v, a, b); v = fminf(a, b);
+  butterfly_pair<16>(v, a, b); v = fminf(a, b);
+  butterfly_pair<8>(v, a, b); v = fminf(a, b);
+  butterfly_pair<4>(v, a, b); v = fminf(a, b);
+  butterfly_pair<2>(v, a, b); v = fminf(a, b);
+  butterfly_pair<1>(v, a, b); v = fminf(a, b);
+  return v;
+}
 __device__ __forceinline__ float wave_max(float v) {
   float a, b;
   butterfly_pair<32>(v, a, b); v = fmaxf(a, b);

@@ -7,6 +7,8 @@
 // tfcc/mkl/kernel/tfcc_mklquantizationkernel.avx256.cpp:55-145 (the AVX2 kernels: nearest-even
 // rounding, fused multiply-add) and the branches of
 // tfcc/mkl/interfaces/tfcc_mklquantizationinterface.cpp:47-69,72-147,191-240,284-333.
+#include <atomic>
+
 #include "common.hpp"
 #include "quant_ops.hpp"
 #include "stream_slots.hpp"
@@ -320,6 +322,33 @@ __device__ __forceinline__ long long quantize_one(float x, double scale, long lo
   return q > r.highest ? r.highest : q;
 }
 
+// quantize_one for values between mn and mx, or NaN: 32-bit whole numbers where all of them fit, half the instructions.
+struct QuantizeScalars {
+  double scale;
+  long long offset;
+  IntRange r;
+  bool fill, narrow;
+  int shift, nan;  // narrow: lowest - offset, and what a NaN becomes
+};
+__device__ __forceinline__ QuantizeScalars make_quantize_scalars(int outType, float mn, float mx) {
+  QuantizeScalars s;
+  s.r = int_range(outType);
+  s.fill = mn == mx;  // tfcc_mklquantizationinterface.cpp:58-61
+  s.scale = 0;
+  s.offset = 0;
+  if (!s.fill) quantized_scale_info(s.r.bits, mn, mx, &s.scale, &s.offset);
+  s.narrow = !s.fill && s.r.bits <= 16 && fabs((double)mn * s.scale) < 0x1p29 && fabs((double)mx * s.scale) < 0x1p29;
+  s.shift = (int)(s.r.lowest - s.offset);
+  s.nan = s.narrow ? (int)quantize_one(__builtin_nanf(""), s.scale, s.offset, s.r) : 0;
+  return s;
+}
+__device__ __forceinline__ long long quantize_one(float x, const QuantizeScalars& s) {
+  if (s.fill) return s.r.lowest;
+  if (!s.narrow) return quantize_one(x, s.scale, s.offset, s.r);
+  const int q = (int)rint((double)x * s.scale) + s.shift;
+  return x != x ? s.nan : min(max(q, (int)s.r.lowest), (int)s.r.highest);
+}
+
 __global__ __launch_bounds__(256) void quantize_kernel(const float* in, size_t total, const float* minV,
                                                        const float* maxV, void* out, int outType, int fromData) {
   const float mn = *minV, mx = *maxV;
@@ -388,8 +417,10 @@ __device__ __forceinline__ float dec(unsigned u) {
 // A small tensor in one launch: every workgroup reads all of it for the range, which every one of them finds alike, and
 // quantizes 4096 elements.  Bound by that read: the caches deliver about 64 bytes per clock to a CU, against three or
 // four launches.
-constexpr unsigned kWholeLimit = 128 * 1024;  // elements; 4096 elements: 18.6 -> 4.8 us per call, 77077: 6.1, 131072: 7.7 against
-// 8.6 for the form behind the limit, whose time does not grow with the size there
+constexpr unsigned kWholeLimit = 128 * 1024;  // elements; 4096 elements: 18.6 -> 3.4 us per call, 77077: 6.3, 131072: 7.7 against
+// 8.6 for the form in two launches, whose time does not grow with the size there
+constexpr unsigned kWholeBest = 32 * 1024;  // where the form below is as fast: 16384 elements 3.9 us here and 4.5 there, 32768 4.4 (4.7
+// from memory) and 4.5
 __global__ __launch_bounds__(1024) void quantize_whole_kernel(const float* in, unsigned total, void* out, int outType,
                                                               float* mnOut, float* mxOut) {
   __shared__ float shMn[16], shMx[16];
@@ -439,15 +470,11 @@ __global__ __launch_bounds__(1024) void quantize_whole_kernel(const float* in, u
     *mxOut = mx;
   }
   if (count == 0) return;
-  const IntRange r = int_range(outType);
-  const bool fillLowest = mn == mx;  // tfcc_mklquantizationinterface.cpp:58-61
-  double scale = 0;
-  long long offset = 0;
-  if (!fillLowest) quantized_scale_info(r.bits, mn, mx, &scale, &offset);
+  const QuantizeScalars scalars = make_quantize_scalars(outType, mn, mx);
   long long q[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) q[e] = fillLowest ? r.lowest : quantize_one(mine[e], scale, offset, r);
-  if (count == 4 && r.bits == 8 && ((uintptr_t)out & 3u) == 0) {
+  for (int e = 0; e < 4; ++e) q[e] = quantize_one(mine[e], scalars);
+  if (count == 4 && scalars.r.bits == 8 && ((uintptr_t)out & 3u) == 0) {
     unsigned word = 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) word |= ((unsigned)q[e] & 0xffu) << (8 * e);
@@ -597,6 +624,114 @@ __global__ void minmax_finish_kernel(float* mn, float* mx) {
   *mx = dec(*reinterpret_cast<const unsigned*>(mx));
 }
 
+// A tensor that the GPU's registers hold, in one launch: a workgroup reads its part once, the workgroups tell one another its
+// minimum and maximum, and each quantizes what it has.  A word of the exchange is a value and the number of the call, which no
+// other call has, so a reader waits for this call's, and nothing has to be cleared or ordered.  The workgroups need
+// not all run at once: one that has waited kTogetherWait for the others reads all of the input itself, as above.
+//
+// Bound by the launch, a store to memory and a load from it; with many elements to a workgroup by the reading.  us, the range
+// and the quantizing in a launch each before (up to 131072 elements the form above), input from memory: 77077 6.8 -> 5.1, 131072
+// 8.6 -> 5.2, 786432 8.9 -> 6.6, 2 M 11.3 -> 8.4, 8 M 21.1 -> 15.7 (17.5 with 64-bit whole numbers for every element).
+constexpr unsigned kTogetherWorkgroups = 256, kTogetherSlots = 256;  // of a launch; streams that have words for one
+constexpr unsigned kTogetherLimit = kTogetherWorkgroups * 1024 * 4 * 8;  // elements: 32 to a thread
+constexpr unsigned long long kTogetherWait = 20000;  // of the 100 MHz clock: 200 us
+__device__ unsigned long long togetherWords[kTogetherSlots * kTogetherWorkgroups * 2];
+
+template <int QUADS>
+__global__ __launch_bounds__(1024) void quantize_together_kernel(const float* in, size_t total, void* out, int outType, float* mnOut,
+                                                                 float* mxOut, unsigned slot, unsigned call) {
+  __shared__ float shMn[16], shMx[16];
+  __shared__ int alone;
+  const size_t total4 = total / 4, first = (size_t)blockIdx.x * (1024 * QUADS) + threadIdx.x;
+  const unsigned rest = (unsigned)(total & 3u);
+  if (threadIdx.x == 0) alone = 0;
+  float v[QUADS][4];
+  float mn = 3.402823466e+38f, mx = -3.402823466e+38f;
+#pragma unroll
+  for (int u = 0; u < QUADS; ++u) {
+    const size_t i = first + u * 1024;
+    if (i < total4) __builtin_memcpy(v[u], in + i * 4, 16);
+    else
+#pragma unroll
+      for (unsigned e = 0; e < 4; ++e) v[u][e] = i == total4 && e < rest ? in[i * 4 + e] : __builtin_nanf("");
+  }
+#pragma unroll
+  for (int u = 0; u < QUADS; ++u) {  // (a NaN is passed over)
+    mn = fminf(fminf(mn, fminf(v[u][0], v[u][1])), fminf(v[u][2], v[u][3]));
+    mx = fmaxf(fmaxf(mx, fmaxf(v[u][0], v[u][1])), fmaxf(v[u][2], v[u][3]));
+  }
+  auto join = [&]() {  // over the workgroup
+    mn = wave_min(mn);
+    mx = wave_max(mx);
+    __syncthreads();  // the last join's values are read
+    if ((threadIdx.x & 63) == 0) {
+      shMn[threadIdx.x >> 6] = mn;
+      shMx[threadIdx.x >> 6] = mx;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      mn = fminf(mn, shMn[w]);
+      mx = fmaxf(mx, shMx[w]);
+    }
+  };
+  join();
+  unsigned long long* const words = togetherWords + (size_t)slot * kTogetherWorkgroups * 2;
+  if (threadIdx.x == 0) {
+    const unsigned long long number = (unsigned long long)call << 32;
+    __hip_atomic_store(words + 2 * blockIdx.x, number | __float_as_uint(mn), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(words + 2 * blockIdx.x + 1, number | __float_as_uint(mx), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (threadIdx.x < gridDim.x) {
+    const unsigned long long start = wall_clock64();
+    while (true) {
+      const unsigned long long a = __hip_atomic_load(words + 2 * threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned long long b = __hip_atomic_load(words + 2 * threadIdx.x + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if ((unsigned)(a >> 32) == call && (unsigned)(b >> 32) == call) {
+        mn = fminf(mn, __uint_as_float((unsigned)a));
+        mx = fmaxf(mx, __uint_as_float((unsigned)b));
+        break;
+      }
+      if (wall_clock64() - start > kTogetherWait) {
+        alone = 1;
+        break;
+      }
+    }
+  }
+  join();
+  if (alone) {  // the same for the whole workgroup
+    for (size_t i = threadIdx.x; i < total; i += 1024) {
+      mn = fminf(mn, in[i]);
+      mx = fmaxf(mx, in[i]);
+    }
+    join();
+  }
+  if (first == 0) {
+    *mnOut = mn;
+    *mxOut = mx;
+  }
+  const QuantizeScalars scalars = make_quantize_scalars(outType, mn, mx);
+  const bool packed = scalars.r.bits == 8 && ((uintptr_t)out & 3u) == 0;
+#pragma unroll
+  for (int u = 0; u < QUADS; ++u) {
+    const size_t i = first + u * 1024;
+    if (i > total4 || (i == total4 && rest == 0)) break;
+    long long q[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) q[e] = quantize_one(v[u][e], scalars);
+    if (packed && i < total4) {
+      unsigned word = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) word |= ((unsigned)q[e] & 0xffu) << (8 * e);
+      static_cast<unsigned*>(out)[i] = word;
+    } else {
+#pragma unroll
+      for (unsigned e = 0; e < 4; ++e)
+        if (i < total4 || e < rest) store_typed(out, outType, i * 4 + e, q[e]);
+    }
+  }
+}
+
 unsigned grid_for(size_t total, unsigned perThread = 1) {
   size_t blocks = (total + 256ull * perThread - 1) / (256ull * perThread);
   if (blocks > 256u * 32u) blocks = 256u * 32u;
@@ -618,6 +753,20 @@ unsigned stream_grid(size_t total4) {
 // The word on which a stream's range reductions count their workgroups; calls that get none reduce the partial results in a
 // launch of its own.
 StreamSlots gArrivalSlots(kArrivalSlots);
+
+std::atomic<unsigned> gTogetherCalls{1};
+
+// as many workgroups as there may be: a thread's loads are all on their way at once, and the words are read side by side
+void launch_together(hipStream_t s, const float* in, uint64_t total, void* out, int outType, float* mn, float* mx, unsigned slot) {
+  const unsigned call = gTogetherCalls.fetch_add(1, std::memory_order_relaxed), pieces = (unsigned)((total + 4095) / 4096);
+  auto launch = [&](auto kernel, unsigned quads) {
+    hipLaunchKernelGGL(kernel, dim3((pieces + quads - 1) / quads), dim3(1024), 0, s, in, (size_t)total, out, outType, mn, mx, slot, call);
+  };
+  if (pieces <= kTogetherWorkgroups) launch(quantize_together_kernel<1>, 1);
+  else if (pieces <= 2 * kTogetherWorkgroups) launch(quantize_together_kernel<2>, 2);
+  else if (pieces <= 4 * kTogetherWorkgroups) launch(quantize_together_kernel<4>, 4);
+  else launch(quantize_together_kernel<8>, 8);
+}
 
 bool valid_type(int t) { return t >= TFCC_ROCM_S8 && t <= TFCC_ROCM_U32; }
 
@@ -776,6 +925,14 @@ int tfcc_rocm_quantize_minmax(void* stream, const float* in, uint64_t total, voi
   // every element where it was read.
   const uintptr_t inAt = (uintptr_t)in, outAt = (uintptr_t)out;
   const bool apart = inAt + 4 * total <= outAt || outAt + total * (int_range(out_type).bits / 8) <= inAt;
+  int dev = 0;
+  unsigned slot = 0;
+  TFCC_HIP_CHECK(hipGetDevice(&dev));
+  const bool withSlot = total > kWholeBest && gArrivalSlots.of(dev, s, &slot);
+  if (apart && withSlot && total <= kTogetherLimit && slot < kTogetherSlots) {
+    launch_together(s, in, total, out, out_type, min_v, max_v, slot);
+    return check_launch("quantize");
+  }
   if (apart && total <= kWholeLimit) {
     hipLaunchKernelGGL(quantize_whole_kernel, dim3((unsigned)((total + 4095) / 4096)), dim3(1024), 0, s, in, (unsigned)total,
                        out, out_type, min_v, max_v);
@@ -783,13 +940,10 @@ int tfcc_rocm_quantize_minmax(void* stream, const float* in, uint64_t total, voi
   }
   unsigned* mnWord = reinterpret_cast<unsigned*>(min_v);
   unsigned* mxWord = reinterpret_cast<unsigned*>(max_v);
-  int dev = 0;
-  unsigned slot = 0;
-  TFCC_HIP_CHECK(hipGetDevice(&dev));
   if (apart && (uintptr_t)in % 16 == 0 && (uintptr_t)out % 4 == 0) {
     // partial results, eight bytes per workgroup, rest in the output buffer until the quantize pass overwrites it
     float* partials = static_cast<float*>(out);
-    if (gArrivalSlots.of(dev, s, &slot)) {
+    if (withSlot) {
       // one workgroup per CU at most: every arrival costs an atomic on one word and a write-back (192 workgroups of 256
       // threads for 786432 elements: 6 us, 48 of 1024: 5.6)
       const unsigned blocks = total >= 256u * 16384u ? 256u : (unsigned)((total + 16383) / 16384);
