@@ -85,6 +85,16 @@ def test_sizes_where_the_transfers_change(mf, rt, dev, shapes):
     round_trip(mf, rt, shapes, False)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("shapes", [
+    [(1023,)], [(1024,), (1025,)],                                     # one workgroup's 4 KB
+    [((384 << 10) // 4,)], [((384 << 10) // 4 + 1,)],                  # up to here in, and a float more
+    [((1536 << 10) // 4,)], [((1536 << 10) // 4 - 8,), (9,)],          # and out, in one piece and in two
+])
+def test_sizes_where_a_workgroup_takes_more(mf, rt, dev, shapes):
+    round_trip(mf, rt, shapes, False)
+
+
 def test_any_mapping_is_taken(mf, rt):
     model = copies(mf, rt, [(mf.FLOAT, (2,)), (mf.INT32, (3,))], True)
     want = {"x0": np.array([1, 2], np.float32), "x1": np.array([3, 4, 5], np.int32)}
