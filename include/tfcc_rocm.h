@@ -97,6 +97,7 @@ typedef struct tfcc_rocm_copy_piece {
   void* dst;
   uint64_t bytes;
 } tfcc_rocm_copy_piece;
+int tfcc_rocm_copy_pieces_from_pinned(void* stream, const tfcc_rocm_copy_piece* pieces, unsigned count);
 int tfcc_rocm_copy_to_pinned(void* stream, const tfcc_rocm_copy_piece* pieces, unsigned count,
                              unsigned* arrivals_device, unsigned* flag_pinned, unsigned epoch);
 /* fill `count` elements of `elem_size` (1, 2, 4 or 8) bytes with the bit pattern `value` */

@@ -88,7 +88,8 @@ def test_sizes_where_the_transfers_change(mf, rt, dev, shapes):
 @pytest.mark.gpu
 @pytest.mark.parametrize("shapes", [
     [(1023,)], [(1024,), (1025,)],                                     # one workgroup's 4 KB
-    [((384 << 10) // 4,)], [((384 << 10) // 4 + 1,)],                  # up to here in, and a float more
+    [((384 << 10) // 4,)], [((384 << 10) // 4 + 1,)],                  # up to here in, which is the first chunk, and a float more
+    [(77,), ((384 << 10) // 4,), ((768 << 10) // 4 + 3,), (5,)],       # chunks that end inside an input and hold the next
     [((1536 << 10) // 4,)], [((1536 << 10) // 4 - 8,), (9,)],          # and out, in one piece and in two
 ])
 def test_sizes_where_a_workgroup_takes_more(mf, rt, dev, shapes):

@@ -99,6 +99,7 @@ SYMBOLS = {
     "tfcc_rocm_host_malloc": (_I, [C.POINTER(C.c_void_p), C.c_size_t]),
     "tfcc_rocm_host_free": (_I, [_VP]),
     "tfcc_rocm_copy_from_pinned": (_I, [_VP, _VP, _VP, C.c_size_t]),
+    "tfcc_rocm_copy_pieces_from_pinned": (_I, [_VP, _VP, _U]),
     "tfcc_rocm_copy_to_pinned": (_I, [_VP, _VP, _U, _VP, _VP, _U]),
     "tfcc_rocm_fill_async": (_I, [_VP, _VP, _U64, _I, C.c_size_t]),
     "tfcc_rocm_sgemm_strided_batched": (_I, [_VP, _VP, _U64, _VP, _U64, _VP, _VP, _U64, _U, _U, _U, _U]),

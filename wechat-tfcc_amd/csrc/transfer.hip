@@ -58,9 +58,16 @@ __device__ __forceinline__ void copy_block(const char* __restrict__ src, char* _
   }
 }
 
+template <int QUADS, bool TO_HOST>
+__device__ __forceinline__ void copy_pieces(const Pieces& p) {
+  unsigned i = 0;
+  while (i + 1 < p.count && blockIdx.x >= p.firstBlock[i + 1]) ++i;
+  copy_block<QUADS, TO_HOST>(p.src[i], p.dst[i], p.bytes[i], blockIdx.x - p.firstBlock[i]);
+}
+
 template <int QUADS>
-__global__ __launch_bounds__(256) void copy_kernel(const char* src, char* dst, unsigned long long bytes) {
-  copy_block<QUADS, false>(src, dst, bytes, blockIdx.x);
+__global__ __launch_bounds__(256) void scatter_kernel(Pieces p) {
+  copy_pieces<QUADS, false>(p);
 }
 
 // Bound by PCIe (57 GB/s): 3 MB in 60 us.  The last workgroup to arrive raises *flag to `epoch`, which the host polls:
@@ -69,9 +76,7 @@ __global__ __launch_bounds__(256) void copy_kernel(const char* src, char* dst, u
 // workgroup, which writes back what the kernels before have left in the L2s, 3 MB 72 us, 87 KB 6.9 instead of 4.1).
 template <int QUADS>
 __global__ __launch_bounds__(256) void gather_kernel(Pieces p, unsigned* arrivals, unsigned* flag, unsigned epoch) {
-  unsigned i = 0;
-  while (i + 1 < p.count && blockIdx.x >= p.firstBlock[i + 1]) ++i;
-  copy_block<QUADS, true>(p.src[i], p.dst[i], p.bytes[i], blockIdx.x - p.firstBlock[i]);
+  copy_pieces<QUADS, true>(p);
   if (flag == nullptr) return;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wavefront's own stores are in host memory before the barrier lets it go
   __syncthreads();
@@ -82,6 +87,32 @@ __global__ __launch_bounds__(256) void gather_kernel(Pieces p, unsigned* arrival
       __hip_atomic_store(flag, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
+}
+
+// launch(pieces, workgroups, whether they take 4 KB each, whether it is the last one), kMaxPieces at a time
+template <class Launch>
+int launch_pieces(const char* what, const tfcc_rocm_copy_piece* pieces, unsigned count, size_t manyBlocks, Launch&& launch) {
+  for (unsigned i = 0; i < count; ++i)
+    TFCC_REQUIRE(pieces[i].src && pieces[i].dst && pieces[i].bytes > 0 && pieces[i].bytes <= (1ull << 40), "%s: bad piece %u", what, i);
+  for (unsigned at = 0; at < count; at += kMaxPieces) {
+    Pieces p;
+    p.count = count - at < kMaxPieces ? count - at : kMaxPieces;
+    unsigned long long blocks = 0, bytes = 0;
+    for (unsigned i = 0; i < p.count; ++i) bytes += pieces[at + i].bytes;
+    const bool many = bytes <= manyBlocks;
+    const unsigned each = block_bytes(many ? 1 : 4);
+    for (unsigned i = 0; i < p.count; ++i) {
+      p.src[i] = static_cast<const char*>(pieces[at + i].src);
+      p.dst[i] = static_cast<char*>(pieces[at + i].dst);
+      p.bytes[i] = pieces[at + i].bytes;
+      p.firstBlock[i] = (unsigned)blocks;
+      blocks += (pieces[at + i].bytes + each - 1) / each;
+      TFCC_REQUIRE(blocks <= 0x7fffffffu, "%s: too many bytes", what);
+    }
+    launch(p, (unsigned)blocks, many, at + kMaxPieces >= count);
+    if (int e = check_launch(what)) return e;
+  }
+  return TFCC_ROCM_OK;
 }
 
 }  // namespace
@@ -107,42 +138,25 @@ int tfcc_rocm_host_free(void* ptr) {
 int tfcc_rocm_copy_from_pinned(void* stream, void* dst_device, const void* src_pinned, size_t bytes) {
   if (bytes == 0) return TFCC_ROCM_OK;
   TFCC_REQUIRE(dst_device && src_pinned, "copy_from_pinned: null argument");
-  const bool many = bytes <= kManyBlocksIn;
-  const size_t each = block_bytes(many ? 1 : 4), blocks = (bytes + each - 1) / each;
-  TFCC_REQUIRE(blocks <= 0x7fffffffu, "copy_from_pinned: %zu bytes", bytes);
-  hipLaunchKernelGGL(many ? copy_kernel<1> : copy_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream),
-                     static_cast<const char*>(src_pinned), static_cast<char*>(dst_device), (unsigned long long)bytes);
-  return check_launch("copy_from_pinned");
+  const tfcc_rocm_copy_piece piece = {src_pinned, dst_device, bytes};
+  return tfcc_rocm_copy_pieces_from_pinned(stream, &piece, 1);
+}
+
+int tfcc_rocm_copy_pieces_from_pinned(void* stream, const tfcc_rocm_copy_piece* pieces, unsigned count) {
+  TFCC_REQUIRE(pieces && count > 0, "copy_from_pinned: null argument");
+  return launch_pieces("copy_from_pinned", pieces, count, kManyBlocksIn, [&](const Pieces& p, unsigned blocks, bool many, bool) {
+    hipLaunchKernelGGL(many ? scatter_kernel<1> : scatter_kernel<4>, dim3(blocks), dim3(256), 0, as_stream(stream), p);
+  });
 }
 
 int tfcc_rocm_copy_to_pinned(void* stream, const tfcc_rocm_copy_piece* pieces, unsigned count, unsigned* arrivals_device,
                              unsigned* flag_pinned, unsigned epoch) {
   TFCC_REQUIRE(pieces && count > 0 && arrivals_device && flag_pinned, "copy_to_pinned: null argument");
-  for (unsigned i = 0; i < count; ++i)
-    TFCC_REQUIRE(pieces[i].src && pieces[i].dst && pieces[i].bytes > 0 && pieces[i].bytes <= (1ull << 40),
-                 "copy_to_pinned: bad piece %u", i);
-  for (unsigned at = 0; at < count; at += kMaxPieces) {
-    Pieces p;
-    p.count = count - at < kMaxPieces ? count - at : kMaxPieces;
-    unsigned long long blocks = 0, bytes = 0;
-    for (unsigned i = 0; i < p.count; ++i) bytes += pieces[at + i].bytes;
-    const bool many = bytes <= kManyBlocksOut;
-    const unsigned each = block_bytes(many ? 1 : 4);
-    for (unsigned i = 0; i < p.count; ++i) {
-      p.src[i] = static_cast<const char*>(pieces[at + i].src);
-      p.dst[i] = static_cast<char*>(pieces[at + i].dst);
-      p.bytes[i] = pieces[at + i].bytes;
-      p.firstBlock[i] = (unsigned)blocks;
-      blocks += (pieces[at + i].bytes + each - 1) / each;
-      TFCC_REQUIRE(blocks <= 0x7fffffffu, "copy_to_pinned: too many bytes");
-    }
-    // the stream runs the launches in order: only the last one tells the host
-    const bool last = at + kMaxPieces >= count;
-    hipLaunchKernelGGL(many ? gather_kernel<1> : gather_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), p, arrivals_device,
+  // the stream runs the launches in order: only the last one tells the host
+  return launch_pieces("copy_to_pinned", pieces, count, kManyBlocksOut, [&](const Pieces& p, unsigned blocks, bool many, bool last) {
+    hipLaunchKernelGGL(many ? gather_kernel<1> : gather_kernel<4>, dim3(blocks), dim3(256), 0, as_stream(stream), p, arrivals_device,
                        last ? flag_pinned : nullptr, epoch);
-    if (int e = check_launch("copy_to_pinned")) return e;
-  }
-  return TFCC_ROCM_OK;
+  });
 }
 
 }  // extern "C"

@@ -1241,28 +1241,48 @@ bool ROCMSession::reserveStaging(size_t bytes) {
 
 // 3 MB: 106 us in one copy from pageable memory.  Here the GPU fetches one chunk while the host puts the next one down,
 // and nothing waits: the kernels that read the data are behind it on the stream.  The first chunk is short so that the
-// GPU starts early, the later ones long because each costs a launch.
-void ROCMSession::upload(void* device, const void* host, size_t bytes) {
+// GPU starts early, the later ones long because each costs a launch, but no longer than the GPU has work for meanwhile;
+// small inputs share a launch.  An encoder layer of 8 x 128 x 768 served, us, by the first and the longest chunk in KB: 256 and
+// 1024 308, 256 and 512 297, 256 and 256 309, 384 and 768 294.
+void ROCMSession::upload(const std::vector<HostWrite>& writes) {
   if (_recording) throw RuntimeError("upload: not possible while the session's stream records a graph");
-  if (bytes == 0) return;
-  if (!reserveStaging(_stagingUsed + bytes)) {
-    check(tfcc_rocm_memcpy_h2d(_stream, device, host, bytes));
+  size_t total = 0;
+  for (const HostWrite& w : writes) total += (w.bytes + 63) / 64 * 64;
+  if (total == 0) return;
+  if (!reserveStaging(_stagingUsed + total)) {
+    for (const HostWrite& w : writes)
+      if (w.bytes > 0) check(tfcc_rocm_memcpy_h2d(_stream, w.device, w.host, w.bytes));
     return;
   }
-  const char* src = static_cast<const char*>(host);
-  char* dst = static_cast<char*>(device);
-  size_t chunk = size_t(256) << 10;
-  while (bytes > 0) {
-    if (_stagingUsed >= _stagingSize) sync();  // every byte of the block is in flight: wait for the stream once
-    const size_t n = std::min(std::min(bytes, chunk), _stagingSize - _stagingUsed);
-    std::memcpy(_staging + _stagingUsed, src, n);
-    check(tfcc_rocm_copy_from_pinned(_stream, dst, _staging + _stagingUsed, n));
-    _stagingUsed += (n + 63) / 64 * 64;
-    src += n;
-    dst += n;
-    bytes -= n;
-    chunk = std::min(chunk * 2, size_t(1) << 20);
+  std::vector<tfcc_rocm_copy_piece> pieces;
+  size_t chunk = size_t(384) << 10, gathered = 0;
+  auto launch = [&] {
+    if (pieces.empty()) return;
+    check(tfcc_rocm_copy_pieces_from_pinned(_stream, pieces.data(), static_cast<unsigned>(pieces.size())));
+    pieces.clear();
+    gathered = 0;
+    chunk = std::min(chunk * 2, size_t(768) << 10);
+  };
+  for (const HostWrite& w : writes) {
+    const char* src = static_cast<const char*>(w.host);
+    char* dst = static_cast<char*>(w.device);
+    for (size_t left = w.bytes; left > 0;) {
+      if (_stagingUsed >= _stagingSize) {  // every byte of the block is in flight: wait for the stream once
+        launch();
+        sync();
+      }
+      const size_t n = std::min(std::min(left, chunk - gathered), _stagingSize - _stagingUsed);
+      std::memcpy(_staging + _stagingUsed, src, n);
+      pieces.push_back({_staging + _stagingUsed, dst, n});
+      _stagingUsed += (n + 63) / 64 * 64;
+      gathered += n;
+      src += n;
+      dst += n;
+      left -= n;
+      if (gathered >= chunk) launch();
+    }
   }
+  launch();
 }
 
 // Polls the word the GPU raises behind the last byte; work that takes longer than a few milliseconds is waited for in

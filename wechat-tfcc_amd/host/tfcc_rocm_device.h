@@ -103,8 +103,14 @@ class ROCMSession : public Session {
     size_t bytes;
     bool pinned;  // the host address lies in a block of PinnedPool
   };
-  // device <- host memory that may be changed as soon as the call returns; the copy itself is ordered on the stream
-  void upload(void* device, const void* host, size_t bytes);
+  struct HostWrite {
+    void* device;
+    const void* host;
+    size_t bytes;
+  };
+  // device <- host memory that may be changed as soon as the call returns; the copies themselves are ordered on the stream
+  void upload(const std::vector<HostWrite>& writes);
+  void upload(void* device, const void* host, size_t bytes) { upload(std::vector<HostWrite>{{device, host, bytes}}); }
   // host <- device, complete when the call returns
   void download(const std::vector<HostRead>& reads);
 

@@ -670,8 +670,14 @@ Graph& Model::getGraph(const std::string& name) {
 }
 
 namespace {
+// A tensor that is on its way to the device, to be handed to the graph when the copies of all of them are on the stream.
+struct PendingInputs {
+  std::vector<ROCMSession::HostWrite> writes;
+  std::vector<std::function<void(Graph&)>> hand;
+};
+
 template <class T>
-void add_input(Graph& graph, const proto::InputView& item, ROCMSession* rocm) {
+void add_input(Graph& graph, const proto::InputView& item, ROCMSession* rocm, PendingInputs& pending) {
   Shape shape(item.shape);
   if (item.bytes != static_cast<size_t>(shape.area()) * sizeof(T)) throw RuntimeError("Invalid data size");
   const SymbolInfo& info = graph.getSymbolManager().getSymbolInfo(item.name);
@@ -683,10 +689,13 @@ void add_input(Graph& graph, const proto::InputView& item, ROCMSession* rocm) {
     return;
   }
   Variable<T> v(shape);
-  if (v.size() > 0) {
-    if (rocm) rocm->upload(v.data(), item.data, item.bytes);
-    else data::set(v, reinterpret_cast<const T*>(item.data));
+  if (rocm) {
+    if (v.size() > 0) pending.writes.push_back({v.data(), item.data, item.bytes});
+    auto kept = std::make_shared<Variable<T>>(std::move(v));
+    pending.hand.push_back([kept, &item](Graph& g) { g.setInput(item.name, std::move(*kept)); });
+    return;
   }
+  if (v.size() > 0) data::set(v, reinterpret_cast<const T*>(item.data));
   graph.setInput(item.name, std::move(v));
 }
 
@@ -719,15 +728,20 @@ void get_output(Graph& graph, RunResult::Output& out, bool rocm, std::vector<ROC
 RunResult Model::run(const std::vector<proto::InputView>& inputs) {
   Graph& graph = getEntranceGraph();
   auto* rocm = dynamic_cast<ROCMSession*>(Session::getThreadDefault());
+  PendingInputs pending;
   for (const proto::InputView& item : inputs) {
     switch (item.dtype) {
 #define TFCC_RUNTIME_INPUT(T, E) \
-  case E: add_input<T>(graph, item, rocm); break;
+  case E: add_input<T>(graph, item, rocm, pending); break;
       TFCC_RUNTIME_FOR_ALL_TYPES(TFCC_RUNTIME_INPUT)
 #undef TFCC_RUNTIME_INPUT
-      case BOOL: add_input<uint8_t>(graph, item, rocm); break;
+      case BOOL: add_input<uint8_t>(graph, item, rocm, pending); break;
       default: throw RuntimeError("Invalid input dtype");
     }
+  }
+  if (rocm) {
+    rocm->upload(pending.writes);
+    for (const auto& hand : pending.hand) hand(graph);
   }
   graph.process();
   RunResult result;
