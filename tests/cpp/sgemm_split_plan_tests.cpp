@@ -36,6 +36,13 @@ int main(int argc, char** argv) {
   EXPECT(kernel_of(4096, 4096, 4096, 4096, (1u << 29) / (4096 + 256) + 1, 4096, false, 1) == kNone);
   EXPECT(kernel_of(4096, 4096, 4096, 4096, (1u << 29) / (4096 + 256) + 1, 4096, true, 1) == kNone);
   EXPECT(kernel_of(4096, 4096, 4096, 4096, 4096, 1u << 21, false, 1) == kNone);
+  // two K groups while a CU has one tile at most, but not for many tiles of a short K
+  EXPECT(k_groups_of_128(1, 128) == 2 && k_groups_of_128(128, 128) == 2 && k_groups_of_128(129, 319) == 1 && k_groups_of_128(129, 320) == 2);
+  EXPECT(k_groups_of_128(256, 320) == 2 && k_groups_of_128(257, 320) == 1 && k_groups_of_128(257, 8192) == 1);
+  // the estimate by tiles: none where the fp32 ops have 128 x 128 tiles, otherwise no less for a k more
+  EXPECT(tfcc_rocm::sgemm_tiles::microseconds(4096, 4096, 4096, 1) == 0 && tfcc_rocm::sgemm_tiles::microseconds(425, 6974, 628, 1) == 0);
+  auto time = [](unsigned k) { return tfcc_rocm::sgemm_tiles::microseconds(1000, 1000, k, 1); };
+  for (unsigned k = 512; k < 4096; ++k) EXPECT(time(k) > 0 && time(k + 1) >= time(k));
   // B given transposed is summed as B as stored, so the same kernel has to take it
   for (unsigned m = 48; m <= 6000; m = m * 5 / 4 + 1)
     for (unsigned n = 48; n <= 9000; n = n * 5 / 4 + 1)

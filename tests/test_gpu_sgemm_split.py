@@ -66,6 +66,30 @@ def test_against_float64_and_the_transposed_form(pkg, dev, kernel, m, n, k):
     assert torch.equal(c[:, :n], out) and bool(torch.isnan(c[:, n:]).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(2048, 2048, 320), (2047, 2041, 321), (1921, 2048, 335), (2048, 1930, 336), (2033, 2048, 337), (2048, 2048, 351),
+                                   (1030, 3000, 400), (1100, 2100, 705), (904, 3244, 1544)])
+def test_two_k_groups_on_128_tiles(pkg, dev, m, n, k):
+    """One tile to a CU at most: K that ends in either group's slab, with rows and columns of a tile missing, the epilogue
+    in the share of the rows that a group finishes, a value that the split cannot represent in each share"""
+    import torch
+    assert kernel_of(m, n, k) == K128 and -(-m // 128) * -(-n // 128) <= 256
+    gen = torch.Generator(device=dev).manual_seed(m + n + k)
+    a, b = torch.randn(m, k, device=dev, generator=gen), torch.randn(k, n, device=dev, generator=gen)
+    bias = torch.randn(n, device=dev, generator=gen)
+    want = a.double() @ b.double()
+    out = pkg.blas_matmul(a, b)
+    assert rel(out, want) <= bound(k)
+    assert torch.equal(pkg.blas_matmul(a, b, bias), out + bias)
+    c = torch.full((m, n + 3), float("nan"), device=dev)
+    pkg.sgemm_general(a, b.t().contiguous(), c, m, n, k, k, k, n + 3, trans_b=True)
+    assert torch.equal(c[:, :n], out) and bool(torch.isnan(c[:, n:]).all())
+    a[5, 1], a[m - 1, k - 1] = float("inf"), float("nan")
+    got = pkg.blas_matmul(a, b)
+    bad = torch.zeros(m, dtype=torch.bool, device=dev)
+    bad[5] = bad[m - 1] = True
+    assert torch.equal(got[~bad], out[~bad]) and not bool(torch.isfinite(got[bad]).any())
+
+
 @pytest.mark.parametrize("kernel,m,n,k", ONE_OF_EACH)
 def test_every_pair_of_pieces(pkg, dev, kernel, m, n, k):
     """One product to a result, of operands that have all three parts on one side, or the second on both: exact, if no term

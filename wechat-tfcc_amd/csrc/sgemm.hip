@@ -16,10 +16,12 @@
 #include "common.hpp"
 #include "sgemm_params.hpp"
 #include "sgemm_split_plan.hpp"
+#include "sgemm_tiles.hpp"
 
 namespace tfcc_rocm {
 
 using sgemm_detail::SgemmParams;
+using namespace sgemm_tiles;
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -427,42 +429,9 @@ int launch(hipStream_t stream, SgemmParams p) {
   return check_launch("sgemm");
 }
 
-// The tile table of the kernels that copy K slabs straight into LDS, ordered by falling tile area.
-const struct { int config; unsigned bm, bn, waves; } kTiles[] = {{0, 64, 64, 4}, {1, 32, 96, 3}, {2, 32, 64, 2}, {3, 32, 32, 1}};
-
-// Tile and number of K groups for m x n x k with K a multiple of 32: the tile that covers the 256 CUs in the fewest
-// tile-area rounds, the larger one on a tie (less operand traffic); as few K groups as give every CU eight
-// wavefronts, each group keeping at least four slabs.
-void choose_dma_tiles(unsigned m, unsigned n, unsigned k, unsigned fillBatch, int& best, unsigned long long& bestTiles,
-                      int& ksplit) {
-  best = 0;
-  unsigned long long bestCost = ~0ull;
-  bestTiles = 0;
-  for (int c = 0; c < 4; ++c) {
-    const unsigned long long tiles =
-        (unsigned long long)((m + kTiles[c].bm - 1) / kTiles[c].bm) * ((n + kTiles[c].bn - 1) / kTiles[c].bn) * fillBatch;
-    const unsigned long long cost = ((tiles + 255) / 256) * (kTiles[c].bm * kTiles[c].bn);
-    if (cost < bestCost) {
-      best = c;
-      bestCost = cost;
-      bestTiles = tiles;
-    }
-  }
-  ksplit = 1;
-  while (ksplit < 4 && bestTiles * kTiles[best].waves * ksplit < 256ull * 8 && k >= 128u * (ksplit * 2)) ksplit *= 2;
-}
-
 // The number of K groups the kernels for B as stored [k, n] would sum this product with (the sums of an element
 // are defined by it, not by the tile shape): B given transposed must use the same, so that transposing B first
 // and multiplying give the same bits as multiplying the transposed view.
-// 128 x 128 tiles: once there are enough of them to fill the 256 CUs twice over, and only when they are mostly
-// result (a batch of 768 products of 64 x 64 x 64 counts 768 such tiles, each three quarters empty: 23 us in them
-// against 11 in 64 x 64 tiles).
-bool takes_128_tiles(unsigned m, unsigned n, unsigned fillBatch) {
-  const unsigned long long big = (unsigned long long)((m + 127) / 128) * ((n + 127) / 128) * fillBatch;
-  return big >= 512 && (unsigned long long)m * n * fillBatch * 100 >= big * (128 * 128) * 75;
-}
-
 int k_groups_of_plain_product(unsigned m, unsigned n, unsigned k, unsigned fillBatch) {
   if (takes_128_tiles(m, n, fillBatch)) return 1;
   int best, ksplit;
@@ -533,19 +502,9 @@ int dispatch(hipStream_t s, const SgemmParams& p, bool vec, bool small, bool tb,
   // sgemm_dma.hip are as fast or faster and keep the product ...
   if (ksplit == 2 && kTiles[best].config == 0) return sgemm_detail::sgemm_wave96_launch(s, p, 2, 2, 2);
   if (ksplit == 2 && kTiles[best].config == 3) return sgemm_detail::sgemm_wave96_launch(s, p, 2, 1, 1);
-  // ... and without K groups the products whose 128 x 96 tiles fill at least 70 % of the CUs in each of their
-  // rounds (or 128 x 128 tiles 85 %), K >= 512: four wavefronts of 32 x 96 (32 x 128) share each copy of B
-  // (1024 x 3072 x 768 with GELU: 39.3 against 42.4 us in 64 x 64 tiles, 1536^3: 69 against 80; in 128 x 128 tiles
-  // 2048^3, now on the bf16 matrix cores, 120 against 136; below those fills, or with a short K, the table's win).  The
-  // sums are the same in every case: the K groups of the table, ascending k inside a group.
-  if (ksplit == 1 && k >= 512) {
-    const unsigned long long wide = (unsigned long long)((m + 127) / 128) * ((n + 95) / 96) * fillBatch;
-    const unsigned long long wide4 = (unsigned long long)((m + 127) / 128) * ((n + 127) / 128) * fillBatch;
-    const bool ok3 = wide * 100 >= 70 * 256 * ((wide + 255) / 256), ok4 = wide4 * 100 >= 85 * 256 * ((wide4 + 255) / 256);
-    const unsigned long long cost3 = ((wide + 255) / 256) * 96, cost4 = ((wide4 + 255) / 256) * 128;
-    if (ok4 && (!ok3 || cost4 < cost3)) return sgemm_detail::sgemm_wave96_launch(s, p, 1, 4);
-    if (ok3) return sgemm_detail::sgemm_wave96_launch(s, p, 1);
-  }
+  // ... and without K groups the products that fill the CUs with workgroups of four wavefronts.  The sums are the same in
+  // every case: the K groups of the table, ascending k inside a group.
+  if (const int blocks = shared_blocks(m, n, k, fillBatch, ksplit)) return sgemm_detail::sgemm_wave96_launch(s, p, 1, blocks);
   // What is left runs on the kernels of sgemm_dma.hip.  Several products in one launch (p.batch counts them;
   // fillBatch = 1 chose the configuration of a single one so that each is summed exactly as on its own): when
   // they fill the chip without the K groups, one group per tile plays all of them; and when 128 x 96 tiles over

@@ -317,7 +317,11 @@ __device__ __forceinline__ bool split_failed(const SgemmParams& p, const Tile& t
 // matrix ops' worth instead of three: 669 us.  256 x 256 tiles, two values: 600, but there are registers for one
 // accumulator only; with a block's six terms summed from zero, smallest first, and then added to it 635, and one
 // product in a row still 3.5e-8.  A wavefront for each SIMD on 128 x 128, more slabs on their way, two K groups
-// of such tiles: all slower.)
+// of such tiles: all slower.  What is left of a value beside its piece as one dot product of pieces with -1, two instructions
+// fewer for each value: the dot products run in the matrix cores, 675 against 634.)
+//
+// KG = 2: two such groups of wavefronts have a tile, every other slab each, and meet in LDS; for products with one tile to a CU
+// at most, where a wavefront for each SIMD has nothing beside it while it waits (sgemm_split_plan.hpp).
 template <int BM, int BN>
 struct SharedLayout {
   // [piece][eight k][row or column] of 16 bytes; 64 bytes between the halves of k put a thread pair's writes on
@@ -326,8 +330,8 @@ struct SharedLayout {
                        STAGE = 3 * (PIECE_A + PIECE_B);
 };
 
-template <int MI, int NI, int WGM, int WGN, bool TRANSB>
-__global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const SgemmParams p) {
+template <int MI, int NI, int WGM, int WGN, int KG, bool TRANSB>
+__global__ __launch_bounds__(64 * WGM * WGN * KG, 2) void sgemm_split_kernel(const SgemmParams p) {
   constexpr int BM = 32 * MI * WGM, BN = 32 * NI * WGN, BK = 16, T = 64 * WGM * WGN;
   constexpr int VA = BM * BK / T, VB = BN * BK / T, OPS_A = 6 * VA, OPS = OPS_A + 6 * VB;  // values per thread
   static_assert((VA == 4 || VA == 8) && VB == 8, "a thread has four or eight values of A and eight of B");
@@ -336,9 +340,11 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
 
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ Findings<BM, BN> found;
-  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int grp = KG == 1 ? 0 : wave / (WGM * WGN), wv = wave - grp * WGM * WGN;
   const int wm = wv / WGN, wn = wv - wm * WGN;  // wave-uniform
-  const int tid = threadIdx.x, lane = tid & 63, lrow = lane & 31, g = lane >> 5;
+  const int tid = KG == 1 ? threadIdx.x : threadIdx.x % T, lane = tid & 63, lrow = lane & 31, g = lane >> 5;
+  unsigned char* const gsm = smem + grp * 3 * STAGE;
   const Tile tile = tile_of<BM, BN, TRANSB>(p);
   if (!tile.exists) return;
   const unsigned m0 = tile.m0, n0 = tile.n0, M = p.M, N = p.N, K = p.K, lda = p.lda, ldb = p.ldb;
@@ -351,7 +357,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
   const int brow = TRANSB ? tid >> 1 : tid & (BN - 1), bhalf = TRANSB ? tid & 1 : tid / BN;
   const unsigned aOff = m0 + arow < M ? ((m0 + arow) * lda + ak) * 4u : kOutside;
   const unsigned bOff = n0 + brow >= N ? kOutside : TRANSB ? ((n0 + brow) * ldb + 8 * bhalf) * 4u : (8 * bhalf * ldb + n0 + brow) * 4u;
-  const unsigned slabs = (K + BK - 1) / BK;
+  const unsigned slabs = (K + KG * BK - 1) / (KG * BK);  // of every K group
+  auto firstK = [&](unsigned s) { return (s * KG + grp) * (unsigned)BK; };
   struct Raw { float a[VA], b[VB]; };
   // the operand from its k `k0` on, `step` bytes to a k: 32-bit scalar arithmetic (a 64-bit comparison would be made on the
   // vector unit, and the descriptor then read back lane by lane)
@@ -362,7 +369,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
   // one of the loads of slab s, A's first
   constexpr int LOADS_A = VA / 4, LOADS = LOADS_A + (TRANSB ? 2 : 8);
   auto load = [&](Raw& r, unsigned s, int which) __attribute__((always_inline)) {
-    const unsigned k0 = s * BK;
+    const unsigned k0 = firstK(s);
     auto quad = [&](float* x, __amdgpu_buffer_rsrc_t d, unsigned off) __attribute__((always_inline)) {
       const v4f v = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(d, off, 0, 0));
 #pragma unroll
@@ -378,15 +385,15 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
                                                                                bOff + ofB * ldb * 4u, 0, 0));
   };
   auto mask = [&](Raw& r, unsigned s) {  // the slab in which K ends, or one behind it
-    const int left = (int)K - (int)(s * BK);
+    const int left = (int)K - (int)firstK(s);
 #pragma unroll
     for (int e = 0; e < VA; ++e) r.a[e] = ak + e < left ? r.a[e] : 0.f;
 #pragma unroll
     for (int e = 0; e < VB; ++e) r.b[e] = 8 * bhalf + e < left ? r.b[e] : 0.f;
   };
   float largestA = 0.f, largestB = 0.f;
-  unsigned char* const aTo = smem + ak / 8 * L::HALF_A + arow * 16 + ak % 8 * 2;
-  unsigned char* const bTo = smem + 3 * L::PIECE_A + bhalf * L::HALF_B + brow * 16;
+  unsigned char* const aTo = gsm + ak / 8 * L::HALF_A + arow * 16 + ak % 8 * 2;
+  unsigned char* const bTo = gsm + 3 * L::PIECE_A + bhalf * L::HALF_B + brow * 16;
 
   v16f main[MI][NI], rest[MI][NI];
 #pragma unroll
@@ -394,8 +401,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
 #pragma unroll
     for (int j = 0; j < NI; ++j) main[i][j] = rest[i][j] = v16f{};
 
-  const unsigned char* const aFrom = smem + g * L::HALF_A + (wm * 32 * MI + lrow) * 16;
-  const unsigned char* const bFrom = smem + 3 * L::PIECE_A + g * L::HALF_B + (wn * 32 * NI + lrow) * 16;
+  const unsigned char* const aFrom = gsm + g * L::HALF_A + (wm * 32 * MI + lrow) * 16;
+  const unsigned char* const bFrom = gsm + 3 * L::PIECE_A + g * L::HALF_B + (wn * 32 * NI + lrow) * 16;
   Raw raw;
   Splitting<VA> ofA;
   Splitting<VB> ofB;
@@ -440,7 +447,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
   }
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    if ((unsigned)(s + 1) * BK > K) mask(ahead[s], s);
+    if (firstK(s) + BK > K) mask(ahead[s], s);
     each<0, OPS>([&](auto o) __attribute__((always_inline)) { splitOp(ahead[s], s * STAGE, o); });
   }
   __syncthreads();
@@ -462,7 +469,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
   constexpr int PT = MI * NI, TOTAL = 6 * PT, SPREAD = 5 * PT;  // SPREAD: matrix ops that the splitting is dealt out behind
   unsigned st0 = 0, st1 = STAGE, st2 = 2 * STAGE;               // stages of slabs s, s + 1, s + 2
   for (unsigned s = 0; s < slabs; ++s) {
-    if ((s + 3) * BK > K) mask(raw, s + 2);
+    if (firstK(s + 2) + BK > K) mask(raw, s + 2);
     each<0, TOTAL>([&](auto mc) __attribute__((always_inline)) {
       constexpr int m = mc, t = m / PT, i = m % PT / NI, j = m % NI;
       v16f& sum = t == 2 ? main[i][j] : rest[i][j];
@@ -498,46 +505,80 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
 #pragma unroll
       for (int r = 0; r < 16; ++r) main[i][j][r] += rest[i][j][r];
 
+  // ---- the K groups' sums meet in LDS; each finishes its share of the rows
+  constexpr int MO = MI / KG;
+  v16f out[MO][NI];
+  if constexpr (KG == 1) {
+#pragma unroll
+    for (int i = 0; i < MO; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j) out[i][j] = main[i][j];
+  } else {
+    static_assert(KG == 2 && MI == 2, "two K groups, a block of rows for each");
+    __syncthreads();
+    v4f* const meeting = reinterpret_cast<v4f*>(smem) + wv * NI * 4 * 64 + lane;  // [receiving group][wavefront][quad of values][lane]
+    constexpr int HALF = WGM * WGN * NI * 4 * 64;
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        v4f v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = grp == 0 ? main[1][j][4 * c + e] : main[0][j][4 * c + e];
+        meeting[(1 - grp) * HALF + (4 * j + c) * 64] = v;
+      }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const v4f v = meeting[grp * HALF + (4 * j + c) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)  // (a sum of two: the same bits either way round)
+          out[0][j][4 * c + e] = (grp == 0 ? main[0][j][4 * c + e] : main[1][j][4 * c + e]) + v[e];
+      }
+  }
+
   // ---- what the split may have got wrong
-  const unsigned rowBase = m0 + wm * MI * 32, colBase = n0 + wn * NI * 32;
+  const unsigned rowBase = m0 + wm * MI * 32 + grp * MO * 32, colBase = n0 + wn * NI * 32;
   float notFinite = 0.f, low = 1.f;
 #pragma unroll
-  for (int i = 0; i < MI; ++i)
+  for (int i = 0; i < MO; ++i)
 #pragma unroll
     for (int j = 0; j < NI; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        notFinite = fmaf(main[i][j][r], 0.f, notFinite);
-        low = fminf(low, __builtin_fabsf(main[i][j][r]));
+        notFinite = fmaf(out[i][j][r], 0.f, notFinite);
+        low = fminf(low, __builtin_fabsf(out[i][j][r]));
       }
-  if (rowBase + 32 * MI > M || colBase + 32 * NI > N) {  // the zeros outside the matrix do not count
+  if (rowBase + 32 * MO > M || colBase + 32 * NI > N) {  // the zeros outside the matrix do not count
     low = 1.f;
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
+    for (int i = 0; i < MO; ++i)
 #pragma unroll
       for (int j = 0; j < NI; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
           if (rowBase + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3) < M && colBase + 32 * j + lrow < N)
-            low = fminf(low, __builtin_fabsf(main[i][j][r]));
+            low = fminf(low, __builtin_fabsf(out[i][j][r]));
   }
   auto raise = [&]() {
     __hip_atomic_fetch_max(&found.largest[arow], __builtin_bit_cast(unsigned, largestA), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     __hip_atomic_fetch_max(&found.largest[BM + brow], __builtin_bit_cast(unsigned, largestB), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
   auto value = [&](auto block, auto r) __attribute__((always_inline)) -> float {
-    const float v = main[block / NI][block % NI][(int)r];  // (a copy: a bit_cast of a vector's element reads its first one)
+    const float v = out[block / NI][block % NI][(int)r];  // (a copy: a bit_cast of a vector's element reads its first one)
     return v;
   };
   auto where = [&](int block, int r, unsigned& row, unsigned& col) __attribute__((always_inline)) {
-    row = wm * MI * 32 + 32 * (block / NI) + 8 * (r >> 2) + 4 * g + (r & 3);
+    row = wm * MI * 32 + grp * MO * 32 + 32 * (block / NI) + 8 * (r >> 2) + 4 * g + (r & 3);
     col = wn * NI * 32 + 32 * (block % NI) + lrow;
   };
-  unsigned again[PT];
+  unsigned again[MO * NI];
   const bool suspicious = notFinite != 0.f || low < 0x1p-64f || largestA >= 0x1p30f || largestB >= 0x1p30f;
-  if (split_failed<BM, BN, T, TRANSB, PT>(p, tile, suspicious, found, again, value, where, raise)) {
+  if (split_failed<BM, BN, T * KG, TRANSB, MO * NI>(p, tile, suspicious, found, again, value, where, raise)) {
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
+    for (int i = 0; i < MO; ++i)
 #pragma unroll
       for (int j = 0; j < NI; ++j) {
         if (!__any(again[i * NI + j] != 0)) continue;
@@ -555,13 +596,13 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
           for (int e = 0; e < 16; ++e) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], sum, 0, 0, 0);
         }
 #pragma unroll
-        for (int r = 0; r < 16; ++r) main[i][j][r] = again[i * NI + j] >> r & 1 ? sum[r] : main[i][j][r];
+        for (int r = 0; r < 16; ++r) out[i][j][r] = again[i * NI + j] >> r & 1 ? sum[r] : out[i][j][r];
       }
   }
 
   // ---- tile store: + bias, + residual, GELU; rows past M and columns past N fail the range check
   const bool inside = rowBase < M && colBase < N;
-  const unsigned ldc = p.ldc, rows = inside ? min(M - rowBase, 32u * MI) : 1u;
+  const unsigned ldc = p.ldc, rows = inside ? min(M - rowBase, 32u * MO) : 1u;
   const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(tile.C + (size_t)rowBase * ldc + colBase, 0,
                                                                       (int)(((rows - 1) * ldc + N - colBase) * 4u), 0x00020000);
   const float* R = tile.R ? tile.R + (size_t)rowBase * N + colBase : nullptr;
@@ -578,13 +619,13 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void sgemm_split_kernel(const Sg
     const __amdgpu_buffer_rsrc_t rr =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(R), 0, (int)(((rows - 1) * N + N - colBase) * 4u), 0x00020000);
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
+    for (int i = 0; i < MO; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const unsigned row = 32 * i + 8 * (r >> 2) + (r & 3);
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
-          float v = main[i][j][r] + bv[j];
+          float v = out[i][j][r] + bv[j];
           if (residual) v += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rr, from[j] + row * N * 4u, 0, 0));
           // same expression as the stand-alone GELU kernel, so that fusing changes no bit
           if (gelu) v = gelu_erf_f32(v);
@@ -881,13 +922,13 @@ int launch(hipStream_t stream, SgemmParams& p, Kernel kern, bool (&attrSet)[16],
   return check_launch("sgemm");
 }
 
-template <int MI, int NI, int WGM, int WGN, bool TRANSB>
+template <int MI, int NI, int WGM, int WGN, int KG, bool TRANSB>
 int launch_shared(hipStream_t stream, SgemmParams p) {
   constexpr int BM = 32 * MI * WGM, BN = 32 * NI * WGN;
-  constexpr size_t lds = 3 * SharedLayout<BM, BN>::STAGE;
+  constexpr size_t lds = KG * 3 * SharedLayout<BM, BN>::STAGE;
   static_assert(lds <= 159 * 1024, "LDS budget");
   static bool attrSet[16] = {};
-  return launch(stream, p, sgemm_split_kernel<MI, NI, WGM, WGN, TRANSB>, attrSet, BM, BN, 64 * WGM * WGN, lds);
+  return launch(stream, p, sgemm_split_kernel<MI, NI, WGM, WGN, KG, TRANSB>, attrSet, BM, BN, 64 * WGM * WGN * KG, lds);
 }
 
 template <int KG, bool TRANSB>
@@ -902,8 +943,14 @@ namespace sgemm_detail {
 
 int sgemm_split_launch(hipStream_t stream, const SgemmParams& p, int kernel, bool transB) {
   switch (kernel) {
-    case sgemm_split_plan::kWide: return transB ? launch_shared<2, 2, 2, 4, true>(stream, p) : launch_shared<2, 2, 2, 4, false>(stream, p);
-    case sgemm_split_plan::k128: return transB ? launch_shared<2, 2, 2, 2, true>(stream, p) : launch_shared<2, 2, 2, 2, false>(stream, p);
+    case sgemm_split_plan::kWide: return transB ? launch_shared<2, 2, 2, 4, 1, true>(stream, p) : launch_shared<2, 2, 2, 4, 1, false>(stream, p);
+    case sgemm_split_plan::k128: {
+      // (of one product: one of a group is summed as it is alone)
+      const unsigned long long tiles = sgemm_tiles::tiles_of(p.M, p.N, p.groups ? 1 : p.batch, 128, 128);
+      if (sgemm_split_plan::k_groups_of_128(tiles, p.K) == 2)
+        return transB ? launch_shared<2, 2, 2, 2, 2, true>(stream, p) : launch_shared<2, 2, 2, 2, 2, false>(stream, p);
+      return transB ? launch_shared<2, 2, 2, 2, 1, true>(stream, p) : launch_shared<2, 2, 2, 2, 1, false>(stream, p);
+    }
     default: return transB ? launch64<4, true>(stream, p) : launch64<4, false>(stream, p);
   }
 }
