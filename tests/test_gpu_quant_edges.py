@@ -24,7 +24,7 @@ def test_quantize_with_the_range_of_the_data(pkg, T, total, dtype, skip):
     assert np.array_equal(T.n(q), O.quantize(x[skip:], lo, hi, dtype))
 
 
-@pytest.mark.parametrize("total", [32768, 32769, 36864, (1 << 20) - 3, (1 << 20) + 1, (2 << 20) + 2, (4 << 20) + 3, 8 << 20, (8 << 20) + 1])
+@pytest.mark.parametrize("total", [40960, 40961, 45057, (1 << 20) - 3, (1 << 20) + 1, (2 << 20) + 2, (4 << 20) + 3, 8 << 20, (8 << 20) + 1])
 @pytest.mark.parametrize("dtype,middle", [("uint8", 0.1), ("int8", -300.0), ("int16", 1.0), ("int32", 0.0), ("uint8", 3e6)])
 def test_quantize_in_workgroups_that_agree_on_the_range(pkg, T, total, dtype, middle):
     """one, two, four and eight pieces to a thread, whole numbers that fit 32 bits and that do not, a NaN and the extremes in

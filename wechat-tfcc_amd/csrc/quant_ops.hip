@@ -419,8 +419,8 @@ __device__ __forceinline__ float dec(unsigned u) {
 // four launches.
 constexpr unsigned kWholeLimit = 128 * 1024;  // elements; 4096 elements: 18.6 -> 3.4 us per call, 77077: 6.3, 131072: 7.7 against
 // 8.6 for the form in two launches, whose time does not grow with the size there
-constexpr unsigned kWholeBest = 32 * 1024;  // where the form below is as fast: 16384 elements 3.9 us here and 4.5 there, 32768 4.4 (4.7
-// from memory) and 4.5
+constexpr unsigned kWholeBest = 40 * 1024;  // up to where the form below is no faster: 16384 elements 3.9 us here and 4.5 there, 32768
+// 4.4 (4.7 from memory) and 4.5; there the host has to ask, in 0.2 us, whether the stream is being captured
 __global__ __launch_bounds__(1024) void quantize_whole_kernel(const float* in, unsigned total, void* out, int outType,
                                                               float* mnOut, float* mxOut) {
   __shared__ float shMn[16], shMx[16];
@@ -626,20 +626,22 @@ __global__ void minmax_finish_kernel(float* mn, float* mx) {
 
 // A tensor that the GPU's registers hold, in one launch: a workgroup reads its part once, the workgroups tell one another its
 // minimum and maximum, and each quantizes what it has.  A word of the exchange is a value and the number of the call, which no
-// other call has, so a reader waits for this call's, and nothing has to be cleared or ordered.  The workgroups need
-// not all run at once: one that has waited kTogetherWait for the others reads all of the input itself, as above.
+// other call has, so a reader waits for this call's, and nothing has to be cleared or ordered.  Calls take turns with
+// kTogetherTurns sets of words; one that meets another call in its set, on another stream, and one whose workgroups do not all run at
+// once is no worse off than slow: a workgroup that has waited kTogetherWait for the others reads all of the input itself, as
+// above.  (A replayed graph would find the words of its last replay, so a recorded call takes the launches below.)
 //
 // Bound by the launch, a store to memory and a load from it; with many elements to a workgroup by the reading.  us, the range
 // and the quantizing in a launch each before (up to 131072 elements the form above), input from memory: 77077 6.8 -> 5.1, 131072
 // 8.6 -> 5.2, 786432 8.9 -> 6.6, 2 M 11.3 -> 8.4, 8 M 21.1 -> 15.7 (17.5 with 64-bit whole numbers for every element).
-constexpr unsigned kTogetherWorkgroups = 256, kTogetherSlots = 256;  // of a launch; streams that have words for one
+constexpr unsigned kTogetherWorkgroups = 256, kTogetherTurns = 256;
 constexpr unsigned kTogetherLimit = kTogetherWorkgroups * 1024 * 4 * 8;  // elements: 32 to a thread
 constexpr unsigned long long kTogetherWait = 20000;  // of the 100 MHz clock: 200 us
-__device__ unsigned long long togetherWords[kTogetherSlots * kTogetherWorkgroups * 2];
+__device__ unsigned long long togetherWords[kTogetherTurns * kTogetherWorkgroups * 2];
 
 template <int QUADS>
 __global__ __launch_bounds__(1024) void quantize_together_kernel(const float* in, size_t total, void* out, int outType, float* mnOut,
-                                                                 float* mxOut, unsigned slot, unsigned call) {
+                                                                 float* mxOut, unsigned call) {
   __shared__ float shMn[16], shMx[16];
   __shared__ int alone;
   const size_t total4 = total / 4, first = (size_t)blockIdx.x * (1024 * QUADS) + threadIdx.x;
@@ -676,7 +678,7 @@ __global__ __launch_bounds__(1024) void quantize_together_kernel(const float* in
     }
   };
   join();
-  unsigned long long* const words = togetherWords + (size_t)slot * kTogetherWorkgroups * 2;
+  unsigned long long* const words = togetherWords + call % kTogetherTurns * (kTogetherWorkgroups * 2);
   if (threadIdx.x == 0) {
     const unsigned long long number = (unsigned long long)call << 32;
     __hip_atomic_store(words + 2 * blockIdx.x, number | __float_as_uint(mn), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -757,10 +759,10 @@ StreamSlots gArrivalSlots(kArrivalSlots);
 std::atomic<unsigned> gTogetherCalls{1};
 
 // as many workgroups as there may be: a thread's loads are all on their way at once, and the words are read side by side
-void launch_together(hipStream_t s, const float* in, uint64_t total, void* out, int outType, float* mn, float* mx, unsigned slot) {
+void launch_together(hipStream_t s, const float* in, uint64_t total, void* out, int outType, float* mn, float* mx) {
   const unsigned call = gTogetherCalls.fetch_add(1, std::memory_order_relaxed), pieces = (unsigned)((total + 4095) / 4096);
   auto launch = [&](auto kernel, unsigned quads) {
-    hipLaunchKernelGGL(kernel, dim3((pieces + quads - 1) / quads), dim3(1024), 0, s, in, (size_t)total, out, outType, mn, mx, slot, call);
+    hipLaunchKernelGGL(kernel, dim3((pieces + quads - 1) / quads), dim3(1024), 0, s, in, (size_t)total, out, outType, mn, mx, call);
   };
   if (pieces <= kTogetherWorkgroups) launch(quantize_together_kernel<1>, 1);
   else if (pieces <= 2 * kTogetherWorkgroups) launch(quantize_together_kernel<2>, 2);
@@ -925,12 +927,8 @@ int tfcc_rocm_quantize_minmax(void* stream, const float* in, uint64_t total, voi
   // every element where it was read.
   const uintptr_t inAt = (uintptr_t)in, outAt = (uintptr_t)out;
   const bool apart = inAt + 4 * total <= outAt || outAt + total * (int_range(out_type).bits / 8) <= inAt;
-  int dev = 0;
-  unsigned slot = 0;
-  TFCC_HIP_CHECK(hipGetDevice(&dev));
-  const bool withSlot = total > kWholeBest && gArrivalSlots.of(dev, s, &slot);
-  if (apart && withSlot && total <= kTogetherLimit && slot < kTogetherSlots) {
-    launch_together(s, in, total, out, out_type, min_v, max_v, slot);
+  if (apart && total > kWholeBest && total <= kTogetherLimit && runs_in_order_now(s)) {
+    launch_together(s, in, total, out, out_type, min_v, max_v);
     return check_launch("quantize");
   }
   if (apart && total <= kWholeLimit) {
@@ -943,7 +941,10 @@ int tfcc_rocm_quantize_minmax(void* stream, const float* in, uint64_t total, voi
   if (apart && (uintptr_t)in % 16 == 0 && (uintptr_t)out % 4 == 0) {
     // partial results, eight bytes per workgroup, rest in the output buffer until the quantize pass overwrites it
     float* partials = static_cast<float*>(out);
-    if (withSlot) {
+    int dev = 0;
+    unsigned slot = 0;
+    TFCC_HIP_CHECK(hipGetDevice(&dev));
+    if (gArrivalSlots.of(dev, s, &slot)) {
       // one workgroup per CU at most: every arrival costs an atomic on one word and a write-back (192 workgroups of 256
       // threads for 786432 elements: 6 us, 48 of 1024: 5.6)
       const unsigned blocks = total >= 256u * 16384u ? 256u : (unsigned)((total + 16383) / 16384);
