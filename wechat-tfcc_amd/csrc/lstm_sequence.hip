@@ -6,7 +6,7 @@
 // the whole sequence, keeps their columns of the state kernel in registers, and the workgroups hand their part of h to
 // each other through memory: 2.1 us per step of 4 x 512, both directions at once (3.0 for 4 x 1024).  What is left is
 // the way of h to memory and back and the polls that came too early.  Up to 768 units a second form keeps h inside an XCD:
-// 1.5 us per step (lstm_xcd_kernel, below); the first one then takes what is recorded in a
+// 1.4 us per step (lstm_xcd_kernel, below); the first one then takes what is recorded in a
 // graph, and what a part of a partitioned GPU gets.
 //
 // The exchange is made of words that a reader polls themselves, so nothing is ordered by fences.  There are two kinds:
@@ -401,17 +401,18 @@ __device__ __forceinline__ unsigned xcd_id() { return __builtin_amdgcn_s_getreg(
 //
 // A wavefront owns UPW units.  A lane takes four k in 256 of all their gates, so a row of h is KQ loads from LDS, and
 // the products are on the vector unit: one row leaves three of the four rows of a 4 x 4 x 1 matrix op empty, and with four the
-// time is the same.  Us per step, 100 steps with both directions, the form below -> this one: 4 x 256 1.75 -> 1.22, 16 x 256 4.9
-// -> 1.7, 4 x 512 2.13 -> 1.53, 8 x 512 2.75 -> 1.86, 16 x 512 4.9 -> 2.56, 4 x 768 2.64 -> 2.20, 12 x 700 4.4 -> 3.4.  Of the 1.53,
-// without it: the products 0.26, the cell's functions 0.28, inputs and results 0.15; the exchange and the rest is 0.88.  (The
-// form below on one XCD, all rows in each: 4 x 512 1.98, 8 x 512 2.71, 4 x 768 3.35.  Words that have arrived not asked for again:
-// 16 x 512 2.85.  Results stored a step later: 2.63; inputs fetched one step at a time, not four: 2.61.)
+// time is the same.  100 steps of both directions, us, the form above -> this one: 1 x 128 162 -> 119, 4 x 256 171 -> 122, 16 x 256
+// 495 -> 158, 4 x 512 212 -> 139, 8 x 512 277 -> 182, 16 x 512 484 -> 243, 4 x 768 265 -> 192, 12 x 700 446 -> 332; one step of 4 x
+// 512 19.5 -> 11.5.  Of 1.5 us for a step of 4 x 512 the products take 0.26 when they are left out, the cell's functions 0.28, inputs and results 0.15;
+// the exchange and the rest is 0.88.  (The form above on one XCD, all rows in each: 4 x 512 2.0 a step, 8 x 512 2.7, 4 x 768 3.35.
+// Words that have arrived not asked for again: 16 x 512 2.85 against 2.6.  Results stored a step later, or inputs fetched one
+// step at a time, not four: 2.6 against 2.55.)
 template <int ROWS, int KQ>
 __global__ __launch_bounds__(512) void lstm_xcd_kernel(SequenceParams p) {
   constexpr int WAVES = 8, T = 64 * WAVES, K = 256 * KQ, UPW = KQ, SUMS = UPW * ROWS;
   constexpr int LEFT = values_left<SUMS, 32, 4>(), COPIES = 16 / (SUMS / LEFT);
   static_assert(LEFT <= COPIES, "a lane finishes one value");
-  __shared__ __attribute__((aligned(16))) float hs[2][ROWS][K];
+  __shared__ __attribute__((aligned(16))) float hs[2][ROWS][K], columns[WAVES * UPW][260];  // (260: a wavefront's writes on all banks)
   __shared__ int gaveUp, apart;
   const unsigned turn = blockIdx.x % kXcds, d = turn / p.groups, group = turn - d * p.groups;
   if (d >= p.directions) return;  // nothing for this XCD
@@ -430,18 +431,53 @@ __global__ __launch_bounds__(512) void lstm_xcd_kernel(SequenceParams p) {
   __syncthreads();
 
   const unsigned u0 = (blockIdx.x / kXcds * WAVES + wave) * UPW;
+  // The state kernel: rows of a gate's units side by side go through LDS, four values to a load (fetched by the lanes that keep
+  // them, a value of a row at a time, 4 x 512 takes 12 us longer and 4 x 768 31).  Rows that do not exist are zeros; what
+  // stands in the place of units that do not is nobody's.
   float w[KQ][4][4][UPW];  // [.][k][gate][unit]
+  {
+    const __amdgpu_buffer_rsrc_t kernel = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(s.kernel), 0, (int)(16u * units * units), 0x00020000);
+    const unsigned first = blockIdx.x / kXcds * (WAVES * UPW);
 #pragma unroll
-  for (int i = 0; i < KQ; ++i)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const unsigned k = 256 * i + 4 * lane + e;
+    for (int i = 0; i < KQ; ++i) {
+      lstm_v4f rows[4][UPW];
+      auto place = [&](int n, unsigned& k, unsigned& unit) {  // 2 UPW loads side by side are a row
+        const unsigned item = tid + n * T;
+        k = item / (2 * UPW);
+        unit = item % (2 * UPW) * 4;
+      };
 #pragma unroll
       for (int g = 0; g < 4; ++g)
 #pragma unroll
-        for (int n = 0; n < UPW; ++n)
-          w[i][e][g][n] = k < units && u0 + n < units ? s.kernel[(size_t)k * 4 * units + (size_t)g * units + u0 + n] : 0.f;
+        for (int n = 0; n < UPW; ++n) {
+          unsigned k, unit;
+          place(n, k, unit);
+          const unsigned at = ((256 * i + k) * 4 + g) * units + first + unit, end = 4 * units * units;
+          rows[g][n] = __builtin_bit_cast(lstm_v4f, __builtin_amdgcn_raw_buffer_load_b128(kernel, 256 * i + k < units ? at * 4u : kNothing, 0, 0));
+          if (at < end && at + 4 > end)  // the last row of the last gate: four values that the matrix ends in are not fetched at all
+#pragma unroll
+            for (unsigned e = 0; e < 3; ++e) rows[g][n][e] = at + e < end ? s.kernel[at + e] : 0.f;
+        }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < UPW; ++n) {
+          unsigned k, unit;
+          place(n, k, unit);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) columns[unit + e][k] = rows[g][n][e];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < UPW; ++n) {
+          const lstm_v4f v = *reinterpret_cast<const lstm_v4f*>(&columns[wave * UPW + n][4 * lane]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[i][e][g][n] = v[e];
+        }
+      }
     }
+  }
   // the unit and the row whose sum this lane ends with, as in the other form
   int base = 0;
   {
