@@ -284,6 +284,8 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
   int* rowTerm = colTerm + BN;                  // [BM]
   unsigned char* stageQ = smem + (BM + BN) * 4; // [BM][BN + 4] bytes, requantized tile
   constexpr int QPITCH = BN + 4;
+  constexpr int CPITCH = WN + 4;  // 32 rows of a wavefront's int32 results
+  int* const stageC = reinterpret_cast<int*>(smem + (BM + BN) * 4) + wave * 32 * CPITCH;
   // lanes l and l+32 hold the two k halves of the same column; the transposing read hands lane
   // (colHalf, s16) column 16*colHalf + s16 of the 32-column block
 #pragma unroll
@@ -332,7 +334,9 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
           int v[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = (int)((unsigned)acc[i][j][4 * rq4 + e] + (unsigned)rt + (unsigned)ct[e]);
-          if constexpr (WRITE_C) {
+          if constexpr (WRITE_C && !REQUANT) {
+            *reinterpret_cast<v4i*>(stageC + l32 * CPITCH + tcol - wn * WN) = v4i{v[0], v[1], v[2], v[3]};
+          } else if constexpr (WRITE_C) {
             if (grow < M && n0 + tcol < N)  // N % 16 == 0: the four columns are in or out together
               *reinterpret_cast<v4i*>(C + (size_t)grow * N + n0 + tcol) = v4i{v[0], v[1], v[2], v[3]};
           }
@@ -349,6 +353,18 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
             }
             *reinterpret_cast<unsigned*>(stageQ + trow * QPITCH + tcol) = q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24);
           }
+        }
+      }
+      if constexpr (WRITE_C && !REQUANT) {
+        // The wavefront's 32 rows lie in LDS: WN / 4 lanes write one row's WN columns.  From the registers a store writes 32
+        // pieces of 32 bytes: us, 1024 x 768 x 3072 10.7 -> 10.3, 2048 x 512 x 2048 10.1 -> 9.6, 640 x 256 x 2048 5.7 -> 5.35.
+        constexpr int PER = WN / 4, ROWS = 64 / PER;
+#pragma unroll
+        for (int t = 0; t < 32 / ROWS; ++t) {
+          const int row = t * ROWS + lane / PER, col = lane % PER * 4;
+          const v4i v = *reinterpret_cast<const v4i*>(stageC + row * CPITCH + col);
+          const unsigned to = m0 + wm * WM + 32 * i + row, at = n0 + wn * WN + col;
+          if (to < M && at < N) *reinterpret_cast<v4i*>(C + (size_t)to * N + at) = v;  // N % 16 == 0: four columns are in or out together
         }
       }
       if constexpr (FLAVOUR != 0) {
@@ -392,7 +408,7 @@ int launch(hipStream_t stream, QGemmParams p) {
   p.perBatchMagic = perBatch.magic; p.perBatchShift = perBatch.shift;
   p.bandMagic = band.magic; p.bandShift = band.shift;
   constexpr size_t ring = (size_t)STAGES * (BM + BN) * BK;
-  constexpr size_t epi = (size_t)(BM + BN) * 4 + (size_t)BM * (BN + 4);
+  constexpr size_t epi = (size_t)(BM + BN) * 4 + (REQUANT ? (size_t)BM * (BN + 4) : (size_t)WGM * WGN * 32 * (BN / WGN + 4) * 4);
   constexpr size_t lds = ring > epi ? ring : epi;
   static_assert(lds <= 160 * 1024, "LDS budget");
   auto kern = qgemm_dma_kernel<BM, BN, WGM, WGN, STAGES, REQUANT, WRITE_C, OWN_COLSUM>;
