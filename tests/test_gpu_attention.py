@@ -146,6 +146,23 @@ def test_attention_with_mask_equals_separate_kernels(pkg, gpu, B, H, S, Tk, D, d
     assert rel_fro(got, ref) <= 1e-5
 
 
+# blocks of 16 query rows: up to 64 keys, and up to 128 with few rows or few blocks; the edges of rows, keys and head widths
+@pytest.mark.parametrize("B,H,S,Tk,D,divisor,layout", [
+    (2, 3, 1, 1, 4, None, "bshd"), (1, 5, 15, 17, 12, 8.0, "bhsd"), (2, 2, 16, 16, 16, 5.0, "bshd"), (1, 3, 17, 63, 20, 8.0, "bhsd"),
+    (1, 12, 29, 29, 64, 8.0, "bshd"), (2, 2, 33, 64, 60, 3.0, "bshd"), (1, 2, 47, 65, 64, 8.0, "bhsd"), (1, 12, 128, 128, 64, 8.0, "bshd"),
+    (1, 3, 130, 127, 44, 6.0, "bhsd"),
+    (40, 9, 16, 120, 32, 8.0, "bshd"), (23, 12, 70, 60, 64, 8.0, "bshd"),  # several blocks to a CU
+])
+def test_attention_in_blocks_of_16_rows(pkg, gpu, B, H, S, Tk, D, divisor, layout):
+    test_attention_equals_separate_kernels(pkg, gpu, B, H, S, Tk, D, divisor, layout)
+
+
+@pytest.mark.parametrize("B,H,S,Tk,D,divisor,per_head", [
+    (1, 12, 29, 29, 64, 8.0, False), (3, 2, 16, 64, 24, 5.0, True), (2, 4, 19, 90, 64, 8.0, True), (9, 3, 9, 128, 8, None, False)])
+def test_attention_with_mask_in_blocks_of_16_rows(pkg, gpu, B, H, S, Tk, D, divisor, per_head):
+    test_attention_with_mask_equals_separate_kernels(pkg, gpu, B, H, S, Tk, D, divisor, per_head)
+
+
 LONG_CASES = [
     # B, H, S, T, D, divisor, layout: key sequences beyond one block of 128
     (1, 12, 384, 384, 64, 8.0, "bshd"),     # the sequence length of the question-answering model the reference documents

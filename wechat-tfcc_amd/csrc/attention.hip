@@ -372,6 +372,170 @@ __global__ __launch_bounds__(8 * ROWS, ROWS == 64 ? 4 : 3) void attention_kernel
   }
 }
 
+// The same with 16 query rows per workgroup of four wavefronts, bound by the chain from the first load to the last store, of
+// which every part is half as long here, rather than by a rate.  No operand goes
+// through LDS on its way in: the 16x16x4 ops take k as 0, 4, 1, 5 and 2, 6, 3, 7 of every eight (above), so of two blocks of
+// eight each half of a wavefront fetches one, four values to a load, and one exchange between the halves makes the operands
+// of two ops.  The scores are the first thing that the wavefronts share.  KEYS: 64 or 128, one or two columns of the softmax
+// to a lane.  12 heads of 64 columns, us, 32 or 64 rows -> 16: 1 x 16 rows 6.2 -> 4.0, 1 x 29 6.7 -> 4.1, 1 x 64 6.9 -> 4.5, 1 x
+// 128 7.9 -> 6.1, 8 x 29 6.8 -> 4.3, 16 x 64 9.0 -> 8.0, 64 x 64 22.0 -> 20.2.
+__device__ __forceinline__ void operands16(const v4f& x, float (&op)[2][2]) {  // [block of eight][op]
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const float low = x[2 * h], high = x[2 * h + 1];  // copies: a bit_cast of a vector's element reads its first one
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, low), __builtin_bit_cast(unsigned, high), false, false);
+    op[0][h] = __builtin_bit_cast(float, (unsigned)r[0]);
+    op[1][h] = __builtin_bit_cast(float, (unsigned)r[1]);
+  }
+}
+
+template <int KEYS>
+__global__ __launch_bounds__(256, 1) void attention_rows16_kernel(const AttentionParams p) {
+  static_assert(KEYS == 64 || KEYS == 128, "one or two columns to a lane");
+  constexpr int ROWS = 16, PER = KEYS / 64, PAIRS_D = kMaxD / 16, PAIRS_T = KEYS / 16, PITCH = KEYS + 4;
+  __shared__ __attribute__((aligned(16))) float Sc[ROWS * PITCH];  // scores, then probabilities
+  const unsigned wg = blockIdx.x;
+  TFCC_ATTENTION_FETCH_ARGUMENTS(p);
+  const unsigned L = (wg & 7u) * p.chunk + (wg >> 3);
+  if ((wg >> 3) >= p.chunk || L >= p.total) return;
+  const unsigned bi = udiv_apply(L, p.blocksMagic, p.blocksShift), blk = L - bi * p.blocksS;
+  const unsigned bo = udiv_apply(bi, p.innerMagic, p.innerShift), bn = bi - bo * p.batchInner;
+  const unsigned s0 = blk * ROWS, S = p.S, T = p.T, D = p.D;
+  const float* __restrict__ Q = p.Q + (size_t)bo * p.outerQ + (size_t)bn * p.innerQ;
+  const float* __restrict__ K = p.K + (size_t)bo * p.outerK + (size_t)bn * p.innerK;
+  const float* __restrict__ V = p.V + (size_t)bo * p.outerV + (size_t)bn * p.innerV;
+  float* __restrict__ O = p.O + (size_t)bo * p.outerO + (size_t)bn * p.innerO;
+  const unsigned lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned Dp = (D + 7u) & ~7u, Tp = (T + 7u) & ~7u;
+
+  // ---- loads, in the order of their use; an offset past the end of its operand returns zero
+  constexpr unsigned kPastEnd = 0xfffffff0u;
+  auto buffer = [&](const float* x, unsigned rows, unsigned ld) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), 0, (int)(((rows - 1) * ld + D) * 4u), 0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t rq = buffer(Q, S, p.ldq), rk = buffer(K, T, p.ldk), rv = buffer(V, T, p.ldv);
+  const unsigned chunk = 2 * (q >> 1) + (q & 1);  // of four values, in a pair of blocks of eight
+  auto load_row = [&](__amdgpu_buffer_rsrc_t from, unsigned row, unsigned rows, unsigned ld, v4f (&x)[PAIRS_D]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < PAIRS_D; ++j) {
+      const unsigned at = 16 * j + 4 * chunk;
+      x[j] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(from, row < rows && at < D ? (row * ld + at) * 4u : kPastEnd, 0, 0));
+    }
+  };
+  v4f qreg[PAIRS_D], kreg[PER][PAIRS_D];
+  load_row(rq, s0 + l16, S, p.ldq, qreg);
+#pragma unroll
+  for (int b = 0; b < PER; ++b) load_row(rk, 16 * (wave + 4 * b) + l16, T, p.ldk, kreg[b]);
+  const bool masked = p.mask != nullptr;
+  float mk[PER] = {};
+  if (masked) {
+    const float* __restrict__ mrow = p.mask + (size_t)bo * p.outerM + (size_t)bn * p.innerM;
+#pragma unroll
+    for (int c = 0; c < PER; ++c)
+      if (lane + 64u * c < T) mk[c] = mrow[lane + 64 * c];
+  }
+  const unsigned kq = (q >> 1) + 4 * (q & 1), col = 16 * wave + l16;
+  float vreg[2 * PAIRS_T][2];
+#pragma unroll
+  for (int kb = 0; kb < 2 * PAIRS_T; ++kb)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const unsigned row = 8 * kb + kq + 2 * h;
+      vreg[kb][h] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, row < T && col < D ? (row * p.ldv + col) * 4u : kPastEnd, 0, 0));
+    }
+
+  // ---- scores: wavefront w has the columns 16w .. and 64 + 16w ..
+  {
+    v4f acc[PER];
+#pragma unroll
+    for (int b = 0; b < PER; ++b) acc[b] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < PAIRS_D; ++j) {
+      float qo[2][2], ko[PER][2][2];
+      operands16(qreg[j], qo);
+#pragma unroll
+      for (int b = 0; b < PER; ++b) operands16(kreg[b][j], ko[b]);
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        if ((unsigned)(16 * j + 8 * e) < Dp) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int b = 0; b < PER; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(qo[e][h], ko[b][e][h], acc[b], 0, 0, 0);
+        }
+    }
+    // a divisor that is a power of two divides exactly like a multiplication by its reciprocal
+    const float divisor = p.divisor;
+    const unsigned bits = __builtin_bit_cast(unsigned, divisor), expo = (bits >> 23) & 0xffu;
+    const bool exact = (bits & 0x007fffffu) == 0 && expo >= 2 && expo <= 252;
+    const float inverse = exact ? 1.0f / divisor : 0.f;
+#pragma unroll
+    for (int b = 0; b < PER; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        Sc[(4 * q + r) * PITCH + 16 * (wave + 4 * b) + l16] = !p.divide ? acc[b][r] : exact ? acc[b][r] * inverse : acc[b][r] / divisor;
+  }
+  __syncthreads();
+
+  // ---- softmax: four rows by a wavefront; columns T .. become the zeros the next product reads
+  {
+    float v[4][PER], mx[4], sum[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      mx[u] = -FLT_MAX;
+#pragma unroll
+      for (int c = 0; c < PER; ++c) {
+        const unsigned i = lane + 64 * c;
+        const float score = Sc[(wave + 4 * u) * PITCH + i];
+        v[u][c] = i < T ? (masked ? score + mk[c] : score) : -FLT_MAX;
+        mx[u] = fmaxf(mx[u], v[u][c]);
+      }
+    }
+    wave_reduce4<true>(mx);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      sum[u] = 0.f;
+#pragma unroll
+      for (int c = 0; c < PER; ++c) {
+        v[u][c] = lane + 64 * c < T ? softmax_exp(v[u][c] - mx[u]) : 0.f;
+        sum[u] += v[u][c];
+      }
+    }
+    wave_reduce4<false>(sum);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float inverse = 1.0f / sum[u];  // as the stand-alone softmax: one division per row
+#pragma unroll
+      for (int c = 0; c < PER; ++c) Sc[(wave + 4 * u) * PITCH + lane + 64 * c] = lane + 64 * c < T ? v[u][c] * inverse : 0.f;
+    }
+  }
+  __syncthreads();
+
+  // ---- probabilities x V: wavefront w has the columns 16w ..
+  if (16 * wave >= D) return;
+  v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < PAIRS_T; ++j) {
+    if ((unsigned)(16 * j) >= Tp) break;
+    float po[2][2];
+    operands16(*reinterpret_cast<const v4f*>(&Sc[l16 * PITCH + 16 * j + 4 * chunk]), po);
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      if ((unsigned)(16 * j + 8 * e) < Tp) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(po[e][h], vreg[2 * j + e][h], acc, 0, 0, 0);
+      }
+  }
+  if (col < D) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const unsigned row = s0 + 4 * q + r;
+      if (row < S) O[(size_t)row * p.ldo + col] = acc[r];
+    }
+  }
+}
+
 // ---- the same for key sequences of any length: the keys are walked in blocks of 128 with a running row maximum and
 // row sum (m, l).  Per block: scores as above; p = exp(score - m_new) with m_new = max(m, block maximum);
 // l = l * exp(m - m_new) + sum(p); the output accumulator of the earlier blocks is scaled by exp(m - m_new) before the
@@ -741,7 +905,12 @@ extern "C" int tfcc_rocm_attention_f32(void* stream, const tfcc_rocm_attention_d
   // (Beyond 128 keys a block of 32 rows walks all the keys again and holds one workgroup per SIMD's registers: it
   // pays only while every block has a CU to itself - 12 heads of 384 rows 25.3 against 28.4 us, 48 heads 70.5 against 54.4.)
   const bool rows32 = stream128 ? blocks32 <= (unsigned long long)cus : perCu32 * 55 < perCu64 * 100;
-  const unsigned rowsPerBlock = rows32 ? 32 : kRows;
+  // Blocks of 16 rows: up to 64 keys always (128 x 12 heads of 64 rows 37.1 -> 33.7 us, 32 x 12 12.3 -> 12.4, 64 x 12 of 32 11.2 -> 10.6).  Beyond, every
+  // block walks twice the keys, which is faster where there are no more blocks than CUs or no more than with 32 rows
+  // (2 x 12 heads of 128 rows 7.9 -> 6.2 us, 40 x 12 of 16 rows and 100 keys 10.4 -> 8.7), and not otherwise (4 x 12 of 100
+  // rows 7.7 -> 8.4, 8 x 12 of 128 10.4 -> 11.6).
+  const bool rows16 = !stream128 && (d->t <= 64 || d->s <= 16 || (d->s + 15) / 16 * heads <= (unsigned long long)cus);
+  const unsigned rowsPerBlock = rows16 ? 16 : rows32 ? 32 : kRows;
   p.blocksS = (d->s + rowsPerBlock - 1) / rowsPerBlock;
   const unsigned long long total = (unsigned long long)p.blocksS * d->batch_outer * d->batch_inner;
   TFCC_REQUIRE(total < (1ull << 31) - 8, "attention: too many blocks");
@@ -775,7 +944,8 @@ extern "C" int tfcc_rocm_attention_f32(void* stream, const tfcc_rocm_attention_d
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsStream32));
     attrSet[dev] = true;
   }
-  if (stream128 && rows32) hipLaunchKernelGGL(attention_stream_kernel<32>, dim3(p.chunk * 8), dim3(256), ldsStream32, as_stream(stream), p);
+  if (rows16) hipLaunchKernelGGL(d->t <= 64 ? attention_rows16_kernel<64> : attention_rows16_kernel<128>, dim3(p.chunk * 8), dim3(256), 0, as_stream(stream), p);
+  else if (stream128 && rows32) hipLaunchKernelGGL(attention_stream_kernel<32>, dim3(p.chunk * 8), dim3(256), ldsStream32, as_stream(stream), p);
   else if (stream128) hipLaunchKernelGGL(attention_stream_kernel<64>, dim3(p.chunk * 8), dim3(kThreads), ldsBytes, as_stream(stream), p);
   else if (rows32) hipLaunchKernelGGL(attention_kernel<32>, dim3(p.chunk * 8), dim3(256), ldsBytes32, as_stream(stream), p);
   else hipLaunchKernelGGL(attention_kernel<64>, dim3(p.chunk * 8), dim3(kThreads), ldsBytes, as_stream(stream), p);

@@ -298,6 +298,28 @@ __device__ __forceinline__ void wave_reduce8(float (&v)[8], int lane) {
   for (int r = 0; r < 8; ++r) v[r] = real((unsigned)__builtin_amdgcn_readlane((int)bits(y), 8 * r));
 }
 
+// The same for four rows: lanes 16r .. 16r + 15 end with row r.
+template <bool MAX>
+__device__ __forceinline__ void wave_reduce4(float (&v)[4]) {
+  auto join = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
+  auto bits = [](float x) { return __builtin_bit_cast(unsigned, x); };
+  auto real = [](unsigned x) { return __builtin_bit_cast(float, x); };
+  float w[2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    const auto r = __builtin_amdgcn_permlane32_swap(bits(v[a]), bits(v[a + 2]), false, false);
+    w[a] = join(real((unsigned)r[0]), real((unsigned)r[1]));
+  }
+  const auto r = __builtin_amdgcn_permlane16_swap(bits(w[0]), bits(w[1]), false, false);
+  float y = join(real((unsigned)r[0]), real((unsigned)r[1])), a, b;
+  butterfly_pair<8>(y, a, b); y = join(a, b);
+  butterfly_pair<4>(y, a, b); y = join(a, b);
+  butterfly_pair<2>(y, a, b); y = join(a, b);
+  butterfly_pair<1>(y, a, b); y = join(a, b);
+#pragma unroll
+  for (int row = 0; row < 4; ++row) v[row] = real((unsigned)__builtin_amdgcn_readlane((int)bits(y), 16 * row));
+}
+
 // e^x for the x <= 0 a softmax forms by subtracting the row maximum (the reference calls the C library's exp,
 // tfcc/mkl/kernel/tfcc_mklactivationkernel.hpp:137-155).  2^(x log2 e) with the hardware's exp2: the product is
 // formed in two parts (rounded product + what the rounding and the rounding of log2 e dropped), and the small part
