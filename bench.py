@@ -680,7 +680,7 @@ def bench_other(torch, pkg, dev, steps, warmup, c3, short_legs=False):
     w = mf.bert_layer_weights(rng, hidden, ffn)
     # batch 8 x 128 positions, and one sequence of 384 positions: the length of the
     # question-answering model the reference documents (samples/ConvertONNXModel.md:16), whose attention walks the
-    # keys in three blocks of 128
+    # keys in runs of 32
     for name, batch, seq in (("c4_bert_base_layer_b8_s128_runtime", 8, 128), ("bert_base_layer_b1_s384_runtime", 1, 384)):
         graph = mf.bert_encoder_layer(w, batch, seq, heads)
         model = rt.Model(mf.write_model([graph], graph.name))

@@ -225,6 +225,35 @@ def test_attention_over_blocks_of_keys(pkg, gpu, B, H, S, Tk, D, divisor, layout
         assert rel_fro(got, sep) <= 2e-6
 
 
+# runs of 32 keys dealt to four wavefronts: the edges of rows, runs and head widths; two blocks of rows per workgroup from 1536 blocks on
+@pytest.mark.parametrize("B,H,S,Tk,D,divisor,layout", [
+    (1, 2, 1, 129, 4, None, "bshd"), (2, 3, 15, 160, 12, 6.0, "bhsd"), (1, 2, 17, 161, 64, 8.0, "bshd"), (1, 3, 33, 255, 44, 8.0, "bhsd"),
+    (1, 12, 16, 513, 64, 8.0, "bshd"), (50, 33, 9, 140, 12, 5.0, "bshd"), (8, 12, 250, 131, 64, 8.0, "bshd"),
+])
+@pytest.mark.parametrize("masked", [False, True])
+def test_attention_over_runs_of_keys(pkg, gpu, B, H, S, Tk, D, divisor, layout, masked):
+    test_attention_over_blocks_of_keys(pkg, gpu, B, H, S, Tk, D, divisor, layout, masked)
+
+
+@pytest.mark.parametrize("S,Tk,D", [(37, 200, 20), (20, 50, 20), (100, 100, 64)])
+def test_attention_into_rows_of_odd_pitch(pkg, gpu, S, Tk, D):
+    """The rows of the result begin anywhere, and what lies between them stays."""
+    import torch
+    rng = np.random.default_rng(S + Tk)
+    q, k, v = (rng.standard_normal((1, 2, r, D)).astype(np.float32) for r in (S, Tk, Tk))
+    tq, tk, tv = gpu.t(q), gpu.t(k), gpu.t(v)
+    ldo = D + 3
+    out = torch.full((2 * S * ldo + 1,), 7.0, dtype=torch.float32, device=tq.device)
+    desc = pkg.attention_desc(tq, tk, tv, out[1:], S, Tk, D, (D, D, D, ldo), batch_inner=2,
+                              inner_strides=(S * D, Tk * D, Tk * D, S * ldo), divisor=3.0)
+    pkg.attention(desc)
+    got = gpu.n(out)
+    assert got[0] == 7.0
+    got = got[1:].reshape(1, 2, S, ldo)
+    assert (got[..., D:] == 7.0).all()
+    assert rel_fro(got[..., :D], reference64(q, k, v, 3.0)) <= 1e-5
+
+
 def test_attention_limits_are_reported(pkg, gpu):
     import torch
     x = torch.zeros(256 * 256, dtype=torch.float32, device=gpu.t(np.zeros(1, np.float32)).device)

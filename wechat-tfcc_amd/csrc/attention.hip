@@ -1,5 +1,5 @@
 // softmax(Q K^T [/ divisor]) V per batch entry in one launch: key sequences of up to 128 rows with the scores of a
-// row block in LDS in one piece (attention_kernel), longer ones in blocks of 128 keys (attention_stream_kernel).
+// row block in LDS in one piece (attention_kernel), and longer ones in runs of 32 keys (attention_stream_kernel).
 //
 // Stands where the reference's runtime runs the attention core of an encoder layer as separate
 // operations on tensors in HBM: Matmul (tfcc_runtime/operations/math/matmul.cpp:27-41), Div by a
@@ -536,311 +536,231 @@ __global__ __launch_bounds__(256, 1) void attention_rows16_kernel(const Attentio
   }
 }
 
-// ---- the same for key sequences of any length: the keys are walked in blocks of 128 with a running row maximum and
-// row sum (m, l).  Per block: scores as above; p = exp(score - m_new) with m_new = max(m, block maximum);
-// l = l * exp(m - m_new) + sum(p); the output accumulator of the earlier blocks is scaled by exp(m - m_new) before the
-// block's p V is added; at the end every row is divided by its l.  The same real function as the three separate
-// kernels, summed in a different order (a row's exponentials are taken against the running maximum and rescaled,
-// not against the final one): results agree with them to a few units in the last place, not bit for bit; the
-// contract checked is the relative error against double precision.  Blocks of 128 keep the LDS footprint of the
-// kernel above (two workgroups per CU) whatever the length.
-template <int ROWS>
-__global__ __launch_bounds__(8 * ROWS) void attention_stream_kernel(const AttentionParams p) {
-  constexpr int kRows = ROWS, kThreads = 8 * ROWS;  // blocks of 64 or 32 query rows, as in attention_kernel
-  static_assert(ROWS == 64 || ROWS == 32, "two or one row blocks of 32");
-  extern __shared__ __align__(16) float lds[];
-  float* KVs = lds;                       // the block's K as [128][kPitchK], then its V as [128][kPitchV]
-  float* Sc = KVs + kMaxT * kPitchV;      // [64][kPitchS]  scores, then probabilities of the block
-  float* rowScale = Sc + kRows * kPitchS; // [64] what the accumulated rows are multiplied by before the block is added
-                                          //      (after the last block: 1 / l)
-
+// ---- the same for key sequences of any length: each of four wavefronts takes every fourth run of 32 keys, with a maximum, a sum
+// and a result of its own for every query row (m, l, o).  Per run: scores; p = exp(score - m_new) with m_new = max(m, the run's
+// maximum); l and o scaled by exp(m - m_new), then the run's p and p V added.  At the end the wavefronts' l and o meet, scaled by
+// exp(m - the largest m), and every row is divided by its l.  The same real function as the three separate kernels, summed in a
+// different order: results agree with them to a few units in the last place, not bit for bit; the contract checked is
+// the relative error against double precision.
+//
+// Nothing goes through LDS before the end, and no wavefront waits for another.  The scores are formed transposed, keys x queries:
+// lane (l16, q) of a 16 x 16 block then holds keys 4q .. 4q + 3 of query l16, which is what the ops of the second product,
+// V^T p^T, take from it as they stand, and m, l and the scale belong to the lane's own query.  Which k an op's four lane groups
+// have is the same choice for both operands, so K, Q and V are fetched four values to a load: row l16 of Q and K from 4q on,
+// and of V's row of a key columns 4 l16 .. + 3, whose e-th values make one block of results (row i of it is column 4i + e).
+// BLOCKS: of 16 query rows, which share the loads of K and V.
+//
+// Few blocks: bound by the chain of a wavefront's runs; many: by the matrix ops (16 x 12 heads of 512 keys: 82 of 131 us) and the vector
+// work between them.  Loads take no vector instruction (a descriptor begins at the run's first key and the offsets stay), and keys
+// past the last one are looked for in the last run alone: 16 x 12 x 512 157 -> 131.  12 heads of 64 columns, us, workgroups of 32 or 64
+// rows walking blocks of 128 keys through LDS -> this: 1 x 160 14.4 -> 6.3, 1 x 384 22.7 -> 12.7, 4 x 256 19.1 -> 14.4, 4 x 384 51 ->
+// 27, 16 x 512 200 -> 131; error against float64 4.0e-7 -> 3.2e-7 with 256 keys, 8.7e-7 -> 5.1e-7 with 2048.
+template <int BLOCKS>
+__global__ __launch_bounds__(256, 2) void attention_stream_kernel(const AttentionParams p) {
+  constexpr int WAVES = 4, ROWS = 16 * BLOCKS, QUADS = kMaxD / 16, GROUPS = 2, RUN = 16 * GROUPS;
+  static_assert(QUADS == 4 && WAVES == 4, "a wavefront finishes one of four quads of columns");
+  __shared__ v4f part[WAVES][BLOCKS][4][64];
+  __shared__ float wm[WAVES][ROWS], wl[WAVES][ROWS];
   const unsigned wg = blockIdx.x;
   TFCC_ATTENTION_FETCH_ARGUMENTS(p);
   const unsigned L = (wg & 7u) * p.chunk + (wg >> 3);
   if ((wg >> 3) >= p.chunk || L >= p.total) return;
   const unsigned bi = udiv_apply(L, p.blocksMagic, p.blocksShift), blk = L - bi * p.blocksS;
   const unsigned bo = udiv_apply(bi, p.innerMagic, p.innerShift), bn = bi - bo * p.batchInner;
-  const unsigned s0 = blk * kRows;
-  const unsigned S = p.S, T = p.T, D = p.D;
+  const unsigned s0 = blk * ROWS, S = p.S, T = p.T, D = p.D;
   const float* __restrict__ Q = p.Q + (size_t)bo * p.outerQ + (size_t)bn * p.innerQ;
   const float* __restrict__ K = p.K + (size_t)bo * p.outerK + (size_t)bn * p.innerK;
   const float* __restrict__ V = p.V + (size_t)bo * p.outerV + (size_t)bn * p.innerV;
   float* __restrict__ O = p.O + (size_t)bo * p.outerO + (size_t)bn * p.innerO;
+  const unsigned lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const bool masked = p.mask != nullptr;
-  const float* __restrict__ mrow = masked ? p.mask + (size_t)bo * p.outerM + (size_t)bn * p.innerM : nullptr;
-  const int lrow = lane & 31, g = lane >> 5;
-  const unsigned Dp = (D + 7u) & ~7u;
-  const int wmS = wave >> 2, wnS = wave & 3;  // scores: ROWS / 32 x 4 wavefronts, one 32 x 32 block each
-  const int wm = wave >> 1, wn = wave & 1;    // second product: the first half of the wavefronts, ROWS / 32 x 2 blocks of 32 x 32
-  constexpr int CH = kMaxD / 4;
-  constexpr int KV_ITEMS = kMaxT * CH / kThreads, Q_ITEMS = kRows * CH / kThreads, KBQ = kMaxD / 8;
+  // An offset past the end of its operand returns zero; the operand begins at the run's first key, so the offsets stay.
   constexpr unsigned kPastEnd = 0xfffffff0u;
-  const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(K), 0, (int)(((T - 1) * p.ldk + D) * 4u), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(V), 0, (int)(((T - 1) * p.ldv + D) * 4u), 0x00020000);
-
-  // ---- Q: through the region of the scores into the registers the score product takes it from, once
-  v4f qf[KBQ];
-  {
-    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(Q), 0, (int)(((S - 1) * p.ldq + D) * 4u), 0x00020000);
+  auto rows_from = [&](const float* x, unsigned row, unsigned rows, unsigned ld, unsigned width) __attribute__((always_inline)) {
+    const unsigned left = row < rows ? rows - row : 0;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x) + (size_t)row * ld, 0, left == 0 ? 0 : (int)(((left - 1) * ld + width) * 4u), 0x00020000);
+  };
+  auto four = [](__amdgpu_buffer_rsrc_t from, unsigned at) __attribute__((always_inline)) {
+    return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(from, at, 0, 0));
+  };
+  const bool masked = p.mask != nullptr;
+  const float* const mask = masked ? p.mask + (size_t)bo * p.outerM + (size_t)bn * p.innerM : nullptr;
+  unsigned ofK[GROUPS][QUADS], ofV[GROUPS][4];
 #pragma unroll
-    for (int it = 0; it < Q_ITEMS; ++it) {
-      const unsigned w = tid + it * kThreads, row = w / CH, ch = w % CH;
-      const v4f q = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
-                                                rq, (s0 + row < S && ch * 4 < D) ? ((s0 + row) * p.ldq + ch * 4) * 4u : kPastEnd, 0, 0));
-      *reinterpret_cast<v4f*>(Sc + row * kPitchK + ch * 4) = q;
+  for (int b = 0; b < GROUPS; ++b)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      ofK[b][j] = 16 * j + 4 * q < D ? ((16 * b + l16) * p.ldk + 16 * j + 4 * q) * 4u : kPastEnd;
+      ofV[b][j] = 4 * l16 < D ? ((16 * b + 4 * q + j) * p.ldv + 4 * l16) * 4u : kPastEnd;
     }
-    __syncthreads();
-    const float* qa = Sc + (32 * wmS + lrow) * kPitchK + 4 * g;
+  v4f qreg[BLOCKS][QUADS], kreg[GROUPS][QUADS], vreg[GROUPS][4];
+  float mk[GROUPS][4] = {};
+  auto load_k = [&](unsigned t0) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t rk = rows_from(K, t0, T, p.ldk, D);
 #pragma unroll
-    for (int kb = 0; kb < KBQ; ++kb) {
-      qf[kb] = v4f{0.f, 0.f, 0.f, 0.f};
-      if ((unsigned)kb * 8 < Dp) qf[kb] = *reinterpret_cast<const v4f*>(qa + kb * 8);
-    }
-  }
-
-  // running maximum and sum of the eight rows this wavefront owns in the softmax step (rows wave + 8 u)
-  constexpr int R = 8, W = kThreads / 64;
-  static_assert(W * R == kRows, "every row of the block has its wavefront");
-  float mrun[R], lrun[R];
+    for (int b = 0; b < GROUPS; ++b)
 #pragma unroll
-  for (int u = 0; u < R; ++u) { mrun[u] = -FLT_MAX; lrun[u] = 0.f; }
-  // context accumulators: one 32 x 32 block per wavefront of the first half (ROWS = 64), or two 16 x 16 blocks per
-  // wavefront of all four (ROWS = 32: rows 16 (wave / 2).., column blocks 2 (wave & 1) and 2 (wave & 1) + 1; see
-  // attention_kernel for the order the k values are fed in)
-  v16f acc;
+      for (int j = 0; j < QUADS; ++j) kreg[b][j] = four(rk, ofK[b][j]);
+    if (masked) {
+      const __amdgpu_buffer_rsrc_t rm = rows_from(mask, t0, T, 1, 1);
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-  v4f acc16[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
-  const int l16 = lane & 15, q16 = lane >> 4, rb16 = wave >> 1, cb16 = 2 * (wave & 1);
-  const int kq16 = (q16 >> 1) + 4 * (q16 & 1);
-
-  const float divisor = p.divisor;
-  const unsigned dbits = __builtin_bit_cast(unsigned, divisor), dexpo = (dbits >> 23) & 0xffu;
-  const bool divideByMul = (dbits & 0x007fffffu) == 0 && dexpo >= 2 && dexpo <= 252;  // a power of two: exact
-  const float inverseDivisor = 1.0f / divisor;
-
-  // With blocks of 32 rows (every workgroup alone on its CU) K of a block is asked for one block ahead, into the
-  // registers that the block before has just emptied into LDS, so that only the first block waits for its keys; with
-  // blocks of 64 rows two workgroups per CU cover each other's waits and the registers are worth more (1 % slower).
-  constexpr bool kAhead = ROWS == 32;
-  v4f kreg[KV_ITEMS];
-  auto fetchK = [&](unsigned t0) {
-    const unsigned Tb = min((unsigned)kMaxT, T - t0);
+      for (int b = 0; b < GROUPS; ++b)
 #pragma unroll
-    for (int it = 0; it < KV_ITEMS; ++it) {
-      const unsigned w = tid + it * kThreads, row = w / CH, ch = w % CH;
-      const bool in = row < Tb && ch * 4 < D;
-      kreg[it] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rk, in ? ((t0 + row) * p.ldk + ch * 4) * 4u : kPastEnd, 0, 0));
+        for (int r = 0; r < 4; ++r)
+          mk[b][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rm, (16 * b + 4 * q + r) * 4u, 0, 0));
     }
   };
-  if constexpr (kAhead) fetchK(0);
-  for (unsigned t0 = 0; t0 < T; t0 += kMaxT) {
-    const unsigned Tb = min((unsigned)kMaxT, T - t0);   // keys of this block
-    const unsigned Tbp = (Tb + 7u) & ~7u;                // k extent of the block's second product
-    v4f vreg[KV_ITEMS];
-    if constexpr (!kAhead) fetchK(t0);
-    float mk[2] = {0.f, 0.f};
-    if (masked) {
+  auto load_v = [&](unsigned t0) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t rv = rows_from(V, t0, T, p.ldv, D);
 #pragma unroll
-      for (int q = 0; q < 2; ++q)
-        if ((unsigned)lane + 64u * q < Tb) mk[q] = mrow[t0 + lane + 64 * q];
-    }
-    __syncthreads();  // the block before is done with K / V and with the probabilities (first block: with Q's staging)
+    for (int b = 0; b < GROUPS; ++b)
 #pragma unroll
-    for (int it = 0; it < KV_ITEMS; ++it) {
-      const int w = tid + it * kThreads, row = w / CH, ch = w % CH;
-      *reinterpret_cast<v4f*>(KVs + row * kPitchK + ch * 4) = kreg[it];
-    }
-    // (V is asked for once K's registers are free: it travels while the scores are computed)
+      for (int r = 0; r < 4; ++r) vreg[b][r] = four(rv, ofV[b][r]);
+  };
+  const __amdgpu_buffer_rsrc_t rq = rows_from(Q, s0, S, p.ldq, D);
 #pragma unroll
-    for (int it = 0; it < KV_ITEMS; ++it) {
-      const unsigned w = tid + it * kThreads, row = w / CH, ch = w % CH;
-      const bool in = row < Tb && ch * 4 < D;
-      vreg[it] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rv, in ? ((t0 + row) * p.ldv + ch * 4) * 4u : kPastEnd, 0, 0));
-    }
-    if constexpr (kAhead) {
-      if (t0 + kMaxT < T) fetchK(t0 + kMaxT);
-    }
-    __syncthreads();
+  for (int n = 0; n < BLOCKS; ++n)
+#pragma unroll
+    for (int j = 0; j < QUADS; ++j)
+      qreg[n][j] = four(rq, 16 * j + 4 * q < D ? ((16 * n + l16) * p.ldq + 16 * j + 4 * q) * 4u : kPastEnd);
+  load_k(wave * RUN);
+  load_v(wave * RUN);
 
-    // ---- scores of the block
-    const bool liveS = (unsigned)(32 * wnS) < Tb;
-    if (liveS) {
-      v4f bf[KBQ];
-      const float* ka = KVs + (32 * wnS + lrow) * kPitchK + 4 * g;
+  // a divisor that is a power of two divides exactly like a multiplication by its reciprocal
+  const float divisor = p.divisor;
+  const unsigned bits = __builtin_bit_cast(unsigned, divisor), expo = (bits >> 23) & 0xffu;
+  const bool exact = (bits & 0x007fffffu) == 0 && expo >= 2 && expo <= 252;
+  const bool dividing = p.divide && !exact;
+  const float factor = p.divide && exact ? 1.0f / divisor : 1.0f;
+  // over the four lanes that share a query
+  auto over_groups = [](float v, auto join) __attribute__((always_inline)) {
+    float a, b;
+    butterfly_pair<32>(v, a, b); v = join(a, b);
+    butterfly_pair<16>(v, a, b); return join(a, b);
+  };
+  float m[BLOCKS], l[BLOCKS];  // l: of this lane's keys
+  v4f o[BLOCKS][4];
 #pragma unroll
-      for (int kb = 0; kb < KBQ; ++kb) {
-        bf[kb] = v4f{0.f, 0.f, 0.f, 0.f};
-        if ((unsigned)kb * 8 < Dp) bf[kb] = *reinterpret_cast<const v4f*>(ka + kb * 8);
-      }
-      v16f sacc;
+  for (int n = 0; n < BLOCKS; ++n) {
+    m[n] = -FLT_MAX;
+    l[n] = 0.f;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
+    for (int e = 0; e < 4; ++e) o[n][e] = v4f{0.f, 0.f, 0.f, 0.f};
+  }
+  for (unsigned t0 = wave * RUN; t0 < T; t0 += WAVES * RUN) {
+    v4f s[BLOCKS][GROUPS];
 #pragma unroll
-      for (int kb = 0; kb < KBQ; ++kb) {
-        if ((unsigned)kb * 8 < Dp) {
+    for (int n = 0; n < BLOCKS; ++n)
 #pragma unroll
-          for (int s = 0; s < 4; ++s) sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(qf[kb][s], bf[kb][s], sacc, 0, 0, 0);
-        }
-      }
-      float* sc = Sc + (32 * wmS + 4 * g) * kPitchS + 32 * wnS + lrow;
-      if (!p.divide) {
+      for (int b = 0; b < GROUPS; ++b) s[n][b] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sc[(8 * (r / 4) + (r & 3)) * kPitchS] = sacc[r];
-      } else if (divideByMul) {
+    for (int j = 0; j < QUADS; ++j) {
+      if ((unsigned)(16 * j) >= D) break;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sc[(8 * (r / 4) + (r & 3)) * kPitchS] = sacc[r] * inverseDivisor;
-      } else {
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sc[(8 * (r / 4) + (r & 3)) * kPitchS] = sacc[r] / divisor;
-      }
+        for (int n = 0; n < BLOCKS; ++n)
+#pragma unroll
+          for (int b = 0; b < GROUPS; ++b) s[n][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kreg[b][j][e], qreg[n][j][e], s[n][b], 0, 0, 0);
     }
-    __syncthreads();
-
-    // ---- K is done with: V takes its place
+    float v[BLOCKS][GROUPS][4];
 #pragma unroll
-    for (int it = 0; it < KV_ITEMS; ++it) {
-      const int w = tid + it * kThreads, row = w / CH, ch = w % CH;
-      *reinterpret_cast<v4f*>(KVs + row * kPitchV + ch * 4) = vreg[it];
+    for (int n = 0; n < BLOCKS; ++n)
+#pragma unroll
+      for (int b = 0; b < GROUPS; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float x = s[n][b][r];
+          v[n][b][r] = x * factor;
+        }
+    auto every = [&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+      for (int n = 0; n < BLOCKS; ++n)
+#pragma unroll
+        for (int b = 0; b < GROUPS; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[n][b][r] = f(v[n][b][r], b, r);
+    };
+    if (dividing) every([&](float x, int, int) { return x / divisor; });
+    if (masked) every([&](float x, int b, int r) { return x + mk[b][r]; });
+    // what is no key weighs nothing, whatever the maximum
+    if (t0 + RUN > T) every([&](float x, int b, int r) { return t0 + 16 * b + 4 * q + r < T ? x : -__builtin_inff(); });
+    load_k(t0 + WAVES * RUN);
+#pragma unroll
+    for (int n = 0; n < BLOCKS; ++n) {
+      float highest = m[n];
+#pragma unroll
+      for (int b = 0; b < GROUPS; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) highest = fmaxf(highest, v[n][b][r]);
+      highest = over_groups(highest, [](float a, float b) { return fmaxf(a, b); });
+      const float scale = softmax_exp(m[n] - highest);  // (in front of the first run there is nothing to scale)
+      m[n] = highest;
+      float sum = 0.f;
+#pragma unroll
+      for (int b = 0; b < GROUPS; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          v[n][b][r] = softmax_exp(v[n][b][r] - highest);
+          sum += v[n][b][r];
+        }
+      l[n] = l[n] * scale + sum;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[n][e][r] *= scale;
     }
-
-    // ---- the block's share of the softmax: rows wave + 8 u, columns lane and lane + 64
-    {
-      float v[R][2], mb[R], sum[R];
 #pragma unroll
-      for (int u = 0; u < R; ++u) {
-        const float* sc = Sc + (wave + W * u) * kPitchS;
-        mb[u] = -FLT_MAX;
+    for (int b = 0; b < GROUPS; ++b)
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const unsigned i = lane + 64 * q;
-          v[u][q] = i < Tb ? (masked ? sc[i] + mk[q] : sc[i]) : -FLT_MAX;
-          mb[u] = fmaxf(mb[u], v[u][q]);
-        }
-      }
-      wave_reduce8<true>(mb, lane);
-      float scale[R];
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int u = 0; u < R; ++u) {
-        const float mnew = fmaxf(mrun[u], mb[u]);
-        scale[u] = t0 == 0 ? 0.f : softmax_exp(mrun[u] - mnew);  // nothing is accumulated before the first block
-        mrun[u] = mnew;
-        sum[u] = 0.f;
+        for (int n = 0; n < BLOCKS; ++n)
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const unsigned i = lane + 64 * q;
-          v[u][q] = i < Tb ? softmax_exp(v[u][q] - mnew) : 0.f;
-          sum[u] += v[u][q];
-        }
-      }
-      wave_reduce8<false>(sum, lane);
-#pragma unroll
-      for (int u = 0; u < R; ++u) {
-        lrun[u] = lrun[u] * scale[u] + sum[u];
-        float* sc = Sc + (wave + W * u) * kPitchS;
-#pragma unroll
-        for (int q = 0; q < 2; ++q) sc[lane + 64 * q] = v[u][q];  // zeros past the block's keys
-        const bool lastBlock = t0 + kMaxT >= T;
-        if (lane == 0) rowScale[wave + W * u] = scale[u];
-        if (lastBlock && lane == 1) rowScale[kRows + wave + W * u] = 1.0f / lrun[u];
-      }
-    }
-    __syncthreads();
-
-    // ---- accumulated rows scaled, then the block's probabilities x V
-    if constexpr (ROWS == 32) {
-      if ((unsigned)(16 * cb16) < D) {
-        constexpr int KB = kMaxT / 8;
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc16[j][r] *= rowScale[16 * rb16 + 4 * q16 + r];
-        const float* pa = Sc + (16 * rb16 + l16) * kPitchS + kq16;
-        const float* vb = KVs + kq16 * kPitchV + 16 * cb16 + l16;
-        float af[KB][2], bfv[2][KB][2];
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            af[kb][h] = 0.f; bfv[0][kb][h] = 0.f; bfv[1][kb][h] = 0.f;
-          }
-          if ((unsigned)kb * 8 < Tbp) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              af[kb][h] = pa[kb * 8 + 2 * h];
-              bfv[0][kb][h] = vb[(kb * 8 + 2 * h) * kPitchV];
-              bfv[1][kb][h] = vb[(kb * 8 + 2 * h) * kPitchV + 16];  // columns past D hold zeros
-            }
-          }
-        }
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-          if ((unsigned)kb * 8 < Tbp) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              acc16[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[kb][h], bfv[0][kb][h], acc16[0], 0, 0, 0);
-              acc16[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[kb][h], bfv[1][kb][h], acc16[1], 0, 0, 0);
-            }
-          }
-        }
-      }
-    } else if (wave < ROWS / 16 && (unsigned)(32 * wn) < D) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] *= rowScale[32 * wm + 8 * (r / 4) + 4 * g + (r & 3)];
-      constexpr int KB = kMaxT / 8, HALF = KB / 2;
-      const float* pa = Sc + (32 * wm + lrow) * kPitchS + 4 * g;
-      const float* vb = KVs + (4 * g) * kPitchV + 32 * wn + lrow;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        v4f af[HALF], bfv[HALF];
-#pragma unroll
-        for (int q = 0; q < HALF; ++q) {
-          const int kb = h * HALF + q;
-          af[q] = v4f{0.f, 0.f, 0.f, 0.f};
-          bfv[q] = v4f{0.f, 0.f, 0.f, 0.f};
-          if ((unsigned)kb * 8 < Tbp) {
-            af[q] = *reinterpret_cast<const v4f*>(pa + kb * 8);
-#pragma unroll
-            for (int s = 0; s < 4; ++s) bfv[q][s] = vb[(kb * 8 + s) * kPitchV];
-          }
-        }
-#pragma unroll
-        for (int q = 0; q < HALF; ++q) {
-          if ((unsigned)(h * HALF + q) * 8 < Tbp) {
-#pragma unroll
-            for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[q][s], bfv[q][s], acc, 0, 0, 0);
-          }
-        }
-      }
-    }
+          for (int e = 0; e < 4; ++e) o[n][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vreg[b][r][e], v[n][b][r], o[n][e], 0, 0, 0);
+    load_v(t0 + WAVES * RUN);
   }
 
-  // ---- rows divided by their sums and stored (the reciprocals were left behind the scales by the last block)
-  if constexpr (ROWS == 32) {
+  // ---- the wavefronts meet
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const unsigned col = 16 * (cb16 + j) + l16;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int trow = 16 * rb16 + 4 * q16 + r;
-        const unsigned row = s0 + trow;
-        if (row < S && col < D) O[(size_t)row * p.ldo + col] = acc16[j][r] * rowScale[kRows + trow];
-      }
+  for (int n = 0; n < BLOCKS; ++n) {
+    l[n] = over_groups(l[n], [](float a, float b) { return a + b; });
+    if (q == 0) {
+      wm[wave][16 * n + l16] = m[n];
+      wl[wave][16 * n + l16] = l[n];
     }
-  } else if (wave < ROWS / 16 && (unsigned)(32 * wn) < D) {
-    const unsigned col = 32 * wn + lrow;
+  }
+  __syncthreads();
+  float total[BLOCKS];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int trow = 32 * wm + 8 * (r / 4) + 4 * g + (r & 3);
-      const unsigned row = s0 + trow;
-      if (row < S && col < D) O[(size_t)row * p.ldo + col] = acc[r] * rowScale[kRows + trow];
+  for (int n = 0; n < BLOCKS; ++n) {
+    float highest = -FLT_MAX;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) highest = fmaxf(highest, wm[w][16 * n + l16]);
+    total[n] = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) total[n] += wl[w][16 * n + l16] * softmax_exp(wm[w][16 * n + l16] - highest);
+    const float scale = softmax_exp(m[n] - highest);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      v4f x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = o[n][e][r] * scale;
+      part[wave][n][r][lane] = x;
     }
+  }
+  __syncthreads();
+  const unsigned col = 16 * q + 4 * wave;
+  if (col >= D) return;
+#pragma unroll
+  for (int n = 0; n < BLOCKS; ++n) {
+    v4f sum = part[0][n][wave][lane];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) sum += part[w][n][wave][lane];
+    sum *= 1.0f / total[n];  // one division per row, as in the stand-alone softmax
+    const unsigned row = s0 + 16 * n + l16;
+    if (row < S) __builtin_memcpy(O + (size_t)row * p.ldo + col, &sum, 16);
   }
 }
 
@@ -884,7 +804,7 @@ extern "C" int tfcc_rocm_attention_f32(void* stream, const tfcc_rocm_attention_d
   p.outerQ = d->stride_q; p.outerK = d->stride_k; p.outerV = d->stride_v; p.outerO = d->stride_out;
   p.innerQ = d->inner_stride_q; p.innerK = d->inner_stride_k; p.innerV = d->inner_stride_v; p.innerO = d->inner_stride_out;
   p.batchInner = d->batch_inner;
-  // up to 128 keys: the scores of a row block in one piece; beyond: blocks of 128 keys with a running maximum and sum
+  // up to 128 keys: the scores of a row block in one piece; beyond: runs of keys with a maximum and a sum each
   const bool stream128 = d->t > (unsigned)kMaxT;
   int cus = 0;
   {
@@ -900,17 +820,20 @@ extern "C" int tfcc_rocm_attention_f32(void* stream, const tfcc_rocm_attention_d
   // 32 rows costs about 0.55 of a block of 64 (K and V are loaded per block).  16 x 12 heads of 128 rows: 17.8 against
   // 19.1 us with 32 rows; 32 x 12 heads: 30.5 against 27.7, so those keep 64.
   const unsigned long long heads = (unsigned long long)d->batch_outer * d->batch_inner;
-  const unsigned long long blocks64 = (d->s + 63) / 64 * heads, blocks32 = (d->s + 31) / 32 * heads;
+  const unsigned long long blocks64 = (d->s + 63) / 64 * heads, blocks32 = (d->s + 31) / 32 * heads,
+                           blocks16 = (d->s + 15) / 16 * heads;
   const unsigned long long perCu64 = (blocks64 + cus - 1) / cus, perCu32 = (blocks32 + cus - 1) / cus;
-  // (Beyond 128 keys a block of 32 rows walks all the keys again and holds one workgroup per SIMD's registers: it
-  // pays only while every block has a CU to itself - 12 heads of 384 rows 25.3 against 28.4 us, 48 heads 70.5 against 54.4.)
-  const bool rows32 = stream128 ? blocks32 <= (unsigned long long)cus : perCu32 * 55 < perCu64 * 100;
+  const bool rows32 = perCu32 * 55 < perCu64 * 100;
   // Blocks of 16 rows: up to 64 keys always (128 x 12 heads of 64 rows 37.1 -> 33.7 us, 32 x 12 12.3 -> 12.4, 64 x 12 of 32 11.2 -> 10.6).  Beyond, every
   // block walks twice the keys, which is faster where there are no more blocks than CUs or no more than with 32 rows
   // (2 x 12 heads of 128 rows 7.9 -> 6.2 us, 40 x 12 of 16 rows and 100 keys 10.4 -> 8.7), and not otherwise (4 x 12 of 100
   // rows 7.7 -> 8.4, 8 x 12 of 128 10.4 -> 11.6).
-  const bool rows16 = !stream128 && (d->t <= 64 || d->s <= 16 || (d->s + 15) / 16 * heads <= (unsigned long long)cus);
-  const unsigned rowsPerBlock = rows16 ? 16 : rows32 ? 32 : kRows;
+  const bool rows16 = !stream128 && (d->t <= 64 || d->s <= 16 || blocks16 <= (unsigned long long)cus);
+  // More than 128 keys: two blocks of 16 rows share the loads of K and V where there are six or more for each CU (8 x 12 heads of 512
+  // rows 72.8 -> 68.4 us, 16 x 12 of 384 86.0 -> 79.5, 8 x 12 of 384 45.7 -> 46.1); with fewer they fill the GPU less evenly (4 x 12
+  // of 384 27.2 -> 29.3, 12 of 1024 35.9 -> 43.8, 12 of 256 6.7 -> 9.6).
+  const bool single = stream128 && blocks16 < 6ull * cus;
+  const unsigned rowsPerBlock = rows16 || single ? 16 : stream128 || rows32 ? 32 : kRows;
   p.blocksS = (d->s + rowsPerBlock - 1) / rowsPerBlock;
   const unsigned long long total = (unsigned long long)p.blocksS * d->batch_outer * d->batch_inner;
   TFCC_REQUIRE(total < (1ull << 31) - 8, "attention: too many blocks");
@@ -924,11 +847,10 @@ extern "C" int tfcc_rocm_attention_f32(void* stream, const tfcc_rocm_attention_d
   p.mask = d->mask;
   p.outerM = d->stride_mask;
   p.innerM = d->inner_stride_mask;
-  constexpr size_t ldsBytes = (size_t)(kLdsFloats + 2 * kRows) * sizeof(float);
+  constexpr size_t ldsBytes = (size_t)kLdsFloats * sizeof(float);
   static_assert(ldsBytes <= 80 * 1024, "two workgroups per CU");
   constexpr size_t ldsBytes32 = (size_t)(kMaxT * kPitchV + 32 * kPitchS) * sizeof(float);
   static_assert(3 * ldsBytes32 <= 160 * 1024, "three workgroups per CU");
-  constexpr size_t ldsStream32 = ldsBytes32 + 2 * 32 * sizeof(float);
   static bool attrSet[16] = {};
   int dev = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));
@@ -938,15 +860,10 @@ extern "C" int tfcc_rocm_attention_f32(void* stream, const tfcc_rocm_attention_d
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsBytes));
     TFCC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_kernel<32>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsBytes32));
-    TFCC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_stream_kernel<64>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsBytes));
-    TFCC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_stream_kernel<32>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsStream32));
     attrSet[dev] = true;
   }
   if (rows16) hipLaunchKernelGGL(d->t <= 64 ? attention_rows16_kernel<64> : attention_rows16_kernel<128>, dim3(p.chunk * 8), dim3(256), 0, as_stream(stream), p);
-  else if (stream128 && rows32) hipLaunchKernelGGL(attention_stream_kernel<32>, dim3(p.chunk * 8), dim3(256), ldsStream32, as_stream(stream), p);
-  else if (stream128) hipLaunchKernelGGL(attention_stream_kernel<64>, dim3(p.chunk * 8), dim3(kThreads), ldsBytes, as_stream(stream), p);
+  else if (stream128) hipLaunchKernelGGL(single ? attention_stream_kernel<1> : attention_stream_kernel<2>, dim3(p.chunk * 8), dim3(256), 0, as_stream(stream), p);
   else if (rows32) hipLaunchKernelGGL(attention_kernel<32>, dim3(p.chunk * 8), dim3(256), ldsBytes32, as_stream(stream), p);
   else hipLaunchKernelGGL(attention_kernel<64>, dim3(p.chunk * 8), dim3(kThreads), ldsBytes, as_stream(stream), p);
   return check_launch("attention");
