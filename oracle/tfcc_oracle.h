@@ -4,7 +4,7 @@
  * This is a plain-C restatement of the arithmetic the reference performs on its
  * MKL (CPU) device for tfcc::blas::matmul, the quantized uint8 x int8 -> int32
  * matmul and the range-based quantize / requantize / dequantize steps.  It is
- * the checker the parity tests, the smoke test and the benchmark's CPU-baseline
+ * what the parity tests, the smoke test and the benchmark's CPU-baseline
  * leg compare the HIP kernels against.  Nothing on the product path may link,
  * load or call it.
  *
