@@ -146,3 +146,12 @@ def test_which_small_quantized_products_are_shared():
         subprocess.check_call(["make", "-C", os.path.join(ROOT, "wechat-tfcc_amd", "host"), "build/qgemm_small_plan_tests"])
     res = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
     assert res.returncode == 0 and "all passed" in res.stdout, res.stdout[-2000:]
+
+
+def test_words_of_the_one_launch_quantize():
+    """No word of an earlier call, and none that nobody has written, is taken for this call's (tests/cpp/quantize_exchange_tests.cpp)."""
+    exe = os.path.join(ROOT, "wechat-tfcc_amd", "host", "build", "quantize_exchange_tests")
+    if not os.path.exists(exe):
+        subprocess.check_call(["make", "-C", os.path.join(ROOT, "wechat-tfcc_amd", "host"), "build/quantize_exchange_tests"])
+    res = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert res.returncode == 0 and "all passed" in res.stdout, res.stdout[-2000:]

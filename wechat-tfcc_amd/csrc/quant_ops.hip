@@ -11,6 +11,7 @@
 
 #include "common.hpp"
 #include "quant_ops.hpp"
+#include "quantize_exchange.hpp"
 #include "stream_slots.hpp"
 
 namespace tfcc_rocm {
@@ -625,23 +626,28 @@ __global__ void minmax_finish_kernel(float* mn, float* mx) {
 }
 
 // A tensor that the GPU's registers hold, in one launch: a workgroup reads its part once, the workgroups tell one another its
-// minimum and maximum, and each quantizes what it has.  A word of the exchange is a value and the number of the call, which no
-// other call has, so a reader waits for this call's, and nothing has to be cleared or ordered.  Calls take turns with
+// minimum and maximum, and each quantizes what it has.  A word of the exchange is half a value and the number of the call
+// (quantize_exchange.hpp), so a reader waits for this call's, and nothing has to be cleared or ordered.  Calls take turns with
 // kTogetherTurns sets of words; one that meets another call in its set, on another stream, and one whose workgroups do not all run at
 // once is no worse off than slow: a workgroup that has waited kTogetherWait for the others reads all of the input itself, as
 // above.  (A replayed graph would find the words of its last replay, so a recorded call takes the launches below.)
 //
 // Bound by the launch, a store to memory and a load from it; with many elements to a workgroup by the reading.  us, the range
-// and the quantizing in a launch each before (up to 131072 elements the form above), input from memory: 77077 6.8 -> 5.1, 131072
-// 8.6 -> 5.2, 786432 8.9 -> 6.6, 2 M 11.3 -> 8.4, 8 M 21.1 -> 15.7 (17.5 with 64-bit whole numbers for every element).
+// and the quantizing in a launch each before (up to 131072 elements the form above), input from memory: 77077 7.3 -> 5.7, 131072
+// 9.0 -> 5.8, 786432 8.8 -> 7.5, 2 M 11.3 -> 9.9, 8 M 21.0 -> 17.5.  (With a whole value and 32 bits of the number to a word 5.5, 5.7, 7.3,
+// 9.4, 17.0; the four words of a workgroup in a load each 7.9, 10.4, 18.4 from 786432 on.)
 constexpr unsigned kTogetherWorkgroups = 256, kTogetherTurns = 256;
 constexpr unsigned kTogetherLimit = kTogetherWorkgroups * 1024 * 4 * 8;  // elements: 32 to a thread
 constexpr unsigned long long kTogetherWait = 20000;  // of the 100 MHz clock: 200 us
-__device__ unsigned long long togetherWords[kTogetherTurns * kTogetherWorkgroups * 2];
+__device__ __attribute__((aligned(64))) unsigned long long togetherWords[kTogetherTurns * kTogetherWorkgroups * quantize_exchange::kWords];
+
+typedef unsigned together_v4u __attribute__((ext_vector_type(4)));
+constexpr int kDeviceScope = 16;  // sc1, as a load of an atomic at device scope has it
 
 template <int QUADS>
 __global__ __launch_bounds__(1024) void quantize_together_kernel(const float* in, size_t total, void* out, int outType, float* mnOut,
-                                                                 float* mxOut, unsigned call) {
+                                                                 float* mxOut, unsigned long long number) {
+  namespace exchange = quantize_exchange;
   __shared__ float shMn[16], shMx[16];
   __shared__ int alone;
   const size_t total4 = total / 4, first = (size_t)blockIdx.x * (1024 * QUADS) + threadIdx.x;
@@ -678,20 +684,31 @@ __global__ __launch_bounds__(1024) void quantize_together_kernel(const float* in
     }
   };
   join();
-  unsigned long long* const words = togetherWords + call % kTogetherTurns * (kTogetherWorkgroups * 2);
+  unsigned long long* const words = togetherWords + number % kTogetherTurns * (kTogetherWorkgroups * exchange::kWords);
   if (threadIdx.x == 0) {
-    const unsigned long long number = (unsigned long long)call << 32;
-    __hip_atomic_store(words + 2 * blockIdx.x, number | __float_as_uint(mn), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(words + 2 * blockIdx.x + 1, number | __float_as_uint(mx), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (unsigned w = 0; w < exchange::kWords; ++w)
+      __hip_atomic_store(words + exchange::kWords * blockIdx.x + w, exchange::word_of(number, __float_as_uint(w < 2 ? mn : mx), w % 2 != 0),
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (threadIdx.x < gridDim.x) {
     const unsigned long long start = wall_clock64();
+    const __amdgpu_buffer_rsrc_t source = __builtin_amdgcn_make_buffer_rsrc(words, 0, kTogetherWorkgroups * exchange::kWords * 8, 0x00020000);
     while (true) {
-      const unsigned long long a = __hip_atomic_load(words + 2 * threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const unsigned long long b = __hip_atomic_load(words + 2 * threadIdx.x + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if ((unsigned)(a >> 32) == call && (unsigned)(b >> 32) == call) {
-        mn = fminf(mn, __uint_as_float((unsigned)a));
-        mx = fmaxf(mx, __uint_as_float((unsigned)b));
+      asm volatile("" ::: "memory");  // the words are asked for again each time
+      unsigned long long theirs[exchange::kWords];
+#pragma unroll
+      for (unsigned w = 0; w < exchange::kWords; w += 2) {
+        const together_v4u two = __builtin_amdgcn_raw_buffer_load_b128(source, 8 * (exchange::kWords * threadIdx.x + w), 0, kDeviceScope);
+        theirs[w] = two[0] | (unsigned long long)two[1] << 32;
+        theirs[w + 1] = two[2] | (unsigned long long)two[3] << 32;
+      }
+      bool all = true;
+#pragma unroll
+      for (unsigned w = 0; w < exchange::kWords; ++w) all = all && exchange::belongs_to(theirs[w], number);
+      if (all) {
+        mn = fminf(mn, __uint_as_float(exchange::value_of(theirs[0], theirs[1])));
+        mx = fmaxf(mx, __uint_as_float(exchange::value_of(theirs[2], theirs[3])));
         break;
       }
       if (wall_clock64() - start > kTogetherWait) {
@@ -756,13 +773,14 @@ unsigned stream_grid(size_t total4) {
 // launch of its own.
 StreamSlots gArrivalSlots(kArrivalSlots);
 
-std::atomic<unsigned> gTogetherCalls{1};
+std::atomic<unsigned long long> gTogetherCalls{0};
 
 // as many workgroups as there may be: a thread's loads are all on their way at once, and the words are read side by side
 void launch_together(hipStream_t s, const float* in, uint64_t total, void* out, int outType, float* mn, float* mx) {
-  const unsigned call = gTogetherCalls.fetch_add(1, std::memory_order_relaxed), pieces = (unsigned)((total + 4095) / 4096);
+  const unsigned long long number = quantize_exchange::number_of(gTogetherCalls.fetch_add(1, std::memory_order_relaxed));
+  const unsigned pieces = (unsigned)((total + 4095) / 4096);
   auto launch = [&](auto kernel, unsigned quads) {
-    hipLaunchKernelGGL(kernel, dim3((pieces + quads - 1) / quads), dim3(1024), 0, s, in, (size_t)total, out, outType, mn, mx, call);
+    hipLaunchKernelGGL(kernel, dim3((pieces + quads - 1) / quads), dim3(1024), 0, s, in, (size_t)total, out, outType, mn, mx, number);
   };
   if (pieces <= kTogetherWorkgroups) launch(quantize_together_kernel<1>, 1);
   else if (pieces <= 2 * kTogetherWorkgroups) launch(quantize_together_kernel<2>, 2);
