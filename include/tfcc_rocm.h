@@ -297,6 +297,10 @@ int tfcc_rocm_quantize(void* stream, const float* in, uint64_t total, const floa
 /* quantize with the range taken from the data: writes *min_v / *max_v (device) first */
 int tfcc_rocm_quantize_minmax(void* stream, const float* in, uint64_t total, void* out,
                               int out_type, float* min_v, float* max_v);
+/* the same with a limit to how long the workgroups of its one-launch form wait for one another before each does others' share
+ * of finding the range as well (0: at once); the results are the same */
+int tfcc_rocm_quantize_minmax_wait(void* stream, const float* in, uint64_t total, void* out,
+                                   int out_type, float* min_v, float* max_v, unsigned wait_us);
 
 /* ---------------------------------------------------------------------------------------------
  * The element-wise neighbours of matmul inside one transformer encoder layer (fp32).

@@ -139,3 +139,20 @@ def test_captured_quantize_of_the_data_s_own_range(pkg, T, total):
         return min(times)
 
     assert best(graph.replay) <= 2.0 * best(lambda: pkg.quantize(t, torch.uint8)) + 20.0
+
+
+@pytest.mark.parametrize("total", [40961, (1 << 20) - 3, (2 << 20) + 2, (4 << 20) + 3, 8 << 20])
+@pytest.mark.parametrize("wait_us", [0, 1])
+def test_quantize_whose_workgroups_do_not_wait(pkg, T, total, wait_us):
+    """a workgroup that has waited long enough finds the range of the parts that are missing itself: one, two, four and eight
+    pieces to a thread, the extremes and a NaN in the first and the last part"""
+    import torch
+    x = np.random.default_rng(total).normal(0.1, 2.0, total).astype(np.float32)
+    x[5], x[-1], x[total // 2] = 17.0, -31.0, np.nan
+    data, want = T.t(x), O.quantize(x, -31.0, 17.0, "uint8")
+    for _ in range(3):
+        q, low, high = torch.zeros(total, dtype=torch.uint8, device="cuda"), T.f1(0.0), T.f1(0.0)
+        pkg.check(pkg.lib().tfcc_rocm_quantize_minmax_wait(pkg._stream(), pkg._ptr(data), total, pkg._ptr(q), pkg._type_code(torch.uint8),
+                                                           pkg._ptr(low), pkg._ptr(high), wait_us))
+        assert (float(T.n(low)[0]), float(T.n(high)[0])) == (-31.0, 17.0)
+        assert np.array_equal(T.n(q), want)

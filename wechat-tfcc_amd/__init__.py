@@ -117,6 +117,7 @@ SYMBOLS = {
     "tfcc_rocm_dequantize": (_I, [_VP, _VP, _I, _U64, _VP, _VP, _VP]),
     "tfcc_rocm_quantize": (_I, [_VP, _VP, _U64, _VP, _VP, _VP, _I]),
     "tfcc_rocm_quantize_minmax": (_I, [_VP, _VP, _U64, _VP, _I, _VP, _VP]),
+    "tfcc_rocm_quantize_minmax_wait": (_I, [_VP, _VP, _U64, _VP, _I, _VP, _VP, _U]),
     "tfcc_rocm_softmax_f32": (_I, [_VP, _VP, _U64, _U, _VP]),
     "tfcc_rocm_layer_norm_f32": (_I, [_VP, _VP, _VP, _VP, _F, _U64, _U, _VP]),
     "tfcc_rocm_gelu_accurate_f32": (_I, [_VP, _VP, _U64, _VP]),

@@ -628,17 +628,24 @@ __global__ void minmax_finish_kernel(float* mn, float* mx) {
 // A tensor that the GPU's registers hold, in one launch: a workgroup reads its part once, the workgroups tell one another its
 // minimum and maximum, and each quantizes what it has.  A word of the exchange is half a value and the number of the call
 // (quantize_exchange.hpp), so a reader waits for this call's, and nothing has to be cleared or ordered.  Calls take turns with
-// kTogetherTurns sets of words; one that meets another call in its set, on another stream, and one whose workgroups do not all run at
-// once is no worse off than slow: a workgroup that has waited kTogetherWait for the others reads all of the input itself, as
-// above.  (A replayed graph would find the words of its last replay, so a recorded call takes the launches below.)
+// kTogetherTurns sets of words.
+//
+// Workgroups that find no room on the GPU beside other work, and words that another call in the same set, on another stream, has
+// overwritten, are not waited for: a workgroup that has waited `waitTicks` reads a part that is missing itself and tells
+// the others, each another one as far as there are as many, until nothing is missing.  So nobody needs anybody, every round
+// of that has one part less to look for, and the input is read about twice, as with a launch for the range.  (A replayed graph would
+// find the words of its last replay, so a recorded call takes the launches below.)
 //
 // Bound by the launch, a store to memory and a load from it; with many elements to a workgroup by the reading.  us, the range
-// and the quantizing in a launch each before (up to 131072 elements the form above), input from memory: 77077 7.3 -> 5.7, 131072
-// 9.0 -> 5.8, 786432 8.8 -> 7.5, 2 M 11.3 -> 9.9, 8 M 21.0 -> 17.5.  (With a whole value and 32 bits of the number to a word 5.5, 5.7, 7.3,
-// 9.4, 17.0; the four words of a workgroup in a load each 7.9, 10.4, 18.4 from 786432 on.)
+// and the quantizing in a launch each before (up to 131072 elements the form above), input from memory: 77077 7.3 -> 5.4, 131072
+// 9.0 -> 5.4, 786432 8.8 -> 6.8, 2 M 11.3 -> 8.9, 8 M 21.0 -> 16.9.  (A workgroup's words stored one after the other by one thread: 7.8,
+// 9.9, 17.9 from 786432 on, and 7.9, 10.4, 18.4 with a load for each as well; minima and maxima in arrays of their own 7.3, 9.3, 17.4.)
+// 8 M elements beside 8192 x 4096 x 8192 products on another stream, whose workgroups leave room as they end: 358 us with a launch for
+// the range, 369 here, and 3300 where a workgroup that had waited read all of the input itself.
 constexpr unsigned kTogetherWorkgroups = 256, kTogetherTurns = 256;
 constexpr unsigned kTogetherLimit = kTogetherWorkgroups * 1024 * 4 * 8;  // elements: 32 to a thread
-constexpr unsigned long long kTogetherWait = 20000;  // of the 100 MHz clock: 200 us
+constexpr unsigned kTogetherWait = 10;  // us (8 M elements beside other work: 366 us with 5, 369 with 10, 376 with 20, 402 with 50, 549 with 200; alone 5
+// are enough and 2 too few: 25 instead of 14 in cache)
 __device__ __attribute__((aligned(64))) unsigned long long togetherWords[kTogetherTurns * kTogetherWorkgroups * quantize_exchange::kWords];
 
 typedef unsigned together_v4u __attribute__((ext_vector_type(4)));
@@ -646,84 +653,115 @@ constexpr int kDeviceScope = 16;  // sc1, as a load of an atomic at device scope
 
 template <int QUADS>
 __global__ __launch_bounds__(1024) void quantize_together_kernel(const float* in, size_t total, void* out, int outType, float* mnOut,
-                                                                 float* mxOut, unsigned long long number) {
+                                                                 float* mxOut, unsigned long long number, unsigned long long waitTicks) {
   namespace exchange = quantize_exchange;
+  constexpr float kNoMinimum = 3.402823466e+38f, kNoMaximum = -3.402823466e+38f;
   __shared__ float shMn[16], shMx[16];
-  __shared__ int alone;
+  __shared__ unsigned long long shMissing[kTogetherWorkgroups / 64];
   const size_t total4 = total / 4, first = (size_t)blockIdx.x * (1024 * QUADS) + threadIdx.x;
   const unsigned rest = (unsigned)(total & 3u);
-  if (threadIdx.x == 0) alone = 0;
-  float v[QUADS][4];
-  float mn = 3.402823466e+38f, mx = -3.402823466e+38f;
-#pragma unroll
-  for (int u = 0; u < QUADS; ++u) {
-    const size_t i = first + u * 1024;
-    if (i < total4) __builtin_memcpy(v[u], in + i * 4, 16);
+  auto read = [&](float (&v)[4], size_t i) __attribute__((always_inline)) {  // NaN behind the end, which a range passes over
+    if (i < total4) __builtin_memcpy(v, in + i * 4, 16);
     else
 #pragma unroll
-      for (unsigned e = 0; e < 4; ++e) v[u][e] = i == total4 && e < rest ? in[i * 4 + e] : __builtin_nanf("");
-  }
-#pragma unroll
-  for (int u = 0; u < QUADS; ++u) {  // (a NaN is passed over)
-    mn = fminf(fminf(mn, fminf(v[u][0], v[u][1])), fminf(v[u][2], v[u][3]));
-    mx = fmaxf(fmaxf(mx, fmaxf(v[u][0], v[u][1])), fmaxf(v[u][2], v[u][3]));
-  }
-  auto join = [&]() {  // over the workgroup
-    mn = wave_min(mn);
-    mx = wave_max(mx);
+      for (unsigned e = 0; e < 4; ++e) v[e] = i == total4 && e < rest ? in[i * 4 + e] : __builtin_nanf("");
+  };
+  auto widen = [](float& low, float& high, const float (&v)[4]) __attribute__((always_inline)) {
+    low = fminf(fminf(low, fminf(v[0], v[1])), fminf(v[2], v[3]));
+    high = fmaxf(fmaxf(high, fmaxf(v[0], v[1])), fmaxf(v[2], v[3]));
+  };
+  auto join = [&](float& low, float& high, auto&& beside) __attribute__((always_inline)) {  // over the workgroup
+    low = wave_min(low);
+    high = wave_max(high);
     __syncthreads();  // the last join's values are read
     if ((threadIdx.x & 63) == 0) {
-      shMn[threadIdx.x >> 6] = mn;
-      shMx[threadIdx.x >> 6] = mx;
+      shMn[threadIdx.x >> 6] = low;
+      shMx[threadIdx.x >> 6] = high;
+      beside();
     }
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < 16; ++w) {
-      mn = fminf(mn, shMn[w]);
-      mx = fmaxf(mx, shMx[w]);
+      low = fminf(low, shMn[w]);
+      high = fmaxf(high, shMx[w]);
     }
   };
-  join();
+  float v[QUADS][4], mn = kNoMinimum, mx = kNoMaximum;
+#pragma unroll
+  for (int u = 0; u < QUADS; ++u) read(v[u], first + u * 1024);
+#pragma unroll
+  for (int u = 0; u < QUADS; ++u) widen(mn, mx, v[u]);
+  join(mn, mx, [] {});
+
   unsigned long long* const words = togetherWords + number % kTogetherTurns * (kTogetherWorkgroups * exchange::kWords);
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (unsigned w = 0; w < exchange::kWords; ++w)
-      __hip_atomic_store(words + exchange::kWords * blockIdx.x + w, exchange::word_of(number, __float_as_uint(w < 2 ? mn : mx), w % 2 != 0),
+  auto tell = [&](unsigned workgroup, float low, float high) __attribute__((always_inline)) {  // a thread a word, in one store
+    const unsigned w = threadIdx.x;
+    if (w < exchange::kWords)
+      __hip_atomic_store(words + exchange::kWords * workgroup + w, exchange::word_of(number, __float_as_uint(w < 2 ? low : high), w % 2 != 0),
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  if (threadIdx.x < gridDim.x) {
+  };
+  tell(blockIdx.x, mn, mx);
+
+  // Thread i hears workgroup i.
+  const __amdgpu_buffer_rsrc_t source = __builtin_amdgcn_make_buffer_rsrc(words, 0, kTogetherWorkgroups * exchange::kWords * 8, 0x00020000);
+  bool heard = threadIdx.x >= gridDim.x;
+  auto ask = [&]() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");  // the words are asked for again each time
+    unsigned long long theirs[exchange::kWords];
+#pragma unroll
+    for (unsigned w = 0; w < exchange::kWords; w += 2) {
+      const together_v4u two = __builtin_amdgcn_raw_buffer_load_b128(source, 8 * (exchange::kWords * threadIdx.x + w), 0, kDeviceScope);
+      theirs[w] = two[0] | (unsigned long long)two[1] << 32;
+      theirs[w + 1] = two[2] | (unsigned long long)two[3] << 32;
+    }
+    heard = true;
+#pragma unroll
+    for (unsigned w = 0; w < exchange::kWords; ++w) heard = heard && exchange::belongs_to(theirs[w], number);
+    if (heard) {
+      mn = fminf(mn, __uint_as_float(exchange::value_of(theirs[0], theirs[1])));
+      mx = fmaxf(mx, __uint_as_float(exchange::value_of(theirs[2], theirs[3])));
+    }
+  };
+  if (!heard) {
     const unsigned long long start = wall_clock64();
-    const __amdgpu_buffer_rsrc_t source = __builtin_amdgcn_make_buffer_rsrc(words, 0, kTogetherWorkgroups * exchange::kWords * 8, 0x00020000);
-    while (true) {
-      asm volatile("" ::: "memory");  // the words are asked for again each time
-      unsigned long long theirs[exchange::kWords];
-#pragma unroll
-      for (unsigned w = 0; w < exchange::kWords; w += 2) {
-        const together_v4u two = __builtin_amdgcn_raw_buffer_load_b128(source, 8 * (exchange::kWords * threadIdx.x + w), 0, kDeviceScope);
-        theirs[w] = two[0] | (unsigned long long)two[1] << 32;
-        theirs[w + 1] = two[2] | (unsigned long long)two[3] << 32;
-      }
-      bool all = true;
-#pragma unroll
-      for (unsigned w = 0; w < exchange::kWords; ++w) all = all && exchange::belongs_to(theirs[w], number);
-      if (all) {
-        mn = fminf(mn, __uint_as_float(exchange::value_of(theirs[0], theirs[1])));
-        mx = fmaxf(mx, __uint_as_float(exchange::value_of(theirs[2], theirs[3])));
-        break;
-      }
-      if (wall_clock64() - start > kTogetherWait) {
-        alone = 1;
-        break;
-      }
-    }
+    do ask();
+    while (!heard && wall_clock64() - start < waitTicks);
   }
-  join();
-  if (alone) {  // the same for the whole workgroup
-    for (size_t i = threadIdx.x; i < total; i += 1024) {
-      mn = fminf(mn, in[i]);
-      mx = fmaxf(mx, in[i]);
+  while (true) {  // one part less is missing each time
+    const unsigned long long silent = __ballot(!heard);
+    join(mn, mx, [&] {
+      if (threadIdx.x < kTogetherWorkgroups) shMissing[threadIdx.x >> 6] = silent;
+    });
+    unsigned missing = 0;
+#pragma unroll
+    for (unsigned w = 0; w < kTogetherWorkgroups / 64; ++w) missing += __popcll(shMissing[w]);
+    if (missing == 0) break;  // the same for the whole workgroup
+    unsigned part = 0, skip = blockIdx.x % missing;
+    for (unsigned w = 0; w < kTogetherWorkgroups / 64; ++w) {
+      unsigned long long left = shMissing[w];
+      const unsigned here = __popcll(left);
+      if (skip >= here) {
+        skip -= here;
+        continue;
+      }
+      while (skip-- > 0) left &= left - 1;
+      part = 64 * w + __builtin_ctzll(left);
+      break;
     }
-    join();
+    float low = kNoMinimum, high = kNoMaximum;
+    for (int u = 0; u < QUADS; ++u) {
+      float theirs[4];
+      read(theirs, (size_t)part * (1024 * QUADS) + threadIdx.x + u * 1024);
+      widen(low, high, theirs);
+    }
+    join(low, high, [] {});
+    tell(part, low, high);
+    if (threadIdx.x == part) {
+      heard = true;
+      mn = fminf(mn, low);
+      mx = fmaxf(mx, high);
+    }
+    if (!heard) ask();
   }
   if (first == 0) {
     *mnOut = mn;
@@ -776,11 +814,12 @@ StreamSlots gArrivalSlots(kArrivalSlots);
 std::atomic<unsigned long long> gTogetherCalls{0};
 
 // as many workgroups as there may be: a thread's loads are all on their way at once, and the words are read side by side
-void launch_together(hipStream_t s, const float* in, uint64_t total, void* out, int outType, float* mn, float* mx) {
+void launch_together(hipStream_t s, const float* in, uint64_t total, void* out, int outType, float* mn, float* mx, unsigned waitUs) {
   const unsigned long long number = quantize_exchange::number_of(gTogetherCalls.fetch_add(1, std::memory_order_relaxed));
   const unsigned pieces = (unsigned)((total + 4095) / 4096);
   auto launch = [&](auto kernel, unsigned quads) {
-    hipLaunchKernelGGL(kernel, dim3((pieces + quads - 1) / quads), dim3(1024), 0, s, in, (size_t)total, out, outType, mn, mx, number);
+    hipLaunchKernelGGL(kernel, dim3((pieces + quads - 1) / quads), dim3(1024), 0, s, in, (size_t)total, out, outType, mn, mx, number,
+                       waitUs * 100ull);  // of the 100 MHz clock
   };
   if (pieces <= kTogetherWorkgroups) launch(quantize_together_kernel<1>, 1);
   else if (pieces <= 2 * kTogetherWorkgroups) launch(quantize_together_kernel<2>, 2);
@@ -937,6 +976,11 @@ int tfcc_rocm_quantize(void* stream, const float* in, uint64_t total, const floa
 
 int tfcc_rocm_quantize_minmax(void* stream, const float* in, uint64_t total, void* out,
                               int out_type, float* min_v, float* max_v) {
+  return tfcc_rocm_quantize_minmax_wait(stream, in, total, out, out_type, min_v, max_v, kTogetherWait);
+}
+
+int tfcc_rocm_quantize_minmax_wait(void* stream, const float* in, uint64_t total, void* out,
+                                   int out_type, float* min_v, float* max_v, unsigned wait_us) {
   TFCC_REQUIRE(in && out && min_v && max_v, "quantize: null argument");
   TFCC_REQUIRE(total > 0, "quantize: empty tensor");
   TFCC_REQUIRE(valid_type(out_type), "quantize: bad type code");
@@ -946,7 +990,7 @@ int tfcc_rocm_quantize_minmax(void* stream, const float* in, uint64_t total, voi
   const uintptr_t inAt = (uintptr_t)in, outAt = (uintptr_t)out;
   const bool apart = inAt + 4 * total <= outAt || outAt + total * (int_range(out_type).bits / 8) <= inAt;
   if (apart && total > kWholeBest && total <= kTogetherLimit && runs_in_order_now(s)) {
-    launch_together(s, in, total, out, out_type, min_v, max_v);
+    launch_together(s, in, total, out, out_type, min_v, max_v, wait_us);
     return check_launch("quantize");
   }
   if (apart && total <= kWholeLimit) {
