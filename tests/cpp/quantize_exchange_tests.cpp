@@ -1,5 +1,5 @@
 // The words of the one-launch quantize (wechat-tfcc_amd/csrc/quantize_exchange.hpp), on the host: no word of another call, however
-// many calls ago, and none that nobody has written is taken for this call's.  No GPU.
+// many calls ago, and none that nobody has written is taken for this call's; and that every workgroup has a CU.  No GPU.
 #include <cstdio>
 #include <initializer_list>
 
@@ -28,6 +28,13 @@ int main() {
       EXPECT(belongs_to(low, number) && belongs_to(high, number) && value_of(low, high) == value);
     }
   }
+  for (int cus : {-1, 0, 1, 32, 64, 128, 255, 256, 304})
+    for (unsigned long long total : {1ull, 4096ull, 4097ull, 40961ull, 32ull * 4096, 128ull * 4096, 128ull * 4096 + 1, 1ull << 20, (1ull << 20) + 1,
+                                     4ull << 20, (4ull << 20) + 1, 8ull << 20, (8ull << 20) + 1, 1ull << 40}) {
+      const unsigned quads = quads_of(total, cus), room = cus <= 0 ? 0 : cus < 256 ? cus : 256;
+      if (quads == 0) EXPECT(total > 8ull * kPiece * room);
+      else EXPECT(workgroups(total, quads) <= room && workgroups(total, quads) * quads * kPiece >= total && (quads == 1 || workgroups(total, quads / 2) > room));
+    }
   if (failures == 0) std::printf("quantize exchange: all passed\n");
   return failures != 0;
 }

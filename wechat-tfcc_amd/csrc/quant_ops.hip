@@ -642,8 +642,7 @@ __global__ void minmax_finish_kernel(float* mn, float* mx) {
 // 9.9, 17.9 from 786432 on, and 7.9, 10.4, 18.4 with a load for each as well; minima and maxima in arrays of their own 7.3, 9.3, 17.4.)
 // 8 M elements beside 8192 x 4096 x 8192 products on another stream, whose workgroups leave room as they end: 358 us with a launch for
 // the range, 369 here, and 3300 where a workgroup that had waited read all of the input itself.
-constexpr unsigned kTogetherWorkgroups = 256, kTogetherTurns = 256;
-constexpr unsigned kTogetherLimit = kTogetherWorkgroups * 1024 * 4 * 8;  // elements: 32 to a thread
+constexpr unsigned kTogetherWorkgroups = quantize_exchange::kWorkgroups, kTogetherTurns = 256;
 constexpr unsigned kTogetherWait = 10;  // us (8 M elements beside other work: 366 us with 5, 369 with 10, 376 with 20, 402 with 50, 549 with 200; alone 5
 // are enough and 2 too few: 25 instead of 14 in cache)
 __device__ __attribute__((aligned(64))) unsigned long long togetherWords[kTogetherTurns * kTogetherWorkgroups * quantize_exchange::kWords];
@@ -813,18 +812,35 @@ StreamSlots gArrivalSlots(kArrivalSlots);
 
 std::atomic<unsigned long long> gTogetherCalls{0};
 
-// as many workgroups as there may be: a thread's loads are all on their way at once, and the words are read side by side
-void launch_together(hipStream_t s, const float* in, uint64_t total, void* out, int outType, float* mn, float* mx, unsigned waitUs) {
+// of the current device, asked for once; 0: unknown
+int compute_units() {
+  static std::atomic<int> known[16];
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  if (dev >= 0 && dev < 16) cus = known[dev].load(std::memory_order_relaxed);
+  if (cus != 0) return cus;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  if (dev >= 0 && dev < 16) known[dev].store(cus, std::memory_order_relaxed);
+  return cus;
+}
+
+void launch_together(hipStream_t s, unsigned quads, const float* in, uint64_t total, void* out, int outType, float* mn, float* mx,
+                     unsigned waitUs) {
   const unsigned long long number = quantize_exchange::number_of(gTogetherCalls.fetch_add(1, std::memory_order_relaxed));
-  const unsigned pieces = (unsigned)((total + 4095) / 4096);
-  auto launch = [&](auto kernel, unsigned quads) {
-    hipLaunchKernelGGL(kernel, dim3((pieces + quads - 1) / quads), dim3(1024), 0, s, in, (size_t)total, out, outType, mn, mx, number,
-                       waitUs * 100ull);  // of the 100 MHz clock
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)quantize_exchange::workgroups(total, quads)), dim3(1024), 0, s, in, (size_t)total, out, outType,
+                       mn, mx, number, waitUs * 100ull);  // of the 100 MHz clock
   };
-  if (pieces <= kTogetherWorkgroups) launch(quantize_together_kernel<1>, 1);
-  else if (pieces <= 2 * kTogetherWorkgroups) launch(quantize_together_kernel<2>, 2);
-  else if (pieces <= 4 * kTogetherWorkgroups) launch(quantize_together_kernel<4>, 4);
-  else launch(quantize_together_kernel<8>, 8);
+  if (quads == 1) launch(quantize_together_kernel<1>);
+  else if (quads == 2) launch(quantize_together_kernel<2>);
+  else if (quads == 4) launch(quantize_together_kernel<4>);
+  else launch(quantize_together_kernel<8>);
 }
 
 bool valid_type(int t) { return t >= TFCC_ROCM_S8 && t <= TFCC_ROCM_U32; }
@@ -989,8 +1005,9 @@ int tfcc_rocm_quantize_minmax_wait(void* stream, const float* in, uint64_t total
   // every element where it was read.
   const uintptr_t inAt = (uintptr_t)in, outAt = (uintptr_t)out;
   const bool apart = inAt + 4 * total <= outAt || outAt + total * (int_range(out_type).bits / 8) <= inAt;
-  if (apart && total > kWholeBest && total <= kTogetherLimit && runs_in_order_now(s)) {
-    launch_together(s, in, total, out, out_type, min_v, max_v, wait_us);
+  const unsigned quads = apart && total > kWholeBest ? quantize_exchange::quads_of(total, compute_units()) : 0;
+  if (quads != 0 && runs_in_order_now(s)) {
+    launch_together(s, quads, in, total, out, out_type, min_v, max_v, wait_us);
     return check_launch("quantize");
   }
   if (apart && total <= kWholeLimit) {
@@ -1008,7 +1025,7 @@ int tfcc_rocm_quantize_minmax_wait(void* stream, const float* in, uint64_t total
     TFCC_HIP_CHECK(hipGetDevice(&dev));
     if (gArrivalSlots.of(dev, s, &slot)) {
       // one workgroup per CU at most: every arrival costs an atomic on one word and a write-back (192 workgroups of 256
-      // threads for 786432 elements: 6 us, 48 of 1024: 5.6)
+      // threads for 786432 elements: 6 us, 48 of 1024: 5.6; so few come here on a GPU with few CUs, the form above takes them on a whole one)
       const unsigned blocks = total >= 256u * 16384u ? 256u : (unsigned)((total + 16383) / 16384);
       hipLaunchKernelGGL((minmax_partial_kernel<16, true>), dim3(blocks), dim3(1024), 0, s, in, (size_t)total, partials, slot,
                          min_v, max_v);

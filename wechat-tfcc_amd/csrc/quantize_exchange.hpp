@@ -1,5 +1,5 @@
-// The words by which the workgroups of a one-launch quantize tell one another their minimum and maximum.  Plain functions of
-// integers, compiled for the kernel and for the tests.
+// A quantize in one launch whose workgroups tell one another their minimum and maximum: the words by which they do, and how
+// many workgroups there are.  Plain functions of integers, compiled for the kernel, its launch and the tests.
 #pragma once
 
 namespace tfcc_rocm {
@@ -18,6 +18,22 @@ constexpr unsigned long long word_of(unsigned long long number, unsigned value, 
 constexpr bool belongs_to(unsigned long long word, unsigned long long number) { return word >> 16 == number; }
 constexpr unsigned value_of(unsigned long long low, unsigned long long high) {
   return (unsigned)(low & 0xffffu) | (unsigned)(high & 0xffffu) << 16;
+}
+
+constexpr unsigned kWorkgroups = 256;  // at most
+constexpr unsigned kPiece = 4096;      // elements that 1024 threads read with a 16-byte load each
+
+constexpr unsigned long long workgroups(unsigned long long total, unsigned quads) {
+  return (total + (unsigned long long)kPiece * quads - 1) / ((unsigned long long)kPiece * quads);
+}
+// Loads of a thread: one, two, four or eight, as few as leave a CU of this GPU for every workgroup (as many workgroups as there
+// may be: the loads of a thread are all on their way at once, and the words are read side by side); 0: not even with eight.  A
+// workgroup that finds no CU keeps the others waiting, which on a part of a partitioned GPU would be every call.
+constexpr unsigned quads_of(unsigned long long total, int cus) {
+  const unsigned long long room = cus <= 0 ? 0 : (unsigned)cus < kWorkgroups ? (unsigned)cus : kWorkgroups;
+  for (unsigned quads = 1; quads <= 8; quads *= 2)
+    if (workgroups(total, quads) <= room) return quads;
+  return 0;
 }
 
 }  // namespace quantize_exchange
