@@ -109,7 +109,8 @@ def test_quantize_on_several_streams_and_under_capture(pkg, T):
 @pytest.mark.parametrize("total", [LIMIT + 1, LIMIT + 16384, 64 * 16384 + 3, 256 * 16384 - 1, 256 * 16384 + 5, 16 << 20])
 def test_captured_quantize_of_the_data_s_own_range(pkg, T, total):
     """Recorded in a graph: the same bytes as outside, and no slower than a launch more (with an atomic per wavefront on the
-    two results 16 M elements took twelve times as long)."""
+    two results 16 M elements took twelve times as long).  A replay of three launches takes 20 to 50 us whatever they do, most
+    of it the host's, and now and then twice that; so two such replays of launches that do nothing are added to the bound."""
     import torch
     x = np.random.default_rng(total).normal(0.0, 3.0, total).astype(np.float32)
     x[0], x[-1] = -40.0, 41.0
@@ -127,9 +128,14 @@ def test_captured_quantize_of_the_data_s_own_range(pkg, T, total):
             assert torch.equal(c, e)
         assert np.array_equal(T.n(captured[0]), want)
 
+    idle, one = torch.cuda.CUDAGraph(), torch.zeros(1, device="cuda")
+    with torch.cuda.graph(idle):
+        for _ in range(3):
+            one.zero_()
+
     def best(f):
         times = []
-        for _ in range(7):
+        for _ in range(15):
             start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             start.record()
             f()
@@ -138,7 +144,7 @@ def test_captured_quantize_of_the_data_s_own_range(pkg, T, total):
             times.append(start.elapsed_time(end) * 1e3)
         return min(times)
 
-    assert best(graph.replay) <= 2.0 * best(lambda: pkg.quantize(t, torch.uint8)) + 20.0
+    assert best(graph.replay) <= 2.0 * best(lambda: pkg.quantize(t, torch.uint8)) + 2.0 * best(idle.replay)
 
 
 @pytest.mark.parametrize("total", [40961, (1 << 20) - 3, (2 << 20) + 2, (4 << 20) + 3, 8 << 20])
