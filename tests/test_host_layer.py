@@ -155,3 +155,12 @@ def test_words_of_the_one_launch_quantize():
         subprocess.check_call(["make", "-C", os.path.join(ROOT, "wechat-tfcc_amd", "host"), "build/quantize_exchange_tests"])
     res = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
     assert res.returncode == 0 and "all passed" in res.stdout, res.stdout[-2000:]
+
+
+def test_where_uploads_are_cut():
+    """Every piece begins on a line, whatever the sizes of the inputs in front of it (tests/cpp/upload_cut_tests.cpp)."""
+    exe = os.path.join(ROOT, "wechat-tfcc_amd", "host", "build", "upload_cut_tests")
+    if not os.path.exists(exe):
+        subprocess.check_call(["make", "-C", os.path.join(ROOT, "wechat-tfcc_amd", "host"), "build/upload_cut_tests"])
+    res = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert res.returncode == 0 and "all passed" in res.stdout, res.stdout[-2000:]

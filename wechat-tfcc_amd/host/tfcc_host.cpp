@@ -10,6 +10,7 @@
 #include "tfcc_rocm.h"
 #include "tfcc_layers.h"
 #include "tfcc_rocm_device.h"
+#include "upload_cut.h"
 
 namespace tfcc {
 
@@ -1240,14 +1241,11 @@ bool ROCMSession::reserveStaging(size_t bytes) {
 }
 
 // 3 MB: 106 us in one copy from pageable memory.  Here the GPU fetches one chunk while the host puts the next one down,
-// and nothing waits: the kernels that read the data are behind it on the stream.  The first chunk is short so that the
-// GPU starts early, the later ones long because each costs a launch, but no longer than the GPU has work for meanwhile;
-// small inputs share a launch.  An encoder layer of 8 x 128 x 768 served, us, by the first and the longest chunk in KB: 256 and
-// 1024 308, 256 and 512 297, 256 and 256 309, 384 and 768 294.
+// and nothing waits: the kernels that read the data are behind it on the stream.
 void ROCMSession::upload(const std::vector<HostWrite>& writes) {
   if (_recording) throw RuntimeError("upload: not possible while the session's stream records a graph");
   size_t total = 0;
-  for (const HostWrite& w : writes) total += (w.bytes + 63) / 64 * 64;
+  for (const HostWrite& w : writes) total += UploadCut::padded(w.bytes);
   if (total == 0) return;
   if (!reserveStaging(_stagingUsed + total)) {
     for (const HostWrite& w : writes)
@@ -1255,13 +1253,12 @@ void ROCMSession::upload(const std::vector<HostWrite>& writes) {
     return;
   }
   std::vector<tfcc_rocm_copy_piece> pieces;
-  size_t chunk = size_t(384) << 10, gathered = 0;
+  UploadCut cut;
   auto launch = [&] {
     if (pieces.empty()) return;
     check(tfcc_rocm_copy_pieces_from_pinned(_stream, pieces.data(), static_cast<unsigned>(pieces.size())));
     pieces.clear();
-    gathered = 0;
-    chunk = std::min(chunk * 2, size_t(768) << 10);
+    cut.launched();
   };
   for (const HostWrite& w : writes) {
     const char* src = static_cast<const char*>(w.host);
@@ -1271,15 +1268,14 @@ void ROCMSession::upload(const std::vector<HostWrite>& writes) {
         launch();
         sync();
       }
-      const size_t n = std::min(std::min(left, chunk - gathered), _stagingSize - _stagingUsed);
+      const size_t n = cut.next(left, _stagingSize - _stagingUsed);
       std::memcpy(_staging + _stagingUsed, src, n);
       pieces.push_back({_staging + _stagingUsed, dst, n});
-      _stagingUsed += (n + 63) / 64 * 64;
-      gathered += n;
+      _stagingUsed += UploadCut::padded(n);
       src += n;
       dst += n;
       left -= n;
-      if (gathered >= chunk) launch();
+      if (cut.put(n)) launch();
     }
   }
   launch();
