@@ -254,6 +254,21 @@ def test_attention_into_rows_of_odd_pitch(pkg, gpu, S, Tk, D):
     assert rel_fro(got[..., :D], reference64(q, k, v, 3.0)) <= 1e-5
 
 
+def test_attention_over_more_rows_than_blocks_of_16_can_have(pkg, gpu):
+    """2^28 query rows: in blocks of 16 the launch would have 2^32 threads.  All heads have the same operands, so the same result."""
+    import torch
+    S, Tk, D, outer, inner = 64, 64, 4, 1 << 11, 1 << 11
+    rng = np.random.default_rng(5)
+    q, k, v = (rng.standard_normal((1, 1, r, D)).astype(np.float32) for r in (S, Tk, Tk))
+    tq, tk, tv = gpu.t(q), gpu.t(k), gpu.t(v)
+    out = torch.zeros((outer, inner, S, D), dtype=torch.float32, device=tq.device)
+    desc = pkg.attention_desc(tq, tk, tv, out, S, Tk, D, (D,) * 4, batch_outer=outer, batch_inner=inner, strides=(0, 0, 0, inner * S * D),
+                              inner_strides=(0, 0, 0, S * D), divisor=2.0)
+    pkg.attention(desc)
+    assert rel_fro(gpu.n(out[0, 0]), reference64(q, k, v, 2.0)[0, 0]) <= 1e-5
+    assert all(bool((o == out[0, 0]).all()) for o in out.split(256))
+
+
 def test_attention_limits_are_reported(pkg, gpu):
     import torch
     x = torch.zeros(256 * 256, dtype=torch.float32, device=gpu.t(np.zeros(1, np.float32)).device)

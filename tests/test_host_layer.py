@@ -164,3 +164,12 @@ def test_where_uploads_are_cut():
         subprocess.check_call(["make", "-C", os.path.join(ROOT, "wechat-tfcc_amd", "host"), "build/upload_cut_tests"])
     res = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
     assert res.returncode == 0 and "all passed" in res.stdout, res.stdout[-2000:]
+
+
+def test_which_attention_kernel_takes_a_call():
+    """Both sides of the rule's lines, and no more threads than a launch may have (tests/cpp/attention_plan_tests.cpp)."""
+    exe = os.path.join(ROOT, "wechat-tfcc_amd", "host", "build", "attention_plan_tests")
+    if not os.path.exists(exe):
+        subprocess.check_call(["make", "-C", os.path.join(ROOT, "wechat-tfcc_amd", "host"), "build/attention_plan_tests"])
+    res = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert res.returncode == 0 and "all passed" in res.stdout, res.stdout[-2000:]

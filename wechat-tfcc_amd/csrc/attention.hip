@@ -14,6 +14,7 @@
 // equals theirs bit for bit.
 #include <float.h>
 
+#include "attention_plan.hpp"
 #include "common.hpp"
 #include "qgemm_params.hpp"  // UDiv: division by multiply-high
 
@@ -24,8 +25,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int kRows = 64;        // query rows per workgroup
-constexpr int kThreads = 512;    // eight wavefronts
-constexpr int kMaxT = 128;       // key rows
+constexpr int kMaxT = attention_plan::kWholeKeys;  // key rows
 constexpr int kMaxD = 64;        // head width
 constexpr int kPitchK = kMaxD + 4;    // floats; 128-bit row reads of 32 consecutive rows hit all banks once
 constexpr int kPitchV = kMaxD + 8;    // 32-bit reads of rows r and r + 4 land 32 banks apart
@@ -804,8 +804,6 @@ extern "C" int tfcc_rocm_attention_f32(void* stream, const tfcc_rocm_attention_d
   p.outerQ = d->stride_q; p.outerK = d->stride_k; p.outerV = d->stride_v; p.outerO = d->stride_out;
   p.innerQ = d->inner_stride_q; p.innerK = d->inner_stride_k; p.innerV = d->inner_stride_v; p.innerO = d->inner_stride_out;
   p.batchInner = d->batch_inner;
-  // up to 128 keys: the scores of a row block in one piece; beyond: runs of keys with a maximum and a sum each
-  const bool stream128 = d->t > (unsigned)kMaxT;
   int cus = 0;
   {
     int dev = 0;
@@ -815,25 +813,8 @@ extern "C" int tfcc_rocm_attention_f32(void* stream, const tfcc_rocm_attention_d
     if (!cuCount[dev]) TFCC_HIP_CHECK(hipDeviceGetAttribute(&cuCount[dev], hipDeviceAttributeMultiprocessorCount, dev));
     cus = cuCount[dev];
   }
-  // A CU works through its blocks roughly one after the other (two resident workgroups overlap little: 19.1 us for
-  // 384 blocks of 64 rows against 12.7 for 192), so what counts is the largest number of rows any CU gets; a block of
-  // 32 rows costs about 0.55 of a block of 64 (K and V are loaded per block).  16 x 12 heads of 128 rows: 17.8 against
-  // 19.1 us with 32 rows; 32 x 12 heads: 30.5 against 27.7, so those keep 64.
-  const unsigned long long heads = (unsigned long long)d->batch_outer * d->batch_inner;
-  const unsigned long long blocks64 = (d->s + 63) / 64 * heads, blocks32 = (d->s + 31) / 32 * heads,
-                           blocks16 = (d->s + 15) / 16 * heads;
-  const unsigned long long perCu64 = (blocks64 + cus - 1) / cus, perCu32 = (blocks32 + cus - 1) / cus;
-  const bool rows32 = perCu32 * 55 < perCu64 * 100;
-  // Blocks of 16 rows: up to 64 keys always (128 x 12 heads of 64 rows 37.1 -> 33.7 us, 32 x 12 12.3 -> 12.4, 64 x 12 of 32 11.2 -> 10.6).  Beyond, every
-  // block walks twice the keys, which is faster where there are no more blocks than CUs or no more than with 32 rows
-  // (2 x 12 heads of 128 rows 7.9 -> 6.2 us, 40 x 12 of 16 rows and 100 keys 10.4 -> 8.7), and not otherwise (4 x 12 of 100
-  // rows 7.7 -> 8.4, 8 x 12 of 128 10.4 -> 11.6).
-  const bool rows16 = !stream128 && (d->t <= 64 || d->s <= 16 || blocks16 <= (unsigned long long)cus);
-  // More than 128 keys: two blocks of 16 rows share the loads of K and V where there are six or more for each CU (8 x 12 heads of 512
-  // rows 72.8 -> 68.4 us, 16 x 12 of 384 86.0 -> 79.5, 8 x 12 of 384 45.7 -> 46.1); with fewer they fill the GPU less evenly (4 x 12
-  // of 384 27.2 -> 29.3, 12 of 1024 35.9 -> 43.8, 12 of 256 6.7 -> 9.6).
-  const bool single = stream128 && blocks16 < 6ull * cus;
-  const unsigned rowsPerBlock = rows16 || single ? 16 : stream128 || rows32 ? 32 : kRows;
+  const attention_plan::Kernel kernel = attention_plan::kernel_of(d->s, d->t, (unsigned long long)d->batch_outer * d->batch_inner, cus);
+  const unsigned rowsPerBlock = attention_plan::rows_of(kernel);
   p.blocksS = (d->s + rowsPerBlock - 1) / rowsPerBlock;
   const unsigned long long total = (unsigned long long)p.blocksS * d->batch_outer * d->batch_inner;
   TFCC_REQUIRE(total < (1ull << 31) - 8, "attention: too many blocks");
@@ -862,9 +843,15 @@ extern "C" int tfcc_rocm_attention_f32(void* stream, const tfcc_rocm_attention_d
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsBytes32));
     attrSet[dev] = true;
   }
-  if (rows16) hipLaunchKernelGGL(d->t <= 64 ? attention_rows16_kernel<64> : attention_rows16_kernel<128>, dim3(p.chunk * 8), dim3(256), 0, as_stream(stream), p);
-  else if (stream128) hipLaunchKernelGGL(single ? attention_stream_kernel<1> : attention_stream_kernel<2>, dim3(p.chunk * 8), dim3(256), 0, as_stream(stream), p);
-  else if (rows32) hipLaunchKernelGGL(attention_kernel<32>, dim3(p.chunk * 8), dim3(256), ldsBytes32, as_stream(stream), p);
-  else hipLaunchKernelGGL(attention_kernel<64>, dim3(p.chunk * 8), dim3(kThreads), ldsBytes, as_stream(stream), p);
+  const dim3 grid(p.chunk * 8), block(attention_plan::threads_of(kernel));
+  switch (kernel) {
+    case attention_plan::kRows64: hipLaunchKernelGGL(attention_kernel<64>, grid, block, ldsBytes, as_stream(stream), p); break;
+    case attention_plan::kRows32: hipLaunchKernelGGL(attention_kernel<32>, grid, block, ldsBytes32, as_stream(stream), p); break;
+    case attention_plan::kRows16:
+      hipLaunchKernelGGL(d->t <= 64 ? attention_rows16_kernel<64> : attention_rows16_kernel<128>, grid, block, 0, as_stream(stream), p);
+      break;
+    case attention_plan::kRuns16: hipLaunchKernelGGL(attention_stream_kernel<1>, grid, block, 0, as_stream(stream), p); break;
+    case attention_plan::kRuns32: hipLaunchKernelGGL(attention_stream_kernel<2>, grid, block, 0, as_stream(stream), p); break;
+  }
   return check_launch("attention");
 }
