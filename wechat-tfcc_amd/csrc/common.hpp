@@ -202,6 +202,15 @@ __device__ static inline int requantize_one_biased_unclamped(unsigned off, const
 __device__ __forceinline__ float ref_max(float a, float b) { return a < b ? b : a; }
 __device__ __forceinline__ float ref_min(float a, float b) { return b < a ? b : a; }
 
+// Between what lanes of a wavefront put into LDS and what its other lanes read of it, and before it is overwritten.  The LDS takes
+// the accesses of a wavefront in their order; the compiler, to which they are another thread's, must not change that.  No
+// instruction comes of it.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The value of lane i ^ MASK for the six steps of a butterfly over the 64 lanes, without the LDS crossbar that
 // __shfl_xor goes through: the two halves and the rows of 16 lanes are exchanged by the swap instructions (a and b
 // come back as the two members of the pair, in lane order of the lower one), the steps inside a row are data-parallel

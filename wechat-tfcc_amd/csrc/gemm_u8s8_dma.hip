@@ -359,6 +359,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
         // The wavefront's 32 rows lie in LDS: WN / 4 lanes write one row's WN columns.  From the registers a store writes 32
         // pieces of 32 bytes: us, 1024 x 768 x 3072 10.7 -> 10.3, 2048 x 512 x 2048 10.1 -> 9.6, 640 x 256 x 2048 5.7 -> 5.35.
         constexpr int PER = WN / 4, ROWS = 64 / PER;
+        wave_lds_order();
 #pragma unroll
         for (int t = 0; t < 32 / ROWS; ++t) {
           const int row = t * ROWS + lane / PER, col = lane % PER * 4;
@@ -366,6 +367,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
           const unsigned to = m0 + wm * WM + 32 * i + row, at = n0 + wn * WN + col;
           if (to < M && at < N) *reinterpret_cast<v4i*>(C + (size_t)to * N + at) = v;  // N % 16 == 0: four columns are in or out together
         }
+        wave_lds_order();
       }
       if constexpr (FLAVOUR != 0) {
         // The rows of block row i (32 per wavefront row) are staged: write them out now, so that the stores are

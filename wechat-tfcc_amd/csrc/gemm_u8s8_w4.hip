@@ -393,8 +393,8 @@ __global__ __launch_bounds__(kThreads) void qgemm_w4_kernel(const QGemmParams p)
   __syncthreads();
 
   int* C = WRITE_C ? p.C + (size_t)bi * p.strideC : nullptr;
-  constexpr int CPITCH = 128 + 4;  // 32 rows of a wavefront's int32 results
-  int* const stageC = reinterpret_cast<int*>(smem + (BM + BN) * 4) + wave * 32 * CPITCH;
+  constexpr int CPITCH = 128 + 4;  // 32 rows of a wavefront's int32 results, twice
+  int* const stagesC = reinterpret_cast<int*>(smem + (BM + BN) * 4) + wave * 2 * 32 * CPITCH;
   unsigned char* Q = REQUANT ? p.Q + (size_t)bi * p.strideC : nullptr;
 
   // Requantized values leave the registers directly: a lane packs the four uint8 of each of its column quads
@@ -409,6 +409,7 @@ __global__ __launch_bounds__(kThreads) void qgemm_w4_kernel(const QGemmParams p)
     for (int i = 0; i < MI; ++i) {
       const int trow = wm * 128 + 32 * i + l32;
       const unsigned grow = m0 + trow;
+      int* const stageC = stagesC + (i & 1) * 32 * CPITCH;  // in turn: block row i is read before the order of i + 1, which i + 2 is behind
       // without an int32 result to store, the 2^31 that turns the accumulator into its offset from INT32_MIN is
       // folded into the row term
       constexpr unsigned kBias = (REQUANT && !WRITE_C) ? 0x80000000u : 0u;
@@ -451,6 +452,7 @@ __global__ __launch_bounds__(kThreads) void qgemm_w4_kernel(const QGemmParams p)
       if constexpr (WRITE_C) {
         // The wavefront's 32 rows of int32 lie in LDS: 32 lanes write the 512 bytes of one.  From the registers a store
         // writes 32 pieces of 32 bytes: us, int32 results, 4096 x 256 x 4096 19.2 -> 18.7, 3072 x 768 x 4096 22.1 -> 20.9.
+        wave_lds_order();
 #pragma unroll
         for (int t = 0; t < 16; ++t) {
           const int row = 2 * t + g, col = 4 * l32;
@@ -501,7 +503,7 @@ int launch_w4(hipStream_t stream, QGemmParams p) {
   p.perBatchMagic = perBatch.magic; p.perBatchShift = perBatch.shift;
   p.bandMagic = band.magic; p.bandShift = band.shift;
   constexpr size_t ring = (size_t)STAGES * (BM + BN) * BK;
-  constexpr size_t epi = (size_t)(BM + BN) * 4 + (WRITE_C ? 4 * 32 * (128 + 4) * 4 : 0);
+  constexpr size_t epi = (size_t)(BM + BN) * 4 + (WRITE_C ? 4 * 2 * 32 * (128 + 4) * 4 : 0);
   constexpr size_t lds = ring > epi ? ring : epi;
   static_assert(lds <= 160 * 1024, "LDS budget");
   auto kern = qgemm_w4_kernel<BK, STAGES, REQUANT, WRITE_C, OWN_COLSUM>;
