@@ -468,6 +468,9 @@ typedef struct tfcc_rocm_lstm_sequence_desc {
 } tfcc_rocm_lstm_sequence_desc;
 size_t tfcc_rocm_lstm_sequence_workspace(unsigned batch, unsigned units, unsigned directions);
 int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc* desc);
+/* the same with the workgroups dealt out so that those which need one another's results (up to 768 units: a group of rows) are not on
+ * one part of the GPU, as a GPU would have them that does not deal out workgroups in turn; slower, with the same results */
+int tfcc_rocm_lstm_sequence_f32_spread(void* stream, const tfcc_rocm_lstm_sequence_desc* desc);
 /* One step of tfcc::rnn::lstm_forward / lstm_backward (tfcc/core/operations/tfcc_rnn.cpp:62-71) in one launch:
  * matmul(h_prev, state kernel) and the LSTM cell above on its sums.  batch <= 8.  The state kernel is passed with its
  * gates interleaved: element [k, 4 * u + g] = state_kernel[k, g * units + u], i.e. the [units, 4, units] view of the

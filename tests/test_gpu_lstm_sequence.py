@@ -22,7 +22,7 @@ def setup(T, seq, batch, length, hidden, directions, seed=0):
     return x, sets
 
 
-def launch(pkg, T, x, sets, backward, wait_us=20000, stream=None):
+def launch(pkg, T, x, sets, backward, wait_us=20000, stream=None, spread=False):
     import torch
     seq, batch, _ = x.shape
     hidden = sets[0]["ih"].shape[1]
@@ -41,7 +41,8 @@ def launch(pkg, T, x, sets, backward, wait_us=20000, stream=None):
         d.out[i], d.h[i], d.c[i], d.backward[i] = out.data_ptr(), h.data_ptr(), c.data_ptr(), int(backward[i])
         outs.append((out, h, c))
     torch.cuda.synchronize()
-    pkg.check(pkg.lib().tfcc_rocm_lstm_sequence_f32(stream, C.byref(d)))
+    call = pkg.lib().tfcc_rocm_lstm_sequence_f32_spread if spread else pkg.lib().tfcc_rocm_lstm_sequence_f32
+    pkg.check(call(stream, C.byref(d)))
     return outs, keep
 
 
@@ -88,6 +89,24 @@ def test_rows_dealt_out_to_xcds(pkg, T, seq, batch, hidden, directions):
     assert gave_up(T, keep) == 0
     again, keep = launch(pkg, T, x, sets, backward)
     for a, b in zip(outs, again):
+        for p, q in zip(a, b):
+            assert np.array_equal(T.n(p), T.n(q))
+
+
+@pytest.mark.parametrize("seq,batch,hidden,directions", [
+    (1, 4, 256, 2), (2, 5, 257, 2), (3, 7, 512, 2), (9, 13, 768, 2), (6, 16, 767, 1), (40, 15, 249, 2), (11, 1, 65, 1)])
+def test_rows_whose_workgroups_share_no_xcd(pkg, T, seq, batch, hidden, directions):
+    """The workgroups of a group side by side, so on all XCDs: they find that out from the first step's words, and h goes through
+    memory from then on.  The same bits as with a group on one XCD, and not by way of the launch behind."""
+    print("lstm spread", seq, batch, hidden, directions, flush=True)
+    x, sets = setup(T, seq, batch, 24, hidden, directions)
+    backward = (True, False)[:directions]
+    outs, keep = launch(pkg, T, x, sets, backward, spread=True)
+    compare(T, outs, x, sets, backward)
+    assert gave_up(T, keep) == 0
+    together, keep = launch(pkg, T, x, sets, backward)
+    assert gave_up(T, keep) == 0
+    for a, b in zip(outs, together):
         for p, q in zip(a, b):
             assert np.array_equal(T.n(p), T.n(q))
 

@@ -158,6 +158,7 @@ SYMBOLS = {
     "tfcc_rocm_argmax_f32": (_I, [_VP, _VP, _U64, _U, _U64, _VP]),
     "tfcc_rocm_lstm_sequence_workspace": (C.c_size_t, [_U, _U, _U]),
     "tfcc_rocm_lstm_sequence_f32": (_I, [_VP, _VP]),
+    "tfcc_rocm_lstm_sequence_f32_spread": (_I, [_VP, _VP]),
     "tfcc_rocm_lstm_step_f32": (_I, [_VP, _U, _U, _VP, _VP, _VP, _VP, _F, _VP, _VP, _VP]),
     "tfcc_rocm_gru_cell_gates_f32": (_I, [_VP, _U, _U, _U, _VP, _VP, _VP, _VP, _VP]),
     "tfcc_rocm_gru_cell_candidate_f32": (_I, [_VP, _U, _U, _VP, _VP, _VP, _VP, _VP, _VP]),

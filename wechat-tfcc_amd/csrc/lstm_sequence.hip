@@ -53,6 +53,7 @@ struct SequenceParams {
   float forget;
   unsigned blocksPerDirection;
   unsigned groups, rowsPerGroup;  // of the form with an XCD for a group of rows; none: the other one
+  unsigned spread;                // that form with the workgroups of a group side by side, so on all XCDs
   unsigned* words;  // [set][direction][batch][pitch]
   unsigned* failed;
   unsigned long long waitTicks;
@@ -399,6 +400,11 @@ __device__ __forceinline__ unsigned xcd_id() { return __builtin_amdgcn_s_getreg(
 // it but time.  The words of the first step go through to memory and carry the XCD they come from; everyone reads all of them,
 // so everyone knows whether they are all from one, and if not, h goes through to memory in all steps.
 //
+// In the terms of the memory model a store for the workgroup hands nothing to another workgroup, whatever XCD it runs on.  That it is
+// seen rests on this chip: such a store goes to the L2, which is where a load at device scope looks.  What does not rest on it
+// is the result: a word is taken only with its step's number, which its value came with in one store of 64 bits, so what is not
+// seen, or seen late, can only end a wait, and then the launch behind computes the sequence.
+//
 // A wavefront owns UPW units.  A lane takes four k in 256 of all their gates, so a row of h is KQ loads from LDS, and
 // the products are on the vector unit: one row leaves three of the four rows of a 4 x 4 x 1 matrix op empty, and with four the
 // time is the same.  100 steps of both directions, us, the form above -> this one: 1 x 128 162 -> 119, 4 x 256 171 -> 122, 16 x 256
@@ -414,7 +420,8 @@ __global__ __launch_bounds__(512) void lstm_xcd_kernel(SequenceParams p) {
   static_assert(LEFT <= COPIES, "a lane finishes one value");
   __shared__ __attribute__((aligned(16))) float hs[2][ROWS][K], columns[WAVES * UPW][260];  // (260: a wavefront's writes on all banks)
   __shared__ int gaveUp, apart;
-  const unsigned turn = blockIdx.x % kXcds, d = turn / p.groups, group = turn - d * p.groups;
+  const unsigned members = gridDim.x / kXcds, turn = p.spread ? blockIdx.x / members : blockIdx.x % kXcds;
+  const unsigned member = p.spread ? blockIdx.x - turn * members : blockIdx.x / kXcds, d = turn / p.groups, group = turn - d * p.groups;
   if (d >= p.directions) return;  // nothing for this XCD
   const int tid = threadIdx.x, lane = tid & 63, gate = lane & 3;
   const unsigned xcd = xcd_id();
@@ -430,14 +437,14 @@ __global__ __launch_bounds__(512) void lstm_xcd_kernel(SequenceParams p) {
   }
   __syncthreads();
 
-  const unsigned u0 = (blockIdx.x / kXcds * WAVES + wave) * UPW;
+  const unsigned u0 = (member * WAVES + wave) * UPW;
   // The state kernel: rows of a gate's units side by side go through LDS, four values to a load (fetched by the lanes that keep
   // them, a value of a row at a time, 4 x 512 takes 12 us longer and 4 x 768 31).  Rows that do not exist are zeros; what
   // stands in the place of units that do not is nobody's.
   float w[KQ][4][4][UPW];  // [.][k][gate][unit]
   {
     const __amdgpu_buffer_rsrc_t kernel = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(s.kernel), 0, (int)(16u * units * units), 0x00020000);
-    const unsigned first = blockIdx.x / kXcds * (WAVES * UPW);
+    const unsigned first = member * (WAVES * UPW);
 #pragma unroll
     for (int i = 0; i < KQ; ++i) {
       lstm_v4f rows[4][UPW];
@@ -747,7 +754,7 @@ size_t tfcc_rocm_lstm_sequence_workspace(unsigned batch, unsigned units, unsigne
   return lstm_plan::workspace_bytes(batch, units, directions, compute_units());
 }
 
-int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc* q) {
+static int sequence(void* stream, const tfcc_rocm_lstm_sequence_desc* q, bool spread) {
   TFCC_REQUIRE(q != nullptr, "lstm_sequence: null argument");
   const size_t need = tfcc_rocm_lstm_sequence_workspace(q->batch, q->units, q->directions);
   TFCC_REQUIRE(need != 0, "lstm_sequence: 1 to 16 rows, 1 to 1024 units, 1 or 2 directions and a CU for eight units of each, got %u, %u, %u",
@@ -765,6 +772,7 @@ int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc
   p.forget = q->forget;
   p.rowsPerGroup = lstm_plan::rows_of_xcd(q->batch, q->units, q->directions, compute_units());
   if (q->seq > kStepMask - 2) p.rowsPerGroup = 0;  // (the words' number has 28 bits)
+  p.spread = spread;
   p.groups = p.rowsPerGroup ? (q->batch + p.rowsPerGroup - 1) / p.rowsPerGroup : 0;
   p.words = static_cast<unsigned*>(q->workspace);
   p.failed = reinterpret_cast<unsigned*>(static_cast<char*>(q->workspace) + need - 64);
@@ -793,5 +801,8 @@ int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc
   if (!turn.recorded) (void)hipGetLastError();
   return status;
 }
+
+int tfcc_rocm_lstm_sequence_f32(void* stream, const tfcc_rocm_lstm_sequence_desc* q) { return sequence(stream, q, false); }
+int tfcc_rocm_lstm_sequence_f32_spread(void* stream, const tfcc_rocm_lstm_sequence_desc* q) { return sequence(stream, q, true); }
 
 }  // extern "C"
