@@ -36,6 +36,10 @@ int main(int argc, char** argv) {
   EXPECT(kernel_of(4096, 4096, 4096, 4096, (1u << 29) / (4096 + 256) + 1, 4096, false, 1) == kNone);
   EXPECT(kernel_of(4096, 4096, 4096, 4096, (1u << 29) / (4096 + 256) + 1, 4096, true, 1) == kNone);
   EXPECT(kernel_of(4096, 4096, 4096, 4096, 4096, 1u << 21, false, 1) == kNone);
+  // long K in a batch: rows at odd addresses, and at whole 16 bytes with the two near one another, keep 64 x 64 tiles; a single product does not
+  EXPECT(plain(1956, 112, 2559, 12) == k64 && plain(896, 107, 2749, 23) == k64 && plain(773, 128, 3117, 22) == k64);
+  EXPECT(plain(227, 5586, 768, 12) != kNone && plain(2752, 896, 5539) == k128);
+  EXPECT(plain(704, 3656, 312) == kNone && plain(704, 3656, 320) == k128);
   // two K groups while a CU has one tile at most, but not for many tiles of a short K
   EXPECT(k_groups_of_128(1, 128) == 2 && k_groups_of_128(128, 128) == 2 && k_groups_of_128(129, 319) == 1 && k_groups_of_128(129, 320) == 2);
   EXPECT(k_groups_of_128(256, 320) == 2 && k_groups_of_128(257, 320) == 1 && k_groups_of_128(257, 8192) == 1);

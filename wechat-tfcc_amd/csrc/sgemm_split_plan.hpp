@@ -42,10 +42,11 @@ inline int kernel_of(unsigned rows, unsigned columns, unsigned depth, unsigned l
     return 8 + 3.2 * (full + (r != 0)) + k * (full * .0743 + (r ? .048 + r * r * 4e-7 : 0));
   };
   // What the fp32 ops take, by operations and by tiles: the larger one, for what leaves CUs without work there is what there is
-  // to gain here (328 x 1536 x 4678: 63 us, 49 by operations, 41 in 64 x 64 tiles).  Of 60000 shapes 5000 go another way than
-  // by operations and with one K group alone; 160 of them, drawn, take 0.83 of the time, 80 batches 0.79, all but five of the
-  // 240 less than 1.03 of it, one 1.13 (704 x 320 x 3656).  Where the fp32 ops have 128 x 128 tiles as well, operations alone decide: that
-  // estimate is nearer there.
+  // to gain here (328 x 1536 x 4678: 64 us, 49 by operations, 41 in 128 x 128 tiles).  Of 120000 drawn products 9000 go another way than
+  // by operations and with one K group alone.  6600 of those, timed: 0.80 of the time in cache, 0.82 from memory; 17 take more than
+  // 1.03 in cache, most in batches of 64 to 82 rows (64 x 268 x 7872, 32 of them, 1.11; 75 x 7958 x 558, 40, 1.13), and 410 from memory, nearly
+  // all single products that leave 64 x 64 tiles for two K groups: these take 0.92 in cache and 1.00 from memory, 1.17 at most
+  // (2752 x 5539 x 896).  Where the fp32 ops have 128 x 128 tiles as well, operations alone decide: that estimate is nearer there.
   const double rate = k % 32 != 0 || n % 4 != 0 ? 105e6 : 115e6;  // operations in a microsecond
   const double byTiles = sgemm_tiles::microseconds(rows, columns, depth, batch), byOperations = 4 + 2. * m * n * k * batch / rate;
   const double below = byTiles > byOperations ? byTiles : byOperations;
@@ -57,9 +58,19 @@ inline int kernel_of(unsigned rows, unsigned columns, unsigned depth, unsigned l
   };
   auto cost64 = [&] { return 4 + 4.5 * ((t64 + 511) / 512) + k * .0108 * ((t64 + 255) / 256); };
   const double costs[3] = {costWide(), cost128(), cost64()};
-  const int best = costs[0] <= costs[1] && costs[0] <= costs[2] ? kWide : costs[1] <= costs[2] ? k128 : k64;
-  const double margin = best == k64 ? (below < 60 ? .75 : .87) : best == k128 && twice ? .88 : 1.;
-  return costs[best] < margin * byOperations || costs[best] < (margin < .92 ? margin : .92) * byTiles ? best : kNone;
+  int best = costs[0] <= costs[1] && costs[0] <= costs[2] ? kWide : costs[1] <= costs[2] ? k128 : k64;
+  const double margin64 = below < 60 ? .75 : .87;
+  // A batch whose operands nothing reads twice comes from memory, and then a long K takes two K groups longer than that, rows at odd
+  // addresses most (1956 x 2559 x 112, 12 of them, 139 us, 105 estimated and 109 in 64 x 64 tiles).  209 products that have 64 x 64 tiles
+  // for it took 0.97 of their time in the others in cache, 1.02 from memory, 33 more than 1.03 in both, up to 1.27.
+  if (batch > 1 && twice && best == k128 && k >= 2500 && costs[k64] < margin64 * byOperations &&
+      costs[k64] < (k % 4 == 0 ? 1.08 : 1.2) * costs[k128])
+    best = k64;
+  const double margin = best == k64 ? margin64 : best == k128 && twice ? .88 : 1.;
+  // One K group, but so many k that the fp32 ops have two: up to 1.03 of their time in cache and 1.12 from memory (704 x 312 x
+  // 3656) where it is thought to be no faster than by a tenth.
+  const double marginByTiles = best == k128 && !twice && k >= 300 ? .9 : .92;
+  return costs[best] < margin * byOperations || costs[best] < (margin < marginByTiles ? margin : marginByTiles) * byTiles ? best : kNone;
 }
 
 }  // namespace sgemm_split_plan
