@@ -164,13 +164,13 @@ def test_attention_with_mask_in_blocks_of_16_rows(pkg, gpu, B, H, S, Tk, D, divi
 
 
 LONG_CASES = [
-    # B, H, S, T, D, divisor, layout: key sequences beyond one block of 128
+    # B, H, S, T, D, divisor, layout: key sequences of more than 128, in runs of 32
     (1, 12, 384, 384, 64, 8.0, "bshd"),     # the sequence length of the question-answering model the reference documents
-    (2, 3, 70, 129, 64, 8.0, "bshd"),       # one key into the second block
-    (1, 2, 100, 512, 36, 6.0, "bhsd"),      # four whole blocks, head width not a multiple of 8
-    (2, 2, 9, 300, 8, None, "bhsd"),        # ragged last block, no divisor
-    (1, 1, 200, 1000, 64, 8.0, "bshd"),     # eight blocks
-    (5, 10, 256, 200, 64, 8.0, "bshd"),     # 400 blocks of 32 query rows are more than the GPU has CUs: blocks of 64 (the cases above run as blocks of 32)
+    (2, 3, 70, 129, 64, 8.0, "bshd"),       # one key into the fifth run, of the first wavefront again
+    (1, 2, 100, 512, 36, 6.0, "bhsd"),      # four whole runs of a wavefront, head width not a multiple of 8
+    (2, 2, 9, 300, 8, None, "bhsd"),        # ragged last run, no divisor
+    (1, 1, 200, 1000, 64, 8.0, "bshd"),     # eight runs of a wavefront, the last one ragged
+    (5, 10, 256, 200, 64, 8.0, "bshd"),     # 800 blocks of 16 query rows, three to a CU
 ]
 
 
@@ -274,7 +274,7 @@ def test_attention_limits_are_reported(pkg, gpu):
     x = torch.zeros(256 * 256, dtype=torch.float32, device=gpu.t(np.zeros(1, np.float32)).device)
     ok = pkg.attention_desc(x, x, x, x, 16, 128, 64, (64,) * 4)
     assert pkg.attention_supported(ok)
-    assert pkg.attention_supported(pkg.attention_desc(x, x, x, x, 16, 129, 64, (64,) * 4))  # blocks of 128 keys
+    assert pkg.attention_supported(pkg.attention_desc(x, x, x, x, 16, 129, 64, (64,) * 4))  # runs of 32 keys
     for s, t, d, ld in [(16, 16, 68, 68), (16, 16, 6, 8), (16, 16, 8, 10)]:
         bad = pkg.attention_desc(x, x, x, x, s, t, d, (ld,) * 4)
         assert not pkg.attention_supported(bad)

@@ -7,7 +7,8 @@ import oracle_lib as O
 
 pytestmark = pytest.mark.gpu
 
-LIMIT = 128 * 1024  # elements a single launch quantizes
+LIMIT = 128 * 1024  # elements that every workgroup reads for the range where a launch is recorded (40 K otherwise)
+TOGETHER = 8 << 20   # elements whose range the workgroups of one launch agree on; more take a launch for it
 
 
 @pytest.mark.parametrize("total", [1, 2, 3, 5, 4095, 4096, 4097, 32771, LIMIT - 1, LIMIT, LIMIT + 1, LIMIT + 4])
@@ -55,7 +56,7 @@ def test_quantize_over_its_own_input(pkg, T, total):
 def test_quantize_small_and_large_tensors_agree(pkg, T, special, dtype):
     import torch
     small = np.array(special, np.float32)
-    large = np.tile(small, LIMIT // 3 + 1)  # beyond the limit: the form in three launches
+    large = np.tile(small, LIMIT // 3 + 1)  # in workgroups that agree on the range
     a, b = (pkg.quantize(T.t(v), getattr(torch, dtype)) for v in (small, large))
     for v, w in zip(a[1:], b[1:]):
         assert np.array_equal(T.n(v), T.n(w), equal_nan=True)
@@ -79,10 +80,12 @@ def test_row_sums_at_any_address(pkg, T, col, dtype):
         assert np.array_equal(T.n(pkg.reduce_sum(t, True)).ravel(), a.sum(1, dtype=np.int64).astype(np.int32))
 
 
-def test_quantize_on_several_streams_and_under_capture(pkg, T):
+@pytest.mark.parametrize("total", [3 * LIMIT, TOGETHER + 4])
+def test_quantize_on_several_streams_and_under_capture(pkg, T, total):
+    """the words of the workgroups that agree on the range, and behind those the arrival words of a stream, side by side"""
     import torch
     rng = np.random.default_rng(3)
-    xs = [rng.normal(0, 1 + i, 3 * LIMIT + i).astype(np.float32) for i in range(4)]
+    xs = [rng.normal(0, 1 + i, total + i).astype(np.float32) for i in range(4)]
     ts, streams = [T.t(x) for x in xs], [torch.cuda.Stream() for _ in xs]
     torch.cuda.synchronize()
     want = [O.quantize(x, float(x.min()), float(x.max()), "uint8") for x in xs]
