@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the matmul hot path on one MI355X.
 
-Headline workload (the one the north-star target is quoted on):
+Headline workload:
   uint8 [4096,4096] (zero-point 128) x int8 [4096,4096] (symmetric) -> int32 accumulate ->
   requantize to uint8 with scale 1/(K*64), zero-point 128, through the fused kernel
   (tfcc_rocm_gemm_u8s8s32_requant_u8, int32 accumulators not written).
@@ -19,7 +19,7 @@ The same JSON line carries
                 timed on this host's cores on a bounded sample, with all threads and with the four the
                 reference's test harness uses; an fp32 leg (C1 and the GEMMs of C4) through a plain
                 OpenMP port and through the CPU BLAS torch ships; the CPU model
-  other         the remaining BASELINE configs (fp32 GEMM + bias, attention-shaped batched fp32,
+  other         the remaining workloads (fp32 GEMM + bias, attention-shaped batched fp32,
                 skinny int8 decode GEMV, int32-writing variant), each with its own roofline figure
 
 usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu] [--no-other] [--no-sampler]
@@ -374,7 +374,7 @@ def cpu_baseline(a, b, size):
 
 
 def bench_other(torch, pkg, dev, steps, warmup, c3, short_legs=False):
-    """Remaining BASELINE configs; each entry: ms, achieved rate, bound, fraction of the bounding peak."""
+    """The remaining workloads; each entry: ms, achieved rate, bound, fraction of the bounding peak."""
     out = {}
     # These launches take microseconds: a handful of them after the host-side set-up of a case measures the clock
     # ramp and the first touch of the rotated buffers, not the kernel.  Whatever --steps / --warmup say, every case
@@ -678,7 +678,7 @@ def bench_other(torch, pkg, dev, steps, warmup, c3, short_legs=False):
     rt = importlib.import_module("wechat_tfcc_amd.runtime_api")
     hidden, heads, ffn = 768, 12, 3072
     w = mf.bert_layer_weights(rng, hidden, ffn)
-    # batch 8 x 128 positions (BASELINE configs[3]), and one sequence of 384 positions: the length of the
+    # batch 8 x 128 positions, and one sequence of 384 positions: the length of the
     # question-answering model the reference documents (samples/ConvertONNXModel.md:16), whose attention walks the
     # keys in runs of 32
     for name, batch, seq in (("c4_bert_base_layer_b8_s128_runtime", 8, 128), ("bert_base_layer_b1_s384_runtime", 1, 384)):
@@ -783,7 +783,7 @@ def main():
         "vs_baseline": None,
         "dtype": "int8 (int32 accumulate, fp64 requantize)",
         "data": "synthetic (seeded uniform uint8 / int8, resident in HBM)",
-        "config": {"workload": "BASELINE configs[2]: A u8[4096,4096] zp 128 x B s8[4096,4096] symmetric -> "
+        "config": {"workload": "A u8[4096,4096] zp 128 x B s8[4096,4096] symmetric -> "
                                "int32 -> requantize u8, scale 1/(K*64), zp 128; fused kernel, uint8 output only",
                    "m": size, "n": size, "k": size},
         "roofline": {"bound": "mfma", "achieved": round(kernel_tops, 2), "peak": PEAK_INT8_TOPS, "unit": "TOP/s",

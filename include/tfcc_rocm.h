@@ -453,9 +453,11 @@ int tfcc_rocm_lstm_cell_f32(void* stream, unsigned batch, unsigned units, const 
  * units of a direction (else the workspace size is 0).  The workspace needs no particular contents; out, h and c may overlap
  * no input.  wait_us: how long the workgroups wait for one another before the sequence is computed in a single one per
  * direction (0: always that).  Calls of a process on one GPU follow one another, whatever their streams (from the second
- * stream's second call on).  Sequences replayed from graphs do not: two at once that do not fit
- * on the GPU together, or one on a stream confined to fewer CUs than it has workgroups (one for eight units of a
- * direction), end through that wait - the results are the same, the time is not. */
+ * stream's second call on).  Sequences replayed from graphs do not, nor do those of another process: two at once that do
+ * not fit on the GPU together, or one on a stream confined to fewer CUs than it has workgroups, end through that wait - the
+ * results are the same, the time is not.  On a whole GPU a sequence has eight workgroups for eight units up to 256, for 16 up
+ * to 512, for 24 up to 768, at most 256, and two of them share a CU up to 256 units, and up to 512 with one direction or eight
+ * rows; in a graph, beyond 768 units and on a part of a GPU it has one for eight units of a direction. */
 typedef struct tfcc_rocm_lstm_sequence_desc {
   unsigned seq, batch, units, directions;
   const float *x[2], *kernel[2], *bias[2], *h0[2], *c0[2];

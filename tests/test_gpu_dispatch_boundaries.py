@@ -210,7 +210,7 @@ def test_sgemm_on_128x96_workgroups(pkg, T, m, n, k, batch):
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k", [
     # the same hand-scheduled kernel with other numbers of 32-column blocks per wavefront: 32 x 64 tiles and four K
-    # groups (the first BASELINE config; ragged), 32 x 32 tiles and four K groups (whole and ragged), 128 x 128 tiles
+    # groups (128 x 768 x 3072; ragged), 32 x 32 tiles and four K groups (whole and ragged), 128 x 128 tiles
     # for products of 512 tiles and more: a single 32-k slab (the two before it take 128 x 128 tiles on the bf16 matrix
     # cores, for B as stored and transposed)
     (128, 3072, 768), (100, 3000, 800), (512, 512, 512), (500, 500, 544), (2048, 4096, 256), (2050, 4100, 320),

@@ -30,7 +30,8 @@
 // What that costs, us, in order, on one card: normal operands; one row of zeros; the last quarter of the rows; one value in a
 // hundred in both operands; one value of 2^31; one NaN; two results that cancel; and any operands on the fp32 ops:
 //   4096^3, 128 x 256 tiles        602   602   589   583   683   1459   595   910
-//   2048^3, 128 x 128               93    96    91   128   126    301    96   120
+//   2048^3, 128 x 128               90    91    89   101   110    296    94   120   (two K groups, as the next)
+//   1024 x 768 x 3072, 128 x 128    36    38    36    46    45    112    38    40
 //   1024 x 1024 x 2048, 64 x 64     30    31    30    45    47    106    31    33
 //
 // Two kernels.  What they have in common is that vector instructions run under bf16 matrix ops: up to six of them between
