@@ -1,5 +1,6 @@
 // The words of the one-launch quantize (wechat-tfcc_amd/csrc/quantize_exchange.hpp), on the host: no word of another call, however
-// many calls ago, and none that nobody has written is taken for this call's; and that every workgroup has a CU.  No GPU.
+// many calls ago, and none that nobody has written is taken for this call's; and that every workgroup has a CU,
+// beside those of other streams too.  No GPU.
 #include <cstdio>
 #include <initializer_list>
 
@@ -35,6 +36,20 @@ int main() {
       if (quads == 0) EXPECT(total > 8ull * kPiece * room);
       else EXPECT(workgroups(total, quads) <= room && workgroups(total, quads) * quads * kPiece >= total && (quads == 1 || workgroups(total, quads / 2) > room));
     }
+  int streams[9];
+  for (unsigned count : {1u, 2u, 3u, 4u, 8u, 9u}) {  // in turn
+    LastStreams last;
+    for (unsigned call = 0; call < 100; ++call) {
+      const unsigned seen = last.with(streams + call % count), most = call + 1 < 8 ? call + 1 : 8;
+      EXPECT(seen == (count < most ? count : most));
+      if (call >= 7 && count > 2) EXPECT(seen > streams_of(4) && seen > streams_of(8) && seen <= streams_of(1));
+      if (call >= 7 && count <= 2) EXPECT(seen <= streams_of(8));
+    }
+    for (unsigned call = 0; call < 20; ++call) {  // the others have ended
+      const unsigned seen = last.with(streams);
+      EXPECT(call < 7 || seen == 1);
+    }
+  }
   if (failures == 0) std::printf("quantize exchange: all passed\n");
   return failures != 0;
 }

@@ -109,6 +109,36 @@ def test_quantize_on_several_streams_and_under_capture(pkg, T, total):
         q.zero_()
 
 
+@pytest.mark.parametrize("total", [3 << 20, TOGETHER])
+def test_large_tensors_of_several_streams(pkg, T, total):
+    """Launches whose workgroups all wait for one another do not fit the GPU side by side: on four streams a call takes no longer than
+    on one (us, on one / on four: 3 M 8.6 / 8.5, 8 M 13.1 / 14.4; all four in one launch each 13.8 and 27; the line lies at half as much again)"""
+    import time
+    import torch
+    xs = [torch.randn(total, device="cuda") for _ in range(4)]
+    many = [torch.cuda.Stream() for _ in xs]
+    want = [O.quantize(T.n(x), float(x.min()), float(x.max()), "uint8") for x in xs]
+
+    def best(streams):
+        times = []
+        for _ in range(7):
+            torch.cuda.synchronize()
+            start = time.perf_counter()
+            for _ in range(20):
+                for x, s, q, ends in zip(xs, streams, qs, ranges):
+                    pkg.check(pkg.lib().tfcc_rocm_quantize_minmax(s.cuda_stream, pkg._ptr(x), total, pkg._ptr(q), pkg._type_code(torch.uint8),
+                                                                  pkg._ptr(ends[:1]), pkg._ptr(ends[1:])))
+            torch.cuda.synchronize()
+            times.append(time.perf_counter() - start)
+        return min(times)
+
+    qs, ranges = [torch.empty(total, dtype=torch.uint8, device="cuda") for _ in xs], [torch.empty(2, device="cuda") for _ in xs]
+    one, four = best(many[:1] * 4), best(many)
+    for q, w in zip(qs, want):
+        assert np.array_equal(T.n(q), w)
+    assert four <= 1.5 * one
+
+
 @pytest.mark.parametrize("total", [LIMIT + 1, LIMIT + 16384, 64 * 16384 + 3, 256 * 16384 - 1, 256 * 16384 + 5, 16 << 20])
 def test_captured_quantize_of_the_data_s_own_range(pkg, T, total):
     """Recorded in a graph: the same bytes as outside, and no slower than a launch more (with an atomic per wavefront on the

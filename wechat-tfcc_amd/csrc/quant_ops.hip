@@ -634,7 +634,7 @@ __global__ void minmax_finish_kernel(float* mn, float* mx) {
 // overwritten, are not waited for: a workgroup that has waited `waitTicks` reads a part that is missing itself and tells
 // the others, each another one as far as there are as many, until nothing is missing.  So nobody needs anybody, every round
 // of that has one part less to look for, and the input is read about twice, as with a launch for the range.  (A replayed graph would
-// find the words of its last replay, so a recorded call takes the launches below.)
+// find the words of its last replay, so a recorded call takes the launches below; so do large calls from several streams.)
 //
 // Bound by the launch, a store to memory and a load from it; with many elements to a workgroup by the reading.  us, the range
 // and the quantizing in a launch each before (up to 131072 elements the form above), input from memory: 77077 7.3 -> 5.4, 131072
@@ -811,23 +811,40 @@ unsigned stream_grid(size_t total4) {
 StreamSlots gArrivalSlots(kArrivalSlots);
 
 std::atomic<unsigned long long> gTogetherCalls{0};
+constexpr int kDevices = 16;
+quantize_exchange::LastStreams gTogetherStreams[kDevices];
 
-// of the current device, asked for once; 0: unknown
-int compute_units() {
-  static std::atomic<int> known[16];
-  int dev = 0, cus = 0;
+// -1: unknown, or one of more than kDevices
+int current_device() {
+  int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) {
     (void)hipGetLastError();
-    return 0;
+    return -1;
   }
-  if (dev >= 0 && dev < 16) cus = known[dev].load(std::memory_order_relaxed);
+  return dev < kDevices ? dev : -1;
+}
+
+// of a device, asked for once; 0: unknown
+int compute_units(int dev) {
+  static std::atomic<int> known[kDevices];
+  if (dev < 0) return 0;
+  int cus = known[dev].load(std::memory_order_relaxed);
   if (cus != 0) return cus;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
     (void)hipGetLastError();
     return 0;
   }
-  if (dev >= 0 && dev < 16) known[dev].store(cus, std::memory_order_relaxed);
+  known[dev].store(cus, std::memory_order_relaxed);
   return cus;
+}
+
+// Loads of a thread of the one launch; 0: the call takes the launches below.
+unsigned together_quads(hipStream_t s, uint64_t total) {
+  const int dev = current_device();
+  const unsigned quads = quantize_exchange::quads_of(total, compute_units(dev));
+  if (quads == 0 || !runs_in_order_now(s)) return 0;
+  if (quads > 1 && gTogetherStreams[dev].with(s) > quantize_exchange::streams_of(quads)) return 0;
+  return quads;
 }
 
 void launch_together(hipStream_t s, unsigned quads, const float* in, uint64_t total, void* out, int outType, float* mn, float* mx,
@@ -1005,8 +1022,8 @@ int tfcc_rocm_quantize_minmax_wait(void* stream, const float* in, uint64_t total
   // every element where it was read.
   const uintptr_t inAt = (uintptr_t)in, outAt = (uintptr_t)out;
   const bool apart = inAt + 4 * total <= outAt || outAt + total * (int_range(out_type).bits / 8) <= inAt;
-  const unsigned quads = apart && total > kWholeBest ? quantize_exchange::quads_of(total, compute_units()) : 0;
-  if (quads != 0 && runs_in_order_now(s)) {
+  const unsigned quads = apart && total > kWholeBest ? together_quads(s, total) : 0;
+  if (quads != 0) {
     launch_together(s, quads, in, total, out, out_type, min_v, max_v, wait_us);
     return check_launch("quantize");
   }
@@ -1025,7 +1042,7 @@ int tfcc_rocm_quantize_minmax_wait(void* stream, const float* in, uint64_t total
     TFCC_HIP_CHECK(hipGetDevice(&dev));
     if (gArrivalSlots.of(dev, s, &slot)) {
       // one workgroup per CU at most: every arrival costs an atomic on one word and a write-back (192 workgroups of 256
-      // threads for 786432 elements: 6 us, 48 of 1024: 5.6; so few come here on a GPU with few CUs, the form above takes them on a whole one)
+      // threads for 786432 elements: 6 us, 48 of 1024: 5.6; so few come here on a GPU with few CUs only, the form above takes them on a whole one)
       const unsigned blocks = total >= 256u * 16384u ? 256u : (unsigned)((total + 16383) / 16384);
       hipLaunchKernelGGL((minmax_partial_kernel<16, true>), dim3(blocks), dim3(1024), 0, s, in, (size_t)total, partials, slot,
                          min_v, max_v);

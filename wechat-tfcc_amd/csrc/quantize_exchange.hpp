@@ -2,6 +2,8 @@
 // many workgroups there are.  Plain functions of integers, compiled for the kernel, its launch and the tests.
 #pragma once
 
+#include <mutex>
+
 namespace tfcc_rocm {
 namespace quantize_exchange {
 
@@ -35,6 +37,37 @@ constexpr unsigned quads_of(unsigned long long total, int cus) {
     if (workgroups(total, quads) <= room) return quads;
   return 0;
 }
+
+// From how many streams in turn calls may come with so many loads to a thread.  The launches of more streams than that find no
+// CU for all of their workgroups, and those of each wait for one another until they give up.  us a call, streams side by
+// side, in one launch / in two: 2 M elements on 4 streams 6.3 / 9.1, on 8 10.2 / 9.0; 4 M on 2 8.5 / 10.1, on 3 17.0 / 9.8, on 8
+// 19.5 / 9.3; 8 M on 2 14.7 / 15.4, on 3 24.7 / 14.5, on 8 28.2 / 14.8.  One load to a thread is better on any number of streams.
+constexpr unsigned streams_of(unsigned quads) { return quads <= 1 ? ~0u : quads == 2 ? 4 : 2; }
+
+// The streams of a device's last calls.
+class LastStreams {
+ public:
+  // another call on this stream; of how many streams the last kCalls calls are, this one among them
+  unsigned with(const void* stream) {
+    std::lock_guard<std::mutex> lock(mutex_);
+    last_[next_++ % kCalls] = stream;
+    const unsigned known = next_ < kCalls ? next_ : kCalls;
+    if (next_ == 2 * kCalls) next_ = kCalls;
+    unsigned streams = 0;
+    for (unsigned i = 0; i < known; ++i) {
+      bool again = false;
+      for (unsigned j = 0; j < i; ++j) again = again || last_[j] == last_[i];
+      streams += again ? 0 : 1;
+    }
+    return streams;
+  }
+
+ private:
+  static constexpr unsigned kCalls = 8;
+  std::mutex mutex_;
+  const void* last_[kCalls] = {};
+  unsigned next_ = 0;
+};
 
 }  // namespace quantize_exchange
 }  // namespace tfcc_rocm
