@@ -1,8 +1,7 @@
-// uint8 x int8 -> int32 matrix product for large aligned shapes: the gfx950-specific pipeline.
+// uint8 x int8 -> int32 matrix product in slabs of K, of any size and alignment: the gfx950-specific pipeline.
 //
-// Same arithmetic as the kernel in gemm_u8s8.hip (which stays the path for unaligned and small
-// shapes); replaces tfcc/mkl/operations/tfcc_mklquantization.cpp:33-69,176-201 and the blocked CPU
-// GEMM below it (tfcc/mkl/gemm/tfcc_mklsinglethreadgemm.h:93-141, tfcc_mklmatmulkernel.h:142-260).
+// Replaces tfcc/mkl/operations/tfcc_mklquantization.cpp:33-69,176-201 and the blocked CPU GEMM below it
+// (tfcc/mkl/gemm/tfcc_mklsinglethreadgemm.h:93-141, tfcc_mklmatmulkernel.h:142-260).
 //
 // Data path of one BM x BN tile (WGM x WGN wavefronts; eight for the 256 x 256 tile, so that every
 // SIMD holds two: one wavefront's LDS reads, waits and VALU work overlap the other's matrix ops):
@@ -23,22 +22,44 @@
 //               256-byte row segments.
 // The true column sums of B (needed because a' = a - 128) are accumulated from the B operands with
 // v_dot4_i32_i8 by the two wavefronts of the first tile row.
+//
+// Operands that are no multiple of 16 bytes in K, N and address: copies take whole 32-bit words at multiples of four bytes
+// and check the range of each word, so K and N of multiples of four need no more than stores of their own (kWords).  At odd
+// bytes the same 16 bytes of a lane come through registers and go to the same place in LDS (kAnyByte), one to two slabs
+// ahead; everything behind the LDS image is the same.  A workgroup alone on its CU is bound by what it asks for per slab, not by the
+// matrix ops (a slab of 64 x 128 x 128 takes 0.41 us in copies, 0.55 through registers, 0.11 of them matrix ops).  Both replace
+// slabs whose B was loaded in words of four columns and transposed with byte permutes: us, before -> copies of words or registers,
+// 960 x 2976 x 900 21.4 -> 16.1, 1024 x 768 x 3076 13.4 -> 10.8, 2920 x 200 x 2500 15.7 -> 11.9, 974 x 7272 x 1136 43 -> 30;
+// 960 x 2973 x 896 21.8 -> 19.4, 1024 x 769 x 3073 17.7 -> 16.2, 1645 x 66 x 2631 10.3 -> 8.6, 952 x 4944 x 6577 108 -> 64.  240
+// drawn products of more than 64 such tiles, a quarter of them aligned as before, take 0.88 of the time; up to 1.06 four to six
+// slabs of odd rows that two K groups of wavefronts shared (2267 x 414 x 175 9.5 -> 10.1).
+// (Two K groups of wavefronts to a tile gain nothing here: 960 x 2976 x 896 14.5 -> 14.6.  Aligned words with one word more,
+// shifted to their places in registers, are more to ask for: 960 x 2976 x 897 20.3 -> 26.3.)
 #include <type_traits>
 
 #include "common.hpp"
 #include "lds_dma.hpp"
 #include "qgemm_dma.hpp"
+#include "qgemm_small.hpp"
 
 namespace tfcc_rocm {
 
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
+typedef v4i words4 __attribute__((aligned(4)));   // four results at any int32
+typedef v4i bytes16 __attribute__((aligned(1)));  // sixteen at any byte
 
 namespace {
 
+// what K, N and the addresses are multiples of: 16 bytes, four, one
+enum Kind { kAligned, kWords, kAnyByte };
+
 constexpr int BK = 128;      // bytes of k per slab: a row piece of A is one full 128-byte memory line
 constexpr int KS = BK / 32;  // 32-deep matrix-op steps per slab
+
+// A barrier for LDS alone: this wavefront's reads have returned and its stores are done, but its loads may be on their way.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // 16 consecutive rows of one logical chunk fall into 16 different 16-byte slots of the 256-byte bank stripe
 __device__ __forceinline__ int swzA(int row) { return (row >> 1) & 7; }
@@ -46,8 +67,11 @@ __device__ __forceinline__ int swzA(int row) { return (row >> 1) & 7; }
 // WRITE_C: the int32 result is stored (always without REQUANT; with it only when the caller wants both).
 // OWN_COLSUM: the true column sums of B are accumulated here (the caller's colsum_b is used as given, whatever
 // it holds, like the reference does); without it the caller has promised that colsum_b holds them.
-template <int BM, int BN, int WGM, int WGN, int STAGES, bool REQUANT, bool WRITE_C, bool OWN_COLSUM>
+// DEPTH: stages of the ring; of kAnyByte, slabs on their way in registers in front of two stages.
+template <int BM, int BN, int WGM, int WGN, int DEPTH, int KIND, bool REQUANT, bool WRITE_C, bool OWN_COLSUM>
 __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGemmParams p) {
+  constexpr bool ANY = KIND == kAnyByte, RAGGED = KIND != kAligned;
+  constexpr int STAGES = ANY ? 2 : DEPTH, HELD = ANY ? DEPTH : 1;
   constexpr int kThreads = WGM * WGN * 64;
   constexpr int WM = BM / WGM, WN = BN / WGN;
   constexpr int MI = WM / 32, NI = WN / 32;
@@ -100,6 +124,8 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
   // buffer descriptors: base, 0 stride, size in bytes, raw 32-bit format; held in SGPRs
   const v4i rsrcA = make_rsrc(A, M * K);
   const v4i rsrcB = make_rsrc(B, K * N);
+  const __amdgpu_buffer_rsrc_t loadA = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(A), 0, (int)(M * K), 0x00020000);
+  const __amdgpu_buffer_rsrc_t loadB = __builtin_amdgcn_make_buffer_rsrc(const_cast<signed char*>(B), 0, (int)(K * N), 0x00020000);
 
   // ---- per-thread copy descriptors: which 16 bytes of the slab this lane moves in each copy.
   // LDS slot s (16 bytes) of the A image holds row s/8, physical chunk s%8 = logical chunk ^ swzA(row).
@@ -128,6 +154,37 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
   auto issueSlab = [&](unsigned slab) {
 #pragma unroll
     for (int c = 0; c < COPIES; ++c) issueCopy(slab, c);
+  };
+  // kAnyByte: the same 16 bytes through registers.  A load may have any byte address; what its range check cannot do is return the
+  // valid bytes of one that crosses the end of the operand, so every load is moved back to end inside the operand, and in the
+  // slabs where that can have changed something the bytes are shifted to their places, zeros behind the end.  Bytes of A
+  // beyond K inside a row and columns of B beyond N are neighbouring data, which only meet zero rows of B or are not stored.
+  // The uint8 -> int8 of A happens here, once per byte.
+  v4i held[HELD == 1 ? 2 : HELD][ANY ? COPIES : 1];  // slab s in set s % HELD, slab 1 in set 1
+  const unsigned lastA = M * K - 16, lastB = K * N - 16;
+  auto fetch = [&](unsigned slab, int set, int c) __attribute__((always_inline)) {
+    const unsigned behind = slab * BK < K ? 0u : ~0u;  // nobody reads such a slab: all lanes ask for the same bytes
+    if (c < A_COPIES)
+      held[set][c] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(loadA, min((aOff[c] + slab * BK) | behind, lastA), 0, 0));
+    else
+      held[set][c] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(loadB, min((bOff[c - A_COPIES] + slab * (BK * N)) | behind, lastB), 0, 0));
+  };
+  auto keep = [&](unsigned slab, int set, int c) __attribute__((always_inline)) {
+    v4i v = held[set][c];
+    if (c < A_COPIES) v = v ^ (int)0x80808080;
+    *reinterpret_cast<v4i*>(smem + slab % STAGES * STAGE_BYTES + (c < A_COPIES ? 0 : A_BYTES) + ((c < A_COPIES ? c : c - A_COPIES) * kThreads + tid) * 16) = v;
+  };
+  auto settle = [&](unsigned slab, int set) __attribute__((always_inline)) {
+    if ((slab + 1) * BK >= K) {
+      asm volatile("" ::: "memory");  // a real (wave-uniform) branch: the wait for the loads stays inside
+#pragma unroll
+      for (int c = 0; c < A_COPIES; ++c) held[set][c] = moved16(held[set][c], max(aOff[c] + slab * BK, lastA) - lastA);
+    }
+    if (((slab + 1) * BK - 1) * N + n0 + BN > K * N) {
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int c = A_COPIES; c < COPIES; ++c) held[set][c] = moved16(held[set][c], max(bOff[c - A_COPIES] + slab * (BK * N), lastB) - lastB);
+    }
   };
 
   v16i acc[MI][NI];
@@ -190,12 +247,11 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
   // them: spread out enough not to queue up behind the other wavefronts' reads (all wavefronts run in
   // phase, one barrier per slab), early enough to have returned when the step ends.
   // uint8 -> int8 is the xor on the A operands; block j's column sums belong to wavefront row j % WGM.
-  // When `refill` is set the copies of slab `refillSlab` are issued as well, spread over the step for
-  // the same reason.
-  auto step = [&](v4i (&ua)[MI], v4i (&ub)[NI], v4i (&la)[MI], v4i (&lb)[NI], unsigned stage, int ks,
-                  auto refill, unsigned refillSlab) {
-    constexpr bool REFILL = decltype(refill)::value;
+  // `copies`, if any, are dealt out between the matrix ops for the same reason.
+  auto step = [&](v4i (&ua)[MI], v4i (&ub)[NI], v4i (&la)[MI], v4i (&lb)[NI], unsigned stage, int ks, auto&& copies) {
+    constexpr bool REFILL = !std::is_same<std::decay_t<decltype(copies)>, std::nullptr_t>::value;
     constexpr int DMA_EVERY = NMFMA / COPIES > 0 ? NMFMA / COPIES : 1;
+    constexpr int PER = ANY ? (COPIES + NMFMA - 1) / NMFMA : 1;  // side by side
     const unsigned char* as = smem + stage * STAGE_BYTES;
     const unsigned char* bs = as + A_BYTES;
 #pragma unroll
@@ -213,13 +269,18 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
 #pragma unroll
       for (int q = 2 * m; q < 2 * m + 2 && q < NLOAD; ++q) loadOne(as, bs, ks, q, la, lb);
       if constexpr (REFILL) {
-        if (m % DMA_EVERY == 0 && m / DMA_EVERY < COPIES) issueCopy(refillSlab, m / DMA_EVERY);
-        if (m == NMFMA - 1) {
+        if constexpr (ANY) {
 #pragma unroll
-          for (int c = NMFMA / DMA_EVERY; c < COPIES; ++c) issueCopy(refillSlab, c);  // more copies than matrix ops
+          for (int c = m * PER; c < (m + 1) * PER && c < COPIES; ++c) copies(c);
+        } else {
+          if (m % DMA_EVERY == 0 && m / DMA_EVERY < COPIES) copies(m / DMA_EVERY);
+          if (m == NMFMA - 1) {
+#pragma unroll
+            for (int c = NMFMA / DMA_EVERY; c < COPIES; ++c) copies(c);  // more copies than matrix ops
+          }
         }
       }
-      if (j == 0) ax = ua[i] ^ (int)0x80808080;
+      if (j == 0) ax = ANY ? ua[i] : ua[i] ^ (int)0x80808080;
       acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ub[j], ax, acc[i][j], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -231,8 +292,16 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
   //              slab kt+STAGES (copies past the end of K read zeros or unused bytes; they are issued
   //              anyway to keep the outstanding-copy count uniform)
   const unsigned KT = (K + BK - 1) / BK;
+  if constexpr (ANY) {
 #pragma unroll
-  for (int s = 0; s < STAGES; ++s) issueSlab(s);
+    for (int d = 0; d < (HELD == 1 ? 2 : HELD); ++d)
+#pragma unroll
+      for (int c = 0; c < COPIES; ++c)
+        if (d == 0 || (unsigned)d < KT) fetch((unsigned)d, d, c);
+  } else {
+#pragma unroll
+    for (int s = 0; s < STAGES; ++s) issueSlab(s);
+  }
   // (everything the tile store needs is worked out and asked for from here on, with the first slabs on their way)
   int offA = p.offsetA, offB = p.offsetB;
   float minC = 0.f, maxC = 0.f;
@@ -257,23 +326,71 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
     if (tid < BN && n0 + tid < N) csPre = (unsigned)csB[n0 + tid];
   }
 
-  wait_vmcnt<COPIES*(STAGES - 1)>();
-  __syncthreads();
+  if constexpr (ANY) {
+    settle(0, 0);
+#pragma unroll
+    for (int c = 0; c < COPIES; ++c) keep(0, 0, c);
+    if constexpr (HELD == 1) {  // both stages are free: no second trip to memory before the first matrix op
+      if (KT > 1) {
+        settle(1, 1);
+#pragma unroll
+        for (int c = 0; c < COPIES; ++c) keep(1, 1, c);
+      }
+    }
+    constexpr unsigned NEXT = HELD == 1 ? 2 : HELD;
+    if (NEXT < KT) {
+#pragma unroll
+      for (int c = 0; c < COPIES; ++c) fetch(NEXT, 0, c);
+    }
+    lds_barrier();
+  } else {
+    wait_vmcnt<COPIES*(STAGES - 1)>();
+    __syncthreads();
+  }
   v4i fa[2][MI], fb[2][NI];
 #pragma unroll
   for (int q = 0; q < NLOAD; ++q) loadOne(smem, smem + A_BYTES, 0, q, fa[0], fb[0]);
   static_assert(KS % 2 == 0, "the operand registers alternate per step");
-  for (unsigned kt = 0; kt < KT; ++kt) {
-    const unsigned cur = kt % STAGES, nxt = (kt + 1) % STAGES;
-    // k steps 0 .. KS-2 of slab kt, each reading the operands of the step after it
+  if constexpr (ANY) {
+    static_assert(KS == 4, "one step for the stores, one for the loads");
+    // Slab kt + 1, asked for HELD slabs ago, goes to the stage that slab kt - 1 has left; then the next one is asked for in its
+    // place.
+    auto oneSlab = [&](unsigned kt, int set, auto first) __attribute__((always_inline)) {
+      const unsigned cur = kt % STAGES, nxt = (kt + 1) % STAGES;
+      if constexpr (decltype(first)::value) {
+        step(fa[0], fb[0], fa[1], fb[1], cur, 1, nullptr);
+        step(fa[1], fb[1], fa[0], fb[0], cur, 2, nullptr);
+      } else {
+        settle(kt + 1, set);
+        step(fa[0], fb[0], fa[1], fb[1], cur, 1, [&](int c) __attribute__((always_inline)) { keep(kt + 1, set, c); });
+        step(fa[1], fb[1], fa[0], fb[0], cur, 2, [&](int c) __attribute__((always_inline)) { fetch(kt + 1 + HELD, set, c); });
+      }
+      step(fa[0], fb[0], fa[1], fb[1], cur, 3, nullptr);
+      lds_barrier();
+      step(fa[1], fb[1], fa[0], fb[0], nxt, 0, nullptr);
+    };
+    unsigned kt = 0;
+    if constexpr (HELD == 1) oneSlab(kt++, 0, std::true_type{});
+    for (; kt + HELD <= KT; kt += HELD) {
 #pragma unroll
-    for (int ks = 0; ks < KS - 1; ++ks)
-      step(fa[ks & 1], fb[ks & 1], fa[(ks + 1) & 1], fb[(ks + 1) & 1], cur, ks + 1, std::false_type{}, 0u);
-    wait_vmcnt<COPIES*(STAGES - 2)>();
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the reads of slab kt have returned
-    __syncthreads();
-    // last k step of slab kt; reads k step 0 of slab kt+1; refills the stage of slab kt
-    step(fa[1], fb[1], fa[0], fb[0], nxt, 0, std::true_type{}, kt + STAGES);
+      for (int u = 0; u < HELD; ++u) oneSlab(kt + u, (u + 1) % HELD, std::false_type{});
+    }
+#pragma unroll
+    for (int u = 0; u < HELD - 1; ++u)
+      if (kt + u < KT) oneSlab(kt + u, (u + 1) % HELD, std::false_type{});
+  } else {
+    for (unsigned kt = 0; kt < KT; ++kt) {
+      const unsigned cur = kt % STAGES, nxt = (kt + 1) % STAGES;
+      // k steps 0 .. KS-2 of slab kt, each reading the operands of the step after it
+#pragma unroll
+      for (int ks = 0; ks < KS - 1; ++ks)
+        step(fa[ks & 1], fb[ks & 1], fa[(ks + 1) & 1], fb[(ks + 1) & 1], cur, ks + 1, nullptr);
+      wait_vmcnt<COPIES*(STAGES - 2)>();
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the reads of slab kt have returned
+      __syncthreads();
+      // last k step of slab kt; reads k step 0 of slab kt+1; refills the stage of slab kt
+      step(fa[1], fb[1], fa[0], fb[0], nxt, 0, [&](int c) __attribute__((always_inline)) { issueCopy(kt + STAGES, c); });
+    }
   }
   wait_vmcnt<0>();
   __syncthreads();
@@ -315,6 +432,18 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
   int* C = WRITE_C ? p.C + (size_t)bi * p.strideC : nullptr;
   unsigned char* Q = REQUANT ? p.Q + (size_t)bi * p.strideC : nullptr;
 
+  // four results that begin in column `col`
+  auto store4 = [&](int* to, v4i v, unsigned col) __attribute__((always_inline)) {
+    if constexpr (!RAGGED) {
+      if (col < N) *reinterpret_cast<v4i*>(to) = v;  // N % 16 == 0: the four columns are in or out together
+    } else if (col + 4 <= N) {
+      *reinterpret_cast<words4*>(to) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 3; ++e)
+        if (col + e < N) to[e] = v[e];
+    }
+  };
   auto storeTile = [&](auto flavour) {
     constexpr int FLAVOUR = decltype(flavour)::value;  // 0 int32 only, 1 double shortcut, 2 exact int64, 3 fill, 4 int32 shortcut, 5 folded
 #pragma unroll
@@ -335,10 +464,10 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = (int)((unsigned)acc[i][j][4 * rq4 + e] + (unsigned)rt + (unsigned)ct[e]);
           if constexpr (WRITE_C && !REQUANT) {
-            *reinterpret_cast<v4i*>(stageC + l32 * CPITCH + tcol - wn * WN) = v4i{v[0], v[1], v[2], v[3]};
+            if constexpr (RAGGED) *reinterpret_cast<v4i*>(reinterpret_cast<int*>(stageQ) + trow * QPITCH + tcol) = v4i{v[0], v[1], v[2], v[3]};
+            else *reinterpret_cast<v4i*>(stageC + l32 * CPITCH + tcol - wn * WN) = v4i{v[0], v[1], v[2], v[3]};
           } else if constexpr (WRITE_C) {
-            if (grow < M && n0 + tcol < N)  // N % 16 == 0: the four columns are in or out together
-              *reinterpret_cast<v4i*>(C + (size_t)grow * N + n0 + tcol) = v4i{v[0], v[1], v[2], v[3]};
+            if (grow < M) store4(C + (size_t)grow * N + n0 + tcol, v4i{v[0], v[1], v[2], v[3]}, n0 + tcol);
           }
           if constexpr (FLAVOUR != 0) {
             unsigned q[4];
@@ -355,7 +484,17 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
           }
         }
       }
-      if constexpr (WRITE_C && !REQUANT) {
+      if constexpr (WRITE_C && !REQUANT && RAGGED) {
+        if (i < MI - 1) continue;
+        // Whole rows of the tile: a piece of a row that begins inside a memory line is two partial lines.
+        __syncthreads();
+#pragma unroll 4
+        for (int idx = tid; idx < BM * BN / 4; idx += kThreads) {
+          const int row = idx / (BN / 4), col = idx % (BN / 4) * 4;
+          const v4i v = *reinterpret_cast<const v4i*>(reinterpret_cast<const int*>(stageQ) + row * QPITCH + col);
+          if (m0 + row < M) store4(C + (size_t)(m0 + row) * N + n0 + col, v, n0 + col);
+        }
+      } else if constexpr (WRITE_C && !REQUANT) {
         // The wavefront's 32 rows lie in LDS: WN / 4 lanes write one row's WN columns.  From the registers a store writes 32
         // pieces of 32 bytes: us, 1024 x 768 x 3072 10.7 -> 10.3, 2048 x 512 x 2048 10.1 -> 9.6, 640 x 256 x 2048 5.7 -> 5.35.
         constexpr int PER = WN / 4, ROWS = 64 / PER;
@@ -365,7 +504,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
           const int row = t * ROWS + lane / PER, col = lane % PER * 4;
           const v4i v = *reinterpret_cast<const v4i*>(stageC + row * CPITCH + col);
           const unsigned to = m0 + wm * WM + 32 * i + row, at = n0 + wn * WN + col;
-          if (to < M && at < N) *reinterpret_cast<v4i*>(C + (size_t)to * N + at) = v;  // N % 16 == 0: four columns are in or out together
+          if (to < M) store4(C + (size_t)to * N + at, v, at);
         }
         wave_lds_order();
       }
@@ -381,7 +520,15 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
           if (grow >= M || gcol >= N) continue;
           const unsigned* src = reinterpret_cast<const unsigned*>(stageQ + row * QPITCH + ch * 16);
           v4i v = {(int)src[0], (int)src[1], (int)src[2], (int)src[3]};
-          *reinterpret_cast<v4i*>(Q + (size_t)grow * N + gcol) = v;
+          unsigned char* const to = Q + (size_t)grow * N + gcol;
+          if constexpr (!RAGGED) {
+            *reinterpret_cast<v4i*>(to) = v;
+          } else if (gcol + 16 <= N) {
+            *reinterpret_cast<bytes16*>(to) = v;
+          } else {
+            const unsigned char* from = reinterpret_cast<const unsigned char*>(src);
+            for (unsigned e = 0; e < N - gcol; ++e) to[e] = from[e];
+          }
         }
       }
     }
@@ -397,7 +544,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void qgemm_dma_kernel(const QGem
   }
 }
 
-template <int BM, int BN, int WGM, int WGN, int STAGES, bool REQUANT, bool WRITE_C, bool OWN_COLSUM>
+template <int BM, int BN, int WGM, int WGN, int DEPTH, int KIND, bool REQUANT, bool WRITE_C, bool OWN_COLSUM>
 int launch(hipStream_t stream, QGemmParams p) {
   constexpr int kThreads = WGM * WGN * 64;
   p.tilesM = (p.M + BM - 1) / BM;
@@ -409,11 +556,11 @@ int launch(hipStream_t stream, QGemmParams p) {
   const UDiv perBatch = udiv_prepare(p.tilesM * p.tilesN), band = udiv_prepare(4u * p.tilesN);
   p.perBatchMagic = perBatch.magic; p.perBatchShift = perBatch.shift;
   p.bandMagic = band.magic; p.bandShift = band.shift;
-  constexpr size_t ring = (size_t)STAGES * (BM + BN) * BK;
-  constexpr size_t epi = (size_t)(BM + BN) * 4 + (REQUANT ? (size_t)BM * (BN + 4) : (size_t)WGM * WGN * 32 * (BN / WGN + 4) * 4);
+  constexpr size_t ring = (size_t)(KIND == kAnyByte ? 2 : DEPTH) * (BM + BN) * BK;
+  constexpr size_t epi = (size_t)(BM + BN) * 4 + (REQUANT ? (size_t)BM * (BN + 4) : KIND == kAligned ? (size_t)WGM * WGN * 32 * (BN / WGN + 4) * 4 : (size_t)BM * (BN + 4) * 4);
   constexpr size_t lds = ring > epi ? ring : epi;
   static_assert(lds <= 160 * 1024, "LDS budget");
-  auto kern = qgemm_dma_kernel<BM, BN, WGM, WGN, STAGES, REQUANT, WRITE_C, OWN_COLSUM>;
+  auto kern = qgemm_dma_kernel<BM, BN, WGM, WGN, DEPTH, KIND, REQUANT, WRITE_C, OWN_COLSUM>;
   static bool attrSet[16] = {};  // per device: the attribute belongs to the function on one device
   int dev = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));
@@ -429,45 +576,76 @@ int launch(hipStream_t stream, QGemmParams p) {
 
 }  // namespace
 
-bool qgemm_dma_supported(const QGemmParams& p, bool requant) {
-  return (p.K % 16 == 0) && (p.N % 16 == 0) && ((uintptr_t)p.A % 16 == 0) && ((uintptr_t)p.B % 16 == 0) &&
-         (p.strideA % 16 == 0) && (p.strideB % 16 == 0) &&
-         (p.C == nullptr || ((uintptr_t)p.C % 16 == 0 && p.strideC % 4 == 0)) &&
-         (!requant || ((uintptr_t)p.Q % 16 == 0 && p.strideC % 16 == 0)) &&
-         ((unsigned long long)p.M + 512) * p.K < (1ull << 32) && ((unsigned long long)p.K + 1024) * p.N + 1024 < (1ull << 32);
-}
-
 namespace {
-template <int BM, int BN, int WGM, int WGN, int STAGES, bool OWN_COLSUM>
-int launch_for_outputs2(hipStream_t stream, const QGemmParams& p, bool requant) {
-  if (!requant) return launch<BM, BN, WGM, WGN, STAGES, false, true, OWN_COLSUM>(stream, p);
-  return p.C ? launch<BM, BN, WGM, WGN, STAGES, true, true, OWN_COLSUM>(stream, p)
-             : launch<BM, BN, WGM, WGN, STAGES, true, false, OWN_COLSUM>(stream, p);
+// Operands and results at multiples of `bytes` (the words of kWords: of four), copies' offsets within 32 bits.
+bool copies_supported(const QGemmParams& p, unsigned bytes) {
+  return p.K % bytes == 0 && p.N % bytes == 0 && (uintptr_t)p.A % bytes == 0 && (uintptr_t)p.B % bytes == 0 && p.strideA % bytes == 0 &&
+         p.strideB % bytes == 0 && ((unsigned long long)p.M + 512) * p.K < (1ull << 32) &&
+         ((unsigned long long)p.K + 1024) * p.N + 1024 < (1ull << 32);
 }
-template <int BM, int BN, int WGM, int WGN, int STAGES>
-int launch_for_outputs(hipStream_t stream, const QGemmParams& p, bool requant) {
-  return p.colsumExact ? launch_for_outputs2<BM, BN, WGM, WGN, STAGES, false>(stream, p, requant)
-                       : launch_for_outputs2<BM, BN, WGM, WGN, STAGES, true>(stream, p, requant);
+bool results_aligned(const QGemmParams& p, bool requant) {
+  return (p.C == nullptr || ((uintptr_t)p.C % 16 == 0 && p.strideC % 4 == 0)) &&
+         (!requant || ((uintptr_t)p.Q % 16 == 0 && p.strideC % 16 == 0));
 }
-}  // namespace
 
-int qgemm_dma_launch(hipStream_t stream, const QGemmParams& p, bool requant) {
-  const unsigned long long big = (unsigned long long)((p.M + 255) / 256) * ((p.N + 255) / 256) * p.batch;
-  if (big >= 192) {
-    if (qgemm_w4_supported(p)) return qgemm_w4_launch(stream, p, requant);
-    return launch_for_outputs<256, 256, 2, 4, 2>(stream, p, requant);
-  }
+template <int BM, int BN, int WGM, int WGN, int DEPTH, int KIND, bool OWN_COLSUM>
+int launch_for_outputs2(hipStream_t stream, const QGemmParams& p, bool requant) {
+  if (!requant) return launch<BM, BN, WGM, WGN, DEPTH, KIND, false, true, OWN_COLSUM>(stream, p);
+  return p.C ? launch<BM, BN, WGM, WGN, DEPTH, KIND, true, true, OWN_COLSUM>(stream, p)
+             : launch<BM, BN, WGM, WGN, DEPTH, KIND, true, false, OWN_COLSUM>(stream, p);
+}
+template <int BM, int BN, int WGM, int WGN, int DEPTH, int KIND>
+int launch_for_outputs(hipStream_t stream, const QGemmParams& p, bool requant) {
+  return p.colsumExact ? launch_for_outputs2<BM, BN, WGM, WGN, DEPTH, KIND, false>(stream, p, requant)
+                       : launch_for_outputs2<BM, BN, WGM, WGN, DEPTH, KIND, true>(stream, p, requant);
+}
+// 128 x 128 tiles or 64 x 128.  Up to 256 of the first (two to a CU at most of the second) the smaller ones, which run side by
+// side: us in 64 and 128 rows, 3189 x 3248 x 768 20.9 and 25.4, 715 x 1424 x 3584 13.4 and 15.0, 742 x 592 x 5024 10.2 and 10.7,
+// int32 alone 1024 x 768 x 3072 10.0 and 10.3.  Only at odd bytes, where B costs more, a K from 1400 on makes up for it (1148 x 3361 x
+// 3161 39 and 35).  With more of them a CU's tiles decide, rounded up, one of 128 rows at 1.75 (57 : 100) of the other, and a short K,
+// whose tiles are mostly start and end, favours those that more run side by side of: 1352 x 240 x 3120 9.0 and 10.1, 3582 x 656
+// x 1456 14.0 and 14.4, 2404 x 560 x 3600 19.0 and 20.8, but 1652 x 624 x 3792 17.9 and 13.8, 2013 x 2064 x 2320 26.9 and
+// 24.1, 1789 x 350 x 3822 17.0 and 15.0.  Of 100 products of 128 to 1408 such tiles three take more than 1.06 of the other (1.18
+// at most).
+bool takes_128_rows(unsigned long long t64, unsigned long long t128, unsigned K, Kind kind) {
+  const unsigned a = t128 > 256 ? (unsigned)((t128 + 255) / 256) * 100 : kind == kAnyByte ? 130 : 160;
+  const unsigned f = K < 512 ? 88 : K < 1400 ? 105 : 120;
+  return a * 100 < (unsigned)((t64 + 255) / 256) * 57 * f;
+}
+
+template <Kind KIND>
+int launch_tiles(hipStream_t stream, const QGemmParams& p, bool requant) {
+  const unsigned long long t64 = (unsigned long long)((p.M + 63) / 64) * ((p.N + 127) / 128) * p.batch;
+  const unsigned long long t128 = (unsigned long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
   // At most one 64x128 tile for each CU: with a CU to itself a workgroup waits for its slabs, not for the matrix cores (a
   // slab of 128 k every 0.53 us with one on its way, 0.41 with three), so its ring takes four stages.  us, two -> four: 256 x
   // 4096 x 4096 21.0 -> 17.2, 640 x 4096 x 1024 20.6 -> 17.0, 1024 x 4096 x 2048 24.8 (in 128x128) -> 18.4, 2048 x 1024 x
   // 1024 11.1 -> 9.3; six stages 19.4, 19.2, 20.7, 10.2.  Up to 768 k there is no difference (1024 x 768 x 768 7.2), and
-  // with more tiles, which then run one after another, four are slower (1024 x 768 x 3072 11.5 against 14.7).
-  const unsigned long long narrow = (unsigned long long)((p.M + 63) / 64) * ((p.N + 127) / 128) * p.batch;
-  if (narrow <= 256 && p.K > 768) return launch_for_outputs<64, 128, 1, 4, 4>(stream, p, requant);
-  // fewer than half a chip of 128x128 tiles: 64x128 tiles (four wavefronts side by side) put twice as many CUs to work
-  const unsigned long long mid = (unsigned long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
-  if (mid < 128) return launch_for_outputs<64, 128, 1, 4, 2>(stream, p, requant);
-  return launch_for_outputs<128, 128, 2, 2, 2>(stream, p, requant);
+  // with more tiles, which then run one after another, four are slower (1024 x 768 x 3072 11.5 against 14.7).  Through registers
+  // two slabs on their way instead of one, at the same line: 1335 x 6012 x 853 33 -> 29, 482 x 4948 x 1527 27 -> 24, 3 slabs 24.3.
+  const bool deep = t64 <= 256 && p.K > 768;
+  if constexpr (KIND == kAnyByte) {
+    if (deep) return launch_for_outputs<64, 128, 1, 4, 2, KIND>(stream, p, requant);
+    if (takes_128_rows(t64, t128, p.K, KIND)) return launch_for_outputs<128, 128, 2, 2, 1, KIND>(stream, p, requant);
+    return launch_for_outputs<64, 128, 1, 4, 1, KIND>(stream, p, requant);
+  } else {
+    if (deep) return launch_for_outputs<64, 128, 1, 4, 4, KIND>(stream, p, requant);
+    if (takes_128_rows(t64, t128, p.K, KIND)) return launch_for_outputs<128, 128, 2, 2, 2, KIND>(stream, p, requant);
+    return launch_for_outputs<64, 128, 1, 4, 2, KIND>(stream, p, requant);
+  }
+}
+}  // namespace
+
+bool qgemm_dma_supported(const QGemmParams& p, bool requant) { return copies_supported(p, 16) && results_aligned(p, requant); }
+
+int qgemm_dma_launch(hipStream_t stream, const QGemmParams& p, bool requant) {
+  if (qgemm_dma_supported(p, requant)) {
+    const unsigned long long big = (unsigned long long)((p.M + 255) / 256) * ((p.N + 255) / 256) * p.batch;
+    if (big < 192) return launch_tiles<kAligned>(stream, p, requant);
+    if (qgemm_w4_supported(p)) return qgemm_w4_launch(stream, p, requant);
+    return launch_for_outputs<256, 256, 2, 4, 2, kAligned>(stream, p, requant);
+  }
+  return copies_supported(p, 4) ? launch_tiles<kWords>(stream, p, requant) : launch_tiles<kAnyByte>(stream, p, requant);
 }
 
 }  // namespace tfcc_rocm

@@ -13,7 +13,7 @@
 //
 // Any K, N and alignment: buffer loads take any byte address, and those that would cross the end of an operand are moved
 // back to end with it.  Arithmetic and epilogue
-// are those of gemm_u8s8.hip (tfcc/mkl/operations/tfcc_mklquantization.cpp:33-69,176-201).
+// are described in gemm_u8s8.hip (tfcc/mkl/operations/tfcc_mklquantization.cpp:33-69,176-201).
 #include "common.hpp"
 #include "gemv.hpp"
 #include "qgemm_params.hpp"
@@ -68,7 +68,7 @@ __device__ __forceinline__ unsigned requantized(int v, const RequantScalars& rq)
   return (unsigned)requantize_one_exact((long long)v, rq);
 }
 
-// Operands shorter than one load (A below 16 bytes or B below 4, so K below 16): a thread per result.
+// Operands shorter than one load of the kernels in slabs (16 bytes, so K below 16): a thread per result.
 __global__ __launch_bounds__(256) void qgemm_tiny_kernel(const QGemmParams p, const QSmallOutputs o, unsigned long long total) {
   const unsigned long long i = (unsigned long long)blockIdx.x * 256 + threadIdx.x;
   int oA, oB;
@@ -353,7 +353,7 @@ bool qgemm_small_splits(hipStream_t stream, unsigned m, unsigned n, unsigned k, 
 }
 
 int qgemm_small_launch(hipStream_t stream, QGemmParams p, const QSmallOutputs& o, bool split) {
-  if ((unsigned long long)p.M * p.K < 16 || (unsigned long long)p.K * p.N < 4) {
+  if ((unsigned long long)p.M * p.K < 16 || (unsigned long long)p.K * p.N < 16) {
     const unsigned long long total = (unsigned long long)p.M * p.N * p.batch;
     if ((total + 255) / 256 > 0x7fffffffull) return set_error(TFCC_ROCM_INVALID_ARGUMENT, "quantized matmul: too many results");
     hipLaunchKernelGGL(qgemm_tiny_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, p, o, total);
