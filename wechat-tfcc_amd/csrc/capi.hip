@@ -107,6 +107,7 @@ int tfcc_rocm_stream_release(void* stream) {
   int dev = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));
   tfcc_rocm::sgemm_detail::sgemm_skinny_release_stream(dev, as_stream(stream));
+  tfcc_rocm::sgemm_detail::sgemm_deal_release_stream(dev, as_stream(stream));
   tfcc_rocm::qgemm_small_release_stream(dev, as_stream(stream));
   return tfcc_rocm::gemv_wide_release_stream(as_stream(stream));
 }

@@ -15,6 +15,7 @@
 // wavefront's column range) so that a lane owns NI consecutive output columns.
 #include "common.hpp"
 #include "sgemm_params.hpp"
+#include "sgemm_deal_plan.hpp"
 #include "sgemm_split_plan.hpp"
 #include "sgemm_tiles.hpp"
 
@@ -446,8 +447,20 @@ int dispatch(hipStream_t s, const SgemmParams& p, bool vec, bool small, bool tb,
   const unsigned m = p.M, n = p.N, k = p.K;
   // One product, or a few that share A, of too few rows and columns for the kernels below to occupy the chip.  (A true
   // batch keeps the tiled kernels, see below.)
-  if (fillBatch == 1 && small && sgemm_detail::sgemm_skinny_better(m, n, k))
-    return sgemm_detail::sgemm_skinny_launch(s, p, tb);
+  if (fillBatch == 1 && small) {
+    // Which of the two kernels whose workgroups share a K: the one for tiles of 32 rows where it is thought to be faster than the
+    // other by a tenth, or than the tiled kernels at all.  Of 220 products of 17 to 1024 rows and 768 k and more it takes 47,
+    // at 0.79 of the time (up to 1.0), another 13 lose a tenth without it.  What the bf16 matrix ops take stays there.
+    const double few = sgemm_detail::sgemm_skinny_microseconds(m, n, k);
+    const sgemm_deal_plan::Plan deal = sgemm_deal_plan::plan_of(m, n, k);
+    if (deal.splits > 0 &&
+        deal.us < (few > 0 ? .9 * few
+                   : sgemm_split_plan::kernel_of(m, n, k, p.lda, p.ldb, p.ldc, tb, fillBatch) == sgemm_split_plan::kNone
+                       ? sgemm_tiles::microseconds(m, n, k, fillBatch)
+                       : 0))
+      return sgemm_detail::sgemm_deal_launch(s, p, deal.splits, deal.blocks, tb);
+    if (few > 0) return sgemm_detail::sgemm_skinny_launch(s, p, tb);
+  }
   if (small) {
     const int split = sgemm_split_plan::kernel_of(m, n, k, p.lda, p.ldb, p.ldc, tb, fillBatch);
     if (split != sgemm_split_plan::kNone) return sgemm_detail::sgemm_split_launch(s, p, split, tb);

@@ -57,11 +57,11 @@ StreamPieces gPieces(sizeof(Meeting), 64, clear_counts);  // 4 MB each
 // walks what K has beyond a multiple of 64 row by row, 7000 in all.  Splits of less than 512 k end before their loads have
 // paid for the arrival: 2048 -> 512 with 9 rows, 7.4 us in splits of 256 against 6.2.  Below 256 k nothing is split in the tiled kernels either, and a product keeps their
 // bits, which are those it has in a batch.
-struct Plan { unsigned splits; bool better; };
+struct Plan { unsigned splits; bool better; double us; };
 Plan plan_of(unsigned m, unsigned n, unsigned k) {
   const unsigned long long tiles = (unsigned long long)((m + 15) / 16) * ((n + 15) / 16);
-  if (k < 256 || tiles > kMaxParts) return Plan{1, false};
-  Plan best{1, false};
+  if (k < 256 || tiles > kMaxParts) return Plan{1, false, 0};
+  Plan best{1, false, 0};
   unsigned long long bestCost = ~0ull;
   for (unsigned s = 1; s == 1 || (s <= k / 512 && tiles * s <= kMaxParts); ++s) {
     const unsigned long long perCu = (tiles * s + 255) / 256;
@@ -71,6 +71,7 @@ Plan plan_of(unsigned m, unsigned n, unsigned k) {
       bestCost = cost;
     }
   }
+  best.us = 2.5 + bestCost * 1e-4;
   const unsigned long long streaming = ((unsigned long long)k * (m <= 4 ? 24 : 29) + (k % 64 != 0 ? 70000 : 0)) * 9 / 10;
   best.better = bestCost < (m > 8 ? (unsigned long long)k * 46 : streaming);
   return best;
@@ -306,7 +307,10 @@ int launch_skinny(hipStream_t stream, SgemmParams p) {
 
 namespace sgemm_detail {
 
-bool sgemm_skinny_better(unsigned m, unsigned n, unsigned k) { return plan_of(m, n, k).better; }
+double sgemm_skinny_microseconds(unsigned m, unsigned n, unsigned k) {
+  const Plan plan = plan_of(m, n, k);
+  return plan.better ? plan.us : 0;
+}
 
 int sgemm_skinny_launch(hipStream_t stream, const SgemmParams& p, bool transB) {
   return transB ? launch_skinny<true>(stream, p) : launch_skinny<false>(stream, p);
