@@ -20,6 +20,8 @@
 // same bits, and so does a launch that may not use the memory in which the splits meet (a stream that is being captured): its
 // workgroups take all splits of a tile, one after the other.  Bias, residual and the erf-form GELU follow as in the other kernels
 // (tfcc/mkl/interfaces/tfcc_mklblasinterface.cpp:41-67, 69-78, 87-118).
+#include <type_traits>
+
 #include "common.hpp"
 #include "sgemm_deal_plan.hpp"
 #include "sgemm_params.hpp"
@@ -50,11 +52,13 @@ StreamPieces gPieces(sizeof(Meeting), 64, clear_counts);  // 12 MB each
 // wait in LDS.  Replayed from a graph, the kernels of sgemm_wave96.hip and sgemm_skinny.hip -> this one: 75 x 4928 x 1344 29.5 -> 30.2
 // us, 96 x 7608 x 824 47.7 -> 46.6, 24 x 3183 x 2827 21.2 -> 23.9, 128 x 2384 x 992 16.7 -> 14.2, 466 x 5928 x 288 36.5 -> 32.9, 128 x 3072 x 768
 // 19.4 -> 23.5, 75 x 3072 x 832 19.4 -> 18.4, 369 x 1220 x 170 10.0 -> 11.5 (one team: 47, 69, 36, 16, 50, 38, 21 and 13).
-template <int NB, bool TRANSB, bool ALONE>
+template <int NB, bool TRANSB, bool ALONE, class Arguments>
 __global__ __launch_bounds__(64 * kWaves * (ALONE ? 2 : 1), ALONE ? 4 : 2) void sgemm_deal_kernel(const float* hotA, const float* hotB, unsigned M, unsigned N, unsigned K,
                                                                     unsigned lda, unsigned ldb, unsigned tilesM, unsigned tilesTotal,
                                                                     unsigned chunk, unsigned splits, unsigned perWave, Meeting* meeting,
-                                                                    const SgemmParams p) {
+                                                                    const Arguments arguments) {
+  const SgemmParams p = arguments.whole();
+  constexpr bool GROUPED = std::is_same<Arguments, SgemmParams>::value;
   constexpr int TEAMS = ALONE ? 2 : 1, THREADS = 64 * kWaves * TEAMS;
   constexpr int SETS = NB == 1 && !ALONE ? 4 : 2, ACCS = 4, ROWS = 1024 / THREADS, OUT = NB * ROWS;  // steps on their way, results that a thread finishes
   constexpr unsigned HELD = ALONE ? 4 : 1;  // splits that wait in LDS
@@ -68,7 +72,7 @@ __global__ __launch_bounds__(64 * kWaves * (ALONE ? 2 : 1), ALONE ? 4 : 2) void 
   const unsigned tn = L / tilesM, tm = L - tn * tilesM, group = blockIdx.y;
   const unsigned m0 = tm * 32, n0 = tn * 32 * NB;
   const float* A = hotA;
-  const float* B = p.groups ? p.groupB[group] : hotB;
+  const float* B = GROUPED && p.groups ? p.groupB[group] : hotB;
 
   // A lane has row lane % 32, NB consecutive columns from NB (lane % 32) on, and eight consecutive k of a step's sixteen.  Rows past
   // the edge read the last one, and their sums are dropped; words past the end of an operand read zeros.
@@ -143,7 +147,7 @@ __global__ __launch_bounds__(64 * kWaves * (ALONE ? 2 : 1), ALONE ? 4 : 2) void 
   auto colOf = [&](int q) __attribute__((always_inline)) { return n0 + NB * edge + q % NB; };
   auto mine = [&](int q) __attribute__((always_inline)) { return rowOf(q) < M && colOf(q) < N; };
   auto loadFinish = [&]() __attribute__((always_inline)) {
-    const float* bias = p.groups ? p.groupBias[group] : p.bias;
+    const float* bias = GROUPED && p.groups ? p.groupBias[group] : p.bias;
 #pragma unroll
     for (int q = 0; q < OUT; ++q) {
       if (q < NB) bv[q] = bias && colOf(q) < N ? bias[colOf(q)] : 0.f;
@@ -253,7 +257,7 @@ __global__ __launch_bounds__(64 * kWaves * (ALONE ? 2 : 1), ALONE ? 4 : 2) void 
       }
     }
   }
-  float* C = p.groups ? p.groupC[group] : p.C;
+  float* C = GROUPED && p.groups ? p.groupC[group] : p.C;
 #pragma unroll
   for (int q = 0; q < OUT; ++q) {
     if (!mine(q)) continue;
@@ -277,9 +281,15 @@ int launch_deal(hipStream_t stream, SgemmParams p, unsigned splits) {
   }
   const bool alone = splits > 1 && meeting == nullptr;  // then in tiles of one block: their number, not that of the splits, fills the chip
   if (alone && !sgemm_detail::set_tiles(p, 32, 32)) return set_error(TFCC_ROCM_INVALID_ARGUMENT, "sgemm: too many tiles");
-  auto kern = alone ? sgemm_deal_kernel<1, TRANSB, true> : sgemm_deal_kernel<NB, TRANSB, false>;
-  hipLaunchKernelGGL(kern, dim3(p.chunk * 8, groups, alone ? 1u : splits), dim3(64 * kWaves * (alone ? 2 : 1)), 0, stream, p.A, p.B, p.M, p.N, p.K, p.lda,
-                     p.ldb, p.tilesM, p.tilesTotal, p.chunk, splits, (p.K + kStep - 1) / kStep / (splits * kWaves), meeting, p);
+  auto launch = [&](const auto& arguments) {
+    using Arguments = std::decay_t<decltype(arguments)>;
+    auto kern = alone ? sgemm_deal_kernel<1, TRANSB, true, Arguments> : sgemm_deal_kernel<NB, TRANSB, false, Arguments>;
+    hipLaunchKernelGGL(kern, dim3(p.chunk * 8, groups, alone ? 1u : splits), dim3(64 * kWaves * (alone ? 2 : 1)), 0, stream, p.A, p.B, p.M,
+                       p.N, p.K, p.lda, p.ldb, p.tilesM, p.tilesTotal, p.chunk, splits, (p.K + kStep - 1) / kStep / (splits * kWaves),
+                       meeting, arguments);
+  };
+  if (p.groups) launch(p);
+  else launch(sgemm_detail::SgemmFinish(p));
   return check_launch("sgemm");
 }
 

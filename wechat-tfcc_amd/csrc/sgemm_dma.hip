@@ -17,6 +17,8 @@
 // Taken for B not transposed.  Addresses need to be multiples of four bytes only, and the range check of a copy looks
 // at every word.  A partial slab of A cannot be zeroed on its way into LDS: RAGGED (K not a multiple of 32) masks the
 // operands of the slab in which K ends as they are read.
+#include <type_traits>
+
 #include "common.hpp"
 #include "lds_dma.hpp"
 #include "sgemm_params.hpp"
@@ -43,8 +45,9 @@ __device__ __forceinline__ int row_swizzle(int row) { return (row >> 1) & 7; }
 // accumulator per would-be group (slab s goes to accumulator s % VSPLIT) and the same final additions in
 // group order - bit for bit the result of KSPLIT = VSPLIT, for launches that fill the chip without
 // splitting K across wavefronts (several products in one launch).
-template <int WGM, int WGN, int NI, int KSPLIT, int STAGES, int VSPLIT, bool RAGGED>
-__global__ __launch_bounds__(WGM * WGN * 64 * KSPLIT) void sgemm_dma_kernel(const SgemmParams p) {
+template <int WGM, int WGN, int NI, int KSPLIT, int STAGES, int VSPLIT, bool RAGGED, class Arguments>
+__global__ __launch_bounds__(WGM * WGN * 64 * KSPLIT) void sgemm_dma_kernel(const Arguments arguments) {
+  const SgemmParams p = arguments.whole();
   static_assert(VSPLIT == 1 || KSPLIT == 1, "accumulators per would-be group only without real groups");
   static_assert(NI == 1 || NI == 3 || NI == 4, "a lane reads its B operands as one word, three words 32 columns apart or four consecutive words");
   constexpr bool STRIDED = NI == 3;  // lane lrow owns columns lrow, lrow + 32, lrow + 64 of the wavefront's block
@@ -74,10 +77,12 @@ __global__ __launch_bounds__(WGM * WGN * 64 * KSPLIT) void sgemm_dma_kernel(cons
   // they need of the argument block is named before the first branch (one round trip to memory instead of one per
   // basic block), and the divisions of the tile mapping are multiplications by constants the launcher worked out.
   asm volatile("" ::"s"(p.chunk), "s"(p.tilesTotal), "s"(p.tilesM), "s"(p.tilesN), "s"(p.perBatchMagic),
-               "s"(p.perBatchShift), "s"(p.bandMagic), "s"(p.bandShift), "s"(p.innerMagic), "s"(p.innerShift),
-               "s"(p.batchInner), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.lda), "s"(p.ldb), "s"(p.groups), "s"(p.A), "s"(p.B),
-               "s"(p.strideA), "s"(p.strideB), "s"(p.innerA), "s"(p.innerB), "s"(p.groupB[0]), "s"(p.groupB[1]), "s"(p.groupB[2]),
-               "s"(p.groupB[3]));
+               "s"(p.perBatchShift), "s"(p.bandMagic), "s"(p.bandShift), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.lda), "s"(p.ldb),
+               "s"(p.A), "s"(p.B));
+  if constexpr (!std::is_same<Arguments, sgemm_detail::SgemmLone>::value) asm volatile("" ::"s"(p.strideA), "s"(p.strideB));
+  if constexpr (std::is_same<Arguments, SgemmParams>::value)
+    asm volatile("" ::"s"(p.innerMagic), "s"(p.innerShift), "s"(p.batchInner), "s"(p.groups), "s"(p.innerA), "s"(p.innerB),
+                 "s"(p.groupB[0]), "s"(p.groupB[1]), "s"(p.groupB[2]), "s"(p.groupB[3]));
   unsigned tm, tn, bi;
   {
     // consecutive workgroup ids land on different XCDs: hand each XCD a contiguous run of tiles
@@ -370,7 +375,7 @@ __global__ __launch_bounds__(WGM * WGN * 64 * KSPLIT) void sgemm_dma_kernel(cons
   }
 }
 
-template <int WGM, int WGN, int NI, int KSPLIT, int STAGES, int VSPLIT, bool RAGGED>
+template <int WGM, int WGN, int NI, int KSPLIT, int STAGES, int VSPLIT, bool RAGGED, class Arguments>
 int launch_form(hipStream_t stream, SgemmParams p) {
   constexpr int GW = WGM * WGN, BM = WGM * 32, BN = WGN * 32 * NI;
   constexpr int STAGE_BYTES = (BM + BN) * BK * 4, UNITS = STAGE_BYTES / 1024;
@@ -378,7 +383,7 @@ int launch_form(hipStream_t stream, SgemmParams p) {
   constexpr size_t lds = (size_t)KSPLIT * (STAGES * STAGE_BYTES + (COPIES * GW != UNITS ? 1024 : 0));
   static_assert(lds <= 160 * 1024 && (size_t)(KSPLIT - 1) * BM * BN * sizeof(float) <= lds, "LDS budget");
   if (!sgemm_detail::set_tiles(p, BM, BN)) return set_error(TFCC_ROCM_INVALID_ARGUMENT, "sgemm: too many tiles");
-  auto kern = sgemm_dma_kernel<WGM, WGN, NI, KSPLIT, STAGES, VSPLIT, RAGGED>;
+  auto kern = sgemm_dma_kernel<WGM, WGN, NI, KSPLIT, STAGES, VSPLIT, RAGGED, Arguments>;
   static bool attrSet[16] = {};  // per device: the attribute belongs to the function on one device
   int dev = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));
@@ -388,14 +393,21 @@ int launch_form(hipStream_t stream, SgemmParams p) {
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attrSet[dev] = true;
   }
-  hipLaunchKernelGGL(kern, dim3(p.chunk * 8), dim3(GW * 64 * KSPLIT), lds, stream, p);
+  hipLaunchKernelGGL(kern, dim3(p.chunk * 8), dim3(GW * 64 * KSPLIT), lds, stream, Arguments(p));
   return check_launch("sgemm");
 }
 
 template <int WGM, int WGN, int NI, int KSPLIT, int STAGES, int VSPLIT = 1>
 int launch(hipStream_t stream, const SgemmParams& p) {
-  return p.K % BK != 0 ? launch_form<WGM, WGN, NI, KSPLIT, STAGES, VSPLIT, true>(stream, p)
-                       : launch_form<WGM, WGN, NI, KSPLIT, STAGES, VSPLIT, false>(stream, p);
+  auto launch = [&](auto ragged) {
+    constexpr bool RAGGED = decltype(ragged)::value;
+    if constexpr (VSPLIT == 1) {  // (several groups in one are a launch of several products)
+      if (sgemm_detail::SgemmLone::takes(p)) return launch_form<WGM, WGN, NI, KSPLIT, STAGES, VSPLIT, RAGGED, sgemm_detail::SgemmLone>(stream, p);
+      if (sgemm_detail::SgemmBatch::takes(p)) return launch_form<WGM, WGN, NI, KSPLIT, STAGES, VSPLIT, RAGGED, sgemm_detail::SgemmBatch>(stream, p);
+    }
+    return launch_form<WGM, WGN, NI, KSPLIT, STAGES, VSPLIT, RAGGED, SgemmParams>(stream, p);
+  };
+  return p.K % BK != 0 ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
 }  // namespace

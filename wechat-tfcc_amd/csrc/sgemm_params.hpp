@@ -28,7 +28,71 @@ struct SgemmParams {
   unsigned tilesM, tilesN, tilesTotal, chunk;
   // division by tilesM * tilesN, by 4 * tilesN and by batchInner as multiply-high and shift (set_tiles)
   unsigned perBatchMagic, perBatchShift, bandMagic, bandShift, innerMagic, innerShift;
+#if defined(__HIPCC__)
+  __device__ __forceinline__ const SgemmParams& whole() const { return *this; }
+#endif
 };
+
+// Shorter argument blocks for what most launches are: one product, a flat batch without epilogue, and (behind the leading
+// scalar arguments of kernels that have those) what the tile store of one product needs.  A launch whose arguments take more than
+// 112 bytes costs the host 0.65 us more in two of three processes: us from launch to launch of an empty kernel, 112 bytes 2.75,
+// 116 bytes 3.4, 320 bytes 3.5 (2.3 whatever the size in the others).  A small product is bound by that: 1 x 768 x 768 4.5 -> 4.1.
+// whole(): the block as the kernels read it, everything else a constant.
+constexpr size_t kShortArguments = 112;
+
+struct SgemmLone {
+  const float *A, *B, *bias, *residual;
+  float* C;
+  unsigned lda, ldb, ldc, M, N, K, tilesM, tilesN, tilesTotal, chunk, bandMagic, bandShift;
+  int act;
+  explicit SgemmLone(const SgemmParams& p)
+      : A(p.A), B(p.B), bias(p.bias), residual(p.residual), C(p.C), lda(p.lda), ldb(p.ldb), ldc(p.ldc), M(p.M), N(p.N), K(p.K),
+        tilesM(p.tilesM), tilesN(p.tilesN), tilesTotal(p.tilesTotal), chunk(p.chunk), bandMagic(p.bandMagic), bandShift(p.bandShift),
+        act(p.act) {}
+  static bool takes(const SgemmParams& p) { return p.groups == 0 && p.batch == 1; }
+  __device__ __forceinline__ SgemmParams whole() const {
+    SgemmParams p{};
+    p.A = A; p.B = B; p.bias = bias; p.residual = residual; p.C = C; p.act = act;
+    p.lda = lda; p.ldb = ldb; p.ldc = ldc; p.M = M; p.N = N; p.K = K; p.batch = p.batchInner = 1;
+    p.tilesM = tilesM; p.tilesN = tilesN; p.tilesTotal = tilesTotal; p.chunk = chunk; p.bandMagic = bandMagic; p.bandShift = bandShift;
+    p.perBatchShift = 31;  // with a magic number of 0: every tile is in batch entry 0
+    return p;
+  }
+};
+
+struct SgemmBatch {
+  const float *A, *B;
+  float* C;
+  unsigned long long strideA, strideB, strideC;
+  unsigned lda, ldb, ldc, M, N, K, tilesM, tilesN, tilesTotal, chunk, perBatchMagic, perBatchShift, bandMagic, bandShift;
+  explicit SgemmBatch(const SgemmParams& p)
+      : A(p.A), B(p.B), C(p.C), strideA(p.strideA), strideB(p.strideB), strideC(p.strideC), lda(p.lda), ldb(p.ldb), ldc(p.ldc), M(p.M),
+        N(p.N), K(p.K), tilesM(p.tilesM), tilesN(p.tilesN), tilesTotal(p.tilesTotal), chunk(p.chunk), perBatchMagic(p.perBatchMagic),
+        perBatchShift(p.perBatchShift), bandMagic(p.bandMagic), bandShift(p.bandShift) {}
+  static bool takes(const SgemmParams& p) { return p.groups == 0 && p.batchInner == 1 && !p.bias && !p.residual && p.act == 0; }
+  __device__ __forceinline__ SgemmParams whole() const {
+    SgemmParams p{};
+    p.A = A; p.B = B; p.C = C; p.strideA = strideA; p.strideB = strideB; p.strideC = strideC;
+    p.lda = lda; p.ldb = ldb; p.ldc = ldc; p.M = M; p.N = N; p.K = K; p.batchInner = 1;
+    p.tilesM = tilesM; p.tilesN = tilesN; p.tilesTotal = tilesTotal; p.chunk = chunk;
+    p.perBatchMagic = perBatchMagic; p.perBatchShift = perBatchShift; p.bandMagic = bandMagic; p.bandShift = bandShift;
+    return p;
+  }
+};
+
+struct SgemmFinish {
+  const float *bias, *residual;
+  float* C;
+  unsigned ldc;
+  int act;
+  explicit SgemmFinish(const SgemmParams& p) : bias(p.bias), residual(p.residual), C(p.C), ldc(p.ldc), act(p.act) {}
+  __device__ __forceinline__ SgemmParams whole() const {
+    SgemmParams p{};
+    p.bias = bias; p.residual = residual; p.C = C; p.ldc = ldc; p.act = act; p.batch = p.batchInner = 1;
+    return p;
+  }
+};
+static_assert(sizeof(SgemmLone) <= kShortArguments && sizeof(SgemmBatch) <= kShortArguments && sizeof(SgemmFinish) == 32, "short");
 
 // Fills in the tile counts for BM x BN tiles; false when there are too many tiles for one grid.
 inline bool set_tiles(SgemmParams& p, unsigned bm, unsigned bn) {

@@ -85,12 +85,14 @@ Plan plan_of(unsigned m, unsigned n, unsigned k) {
 // What is under way has to be the same on every path to a matrix op, or the compiler waits for every load before it uses the
 // first (with a condition in front of every load 1 x 16384 x 64 in a graph took 37 us instead of 26): whole batches are asked for without a condition, and the last 0 to 3 steps of a wavefront have code of their own
 // for each number.
-template <bool TRANSB, int TEAMS>
+template <bool TRANSB, int TEAMS, class Arguments>
 __global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(const float* hotA, const float* hotB, unsigned M,
                                                                               unsigned N, unsigned K, unsigned lda, unsigned ldb,
                                                                               unsigned tilesM, unsigned tilesTotal, unsigned chunk,
                                                                               unsigned splits, unsigned perWave, Meeting* meeting,
-                                                                              const SgemmParams p) {
+                                                                              const Arguments arguments) {
+  const SgemmParams p = arguments.whole();
+  constexpr bool GROUPED = std::is_same<Arguments, SgemmParams>::value;
   constexpr unsigned ROUNDS = TEAMS == 1 ? 1 : 3, HELD = TEAMS * ROUNDS;  // splits that wait in LDS
   __shared__ float part[HELD * kWaves][4][64];
   __shared__ unsigned arrived;
@@ -103,7 +105,7 @@ __global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(co
   const unsigned tn = L / tilesM, tm = L - tn * tilesM, group = blockIdx.y;
   const unsigned m0 = tm * 16, n0 = tn * 16;
   const float* A = hotA;
-  const float* B = p.groups ? p.groupB[group] : hotB;
+  const float* B = GROUPED && p.groups ? p.groupB[group] : hotB;
   // (no range check: every offset below lies inside the operand)
   const __amdgpu_buffer_rsrc_t rsrcA = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A), 0, -1, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrcB = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), 0, -1, 0x00020000);
@@ -140,7 +142,7 @@ __global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(co
   const bool finisher = threadIdx.x < 256, mine = finisher && grow < M && gcol < N;
   float bv = 0.f, rv = 0.f;
   auto loadFinish = [&]() __attribute__((always_inline)) {
-    const float* bias = p.groups ? p.groupBias[group] : p.bias;
+    const float* bias = GROUPED && p.groups ? p.groupBias[group] : p.bias;
     if (mine && bias) bv = bias[gcol];
     if (mine && p.residual) rv = p.residual[(size_t)grow * N + gcol];
   };
@@ -279,7 +281,7 @@ __global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(co
   v += bv;
   if (p.residual) v += rv;
   if (p.act == 1) v = gelu_erf_f32(v);
-  float* C = p.groups ? p.groupC[group] : p.C;
+  float* C = GROUPED && p.groups ? p.groupC[group] : p.C;
   C[(size_t)grow * p.ldc + gcol] = v;
 }
 
@@ -296,10 +298,15 @@ int launch_skinny(hipStream_t stream, SgemmParams p) {
     meeting = static_cast<Meeting*>(gPieces.of(dev, stream));
   }
   const bool alone = splits > 1 && meeting == nullptr;
-  auto kern = alone ? sgemm_skinny_kernel<TRANSB, 2> : sgemm_skinny_kernel<TRANSB, 1>;
-  hipLaunchKernelGGL(kern, dim3(p.chunk * 8, groups, alone ? 1u : splits), dim3(64 * kWaves * (alone ? 2 : 1)), 0, stream, p.A, p.B,
-                     (unsigned)p.M, (unsigned)p.N, (unsigned)p.K, (unsigned)p.lda, (unsigned)p.ldb, p.tilesM, p.tilesTotal, p.chunk,
-                     splits, p.K / 16 / (splits * kWaves), meeting, p);
+  auto launch = [&](const auto& arguments) {
+    using Arguments = std::decay_t<decltype(arguments)>;
+    auto kern = alone ? sgemm_skinny_kernel<TRANSB, 2, Arguments> : sgemm_skinny_kernel<TRANSB, 1, Arguments>;
+    hipLaunchKernelGGL(kern, dim3(p.chunk * 8, groups, alone ? 1u : splits), dim3(64 * kWaves * (alone ? 2 : 1)), 0, stream, p.A, p.B,
+                       (unsigned)p.M, (unsigned)p.N, (unsigned)p.K, (unsigned)p.lda, (unsigned)p.ldb, p.tilesM, p.tilesTotal, p.chunk,
+                       splits, p.K / 16 / (splits * kWaves), meeting, arguments);
+  };
+  if (p.groups) launch(p);
+  else launch(sgemm_detail::SgemmFinish(p));
   return check_launch("sgemm");
 }
 

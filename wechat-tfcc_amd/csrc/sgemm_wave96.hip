@@ -37,6 +37,8 @@
 // 87-118).  Taken for B not transposed.  The copies need addresses that are multiples of four bytes only, and their range
 // check looks at every word, so operands that are not aligned to 16 bytes, rows whose length is no multiple of four and
 // a K that is no multiple of 32 take the RAGGED form of the same loop.
+#include <type_traits>
+
 #include "common.hpp"
 #include "copy_offsets.hpp"
 #include "lds_dma.hpp"
@@ -58,10 +60,11 @@ __device__ __forceinline__ int a_row_swizzle(int row) {
   return BK == 32 ? (row >> 1) & 7 : BK == 16 ? (row >> 2) & 3 : (row >> 2) & 1;
 }
 
-template <int WGM, int KSPLIT, int BK, int STAGES, bool PLAIN, int NI, bool RAMP, bool RAGGED>
+template <int WGM, int KSPLIT, int BK, int STAGES, bool PLAIN, int NI, bool RAMP, bool RAGGED, class Arguments>
 __global__ __launch_bounds__(64 * WGM * KSPLIT > 256 ? 64 * WGM * KSPLIT : 256) void sgemm_wave96_kernel(
     const float* hotA, const float* hotB, const float* hotB1, const float* hotB2, unsigned hotM, unsigned hotN,
-    unsigned hotK, unsigned hotLda, unsigned hotLdb, unsigned hotBatch, const SgemmParams p) {
+    unsigned hotK, unsigned hotLda, unsigned hotLdb, unsigned hotBatch, const Arguments arguments) {
+  const SgemmParams p = arguments.whole();
   // The leading arguments repeat what the first copies need: scalar arguments at the front of the list arrive in
   // registers with the wavefront, the structure has to be fetched from the argument block first, and nothing of it
   // is looked at before the first slabs are on their way when PLAIN (every batch entry's A starts at hotA, and
@@ -121,7 +124,7 @@ __global__ __launch_bounds__(64 * WGM * KSPLIT > 256 ? 64 * WGM * KSPLIT : 256) 
   }
   const unsigned m0 = tm * BM, n0 = tn * BN;
   const unsigned M = hotM, N = hotN, K = hotK;
-  const bool grouped = (hotBatch >> 30) & 1u;
+  const bool grouped = std::is_same<Arguments, SgemmParams>::value && ((hotBatch >> 30) & 1u);
   const float* A = hotA;
   const float* B = hotB;
   if (grouped) {
@@ -486,24 +489,35 @@ int launch_wave96(hipStream_t stream, SgemmParams p) {
   TFCC_REQUIRE(p.batch < (1u << 30), "sgemm: batch of %u", p.batch);
   // a piece of four columns that crosses the end of B's last row passes the range check on the lane offset alone
   const bool ragged = p.K % 32 != 0 || p.N % 4 != 0;
-  auto kern = plain ? (ragged ? sgemm_wave96_kernel<WGM, KSPLIT, BK, STAGES, true, NI, RAMP, true>
-                              : sgemm_wave96_kernel<WGM, KSPLIT, BK, STAGES, true, NI, RAMP, false>)
-                    : (ragged ? sgemm_wave96_kernel<WGM, KSPLIT, BK, STAGES, false, NI, RAMP, true>
-                              : sgemm_wave96_kernel<WGM, KSPLIT, BK, STAGES, false, NI, RAMP, false>);
-  static bool attrSet[16][4] = {};  // per device: the attribute belongs to the function on one device
+  const unsigned hotBatch = p.batch | (p.groups ? 1u << 30 : 0u);
   int dev = 0;
   TFCC_HIP_CHECK(hipGetDevice(&dev));
   TFCC_REQUIRE(dev >= 0 && dev < 16, "device index %d", dev);
-  const int which = (plain ? 1 : 0) + (ragged ? 2 : 0);
-  if (!attrSet[dev][which]) {
-    TFCC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attrSet[dev][which] = true;
+  static bool attrSet[16][6] = {};  // per device: the attribute belongs to the function on one device
+  auto launch = [&](auto plainForm, auto raggedForm, const auto& arguments, int which) {
+    auto kern = sgemm_wave96_kernel<WGM, KSPLIT, BK, STAGES, decltype(plainForm)::value, NI, RAMP, decltype(raggedForm)::value,
+                                    std::decay_t<decltype(arguments)>>;
+    if (!attrSet[dev][which]) {
+      TFCC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      attrSet[dev][which] = true;
+    }
+    hipLaunchKernelGGL(kern, dim3(p.chunk * 8), dim3(64 * WGM * KSPLIT), lds, stream, p.A, p.groups ? p.groupB[0] : p.B,
+                       p.groups ? p.groupB[1] : nullptr, p.groups ? p.groupB[2] : nullptr, (unsigned)p.M, (unsigned)p.N,
+                       (unsigned)p.K, (unsigned)p.lda, (unsigned)p.ldb, hotBatch, arguments);
+    return (int)TFCC_ROCM_OK;
+  };
+  const std::true_type yes;
+  const std::false_type no;
+  int status;
+  if (sgemm_detail::SgemmLone::takes(p)) {
+    const sgemm_detail::SgemmFinish finish(p);
+    status = ragged ? launch(yes, yes, finish, 4) : launch(yes, no, finish, 5);
+  } else if (plain) {
+    status = ragged ? launch(yes, yes, p, 3) : launch(yes, no, p, 1);
+  } else {
+    status = ragged ? launch(no, yes, p, 2) : launch(no, no, p, 0);
   }
-  const unsigned hotBatch = p.batch | (p.groups ? 1u << 30 : 0u);
-  hipLaunchKernelGGL(kern, dim3(p.chunk * 8), dim3(64 * WGM * KSPLIT), lds, stream, p.A, p.groups ? p.groupB[0] : p.B,
-                     p.groups ? p.groupB[1] : nullptr, p.groups ? p.groupB[2] : nullptr, (unsigned)p.M, (unsigned)p.N,
-                     (unsigned)p.K, (unsigned)p.lda, (unsigned)p.ldb, hotBatch, p);
+  if (status != TFCC_ROCM_OK) return status;
   return check_launch("sgemm");
 }
 

@@ -76,10 +76,21 @@ __device__ __forceinline__ void stream_partial_sums(const float* __restrict__ A,
         }
       }
     } else {
-      for (unsigned r = 0; r < (unsigned)PIECE && sub * PIECE + r < rows; ++r) {
-        const float b = bp[(size_t)r * ldb];
+      // The chunk in which K ends: rows past the end read the last one and count as zeros.  Eight at a time like the others: row
+      // by row each waited for the one before (replayed 2 x 144 x 232 3.9 -> 2.5 us, 1 x 91 x 3560 5.1 -> 3.8, 1 x 232 x 1344
+      // 5.5 -> 3.8, 8 x 133 x 4045 4.1 -> 3.9).
+      for (unsigned r = 0; r < (unsigned)PIECE && r < rows; r += kRows) {
+        float b[kRows];
 #pragma unroll
-        for (int m = 0; m < MR; ++m) acc[m] = fmaf(mine[m][sub * PIECE + r], b, acc[m]);
+        for (unsigned u = 0; u < (unsigned)kRows; ++u) {
+          const unsigned row = sub * PIECE + r + u;
+          b[u] = B[(size_t)(k + min(row, rows - 1)) * ldb + colRead];
+          b[u] = row < rows ? b[u] : 0.f;
+        }
+#pragma unroll
+        for (int m = 0; m < MR; ++m)
+#pragma unroll
+          for (int q = 0; q < kRows; ++q) acc[m] = fmaf(mine[m][sub * PIECE + r + q], b[q], acc[m]);
       }
     }
   }
@@ -100,8 +111,9 @@ __device__ __forceinline__ float summed(float (*smem)[MR][64], unsigned row, uns
   return v;
 }
 
-template <int MR, int COLS>
-__global__ __launch_bounds__(kWaves * 64) void sgemv_kernel(SgemmParams p) {
+template <int MR, int COLS, class Arguments>
+__global__ __launch_bounds__(kWaves * 64) void sgemv_kernel(const Arguments arguments) {
+  const SgemmParams p = arguments.whole();
   // [wave][row of A][64]: first each wavefront's current 64 values of every row of A, at the end its partial sums
   __shared__ __attribute__((aligned(16))) float smem[kWaves][MR][64];
   const unsigned lane = threadIdx.x & 63;
@@ -181,9 +193,15 @@ __global__ __launch_bounds__(kWaves * 64) void lstm_step_kernel(LstmStepParams p
   }
 }
 
+// The short arguments where the launch counts.  A wide B keeps the card busy for longer than a launch takes, and with them the
+// compiler orders the loads of the 64-column kernel worse: 8 x 4096 x 11008 37.8 us with the whole block, 45.3 with the short one.
 template <int MR, int COLS>
 int launch_rows(hipStream_t stream, const SgemmParams& p) {
-  hipLaunchKernelGGL((sgemv_kernel<MR, COLS>), dim3((p.N + COLS - 1) / COLS, p.batch), dim3(kWaves * 64), 0, stream, p);
+  const dim3 grid((p.N + COLS - 1) / COLS, p.batch), block(kWaves * 64);
+  if (COLS == 32 && sgemm_detail::SgemmLone::takes(p))
+    hipLaunchKernelGGL((sgemv_kernel<MR, COLS, sgemm_detail::SgemmLone>), grid, block, 0, stream, sgemm_detail::SgemmLone(p));
+  else
+    hipLaunchKernelGGL((sgemv_kernel<MR, COLS, SgemmParams>), grid, block, 0, stream, p);
   return check_launch("sgemv");
 }
 
