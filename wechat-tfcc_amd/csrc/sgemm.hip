@@ -451,7 +451,8 @@ int dispatch(hipStream_t s, const SgemmParams& p, bool vec, bool small, bool tb,
     // Which of the two kernels whose workgroups share a K: the one for tiles of 32 rows where it is thought to be faster than the
     // other by a tenth, or than the tiled kernels at all.  Of 220 products of 17 to 1024 rows and 768 k and more it takes 47,
     // at 0.79 of the time (up to 1.0), another 13 lose a tenth without it.  What the bf16 matrix ops take stays there.
-    const double few = sgemm_detail::sgemm_skinny_microseconds(m, n, k);
+    const sgemm_detail::SkinnyPlan skinny = sgemm_detail::sgemm_skinny_plan(m, n, k);
+    const double few = skinny.better ? skinny.us : 0;
     const sgemm_deal_plan::Plan deal = sgemm_deal_plan::plan_of(m, n, k);
     if (deal.splits > 0 &&
         deal.us < (few > 0 ? .9 * few
@@ -459,7 +460,7 @@ int dispatch(hipStream_t s, const SgemmParams& p, bool vec, bool small, bool tb,
                        ? sgemm_tiles::microseconds(m, n, k, fillBatch)
                        : 0))
       return sgemm_detail::sgemm_deal_launch(s, p, deal.splits, deal.blocks, tb);
-    if (few > 0) return sgemm_detail::sgemm_skinny_launch(s, p, tb);
+    if (few > 0) return sgemm_detail::sgemm_skinny_launch(s, p, skinny, tb);
   }
   if (small) {
     const int split = sgemm_split_plan::kernel_of(m, n, k, p.lda, p.ldb, p.ldc, tb, fillBatch);

@@ -136,10 +136,14 @@ int sgemv_launch(hipStream_t stream, const SgemmParams& p);
 
 // The kernel for few rows (sgemm_skinny.hip): one product, or the grouped form; any alignment, B as stored or transposed,
 // operands below 2^30 elements.
-// About how long, 0 for a product that other kernels are better at.
-double sgemm_skinny_microseconds(unsigned m, unsigned n, unsigned k);
+struct SkinnyPlan {
+  unsigned splits, rows;  // workgroups that share a tile's K; blocks of sixteen rows in a tile
+  bool better;            // than the other kernels
+  double us;
+};
+SkinnyPlan sgemm_skinny_plan(unsigned m, unsigned n, unsigned k);
 void sgemm_skinny_release_stream(int dev, hipStream_t stream);
-int sgemm_skinny_launch(hipStream_t stream, const SgemmParams& p, bool transB);
+int sgemm_skinny_launch(hipStream_t stream, const SgemmParams& p, const SkinnyPlan& plan, bool transB);
 
 // The kernel for a K that is dealt out over the wavefronts of one or several workgroups (sgemm_deal.hip), as sgemm_deal_plan.hpp
 // says: one product, or the grouped form; any alignment, B as stored or transposed, operands below 2^30 elements.

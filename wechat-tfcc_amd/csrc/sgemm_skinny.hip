@@ -2,14 +2,13 @@
 // 24 workgroups of four wavefronts, each walking a quarter of K slab by slab; the matrix cores of 24 CUs and their loads
 // decide (19 us for 9 MB of B).
 //
-// A workgroup owns 16 rows x 16 columns and deals the steps of K (16 k each) among eight wavefronts; where the tiles leave
+// A workgroup owns 16 (or 32) rows x 16 columns and deals the steps of K (16 k each) among eight wavefronts; where the tiles leave
 // CUs without work, several workgroups share a tile's steps.  Nothing is shared before the partial tiles meet, so nothing
 // goes through LDS on the way in: a lane loads its operands of the 16x16x4 matrix op as they lie, four consecutive k of a
 // row of A in one load and the same four k of its column of B, with two batches of four steps under way.  Bound by what a
 // CU can have on its way from memory.  (Tiles of 16 x 32, whole lines of B, take twice as long: half the workgroups.)
 //
-// With weights from memory, against the kernel that streams B under up to eight rows: 1 x 1001 x 1237 12.2 -> 5.1 us,
-// 8 x 3072 x 768 11.1 -> 6.9, 1 x 8192 x 2048 34 -> 20; and against the tiles of 32 rows: 32 x 3072 x 768 19.6 -> 8.6,
+// With weights from memory, against the tiles of 32 rows: 32 x 3072 x 768 19.6 -> 8.6 us,
 // 9 x 4096 x 1024 24.3 -> 8.5, 16 x 8192 x 2048 70 -> 26, 64 x 8192 x 300 50 -> 12.4, 32 x 768 x 768 6.3 -> 4.8,
 // 48 x 1001 x 1237 8.2 -> 5.9.
 //
@@ -24,7 +23,9 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "sgemm_deal_plan.hpp"
 #include "sgemm_params.hpp"
+#include "sgemm_tiles.hpp"
 #include "stream_slots.hpp"
 
 namespace tfcc_rocm {
@@ -38,7 +39,7 @@ constexpr int kWaves = 8;  // two workgroups to a CU: tiles that are no multiple
 constexpr int kBatch = 4;  // steps asked for at once
 
 // The memory in which the splits of a tile meet: a piece per stream, asked for by the first product that splits.
-constexpr unsigned kMaxParts = 1024, kMaxGroups = 4;  // kMaxParts: tiles x splits of a product
+constexpr unsigned kMaxParts = 1024, kMaxGroups = 4;  // kMaxParts: blocks of 16 x 16 x splits of a product
 constexpr unsigned kPieceTiles = kMaxParts * kMaxGroups;
 struct Meeting {
   float partials[256 * (size_t)kPieceTiles];
@@ -53,15 +54,39 @@ StreamPieces gPieces(sizeof(Meeting), 64, clear_counts);  // 4 MB each
 // alone, so that it is summed the same way alone, in a group and with B transposed.  Nanoseconds as measured, launch aside:
 // a CU takes 2.8 per k of every tile it has; arriving and adding up costs 1300 and 200 more per split; the 32-row tiles with
 // four K groups take 5.1 per k while there is one for each CU.  (The line stands at 4.6, so that what is in doubt stays
-// where it was.)  Up to eight rows the streaming kernel takes 2.4 to 2.9 per k, whatever N, on one CU for 32 columns, and
-// walks what K has beyond a multiple of 64 row by row, 7000 in all.  Splits of less than 512 k end before their loads have
-// paid for the arrival: 2048 -> 512 with 9 rows, 7.4 us in splits of 256 against 6.2.  Below 256 k nothing is split in the tiled kernels either, and a product keeps their
-// bits, which are those it has in a batch.
-struct Plan { unsigned splits; bool better; double us; };
-Plan plan_of(unsigned m, unsigned n, unsigned k) {
+// where it was.)  Splits of less than 512 k end before their loads have paid for the arrival: 2048 -> 512 with 9 rows, 7.4 us in
+// splits of 256 against 6.2.  Below 256 k nothing is split in the tiled kernels either, and a product of more than eight rows keeps
+// their bits, which are those it has in a batch.
+//
+// Up to eight rows the other kernel is the streaming one (sgemv.hip), which has a CU for 32 columns and walks what K has
+// beyond a multiple of 64 eight rows at a time.  See takes_few_rows.
+//
+// More than sixteen rows have tiles of 32 as well, which read B once for two blocks of rows, one workgroup to a CU: they are taken
+// where the times below, fitted to 900 launches of 170 products of 17 to 100 rows and met within 5 %, say so.  Against the tiled kernels,
+// whose estimate is met without a remainder and from cache (1.19 of it with weights from memory, 1.27 with a K or an N that is no
+// multiple of their pieces), and against tiles of 16: 26 x 1328 x 3072 10.7 -> 8.4 us, 18 x 1006 x 3222 8.6 -> 6.7, 29 x 768 x 3072
+// 7.1 -> 6.1, 41 x 968 x 1952 8.3 -> 7.1, 94 x 3048 x 400 10.2 -> 9.0.
+using sgemm_detail::SkinnyPlan;
+
+// Up to eight rows: here or in the streaming kernel.  300 products, replayed with weights from memory / from cache, streaming -> here: 8 x
+// 64 x 2048 3.8/3.6 -> 2.2/2.1 us, 4 x 496 x 302 11.4/6.1 -> 3.1/2.7, 8 x 832 x 960 5.3/4.8 -> 3.8/3.4, 1 x 424 x 1588 4.3/3.0 ->
+// 3.1/2.7; launched, 4 x 3072 x 768 12.0/8.0 -> 6.6/6.4, 1 x 8192 x 2048 20.5 -> 14.6, 8 x 2304 x 4000 14.0/11.0 -> 9.9/8.0.
+// The streaming kernel keeps one row of up to 1024 k, a multiple of its chunks of 64 (1 x 960 x 128 3.5/2.9, here 3.5/3.3; 1 x 192 x 966
+// 2.7/2.35, here 2.4/2.2, but its launch, which is the longer part, costs the host 0.15 less), and what reads
+// whole lines of B on most of the CUs, but for a short K: 1 x 5120 x 5120 27, here 34, 4 x 1024 x 5376 6.5/6.0, here 8.6/7.8, 4 x 4096
+// x 11008 36, here 47; 6 x 192 x 9216 6.4/5.7 -> 4.0/3.6, 2 x 16 x 5984 2.9/2.5 -> 2.4/2.3.  Other widths come here (4 x 1024 x 7100 10.6 -> 8.3,
+// 1 x 3000 x 7100 24 -> 16), and so do more than two rows of a K with a rest (4 x 700 x 6144 13.8 -> 7.0), except of wide and deep ones, which
+// the memory decides and 64-byte pieces do not suit (2 x 2000 x 15000 25, here 28, 4 x 4096 x 11000 39, here 45; 4 x 1000 x 16001 15.9 -> 13.2).
+bool takes_few_rows(unsigned m, unsigned n, unsigned k) {
+  if (n <= 4096) return m > 1 || k > 1024 || k % 64 != 0;
+  if (n % 32 != 0 || (k % 64 != 0 && m > 2)) return n < 10240 || k <= 1600;
+  return n < 10240 && k <= (m > 4 ? 512u : m > 2 ? 256u : 128u);
+}
+
+SkinnyPlan plan_of(unsigned m, unsigned n, unsigned k) {
   const unsigned long long tiles = (unsigned long long)((m + 15) / 16) * ((n + 15) / 16);
-  if (k < 256 || tiles > kMaxParts) return Plan{1, false, 0};
-  Plan best{1, false, 0};
+  if (k < (m > 8 ? 256u : 16u) || tiles > kMaxParts) return SkinnyPlan{1, 1, false, 0};
+  SkinnyPlan best{1, 1, false, 0};
   unsigned long long bestCost = ~0ull;
   for (unsigned s = 1; s == 1 || (s <= k / 512 && tiles * s <= kMaxParts); ++s) {
     const unsigned long long perCu = (tiles * s + 255) / 256;
@@ -72,8 +97,27 @@ Plan plan_of(unsigned m, unsigned n, unsigned k) {
     }
   }
   best.us = 2.5 + bestCost * 1e-4;
-  const unsigned long long streaming = ((unsigned long long)k * (m <= 4 ? 24 : 29) + (k % 64 != 0 ? 70000 : 0)) * 9 / 10;
-  best.better = bestCost < (m > 8 ? (unsigned long long)k * 46 : streaming);
+  best.better = m > 8 ? bestCost < (unsigned long long)k * 46 : takes_few_rows(m, n, k);
+  if (m <= 16) return best;
+  double line = .92 * best.us;
+  if (!best.better) {
+    line = (k % 32 != 0 || n % 4 != 0 ? 1.15 : 1.05) * sgemm_tiles::microseconds(m, n, k, 1);
+    const sgemm_deal_plan::Plan deal = sgemm_deal_plan::plan_of(m, n, k);
+    if (deal.splits > 0 && .9 * deal.us < line) line = .9 * deal.us;
+  }
+  for (unsigned rows = best.better ? 2 : 1; rows <= 2; ++rows) {
+    const unsigned long long count = (unsigned long long)((m + 16 * rows - 1) / (16 * rows)) * ((n + 15) / 16);
+    for (unsigned s = 1; s == 1 || s <= k / 512; ++s) {
+      if (count * rows * s > kMaxParts) break;
+      const double perCu = (double)((count * s + 255) / 256), filled = count * s / 256., thousands = k / (1000. * s);
+      const double us = rows == 1 ? 2.94 + perCu * (2.04 * thousands + .2) + .39 * filled * thousands + (s > 1 ? .07 + .38 * s : 0)
+                                  : 1.66 + perCu * (3.52 * thousands + 1.19) + .97 * filled * thousands + (s > 1 ? .66 + .28 * s : 0);
+      if (us < line) {
+        line = us;
+        best = SkinnyPlan{s, rows, true, us};
+      }
+    }
+  }
   return best;
 }
 
@@ -85,8 +129,8 @@ Plan plan_of(unsigned m, unsigned n, unsigned k) {
 // What is under way has to be the same on every path to a matrix op, or the compiler waits for every load before it uses the
 // first (with a condition in front of every load 1 x 16384 x 64 in a graph took 37 us instead of 26): whole batches are asked for without a condition, and the last 0 to 3 steps of a wavefront have code of their own
 // for each number.
-template <bool TRANSB, int TEAMS, class Arguments>
-__global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(const float* hotA, const float* hotB, unsigned M,
+template <bool TRANSB, int ROWS, int TEAMS, class Arguments>
+__global__ __launch_bounds__(64 * kWaves * TEAMS, ROWS == 2 ? 2 : 4) void sgemm_skinny_kernel(const float* hotA, const float* hotB, unsigned M,
                                                                               unsigned N, unsigned K, unsigned lda, unsigned ldb,
                                                                               unsigned tilesM, unsigned tilesTotal, unsigned chunk,
                                                                               unsigned splits, unsigned perWave, Meeting* meeting,
@@ -94,7 +138,7 @@ __global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(co
   const SgemmParams p = arguments.whole();
   constexpr bool GROUPED = std::is_same<Arguments, SgemmParams>::value;
   constexpr unsigned ROUNDS = TEAMS == 1 ? 1 : 3, HELD = TEAMS * ROUNDS;  // splits that wait in LDS
-  __shared__ float part[HELD * kWaves][4][64];
+  __shared__ float part[HELD * kWaves][4 * ROWS][64];
   __shared__ unsigned arrived;
   const unsigned lane = threadIdx.x & 63;
   const unsigned waveInGroup = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -103,7 +147,7 @@ __global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(co
   const unsigned L = (blockIdx.x & 7u) * chunk + (blockIdx.x >> 3);
   if ((blockIdx.x >> 3) >= chunk || L >= tilesTotal) return;
   const unsigned tn = L / tilesM, tm = L - tn * tilesM, group = blockIdx.y;
-  const unsigned m0 = tm * 16, n0 = tn * 16;
+  const unsigned m0 = tm * (16 * ROWS), n0 = tn * 16;
   const float* A = hotA;
   const float* B = GROUPED && p.groups ? p.groupB[group] : hotB;
   // (no range check: every offset below lies inside the operand)
@@ -112,13 +156,21 @@ __global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(co
 
   // rows and columns past the edge read the last one, and their sums are dropped
   const unsigned g = lane >> 4, edge = lane & 15u;
-  const unsigned row = min(m0 + edge, M - 1), col = min(n0 + edge, N - 1);
-  const unsigned aOff = (row * lda + 4 * g) * 4u;
+  const unsigned col = min(n0 + edge, N - 1);
+  unsigned row[ROWS], aOff[ROWS];
+#pragma unroll
+  for (unsigned r = 0; r < (unsigned)ROWS; ++r) {
+    row[r] = min(m0 + 16 * r + edge, M - 1);
+    aOff[r] = (row[r] * lda + 4 * g) * 4u;
+  }
   const unsigned bOff = (TRANSB ? col * ldb + 4 * g : 4 * g * ldb + col) * 4u;
-  struct Ops { float a[4], b[4]; };
+  struct Ops { float a[ROWS][4], b[4]; };
   auto load = [&](Ops& o, unsigned k) __attribute__((always_inline)) {
-    const auto a = __builtin_amdgcn_raw_buffer_load_b128(rsrcA, aOff, k * 4u, 0);
-    __builtin_memcpy(o.a, &a, 16);
+#pragma unroll
+    for (unsigned r = 0; r < (unsigned)ROWS; ++r) {
+      const auto a = __builtin_amdgcn_raw_buffer_load_b128(rsrcA, aOff[r], k * 4u, 0);
+      __builtin_memcpy(o.a[r], &a, 16);
+    }
     if (TRANSB) {
       const auto b = __builtin_amdgcn_raw_buffer_load_b128(rsrcB, bOff, k * 4u, 0);
       __builtin_memcpy(o.b, &b, 16);
@@ -137,9 +189,9 @@ __global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(co
   unsigned split = TEAMS == 1 ? blockIdx.z : team;
   unsigned first = split * kWaves + wave;
 
-  // what the finish needs: thread t of the first 256 finishes value t / 64
-  const unsigned fe = (threadIdx.x >> 6) & 3u, grow = m0 + 4 * g + fe, gcol = n0 + edge;
-  const bool finisher = threadIdx.x < 256, mine = finisher && grow < M && gcol < N;
+  // what the finish needs: thread t of the first 256 of every row block finishes value t / 64
+  const unsigned fe = (threadIdx.x >> 6) & (4u * ROWS - 1), grow = m0 + 16 * (fe >> 2) + 4 * g + (fe & 3u), gcol = n0 + edge;
+  const bool finisher = threadIdx.x < 256 * ROWS, mine = finisher && grow < M && gcol < N;
   float bv = 0.f, rv = 0.f;
   auto loadFinish = [&]() __attribute__((always_inline)) {
     const float* bias = GROUPED && p.groups ? p.groupBias[group] : p.bias;
@@ -147,10 +199,12 @@ __global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(co
     if (mine && p.residual) rv = p.residual[(size_t)grow * N + gcol];
   };
 
-  skinny_v4f acc[kBatch];  // one for each step of a batch: short chains, for the rounding and for the matrix ops' latency
+  skinny_v4f acc[ROWS][kBatch];  // one for each step of a batch: short chains, for the rounding and for the matrix ops' latency
   auto multiply = [&](const Ops& o, int u) __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s) acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[s], o.b[s], acc[u], 0, 0, 0);
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) acc[r][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[r][s], o.b[s], acc[r][u], 0, 0, 0);
   };
   auto multiplySteps = [&](int which, auto steps) __attribute__((always_inline)) {
 #pragma unroll
@@ -171,7 +225,7 @@ __global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(co
   const unsigned oneMore = whole - perWave * lanes;
   auto sumSplit = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) acc[u] = skinny_v4f{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < kBatch * ROWS; ++u) acc[u / kBatch][u % kBatch] = skinny_v4f{0.f, 0.f, 0.f, 0.f};
     const unsigned steps = perWave + (first < oneMore ? 1u : 0u);
     if (TEAMS == 1 && steps < kBatch) {
       with(steps, [&](auto few) {
@@ -213,14 +267,18 @@ __global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(co
 #pragma unroll
       for (unsigned s = 0; s < 4; ++s) {
         const bool in = whole * 16 + 4 * g + s < K;
-        o.a[s] = in ? A[(size_t)row * lda + whole * 16 + 4 * g + s] : 0.f;
+#pragma unroll
+        for (unsigned r = 0; r < (unsigned)ROWS; ++r) o.a[r][s] = in ? A[(size_t)row[r] * lda + whole * 16 + 4 * g + s] : 0.f;
         const size_t k = whole * 16 + 4 * g + s;
         o.b[s] = in ? B[TRANSB ? (size_t)col * ldb + k : k * ldb + col] : 0.f;
       }
       multiply(o, 0);
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) part[held * kWaves + wave][e][lane] = (acc[0][e] + acc[1][e]) + (acc[2][e] + acc[3][e]);
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        part[held * kWaves + wave][4 * r + e][lane] = (acc[r][0][e] + acc[r][1][e]) + (acc[r][2][e] + acc[r][3][e]);
   };
   float v = 0.f;
   auto meet = [&](unsigned from, unsigned to) __attribute__((always_inline)) {  // adds the held splits from .. to - 1
@@ -262,9 +320,9 @@ __global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(co
     // The partial tile goes past the caches, and waiting for the store is all the order there has to be in front of the
     // count; the workgroup that arrives last adds the partial tiles in the order of the splits.
     const unsigned tile = group * tilesTotal + L;
-    float* mineAt = meeting->partials + (size_t)tile * splits * 256;
+    float* mineAt = meeting->partials + (size_t)tile * splits * (256 * ROWS);
     unsigned* count = meeting->counts + tile;
-    if (finisher) __hip_atomic_store(mineAt + blockIdx.z * 256 + threadIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (finisher) __hip_atomic_store(mineAt + blockIdx.z * (256 * ROWS) + threadIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) arrived = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -274,7 +332,7 @@ __global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(co
     if (finisher) {
       v = __hip_atomic_load(mineAt + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       for (unsigned s = 1; s < splits; ++s)
-        v += __hip_atomic_load(mineAt + s * 256 + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        v += __hip_atomic_load(mineAt + s * (256 * ROWS) + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
   if (!mine) return;
@@ -286,21 +344,24 @@ __global__ __launch_bounds__(64 * kWaves * TEAMS, 4) void sgemm_skinny_kernel(co
 }
 
 template <bool TRANSB>
-int launch_skinny(hipStream_t stream, SgemmParams p) {
+int launch_skinny(hipStream_t stream, SgemmParams p, const SkinnyPlan& plan) {
   const unsigned groups = p.groups ? p.groups : 1u;
   p.batch = 1;
-  if (!sgemm_detail::set_tiles(p, 16, 16)) return set_error(TFCC_ROCM_INVALID_ARGUMENT, "sgemm: too many tiles");
-  const unsigned splits = plan_of(p.M, p.N, p.K).splits;
+  const unsigned splits = plan.splits;
   Meeting* meeting = nullptr;
   if (splits > 1) {
     int dev = 0;
     TFCC_HIP_CHECK(hipGetDevice(&dev));
     meeting = static_cast<Meeting*>(gPieces.of(dev, stream));
   }
-  const bool alone = splits > 1 && meeting == nullptr;
+  // (The same bits with one row block as with two.)
+  const bool alone = splits > 1 && meeting == nullptr, two = plan.rows == 2 && !alone;
+  if (!sgemm_detail::set_tiles(p, two ? 32 : 16, 16)) return set_error(TFCC_ROCM_INVALID_ARGUMENT, "sgemm: too many tiles");
   auto launch = [&](const auto& arguments) {
     using Arguments = std::decay_t<decltype(arguments)>;
-    auto kern = alone ? sgemm_skinny_kernel<TRANSB, 2, Arguments> : sgemm_skinny_kernel<TRANSB, 1, Arguments>;
+    auto kern = alone ? sgemm_skinny_kernel<TRANSB, 1, 2, Arguments>
+                : two ? sgemm_skinny_kernel<TRANSB, 2, 1, Arguments>
+                      : sgemm_skinny_kernel<TRANSB, 1, 1, Arguments>;
     hipLaunchKernelGGL(kern, dim3(p.chunk * 8, groups, alone ? 1u : splits), dim3(64 * kWaves * (alone ? 2 : 1)), 0, stream, p.A, p.B,
                        (unsigned)p.M, (unsigned)p.N, (unsigned)p.K, (unsigned)p.lda, (unsigned)p.ldb, p.tilesM, p.tilesTotal, p.chunk,
                        splits, p.K / 16 / (splits * kWaves), meeting, arguments);
@@ -314,13 +375,10 @@ int launch_skinny(hipStream_t stream, SgemmParams p) {
 
 namespace sgemm_detail {
 
-double sgemm_skinny_microseconds(unsigned m, unsigned n, unsigned k) {
-  const Plan plan = plan_of(m, n, k);
-  return plan.better ? plan.us : 0;
-}
+SkinnyPlan sgemm_skinny_plan(unsigned m, unsigned n, unsigned k) { return plan_of(m, n, k); }
 
-int sgemm_skinny_launch(hipStream_t stream, const SgemmParams& p, bool transB) {
-  return transB ? launch_skinny<true>(stream, p) : launch_skinny<false>(stream, p);
+int sgemm_skinny_launch(hipStream_t stream, const SgemmParams& p, const SkinnyPlan& plan, bool transB) {
+  return transB ? launch_skinny<true>(stream, p, plan) : launch_skinny<false>(stream, p, plan);
 }
 
 void sgemm_skinny_release_stream(int dev, hipStream_t stream) { gPieces.release(dev, stream); }

@@ -1,5 +1,6 @@
-// fp32 matmul for up to eight rows of A (one decode step, one recurrent step): the product is bound by the single
-// pass over B, so it runs on the vector ALUs with B streamed straight from memory and no tile staging.
+// fp32 matmul for up to eight rows of A (one decode step, one recurrent step), where B is wide (sgemm_skinny.hip has the line): the
+// product is bound by the single pass over B, so it runs on the vector ALUs with B streamed straight from memory and no
+// tile staging.
 //
 // A workgroup of sixteen wavefronts owns 64 (or 32) columns.  Wavefront w walks rows [w * per, (w + 1) * per) of B
 // in chunks of 64, one column per lane (a row of B is read as 256 contiguous bytes per wavefront, or two rows as
