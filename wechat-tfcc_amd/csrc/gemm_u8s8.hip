@@ -72,7 +72,8 @@ extern "C" int tfcc_rocm_gemm_u8s8s32(void* stream, const tfcc_rocm_qgemm_desc* 
     return gemv_packed_launch(as_stream(stream), p.A, desc->packed_b, p.rowsumA, p.colsumB, p.offsetA, p.offsetB,
                               ranges, rangeOut, p.M, p.N, p.K, c, 0.f, nullptr, nullptr);
   }
-  if (p.batch == 1 && p.M <= 8 && (unsigned long long)p.N * p.K >= (1u << 20) && gemv_supported(p.A, p.B, p.M, p.N, p.K)) {
+  if (p.batch == 1 && p.M <= 8 && (unsigned long long)p.N * p.K >= (1u << 20) &&
+      (gemv_supported(p.A, p.B, p.M, p.N, p.K) || gemv_wide_takes_ragged(p.M, p.N, p.K, p.colsumExact != 0))) {
     const float* ranges[4] = {p.minA, p.maxA, p.minB, p.maxB};
     float* rangeOut[2] = {p.minC, p.maxC};
     return gemv_launch(as_stream(stream), p.A, p.B, p.rowsumA, p.colsumB, p.offsetA, p.offsetB, ranges, rangeOut,

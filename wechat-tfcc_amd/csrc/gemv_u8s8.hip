@@ -315,17 +315,9 @@ bool gemv_supported(const void* a, const void* b, unsigned m, unsigned n, unsign
          (uintptr_t)b % 4 == 0 && ((unsigned long long)k + 2048) * n + 512 < (1ull << 31);
 }
 
-int gemv_launch(hipStream_t stream, const unsigned char* a, const signed char* b, const int* rowsumA,
-                const int* colsumB, int offsetA, int offsetB, const float* const ranges[4],
-                float* const rangeOut[2], unsigned m, unsigned n, unsigned k, int* accOut,
-                float scaleA, const float* scaleB, float* f32Out, bool colsumExact) {
-  if (gemv_wide_supported(a, b, m, n, k))
-    return gemv_wide_launch(stream, false, a, b, rowsumA, colsumB, offsetA, offsetB, ranges, rangeOut, m, n, k, accOut,
-                            scaleA, scaleB, f32Out, colsumExact);
-  // The one-pass kernel's workgroups have all of K: 3 us and 0.11 more for every 64 k (8 x 12288 x 512: 24.3 us).  A long
-  // K goes to tiles that several workgroups share (8.4 us), where those may have memory to meet in.
-  // The line lies where weights from HBM pay for it: of 400 products none takes longer with them, on the average 0.65 of the
-  // time; with weights in cache 0.79, up to K = 3000 1.05 (1.17 at most; from HBM 0.88 there).
+static QGemmParams small_params(const unsigned char* a, const signed char* b, const int* rowsumA, const int* colsumB, int offsetA,
+                                int offsetB, const float* const ranges[4], float* const rangeOut[2], unsigned m, unsigned n,
+                                unsigned k, int* accOut, bool colsumExact) {
   QGemmParams q{};
   q.A = a; q.B = b; q.rowsumA = rowsumA; q.colsumB = colsumB; q.C = accOut;
   q.strideC = (uint64_t)m * n;
@@ -335,10 +327,36 @@ int gemv_launch(hipStream_t stream, const unsigned char* a, const signed char* b
     q.minA = ranges[0]; q.maxA = ranges[1]; q.minB = ranges[2]; q.maxB = ranges[3];
     if (rangeOut) { q.minC = rangeOut[0]; q.maxC = rangeOut[1]; }
   }
+  return q;
+}
+
+int gemv_launch(hipStream_t stream, const unsigned char* a, const signed char* b, const int* rowsumA,
+                const int* colsumB, int offsetA, int offsetB, const float* const ranges[4],
+                float* const rangeOut[2], unsigned m, unsigned n, unsigned k, int* accOut,
+                float scaleA, const float* scaleB, float* f32Out, bool colsumExact) {
+  if (gemv_wide_supported(a, b, m, n, k) || gemv_wide_takes_ragged(m, n, k, colsumExact))
+    return gemv_wide_launch(stream, false, a, b, rowsumA, colsumB, offsetA, offsetB, ranges, rangeOut, m, n, k, accOut,
+                            scaleA, scaleB, f32Out, colsumExact);
+  // The one-pass kernel's workgroups have all of K: 3 us and 0.11 more for every 64 k (8 x 12288 x 512: 24.3 us).  A long
+  // K goes to tiles that several workgroups share (8.4 us), where those may have memory to meet in.
+  // The line lies where weights from HBM pay for it: of 400 products none takes longer with them, on the average 0.65 of the
+  // time; with weights in cache 0.79, up to K = 3000 1.05 (1.17 at most; from HBM 0.88 there).
+  const QGemmParams q = small_params(a, b, rowsumA, colsumB, offsetA, offsetB, ranges, rangeOut, m, n, k, accOut, colsumExact);
   if (qgemm_small_supported(q) && qgemm_small_splits(stream, m, n, k, 300 + 11 * (k / 64)))
     return qgemm_small_launch(stream, q, QSmallOutputs{f32Out, scaleB, scaleA}, true);
   return gemv_onepass_launch(stream, a, b, rowsumA, colsumB, offsetA, offsetB, ranges, rangeOut, m, n, k, accOut, scaleA,
                              scaleB, f32Out);
+}
+
+int gemv_alone_launch(hipStream_t stream, const unsigned char* a, const signed char* b, const int* rowsumA,
+                      const int* colsumB, int offsetA, int offsetB, const float* const ranges[4],
+                      float* const rangeOut[2], unsigned m, unsigned n, unsigned k, int* accOut,
+                      float scaleA, const float* scaleB, float* f32Out, bool colsumExact) {
+  if (gemv_supported(a, b, m, n, k))
+    return gemv_onepass_launch(stream, a, b, rowsumA, colsumB, offsetA, offsetB, ranges, rangeOut, m, n, k, accOut, scaleA, scaleB,
+                               f32Out);
+  return qgemm_small_launch(stream, small_params(a, b, rowsumA, colsumB, offsetA, offsetB, ranges, rangeOut, m, n, k, accOut, colsumExact),
+                            QSmallOutputs{f32Out, scaleB, scaleA});
 }
 
 int gemv_onepass_launch(hipStream_t stream, const unsigned char* a, const signed char* b, const int* rowsumA,
@@ -395,7 +413,7 @@ extern "C" int tfcc_rocm_gemv_u8s8s32_flags(void* stream, const uint8_t* a, cons
   TFCC_REQUIRE(acc_out || f32_out, "skinny quantized matmul: no output");
   TFCC_REQUIRE(!f32_out || scale_b, "skinny quantized matmul: dequantize needs scale_b");
   hipStream_t s = as_stream(stream);
-  if (gemv_supported(a, b, m, n, k))
+  if (gemv_supported(a, b, m, n, k) || gemv_wide_takes_ragged(m, n, k, colsumExact))
     return gemv_launch(s, a, reinterpret_cast<const signed char*>(b), rowsum_a, colsum_b, offset_a,
                        offset_b, nullptr, nullptr, m, n, k, acc_out, scale_a, scale_b, f32_out, colsumExact);
   // ragged shapes and alignments: the kernel for small products of any alignment finishes the floats itself

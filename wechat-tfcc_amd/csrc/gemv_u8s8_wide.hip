@@ -15,7 +15,7 @@
 // row, its LDS traffic and its sums are left out.
 //
 // Two shapes of workgroup:
-//   gemv_wide16_kernel  sixteen wavefronts, one step each: every byte of B the launch reads is asked for in the
+//   gemv_wide16_kernel  sixteen (or eight) wavefronts, one step each: every byte of B the launch reads is asked for in the
 //                       first microsecond (a decode-sized B is bound by how many bytes are in flight).  The
 //                       wavefronts meet in an LDS tile through 64-bit adds that carry two rows each: the matrix op
 //                       starts from a bias instead of zero, so every partial sum is non-negative and the low row
@@ -38,6 +38,7 @@
 #include "common.hpp"
 #include "gemv.hpp"
 #include "gemv_workspace.hpp"
+#include "qgemm_small.hpp"
 
 namespace tfcc_rocm {
 
@@ -163,13 +164,17 @@ struct Tile16 {
 // passes -amdgpu-kernarg-preload-count, which has the first arguments of a kernel (scalars and pointers, up to the
 // free user SGPRs) delivered in registers at wavefront start instead of fetched from the argument block, a round trip
 // of about 0.6 us at the head of a 12 us kernel.  The argument block still carries everything.
-template <int MR, bool EXACT>
-__global__ __launch_bounds__(1024) void gemv_wide16_kernel(const signed char* hotB, const unsigned char* hotA,
+//
+// RAGGED: any N, K and alignment (the loads take any byte address).  A lane whose 16 columns reach past N reads the beginning of
+// the next row there, which is not stored; rows of B past K are zeros, whatever A has there.  Only a load that would cross the end
+// of an operand has to be put right, in the last row of B or of A: it is moved back to end with it.
+template <int WAVES, int MR, bool EXACT, bool RAGGED>
+__global__ __launch_bounds__(64 * WAVES) void gemv_wide16_kernel(const signed char* hotB, const unsigned char* hotA,
                                                            unsigned hotM, unsigned hotN, unsigned hotK,
                                                            unsigned hotColBlocks, unsigned hotKParts, unsigned hotChunk,
                                                            const GemvWideParams p) {
   static_assert(MR == 1 || MR == 4 || MR == 8, "rows of A are padded to 1, 4 or 8");
-  constexpr int kWaves = 16, kThreads = kWaves * 64;
+  constexpr int kThreads = WAVES * 64;
   using Tile = Tile16<MR, EXACT>;
   __shared__ unsigned long long tile[Tile::kWords];
 
@@ -192,9 +197,10 @@ __global__ __launch_bounds__(1024) void gemv_wide16_kernel(const signed char* ho
 
   // What the end of the kernel needs from memory is asked for now: column tid % 256 and the rows this thread
   // finishes, so that the only wait left there is the atomic's own.
-  constexpr int RPT = MR >= 2 ? 2 : 1;  // rows per thread in the last phase: a pair shares a workspace word
+  // rows per thread in the last phase, at least the pair that shares a workspace word
+  constexpr int PER_COLUMN = kThreads / kCols, RPT = MR == 1 ? 1 : MR / PER_COLUMN > 2 ? MR / PER_COLUMN : 2;
   const unsigned ec = tid % kCols, egn = n0 + ec;
-  const int r0 = (tid / kCols) * RPT;   // four threads per column, as many of them as there are pairs of rows
+  const int r0 = (tid / kCols) * RPT;   // PER_COLUMN threads per column, as many of them as there are rows for
   const bool finisher = r0 < MR && egn < N;
   int eColsum = 0, eRowsum[RPT] = {};
   float eScale = 0.f;
@@ -208,10 +214,10 @@ __global__ __launch_bounds__(1024) void gemv_wide16_kernel(const signed char* ho
   float mnA = 0.f, mxA = 0.f, mnB = 0.f, mxB = 0.f;  // ranges in device memory override the immediate offsets
   if (p.minA) { mnA = *p.minA; mxA = *p.maxA; mnB = *p.minB; mxB = *p.maxB; }
 
-  // columns past N: a lane whose 16 columns lie outside reads nothing (N is a multiple of 16)
+  // a lane whose 16 columns all lie past N reads nothing
   const bool colsInside = n0 + 16u * j < N;
   const unsigned steps = (K + 63) / 64;
-  const unsigned step = part * kWaves + wave;
+  const unsigned step = part * WAVES + wave;
   const unsigned k0 = step * 64 + kg * 16;  // this lane's 16 rows
   // The tile is cleared behind a barrier that waits for this wavefront's LDS stores only (the compiler puts no wait
   // for outstanding loads in front of a barrier on this target), so the loads of B may already be on their way:
@@ -229,17 +235,28 @@ __global__ __launch_bounds__(1024) void gemv_wide16_kernel(const signed char* ho
   // lane j supplies row j of the matrix op's A operand: rows 4q and 4q + 1 are rows 2q and 2q + 1 of A
   const unsigned aRow = (j & 3) < 2 ? 2u * (j >> 2) + (j & 3) : 0xffffffffu;
   constexpr int kOnesRow = MR == 8 ? 2 : MR == 4 ? 8 : 1;  // the operand row that holds ones (column sums)
-  const v4i aRaw = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
-                                               rsrcA, (aRow < M && k0 < K) ? aRow * K + k0 : 0xfffffff0u, 0, 0));
+  const bool hasA = aRow < M && k0 < K, live = colsInside && step < steps;
+  const unsigned offA = aRow * K + k0, offB = k0 * N + n0 + 16u * j, lastA = M * K - 16, lastB = K * N - 16;
+  const unsigned lastRow = (K - 1) * N + n0 + 16u * j;  // RAGGED: the one load of a lane that may cross the end of B ...
+  v4i rest = {0, 0, 0, 0};                              // ... and what it would have given
+  v4i aRaw = __builtin_bit_cast(
+      v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrcA, hasA ? (RAGGED ? min(offA, lastA) : offA) : 0xfffffff0u, 0, 0));
   {
-    const bool live = colsInside && step < steps;
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
-      const unsigned off = live ? (k0 + q) * N + n0 + 16u * j : 0xfffffff0u;
+      const unsigned off = live && (!RAGGED || offB + q * N <= lastB) ? offB + q * N : 0xfffffff0u;
       raw[q] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrcB, off, 0, 0));
     }
+    if (RAGGED && step == steps - 1) rest = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrcB, lastB, 0, 0));
   }
   if constexpr (kLoadsFirst) clearTile();
+  if (RAGGED && step == steps - 1) {
+    aRaw = moved16(aRaw, hasA ? max(offA, lastA) - lastA : 0u);
+    rest = moved16(rest, lastRow > lastB ? lastRow - lastB : 0u);
+#pragma unroll
+    for (unsigned q = 0; q < 16; ++q)
+      if (k0 + q == K - 1 && lastRow > lastB) raw[q] = rest;
+  }
   // A operand: rows 0..M-1 of A (uint8 -> int8 by the xor), zeros, ones in row MR
   v4i a = {0, 0, 0, 0};
   if (aRow < M) {
@@ -297,11 +314,11 @@ __global__ __launch_bounds__(1024) void gemv_wide16_kernel(const signed char* ho
   __syncthreads();
 
   if (!finisher) return;
-  // ---- this thread's rows r0 .. r0 + RPT - 1 of column ec: every one of the sixteen wavefronts added its bias
+  // ---- this thread's rows r0 .. r0 + RPT - 1 of column ec: every wavefront added its bias
   unsigned sum[RPT];
   {
     const int slot = (ec & 15) * 16 + (ec >> 4);
-    constexpr unsigned kAllBias = kWaves * kTileBias;
+    constexpr unsigned kAllBias = WAVES * kTileBias;
     auto field = [&](int row) {
       const unsigned long long word = tile[(row >> 1) * kPairPitch + slot];
       return (unsigned)(row & 1 ? word >> 32 : word) - kAllBias;
@@ -534,23 +551,23 @@ int static_workspace(unsigned long long** out) {
   return TFCC_ROCM_OK;
 }
 
-template <bool SIXTEEN, int MR, bool EXACT>
-int launch_wide(hipStream_t stream, const GemvWideParams& p) {
-  if (SIXTEEN) {
-    hipLaunchKernelGGL((gemv_wide16_kernel<MR, EXACT>), dim3(p.chunk * 8), dim3(1024), 0, stream, p.B, p.A, p.M, p.N, p.K,
-                       p.colBlocks, p.kParts, p.chunk, p);
-  } else {
+template <int MR, bool EXACT>
+int launch_wide(hipStream_t stream, const GemvWideParams& p, int waves, bool ragged) {
+  auto one = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(p.chunk * 8), dim3(64 * waves), 0, stream, p.B, p.A, p.M, p.N, p.K, p.colBlocks, p.kParts, p.chunk, p);
+  };
+  if (p.stepsPerWave != 1)
     hipLaunchKernelGGL((gemv_wide_kernel<MR, EXACT>), dim3(p.chunk * 8), dim3(256), 0, stream, p.B, p.A, p.M, p.N, p.K,
                        p.colBlocks, p.kParts, p.stepsPerWave, p.chunk, p);
-  }
+  else if (waves == 16) one(ragged ? gemv_wide16_kernel<16, MR, EXACT, true> : gemv_wide16_kernel<16, MR, EXACT, false>);
+  else one(ragged ? gemv_wide16_kernel<8, MR, EXACT, true> : gemv_wide16_kernel<8, MR, EXACT, false>);
   return check_launch("skinny quantized matmul (split over K)");
 }
 
-template <bool SIXTEEN>
-int launch_wide_rows(hipStream_t stream, const GemvWideParams& p, bool exact) {
-  if (p.M == 1) return exact ? launch_wide<SIXTEEN, 1, true>(stream, p) : launch_wide<SIXTEEN, 1, false>(stream, p);
-  if (p.M <= 4) return exact ? launch_wide<SIXTEEN, 4, true>(stream, p) : launch_wide<SIXTEEN, 4, false>(stream, p);
-  return exact ? launch_wide<SIXTEEN, 8, true>(stream, p) : launch_wide<SIXTEEN, 8, false>(stream, p);
+int launch_wide_rows(hipStream_t stream, const GemvWideParams& p, int waves, bool ragged, bool exact) {
+  if (p.M == 1) return exact ? launch_wide<1, true>(stream, p, waves, ragged) : launch_wide<1, false>(stream, p, waves, ragged);
+  if (p.M <= 4) return exact ? launch_wide<4, true>(stream, p, waves, ragged) : launch_wide<4, false>(stream, p, waves, ragged);
+  return exact ? launch_wide<8, true>(stream, p, waves, ragged) : launch_wide<8, false>(stream, p, waves, ragged);
 }
 
 }  // namespace
@@ -561,6 +578,18 @@ bool gemv_wide_supported(const void* a, const void* b, unsigned m, unsigned n, u
          (unsigned long long)m * k < (1ull << 31) &&
          // worth it from a few hundred wavefront steps on; below that the one-pass kernel's launch is all there is
          (unsigned long long)((k + 63) / 64) * ((n + kCols - 1) / kCols) >= 512;
+}
+
+// Against the kernel for small products of any alignment, us: 7900 x 5814 20.8 -> 12.6, 5799 x 9800 20.1 -> 13.4, 4755 x 4616 11.1 -> 9.0,
+// 2897 x 10788 12.9 -> 9.5, with exact sums 2448 x 4782 8.6 -> 7.3, 2052 x 3704 7.8 -> 6.4, 10124 x 1235 9.4 -> 7.8.  Below the line 6 x
+// 2432 x 7191 8.8 -> 9.3, 2 x 924 x 11952 6.5 -> 6.7, 8 x 4040 x 6689 10.9 -> 11.5, with exact sums 6 x 1766 x 5686 6.5 ->
+// 7.1, 4 x 883 x 10148 5.4 -> 6.4 (a K that short is read at once there too).
+bool gemv_wide_takes_ragged(unsigned m, unsigned n, unsigned k, bool colsumExact) {
+  const unsigned long long blocks = (n + kCols - 1) / kCols, steps = (k + 63) / 64;
+  const unsigned least = colsumExact ? (n % 4 == 0 ? 420 : 700) : n % 4 == 0 ? 1400 : 1900;  // wavefronts
+  return m >= 1 && m <= (unsigned)kMaxM && n >= 16 && k >= 16 && ((unsigned long long)k + 4160) * n + 4096 < (1ull << 31) &&
+         ((unsigned long long)m + 64) * k + 4096 < (1ull << 31) && blocks * steps >= least && steps >= 22 &&
+         blocks * ((steps + 15) / 16) <= 1024;
 }
 
 unsigned gemv_wide_static_max_n() { return kMaxStaticN; }
@@ -587,12 +616,18 @@ int gemv_wide_launch(hipStream_t stream, bool staticWorkspace, const unsigned ch
   p.M = m; p.N = n; p.K = k;
   p.colBlocks = (n + kCols - 1) / kCols;
   const unsigned steps = (k + 63) / 64;
+  const bool ragged = !gemv_wide_supported(a, b, m, n, k);
   int waves = kDefaultWaves;
   unsigned spw = kDefaultStepsPerWave;
   // more steps per wavefront once the grid would exceed about four workgroups per CU (sixteen wavefronts make
   // one step each: a product that needs more goes to four wavefronts of several steps)
   if (waves == 16 && (spw != 1 || (unsigned long long)p.colBlocks * ((steps + 15) / 16) > 1024)) { waves = 4; spw = 4; }
   while ((unsigned long long)p.colBlocks * ((steps + waves * spw - 1) / (waves * spw)) > 1024 && spw < 64) spw *= 2;
+  // Sixteen wavefronts of one step leave most CUs without work while there are few, and a workgroup's bytes go through one CU: eight
+  // of them, us: 1984 x 5056 7.6 -> 6.3, 3200 x 2688 7.6 -> 6.5, 1344 x 9792 7.8 -> 6.7; past 900 wavefronts 6336 x 2560 7.2 -> 7.6, 5760 x
+  // 9792 12.8 -> 13.8.  Ragged loads take a CU longer: 2104 x 9276 8.3 -> 7.9, 5789 x 3292 8.9 -> 8.5, 3024 x 8698 9.5 -> 9.9.  (Four:
+  // more parts to add up, 1984 x 5056 7.6, 1344 x 9792 7.8.)
+  if (spw == 1 && (unsigned long long)p.colBlocks * steps < (ragged ? 1400u : 900u)) waves = 8;
   p.stepsPerWave = spw;
   p.kParts = (steps + waves * spw - 1) / (waves * spw);
   p.chunk = (p.colBlocks * p.kParts + 7) / 8;
@@ -623,8 +658,8 @@ int gemv_wide_launch(hipStream_t stream, bool staticWorkspace, const unsigned ch
       // the stream is being recorded and has no workspace of this width yet: nothing may be allocated now, so this
       // launch goes to the kernel that needs none (same sums; slower on a decode-sized B).  A product of the same
       // width issued once before the recording, or the entry point without allocation, avoids this.
-      return gemv_onepass_launch(stream, a, b, rowsumA, colsumB, offsetA, offsetB, ranges, rangeOut, m, n, k, accOut,
-                                 scaleA, scaleB, f32Out);
+      return gemv_alone_launch(stream, a, b, rowsumA, colsumB, offsetA, offsetB, ranges, rangeOut, m, n, k, accOut, scaleA, scaleB,
+                               f32Out, colsumExact);
     if (e == TFCC_ROCM_OUT_OF_MEMORY) return set_error(e, "skinny quantized matmul: no memory for the workspace");
     if (e) return set_error(e, "skinny quantized matmul: workspace set-up failed");
     p.tiles = static_cast<unsigned long long*>(lease.mem);
@@ -635,7 +670,7 @@ int gemv_wide_launch(hipStream_t stream, bool staticWorkspace, const unsigned ch
     }
   }
   int status;
-  status = waves == 16 ? launch_wide_rows<true>(stream, p, colsumExact) : launch_wide_rows<false>(stream, p, colsumExact);
+  status = launch_wide_rows(stream, p, waves, ragged, colsumExact);
   if (status != TFCC_ROCM_OK && leased) gWorkspaces.mark_dirty(key);
   return status;
 }
