@@ -27,6 +27,10 @@ namespace qgemm_small_plan {
 // the two rules looked at, none is slower than in one piece from HBM and three are from the cache, by up to 1.12; on the
 // average they take 0.58 and 0.63 of the time.  3 x 11304 x 910 27.3 -> 9.3, 32 x 8192 x 512 18.5 -> 7.8, 99 x 3481 x 512
 // 11.7 -> 7.8; 526 x 1832 x 400 stays at 7.5 (10.2 split).
+// Where up to three trips would take more wavefronts than that, four to eight do: of 60 such products, one in twelve of those of
+// more than 1300 k that come here, the 40 that are thought to take three quarters of the time at most take 0.72 of it, none more than 0.98
+// (43 x 7005 x 1920 25.5 -> 12.1, 830 x 5881 x 96 22.8 -> 11.3, 29 x 7565 x 4331 35.5 -> 21.4); the others 0.98, up to 1.12 (221 x 4120 x 1101
+// 15.9 -> 17.8).
 constexpr int kCols = 64;                   // columns of a tile
 constexpr unsigned kMaxResults = 1u << 19;  // of a product that is split
 
@@ -50,8 +54,8 @@ inline Plan plan_of(unsigned m, unsigned n, unsigned k, unsigned batch) {
   p.cost = p.rows == 32 ? 400 + (p.waves == 4 ? 170 : 210) * trips(p.waves)
                         : p.waves == 4 ? 300 + 120 * trips(4) : p.waves == 8 ? 380 + 180 * trips(8) : 420 + 300 * trips(16);
   if (steps <= 20 || p.rows == 64 || tiles16 * 16 * kCols > kMaxResults) return p;
-  for (unsigned waves = 4; waves <= 8; waves += 4)
-    for (unsigned want = 1; want <= 3; ++want) {  // trips
+  auto choose = [&](unsigned waves, unsigned least, unsigned most, double margin) {
+    for (unsigned want = least; want <= most; ++want) {  // trips
       const unsigned splits = (steps + 2 * (waves - 1) * want - 1) / (2 * (waves - 1) * want);
       const unsigned cost = (waves == 4 ? 300 + 120 * want : 380 + 180 * want) + 240;
       if (splits < 2 || splits > 32 || tiles16 * splits * waves > 2048 || cost + 70 > p.cost || cost >= p.splitCost) continue;
@@ -63,8 +67,12 @@ inline Plan plan_of(unsigned m, unsigned n, unsigned k, unsigned batch) {
       const double one = p.rows == 32    ? 240 + steps * (10.5 + 9 * oddA + 4 * oddB) + all * (3. * steps - 10)
                          : p.waves == 16 ? 490 + steps * (5.6 + 3.8 * oddA + 3.6 * oddB) + all * (3.1 * steps - 91)
                                          : 600 + steps * 3.5 * odd + all * (2.2 * steps - 22);
-      p.better = 390 + want * (143 + 25 * odd) + shared * (48 - 4.4 * want) < one;
+      p.better = 390 + want * (143 + 25 * odd) + shared * (48 - 4.4 * want) < margin * one;
     }
+  };
+  for (unsigned waves = 4; waves <= 8; waves += 4) choose(waves, 1, 3, 1.);
+  if (p.splits == 1)
+    for (unsigned waves = 4; waves <= 8; waves += 4) choose(waves, 4, 8, .75);
   return p;
 }
 
