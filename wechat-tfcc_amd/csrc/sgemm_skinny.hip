@@ -101,9 +101,10 @@ SkinnyPlan plan_of(unsigned m, unsigned n, unsigned k) {
   if (m <= 16) return best;
   double line = .92 * best.us;
   if (!best.better) {
-    line = (k % 32 != 0 || n % 4 != 0 ? 1.15 : 1.05) * sgemm_tiles::microseconds(m, n, k, 1);
+    const double tiled = sgemm_tiles::microseconds(m, n, k, 1);
+    line = (k % 32 != 0 || n % 4 != 0 ? 1.15 : 1.05) * tiled;
     const sgemm_deal_plan::Plan deal = sgemm_deal_plan::plan_of(m, n, k);
-    if (deal.splits > 0 && .9 * deal.us < line) line = .9 * deal.us;
+    if (deal.splits > 0 && deal.us < tiled && .9 * deal.us < line) line = .9 * deal.us;  // the one that takes it otherwise
   }
   for (unsigned rows = best.better ? 2 : 1; rows <= 2; ++rows) {
     const unsigned long long count = (unsigned long long)((m + 16 * rows - 1) / (16 * rows)) * ((n + 15) / 16);
