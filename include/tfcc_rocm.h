@@ -65,8 +65,8 @@ int tfcc_rocm_stream_create(void** stream);
 int tfcc_rocm_stream_destroy(void* stream);
 /* Gives back what the library keeps for `stream` on the current device: the workspace the skinny quantized product
  * allocates per stream on first use (tfcc_rocm_gemv_u8s8s32; blocks it outgrew included - they stay allocated until
- * here, because launches recorded earlier may still use them).  The stream must be idle and no graph recorded on it
- * may be replayed afterwards.  tfcc_rocm_stream_destroy does this itself; call it for streams the library did not
+ * here, because launches made earlier may still use them).  The stream must be idle; graphs recorded on it use none of
+ * this.  tfcc_rocm_stream_destroy does this itself; call it for streams the library did not
  * create (a framework's own) before they go away.  No counterpart in the reference (its sessions own no such state). */
 int tfcc_rocm_stream_release(void* stream);
 int tfcc_rocm_stream_synchronize(void* stream);

@@ -39,6 +39,7 @@
 #include "gemv.hpp"
 #include "gemv_workspace.hpp"
 #include "qgemm_small.hpp"
+#include "stream_slots.hpp"
 
 namespace tfcc_rocm {
 
@@ -513,25 +514,31 @@ __global__ __launch_bounds__(256) void gemv_wide_kernel(const signed char* hotB,
 
 // ---- workspaces.  The ordinary entry points use one per (device, stream), allocated on first use and kept
 // (gemv_workspace.hpp has the rules): launches on one stream run in order, so they can share it; launches on
-// different streams may overlap.
+// different streams may overlap.  So may the replays of a graph and its stream's own launches, or two graphs that were recorded
+// on one stream, and the threads behind hipStreamPerThread: what is recorded, and that stream, get no workspace.
 gemv_ws::Registry gWorkspaces;
 
 unsigned long long workspace_key(int dev, hipStream_t stream) {
   return ((unsigned long long)(unsigned)dev << 56) ^ (unsigned long long)(uintptr_t)stream;
 }
-int workspace_alloc(void** mem, size_t bytes) {
-  if (hipMalloc(mem, bytes) != hipSuccess) return TFCC_ROCM_OUT_OF_MEMORY;
-  // (the fill runs on the null stream, and the stream that is going to use the words need not wait for that one)
-  if (hipMemset(*mem, 0, bytes) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
-    (void)hipFree(*mem);
-    return TFCC_ROCM_HIP_ERROR;
-  }
-  return 0;
-}
 void workspace_free(void* mem) { (void)hipFree(mem); }
 
 __global__ void clear_words_kernel(unsigned long long* words, size_t count) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x) words[i] = 0;
+}
+
+// A workspace of at least `blocks` column blocks for the stream, or false: then the product goes to a kernel without one.
+bool lease_workspace(hipStream_t stream, unsigned long long key, size_t blocks, gemv_ws::Lease* lease) {
+  if (!runs_in_order_now(stream)) return false;
+  const auto alloc = [stream](void** mem, size_t bytes) -> int {
+    *mem = allocate_beside_captures(bytes);
+    if (*mem == nullptr) return TFCC_ROCM_OUT_OF_MEMORY;
+    hipLaunchKernelGGL(clear_words_kernel, dim3(256), dim3(256), 0, stream, static_cast<unsigned long long*>(*mem), bytes / sizeof(unsigned long long));
+    const int e = check_launch("workspace clear");
+    if (e != TFCC_ROCM_OK) workspace_free(*mem);
+    return e;
+  };
+  return gWorkspaces.acquire(key, blocks, (size_t)kMaxM * kCols * sizeof(unsigned long long), true, alloc, lease) == gemv_ws::kOk;
 }
 
 // The address of `scratch` on the current device, looked up once per device.
@@ -648,23 +655,14 @@ int gemv_wide_launch(hipStream_t stream, bool staticWorkspace, const unsigned ch
   } else if (p.kParts > 1) {
     int dev = 0;
     TFCC_HIP_CHECK(hipGetDevice(&dev));
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    TFCC_HIP_CHECK(hipStreamIsCapturing(stream, &capture));
     key = workspace_key(dev, stream);
     gemv_ws::Lease lease;
-    const int e = gWorkspaces.acquire(key, p.colBlocks, (size_t)kMaxM * kCols * sizeof(unsigned long long),
-                                      capture == hipStreamCaptureStatusNone, workspace_alloc, &lease);
-    if (e == gemv_ws::kWouldAllocate)
-      // the stream is being recorded and has no workspace of this width yet: nothing may be allocated now, so this
-      // launch goes to the kernel that needs none (same sums; slower on a decode-sized B).  A product of the same
-      // width issued once before the recording, or the entry point without allocation, avoids this.
+    if (!lease_workspace(stream, key, p.colBlocks, &lease))  // the same sums, slower on a decode-sized B
       return gemv_alone_launch(stream, a, b, rowsumA, colsumB, offsetA, offsetB, ranges, rangeOut, m, n, k, accOut, scaleA, scaleB,
                                f32Out, colsumExact);
-    if (e == TFCC_ROCM_OUT_OF_MEMORY) return set_error(e, "skinny quantized matmul: no memory for the workspace");
-    if (e) return set_error(e, "skinny quantized matmul: workspace set-up failed");
     p.tiles = static_cast<unsigned long long*>(lease.mem);
     leased = true;
-    if (lease.mustClear) {  // a fill kernel, not a memset: this may be inside a recording
+    if (lease.mustClear) {
       hipLaunchKernelGGL(clear_words_kernel, dim3(256), dim3(256), 0, stream, p.tiles, lease.blocks * kMaxM * kCols);
       if (int ce = check_launch("workspace clear")) { gWorkspaces.mark_dirty(key); return ce; }
     }

@@ -2,10 +2,10 @@
 //
 // Rules it keeps, whatever the allocator behind it:
 //   * a workspace that has been handed to a launch is never freed while its stream may still use it: when a wider
-//     product needs a larger one, the old block is retired, not released - launches recorded earlier (a captured
-//     graph replays with the pointer it was recorded with) keep a valid, all-zero workspace;
-//   * growing needs an allocation, and the caller says whether one is allowed right now (not while the stream is
-//     being captured): if not, acquire() reports kWouldAllocate and the caller takes a path without a workspace;
+//     product needs a larger one, the old block is retired, not released, and launches made earlier keep theirs;
+//   * growing needs an allocation, and the caller says whether one is allowed right now: if not, acquire() reports
+//     kWouldAllocate; a failed one is reported by the allocator's code.  Either way the caller takes a path without a
+//     workspace;
 //   * an entry whose last launch did not go through is marked, and the next acquire() reports that the block must
 //     be cleared on the stream before it is used again;
 //   * release() gives back everything kept for one stream, forget-me-not for streams that are about to go away.
@@ -31,12 +31,12 @@ struct Lease {
 
 class Registry {
  public:
-  using AllocFn = int (*)(void** mem, size_t bytes);  // allocates and zero-fills; 0 on success, else an error code
   using FreeFn = void (*)(void* mem);
 
   // A workspace of at least `blocks` column blocks of `bytesPerBlock` for `key`.  Returns kOk, kWouldAllocate
-  // (only when !mayAllocate) or the allocator's error code.
-  int acquire(unsigned long long key, size_t blocks, size_t bytesPerBlock, bool mayAllocate, AllocFn alloc, Lease* out) {
+  // (only when !mayAllocate) or the allocator's error code.  alloc(void** mem, size_t bytes): allocates and zero-fills; 0 on success.
+  template <class AllocFn>
+  int acquire(unsigned long long key, size_t blocks, size_t bytesPerBlock, bool mayAllocate, const AllocFn& alloc, Lease* out) {
     std::lock_guard<std::mutex> lock(mutex_);
     auto found = entries_.find(key);
     if (!mayAllocate && (found == entries_.end() || found->second.blocks < blocks)) return kWouldAllocate;

@@ -24,6 +24,18 @@ inline bool runs_in_order_now(hipStream_t stream) {
   return capturing == hipStreamCaptureStatusNone;
 }
 
+// Device memory, null if there is none: an allocation that breaks no capture that another thread has under way, and leaves no error.
+inline void* allocate_beside_captures(size_t bytes) {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  void* mem = nullptr;
+  const bool made = relaxed && hipMalloc(&mem, bytes) == hipSuccess;
+  if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (made) return mem;
+  (void)hipGetLastError();
+  return nullptr;
+}
+
 class StreamSlots {
  public:
   explicit StreamSlots(unsigned count) : count_(count) {}
@@ -72,16 +84,8 @@ class StreamPieces {
     const auto found = given_.find({dev, stream});
     if (found != given_.end()) return found->second;
     if (given_.size() == count_) return nullptr;
-    // an allocation may not break a capture that another thread has under way
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-    void* piece = nullptr;
-    const bool made = relaxed && hipMalloc(&piece, bytes_) == hipSuccess;
-    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
-    if (!made) {
-      (void)hipGetLastError();
-      return nullptr;
-    }
+    void* const piece = allocate_beside_captures(bytes_);
+    if (piece == nullptr) return nullptr;
     if (prepare_(stream, piece) != 0) {
       (void)hipFree(piece);
       return nullptr;
