@@ -9,8 +9,9 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-# m, k, n: any alignment (its workspace in parts of sixteen and of eight wavefronts), aligned, aligned with several steps a wavefront
-SHAPES = [(3, 5748, 10293), (2, 3001, 3999), (4, 2048, 8192), (8, 4096, 2304), (1, 16384, 17408)]
+# m, k, n: any alignment (its workspace in parts of sixteen and of eight wavefronts), aligned, aligned with a K that sixteen wavefronts
+# have in one part, aligned with several steps a wavefront
+SHAPES = [(3, 5748, 10293), (2, 3001, 3999), (4, 2048, 8192), (8, 4096, 2304), (4, 1024, 8192), (1, 16384, 17408)]
 
 
 def _operands(T, m, k, n, count):
@@ -63,7 +64,7 @@ def test_graphs_of_one_stream_replayed_on_two(pkg, T, m, k, n):
     torch.cuda.synchronize()
 
 
-@pytest.mark.parametrize("m,k,n", SHAPES[:4])
+@pytest.mark.parametrize("m,k,n", SHAPES[:5])
 def test_threads_on_the_per_thread_stream(pkg, T, m, k, n):
     import torch
     print("gemv threads", m, k, n, flush=True)
@@ -87,6 +88,26 @@ def test_threads_on_the_per_thread_stream(pkg, T, m, k, n):
         t.join()
     torch.cuda.synchronize()
     assert not failed
+    for some, (_, want) in zip(outs, cases):
+        for out in some:
+            assert np.array_equal(T.n(out), want)
+
+
+@pytest.mark.parametrize("m,k,n", [(4, 1024, 8192), (1, 944, 12800), (8, 768, 16016)])
+def test_calls_without_allocation_whose_k_is_one_part(pkg, T, m, k, n):
+    """They do not touch the one workspace of the entry point that allocates nothing: on two streams, without order."""
+    import torch
+    print("gemv one part", m, k, n, flush=True)
+    tb, cases = _operands(T, m, k, n, 2)
+    col, streams = pkg.reduce_sum(tb, False), [torch.cuda.Stream() for _ in range(2)]
+    rows = [pkg.reduce_sum(a, True) for a, _ in cases]
+    outs = [[torch.zeros((m, n), dtype=torch.int32, device="cuda") for _ in range(20)] for _ in cases]
+    torch.cuda.synchronize()
+    for pair in zip(*outs):
+        for i, (out, stream) in enumerate(zip(pair, streams)):
+            with torch.cuda.stream(stream):
+                pkg.gemv_dequant(cases[i][0], tb, rows[i], col, 3, -5, 1.0, None, acc=out, no_alloc=True)
+    torch.cuda.synchronize()
     for some, (_, want) in zip(outs, cases):
         for out in some:
             assert np.array_equal(T.n(out), want)

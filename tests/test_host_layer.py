@@ -120,6 +120,15 @@ def test_gemv_workspace_bookkeeping():
     assert res.returncode == 0 and "bookkeeping ok" in res.stdout, res.stdout[-2000:]
 
 
+def test_how_the_k_of_skinny_quantized_products_is_dealt_out():
+    """A launch without a workspace keeps a short K in one part (tests/cpp/gemv_wide_plan_tests.cpp)."""
+    exe = os.path.join(ROOT, "wechat-tfcc_amd", "host", "build", "gemv_wide_plan_tests")
+    if not os.path.exists(exe):
+        subprocess.check_call(["make", "-C", os.path.join(ROOT, "wechat-tfcc_amd", "host"), "build/gemv_wide_plan_tests"])
+    res = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert res.returncode == 0 and "all passed" in res.stdout, res.stdout[-2000:]
+
+
 def test_lstm_sequences_that_do_not_fit_on_the_gpu_are_left_to_the_steps():
     """A GPU with fewer CUs than the launch has workgroups: no workspace, so no launch (tests/cpp/lstm_plan_tests.cpp)."""
     exe = os.path.join(ROOT, "wechat-tfcc_amd", "host", "build", "lstm_plan_tests")

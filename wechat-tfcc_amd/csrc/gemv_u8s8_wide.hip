@@ -37,6 +37,7 @@
 
 #include "common.hpp"
 #include "gemv.hpp"
+#include "gemv_wide_plan.hpp"
 #include "gemv_workspace.hpp"
 #include "qgemm_small.hpp"
 #include "stream_slots.hpp"
@@ -48,13 +49,11 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 
 namespace {
 
-constexpr int kCols = 256;     // columns per workgroup
+using gemv_wide_plan::kCols;
 constexpr int kMaxM = 8;
 constexpr unsigned kMaxStaticN = 32768;  // widest B the workspace inside the library serves
 constexpr unsigned kMaxStaticBlocks = kMaxStaticN / kCols;
 constexpr unsigned long long kPackMask = (1ull << 29) - 1;
-constexpr int kDefaultWaves = 16;               // wavefronts per workgroup
-constexpr unsigned kDefaultStepsPerWave = 1;    // 64-row steps per wavefront
 
 struct GemvWideParams {
   const unsigned char* A;
@@ -622,53 +621,45 @@ int gemv_wide_launch(hipStream_t stream, bool staticWorkspace, const unsigned ch
   p.offsetA = offsetA; p.offsetB = offsetB;
   p.M = m; p.N = n; p.K = k;
   p.colBlocks = (n + kCols - 1) / kCols;
-  const unsigned steps = (k + 63) / 64;
   const bool ragged = !gemv_wide_supported(a, b, m, n, k);
-  int waves = kDefaultWaves;
-  unsigned spw = kDefaultStepsPerWave;
-  // more steps per wavefront once the grid would exceed about four workgroups per CU (sixteen wavefronts make
-  // one step each: a product that needs more goes to four wavefronts of several steps)
-  if (waves == 16 && (spw != 1 || (unsigned long long)p.colBlocks * ((steps + 15) / 16) > 1024)) { waves = 4; spw = 4; }
-  while ((unsigned long long)p.colBlocks * ((steps + waves * spw - 1) / (waves * spw)) > 1024 && spw < 64) spw *= 2;
-  // Sixteen wavefronts of one step leave most CUs without work while there are few, and a workgroup's bytes go through one CU: eight
-  // of them, us: 1984 x 5056 7.6 -> 6.3, 3200 x 2688 7.6 -> 6.5, 1344 x 9792 7.8 -> 6.7; past 900 wavefronts 6336 x 2560 7.2 -> 7.6, 5760 x
-  // 9792 12.8 -> 13.8.  Ragged loads take a CU longer: 2104 x 9276 8.3 -> 7.9, 5789 x 3292 8.9 -> 8.5, 3024 x 8698 9.5 -> 9.9.  (Four:
-  // more parts to add up, 1984 x 5056 7.6, 1344 x 9792 7.8.)
-  if (spw == 1 && (unsigned long long)p.colBlocks * steps < (ragged ? 1400u : 900u)) waves = 8;
-  p.stepsPerWave = spw;
-  p.kParts = (steps + waves * spw - 1) / (waves * spw);
+  // (The calls that share the workspace inside the library touch it only where sixteen wavefronts do not cover K either.)
+  gemv_wide_plan::Plan plan = gemv_wide_plan::plan_of(n, k, ragged, !staticWorkspace);
+  unsigned long long key = 0;
+  bool leased = false;
+  gemv_ws::Lease lease;
+  if (!staticWorkspace && plan.parts > 1) {
+    int dev = 0;
+    TFCC_HIP_CHECK(hipGetDevice(&dev));
+    key = workspace_key(dev, stream);
+    leased = lease_workspace(stream, key, p.colBlocks, &lease);
+    if (!leased) plan = gemv_wide_plan::plan_of(n, k, ragged, false);
+    if (!leased && plan.parts > 1)  // the same sums, slower on a decode-sized B
+      return gemv_alone_launch(stream, a, b, rowsumA, colsumB, offsetA, offsetB, ranges, rangeOut, m, n, k, accOut, scaleA, scaleB,
+                               f32Out, colsumExact);
+  }
+  p.stepsPerWave = plan.stepsPerWave;
+  p.kParts = plan.parts;
   p.chunk = (p.colBlocks * p.kParts + 7) / 8;
   // Two rows per workspace word while the sum of the parts' biased partial sums stays inside a 29-bit field: a part
   // of R rows sums to at most R x 255 x 128 in absolute value, the bias is the next power of two, and a biased sum
   // is below twice the bias.
   {
-    const unsigned long long bound = (unsigned long long)waves * spw * 64 * 32640ull;
+    const unsigned long long bound = (unsigned long long)plan.waves * plan.stepsPerWave * 64 * 32640ull;
     unsigned long long bias = 1;
     while (bias <= bound) bias <<= 1;
     p.packBias = (p.kParts < 64 && p.kParts * 2 * bias <= (1ull << 29)) ? (unsigned)bias : 0u;
   }
-  unsigned long long key = 0;
-  bool leased = false;
   if (staticWorkspace) {
     TFCC_REQUIRE(n <= kMaxStaticN, "skinny quantized matmul without allocation: n %u beyond the %u columns its workspace holds", n, kMaxStaticN);
     if (int e = static_workspace(&p.tiles)) return e;
-  } else if (p.kParts > 1) {
-    int dev = 0;
-    TFCC_HIP_CHECK(hipGetDevice(&dev));
-    key = workspace_key(dev, stream);
-    gemv_ws::Lease lease;
-    if (!lease_workspace(stream, key, p.colBlocks, &lease))  // the same sums, slower on a decode-sized B
-      return gemv_alone_launch(stream, a, b, rowsumA, colsumB, offsetA, offsetB, ranges, rangeOut, m, n, k, accOut, scaleA, scaleB,
-                               f32Out, colsumExact);
+  } else if (leased) {
     p.tiles = static_cast<unsigned long long*>(lease.mem);
-    leased = true;
     if (lease.mustClear) {
       hipLaunchKernelGGL(clear_words_kernel, dim3(256), dim3(256), 0, stream, p.tiles, lease.blocks * kMaxM * kCols);
       if (int ce = check_launch("workspace clear")) { gWorkspaces.mark_dirty(key); return ce; }
     }
   }
-  int status;
-  status = launch_wide_rows(stream, p, waves, ragged, colsumExact);
+  const int status = launch_wide_rows(stream, p, plan.waves, ragged, colsumExact);
   if (status != TFCC_ROCM_OK && leased) gWorkspaces.mark_dirty(key);
   return status;
 }
