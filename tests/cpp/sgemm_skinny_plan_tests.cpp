@@ -1,0 +1,53 @@
+// Which fp32 products take the kernels whose workgroups share a K (wechat-tfcc_amd/csrc/sgemm_skinny_plan.hpp), on the host: no GPU.
+// With arguments, groups of m n k: prints kernel, splits and row blocks or column blocks of each product.
+#include <cstdio>
+#include <cstdlib>
+
+#include "sgemm_skinny_plan.hpp"
+#include "sgemm_split_plan.hpp"
+
+using namespace tfcc_rocm;
+using namespace tfcc_rocm::sgemm_skinny_plan;
+
+static int failures = 0;
+#define EXPECT(cond)                                         \
+  do {                                                       \
+    if (!(cond)) {                                           \
+      ++failures;                                            \
+      std::printf("FAIL line %d: %s\n", __LINE__, #cond);    \
+    }                                                        \
+  } while (0)
+
+// of m x k times k x n, dense
+static Choice chosen(unsigned m, unsigned k, unsigned n) {
+  return choose(m, n, k, [&] { return sgemm_split_plan::kernel_of(m, n, k, k, n, n, false, 1) != sgemm_split_plan::kNone; });
+}
+
+int main(int argc, char** argv) {
+  if (argc > 1) {
+    const char* const names[] = {"other", "skinny", "deal"};
+    for (int i = 1; i + 2 < argc; i += 3) {
+      const Choice c = chosen(std::atoi(argv[i]), std::atoi(argv[i + 1]), std::atoi(argv[i + 2]));
+      std::printf("%s %u %u\n", names[c.kernel], c.kernel == kDeal ? c.deal.splits : c.skinny.splits, c.kernel == kDeal ? c.deal.blocks : c.skinny.rows);
+    }
+    return 0;
+  }
+  for (unsigned m = 1; m <= 3000; m = m * 6 / 5 + 1)
+    for (unsigned n = 1; n <= 20000; n = n * 6 / 5 + 1)
+      for (unsigned k = 1; k <= 20000; k = k * 6 / 5 + 1) {
+        int asked = 0;
+        const Choice c = choose(m, n, k, [&] { return ++asked > 100; });
+        const sgemm_deal_plan::Plan deal = sgemm_deal_plan::plan_of(m, n, k);
+        EXPECT(c.deal.splits == deal.splits && c.deal.blocks == deal.blocks && c.deal.us == deal.us);
+        EXPECT(asked <= (c.deal.splits > 0 && !c.skinny.better ? 1 : 0));  // the rule of the bf16 ops only where it decides
+        EXPECT(c.kernel != kDeal || c.deal.splits > 0);
+        if (c.kernel != kSkinny) continue;
+        // splits of at least 512 k, the partial tiles within the memory in which they meet
+        const unsigned tall = 16 * c.skinny.rows;
+        const unsigned long long tiles = (unsigned long long)((m + tall - 1) / tall) * ((n + 15) / 16);
+        EXPECT(c.skinny.better && (c.skinny.rows == 1 || (c.skinny.rows == 2 && m > 16)));
+        EXPECT(c.skinny.splits == 1 || (k / c.skinny.splits >= 512 && tiles * c.skinny.rows * c.skinny.splits <= kMaxParts));
+      }
+  if (failures == 0) std::printf("sgemm skinny plan: all passed\n");
+  return failures != 0;
+}

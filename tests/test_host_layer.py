@@ -147,6 +147,15 @@ def test_how_the_k_of_fp32_products_is_dealt_out():
     assert res.returncode == 0 and "all passed" in res.stdout, res.stdout[-2000:]
 
 
+def test_which_fp32_products_share_a_k():
+    """The limits of the rule, and that the plan of the other kernel is worked out once (tests/cpp/sgemm_skinny_plan_tests.cpp)."""
+    exe = os.path.join(ROOT, "wechat-tfcc_amd", "host", "build", "sgemm_skinny_plan_tests")
+    if not os.path.exists(exe):
+        subprocess.check_call(["make", "-C", os.path.join(ROOT, "wechat-tfcc_amd", "host"), "build/sgemm_skinny_plan_tests"])
+    res = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert res.returncode == 0 and "all passed" in res.stdout, res.stdout[-2000:]
+
+
 def test_which_fp32_products_run_on_the_bf16_matrix_cores():
     """The limits of the rule, and that B given transposed goes where B as stored goes (tests/cpp/sgemm_split_plan_tests.cpp)."""
     exe = os.path.join(ROOT, "wechat-tfcc_amd", "host", "build", "sgemm_split_plan_tests")

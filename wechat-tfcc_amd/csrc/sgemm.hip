@@ -15,7 +15,7 @@
 // wavefront's column range) so that a lane owns NI consecutive output columns.
 #include "common.hpp"
 #include "sgemm_params.hpp"
-#include "sgemm_deal_plan.hpp"
+#include "sgemm_skinny_plan.hpp"
 #include "sgemm_split_plan.hpp"
 #include "sgemm_tiles.hpp"
 
@@ -448,19 +448,11 @@ int dispatch(hipStream_t s, const SgemmParams& p, bool vec, bool small, bool tb,
   // One product, or a few that share A, of too few rows and columns for the kernels below to occupy the chip.  (A true
   // batch keeps the tiled kernels, see below.)
   if (fillBatch == 1 && small) {
-    // Which of the two kernels whose workgroups share a K: the one for tiles of 32 rows where it is thought to be faster than the
-    // other by a tenth, or than the tiled kernels at all.  Of 220 products of 17 to 1024 rows and 768 k and more it takes 47,
-    // at 0.79 of the time (up to 1.0), another 13 lose a tenth without it.  What the bf16 matrix ops take stays there.
-    const sgemm_detail::SkinnyPlan skinny = sgemm_detail::sgemm_skinny_plan(m, n, k);
-    const double few = skinny.better ? skinny.us : 0;
-    const sgemm_deal_plan::Plan deal = sgemm_deal_plan::plan_of(m, n, k);
-    if (deal.splits > 0 &&
-        deal.us < (few > 0 ? .9 * few
-                   : sgemm_split_plan::kernel_of(m, n, k, p.lda, p.ldb, p.ldc, tb, fillBatch) == sgemm_split_plan::kNone
-                       ? sgemm_tiles::microseconds(m, n, k, fillBatch)
-                       : 0))
-      return sgemm_detail::sgemm_deal_launch(s, p, deal.splits, deal.blocks, tb);
-    if (few > 0) return sgemm_detail::sgemm_skinny_launch(s, p, skinny, tb);
+    const sgemm_skinny_plan::Choice c = sgemm_skinny_plan::choose(m, n, k, [&] {
+      return sgemm_split_plan::kernel_of(m, n, k, p.lda, p.ldb, p.ldc, tb, fillBatch) != sgemm_split_plan::kNone;
+    });
+    if (c.kernel == sgemm_skinny_plan::kDeal) return sgemm_detail::sgemm_deal_launch(s, p, c.deal.splits, c.deal.blocks, tb);
+    if (c.kernel == sgemm_skinny_plan::kSkinny) return sgemm_detail::sgemm_skinny_launch(s, p, c.skinny, tb);
   }
   if (small) {
     const int split = sgemm_split_plan::kernel_of(m, n, k, p.lda, p.ldb, p.ldc, tb, fillBatch);

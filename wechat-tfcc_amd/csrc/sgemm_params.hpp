@@ -4,6 +4,7 @@
 
 #include "common.hpp"
 #include "qgemm_params.hpp"  // UDiv: division by multiply-high
+#include "sgemm_skinny_plan.hpp"
 
 namespace tfcc_rocm {
 namespace sgemm_detail {
@@ -136,14 +137,8 @@ int sgemv_launch(hipStream_t stream, const SgemmParams& p);
 
 // The kernel for few rows (sgemm_skinny.hip): one product, or the grouped form; any alignment, B as stored or transposed,
 // operands below 2^30 elements.
-struct SkinnyPlan {
-  unsigned splits, rows;  // workgroups that share a tile's K; blocks of sixteen rows in a tile
-  bool better;            // than the other kernels
-  double us;
-};
-SkinnyPlan sgemm_skinny_plan(unsigned m, unsigned n, unsigned k);
 void sgemm_skinny_release_stream(int dev, hipStream_t stream);
-int sgemm_skinny_launch(hipStream_t stream, const SgemmParams& p, const SkinnyPlan& plan, bool transB);
+int sgemm_skinny_launch(hipStream_t stream, const SgemmParams& p, const sgemm_skinny_plan::Plan& plan, bool transB);
 
 // The kernel for a K that is dealt out over the wavefronts of one or several workgroups (sgemm_deal.hip), as sgemm_deal_plan.hpp
 // says: one product, or the grouped form; any alignment, B as stored or transposed, operands below 2^30 elements.

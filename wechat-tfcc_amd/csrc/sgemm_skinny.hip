@@ -23,15 +23,16 @@
 #include <type_traits>
 
 #include "common.hpp"
-#include "sgemm_deal_plan.hpp"
 #include "sgemm_params.hpp"
-#include "sgemm_tiles.hpp"
+#include "sgemm_skinny_plan.hpp"
 #include "stream_slots.hpp"
 
 namespace tfcc_rocm {
 namespace {
 
 using sgemm_detail::SgemmParams;
+using sgemm_skinny_plan::kMaxParts;
+using sgemm_skinny_plan::Plan;
 
 typedef float skinny_v4f __attribute__((ext_vector_type(4)));
 
@@ -39,8 +40,7 @@ constexpr int kWaves = 8;  // two workgroups to a CU: tiles that are no multiple
 constexpr int kBatch = 4;  // steps asked for at once
 
 // The memory in which the splits of a tile meet: a piece per stream, asked for by the first product that splits.
-constexpr unsigned kMaxParts = 1024, kMaxGroups = 4;  // kMaxParts: blocks of 16 x 16 x splits of a product
-constexpr unsigned kPieceTiles = kMaxParts * kMaxGroups;
+constexpr unsigned kMaxGroups = 4, kPieceTiles = kMaxParts * kMaxGroups;
 struct Meeting {
   float partials[256 * (size_t)kPieceTiles];
   unsigned counts[kPieceTiles];  // zero between launches: the workgroup that arrives last sees to it
@@ -49,78 +49,6 @@ int clear_counts(hipStream_t stream, void* piece) {
   return tfcc_rocm_fill_async(stream, static_cast<Meeting*>(piece)->counts, 0, sizeof(unsigned), kPieceTiles);
 }
 StreamPieces gPieces(sizeof(Meeting), 64, clear_counts);  // 4 MB each
-
-// Whether a product takes this kernel, and over how many workgroups a tile's K is split: from the sizes of one product
-// alone, so that it is summed the same way alone, in a group and with B transposed.  Nanoseconds as measured, launch aside:
-// a CU takes 2.8 per k of every tile it has; arriving and adding up costs 1300 and 200 more per split; the 32-row tiles with
-// four K groups take 5.1 per k while there is one for each CU.  (The line stands at 4.6, so that what is in doubt stays
-// where it was.)  Splits of less than 512 k end before their loads have paid for the arrival: 2048 -> 512 with 9 rows, 7.4 us in
-// splits of 256 against 6.2.  Below 256 k nothing is split in the tiled kernels either, and a product of more than eight rows keeps
-// their bits, which are those it has in a batch.
-//
-// Up to eight rows the other kernel is the streaming one (sgemv.hip), which has a CU for 32 columns and walks what K has
-// beyond a multiple of 64 eight rows at a time.  See takes_few_rows.
-//
-// More than sixteen rows have tiles of 32 as well, which read B once for two blocks of rows, one workgroup to a CU: they are taken
-// where the times below, fitted to 900 launches of 170 products of 17 to 100 rows and met within 5 %, say so.  Against the tiled kernels,
-// whose estimate is met without a remainder and from cache (1.19 of it with weights from memory, 1.27 with a K or an N that is no
-// multiple of their pieces), and against tiles of 16: 26 x 1328 x 3072 10.7 -> 8.4 us, 18 x 1006 x 3222 8.6 -> 6.7, 29 x 768 x 3072
-// 7.1 -> 6.1, 41 x 968 x 1952 8.3 -> 7.1, 94 x 3048 x 400 10.2 -> 9.0.
-using sgemm_detail::SkinnyPlan;
-
-// Up to eight rows: here or in the streaming kernel.  300 products, replayed with weights from memory / from cache, streaming -> here: 8 x
-// 64 x 2048 3.8/3.6 -> 2.2/2.1 us, 4 x 496 x 302 11.4/6.1 -> 3.1/2.7, 8 x 832 x 960 5.3/4.8 -> 3.8/3.4, 1 x 424 x 1588 4.3/3.0 ->
-// 3.1/2.7; launched, 4 x 3072 x 768 12.0/8.0 -> 6.6/6.4, 1 x 8192 x 2048 20.5 -> 14.6, 8 x 2304 x 4000 14.0/11.0 -> 9.9/8.0.
-// The streaming kernel keeps one row of up to 1024 k, a multiple of its chunks of 64 (1 x 960 x 128 3.5/2.9, here 3.5/3.3; 1 x 192 x 966
-// 2.7/2.35, here 2.4/2.2, but its launch, which is the longer part, costs the host 0.15 less), and what reads
-// whole lines of B on most of the CUs, but for a short K: 1 x 5120 x 5120 27, here 34, 4 x 1024 x 5376 6.5/6.0, here 8.6/7.8, 4 x 4096
-// x 11008 36, here 47; 6 x 192 x 9216 6.4/5.7 -> 4.0/3.6, 2 x 16 x 5984 2.9/2.5 -> 2.4/2.3.  Other widths come here (4 x 1024 x 7100 10.6 -> 8.3,
-// 1 x 3000 x 7100 24 -> 16), and so do more than two rows of a K with a rest (4 x 700 x 6144 13.8 -> 7.0), except of wide and deep ones, which
-// the memory decides and 64-byte pieces do not suit (2 x 2000 x 15000 25, here 28, 4 x 4096 x 11000 39, here 45; 4 x 1000 x 16001 15.9 -> 13.2).
-bool takes_few_rows(unsigned m, unsigned n, unsigned k) {
-  if (n <= 4096) return m > 1 || k > 1024 || k % 64 != 0;
-  if (n % 32 != 0 || (k % 64 != 0 && m > 2)) return n < 10240 || k <= 1600;
-  return n < 10240 && k <= (m > 4 ? 512u : m > 2 ? 256u : 128u);
-}
-
-SkinnyPlan plan_of(unsigned m, unsigned n, unsigned k) {
-  const unsigned long long tiles = (unsigned long long)((m + 15) / 16) * ((n + 15) / 16);
-  if (k < (m > 8 ? 256u : 16u) || tiles > kMaxParts) return SkinnyPlan{1, 1, false, 0};
-  SkinnyPlan best{1, 1, false, 0};
-  unsigned long long bestCost = ~0ull;
-  for (unsigned s = 1; s == 1 || (s <= k / 512 && tiles * s <= kMaxParts); ++s) {
-    const unsigned long long perCu = (tiles * s + 255) / 256;
-    const unsigned long long cost = perCu * k * 28 / s + (s > 1 ? 13000 + 2000 * s : 0);
-    if (cost < bestCost) {
-      best.splits = s;
-      bestCost = cost;
-    }
-  }
-  best.us = 2.5 + bestCost * 1e-4;
-  best.better = m > 8 ? bestCost < (unsigned long long)k * 46 : takes_few_rows(m, n, k);
-  if (m <= 16) return best;
-  double line = .92 * best.us;
-  if (!best.better) {
-    const double tiled = sgemm_tiles::microseconds(m, n, k, 1);
-    line = (k % 32 != 0 || n % 4 != 0 ? 1.15 : 1.05) * tiled;
-    const sgemm_deal_plan::Plan deal = sgemm_deal_plan::plan_of(m, n, k);
-    if (deal.splits > 0 && deal.us < tiled && .9 * deal.us < line) line = .9 * deal.us;  // the one that takes it otherwise
-  }
-  for (unsigned rows = best.better ? 2 : 1; rows <= 2; ++rows) {
-    const unsigned long long count = (unsigned long long)((m + 16 * rows - 1) / (16 * rows)) * ((n + 15) / 16);
-    for (unsigned s = 1; s == 1 || s <= k / 512; ++s) {
-      if (count * rows * s > kMaxParts) break;
-      const double perCu = (double)((count * s + 255) / 256), filled = count * s / 256., thousands = k / (1000. * s);
-      const double us = rows == 1 ? 2.94 + perCu * (2.04 * thousands + .2) + .39 * filled * thousands + (s > 1 ? .07 + .38 * s : 0)
-                                  : 1.66 + perCu * (3.52 * thousands + 1.19) + .97 * filled * thousands + (s > 1 ? .66 + .28 * s : 0);
-      if (us < line) {
-        line = us;
-        best = SkinnyPlan{s, rows, true, us};
-      }
-    }
-  }
-  return best;
-}
 
 // TEAMS teams of eight wavefronts.  One: the workgroup has the split blockIdx.z of its tile and meets the others in `meeting`
 // (null for a product that is not split).  Two, where there is no such memory: the workgroup has all splits, the teams
@@ -345,7 +273,7 @@ __global__ __launch_bounds__(64 * kWaves * TEAMS, ROWS == 2 ? 2 : 4) void sgemm_
 }
 
 template <bool TRANSB>
-int launch_skinny(hipStream_t stream, SgemmParams p, const SkinnyPlan& plan) {
+int launch_skinny(hipStream_t stream, SgemmParams p, const Plan& plan) {
   const unsigned groups = p.groups ? p.groups : 1u;
   p.batch = 1;
   const unsigned splits = plan.splits;
@@ -376,9 +304,7 @@ int launch_skinny(hipStream_t stream, SgemmParams p, const SkinnyPlan& plan) {
 
 namespace sgemm_detail {
 
-SkinnyPlan sgemm_skinny_plan(unsigned m, unsigned n, unsigned k) { return plan_of(m, n, k); }
-
-int sgemm_skinny_launch(hipStream_t stream, const SgemmParams& p, const SkinnyPlan& plan, bool transB) {
+int sgemm_skinny_launch(hipStream_t stream, const SgemmParams& p, const Plan& plan, bool transB) {
   return transB ? launch_skinny<true>(stream, p, plan) : launch_skinny<false>(stream, p, plan);
 }
 
