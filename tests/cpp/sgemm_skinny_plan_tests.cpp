@@ -46,8 +46,12 @@ int main(int argc, char** argv) {
         const unsigned tall = 16 * c.skinny.rows;
         const unsigned long long tiles = (unsigned long long)((m + tall - 1) / tall) * ((n + 15) / 16);
         EXPECT(c.skinny.better && (c.skinny.rows == 1 || (c.skinny.rows == 2 && m > 16)));
+        // two row blocks: one workgroup to a CU, and an XCD has a run of tiles with all their splits on 32 CUs
+        if (c.skinny.rows == 2 && tiles * c.skinny.splits <= 256) EXPECT((tiles + 7) / 8 * c.skinny.splits <= 32);
         EXPECT(c.skinny.splits == 1 || (k / c.skinny.splits >= 512 && tiles * c.skinny.rows * c.skinny.splits <= kMaxParts));
       }
+  // 84 tiles: eleven on an XCD, so three splits are 33 workgroups there
+  EXPECT(chosen(17, 3163, 1336).skinny.rows == 1 && chosen(211, 1903, 192).skinny.rows == 1 && chosen(20, 5051, 784).skinny.rows == 1);
   if (failures == 0) std::printf("sgemm skinny plan: all passed\n");
   return failures != 0;
 }

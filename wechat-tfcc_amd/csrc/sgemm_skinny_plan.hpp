@@ -31,7 +31,9 @@ struct Plan {
 // where the times below, fitted to 900 launches of 170 products of 17 to 100 rows and met within 5 %, say so.  Against the tiled kernels,
 // whose estimate is met without a remainder and from cache (1.19 of it with weights from memory, 1.27 with a K or an N that is no
 // multiple of their pieces), and against tiles of 16: 26 x 1328 x 3072 10.7 -> 8.4 us, 18 x 1006 x 3222 8.6 -> 6.7, 29 x 768 x 3072
-// 7.1 -> 6.1, 41 x 968 x 1952 8.3 -> 7.1, 94 x 3048 x 400 10.2 -> 9.0.
+// 7.1 -> 6.1, 41 x 968 x 1952 8.3 -> 7.1, 94 x 3048 x 400 10.2 -> 9.0.  A CU takes one such workgroup, and an XCD has a run of tiles with
+// all their splits: 84 tiles in three splits are 33 workgroups on 32 CUs (17 x 3163 x 1336 12.3 us, 8.7 in tiles of 16; 211 x 1903 x 192 9.5
+// and 6.3).
 
 // Up to eight rows: here or in the streaming kernel.  300 products, replayed with weights from memory / from cache, streaming -> here: 8 x
 // 64 x 2048 3.8/3.6 -> 2.2/2.1 us, 4 x 496 x 302 11.4/6.1 -> 3.1/2.7, 8 x 832 x 960 5.3/4.8 -> 3.8/3.4, 1 x 424 x 1588 4.3/3.0 ->
@@ -75,7 +77,8 @@ inline Plan plan_of(unsigned m, unsigned n, unsigned k, const sgemm_deal_plan::P
     const unsigned long long count = (unsigned long long)((m + 16 * rows - 1) / (16 * rows)) * ((n + 15) / 16);
     for (unsigned s = 1; s == 1 || s <= k / 512; ++s) {
       if (count * rows * s > kMaxParts) break;
-      const double perCu = (double)((count * s + 255) / 256), filled = count * s / 256., thousands = k / (1000. * s);
+      const double perCu = (double)(rows == 1 ? (count * s + 255) / 256 : ((count + 7) / 8 * s + 31) / 32);
+      const double filled = count * s / 256., thousands = k / (1000. * s);
       const double us = rows == 1 ? 2.94 + perCu * (2.04 * thousands + .2) + .39 * filled * thousands + (s > 1 ? .07 + .38 * s : 0)
                                   : 1.66 + perCu * (3.52 * thousands + 1.19) + .97 * filled * thousands + (s > 1 ? .66 + .28 * s : 0);
       if (us < line) {
