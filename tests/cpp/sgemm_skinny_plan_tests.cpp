@@ -52,6 +52,9 @@ int main(int argc, char** argv) {
       }
   // 84 tiles: eleven on an XCD, so three splits are 33 workgroups there
   EXPECT(chosen(17, 3163, 1336).skinny.rows == 1 && chosen(211, 1903, 192).skinny.rows == 1 && chosen(20, 5051, 784).skinny.rows == 1);
+  // whole tiles, few columns and a K past 1024: tiled; more columns or a shorter K: two blocks
+  EXPECT(chosen(960, 1120, 128).kernel == kOther && chosen(674, 1344, 144).kernel == kOther && chosen(754, 1216, 136).kernel == kOther);
+  EXPECT(chosen(51, 1152, 1408).skinny.rows == 2 && chosen(618, 896, 112).skinny.rows == 2 && chosen(17, 1216, 2944).skinny.rows == 2);
   if (failures == 0) std::printf("sgemm skinny plan: all passed\n");
   return failures != 0;
 }

@@ -34,6 +34,12 @@ struct Plan {
 // 7.1 -> 6.1, 41 x 968 x 1952 8.3 -> 7.1, 94 x 3048 x 400 10.2 -> 9.0.  A CU takes one such workgroup, and an XCD has a run of tiles with
 // all their splits: 84 tiles in three splits are 33 workgroups on 32 CUs (17 x 3163 x 1336 12.3 us, 8.7 in tiles of 16; 211 x 1903 x 192 9.5
 // and 6.3).
+//
+// The tiled kernels' estimate lies between weights from cache and from memory, and tiles without a remainder take 0.78 of it from cache.  Two
+// blocks gain from memory, where there are many weights; with few columns there are not, and past 1024 k the rows no longer stay in the L2 of
+// every XCD either: 960 x 1120 x 128 6.5 -> 8.7 us (with weights from memory 7.6 -> 8.6), 674 x 1344 x 144 7.5 -> 8.9 (9.9 -> 9.0), 754 x 1216 x 136 7.1
+// -> 8.6 from cache.  Those stay with the tiled kernels.  More columns: 51 x 1152 x 1408 6.8 -> 7.3 (12.0 -> 8.7), 17 x 1216 x 2944 7.4 ->
+// 6.3 (12.3 -> 8.7).
 
 // Up to eight rows: here or in the streaming kernel.  300 products, replayed with weights from memory / from cache, streaming -> here: 8 x
 // 64 x 2048 3.8/3.6 -> 2.2/2.1 us, 4 x 496 x 302 11.4/6.1 -> 3.1/2.7, 8 x 832 x 960 5.3/4.8 -> 3.8/3.4, 1 x 424 x 1588 4.3/3.0 ->
@@ -70,7 +76,7 @@ inline Plan plan_of(unsigned m, unsigned n, unsigned k, const sgemm_deal_plan::P
   double line = .92 * best.us;
   if (!best.better) {
     const double tiled = sgemm_tiles::microseconds(m, n, k, 1);
-    line = (k % 32 != 0 || n % 4 != 0 ? 1.15 : 1.05) * tiled;
+    line = (k % 32 != 0 || n % 4 != 0 ? 1.15 : 2 * m > n && k > 1024 ? .78 : 1.05) * tiled;
     if (deal.splits > 0 && deal.us < tiled && .9 * deal.us < line) line = .9 * deal.us;  // the one that takes it otherwise
   }
   for (unsigned rows = best.better ? 2 : 1; rows <= 2; ++rows) {
