@@ -41,6 +41,8 @@ int main(int argc, char** argv) {
         EXPECT(c.deal.splits == deal.splits && c.deal.blocks == deal.blocks && c.deal.us == deal.us);
         EXPECT(asked <= (c.deal.splits > 0 && !c.skinny.better ? 1 : 0));  // the rule of the bf16 ops only where it decides
         EXPECT(c.kernel != kDeal || c.deal.splits > 0);
+        // replayed, a tile of 32 x 32 has one CU: neither a second round of them nor what fills the chip without splits
+        EXPECT(c.kernel != kDeal || (sgemm_deal_plan::tiles_of(m, n, 1) <= 256 && !c.skinny.unsplit));
         if (c.kernel != kSkinny) continue;
         // splits of at least 512 k, the partial tiles within the memory in which they meet
         const unsigned tall = 16 * c.skinny.rows;
@@ -55,6 +57,10 @@ int main(int argc, char** argv) {
   // whole tiles, few columns and a K past 1024: tiled; more columns or a shorter K: two blocks
   EXPECT(chosen(960, 1120, 128).kernel == kOther && chosen(674, 1344, 144).kernel == kOther && chosen(754, 1216, 136).kernel == kOther);
   EXPECT(chosen(51, 1152, 1408).skinny.rows == 2 && chosen(618, 896, 112).skinny.rows == 2 && chosen(17, 1216, 2944).skinny.rows == 2);
+  EXPECT(chosen(128, 3072, 768).kernel == kDeal && chosen(512, 6336, 456).kernel == kDeal && chosen(128, 2496, 1280).kernel == kDeal);
+  EXPECT(chosen(288, 7296, 920).kernel == kOther && chosen(485, 4448, 104).kernel == kSkinny && chosen(485, 4448, 104).skinny.splits == 1);
+  // whole tiles and few columns
+  EXPECT(chosen(398, 1344, 208).kernel != kDeal && chosen(332, 1664, 344).kernel != kDeal && chosen(128, 1344, 768).kernel != kDeal);
   if (failures == 0) std::printf("sgemm skinny plan: all passed\n");
   return failures != 0;
 }

@@ -29,12 +29,16 @@ inline double microseconds(unsigned m, unsigned n, unsigned k, unsigned splits, 
          (splits > 1 ? 1.27 + .2 * splits * blocks : 0);
 }
 
-// The sizes that the fit covers; splits of 250 k and more, for shorter ones end before their loads have paid for the meeting.  Fewer
-// than 64 tiles of 32 x 32 would gain as much, but not in a stream that is being captured, where a tile has one workgroup and the
-// kernel of 16 x 16 tiles four times as many (286 x 8129 x 70 18 -> 15 us, captured 31 -> 60).
+// The sizes that the fit covers; splits of 250 k and more, for shorter ones end before their loads have paid for the meeting.  In a
+// stream that is being captured a tile of 32 x 32 has one workgroup, whatever the splits.  Fewer than 64 of them would gain as much launched,
+// but the kernel of 16 x 16 tiles has four times as many there (286 x 8129 x 70 18 -> 15 us, captured 31 -> 60); more than 256 are a
+// second round, and gain little launched: 24 products with 259 to 336 tiles took 0.92 of the tiled kernels' time launched and 1.42 captured (288 x
+// 7296 x 920 52.8 -> 48.9, captured 54.3 -> 82.0).  160 products in between: launched 0.76 from cache and 0.62 with weights from memory, captured
+// 1.04 and 0.92, 1.2 to 1.5 from cache those of up to some 2000 k (128 x 3072 x 768 15.1 -> 12.7, captured 15.7 -> 22.3; from memory 25.6 -> 13.1,
+// captured 27.3 -> 27.8).
 inline Plan plan_of(unsigned m, unsigned n, unsigned k) {
   Plan best{0, 1, 1e30};
-  if (m < 17 || n < 32 || k < 768 || tiles_of(m, n, 1) < 64 || tiles_of(m, n, 1) > 700) return best;
+  if (m < 17 || n < 32 || k < 768 || tiles_of(m, n, 1) < 64 || tiles_of(m, n, 1) > 256) return best;
   for (unsigned blocks = 1; blocks <= 2; ++blocks)
     for (unsigned s = 1; s <= kMaxSplits; ++s) {
       if (s > 1 && (k / s < 250 || tiles_of(m, n, blocks) * blocks * 1024 * s > kMaxParts)) break;

@@ -14,6 +14,7 @@ struct Plan {
   unsigned splits, rows;  // workgroups that share a tile's K; blocks of sixteen rows in a tile
   bool better;            // than the other kernels
   double us;
+  bool unsplit;           // tiles of sixteen rows fill the chip without splits
 };
 
 // Whether a product takes this kernel, and over how many workgroups a tile's K is split: from the sizes of one product
@@ -56,11 +57,23 @@ inline bool takes_few_rows(unsigned m, unsigned n, unsigned k) {
   return n < 10240 && k <= (m > 4 ? 512u : m > 2 ? 256u : 128u);
 }
 
+// What the dealt kernel has to be thought to take less than, to be taken instead of the tiled ones.  Their estimate lies between weights
+// from cache and from memory.  Tiles without a remainder and with a short K are nearer to the former, 0.78 of it, while weights from memory are
+// what the dealt kernel gains most from; with few columns there are not many weights, and what would be lost counts: with a line
+// at 0.97 as for wider ones, launched from cache / memory and replayed from cache / memory, 398 x 1344 x 208 took 1.11/0.85 and 1.40/1.10 of
+// the tiled kernels' time, 332 x 1664 x 344 1.07/0.80 and 1.41/1.07, 896 x 2048 x 124 1.09/0.78 and 1.42/1.07; 128 x 1344 x 768, where both are
+// thought to be equal, 1.10/0.83 and 1.42/1.02.
+inline double dealt_below(unsigned m, unsigned n, unsigned k) {
+  const double tiled = sgemm_tiles::microseconds(m, n, k, 1);
+  if (tiled >= 15 || k % 32 != 0 || n % 4 != 0) return tiled;
+  return 2 * m > n ? .84 * tiled : .97 * tiled;
+}
+
 // deal: what sgemm_deal_plan.hpp has for the same product.
 inline Plan plan_of(unsigned m, unsigned n, unsigned k, const sgemm_deal_plan::Plan& deal) {
   const unsigned long long tiles = (unsigned long long)((m + 15) / 16) * ((n + 15) / 16);
-  if (k < (m > 8 ? 256u : 16u) || tiles > kMaxParts) return Plan{1, 1, false, 0};
-  Plan best{1, 1, false, 0};
+  if (k < (m > 8 ? 256u : 16u) || tiles > kMaxParts) return Plan{1, 1, false, 0, false};
+  Plan best{1, 1, false, 0, false};
   unsigned long long bestCost = ~0ull;
   for (unsigned s = 1; s == 1 || (s <= k / 512 && tiles * s <= kMaxParts); ++s) {
     const unsigned long long perCu = (tiles * s + 255) / 256;
@@ -73,11 +86,12 @@ inline Plan plan_of(unsigned m, unsigned n, unsigned k, const sgemm_deal_plan::P
   best.us = 2.5 + bestCost * 1e-4;
   best.better = m > 8 ? bestCost < (unsigned long long)k * 46 : takes_few_rows(m, n, k);
   if (m <= 16) return best;
+  best.unsplit = best.better && best.splits == 1;
   double line = .92 * best.us;
   if (!best.better) {
     const double tiled = sgemm_tiles::microseconds(m, n, k, 1);
     line = (k % 32 != 0 || n % 4 != 0 ? 1.15 : 2 * m > n && k > 1024 ? .78 : 1.05) * tiled;
-    if (deal.splits > 0 && deal.us < tiled && .9 * deal.us < line) line = .9 * deal.us;  // the one that takes it otherwise
+    if (deal.splits > 0 && deal.us < dealt_below(m, n, k) && .9 * deal.us < line) line = .9 * deal.us;  // the one that takes it otherwise
   }
   for (unsigned rows = best.better ? 2 : 1; rows <= 2; ++rows) {
     const unsigned long long count = (unsigned long long)((m + 16 * rows - 1) / (16 * rows)) * ((n + 15) / 16);
@@ -89,7 +103,7 @@ inline Plan plan_of(unsigned m, unsigned n, unsigned k, const sgemm_deal_plan::P
                                   : 1.66 + perCu * (3.52 * thousands + 1.19) + .97 * filled * thousands + (s > 1 ? .66 + .28 * s : 0);
       if (us < line) {
         line = us;
-        best = Plan{s, rows, true, us};
+        best = Plan{s, rows, true, us, best.unsplit};
       }
     }
   }
@@ -106,14 +120,15 @@ struct Choice {
 // Which of the two kernels whose workgroups share a K: the one for tiles of 32 rows where it is thought to be faster than the
 // other by a tenth, or than the tiled kernels at all.  Of 220 products of 17 to 1024 rows and 768 k and more it takes 47,
 // at 0.79 of the time (up to 1.0), another 13 lose a tenth without it.  What the bf16 matrix ops take stays there (bf16, asked for
-// where it matters).
+// where it matters), and so does what fills the chip in tiles of 16 without splits: launched it would gain a quarter, but replayed, when
+// the dealt kernel has a CU for a tile, take 1.8 of the time (485 x 4448 x 104 16.5 us, dealt 12.5 launched and 29.9 replayed).
 template <class Asked>
 inline Choice choose(unsigned m, unsigned n, unsigned k, const Asked& bf16) {
-  Choice c{kOther, {1, 1, false, 0}, sgemm_deal_plan::plan_of(m, n, k)};
+  Choice c{kOther, {1, 1, false, 0, false}, sgemm_deal_plan::plan_of(m, n, k)};
   c.skinny = plan_of(m, n, k, c.deal);
   if (c.skinny.better) c.kernel = kSkinny;
-  if (c.deal.splits > 0 &&
-      c.deal.us < (c.skinny.better ? .9 * c.skinny.us : bf16() ? 0 : sgemm_tiles::microseconds(m, n, k, 1)))
+  if (c.deal.splits > 0 && !c.skinny.unsplit &&
+      c.deal.us < (c.skinny.better ? .9 * c.skinny.us : bf16() ? 0 : dealt_below(m, n, k)))
     c.kernel = kDeal;
   return c;
 }
