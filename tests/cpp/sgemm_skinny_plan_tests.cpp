@@ -61,6 +61,13 @@ int main(int argc, char** argv) {
   EXPECT(chosen(288, 7296, 920).kernel == kOther && chosen(485, 4448, 104).kernel == kSkinny && chosen(485, 4448, 104).skinny.splits == 1);
   // whole tiles and few columns
   EXPECT(chosen(398, 1344, 208).kernel != kDeal && chosen(332, 1664, 344).kernel != kDeal && chosen(128, 1344, 768).kernel != kDeal);
+  // one and two rows of whole chunks: few columns, and a B that the L2s hold, are streamed; a remainder, more rows or columns are not
+  for (unsigned m = 1; m <= 2; ++m) {
+    EXPECT(chosen(m, 1472, 64).kernel == kOther && chosen(m, 1216, 640).kernel == kOther && chosen(m, 2048, 3840).kernel == kOther);
+    EXPECT(chosen(m, 1792, 64).kernel == kSkinny && chosen(m, 1472, 768).kernel == kSkinny && chosen(m, 1473, 64).kernel == kSkinny);
+    EXPECT(chosen(m, 2304, 2304).kernel == kSkinny && chosen(m, 2048, 4096).kernel == kSkinny && chosen(m, 2048, 3841).kernel == kSkinny);
+  }
+  EXPECT(chosen(3, 1472, 64).kernel == kSkinny && chosen(3, 2048, 3840).kernel == kSkinny);
   if (failures == 0) std::printf("sgemm skinny plan: all passed\n");
   return failures != 0;
 }

@@ -51,8 +51,19 @@ struct Plan {
 // x 11008 36, here 47; 6 x 192 x 9216 6.4/5.7 -> 4.0/3.6, 2 x 16 x 5984 2.9/2.5 -> 2.4/2.3.  Other widths come here (4 x 1024 x 7100 10.6 -> 8.3,
 // 1 x 3000 x 7100 24 -> 16), and so do more than two rows of a K with a rest (4 x 700 x 6144 13.8 -> 7.0), except of wide and deep ones, which
 // the memory decides and 64-byte pieces do not suit (2 x 2000 x 15000 25, here 28, 4 x 4096 x 11000 39, here 45; 4 x 1000 x 16001 15.9 -> 13.2).
+// One and two rows of whole chunks stay there too where splitting K does not pay.  Few columns: two or three splits of up to 1600 k meet for
+// longer than they save (1 x 1472 x 64 launched 4.1 -> 4.8 us and replayed 3.9 -> 5.2, with weights from memory 4.4 -> 4.7 and 4.4 -> 5.2; from
+// 768 columns on memory decides, 1 x 1472 x 768 4.5 -> 4.7 and 6.9 -> 5.3).  And a B of 20 to 32 MB in whole lines, which the L2s of the eight
+// XCDs hold together and the streaming kernel reads in turn (1 x 2048 x 3840 launched 5.1 -> 7.0, from memory 11.5 -> 11.0; with fewer
+// columns there is more to gain from memory, 1 x 2304 x 2304 5.5 -> 5.9 and 11.2 -> 8.3).
 inline bool takes_few_rows(unsigned m, unsigned n, unsigned k) {
-  if (n <= 4096) return m > 1 || k > 1024 || k % 64 != 0;
+  if (n <= 4096) {
+    if (m > 2 || k % 64 != 0) return true;
+    if (k > 1152 && k <= 1600 && n <= 640) return false;
+    const unsigned long long words = (unsigned long long)k * n;
+    if (n % 128 == 0 && n >= 2688 && words > 5400000 && words < 8000000) return false;
+    return m > 1 || k > 1024;
+  }
   if (n % 32 != 0 || (k % 64 != 0 && m > 2)) return n < 10240 || k <= 1600;
   return n < 10240 && k <= (m > 4 ? 512u : m > 2 ? 256u : 128u);
 }
