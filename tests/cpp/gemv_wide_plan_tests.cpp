@@ -35,6 +35,10 @@ int main() {
         if (steps <= 16 && blocks <= 1024) EXPECT(without.parts == 1);
         else EXPECT(with.waves == without.waves && with.stepsPerWave == without.stepsPerWave && with.parts == without.parts);
       }
+  // any alignment: rows at odd addresses not while sixteen wavefronts to a workgroup leave CUs without work, nor just above the least work
+  EXPECT(!ragged_pays(10293, 2299, true) && !ragged_pays(1839, 11815, true) && !ragged_pays(2543, 4516, true) && !ragged_pays(11368, 2024, false));
+  EXPECT(ragged_pays(4782, 2448, true) && ragged_pays(9271, 2352, true) && ragged_pays(8635, 4002, true) && ragged_pays(5814, 7900, false) &&
+         ragged_pays(3704, 2052, true) && ragged_pays(11368, 2024, true));
   std::printf(failures ? "%d failures\n" : "all passed\n", failures);
   return failures != 0;
 }

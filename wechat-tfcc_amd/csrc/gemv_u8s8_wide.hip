@@ -586,15 +586,10 @@ bool gemv_wide_supported(const void* a, const void* b, unsigned m, unsigned n, u
          (unsigned long long)((k + 63) / 64) * ((n + kCols - 1) / kCols) >= 512;
 }
 
-// Against the kernel for small products of any alignment, us: 7900 x 5814 20.8 -> 12.6, 5799 x 9800 20.1 -> 13.4, 4755 x 4616 11.1 -> 9.0,
-// 2897 x 10788 12.9 -> 9.5, with exact sums 2448 x 4782 8.6 -> 7.3, 2052 x 3704 7.8 -> 6.4, 10124 x 1235 9.4 -> 7.8.  Below the line 6 x
-// 2432 x 7191 8.8 -> 9.3, 2 x 924 x 11952 6.5 -> 6.7, 8 x 4040 x 6689 10.9 -> 11.5, with exact sums 6 x 1766 x 5686 6.5 ->
-// 7.1, 4 x 883 x 10148 5.4 -> 6.4 (a K that short is read at once there too).
 bool gemv_wide_takes_ragged(unsigned m, unsigned n, unsigned k, bool colsumExact) {
   const unsigned long long blocks = (n + kCols - 1) / kCols, steps = (k + 63) / 64;
-  const unsigned least = colsumExact ? (n % 4 == 0 ? 420 : 700) : n % 4 == 0 ? 1400 : 1900;  // wavefronts
   return m >= 1 && m <= (unsigned)kMaxM && n >= 16 && k >= 16 && ((unsigned long long)k + 4160) * n + 4096 < (1ull << 31) &&
-         ((unsigned long long)m + 64) * k + 4096 < (1ull << 31) && blocks * steps >= least && steps >= 22 &&
+         ((unsigned long long)m + 64) * k + 4096 < (1ull << 31) && steps >= 22 && gemv_wide_plan::ragged_pays(n, k, colsumExact) &&
          blocks * ((steps + 15) / 16) <= 1024;
 }
 

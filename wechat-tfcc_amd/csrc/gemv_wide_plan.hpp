@@ -33,5 +33,18 @@ inline Plan plan_of(unsigned n, unsigned k, bool ragged, bool meets) {
   return p;
 }
 
+// Whether there is enough work for the form of any alignment, in wavefronts of 64 x 256.  Against the kernel for small products of any
+// alignment, us: 7900 x 5814 20.8 -> 12.6, 5799 x 9800 20.1 -> 13.4, with exact sums 2448 x 4782 8.6 -> 7.3, 2052 x 3704 7.8 -> 6.4, 10124 x
+// 1235 9.4 -> 7.8.  Below the line 6 x 2432 x 7191 8.8 -> 9.3, 2 x 924 x 11952 6.5 -> 6.7, 8 x 4040 x 6689 10.9 -> 11.5, with exact sums 6 x
+// 1766 x 5686 6.5 -> 7.1, 4 x 883 x 10148 5.4 -> 6.4 (a K that short is read at once there too), 5 x 4516 x 2543 6.2 -> 7.5.  With sixteen
+// wavefronts to a workgroup, from 1400 on, so few of them leave CUs without work, and rows at odd addresses take a CU's load path twice as
+// long: 32 products of 1400 to 2100 took 0.86 to 1.26 of the time there, none gained on the average (5 x 2299 x 10293 8.4 -> 10.0, 6 x 11815 x 1839
+// 9.1 -> 10.6), 17 without exact sums of 1400 to 1700 0.97 (8 x 2024 x 11368 7.4 -> 8.8); from 2100 on 0.8 (4 x 4002 x 8635 0.74).
+inline bool ragged_pays(unsigned n, unsigned k, bool exact) {
+  const unsigned long long work = (unsigned long long)((n + kCols - 1) / kCols) * ((k + 63) / 64);
+  if (!exact) return work >= (n % 4 == 0 ? 1700u : 2100u);
+  return n % 4 == 0 ? work >= 420 : work >= 2100 || (work >= 720 && work < 1400);
+}
+
 }  // namespace gemv_wide_plan
 }  // namespace tfcc_rocm
