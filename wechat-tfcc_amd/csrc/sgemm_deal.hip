@@ -58,6 +58,7 @@ __global__ __launch_bounds__(64 * kWaves * (ALONE ? 2 : 1), ALONE ? 4 : 2) void 
                                                                     unsigned chunk, unsigned splits, unsigned perWave, Meeting* meeting,
                                                                     const Arguments arguments) {
   const SgemmParams p = arguments.whole();
+  static_assert(NB == 1 || NB == 2, "a lane's columns of a row of B in one load");
   constexpr bool GROUPED = std::is_same<Arguments, SgemmParams>::value;
   constexpr int TEAMS = ALONE ? 2 : 1, THREADS = 64 * kWaves * TEAMS;
   constexpr int SETS = NB == 1 && !ALONE ? 4 : 2, ACCS = 4, ROWS = 1024 / THREADS, OUT = NB * ROWS;  // steps on their way, results that a thread finishes
@@ -113,12 +114,9 @@ __global__ __launch_bounds__(64 * kWaves * (ALONE ? 2 : 1), ALONE ? 4 : 2) void 
         if constexpr (NB == 1) {
           const auto w = __builtin_amdgcn_raw_buffer_load_b32(rsrcB, bOff[s], 0, 0);
           __builtin_memcpy(b, &w, 4);
-        } else if constexpr (NB == 2) {
+        } else {
           const auto w = __builtin_amdgcn_raw_buffer_load_b64(rsrcB, bOff[s], 0, 0);
           __builtin_memcpy(b, &w, 8);
-        } else {
-          const auto w = __builtin_amdgcn_raw_buffer_load_b128(rsrcB, bOff[s], 0, 0);
-          __builtin_memcpy(b, &w, 16);
         }
 #pragma unroll
         for (int j = 0; j < NB; ++j) o.b[j][s] = b[j];
