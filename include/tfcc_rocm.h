@@ -65,7 +65,8 @@ int tfcc_rocm_stream_create(void** stream);
 int tfcc_rocm_stream_destroy(void* stream);
 /* Gives back what the library keeps for `stream` on the current device: the workspace the skinny quantized product
  * allocates per stream on first use (tfcc_rocm_gemv_u8s8s32; blocks it outgrew included - they stay allocated until
- * here, because launches made earlier may still use them).  The stream must be idle; graphs recorded on it use none of
+ * here, because launches made earlier may still use them), and the memory in which the splits of fp32 products (12 MB and 4 MB)
+ * and of small int8 products (4 MB) meet.  The stream must be idle; graphs recorded on it use none of
  * this.  tfcc_rocm_stream_destroy does this itself; call it for streams the library did not
  * create (a framework's own) before they go away.  No counterpart in the reference (its sessions own no such state). */
 int tfcc_rocm_stream_release(void* stream);

@@ -1,5 +1,5 @@
 """int8 products of up to eight rows at any N, K and alignment, split over K: the last row and column of each operand, a K that ends in
-any row of a lane's sixteen, both numbers of wavefronts, given and formed column sums, and recorded on a stream that has a workspace and on one that has none.
+any row of a lane's sixteen, both numbers of wavefronts, given and formed column sums, and under capture with and without a workspace.
 Whole numbers, so the sums are exactly those of 64-bit integers."""
 import numpy as np
 import pytest

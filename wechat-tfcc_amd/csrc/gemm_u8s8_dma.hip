@@ -31,7 +31,7 @@
 // slabs whose B was loaded in words of four columns and transposed with byte permutes: us, before -> copies of words or registers,
 // 960 x 2976 x 900 21.4 -> 16.1, 1024 x 768 x 3076 13.4 -> 10.8, 2920 x 200 x 2500 15.7 -> 11.9, 974 x 7272 x 1136 43 -> 30;
 // 960 x 2973 x 896 21.8 -> 19.4, 1024 x 769 x 3073 17.7 -> 16.2, 1645 x 66 x 2631 10.3 -> 8.6, 952 x 4944 x 6577 108 -> 64.  240
-// drawn products of more than 64 such tiles, a quarter of them aligned as before, take 0.88 of the time; up to 1.06 four to six
+// drawn products of more than 64 such tiles, a quarter of them aligned as before, take 0.88 of the time (300 of another draw 0.90, 1.05 at most); up to 1.06 four to six
 // slabs of odd rows that two K groups of wavefronts shared (2267 x 414 x 175 9.5 -> 10.1).
 // (Two K groups of wavefronts to a tile gain nothing here: 960 x 2976 x 896 14.5 -> 14.6.  Aligned words with one word more,
 // shifted to their places in registers, are more to ask for: 960 x 2976 x 897 20.3 -> 26.3.)

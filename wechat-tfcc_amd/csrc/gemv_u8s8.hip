@@ -340,7 +340,8 @@ int gemv_launch(hipStream_t stream, const unsigned char* a, const signed char* b
   // The one-pass kernel's workgroups have all of K: 3 us and 0.11 more for every 64 k (8 x 12288 x 512: 24.3 us).  A long
   // K goes to tiles that several workgroups share (8.4 us), where those may have memory to meet in.
   // The line lies where weights from HBM pay for it: of 400 products none takes longer with them, on the average 0.65 of the
-  // time; with weights in cache 0.79, up to K = 3000 1.05 (1.17 at most; from HBM 0.88 there).
+  // time; with weights in cache 0.79, up to K = 3000 1.05 (1.17 at most; from HBM 0.88 there).  Plans of up to three trips to memory: sizes with more
+  // are large enough for the kernel above.
   const QGemmParams q = small_params(a, b, rowsumA, colsumB, offsetA, offsetB, ranges, rangeOut, m, n, k, accOut, colsumExact);
   if (qgemm_small_supported(q) && qgemm_small_splits(stream, m, n, k, 300 + 11 * (k / 64)))
     return qgemm_small_launch(stream, q, QSmallOutputs{f32Out, scaleB, scaleA}, true);

@@ -11,8 +11,7 @@
 // were no better (fewer workgroups, or more splits to meet).
 //
 // us, before (the kernels of sgemm_wave96.hip and sgemm_skinny.hip) -> now: 128 x 3072 x 768 19.1 -> 13.1, 128 x 4096 x 1024 24.6 -> 16.2, 64 x 2373 x
-// 1536 17.6 -> 11.3, 256 x 2048 x 512 13.5 -> 10.3, 624 x 3457 x 96 14.6 -> 11.4, 949 x 3011 x 69 18.6 -> 14.0, 96 x 7608 x 824
-// 30.8 -> 19.5, 75 x 4928 x 1344 29.3 -> 18.4.
+// 1536 17.6 -> 11.3, 256 x 2048 x 512 13.5 -> 10.3, 96 x 7608 x 824 30.8 -> 19.5, 75 x 4928 x 1344 29.3 -> 18.4.
 //
 // An element is the sum of its wavefronts' partial sums, added in the order of the wavefronts, then of the splits; wavefront w of
 // W has the steps w, w + W, ..., dealt in ascending order to four accumulators.  Against float64 that leaves a quarter of the
@@ -51,7 +50,9 @@ StreamPieces gPieces(sizeof(Meeting), 64, clear_counts);  // 12 MB each
 // ALONE: the workgroup has all splits of its tile, in two teams of eight wavefronts that take turns; the partial tiles of four splits
 // wait in LDS.  Replayed from a graph, the kernels of sgemm_wave96.hip and sgemm_skinny.hip -> this one: 75 x 4928 x 1344 29.5 -> 30.2
 // us, 96 x 7608 x 824 47.7 -> 46.6, 24 x 3183 x 2827 21.2 -> 23.9, 128 x 2384 x 992 16.7 -> 14.2, 466 x 5928 x 288 36.5 -> 32.9, 128 x 3072 x 768
-// 19.4 -> 23.5, 75 x 3072 x 832 19.4 -> 18.4, 369 x 1220 x 170 10.0 -> 11.5 (one team: 47, 69, 36, 16, 50, 38, 21 and 13).
+// 19.4 -> 23.5, 75 x 3072 x 832 19.4 -> 18.4, 369 x 1220 x 170 10.0 -> 11.5 (one team: 47, 69, 36, 16, 50, 38, 21 and 13).  Bound by what one CU
+// loads: the last of an odd number of splits shared by both teams took 1.02 to 1.1 of the time, one team with eight steps on their way
+// across the splits' borders 1.06 to 1.3 (256 x 2048 x 512 13.4 -> 16.4).  Which products that loses too much for: sgemm_deal_plan.hpp.
 template <int NB, bool TRANSB, bool ALONE, class Arguments>
 __global__ __launch_bounds__(64 * kWaves * (ALONE ? 2 : 1), ALONE ? 4 : 2) void sgemm_deal_kernel(const float* hotA, const float* hotB, unsigned M, unsigned N, unsigned K,
                                                                     unsigned lda, unsigned ldb, unsigned tilesM, unsigned tilesTotal,

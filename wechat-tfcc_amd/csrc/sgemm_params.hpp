@@ -37,7 +37,8 @@ struct SgemmParams {
 // Shorter argument blocks for what most launches are: one product, a flat batch without epilogue, and (behind the leading
 // scalar arguments of kernels that have those) what the tile store of one product needs.  A launch whose arguments take more than
 // 112 bytes costs the host 0.65 us more in two of three processes: us from launch to launch of an empty kernel, 112 bytes 2.75,
-// 116 bytes 3.4, 320 bytes 3.5 (2.3 whatever the size in the others).  A small product is bound by that: 1 x 768 x 768 4.5 -> 4.1.
+// 116 bytes 3.4, 320 bytes 3.5 (2.3 whatever the size in the others).  A small product is bound by its launch: 1 x 768 x 768 4.42 -> 4.21 in one of them, 4.30 -> 4.23 in
+// another, where runs of one side differ by as much.
 // whole(): the block as the kernels read it, everything else a constant.
 constexpr size_t kShortArguments = 112;
 
